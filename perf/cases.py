@@ -1,0 +1,499 @@
+"""The work a user of this package has it do, as cases that can be timed and whose outputs can be compared.
+
+Twelve kinds of case, one listed of each; `draw` takes a kind and spreads its sizes over the range the listed one stands
+for.  Image sizes are given in latent pixels (1/8 of the image's): 64 x 64 is a 512 x 512 image, 104 x 152 is 832 x 1216,
+128 x 128 is 1024 x 1024, the size SDXL is quoted on.  SDXL runs at every one of those aspect ratios, with and without
+guidance (two UNet rows per image or one), so batches, token counts and pixel counts are seldom powers of two.
+Model weights are random at the spread of the usual initialisers, adapters ~ N(0, 0.02), activations ~ N(0, 1).
+"""
+from __future__ import annotations
+
+import functools
+
+import torch
+
+BF = torch.bfloat16
+DEV = "cuda:0"
+CL = torch.channels_last
+
+# SDXL's linear layers with adapters: (in, out, GEGLU epilogue)
+LINEARS = ((640, 640, False), (1280, 1280, False), (2048, 640, False), (2048, 1280, False), (640, 5120, True),
+           (1280, 10240, True), (2560, 640, False), (5120, 1280, False))
+# SDXL's residual blocks: (in, out, resolution level)
+RESNETS = ((320, 320, 0), (640, 320, 0), (960, 320, 0), (320, 640, 1), (640, 640, 1), (960, 640, 1), (1280, 640, 1),
+           (1920, 640, 1), (640, 1280, 2), (1280, 1280, 2), (1920, 1280, 2), (2560, 1280, 2))
+RANKS = (8, 16, 32, 64, 128)
+
+
+def listed():
+    return [
+        # One adapter layer called on the 77 text tokens of a guidance pair (cross-attention to_k / to_v): the smallest call.
+        dict(name="linear_text_tokens", kind="linear", rows=154, layer=3, ranks="64,32", residual=False),
+        # The full-precision path: one LoRA-patched linear at the 64x64 level (BASELINE.json's first configuration).
+        dict(name="linear_fp32", kind="linear_fp32", rows=8192, layer=0, rank=32),
+        # Self-attention of the 64x64 level for an 832 x 1216 image: 52 * 76 = 3952 tokens, no multiple of any tile.
+        dict(name="attention_832x1216", kind="attention", batch=2, heads=10, tokens=3952, keys=3952),
+        # One transformer block at the 32x32 level with a rank-64 adapter on its linears (the second configuration).
+        dict(name="block_32x32", kind="block", batch=2, width=1280, height=32, row=32, ranks="64"),
+        # A residual block of the up path (concatenated input, 1x1 shortcut, time embedding) for an 832 x 1216 image.
+        dict(name="resnet_832x1216", kind="resnet", batch=2, block=7, height=104, row=152),
+        # Requests with different adapters and image sizes in one batch: shrink + expand per request (the fourth configuration).
+        dict(name="requests_mixed", kind="requests", layer=1, tokens="1024,988,1024,256,1024,576,988,1024",
+             ranks="64,8,128,32,16,64,128,32"),
+        # Katz's hand-over: an adapter that a loader left in host memory as float16 is merged into the weights it targets.
+        dict(name="merge_from_host", kind="merge", width=1280, depth=5, rank=64),
+        # The captured UNet step at 1024 x 1024 with two adapters and one ControlNet's residuals (the third configuration).
+        dict(name="step_1024x1024", kind="step", batch=2, height=128, row=128, ranks="64,32", controlnet=True),
+        # The captured UNet step of one guidance-free 832 x 1216 image with one small adapter.
+        dict(name="step_832x1216_single", kind="step", batch=1, height=104, row=152, ranks="16", controlnet=False),
+        # The plain module call in the guided Euler loop (two steps) of a 512 x 512 image, as an unprepared program runs it.
+        dict(name="eager_512x512", kind="eager", height=64, row=64, ranks="32", steps=2),
+        # A server between two requests: other adapters are activated and the first step with them runs, twice.
+        dict(name="switch_768x768", kind="switch", height=96, row=96, ranks="64,32", other="16", host=False),
+        # The captured loop: ControlNet, UNet with two adapters, guidance and Euler update (the fifth configuration, 2 of its steps).
+        dict(name="loop_1024x1024", kind="loop", height=128, row=128, ranks="64,32", steps=2),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(lo * (hi / lo) ** rng.random()))
+
+
+def _rank_text(rng, none=False):
+    """None, one or two active adapters, as far as one launch packs them (128 columns)."""
+    n = rng.choice((0, 1, 2) if none else (1, 2))
+    r = [rng.choice(RANKS[:4] if n == 2 else RANKS) for _ in range(n)]
+    return ",".join(map(str, r))
+
+
+def _image(rng, lo, hi):
+    """Height and row length in latent pixels, multiples of 4 (the UNet halves them twice)."""
+    return 4 * rng.randint(lo // 4, hi // 4), 4 * rng.randint(lo // 4, hi // 4)
+
+
+def draw(rng):
+    kind = rng.choice(("linear", "linear_fp32", "attention", "block", "resnet", "requests", "merge", "step", "eager", "switch",
+                       "loop"))
+    if kind == "linear":
+        return dict(kind=kind, rows=_log_int(rng, 1, 16384), layer=rng.randrange(len(LINEARS)), ranks=_rank_text(rng, none=True),
+                    residual=rng.random() < 0.5)
+    if kind == "linear_fp32":
+        return dict(kind=kind, rows=_log_int(rng, 64, 16384), layer=rng.choice((0, 1, 2, 3, 6, 7)), rank=rng.choice(RANKS))
+    if kind == "attention":
+        heads, down = rng.choice(((10, 2), (20, 4)))
+        h, w = _image(rng, 64, 152)
+        t = (h // down) * (w // down)
+        return dict(kind=kind, batch=rng.randint(1, 4), heads=heads, tokens=t, keys=rng.choice((t, t, 77, 154)))
+    if kind == "block":
+        width, down = rng.choice(((640, 2), (1280, 4)))
+        h, w = _image(rng, 64, 152)
+        return dict(kind=kind, batch=rng.randint(1, 4), width=width, height=h // down, row=w // down, ranks=_rank_text(rng, none=True))
+    if kind == "resnet":
+        h, w = _image(rng, 64, 152)
+        return dict(kind=kind, batch=rng.randint(1, 4), block=rng.randrange(len(RESNETS)), height=h, row=w)
+    if kind == "requests":
+        n = rng.randint(2, 16)
+        layer, down = rng.choice(((0, 2), (1, 4)))
+        toks = [(rng.randint(16, 32) * 4 // down) * (rng.randint(16, 32) * 4 // down) for _ in range(n)]
+        return dict(kind=kind, layer=layer, tokens=",".join(map(str, toks)), ranks=",".join(str(rng.choice(RANKS)) for _ in range(n)))
+    if kind == "merge":
+        return dict(kind=kind, width=rng.choice((640, 1280)), depth=rng.randint(1, 6), rank=rng.choice(RANKS))
+    if kind == "step":
+        h, w = _image(rng, 64, 128)
+        return dict(kind=kind, batch=rng.randint(1, 2), height=h, row=w, ranks=_rank_text(rng, none=True), controlnet=rng.random() < 0.5)
+    if kind == "eager":
+        h, w = _image(rng, 64, 128)
+        return dict(kind=kind, height=h, row=w, ranks=_rank_text(rng, none=True), steps=rng.randint(1, 2))
+    if kind == "switch":
+        h, w = _image(rng, 64, 128)
+        return dict(kind=kind, height=h, row=w, ranks=_rank_text(rng), other=_rank_text(rng), host=rng.random() < 0.5)
+    h, w = _image(rng, 64, 128)
+    return dict(kind=kind, height=h, row=w, ranks=_rank_text(rng, none=True), steps=rng.randint(1, 2))
+
+
+# ---- inputs ---------------------------------------------------------------------------------------------------------
+class _Source:
+    """Normal numbers from a seed; large tensors are cut from one pool at an offset of their own."""
+
+    def __init__(self, seed):
+        self.g = torch.Generator(device=DEV).manual_seed(seed)
+        self.pool = None
+        self.at = 0
+
+    def normal(self, *shape, std=1.0, dtype=BF):
+        return (torch.randn(*shape, generator=self.g, device=DEV) * std).to(dtype)
+
+    def image(self, *shape, std=1.0):
+        return self.normal(*shape, std=std).contiguous(memory_format=CL)
+
+    def fill(self, t, std, mean=0.0):
+        if self.pool is None:
+            self.pool = torch.randn(1 << 25, generator=self.g, device=DEV).to(BF)
+        n = t.numel()
+        self.at = (self.at + 7919 * 4099) % (self.pool.numel() - n)
+        t.view(-1).copy_(self.pool[self.at:self.at + n]).mul_(std)
+        if mean:
+            t.add_(mean)
+
+
+def _materialise(make, src):
+    """A module of the package with random weights in the kernels' format, built without torch's initialisers."""
+    import katz_amd.layers as layers
+
+    layers.SKIP_INIT = True
+    try:
+        with torch.device("meta"):
+            m = make()
+    finally:
+        layers.SKIP_INIT = False
+    m = m.to(BF).to_empty(device=DEV)
+    with torch.no_grad():
+        for name, p in m.named_parameters():
+            if p.dim() > 1:
+                src.fill(p.data, (3.0 * p[0].numel()) ** -0.5)
+            elif name.endswith("weight"):
+                src.fill(p.data, 0.1, 1.0)
+            else:
+                src.fill(p.data, 0.02)
+    return m.to(memory_format=CL).eval()
+
+
+def _ranks(text):
+    return [int(r) for r in text.split(",") if r]
+
+
+def _linears(m):
+    from katz_amd.layers import LoRALinear
+
+    return {n: l for n, l in m.named_modules() if isinstance(l, LoRALinear)}
+
+
+def _adapters(src, m, ranks, prefix, host=False):
+    """Random adapters of these ranks on every linear of the module (float16 in host memory, as a loader leaves them, or
+    bfloat16 on the GPU)."""
+    names = []
+    for i, r in enumerate(ranks):
+        name = f"{prefix}{i}"
+        for l in _linears(m).values():
+            down, up = torch.empty(r, l.in_features, dtype=BF, device=DEV), torch.empty(l.out_features, r, dtype=BF, device=DEV)
+            src.fill(down, 0.02)
+            src.fill(up, 0.02)
+            if host:
+                down, up = down.to(torch.float16).cpu(), up.to(torch.float16).cpu()
+            l.add_adapter(name, down, up)
+        names.append(name)
+    return names
+
+
+WEIGHTS = (0.8, 0.6)   # of the first and the second active adapter
+
+
+def _unet(src, case, host=False):
+    from katz_amd.unet_2d_condition import UNet2DConditionModel, UNetConfig
+
+    unet = _materialise(lambda: UNet2DConditionModel(UNetConfig.sdxl()), src)
+    names = _adapters(src, unet, _ranks(case["ranks"]), "a", host)
+    unet.to_runtime(DEV, BF)
+    return unet, names
+
+
+def _conditions(src, b, case):
+    size = [8.0 * case["height"], 8.0 * case["row"], 0.0, 0.0, 8.0 * case["height"], 8.0 * case["row"]]
+    return (src.normal(b, 77, 2048), dict(text_embeds=src.normal(b, 1280), time_ids=torch.tensor([size] * b, device=DEV)))
+
+
+def _residuals(src, b, h, w):
+    shapes = [(320, 1)] * 3 + [(320, 2), (640, 2), (640, 2), (640, 4), (1280, 4), (1280, 4)]
+    return ([src.image(b, c, h // d, w // d, std=0.1) for c, d in shapes], src.image(b, 1280, h // 4, w // 4, std=0.1))
+
+
+def prepare(case, seed):
+    src, kind = _Source(seed), case["kind"]
+    with torch.no_grad():
+        state = globals()["_prepare_" + kind](case, src)
+    state["kind"] = kind
+    return state
+
+
+def _prepare_linear(case, src):
+    from katz_amd.layers import LoRALinear
+
+    k, n, geglu = LINEARS[case["layer"]]
+    layer = _materialise(lambda: LoRALinear(k, n, bias=k != 2048, geglu=geglu), src)
+    layer.set_active(_adapters(src, layer, _ranks(case["ranks"]), "a"), WEIGHTS)
+    layer.prepare()
+    residual = case["residual"] and not geglu
+    return dict(layer=layer, x=src.normal(case["rows"], k), residual=src.normal(case["rows"], n) if residual else None)
+
+
+def _prepare_linear_fp32(case, src):
+    k, n, _ = LINEARS[case["layer"]]
+    f32 = torch.float32
+    r = -(-case["rank"] // 32) * 32
+    a, b = torch.zeros(r, k, device=DEV), torch.zeros(n, r, device=DEV)
+    a[:case["rank"]] = src.normal(case["rank"], k, std=0.02, dtype=f32)
+    b[:, :case["rank"]] = src.normal(n, case["rank"], std=0.02, dtype=f32)
+    return dict(x=src.normal(case["rows"], k, dtype=f32), w=src.normal(n, k, std=0.02, dtype=f32), bias=src.normal(n, std=0.02, dtype=f32),
+                a=a, b=b, scale=torch.full((r,), 0.8, device=DEV))
+
+
+def _prepare_attention(case, src):
+    # q, k and v of a self-attention are column slices of one projection, those of a cross-attention three tensors
+    b, t, s, c = case["batch"], case["tokens"], case["keys"], case["heads"] * 64
+    if s == t:
+        q, k, v = src.normal(b, t, 3 * c).split(c, dim=-1)
+    else:
+        q, k, v = src.normal(b, t, c), src.normal(b, s, c), src.normal(b, s, c)
+    return dict(q=q, k=k, v=v, heads=case["heads"])
+
+
+def _prepare_block(case, src):
+    from katz_amd.layers import BasicTransformerBlock
+
+    width = case["width"]
+    blk = _materialise(lambda: BasicTransformerBlock(width, width // 64, 64, 2048), src)
+    names = _adapters(src, blk, _ranks(case["ranks"]), "a")
+    for l in _linears(blk).values():
+        l.set_active(names, WEIGHTS)
+    return dict(block=blk, h=src.normal(case["batch"], case["height"] * case["row"], width), ctx=src.normal(case["batch"], 77, 2048))
+
+
+def _prepare_resnet(case, src):
+    from katz_amd.layers import ResnetBlock2D
+
+    cin, cout, level = RESNETS[case["block"]]
+    res = _materialise(lambda: ResnetBlock2D(in_channels=cin, out_channels=cout, temb_channels=1280, eps=1e-5), src)
+    b = case["batch"]
+    return dict(block=res, x=src.image(b, cin, case["height"] >> level, case["row"] >> level), temb=src.normal(b, 1280))
+
+
+def _prepare_requests(case, src):
+    k, n, _ = LINEARS[case["layer"]]
+    tokens, ranks = [int(t) for t in case["tokens"].split(",")], _ranks(case["ranks"])
+    rp = 128 if max(ranks) > 64 else 64 if max(ranks) > 32 else 32
+    a, b = torch.zeros(len(ranks), rp, k, dtype=BF, device=DEV), torch.zeros(len(ranks), n, rp, dtype=BF, device=DEV)
+    for i, r in enumerate(ranks):
+        a[i, :r] = src.normal(r, k, std=0.02)
+        b[i, :, :r] = src.normal(n, r, std=0.02)
+    start = [0]
+    for t in tokens:
+        start.append(start[-1] + t)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    return dict(x=src.normal(start[-1], k), y=src.normal(start[-1], n), a=a, b=b, start=torch.tensor(start, **i32),
+                adapter=torch.arange(len(ranks), **i32), rank=torch.tensor([-(-r // 32) * 32 for r in ranks], **i32),
+                scale=torch.full((len(ranks),), 0.7, device=DEV), longest=max(tokens))
+
+
+def _prepare_merge(case, src):
+    from katz_amd.layers import Transformer2DModel
+
+    width, r = case["width"], case["rank"]
+    model = _materialise(lambda: Transformer2DModel(width // 64, 64, width, case["depth"], 2048), src)
+    adapter, match = {}, {}
+    for name, l in _linears(model).items():
+        adapter[name + ".down"] = src.normal(r, l.in_features, std=0.02, dtype=torch.float16).cpu()
+        adapter[name + ".up"] = src.normal(l.out_features, r, std=0.02, dtype=torch.float16).cpu()
+        match[name + ".weight"] = dict(lora_down_key=name + ".down", lora_up_key=name + ".up")
+    return dict(model=model, adapter=adapter, match=match)
+
+
+def _prepare_step(case, src):
+    from katz_amd.graph import GraphedUNetStep
+
+    b, h, w = case["batch"], case["height"], case["row"]
+    unet, names = _unet(src, case)
+    unet.set_adapters(names, list(WEIGHTS[:len(names)]))
+    ctx, added = _conditions(src, b, case)
+    sample, t = src.image(b, 4, h, w), torch.tensor([500.0], device=DEV)
+    down, mid = _residuals(src, b, h, w) if case["controlnet"] else (None, None)
+    return dict(step=GraphedUNetStep(unet, sample, t, ctx, added, down, mid), sample=sample, t=t, down=down, mid=mid)
+
+
+def _schedule(steps):
+    from katz_amd.scheduler import EulerDiscreteScheduler
+
+    sch = EulerDiscreteScheduler.sdxl()
+    sch.set_timesteps(steps, device=DEV)
+    return sch
+
+
+def _prepare_eager(case, src):
+    unet, names = _unet(src, case)
+    unet.set_adapters(names, list(WEIGHTS[:len(names)]))
+    ctx, added = _conditions(src, 2, case)
+    sch = _schedule(case["steps"])
+    latents = src.normal(1, 4, case["height"], case["row"]) * float(sch.init_noise_sigma)
+    return dict(model=lambda x, t: unet(x, t, ctx, added_cond_kwargs=added).sample, scheduler=sch, latents=latents)
+
+
+def _prepare_switch(case, src):
+    unet, first = _unet(src, case, case["host"])
+    second = _adapters(src, unet, _ranks(case["other"]), "b", case["host"])
+    ctx, added = _conditions(src, 2, case)
+    return dict(unet=unet, sets=(first, second), sample=src.image(2, 4, case["height"], case["row"]), t=torch.tensor([500.0], device=DEV),
+                ctx=ctx, added=added)
+
+
+def _prepare_loop(case, src):
+    from katz_amd.controlnet import ControlNetModel
+    from katz_amd.graph import GraphedDenoiseStep
+    from katz_amd.unet_2d_condition import UNetConfig
+
+    h, w = case["height"], case["row"]
+    unet, names = _unet(src, case)
+    unet.set_adapters(names, list(WEIGHTS[:len(names)]))
+    net = _materialise(lambda: ControlNetModel(UNetConfig.sdxl()), src).to_runtime(DEV, BF)
+    ctx, added = _conditions(src, 2, case)
+    sch = _schedule(case["steps"])
+    latents = src.normal(1, 4, h, w) * float(sch.init_noise_sigma)
+    cond = torch.rand(2, 3, 8 * h, 8 * w, generator=src.g, device=DEV).to(BF)
+    return dict(step=GraphedDenoiseStep(unet, net, latents, ctx, added, cond, 7.5, 0.5), latents=latents, scheduler=sch)
+
+
+# ---- one pass ------------------------------------------------------------------------------------------------------
+def run(s):
+    from katz_amd import ops
+
+    kind = s["kind"]
+    with torch.no_grad():
+        if kind == "linear":
+            return s["layer"](s["x"], residual=s["residual"])
+        if kind == "linear_fp32":
+            return ops.lora_linear(s["x"], s["w"], s["bias"], s["a"], s["b"], s["scale"])
+        if kind == "attention":
+            return ops.attention(s["q"], s["k"], s["v"], s["heads"])
+        if kind == "block":
+            return s["block"](s["h"], s["ctx"])
+        if kind == "resnet":
+            return s["block"](s["x"], s["temb"])
+        if kind == "requests":
+            return ops.sgmv_fused_(s["y"], s["x"], s["a"], s["b"], s["start"], s["adapter"], s["rank"], s["scale"], s["longest"])
+        if kind == "merge":
+            from katz_amd.shm_adapters import patch_on_lora
+
+            patch_on_lora(s["model"], s["adapter"], s["match"], scale=0.05)
+            return [l.weight for l in _linears(s["model"]).values()]
+        if kind == "step":
+            return s["step"](s["sample"], s["t"], down_block_additional_residuals=s["down"], mid_block_additional_residual=s["mid"])
+        if kind == "eager":
+            from katz_amd.scheduler import denoise_loop
+
+            return denoise_loop(s["model"], s["scheduler"], s["latents"], 7.5)
+        if kind == "switch":
+            out = []
+            for names in s["sets"]:
+                s["unet"].set_adapters(names, list(WEIGHTS[:len(names)]))
+                out.append(s["unet"](s["sample"], s["t"], s["ctx"], added_cond_kwargs=s["added"]).sample)
+            return out
+        return s["step"].run(s["latents"], s["scheduler"])
+
+
+# ---- what a pass cannot do without -----------------------------------------------------------------------------------
+@functools.lru_cache(maxsize=None)
+def _meta(kind):
+    from katz_amd.controlnet import ControlNetModel
+    from katz_amd.unet_2d_condition import UNet2DConditionModel, UNetConfig
+
+    with torch.device("meta"):
+        return (UNet2DConditionModel if kind == "unet" else ControlNetModel)(UNetConfig.sdxl())
+
+
+def _linear_flops(rows, k, n, r):
+    return 2.0 * rows * k * n + 2.0 * rows * r * (k + n)
+
+
+def _block_flops(b, t, c, r, ctx=77):
+    """A transformer block: q, k, v, out of both attentions, the attentions, the feed-forward."""
+    lin = 6 * _linear_flops(b * t, c, c, r) + 2 * _linear_flops(b * ctx, 2048, c, r)
+    return lin + 4.0 * b * t * (t + ctx) * c + _linear_flops(b * t, c, 8 * c, r) + _linear_flops(b * t, 4 * c, c, r)
+
+
+def _resnet_flops(b, px, cin, cout):
+    return 2.0 * b * px * (9 * cout * (cin + cout) + (cin * cout if cin != cout else 0)) + 2.0 * b * 1280 * cout
+
+
+def _model_flops(kind, b, h, w, r):
+    m = _meta(kind)
+    total = 2.0 * b * h * w * 9 * 2 * 4 * 320
+
+    def transformer(a, px):
+        c = a.proj_in.in_features
+        return 2 * _linear_flops(b * px, c, c, r) + len(a.transformer_blocks) * _block_flops(b, px, c, r)
+
+    def stage(blk, level, px):
+        f = sum(_resnet_flops(b, px, x.conv1.in_channels, x.conv1.out_channels) for x in blk.resnets)
+        f += sum(transformer(a, px) for a in getattr(blk, "attentions", ()))
+        for d in getattr(blk, "downsamplers", None) or ():
+            f += 2.0 * b * px / 4 * 9 * d.conv.in_channels * d.conv.out_channels
+        for u in getattr(blk, "upsamplers", None) or ():
+            f += 2.0 * b * px * 4 * 9 * u.conv.in_channels * u.conv.out_channels
+        return f
+
+    for i, blk in enumerate(m.down_blocks):
+        total += stage(blk, i, h * w / 4 ** i)
+    total += stage(m.mid_block, 2, h * w / 16)
+    for i, blk in enumerate(getattr(m, "up_blocks", ())):
+        total += stage(blk, 2 - i, h * w / 4 ** (2 - i))
+    for zc, px in zip(getattr(m, "controlnet_down_blocks", ()), [h * w] * 3 + [h * w / 4] * 3 + [h * w / 16] * 3):
+        total += 2.0 * b * px * zc.in_channels * zc.out_channels
+    return total
+
+
+def _model_bytes(kind, r):
+    m = _meta(kind)
+    return 2.0 * sum(p.numel() for p in m.parameters()) + 2.0 * r * sum(l.in_features + l.out_features for l in _linears(m).values())
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("step", "eager", "switch", "loop"):
+        h, w, r = case["height"], case["row"], sum(_ranks(case["ranks"]))
+        b = case.get("batch", 2)
+        io = 2.0 * b * (2 * 4 * h * w + 77 * 2048 + 1280)
+        if kind == "step":
+            per_row = h * w * (3 * 320 + (320 + 2 * 640) / 4 + (640 + 3 * 1280) / 16)
+            return dict(bytes=_model_bytes("unet", r) + io + (2.0 * b * per_row if case["controlnet"] else 0), flops=_model_flops("unet", b, h, w, r))
+        if kind == "eager":
+            return dict(bytes=case["steps"] * (_model_bytes("unet", r) + io), flops=case["steps"] * _model_flops("unet", b, h, w, r))
+        if kind == "switch":
+            r2 = sum(_ranks(case["other"]))
+            return dict(bytes=_model_bytes("unet", r) + _model_bytes("unet", r2) + 2 * io,
+                        flops=_model_flops("unet", b, h, w, r) + _model_flops("unet", b, h, w, r2))
+        return dict(bytes=case["steps"] * (_model_bytes("unet", r) + _model_bytes("controlnet", 0) + io) + 2.0 * 2 * 3 * 64 * h * w,
+                    flops=case["steps"] * (_model_flops("unet", b, h, w, r) + _model_flops("controlnet", b, h, w, 0)))
+    if kind in ("linear", "linear_fp32"):
+        m, (k, n, geglu) = case["rows"], LINEARS[case["layer"]]
+        r = case["rank"] if kind == "linear_fp32" else sum(_ranks(case["ranks"]))
+        out = m * n / 2 if geglu and kind == "linear" else m * n * (2 if case.get("residual") and not geglu else 1)
+        return dict(bytes=(4.0 if kind == "linear_fp32" else 2.0) * (m * k + k * n + out + r * (k + n)), flops=_linear_flops(m, k, n, r))
+    if kind == "attention":
+        b, t, s, c = case["batch"], case["tokens"], case["keys"], 64 * case["heads"]
+        return dict(bytes=2.0 * b * c * (2 * t + 2 * s), flops=4.0 * b * t * s * c)
+    if kind == "block":
+        b, t, c, r = case["batch"], case["height"] * case["row"], case["width"], sum(_ranks(case["ranks"]))
+        weights = 18 * c * c + 2 * 2048 * c + r * (27 * c + 2 * 2048)
+        return dict(bytes=2.0 * (2 * b * t * c + b * 77 * 2048 + weights), flops=_block_flops(b, t, c, r))
+    if kind == "resnet":
+        cin, cout, level = RESNETS[case["block"]]
+        b, px = case["batch"], (case["height"] >> level) * (case["row"] >> level)
+        return dict(bytes=2.0 * (b * px * (cin + cout) + 9 * cout * (cin + cout) + (cin * cout if cin != cout else 0) + 1280 * cout),
+                    flops=_resnet_flops(b, px, cin, cout))
+    if kind == "requests":
+        k, n, _ = LINEARS[case["layer"]]
+        pairs = list(zip((int(t) for t in case["tokens"].split(",")), _ranks(case["ranks"])))
+        rows = sum(t for t, _ in pairs)
+        return dict(bytes=2.0 * (rows * (k + 2 * n) + sum(r for _, r in pairs) * (k + n)), flops=sum(2.0 * t * r * (k + n) for t, r in pairs))
+    c, d, r = case["width"], case["depth"], case["rank"]
+    weights, ends = 2 * c * c + d * (18 * c * c + 2 * 2048 * c), 4 * c + d * (27 * c + 2 * 2048)
+    return dict(bytes=2.0 * (2 * weights + r * ends), flops=2.0 * r * weights)
+
+
+def tolerance(case):
+    kind = case["kind"]
+    if kind == "linear_fp32":
+        return dict(rel=1e-5)
+    if kind == "merge":
+        return dict(rel=4e-3)       # one rounding of the sum to bf16
+    if kind in ("step", "eager", "switch", "loop"):
+        return dict(rel=2e-2)       # some 700 layers, each rounding its result to bf16
+    return dict(rel=1e-2)
