@@ -208,6 +208,12 @@ int kh_lora_merge_grouped_bf16(const uint64_t* table, const int32_t* tile_start,
 int kh_lora_linear_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,
                        const float* col_scale, const float* residual, float* y, int64_t M, int64_t N, int64_t K,
                        int64_t R, void* stream);
+/* The same formula on the fp32 matrix instruction, in two launches: t_scratch [M,R] fp32 (written; may be NULL when R == 0)
+ * receives (x A_cat^T) * col_scale, then the base GEMM takes the rank columns as extra K steps.  K % 4 == 0, R % 4 == 0
+ * and 16-byte aligned pointers, else KH_ERR_UNSUPPORTED / KH_ERR_ALIGNMENT (then: kh_lora_linear_f32). */
+int kh_lora_linear_split_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,
+                             const float* col_scale, float* t_scratch, const float* residual, float* y, int64_t M,
+                             int64_t N, int64_t K, int64_t R, void* stream);
 
 /* ---- K2: segmented multi-adapter shrink / expand ----------------------------------------------
  * Per-request adapters in one batch: segment s = rows [seg_start[s], seg_start[s+1]) uses adapter

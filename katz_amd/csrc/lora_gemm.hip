@@ -331,7 +331,8 @@ int launch_rank(const LoraGemmParams& p, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32 variant (debug / fp32 parity path): plain FMA tiles, same fusion (T kept in LDS).
+// fp32 variant for sizes or pointers that 16-byte pieces do not fill (K or R % 4 != 0; lora_gemm_f32.hip has the fast one):
+// plain FMA tiles, T kept in LDS.
 // ---------------------------------------------------------------------------------------------
 constexpr int F_BM = 64, F_BN = 64, F_BK = 16, F_RMAX = 128;
 

@@ -173,8 +173,12 @@ def lora_linear(
     elif dt == torch.float32:
         if geglu:
             raise ValueError("the GEGLU epilogue exists for bf16 only")
-        rc = lib.kh_lora_linear_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale),
-                                    _ptr(residual), _ptr(out), M, N, K, R, _stream())
+        t = torch.empty((M, R), dtype=dt, device=x.device) if R else None
+        rc = lib.kh_lora_linear_split_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale), _ptr(t),
+                                          _ptr(residual), _ptr(out), M, N, K, R, _stream())
+        if rc in (-2, -3):   # KH_ERR_UNSUPPORTED / KH_ERR_ALIGNMENT: rows that 16-byte pieces do not fill take the scalar kernel
+            rc = lib.kh_lora_linear_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale),
+                                        _ptr(residual), _ptr(out), M, N, K, R, _stream())
     else:
         raise TypeError(f"lora_linear supports bfloat16 and float32, got {dt}")
     _lib.check(rc, "kh_lora_linear")
