@@ -204,6 +204,13 @@ int kh_lora_linear_grouped_bf16(const void* x, const uint64_t* table, int64_t n_
 int kh_lora_merge_grouped_bf16(const uint64_t* table, const int32_t* tile_start, const float* layer_scale,
                                int64_t n_layers, int64_t total_tiles, int64_t max_rank, float scale, int operands_fp16,
                                void* stream);
+/* n HOST arrays to offset[i] of the DEVICE buffer dst (offsets ascending, arrays disjoint), gathered by worker threads
+ * into two halves of `staging` (PINNED host memory, at least 8 KiB, the caller's again on return) while the other half is
+ * copied on `stream`.  src / bytes / offset: HOST arrays.  Returns when the host memory has been read and copied; work
+ * enqueued on `stream` afterwards sees the data.  Not under graph capture.  What a loader process left in shared memory
+ * (load_lora_shm_multi.py:40-61) is uploaded with one call. */
+int kh_upload_many(const void* const* src, const int64_t* bytes, const int64_t* offset, int64_t n, void* dst, void* staging,
+                   int64_t staging_bytes, void* stream);
 /* fp32 variant of the same formula (fp32 parity path); R <= 128, any M/N/K. */
 int kh_lora_linear_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,
                        const float* col_scale, const float* residual, float* y, int64_t M, int64_t N, int64_t K,

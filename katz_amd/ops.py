@@ -14,6 +14,7 @@ import os
 import weakref
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -547,6 +548,26 @@ def lora_linear_xattn(x: torch.Tensor, weight: torch.Tensor, k: torch.Tensor, v:
     return out
 
 
+def upload_many(tensors: Sequence[torch.Tensor], device):
+    """CPU tensors to `device` in one call (kh_upload_many): returns (the device buffer, a device address per tensor).  The
+    caller keeps the buffer until the work that reads it has been enqueued on the current stream."""
+    src = [t if t.is_contiguous() else t.contiguous() for t in tensors]
+    n = len(src)
+    nbytes = np.fromiter((t.numel() * t.element_size() for t in src), np.int64, n)
+    offset = np.zeros(n, np.int64)
+    np.cumsum((nbytes[:-1] + 255) // 256 * 256, out=offset[1:])
+    ptrs = np.fromiter((t.data_ptr() for t in src), np.uint64, n)
+    total = int(offset[-1] + nbytes[-1])
+    # two staging halves of 1 .. 8 MB: several chunks per upload, so that gathering and copying overlap
+    staging = torch.empty(2 * min(8 << 20, max(1 << 20, total // 6)), dtype=torch.uint8, pin_memory=True)
+    with torch.cuda.device(device):
+        dst = torch.empty((total,), dtype=torch.uint8, device=device)
+        rc = _lib.load().kh_upload_many(ptrs.ctypes.data, nbytes.ctypes.data, offset.ctypes.data, n, _ptr(dst), _ptr(staging), staging.numel(), _stream())
+    _lib.check(rc, "kh_upload_many")
+    base = dst.data_ptr()
+    return dst, [base + o for o in offset.tolist()]
+
+
 def lora_merge_grouped(weights: Sequence[torch.Tensor], ups: Sequence[torch.Tensor], downs: Sequence[torch.Tensor],
                        scale: float = 1.0, layer_scales: Optional[Sequence[float]] = None) -> None:
     """W_l += scale * layer_scales[l] * up_l @ down_l for all layers in ONE launch, in place (kh_lora_merge_grouped_bf16).
@@ -580,14 +601,20 @@ def lora_merge_grouped(weights: Sequence[torch.Tensor], ups: Sequence[torch.Tens
         rows.append((w.data_ptr(), u.data_ptr(), d.data_ptr(), N, K, r))
         starts.append(starts[-1] + ((N + 127) // 128) * ((K + 127) // 128))
         max_rank = max(max_rank, r)
-    table = torch.tensor(rows, dtype=torch.int64).to(dev, non_blocking=True)
-    tile_start = torch.tensor(starts, dtype=torch.int32).to(dev, non_blocking=True)
-    ls = None if layer_scales is None else torch.tensor(list(layer_scales), dtype=torch.float32).to(dev, non_blocking=True)
-    rc = lib.kh_lora_merge_grouped_bf16(_ptr(table), _ptr(tile_start), _ptr(ls), n, starts[-1], max_rank, float(scale),
-                                        1 if op_dtype == torch.float16 else 0, _stream())
-    _lib.check(rc, "kh_lora_merge_grouped_bf16")
+    lora_merge_rows(rows, starts, max_rank, op_dtype, dev, scale, layer_scales)
     for w in weights:
         torch.autograd.graph.increment_version(w)
+
+
+def lora_merge_rows(rows, starts, max_rank: int, op_dtype, dev, scale: float = 1.0, layer_scales=None) -> None:
+    """kh_lora_merge_grouped_bf16 on rows {W, up, down, N, K, r} that the caller has checked (lora_merge_grouped)."""
+    lib = _lib.load()
+    table = torch.from_numpy(np.array(rows, dtype=np.int64)).to(dev, non_blocking=True)
+    tile_start = torch.from_numpy(np.array(starts, dtype=np.int32)).to(dev, non_blocking=True)
+    ls = None if layer_scales is None else torch.tensor(list(layer_scales), dtype=torch.float32).to(dev, non_blocking=True)
+    rc = lib.kh_lora_merge_grouped_bf16(_ptr(table), _ptr(tile_start), _ptr(ls), len(rows), starts[-1], max_rank, float(scale),
+                                        1 if op_dtype == torch.float16 else 0, _stream())
+    _lib.check(rc, "kh_lora_merge_grouped_bf16")
     # the table tensors are freed when this returns: torch's caching allocator keeps the memory valid for work already
     # enqueued on the current stream, which is where the kernel runs
 

@@ -114,7 +114,7 @@ def patch_on_lora(unet, lora_state_dict: Mapping[str, torch.Tensor], key_match: 
     accumulation, W + scale * product rounded once (the reference rounds up @ down and the scaled product to fp16
     first, and writes the result back with load_state_dict).  Returns the number of patched weights."""
     params = dict(unet.named_parameters())
-    ws, ups, downs = [], [], []
+    rows, starts, ws, mats, max_rank, op_dtype, seen = [], [0], [], [], 0, None, set()
     for wkey, m in key_match.items():
         if wkey not in params:
             raise KeyError(f"{wkey} is not a parameter of the UNet")
@@ -128,11 +128,32 @@ def patch_on_lora(unet, lora_state_dict: Mapping[str, torch.Tensor], key_match: 
             raise ValueError(f"{wkey}: adapter shapes {tuple(up.shape)} x {tuple(down.shape)} do not match {tuple(w.shape)}")
         if down.dtype not in (torch.float16, torch.bfloat16):
             down, up = down.to(torch.bfloat16), up.to(torch.bfloat16)
-        ws.append(w.data)
-        downs.append(down.to(w.device, non_blocking=True).contiguous())
-        ups.append(up.to(w.device, non_blocking=True).contiguous())
-    with torch.no_grad():
-        ops.lora_merge_grouped(ws, ups, downs, scale=scale)
-    for wkey in key_match:
-        torch.autograd.graph.increment_version(params[wkey])   # `.data` above is a separate version counter
+        if ws and w.device != ws[0].device:
+            raise ValueError(f"{wkey}: every weight must live on one GPU")
+        if up.dtype != down.dtype or (op_dtype is not None and down.dtype != op_dtype):
+            raise ValueError(f"{wkey}: the adapter's matrices must have one dtype")
+        if r < 1 or r > 128:
+            raise ValueError(f"rank {r} outside 1..128")
+        if w.data_ptr() in seen:
+            raise ValueError("a weight appears twice in one merge (the tiles of the two rows would race)")
+        seen.add(w.data_ptr())
+        op_dtype = down.dtype
+        ws.append(w)
+        mats += [up, down]
+        rows.append([w.data_ptr(), 0, 0, n_out, n_in, r])
+        starts.append(starts[-1] + ((n_out + 127) // 128) * ((n_in + 127) // 128))
+        max_rank = max(max_rank, r)
+    if not ws:
+        return 0
+    dev = ws[0].device
+    mats = [t if not t.is_cuda else t.to(dev).contiguous() for t in mats]
+    host = [t for t in mats if not t.is_cuda]
+    keep, at = ops.upload_many(host, dev) if host else (None, [])
+    at = iter(at)
+    for i, t in enumerate(mats):
+        rows[i // 2][1 + i % 2] = t.data_ptr() if t.is_cuda else next(at)
+    ops.lora_merge_rows(rows, starts, max_rank, op_dtype, dev, scale)
+    del keep, mats    # stream-ordered: the launch above is enqueued
+    for w in ws:
+        torch.autograd.graph.increment_version(w)
     return len(ws)

@@ -33,3 +33,18 @@ def test_lora_linear_f32_matrix_kernel(M, N, K, R):
     torch.cuda.synchronize()
     ref = O.lora_linear(x.double(), w.double(), b.double(), [(A.double(), Bm.double(), 1.5)] if R else [], res.double()).float()
     assert_close_rel(y, ref, 1e-5, "fp32 linear")
+
+
+def test_upload_many_sizes():
+    """kh_upload_many: arrays smaller and larger than a staging half, empty gaps, one array, bit for bit."""
+    from katz_amd import ops
+
+    say("upload many")
+    g = torch.Generator().manual_seed(1)
+    for sizes in ([1], [3, 5, 1 << 20, 7], [(9 << 20) + 13, 1, (3 << 20) + 1], [257] * 300):
+        src = [torch.randint(0, 256, (n,), generator=g, dtype=torch.uint8) for n in sizes]
+        buf, at = ops.upload_many(src, dev())
+        torch.cuda.synchronize()
+        for t, a in zip(src, at):
+            o = a - buf.data_ptr()
+            assert torch.equal(buf[o:o + t.numel()].cpu(), t), sizes
