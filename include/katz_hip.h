@@ -204,6 +204,20 @@ int kh_lora_linear_grouped_bf16(const void* x, const uint64_t* table, int64_t n_
 int kh_lora_merge_grouped_bf16(const uint64_t* table, const int32_t* tile_start, const float* layer_scale,
                                int64_t n_layers, int64_t total_tiles, int64_t max_rank, float scale, int operands_fp16,
                                void* stream);
+/* The packed adapter buffers of many layers (A_cat, B_cat, col_scale of kh_lora_linear_bf16; behind a folded LayerNorm also
+ * A_cat * gamma and its row terms, see kh_lora_linear_norm_bf16) from the adapters' own matrices: set_adapters of
+ * diffusers-hf/src/diffusers/loaders/unet.py:565-618 for a whole model in two launches.  layers: DEVICE table, per layer
+ * fourteen 64-bit words {a_cat, a_norm or 0, gamma, beta, ca1, ca2, b_cat, col_scale (addresses; a_cat / a_norm / gamma / beta /
+ * b_cat bf16, the others float), K, N, R, geglu, first piece, pieces}; geglu != 0: B_cat rows in the interleaved order.
+ * pieces: DEVICE table, per adapter of a layer six words {down [rank,K], up [N,rank] (addresses), rank, first packed column,
+ * dtype (0 bf16, 1 fp16, 2 fp32), multiplier (fp32 bits)}.  Columns no piece covers are zero.  K % 8 == 0, R % 8 == 0,
+ * R <= 2048, every matrix 16-byte aligned.  a_start: DEVICE int32 [n_layers + 1], sums of R; b_start likewise, sums of
+ * ceil(N / (256 / (R / 8))); a_rows, b_blocks: their last entries. */
+int kh_lora_pack_bf16(const void* layers, const void* pieces, const int32_t* a_start, const int32_t* b_start,
+                      int64_t n_layers, int64_t a_rows, int64_t b_blocks, void* stream);
+/* col_scale of many layers (scale_lora_layers, diffusers-hf/src/diffusers/utils/peft_utils.py:103-123): DEVICE table of n rows
+ * {float* array, first element, elements, value (fp32 bits)} of 64-bit words. */
+int kh_lora_rescale(const int64_t* table, int64_t n, void* stream);
 /* n HOST arrays to offset[i] of the DEVICE buffer dst (offsets ascending, arrays disjoint), gathered by worker threads
  * into two halves of `staging` (PINNED host memory, at least 8 KiB, the caller's again on return) while the other half is
  * copied on `stream`.  src / bytes / offset: HOST arrays.  Returns when the host memory has been read and copied; work

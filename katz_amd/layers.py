@@ -19,8 +19,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from .lora import (MAX_PACKED_RANK, Adapter, PackedAdapters, fold_layer_norm, interleave_geglu_rows, pack_adapters,
-                   rescale_)
+from .lora import (MAX_PACKED_RANK, Adapter, PackedAdapters, fold_norm_into_adapters, fold_norm_into_weight, interleave_geglu_rows,
+                   norm_key, pack_adapters, pack_many, pack_many_takes, rescale_, rescale_many, stacked)
 
 CL = torch.channels_last
 
@@ -89,8 +89,10 @@ class LoRALinear(nn.Module):
         self.adapters_enabled = True
         self._packed: Optional[PackedAdapters] = None
         self._packed_key = None
+        self._fold_norm = ()     # (LayerNorm,) in front of this layer, set by the transformer block (a tuple: not a submodule)
+        self._context = 0        # output width, for the to_k / to_v of a cross-attention: grouped launches run them together
         self._rt = None          # (weight version, weight ptr, runtime weight, runtime bias)
-        self._ln_rt = None       # (key, folded operands) for the LayerNorm in front of this layer
+        self._ln_w = None        # (key, W', c1, c2): the weights with the LayerNorm in front of this layer folded in
         self._fused: Dict[str, float] = {}   # adapter name -> multiplier merged into weight
         self.reset_parameters()
 
@@ -116,13 +118,21 @@ class LoRALinear(nn.Module):
         self.active = [n for n in self.active if n != name]
         self._packed_key = None
 
-    def set_active(self, names: Sequence[str], weights: Optional[Sequence[float]] = None) -> None:
-        self.active = [n for n in names if n in self.adapters]
+    def assign_active(self, names: Sequence[str], weights: Optional[Sequence[float]] = None) -> None:
+        """set_active without the rebuild: refresh_many does that for many layers at once."""
+        ads = self.adapters
+        self.active = [n for n in names if n in ads]
         if weights is not None:
             for n, w in zip(names, weights):
-                if n in self.adapters:
-                    self.adapters[n].weight = float(w)
+                if n in ads:
+                    ads[n].weight = float(w)
+
+    def set_active(self, names: Sequence[str], weights: Optional[Sequence[float]] = None) -> None:
+        self.assign_active(names, weights)
         self.refresh_adapters()
+
+    def fold_norm(self):
+        return self._fold_norm[0] if self._fold_norm and LN_FOLD else None
 
     def set_global_scale(self, scale: float) -> None:
         """cross_attention_kwargs["scale"]: scale_lora_layers, diffusers-hf/src/diffusers/utils/peft_utils.py:103-123."""
@@ -130,12 +140,16 @@ class LoRALinear(nn.Module):
             self.global_scale = float(scale)
             self.refresh_adapters()
 
+    def wanted_pack(self):
+        """(adapter names to pack, key of that pack)."""
+        names = [n for n in self.active if n not in self._fused] if self.adapters_enabled else []
+        return names, tuple((n, id(self.adapters[n].down)) for n in names)
+
     def refresh_adapters(self) -> None:
         """(Re)build the packed buffers; a pure scale change only rewrites col_scale in place, so a
         captured HIP graph that reads the buffers stays valid."""
         global _pack_epoch
-        names = [n for n in self.active if n not in self._fused] if self.adapters_enabled else []
-        key = tuple((n, id(self.adapters[n].down)) for n in names)
+        names, key = self.wanted_pack()
         if not names:
             if self._packed is not None:
                 _pack_epoch += 1
@@ -224,13 +238,16 @@ class LoRALinear(nn.Module):
     def _ln_terms(self, norm: "LayerNorm"):
         """(W', c1, c2, A', ca1, ca2) of this layer behind `norm` (lora.fold_layer_norm), rebuilt when the weights, the
         norm's parameters or the packed adapters change."""
-        _, w, b = self._rt
+        ver, w, b = self._rt
         p = self._packed
-        key = (self._rt[0], id(norm), norm.weight._version, norm.bias._version, norm.weight.data_ptr(),
-               None if p is None else (p.a_cat.data_ptr(), p.a_cat._version))
-        if self._ln_rt is None or self._ln_rt[0] != key:
-            self._ln_rt = (key, fold_layer_norm(w, b, norm.weight, norm.bias, None if p is None else p.a_cat))
-        return self._ln_rt[1]
+        nk = norm_key(norm)
+        if self._ln_w is None or self._ln_w[0] != (ver, nk):
+            self._ln_w = ((ver, nk),) + fold_norm_into_weight(w, b, norm.weight, norm.bias)
+        if p is None:
+            return self._ln_w[1:] + (None, None, None)
+        if p.ln is None or p.ln[0] != nk:
+            p.ln = (nk,) + fold_norm_into_adapters(p.a_cat, norm.weight, norm.bias)
+        return self._ln_w[1:] + p.ln[1:]
 
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, ln=None,
                 stats_out: Optional[RowStats] = None) -> torch.Tensor:
@@ -323,6 +340,41 @@ class LoRALinear(nn.Module):
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, geglu={self.geglu}"
+
+
+def refresh_many(modules) -> None:
+    """refresh_adapters of many modules.  Linear layers on the GPU whose packs have to be built get them from two launches over
+    all of them, those whose scales alone have changed from one; everything else refreshes by itself."""
+    global _pack_epoch
+    build: Dict[object, list] = {}
+    scale: Dict[object, list] = {}
+    for m in modules:
+        if not isinstance(m, LoRALinear):
+            m.refresh_adapters()
+            continue
+        names, key = m.wanted_pack()
+        if not names or m._rt is None:
+            m.refresh_adapters()
+        elif key == m._packed_key and m._packed is not None:
+            p = m._packed
+            if not p.col_scale.is_cuda:
+                m.refresh_adapters()
+                continue
+            rows = scale.setdefault(p.col_scale.device, [])
+            for pk in (p, *p.overflow):
+                for n, c, r in pk.spans:
+                    rows.append((pk.col_scale, c, r, m.adapters[n].multiplier(m.global_scale)))
+        elif pack_many_takes(m, names):
+            build.setdefault(m.weight.device, []).append((m, names, key))
+        else:
+            m.refresh_adapters()
+    for dev, rows in scale.items():
+        rescale_many(rows, dev)
+    for todo in build.values():
+        todo.sort(key=lambda e: e[0]._context if e[0]._context else 1 << 30)   # context projections first, one width behind the other
+        for (m, _, key), p in zip(todo, pack_many([e[0] for e in todo], [e[1] for e in todo])):
+            m._packed, m._packed_key = p, key
+        _pack_epoch += 1
 
 
 class GroupNorm(nn.Module):
@@ -799,8 +851,12 @@ class Attention(nn.Module):
         self.to_out = nn.ModuleList([LoRALinear(inner, query_dim, bias=out_bias), nn.Dropout(0.0)])
         self.processor = processor or KatzAttnProcessor()
         self.is_cross = cross_attention_dim is not None
+        if self.is_cross:
+            self.to_k._context = self.to_v._context = inner
         self.ctx_kv = None  # (context tensor, k, v) filled by ContextKVProjector for the current step
         self._qkv = None    # fused to_q/to_k/to_v state (self-attention only)
+        self._qkv_w = None  # (key, stacked weights): they outlive a change of adapters
+        self._qkv_ln = None # (key, W', c1, c2): the stacked weights with the norm in front folded in
 
     def fused_qkv(self, x: torch.Tensor, ln=None):
         """to_q / to_k / to_v of a self-attention as ONE GEMM over the stacked weights ([3N,K]: three
@@ -821,14 +877,20 @@ class Attention(nn.Module):
             ok = same and (packs[0] is None or LORA_MODE == "split") and all(l.bias is None for l in layers)
             st = dict(sig=sig, ok=ok)
             if ok:
-                st["w"] = torch.cat([l.weight.detach() for l in layers], dim=0).contiguous()
+                if self._qkv_w is None or self._qkv_w[0] != sig[1]:
+                    self._qkv_w = (sig[1], torch.cat([l.weight.detach() for l in layers], dim=0).contiguous())
+                st["w"] = self._qkv_w[1]
                 st["R"] = 0 if packs[0] is None else packs[0].R
                 if st["R"]:
                     R = st["R"]
                     st["r_used"] = max(p.r_used for p in packs)
-                    st["a"] = torch.cat([p.a_cat for p in packs], dim=0).contiguous()
-                    st["s"] = torch.cat([p.col_scale for p in packs], dim=0).contiguous()
-                    st["b"] = torch.cat([p.b_cat for p in packs], dim=0).contiguous()
+                    cat = lambda ts: torch.cat(ts, dim=0).contiguous()
+                    a, sc, bc = ([getattr(p, n) for p in packs] for n in ("a_cat", "col_scale", "b_cat"))
+                    st["a"], st["s"], st["b"] = stacked(a), stacked(sc), stacked(bc)
+                    if st["b"] is None:
+                        st["b"] = cat(bc)
+                    if st["a"] is None or st["s"] is None:
+                        st["a"], st["s"] = cat(a), cat(sc)
                     for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
                         p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
             self._qkv = st
@@ -837,11 +899,21 @@ class Attention(nn.Module):
         if ln is not None and ln[1] is not None and ln[1].valid and LN_FOLD:
             # the norm in front is folded into the stacked GEMM (ln = (LayerNorm, RowStats of x))
             norm, stats = ln
-            key = (id(norm), norm.weight._version, norm.bias._version, norm.weight.data_ptr())
-            if st.get("ln_key") != key:
-                st["ln"] = fold_layer_norm(st["w"], None, norm.weight, norm.bias, st["a"] if st["R"] else None)
-                st["ln_key"] = key
-            wp, c1, c2, ap, ca1, ca2 = st["ln"]
+            key = norm_key(norm)
+            if self._qkv_ln is None or self._qkv_ln[0] != (key, sig[1]):
+                self._qkv_ln = ((key, sig[1]),) + fold_norm_into_weight(st["w"], None, norm.weight, norm.bias)
+            _, wp, c1, c2 = self._qkv_ln
+            ap = ca1 = ca2 = None
+            if st["R"]:
+                if st.get("ln_key") != key:
+                    parts = [l._packed.ln for l in layers]
+                    ln = None
+                    if all(t is not None and t[0] == key for t in parts):   # built with the packs, side by side
+                        ln = tuple(stacked([t[j] for t in parts]) for j in (1, 2, 3))
+                    if ln is None or any(t is None for t in ln):
+                        ln = fold_norm_into_adapters(st["a"], norm.weight, norm.bias)
+                    st["ln"], st["ln_key"] = ln, key
+                ap, ca1, ca2 = st["ln"]
             y = ops.lora_linear_norm(x, wp, None, ap, st["s"] if st["R"] else None, st["b"] if st["R"] else None,
                                      two_launches=LORA_SHRINK == "separate", n_split=N if st["R"] else 0,
                                      r_used=st["r_used"] if st["R"] else 0, ln=(stats.buf, c1, c2, ca1, ca2, norm.eps))
@@ -920,6 +992,10 @@ class BasicTransformerBlock(nn.Module):
             self.norm2 = self.attn2 = None
         self.norm3 = LayerNorm(dim, 1e-5)
         self.ff = FeedForward(dim)
+        for norm, layers in ((self.norm1, (self.attn1.to_q, self.attn1.to_k, self.attn1.to_v)),
+                             (self.norm2, () if self.attn2 is None else (self.attn2.to_q,)), (self.norm3, (self.ff.net[0].proj,))):
+            for l in layers:
+                l._fold_norm = (norm,)
 
     def forward(self, h, encoder_hidden_states=None, stats: Optional[RowStats] = None, last: bool = False):
         """stats: the row statistics of h as its producer left them (or invalid); on return they describe the result,
@@ -1005,8 +1081,10 @@ class ContextKVProjector:
             y = torch.empty((G, M, width), dtype=torch.bfloat16, device=dev)
             t = a_all = s_all = None
             if R > 0:
-                a_all = torch.cat([p.a_cat for p in packs], dim=0).contiguous()
-                s_all = torch.cat([p.col_scale for p in packs], dim=0).contiguous()
+                a_all, s_all = stacked([p.a_cat for p in packs]), stacked([p.col_scale for p in packs])
+                if a_all is None or s_all is None:
+                    a_all = torch.cat([p.a_cat for p in packs], dim=0).contiguous()
+                    s_all = torch.cat([p.col_scale for p in packs], dim=0).contiguous()
                 for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
                     p.a_cat = a_all[g * R:(g + 1) * R]
                     p.col_scale = s_all[g * R:(g + 1) * R]

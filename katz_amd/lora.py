@@ -15,10 +15,14 @@ rewrites col_scale.
 """
 from __future__ import annotations
 
+import struct
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
+
+from . import ops
 
 RANK_PAD = 64   # packed rank is padded to the K-stage depth of the GEMM that consumes it
 MAX_PACKED_RANK = 128
@@ -53,6 +57,8 @@ class PackedAdapters:
     # adapters, continued).  Only LoRALinear's own forward applies them; the fused launches that stack several
     # layers' packs take the per-layer path when a layer has any.
     overflow: List["PackedAdapters"] = field(default_factory=list)
+    # behind a folded LayerNorm: (norm_key of that norm, A_cat * weight, its row sums, A_cat . bias), fold_layer_norm's last three
+    ln: Optional[tuple] = None
 
     @property
     def R(self) -> int:
@@ -132,6 +138,109 @@ def pack_adapters(adapters: Dict[str, Adapter], active: Sequence[str], in_featur
     return built[0]
 
 
+def norm_key(norm) -> tuple:
+    """Identifies the parameters a LayerNorm has now."""
+    return (id(norm), norm.weight._version, norm.bias._version, norm.weight.data_ptr())
+
+
+def stacked(views: Sequence[torch.Tensor]) -> Optional[torch.Tensor]:
+    """Tensors that lie one behind the other in one buffer (pack_many), as one tensor over their first axis; None otherwise."""
+    first = views[0]
+    at, store, rows = first.data_ptr(), first.untyped_storage().data_ptr(), 0
+    for v in views:
+        if v.data_ptr() != at or not v.is_contiguous() or v.shape[1:] != first.shape[1:] or v.untyped_storage().data_ptr() != store:
+            return None
+        at += v.numel() * v.element_size()
+        rows += v.shape[0]
+    return first.as_strided((rows,) + tuple(first.shape[1:]), first.stride())
+
+
+_PIECE_DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+
+
+def pack_many_takes(layer, names: Sequence[str]) -> bool:
+    """Can pack_many build this layer's pack (else: pack_adapters)?"""
+    w = layer.weight
+    if not w.is_cuda or w.dtype != torch.bfloat16 or layer.in_features % 8 != 0 or layer.out_features % 8 != 0:
+        return False
+    total = 0
+    for n in names:
+        ad = layer.adapters[n]
+        r = ad.down.shape[0]
+        total += r
+        for t, shape in ((ad.down, (r, layer.in_features)), (ad.up, (layer.out_features, r))):
+            if t.dtype not in _PIECE_DTYPES or t.shape != shape or (t.is_cuda and (t.device != w.device or not t.is_contiguous() or t.data_ptr() % 16)):
+                return False
+    return 0 < total <= MAX_PACKED_RANK and (not layer.geglu or layer.out_features % 64 == 0)
+
+
+def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAdapters]:
+    """pack_adapters for many layers of one device in two launches (kh_lora_pack_bf16); adapters in host memory are uploaded
+    with one call.  All packs of a kind share one buffer, in the order of `layers`, so layers that run as one launch (q / k / v of
+    a self-attention, the context projections) find their stacked operands in place (`stacked`).  layer.fold_norm: a function
+    that gives the LayerNorm in front of the layer or None."""
+    dev = layers[0].weight.device
+    host = [t for l, ns in zip(layers, names) for n in ns for t in (l.adapters[n].down, l.adapters[n].up) if not t.is_cuda]
+    keep, where = None, {}
+    if host:
+        keep, addresses = ops.upload_many(host, dev)
+        where = {id(t): a for t, a in zip(host, addresses)}
+    address = lambda t: t.data_ptr() if t.is_cuda else where[id(t)]
+    bits = lambda x: struct.unpack("<I", struct.pack("<f", x))[0]
+    ranks = [sum(l.adapters[n].rank for n in ns) for l, ns in zip(layers, names)]
+    padded = [-(-r // RANK_PAD) * RANK_PAD for r in ranks]
+    norms = [l.fold_norm() for l in layers]
+    norms = [g if g is not None and g.weight.dtype == torch.bfloat16 and g.weight.device == dev else None for g in norms]
+    sizes_a = [R * l.in_features for l, R in zip(layers, padded)]
+    sizes_b = [R * l.out_features for l, R in zip(layers, padded)]
+    folded = [i for i, g in enumerate(norms) if g is not None]
+    buf = lambda n, dt: torch.empty((n,), dtype=dt, device=dev)
+    A, B, S = buf(sum(sizes_a), torch.bfloat16), buf(sum(sizes_b), torch.bfloat16), buf(sum(padded), torch.float32)
+    AN = buf(sum(sizes_a[i] for i in folded), torch.bfloat16)
+    C1, C2 = (buf(sum(padded[i] for i in folded), torch.float32) for _ in range(2))
+    a_views, b_views, s_views = A.split(sizes_a), B.split(sizes_b), S.split(padded)
+    an_views, c1_views, c2_views = AN.split([sizes_a[i] for i in folded]), C1.split([padded[i] for i in folded]), C2.split([padded[i] for i in folded])
+    pa, pb, ps, pan, pc1, pc2 = (t.data_ptr() for t in (A, B, S, AN, C1, C2))
+    rows, pieces, packs, f = [], [], [], 0
+    b_blocks = []
+    for i, (l, ns, R) in enumerate(zip(layers, names, padded)):
+        K, N, g = l.in_features, l.out_features, norms[i]
+        ln = None
+        if g is not None:
+            rows.append((pa, pan, g.weight.data_ptr(), g.bias.data_ptr(), pc1, pc2, pb, ps, K, N, R, int(l.geglu), len(pieces), len(ns)))
+            ln = (norm_key(g), an_views[f].view(R, K), c1_views[f], c2_views[f])
+            f += 1
+            pan += 2 * R * K
+            pc1 += 4 * R
+            pc2 += 4 * R
+        else:
+            rows.append((pa, 0, 0, 0, 0, 0, pb, ps, K, N, R, int(l.geglu), len(pieces), len(ns)))
+        spans, c = [], 0
+        for n in ns:
+            ad = l.adapters[n]
+            r = ad.down.shape[0]
+            if ad.up.dtype != ad.down.dtype:
+                raise TypeError(f"adapter {n!r}: down and up have different dtypes")
+            pieces.append((address(ad.down), address(ad.up), r, c, _PIECE_DTYPES[ad.down.dtype], bits(ad.multiplier(l.global_scale))))
+            spans.append((n, c, r))
+            c += r
+        packs.append(PackedAdapters(a_views[i].view(R, K), b_views[i].view(N, R), s_views[i], spans, ln=ln))
+        per_block = 256 // (R // 8)
+        b_blocks.append(-(-N // per_block))
+        pa += 2 * R * K
+        pb += 2 * R * N
+        ps += 4 * R
+    start = lambda counts: np.concatenate([np.zeros(1, np.int32), np.cumsum(counts, dtype=np.int32)])
+    ops.lora_pack(np.array(rows, dtype=np.int64), np.array(pieces, dtype=np.int64), start(padded), start(b_blocks), dev)
+    del keep    # stream-ordered: the launches above are enqueued
+    return packs
+
+
+def rescale_many(rows, device) -> None:
+    """rescale_ for many packs on one GPU in one launch; rows: (col_scale, first column, columns, value)."""
+    ops.lora_rescale(np.array([(t.data_ptr(), c, r, struct.unpack("<I", struct.pack("<f", v))[0]) for t, c, r, v in rows], dtype=np.int64), device)
+
+
 def rescale_(packed: PackedAdapters, adapters: Dict[str, Adapter], global_scale: float = 1.0) -> None:
     """Rewrite col_scale only (scale_lora_layers / set_adapters weight change); A_cat/B_cat stay put."""
     for pk in [packed, *packed.overflow]:
@@ -199,28 +308,33 @@ def module_weight(weight_for_adapter, module_name: str) -> float:
     raise RuntimeError(f"No LoRA weight found for module {module_name}.")
 
 
+def _fold_terms(m: torch.Tensor, gamma: torch.Tensor, beta):
+    g = gamma.detach().double()
+    md = m.detach().double()
+    mp = (md * g).to(m.dtype)
+    s1 = mp.double().sum(dim=1)
+    s2 = md @ beta.detach().double() if beta is not None else torch.zeros_like(s1)
+    return mp.contiguous(), s1, s2
+
+
+def fold_norm_into_weight(weight: torch.Tensor, bias, gamma: torch.Tensor, beta):
+    """(W', c1, c2) of fold_layer_norm: they depend on the weights and the norm only."""
+    wp, c1, c2 = _fold_terms(weight, gamma, beta)
+    if bias is not None:
+        c2 = c2 + bias.detach().double()
+    return wp, c1.float().contiguous(), c2.float().contiguous()
+
+
+def fold_norm_into_adapters(a_cat: torch.Tensor, gamma: torch.Tensor, beta):
+    """(A', ca1, ca2) of fold_layer_norm."""
+    ap, ca1, ca2 = _fold_terms(a_cat, gamma, beta)
+    return ap, ca1.float().contiguous(), ca2.float().contiguous()
+
+
 def fold_layer_norm(weight: torch.Tensor, bias, gamma: torch.Tensor, beta, a_cat=None):
     """The operands of a linear whose LayerNorm (weight gamma, bias beta over the input features) is folded into the GEMM
     (kh_lora_linear_norm_bf16):  LN(x) W^T + b = rstd * (x W'^T - mean * c1) + c2.
     Returns (W', c1, c2, A', ca1, ca2): W' = W * gamma per input column (rounded to the weight's dtype), c1 the row sums
     of the rounded W', c2 = b + W beta; A' / ca1 / ca2 the same for the stacked adapter A matrices (None without)."""
-    g = gamma.detach().double()
-    b = None if beta is None else beta.detach().double()
-
-    def terms(m):
-        md = m.detach().double()
-        mp = (md * g).to(m.dtype)
-        s1 = mp.double().sum(dim=1)
-        s2 = md @ b if b is not None else torch.zeros_like(s1)
-        return mp.contiguous(), s1, s2
-
-    wp, c1, c2 = terms(weight)
-    if bias is not None:
-        c2 = c2 + bias.detach().double()
-    out = [wp, c1.float().contiguous(), c2.float().contiguous()]
-    if a_cat is not None:
-        ap, ca1, ca2 = terms(a_cat)
-        out += [ap, ca1.float().contiguous(), ca2.float().contiguous()]
-    else:
-        out += [None, None, None]
-    return tuple(out)
+    return (*fold_norm_into_weight(weight, bias, gamma, beta),
+            *(fold_norm_into_adapters(a_cat, gamma, beta) if a_cat is not None else (None, None, None)))

@@ -568,6 +568,23 @@ def upload_many(tensors: Sequence[torch.Tensor], device):
     return dst, [base + o for o in offset.tolist()]
 
 
+def lora_pack(layers, pieces, a_start, b_start, device) -> None:
+    """kh_lora_pack_bf16 on host tables (numpy int64 [n,14] and [m,6], int32 [n+1] twice)."""
+    dev = lambda a: torch.from_numpy(a).to(device, non_blocking=True)
+    lt, pt, at, bt = dev(layers), dev(pieces), dev(a_start), dev(b_start)
+    with torch.cuda.device(device):
+        rc = _lib.load().kh_lora_pack_bf16(_ptr(lt), _ptr(pt), _ptr(at), _ptr(bt), layers.shape[0], int(a_start[-1]), int(b_start[-1]), _stream())
+    _lib.check(rc, "kh_lora_pack_bf16")
+
+
+def lora_rescale(rows, device) -> None:
+    """kh_lora_rescale on host rows (numpy int64 [n,4])."""
+    table = torch.from_numpy(rows).to(device, non_blocking=True)
+    with torch.cuda.device(device):
+        rc = _lib.load().kh_lora_rescale(_ptr(table), rows.shape[0], _stream())
+    _lib.check(rc, "kh_lora_rescale")
+
+
 def lora_merge_grouped(weights: Sequence[torch.Tensor], ups: Sequence[torch.Tensor], downs: Sequence[torch.Tensor],
                        scale: float = 1.0, layer_scales: Optional[Sequence[float]] = None) -> None:
     """W_l += scale * layer_scales[l] * up_l @ down_l for all layers in ONE launch, in place (kh_lora_merge_grouped_bf16).
@@ -1125,7 +1142,7 @@ def conv_out_cfg_euler(x: torch.Tensor, w_packed: torch.Tensor, bias: Optional[t
 # --------------------------------------------------------------------------------------- per-launch timing
 KERNEL_TAGS = {1: "lora_gemm", 2: "lora_gemm_f32", 3: "attention", 4: "group_norm_stats", 5: "group_norm_apply",
                6: "layer_norm", 7: "geglu", 8: "residual_add", 9: "concat_residual", 10: "sgmv_shrink",
-               11: "sgmv_expand", 12: "lora_shrink", 13: "conv3x3", 14: "cfg_euler", 15: "upsample", 16: "lora_merge", 17: "conv_out_step", 18: "sgmv_fused"}
+               11: "sgmv_expand", 12: "lora_shrink", 13: "conv3x3", 14: "cfg_euler", 15: "upsample", 16: "lora_merge", 17: "conv_out_step", 18: "sgmv_fused", 19: "lora_pack"}
 
 
 def profile_begin() -> None:

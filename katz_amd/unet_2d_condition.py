@@ -25,7 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from .layers import Conv3x3, LoRALinear, TimestepEmbedding, fused_norm_silu
+from .layers import Conv1x1, Conv3x3, LoRALinear, TimestepEmbedding, fused_norm_silu, refresh_many
 from .lora import expand_lora_scales_for_one_adapter, module_weight
 from .unet_blocks import (CrossAttnDownBlock2D, CrossAttnUpBlock2D, DownBlock2D, UNetMidBlock2DCrossAttn, UpBlock2D)
 
@@ -230,11 +230,22 @@ class UNet2DConditionModel(nn.Module):
     def lora_convs(self) -> Dict[str, Any]:
         """Convolutions that can carry a LoRA: 3x3 (resnet conv1 / conv2, down / upsampler convs) and the resnets' 1x1
         conv_shortcut."""
-        from .layers import Conv1x1, Conv3x3
         return {n: m for n, m in self.named_modules() if isinstance(m, (Conv3x3, Conv1x1))}
 
     def _lora_targets(self) -> Dict[str, Any]:
-        return {**self.lora_linears(), **self.lora_convs()}
+        """lora_linears() then lora_convs(), in one walk over the module tree."""
+        linears, convs = {}, {}
+        stack = [("", self)]
+        while stack:
+            prefix, m = stack.pop()
+            if isinstance(m, LoRALinear):
+                linears[prefix] = m
+            elif isinstance(m, (Conv3x3, Conv1x1)):
+                convs[prefix] = m
+            elif m._modules:
+                dot = prefix + "." if prefix else ""
+                stack.extend((dot + n, c) for n, c in reversed(m._modules.items()) if c is not None)
+        return {**linears, **convs}
 
     def load_lora_into_unet(self, state_dict: Dict[str, torch.Tensor], network_alphas: Optional[Dict[str, float]] = None,
                             adapter_name: Optional[str] = None) -> str:
@@ -294,7 +305,8 @@ class UNet2DConditionModel(nn.Module):
             raise ValueError(f"Length of adapter names {len(names)} is not equal to the length of their weights {len(weights)}.")
         weights = [1.0 if w is None else w for w in weights]
         lin = self._lora_targets()
-        if any(isinstance(w, dict) for w in weights):
+        plain = not any(isinstance(w, dict) for w in weights)
+        if not plain:
             # per-block scales, e.g. {"down": 0.9, "mid": 1.0, "up": {"block_0": 0.6, "block_1": [0.4, 0.8, 1.0]}}
             # (_maybe_expand_lora_scales, diffusers-hf/src/diffusers/loaders/unet_loader_utils.py:41-58)
             bwt = {"down": [i for i, b in enumerate(self.down_blocks) if hasattr(b, "attentions")],
@@ -303,18 +315,22 @@ class UNet2DConditionModel(nn.Module):
             weights = [expand_lora_scales_for_one_adapter(w, bwt, tpb, list(lin.keys())) for w in weights]
         for mod_name, m in lin.items():
             # per-block dictionaries address transformers only; other modules (resnet convs) keep scale 1 under them
-            m.set_active(names, [module_weight(w, mod_name) if (not isinstance(w, dict) or ".attentions." in mod_name) else 1.0
-                                 for w in weights])
+            ws = weights if plain else [module_weight(w, mod_name) if (not isinstance(w, dict) or ".attentions." in mod_name) else 1.0
+                                        for w in weights]
+            (m.assign_active if isinstance(m, LoRALinear) else m.set_active)(names, ws)
+        refresh_many(m for m in lin.values() if isinstance(m, LoRALinear))
+
+    def _enable_adapters(self, on: bool) -> None:
+        targets = self._lora_targets()
+        for m in targets.values():
+            m.adapters_enabled = on
+        refresh_many(targets.values())
 
     def disable_lora(self) -> None:
-        for m in self._lora_targets().values():
-            m.adapters_enabled = False
-            m.refresh_adapters()
+        self._enable_adapters(False)
 
     def enable_lora(self) -> None:
-        for m in self._lora_targets().values():
-            m.adapters_enabled = True
-            m.refresh_adapters()
+        self._enable_adapters(True)
 
     def fuse_lora(self, lora_scale: float = 1.0, adapter_names: Optional[Sequence[str]] = None,
                   safe_fusing: bool = False) -> None:
@@ -413,8 +429,14 @@ class UNet2DConditionModel(nn.Module):
             m.refresh_adapters()
 
     def scale_lora_layers(self, scale: float) -> None:
+        changed = []
         for m in self._lora_targets().values():
-            m.set_global_scale(scale)
+            if not isinstance(m, LoRALinear):
+                m.set_global_scale(scale)
+            elif scale != m.global_scale:
+                m.global_scale = float(scale)
+                changed.append(m)
+        refresh_many(changed)
 
     def set_attn_processor(self, processor) -> None:
         """unet_2d_condition.py:800-832: one processor for all, or a dict keyed '<module>.processor'."""

@@ -35,6 +35,55 @@ def test_lora_linear_f32_matrix_kernel(M, N, K, R):
     assert_close_rel(y, ref, 1e-5, "fp32 linear")
 
 
+@pytest.mark.parametrize("host,dtype,ranks", [(False, torch.bfloat16, (64, 32)), (True, torch.float16, (16,)), (False, torch.float32, (4, 8, 100)), (True, torch.bfloat16, (5, 7))],
+                         ids=str)
+def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
+    """set_adapters through kh_lora_pack_bf16 / kh_lora_rescale: every layer's buffers bit for bit against pack_adapters and
+    fold_layer_norm, ranks that no 16-byte piece fits included; a change of weights alone keeps the buffers; switching off and
+    on again; adapters in host memory (kh_upload_many) and on the GPU."""
+    import katz_amd.layers as L
+    from katz_amd.lora import fold_norm_into_adapters, pack_adapters
+    from katz_amd.unet_2d_condition import UNet2DConditionModel, UNetConfig
+
+    say("pack", host, dtype, ranks)
+    d = dev()
+    torch.manual_seed(3)
+    with torch.device(d):
+        unet = UNet2DConditionModel(UNetConfig.tiny())
+    unet.to_runtime(d, BF)
+    g = torch.Generator().manual_seed(5)
+    for i, r in enumerate(ranks):
+        for l in unet.lora_linears().values():
+            l.add_adapter(f"a{i}", *(t.to(dtype) if host else t.to(d, dtype) for t in (torch.randn(r, l.in_features, generator=g), torch.randn(l.out_features, r, generator=g))))
+    names, weights = [f"a{i}" for i in range(len(ranks))], [0.3 + 0.4 * i for i in range(len(ranks))]
+
+    def check():
+        for name, l in unet.lora_linears().items():
+            ref = pack_adapters(l.adapters, names, l.in_features, l.out_features, BF, d, l.global_scale, geglu_interleave=l.geglu)
+            p = l._packed
+            assert torch.equal(p.a_cat, ref.a_cat) and torch.equal(p.b_cat, ref.b_cat) and torch.equal(p.col_scale, ref.col_scale), name
+            assert p.spans == ref.spans and p.r_used == ref.r_used
+            norm = l.fold_norm()
+            assert (p.ln is not None) == (norm is not None)
+            if norm is not None:
+                ap, c1, c2 = fold_norm_into_adapters(p.a_cat, norm.weight, norm.bias)
+                assert torch.equal(p.ln[1], ap), name
+                assert torch.allclose(p.ln[2], c1, rtol=1e-6, atol=1e-6) and torch.allclose(p.ln[3], c2, rtol=1e-6, atol=1e-6), name
+
+    unet.set_adapters(names, weights)
+    check()
+    where = {n: l._packed.a_cat.data_ptr() for n, l in unet.lora_linears().items()}
+    unet.set_adapters(names, [w + 1 for w in weights])           # scales only: the same buffers
+    check()
+    assert where == {n: l._packed.a_cat.data_ptr() for n, l in unet.lora_linears().items()}
+    unet.scale_lora_layers(0.5)
+    check()
+    unet.disable_lora()
+    assert all(l._packed is None for l in unet.lora_linears().values())
+    unet.enable_lora()
+    check()
+
+
 def test_upload_many_sizes():
     """kh_upload_many: arrays smaller and larger than a staging half, empty gaps, one array, bit for bit."""
     from katz_amd import ops
