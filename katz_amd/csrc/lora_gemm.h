@@ -237,6 +237,10 @@ int lora_gemm_ksplit_launch_conv(const LoraGemmParams& p, int row_groups, hipStr
 // the convolution that also leaves GroupNorm statistics (gn_cg / gn_hw set): row groups of the 160-column tiles it would run
 // on, 0 when the rules give it other tiles or the groups do not fit them
 int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
+// Fine tiles (lora_gemm_fine.hip), for sizes that give each CU at most one of them, with the sums in the order of the 128 x 128 (order 0) or
+// the 64 x 160 kernel (order 4); plain or K-extended GEMM and (order 4) 3x3 convolutions.  Form -1: not suited.
+int lora_gemm_fine_form(const LoraGemmParams& p, int order);
+int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream);
 // Wide-tile variant (lora_gemm_wide.hip): 256 x 320 tiles, 8 waves; plain or K-extended GEMM with bias / residual /
 // GEGLU; M % 256 == 0, N % 320 == 0, K % 64 == 0.
 bool lora_gemm_wide_ok(const LoraGemmParams& p);

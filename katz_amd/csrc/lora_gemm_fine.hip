@@ -1,0 +1,532 @@
+// K1 / K1c, fine tiles: y = x W^T (+ T B_cat^T, + bias, + residual, LayerNorm folded in / row statistics out) and 3x3
+// convolutions on BM x BN output tiles small enough that a few hundred rows still give every CU a workgroup.
+//
+// Same arithmetic as the two-launch form of lora_gemm_pipe.hip (the reference's LoRA linear,
+// diffusers-hf/src/diffusers/models/lora.py:224-225, T made by a launch in front), bit for bit as the kernel that runs at
+// more rows: the order of every sum is that kernel's (below).
+//
+// What bounds these calls: not the matrix pipe and not HBM's rate but a CU's operand stream.  A CU takes about 55 GB/s of
+// lines that come from memory and 110 GB/s of lines its L2 has, all CUs together 17 TB/s out of the L2s; a 128 x 128 tiling of M = 1000 /
+// N = 1280 streams 32 KB a stage into each of 80 CUs and takes 16 us, whether M is 150 or 2000.  Hence
+//   * small tiles: 64 x 80 gives 256 workgroups there, 18 KB a stage;
+//   * four waves that only move operands beside four that only compute: a wave that does both stands in the queue of the address
+//     unit (16 clocks per 1 KB instruction) while its MFMAs wait (64 x 160 tiles: 1330 clocks a stage together, 860 apart);
+//   * a ring of as many stages as LDS holds (up to 8), and
+//   * the XCD's block of W fetched into its L2 by all its workgroups before the K loop meets it.
+//
+// Orders (ORD): the 128 x 128 / 256 x 320 kernels add along K one 16-column step after the other (0), the 64 x 160 kernel in four
+// slices of 16 of every 64 columns that are added at the end (4).  v_mfma 16x16x32 gives the bits of two chained 16-column steps of
+// 32x32x16, and 16x16x16 those of one, so 16-row tiles can follow either.  Row statistics are sums over 128 columns (order 0) or
+// 160 (order 4): layers that leave them run on tiles of that width.
+//
+// Operands reach LDS by buffer loads (8 rows x 128 bytes per instruction, XOR-swizzled pieces, rows past M read zeros).
+#include "kh_common.h"
+#include "lora_gemm.h"
+
+namespace {
+
+typedef __attribute__((address_space(3))) void* lptr_t;
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+template <int VM, int LGKM>
+__device__ __forceinline__ void wait_cnt() {  // gfx9 encoding: vmcnt = [15:14|3:0], expcnt = [6:4], lgkmcnt = [11:8]
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((LGKM & 15) << 8) | ((VM >> 4) << 14));
+}
+
+// a bare barrier (a fence would drain the prefetches), kept in place among the memory accesses around it
+__device__ __forceinline__ void ring_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+constexpr int cmin(int a, int b) { return a < b ? a : b; }
+
+template <int BM_, int BN_, int ORD_>
+struct FCfg {
+  static constexpr int BM = BM_, BN = BN_, ORD = ORD_;
+  // computing waves: WM row groups x WN column groups x WK k-slices
+  static constexpr int WK = ORD == 0 ? 1 : 4, WN = ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
+  // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
+  static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
+  static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 0 ? 2 : 1;   // a wave's MFMA tiles, its k-steps per stage
+  static constexpr bool DB = TM * TN * G * 4 <= 96;      // two fragment buffers where the registers allow it
+  static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
+  static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
+  static constexpr int UNITS = ROWS / UR, LPS_LO = UNITS / 4, N_HI = UNITS % 4, LPS_HI = LPS_LO + (N_HI ? 1 : 0);
+  static constexpr int XQ = BM / UR / 4;                                         // DMA units q < XQ are x rows for every wave
+  static constexpr int LDC = BN + 8;
+  // partial sums of the k-slices (NH passes over the row tiles) / row statistics
+  static constexpr int NH = WK > 1 && 4 * TM * TN * G > 80 ? 2 : 1;
+  static constexpr int PART = WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
+  static constexpr int TAIL = PART + BM * LDC * 2;
+  static constexpr int NST = cmin(8, (159 * 1024 - KH_LN_LDS) / STAGE), PD = NST - 1;   // as many stages as fit, but at most 8
+  static constexpr int TOUCH_OFF = cmax(NST * STAGE, TAIL), LDS = TOUCH_OFF + 1024;     // (where prefetched dwords nobody reads land)
+  static constexpr int OPC = BM * (BN / 8), OPT = (OPC + 511) / 512;             // 16-byte output pieces: per tile, per thread
+  static_assert(WM * WN * WK == 4 && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
+  static_assert(BM % 32 == 0 && XQ * UR * 4 == BM && ROWS % UR == 0, "whole DMA instructions");
+  static_assert(NST >= 3 && LPS_HI * (PD - 1) < 63 && LDS + KH_LN_LDS <= 160 * 1024, "ring");
+};
+
+// CONV: x is an NHWC image and row m of the GEMM is output pixel m of a 3x3 convolution with padding 1 (K = 9 * Cin ordered
+// (kh, kw, ci)): a stage is 64 channels of one tap, taps outside the image read zeros (an offset beyond the buffer).
+// Rows come in segments of seg_rows (an image of the convolution, everything otherwise) that start a tile of their own.
+template <class C, bool CONV>
+__global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
+#if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, NST = C::NST, PD = C::PD;
+  constexpr int BK = C::BK, ROWB = C::ROWB, UR = C::UR, PPR = C::PPR, STAGE = C::STAGE, LPS_LO = C::LPS_LO, LPS_HI = C::LPS_HI, XQ = C::XQ;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool producer = wave >= 4;                     // waves 4 .. 7 move operands, waves 0 .. 3 compute
+  const int pw = wave & 3, wm = pw / (C::WK * C::WN), wn = pw / C::WK % C::WN, wk = pw % C::WK;
+  const int lr = lane % C::MF, lg = lane / C::MF;      // row inside an MFMA tile, 16-byte (8-byte) piece of a k-step
+
+    // tile of this workgroup: XCD b % 8 owns a block of xr_m x xr_n tiles (its W rows stay in its L2)
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int m_blk = (xcd / p.xg_n) * p.xr_m + local / p.xr_n;
+  const int n_blk = (xcd % p.xg_n) * p.xr_n + local % p.xr_n;
+  if (local / p.xr_n >= p.xr_m || m_blk >= p.m_tiles || n_blk >= p.n_tiles) return;  // padding of the grid
+  const int M = p.M, N = p.N, K = p.K;
+  const int seg = m_blk / seg_tiles, m0 = seg * seg_rows + (m_blk % seg_tiles) * BM, n0 = n_blk * BN;
+  const int seg_end = (seg + 1) * seg_rows, rows = (seg_end < M ? seg_end : M) - m0;   // rows of this tile that exist (may exceed BM)
+  // T made by a launch in front: its rank columns are extra K tiles
+  constexpr bool EXT = !CONV;
+  const int KT1 = K / BK, r_ext = p.r_used > 0 ? p.r_used : p.R;
+  const int KT = KT1 + (EXT && p.t_ext != nullptr ? (r_ext + BK - 1) / BK : 0);
+  const bool has_hi = pw < C::N_HI;
+
+  // per-row and per-column terms: requested now, used after the K loop (older than every DMA load, so no wait falls in between)
+  KhLnTileStats<BM, 512> ln_stats;
+  float c1v = 0.f, c2v = 0.f;
+  uint16_t biasv = 0;
+  if (p.ln_part != nullptr) {
+    ln_stats.load(p.ln_part, m0, M, tid);
+    if (tid < BN) { c1v = p.ln_c1[n0 + tid]; c2v = p.ln_c2[n0 + tid]; }
+  } else if (p.bias != nullptr && tid < BN) {
+    biasv = reinterpret_cast<const uint16_t*>(p.bias)[n0 + tid];
+  }
+
+  // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
+  // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row): 16 rows at one piece fill the 64 banks.
+  auto swz = [](int row) { return (PPR == 8 ? row >> 1 : row) & (PPR - 1); };
+  constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
+  uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
+  int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
+#pragma unroll
+  for (int q = 0; q < LPS_HI; ++q) {
+    int u = pw + 4 * q;
+    u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
+    const int r = u * UR + lane / PPR;
+    const uint32_t pcb = (uint32_t)(((lane % PPR) ^ swz(r)) * 16);
+    if (CONV && q < XQ) {
+      int row = m0 + r; row = row < M ? row : M - 1;
+      const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
+      const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
+      int mask = 0;
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) {
+        const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
+        mask |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
+      }
+      tapmask[q < XQ ? q : 0] = mask;
+      // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
+      voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
+    } else if (q < XQ) {
+      voff[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + pcb;        // rows past M lie beyond the buffer: zeros
+    } else {
+      voff[q] = (uint32_t)(n0 + r - BM) * (uint32_t)K * 2u + pcb;
+    }
+    if (EXT && p.t_ext != nullptr)
+      voff2[q] = q < XQ ? ((uint32_t)(m0 + r) * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb
+                        : (uint32_t)(n0 + r - BM) * (uint32_t)p.R * 2u + pcb;
+  }
+  const size_t x_bytes = CONV ? (size_t)(M / (p.conv_ho * p.conv_wo)) * p.conv_h * p.conv_w * p.conv_cin * 2 : (size_t)M * K * 2;
+  const size_t x_lead = CONV ? (size_t)(p.conv_w + 1) * p.conv_cin * 2 : 0;
+  const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.x) - x_lead), 0,
+                                                         (int)(x_bytes + x_lead), 0x00020000);
+  const rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w), 0, (int)((size_t)N * K * 2), 0x00020000);
+  const bool has_t = EXT && p.t_ext != nullptr;
+  const rsrc_t rs_t = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.t_ext : p.x), 0,
+                                                         has_t ? (int)((size_t)M * p.ldt * 2) : 0, 0x00020000);
+  const rsrc_t rs_bx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.b_cat : p.w), 0,
+                                                          has_t ? (int)((size_t)N * p.R * 2) : 0, 0x00020000);
+  // CONV: K tiles are requested in order, so the tap and the channel offset of the next request are running scalars
+  int cv_tap = 0, cv_kw = 0, cv_c0 = 0, cv_shift = 0, cv_row = 0;
+  uint32_t xvo[XQ];
+#pragma unroll
+  for (int q = 0; q < XQ; ++q) xvo[q] = (!CONV || (tapmask[CONV ? q : 0] & 1)) ? voff[q] : OOB;
+  auto issue = [&](int t, int st) {                    // K tile t into the ring stage at byte offset st
+    char* stage = smem + st;
+    const int so = t * ROWB;
+    if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
+      const int c = (t - KT1) * BK;
+#pragma unroll
+      for (int q = 0; q < LPS_HI; ++q) {
+        if (q < LPS_LO || has_hi) {
+          const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16,
+                                                   col < r_ext ? voff2[EXT ? q : 0] : OOB, c * 2, 0, 0);
+        }
+      }
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < LPS_HI; ++q) {
+      if (q < LPS_LO || has_hi) {
+        lptr_t dst = (lptr_t)(stage + (pw + 4 * q) * 1024);
+        if (q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, dst, 16, xvo[q], CONV ? (cv_shift + cv_c0) * 2 : so, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, voff[q], so, 0, 0);
+      }
+    }
+    if (CONV) {
+      cv_c0 += BK;
+      if (cv_c0 == p.conv_cin) {
+        cv_c0 = 0; ++cv_tap; ++cv_kw; cv_shift += p.conv_cin;
+        if (cv_kw == 3) { cv_kw = 0; cv_row += p.conv_w * p.conv_cin; cv_shift = cv_row; }
+#pragma unroll
+        for (int q = 0; q < XQ; ++q) xvo[q] = ((tapmask[CONV ? q : 0] >> cv_tap) & 1) ? voff[q] : OOB;
+      }
+    }
+  };
+  // until at most n of this wave's younger K tiles are outstanding (and its LDS reads are done)
+  auto wait_younger = [&](int n) {
+    if (n >= PD - 1) { if (has_hi) wait_cnt<LPS_HI * (PD - 1), 0>(); else wait_cnt<LPS_LO * (PD - 1), 0>(); return; }
+    switch (n) {
+      case 6: if (has_hi) wait_cnt<LPS_HI * (PD > 6 ? 6 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 6 ? 6 : 0), 0>(); break;
+      case 5: if (has_hi) wait_cnt<LPS_HI * (PD > 5 ? 5 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 5 ? 5 : 0), 0>(); break;
+      case 4: if (has_hi) wait_cnt<LPS_HI * (PD > 4 ? 4 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 4 ? 4 : 0), 0>(); break;
+      case 3: if (has_hi) wait_cnt<LPS_HI * (PD > 3 ? 3 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 3 ? 3 : 0), 0>(); break;
+      case 2: if (has_hi) wait_cnt<LPS_HI * (PD > 2 ? 2 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 2 ? 2 : 0), 0>(); break;
+      case 1: if (has_hi) wait_cnt<LPS_HI, 0>(); else wait_cnt<LPS_LO, 0>(); break;
+      default: wait_cnt<0, 0>(); break;
+    }
+  };
+
+  // fragments: row lr of each block of MF rows; of a k-step the lane's 16-byte piece lg (16x16x16: its 8 bytes lg)
+  constexpr bool HALF = C::ORD == 4 && C::MF == 16;
+  using Frag = typename std::conditional<HALF, s16x4, bf16x8>::type;
+  using Acc = typename std::conditional<C::MF == 32, f32x16, f32x4>::type;
+  struct Fr { Frag a[KS][TM], b[KS][TN]; };
+  int fa[KS], fb[KS];
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * wk + lg) ^ swz(lr)) * 16;
+    fa[k] = (wm * (BM / C::WM) + lr) * ROWB + po;
+    fb[k] = (BM + wn * (BN / C::WN) + lr) * ROWB + po;
+  }
+  auto read_frags = [&](int st, Fr& f) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) f.a[k][i] = *reinterpret_cast<const Frag*>(smem + st + fa[k] + i * C::MF * ROWB);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) f.b[k][j] = *reinterpret_cast<const Frag*>(smem + st + fb[k] + j * C::MF * ROWB);
+    }
+  };
+  Acc acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 4 * C::G; ++e) acc[i][j][e] = 0.f;
+  auto mma = [&](const Fr& f) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          if constexpr (HALF) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
+          else if constexpr (C::MF == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
+          else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
+        }
+  };
+
+  // K loop.  Step t: tile t is in the computing waves' registers (cur); tile t+1 becomes visible at the barrier, after which
+  // every wave has read tile t out of its stage, so that stage takes tile t + NST.  Both kinds of waves pass KT barriers.
+  if (producer) {
+    kh_prefetch_lines(p.pf, p.pf_lines, smem + pw * 1024, blockIdx.x, gridDim.x, tid - 256, 256);
+#pragma unroll
+    for (int t = 0; t < PD; ++t)
+      if (t < KT) issue(t, t * STAGE);
+    wait_younger(KT - 1);
+    ring_barrier();
+    if (KT > PD) issue(PD, PD * STAGE);
+    int st = 0, t = 0;                                 // stage of tile t
+    for (; t + NST < KT; ++t) {
+      wait_younger(PD - 1);
+      ring_barrier();
+      issue(t + NST, st);
+      st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+    }
+    for (; t + 1 < KT; ++t) {
+      wait_younger(KT - 2 - t);
+      ring_barrier();
+    }
+  } else {
+    // The XCD's block of W is contiguous rows: its workgroups fetch it into their L2 between them, a line a lane,
+    // before the K loop meets it.  In the loop all of them ask for the same lines at the same time, and a CU takes about 55 GB/s
+    // of lines that come from memory, 110 GB/s of lines that its L2 has (M 988, N 1280, K 1280: 10.4 -> 9.4 us; 128 x 80 tiles
+    // at M 2048, K 5120: 39.9 -> 37.0; x, which the launch in front has just written, is not worth it).
+    const int nloc = p.xr_m * p.xr_n;
+    auto touch = [&](const void* base, size_t bytes_total, size_t first_byte, size_t bytes) {
+      const rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes_total, 0x00020000);
+      const uint32_t lines = (uint32_t)(bytes >> 7);
+      for (uint32_t l = (uint32_t)(local * 256 + tid); l < lines; l += (uint32_t)nloc * 256u)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(smem + C::TOUCH_OFF + pw * 256), 4, (uint32_t)first_byte + (l << 7), 0, 0, 0);
+    };
+    const int nf = (xcd % p.xg_n) * p.xr_n * BN, nr = (nf + p.xr_n * BN < N ? nf + p.xr_n * BN : N) - nf;
+    touch(p.w, (size_t)N * K * 2, (size_t)nf * K * 2, (size_t)nr * K * 2);
+    ring_barrier();
+    int st = 0;
+    if constexpr (!C::DB) {
+      for (int t = 0; t < KT; ++t) {
+        Fr f;
+        read_frags(st, f);
+        mma(f);
+        st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+        if (t + 1 < KT) ring_barrier();
+      }
+    } else {
+    Fr f0, f1;
+    read_frags(0, f0);
+    auto step = [&](const Fr& cur, Fr& nxt) {
+      st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+      wait_cnt<63, 0>();
+      ring_barrier();
+      read_frags(st, nxt);
+      mma(cur);
+    };
+    int t = 0;
+    for (; t + 2 < KT; t += 2) {
+      step(f0, f1);
+      step(f1, f0);
+    }
+    if (t + 1 < KT) { step(f0, f1); mma(f1); }
+    else mma(f0);
+    }
+  }
+
+  // residual pieces of this thread, requested before the reductions
+  u32x4 rr[C::OPT];
+  if (p.res != nullptr) {
+#pragma unroll
+    for (int q = 0; q < C::OPT; ++q) {
+      const int c = tid + q * 512, srow = c / (BN / 8), ch = c % (BN / 8);
+      rr[q] = (c < C::OPC && srow < rows) ? *reinterpret_cast<const u32x4*>(p.res + (size_t)(m0 + srow) * N + n0 + ch * 8) : u32x4{0, 0, 0, 0};
+    }
+  }
+  float* sMu = reinterpret_cast<float*>(smem + C::LDS);      // [128] mean, [128] 1/std, [BN] x 2
+  float* sRs = sMu + 128;
+  float* sc1 = sRs + 128;
+  float* sc2 = sc1 + BN;
+  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && BM <= 128, "per-row and per-column terms");
+  if (p.ln_part != nullptr) ln_stats.finish(K, p.ln_eps, tid, sMu, sRs, false);
+  if (tid < BN) { sc1[tid] = c1v; sc2[tid] = p.ln_part != nullptr ? c2v : bf16_bits_to_f32(biasv); }
+  __syncthreads();   // the ring is dead: partial sums and the staging tiles reuse it
+
+  // the k-slices meet in LDS: every wave leaves all its tiles and finishes every WK-th of them
+  f32x4* part = reinterpret_cast<f32x4*>(smem);
+  bf16_t* sC = reinterpret_cast<bf16_t*>(smem + C::PART);
+  auto finish = [&](const f32x4 s, int i, int j, int g) {   // four rows of one column of tile (i, j)
+    const int trow = wm * (BM / C::WM) + i * C::MF + (C::MF == 32 ? 8 * g : 0) + 4 * lg, col = wn * (BN / C::WN) + j * C::MF + lr;
+    f32x4 mu = {0.f, 0.f, 0.f, 0.f}, rs = {1.f, 1.f, 1.f, 1.f};
+    if (p.ln_part != nullptr) { mu = *reinterpret_cast<const f32x4*>(sMu + trow); rs = *reinterpret_cast<const f32x4*>(sRs + trow); }
+    const float c1 = sc1[col], c2 = sc2[col];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sC[(trow + e) * C::LDC + col] = (bf16_t)(rs[e] * (s[e] - mu[e] * c1) + c2);
+  };
+  auto group = [&](const Acc& v, int g) { return f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; };
+  if constexpr (C::WK == 1) {
+    if (!producer) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) finish(group(acc[i][j], 0), i, j, 0);
+    }
+  } else {
+    constexpr int UH = TM / C::NH * TN * C::G;           // groups of a pass
+#pragma unroll
+    for (int h = 0; h < C::NH; ++h) {
+      if (h > 0) __syncthreads();
+      if (!producer) {
+#pragma unroll
+        for (int i = 0; i < TM / C::NH; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < C::G; ++g) part[(pw * UH + (i * TN + j) * C::G + g) * 64 + lane] = group(acc[h * (TM / C::NH) + i][j], g);
+      }
+      __syncthreads();
+      if (!producer) {
+#pragma unroll
+        for (int u = 0; u < UH / C::WK; ++u) {
+          const int at = u * C::WK + wk, ij = at / C::G;
+          f32x4 s = part[at * 64 + lane];
+#pragma unroll
+          for (int k = 1; k < C::WK; ++k) {              // slice after slice
+            const f32x4 o = part[(k * UH + at) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] += o[e];
+          }
+          finish(s, h * (TM / C::NH) + ij / TN, ij % TN, at % C::G);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const KhOut yout(p.y, (size_t)M * N * 2);
+  float* sp = reinterpret_cast<float*>(smem);          // row statistics: [BM][BN / 8][2], the partial sums are dead
+#pragma unroll
+  for (int q = 0; q < C::OPT; ++q) {
+    const int c = tid + q * 512, srow = c / (BN / 8), ch = c % (BN / 8);
+    const bool ok = c < C::OPC && srow < rows;
+    u32x4 o = ok ? *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + ch * 8) : u32x4{0, 0, 0, 0};
+    if (p.res != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(bf16_lo(o[e]) + bf16_lo(rr[q][e]), bf16_hi(o[e]) + bf16_hi(rr[q][e]));
+    }
+    if (ok) yout.store16(((size_t)(m0 + srow) * N + n0 + ch * 8) * 2, o);
+    if (!CONV && p.st_part != nullptr) {
+      float ps, pq;
+      kh_piece_sums(o, ps, pq);
+      if constexpr (BN == 128) {                         // the 16 pieces of a row sit in 16 neighbouring lanes
+        ps = kh_row16_sum(ps);
+        pq = kh_row16_sum(pq);
+        if (ch == 0 && ok) kh_ln_store_stats(p.st_part, m0 + srow, M, n_blk, p.n_tiles, ps, pq);
+      } else if (c < C::OPC) {
+        *reinterpret_cast<u32x2*>(sp + 2 * c) = u32x2{__float_as_uint(ps), __float_as_uint(pq)};
+      }
+    }
+    if (CONV && C::ORD != 0 && p.gn_part != nullptr && p.res != nullptr && ok) *reinterpret_cast<u32x4*>(sC + srow * C::LDC + ch * 8) = o;
+  }
+  if (!CONV && BN != 128 && p.st_part != nullptr) {
+    __syncthreads();
+    if (tid < BM && tid < rows) {
+      float s = 0.f, q2 = 0.f;
+#pragma unroll
+      for (int ch = 0; ch < BN / 8; ++ch) { s += sp[2 * (tid * (BN / 8) + ch)]; q2 += sp[2 * (tid * (BN / 8) + ch) + 1]; }
+      kh_ln_store_stats(p.st_part, m0 + tid, M, n_blk, p.n_tiles, s, q2);
+    }
+  }
+  if constexpr (CONV && C::ORD != 0) if (p.gn_part != nullptr) {
+    // GroupNorm statistics as a by-product (LoraGemmParams::gn_part): (sum, sum of squares) of the stored values plus the per-(image,
+    // channel) term over this tile's pixels of one image and whole groups of channels; sums in fixed orders
+    constexpr int PCS = BN / 8, RP = 25;                      // 16-byte pieces per row, row parts (those of the 64 x 160 kernel)
+    float* colp = sp;                                         // [RP][BN][2]
+    float* cols = colp + RP * BN * 2;                         // [BN][2]
+    static_assert((RP * BN * 2 + BN * 2) * 4 <= C::PART, "column sums fit the dead partial sums");
+    const int cg = p.gn_cg, ng = BN / cg, G = N / cg, nrow = rows < BM ? rows : BM;
+    const float ad = (tid < BN && p.gn_add != nullptr) ? (float)p.gn_add[(size_t)seg * N + n0 + tid] : 0.f;
+    __syncthreads();
+    if (tid < RP * PCS) {
+      const int ch = tid % PCS, prt = tid / PCS;
+      float cs[8], cq[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) cs[e] = cq[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < (BM + RP - 1) / RP; ++i) {
+        const int r = prt + i * RP;
+        if (r < nrow) {
+          const u32x4 v = *reinterpret_cast<const u32x4*>(sC + r * C::LDC + ch * 8);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float a = bf16_lo(v[e]), b2 = bf16_hi(v[e]);
+            cs[2 * e] += a; cq[2 * e] = fmaf(a, a, cq[2 * e]);
+            cs[2 * e + 1] += b2; cq[2 * e + 1] = fmaf(b2, b2, cq[2 * e + 1]);
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) *reinterpret_cast<f32x2*>(colp + (prt * BN + ch * 8 + e) * 2) = f32x2{cs[e], cq[e]};
+    }
+    __syncthreads();
+    if (tid < BN) {
+      float s = 0.f, q = 0.f;
+#pragma unroll
+      for (int prt = 0; prt < RP; ++prt) { const f32x2 v = *reinterpret_cast<const f32x2*>(colp + (prt * BN + tid) * 2); s += v[0]; q += v[1]; }
+      *reinterpret_cast<f32x2*>(cols + tid * 2) = f32x2{s + (float)nrow * ad, q + 2.f * ad * s + (float)nrow * ad * ad};
+    }
+    __syncthreads();
+    if (tid < ng) {
+      float s = 0.f, q = 0.f;
+      for (int c = tid * cg; c < (tid + 1) * cg; ++c) { s += cols[2 * c]; q += cols[2 * c + 1]; }
+      *reinterpret_cast<f32x2*>(p.gn_part + (((size_t)seg * G + n0 / cg + tid) * seg_tiles + m_blk % seg_tiles) * 2) = f32x2{s, q};
+    }
+  }
+#endif
+}
+
+template <class C, bool CONV>
+int launch_fine(LoraGemmParams p, hipStream_t stream) {
+  const int seg_rows = CONV ? p.conv_ho * p.conv_wo : p.M;
+  const int seg_tiles = (seg_rows + C::BM - 1) / C::BM;
+  p.m_tiles = p.M / seg_rows * seg_tiles;
+  p.n_tiles = p.N / C::BN;
+  if (p.N % C::BN != 0 || (p.t_nsplit > 0 && p.t_nsplit % C::BN != 0)) return KH_ERR_UNSUPPORTED;
+  if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
+  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
+  // the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
+  double best = 0;
+  p.xg_n = 0;
+  for (int gm = 1; gm <= 8; gm *= 2) {
+    const int gn = 8 / gm;
+    const int rm = (p.m_tiles + gm - 1) / gm, rn = (p.n_tiles + gn - 1) / gn;
+    const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
+    if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
+  }
+  const unsigned grid = 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
+  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
+            seg_rows, seg_tiles);
+  KH_RETURN_LAST_ERROR();
+}
+
+}  // namespace
+
+// Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6).
+//
+// Which of them, for a layer whose sums follow `order`: one that fits one round of the 256 CUs (a workgroup fills a CU, so a second round
+// costs as much as the first), the smaller first; -1 where none does and the larger tiles of the other families win.  A
+// convolution that leaves GroupNorm statistics does so per 64 rows.  Measured, weights cold, us (M, N, K: before -> these):
+// 512 / 1280 / 1280 18.4 -> 9.4 (with row statistics 10.9); 988 / 1280 / 1280 18.5 -> 9.5 (11.4); 2048 / 1280 / 1280 16.5 -> 13.1;
+// 988 / 1280 / 5120 44.3 -> 29.6; 2048 / 1280 / 5120 46.6 -> 40.2; 154 / 1280 / 2048 23.5 -> 12.7; a round too many: 1152 / 1280 /
+// 1280 on 64 x 80 16.0 against 11.7 on 128 x 80.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 32.
+int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
+  const size_t lim = (size_t)1 << 31;
+  const bool conv = p.conv_cin > 0;
+  if (p.geglu || p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return -1;
+  if (p.ldt % 8 != 0 || (size_t)p.N * p.K * 2 >= lim || (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 >= lim) return -1;
+  if (conv) {
+    const size_t xb = ((size_t)(p.M / (p.conv_ho * p.conv_wo)) * p.conv_h + 1) * p.conv_w * p.conv_cin * 2 + 2 * (size_t)p.conv_cin;
+    if (p.conv_cin % 64 != 0 || xb >= lim || p.R > 0) return -1;
+  } else if ((size_t)p.M * p.K * 2 >= lim) {
+    return -1;
+  }
+  const long hw = conv ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
+  auto fits = [&](int bm, int bn) {
+    return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && nb * ((hw + bm - 1) / bm) * (p.N / bn) <= 256;
+  };
+  if (order == 0) return p.st_part != nullptr ? (fits(32, 128) ? 2 : fits(64, 128) ? 3 : -1) : (fits(64, 80) ? 0 : fits(128, 80) ? 1 : -1);
+  if (p.gn_part != nullptr && (p.gn_cg <= 0 || 80 % p.gn_cg != 0 || hw % 64 != 0)) return -1;
+  if (p.gn_part != nullptr ? fits(64, 80) : fits(32, 160)) return p.gn_part != nullptr ? 6 : 4;
+  return fits(64, 160) ? 5 : -1;
+}
+
+int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
+  const bool conv = p.conv_cin > 0;
+  switch (form) {
+    case 0: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 80, 0>, false>(p, stream);
+    case 1: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<128, 80, 0>, false>(p, stream);
+    case 2: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 128, 0>, false>(p, stream);
+    case 3: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 128, 0>, false>(p, stream);
+    case 4: return conv ? launch_fine<FCfg<32, 160, 4>, true>(p, stream) : launch_fine<FCfg<32, 160, 4>, false>(p, stream);
+    case 5: return conv ? launch_fine<FCfg<64, 160, 4>, true>(p, stream) : launch_fine<FCfg<64, 160, 4>, false>(p, stream);
+    case 6: return conv ? launch_fine<FCfg<64, 80, 4>, true>(p, stream) : KH_ERR_UNSUPPORTED;
+    default: return KH_ERR_UNSUPPORTED;
+  }
+}

@@ -1330,6 +1330,7 @@ int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p) {
 int lora_gemm_pipe_launch_conv(const LoraGemmParams& p, hipStream_t stream) {
   if (p.gn_part != nullptr) {   // the caller has asked lora_gemm_conv_gn_row_groups
     const int rg = lora_gemm_conv_gn_row_groups(p);
+    if (const int form = rg == 2 ? lora_gemm_fine_form(p, 4) : -1; form >= 0) return lora_gemm_fine_launch(p, form, stream);
     return rg == 0 ? KH_ERR_UNSUPPORTED : lora_gemm_ksplit_launch_conv(p, rg, stream);
   }
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
@@ -1339,7 +1340,10 @@ int lora_gemm_pipe_launch_conv(const LoraGemmParams& p, hipStream_t stream) {
     // (whole rounds of 128x160 tiles also where 128-column tiles would divide N: the upsamplers' 1280 -> 1280 at 64x64 took
     // 342 us on the 128x128 tiles and takes 249 us on these, 640 -> 640 at 128x128 290 -> 264 us)
     if ((tiles > 256 && tiles <= 384 && m128 * n160 <= 256) || (m128 * n160) % 256 == 0) return lora_gemm_ksplit_launch_conv(p, 4, stream);
-    if (tiles <= 192 && m64 * n160 <= 256 && m64 * n160 > tiles && p.K >= 2560) return lora_gemm_ksplit_launch_conv(p, 2, stream);
+    if (tiles <= 192 && m64 * n160 <= 256 && m64 * n160 > tiles && p.K >= 2560) {
+      const int form = lora_gemm_fine_form(p, 4);   // (-1: images whose partial tiles make it more than one round)
+      return form >= 0 ? lora_gemm_fine_launch(p, form, stream) : lora_gemm_ksplit_launch_conv(p, 2, stream);
+    }
   }
   if (tiles <= 256 && p.conv_cin % 64 == 0) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>, true>(p, stream);
   return launch_pcfg<PCfg<128, 128, 2, 2, 0, 4>, true>(p, stream);
@@ -1369,6 +1373,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     case 40: return lora_gemm_ksplit_launch(p, 2, stream);
     case 41: return lora_gemm_ksplit_launch(p, 4, stream);
     case 42: return lora_gemm_wide_launch(p, stream);
+    case 50: case 51: case 52: case 53: case 54: case 55: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
     default: break;
   }
   // Default choice.  The limiter is the vector L1 path (every operand byte enters LDS through it), so
@@ -1390,11 +1395,15 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     if (p.N % 160 == 0 && lora_gemm_ksplit_ok(p)) {
       const long n160 = p.N / 160;
       if (tiles > 256 && tiles <= 384 && (long)((p.M + 127) / 128) * n160 <= 256) return lora_gemm_ksplit_launch(p, 4, stream);
-      if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560)
-        return lora_gemm_ksplit_launch(p, 2, stream);
+      if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560) {
+        const int form = lora_gemm_fine_form(p, 4);
+        return form >= 0 ? lora_gemm_fine_launch(p, form, stream) : lora_gemm_ksplit_launch(p, 2, stream);
+      }
     }
+    // few enough rows for one round of small tiles
+    if (const int form = lora_gemm_fine_form(p, 0); form >= 0) return lora_gemm_fine_launch(p, form, stream);
     if (tiles >= 480 && p.K >= 1024 && !p.geglu) return deep_stage_ok(p) ? launch_pcfg<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream) : launch_pcfg<PCfg<256, 128, 4, 2, 0, 4>>(p, stream);
-    if (tiles <= 256 && p.M >= 1024 && deep_stage_ok(p)) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
+    if (tiles <= 256 && deep_stage_ok(p)) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
   }
   return launch_prank<128, 128, 2, 2, 4>(p, stream);
 }

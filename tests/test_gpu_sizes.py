@@ -97,3 +97,62 @@ def test_upload_many_sizes():
         for t, a in zip(src, at):
             o = a - buf.data_ptr()
             assert torch.equal(buf[o:o + t.numel()].cpu(), t), sizes
+
+
+@pytest.mark.parametrize("M,N,K,R,r_used", [(1, 640, 64, 0, 0), (31, 640, 128, 32, 16), (64, 1280, 640, 128, 96), (65, 640, 576, 64, 0), (154, 1280, 2048, 0, 0),
+                                            (988, 640, 1280, 128, 0), (1976, 640, 2560, 32, 0), (129, 1280, 5120, 64, 32)])
+def test_fine_tiles_give_the_bits_of_the_large_ones(M, N, K, R, r_used):
+    """Codes 50 .. 53 (64 x 80, 128 x 80, 32 x 128, 64 x 128) add up like the 128 x 128 kernel (16), 54 / 55 (32 x 160, 64 x 160) like the
+    64 x 160 one (40): edges of their rows, K shorter than the ring, rank columns that fill no stage."""
+    from katz_amd import ops
+
+    say("fine tiles", M, N, K, R, r_used)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N)
+    t, bc = (rnd(M, R), rnd(N, R) * 0.05) if R else (None, None)
+    if r_used:
+        t[:, r_used:] = 0
+        bc[:, r_used:] = 0
+    for rs in (None, res):
+        run = (lambda c: ops.lora_linear_pre(x, w, b, t, bc, residual=rs, tile=c, r_used=r_used)) if R else (lambda c: ops.lora_linear(x, w, b, residual=rs, tile=c))
+        for codes, ref in (((50, 51, 52, 53), 16), ((54, 55), 40)):
+            if ref == 40 and R % 64:
+                continue
+            want = run(ref)
+            for c in codes:
+                assert torch.equal(run(c), want), (c, rs is not None)
+    ref = x.double() @ w.double().T + b.double() + (t.double() @ bc.double().T if R else 0)
+    y = ops.lora_linear_pre(x, w, b, t, bc, r_used=r_used) if R else ops.lora_linear(x, w, b)
+    assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3
+
+
+@pytest.mark.parametrize("rows,N,K,stats,fold", [(33, 1280, 640, True, True), (512, 1280, 1280, True, False), (700, 640, 640, True, True), (988, 1280, 1280, False, True),
+                                                 (1100, 1280, 1280, True, True), (200, 1280, 5120, True, False), (1200, 1280, 5120, True, True)])
+def test_fine_tiles_with_folded_norms_do_not_depend_on_the_rows(rows, N, K, stats, fold):
+    """The first rows of a call on as many rows as keep the order of the sums (larger tiles) and a call on them alone: the same
+    results and row statistics, bit for bit."""
+    from katz_amd import ops
+    from katz_amd.lora import fold_norm_into_weight
+
+    say("fine tiles, folded norms", rows, N, K, stats, fold)
+    d = dev()
+    g = torch.Generator().manual_seed(rows + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    M = 2048 if N == 1280 else 6000
+    x, w, b, res = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N)
+    wk, c1, c2 = fold_norm_into_weight(w, b, 1 + 0.1 * rnd(K), 0.1 * rnd(K))
+    st_in = ops.row_stats_buffer(M, d).zero_()
+    st_in[0, :, 0], st_in[0, :, 1] = x.float().sum(1), (x.float() ** 2).sum(1)
+
+    def run(m):
+        st = ops.row_stats_buffer(m, d) if stats else None
+        ln = (st_in[:, :m].contiguous(), c1, c2, None, None, 1e-5) if fold else None
+        y = ops.lora_linear_norm(x[:m], wk if fold else w, None if fold else b, residual=res[:m], ln=ln, stats_out=st)
+        return y, st
+
+    (y, st), (yl, stl) = run(rows), run(M)
+    assert torch.equal(y, yl[:rows])
+    if stats:
+        assert torch.equal(st, stl[:, :rows])
