@@ -112,6 +112,25 @@ __device__ __forceinline__ void kh_prefetch_lines(const void* const (&pf)[3], co
 #endif
 }
 
+// Bring a block of W into this XCD's L2: the 128-byte lines of K columns 64 c0 .. 64 (c0 + nc) of rows row0 .. row0 + rows, thread i of n
+// taking lines i, i + n, ... (loaded like the hint above: into LDS nobody reads).  The workgroups of an XCD that share the block take
+// a share each.  Without it all of them meet the same cold lines at the same time, and a CU takes about 55 GB/s of lines that come from
+// memory, 110 GB/s of lines its L2 has.
+__device__ __forceinline__ void kh_touch_rows(const bf16_t* w, int N, int K, int row0, int rows, int c0, int nc, char* wave_lds, int i, int n) {
+#if __HIP_DEVICE_COMPILE__
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w), 0, (int)((size_t)N * K * 2), 0x00020000);
+  if (row0 + rows > N) rows = N - row0;
+  if (64 * (c0 + nc) > K) nc = K / 64 - c0;
+  for (int l = i; l < rows * nc; l += n) {
+    const int r = l / nc;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)wave_lds, 4,
+                                             (uint32_t)(row0 + r) * (uint32_t)K * 2u + (uint32_t)(c0 + l - r * nc) * 128u, 0, 0, 0);
+  }
+#endif
+}
+// ... from the start of a kernel, where the block is at most 3 MB of the XCD's 4 MB (and W below 2 GiB)
+__device__ __forceinline__ bool kh_touch_pays(int N, int K, int rows) { return (size_t)rows * K * 2 <= (3u << 20) && (size_t)N * K * 2 < (1ull << 31); }
+
 // The same from waves that have nothing else to do (the idle half of an in-launch shrink workgroup): as many rounds as
 // the ranges need, up to 16 (the first range) / 4 (the others), in a loop.
 __device__ __forceinline__ void kh_prefetch_lines_idle(const void* const (&pf)[3], const uint32_t (&lines)[3], char* wave_lds, int wg, int n_wg,

@@ -44,15 +44,19 @@ __device__ __forceinline__ void ring_barrier() {
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
-template <int BM_, int BN_, int ORD_>
+constexpr int GTAB_LO = 0x3800, GTAB_N = 2560;           // gates 2^-15 <= |gate| < 32, per sign
+
+template <int BM_, int BN_, int ORD_, bool GLU_ = false>
 struct FCfg {
   static constexpr int BM = BM_, BN = BN_, ORD = ORD_;
+  static constexpr bool GLU = GLU_;                      // GEGLU epilogue
+  static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : 4, WN = ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
+  static constexpr int WK = ORD == 0 ? 1 : 4, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
   // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
   static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
   static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 0 ? 2 : 1;   // a wave's MFMA tiles, its k-steps per stage
-  static constexpr bool DB = TM * TN * G * 4 <= 96;      // two fragment buffers where the registers allow it
+  static constexpr bool DB = TM * TN * G * 4 <= 96 && !GLU;      // two fragment buffers where the registers allow it
   static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
   static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
   static constexpr int UNITS = ROWS / UR, LPS_LO = UNITS / 4, N_HI = UNITS % 4, LPS_HI = LPS_LO + (N_HI ? 1 : 0);
@@ -60,14 +64,14 @@ struct FCfg {
   static constexpr int LDC = BN + 8;
   // partial sums of the k-slices (NH passes over the row tiles) / row statistics
   static constexpr int NH = WK > 1 && 4 * TM * TN * G > 80 ? 2 : 1;
-  static constexpr int PART = WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
+  static constexpr int PART = GLU ? 0 : WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
   static constexpr int TAIL = PART + BM * LDC * 2;
-  static constexpr int NST = cmin(8, (159 * 1024 - KH_LN_LDS) / STAGE), PD = NST - 1;   // as many stages as fit, but at most 8
-  static constexpr int TOUCH_OFF = cmax(NST * STAGE, TAIL), LDS = TOUCH_OFF + 1024;     // (where prefetched dwords nobody reads land)
+  static constexpr int NST = cmin(8, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;   // as many stages as fit, but at most 8
+  static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + 1024;   // (where prefetched dwords nobody reads land)
   static constexpr int OPC = BM * (BN / 8), OPT = (OPC + 511) / 512;             // 16-byte output pieces: per tile, per thread
   static_assert(WM * WN * WK == 4 && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
   static_assert(BM % 32 == 0 && XQ * UR * 4 == BM && ROWS % UR == 0, "whole DMA instructions");
-  static_assert(NST >= 3 && LPS_HI * (PD - 1) < 63 && LDS + KH_LN_LDS <= 160 * 1024, "ring");
+  static_assert(NST >= 2 && LPS_HI * (PD - 1) < 63 && LDS + KH_LN_LDS <= 160 * 1024, "ring");
 };
 
 // CONV: x is an NHWC image and row m of the GEMM is output pixel m of a 3x3 convolution with padding 1 (K = 9 * Cin ordered
@@ -269,23 +273,26 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
       ring_barrier();
     }
   } else {
-    // The XCD's block of W is contiguous rows: its workgroups fetch it into their L2 between them, a line a lane,
-    // before the K loop meets it.  In the loop all of them ask for the same lines at the same time, and a CU takes about 55 GB/s
-    // of lines that come from memory, 110 GB/s of lines that its L2 has (M 988, N 1280, K 1280: 10.4 -> 9.4 us; 128 x 80 tiles
-    // at M 2048, K 5120: 39.9 -> 37.0; x, which the launch in front has just written, is not worth it).
-    const int nloc = p.xr_m * p.xr_n;
-    auto touch = [&](const void* base, size_t bytes_total, size_t first_byte, size_t bytes) {
-      const rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes_total, 0x00020000);
-      const uint32_t lines = (uint32_t)(bytes >> 7);
-      for (uint32_t l = (uint32_t)(local * 256 + tid); l < lines; l += (uint32_t)nloc * 256u)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(smem + C::TOUCH_OFF + pw * 256), 4, (uint32_t)first_byte + (l << 7), 0, 0, 0);
+    // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
+    // 9.4 us; 64 x 160 tiles at K 5120 42.7 -> 33.2; x, which the launch in front has just written, is not worth it)
+    auto touch = [&](int t, int n) {
+      if (t < KT1)
+        kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
     };
-    const int nf = (xcd % p.xg_n) * p.xr_n * BN, nr = (nf + p.xr_n * BN < N ? nf + p.xr_n * BN : N) - nf;
-    touch(p.w, (size_t)N * K * 2, (size_t)nf * K * 2, (size_t)nr * K * 2);
+    touch(0, 24);
+    uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
+    if constexpr (C::GLU) {
+#pragma unroll 4
+      for (int i = tid; i < 2 * GTAB_N; i += 256) {
+        const uint32_t bits = (uint32_t)(i >= GTAB_N ? 0x8000 + (i - GTAB_N) : i) + GTAB_LO;
+        gtab[i] = (uint16_t)pack_bf16x2(kh_gelu_erf(bf16_lo(bits)), 0.f);
+      }
+    }
     ring_barrier();
     int st = 0;
     if constexpr (!C::DB) {
       for (int t = 0; t < KT; ++t) {
+        if ((t & 7) == 0) touch(t + 24, 8);
         Fr f;
         read_frags(st, f);
         mma(f);
@@ -304,6 +311,7 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
     };
     int t = 0;
     for (; t + 2 < KT; t += 2) {
+      if ((t & 7) == 0) touch(t + 24, 8);
       step(f0, f1);
       step(f1, f0);
     }
@@ -380,6 +388,40 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
     }
   }
   __syncthreads();
+  if constexpr (C::GLU) {
+    // staged columns come in groups of 64 = 32 value columns then their 32 gate columns
+    constexpr int OPR = BN / 16, GCH = (BM * OPR + 511) / 512;
+    const int out_ld = N / 2;
+    const KhOut gout(p.y, (size_t)M * out_ld * 2);
+    const uint16_t* gtab = reinterpret_cast<const uint16_t*>(smem + C::TAB_OFF);
+#pragma unroll
+    for (int q = 0; q < GCH; ++q) {
+      const int c = tid + q * 512, srow = c / OPR, oc = c % OPR, grp = oc >> 2, sub = oc & 3;
+      if (c >= BM * OPR || srow >= rows) continue;
+      const u32x4 hv = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + grp * 64 + sub * 8);
+      const u32x4 gv = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + grp * 64 + 32 + sub * 8);
+      u32x4 ar;                                            // gelu(gate) rounded to bf16 before the product
+      bool outside = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t lo = gv[e] & 0xffffu, hi = gv[e] >> 16;
+        const uint32_t olo = (lo & 0x7fffu) - GTAB_LO, ohi = (hi & 0x7fffu) - GTAB_LO;
+        outside = outside || olo >= (uint32_t)GTAB_N || ohi >= (uint32_t)GTAB_N;
+        const uint32_t ilo = (olo < (uint32_t)GTAB_N ? olo : 0u) + (lo >> 15) * GTAB_N;
+        const uint32_t ihi = (ohi < (uint32_t)GTAB_N ? ohi : 0u) + (hi >> 15) * GTAB_N;
+        ar[e] = (uint32_t)gtab[ilo] | ((uint32_t)gtab[ihi] << 16);
+      }
+      if (outside) {                                       // tiny, huge or non-finite gates: evaluate directly
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ar[e] = pack_bf16x2(kh_gelu_erf(bf16_lo(gv[e])), kh_gelu_erf(bf16_hi(gv[e])));
+      }
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(bf16_lo(hv[e]) * bf16_lo(ar[e]), bf16_hi(hv[e]) * bf16_hi(ar[e]));
+      gout.store16(((size_t)(m0 + srow) * out_ld + (n0 >> 1) + grp * 32 + sub * 8) * 2, o);
+    }
+    return;
+  }
   const KhOut yout(p.y, (size_t)M * N * 2);
   float* sp = reinterpret_cast<float*>(smem);          // row statistics: [BM][BN / 8][2], the partial sums are dead
 #pragma unroll
@@ -488,18 +530,20 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
 
 }  // namespace
 
-// Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6).
+// Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
+// GEGLU on 64 x 320 (7), 128 x 320 (8).
 //
 // Which of them, for a layer whose sums follow `order`: one that fits one round of the 256 CUs (a workgroup fills a CU, so a second round
 // costs as much as the first), the smaller first; -1 where none does and the larger tiles of the other families win.  A
 // convolution that leaves GroupNorm statistics does so per 64 rows.  Measured, weights cold, us (M, N, K: before -> these):
 // 512 / 1280 / 1280 18.4 -> 9.4 (with row statistics 10.9); 988 / 1280 / 1280 18.5 -> 9.5 (11.4); 2048 / 1280 / 1280 16.5 -> 13.1;
 // 988 / 1280 / 5120 44.3 -> 29.6; 2048 / 1280 / 5120 46.6 -> 40.2; 154 / 1280 / 2048 23.5 -> 12.7; a round too many: 1152 / 1280 /
-// 1280 on 64 x 80 16.0 against 11.7 on 128 x 80.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 32.
+// 1280 on 64 x 80 16.0 against 11.7 on 128 x 80.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 31.
+// GEGLU: 512 / 10240 / 1280 30.6 -> 23.6, 988 / 10240 / 1280 48.5 -> 34.3, 2048 / 5120 / 640 28.0 -> 22.3.
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   const size_t lim = (size_t)1 << 31;
   const bool conv = p.conv_cin > 0;
-  if (p.geglu || p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return -1;
+  if (p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return -1;
   if (p.ldt % 8 != 0 || (size_t)p.N * p.K * 2 >= lim || (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 >= lim) return -1;
   if (conv) {
     const size_t xb = ((size_t)(p.M / (p.conv_ho * p.conv_wo)) * p.conv_h + 1) * p.conv_w * p.conv_cin * 2 + 2 * (size_t)p.conv_cin;
@@ -511,6 +555,10 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   auto fits = [&](int bm, int bn) {
     return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && nb * ((hw + bm - 1) / bm) * (p.N / bn) <= 256;
   };
+  if (p.geglu) {   // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
+    if (order != 0 || p.st_part != nullptr || p.res != nullptr) return -1;
+    return fits(64, 320) ? (hw + 63) / 64 * (p.N / 320) > 128 ? 7 : -1 : fits(128, 320) ? 8 : -1;
+  }
   if (order == 0) return p.st_part != nullptr ? (fits(32, 128) ? 2 : fits(64, 128) ? 3 : -1) : (fits(64, 80) ? 0 : fits(128, 80) ? 1 : -1);
   if (p.gn_part != nullptr && (p.gn_cg <= 0 || 80 % p.gn_cg != 0 || hw % 64 != 0)) return -1;
   if (p.gn_part != nullptr ? fits(64, 80) : fits(32, 160)) return p.gn_part != nullptr ? 6 : 4;
@@ -519,6 +567,7 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
 
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
   const bool conv = p.conv_cin > 0;
+  if (p.geglu && form < 7) return KH_ERR_UNSUPPORTED;
   switch (form) {
     case 0: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 80, 0>, false>(p, stream);
     case 1: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<128, 80, 0>, false>(p, stream);
@@ -527,6 +576,8 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 4: return conv ? launch_fine<FCfg<32, 160, 4>, true>(p, stream) : launch_fine<FCfg<32, 160, 4>, false>(p, stream);
     case 5: return conv ? launch_fine<FCfg<64, 160, 4>, true>(p, stream) : launch_fine<FCfg<64, 160, 4>, false>(p, stream);
     case 6: return conv ? launch_fine<FCfg<64, 80, 4>, true>(p, stream) : KH_ERR_UNSUPPORTED;
+    case 7: return p.geglu ? launch_fine<FCfg<64, 320, 0, true>, false>(p, stream) : KH_ERR_UNSUPPORTED;
+    case 8: return p.geglu ? launch_fine<FCfg<128, 320, 0, true>, false>(p, stream) : KH_ERR_UNSUPPORTED;
     default: return KH_ERR_UNSUPPORTED;
   }
 }

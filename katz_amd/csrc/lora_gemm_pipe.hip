@@ -722,6 +722,12 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lora_gemm_pipe_kernel(const Lor
   if (m0 >= p.M) return;   // segmented launches size the grid for the longest segment
   const int K = p.K, M = p.M, N = p.N;
   constexpr int BKP = C::BKP, ROWB = C::ROWB;
+  // the XCD's block of W into its L2 (into LDS that this wave's own first loads overwrite afterwards), by at least half its CUs: 988 /
+  // 3840 / 1280 18.3 -> 16.6 us (the other instantiations have no registers for it or gain nothing)
+  if (!IL && !CONV && LNF != 3 && !XA && BM == 128 && BN == 128 && C::NT == 512 && p.grp == nullptr && p.sg_mode == 0 &&
+      p.xr_m * p.xr_n >= 16 && kh_touch_pays(N, K, p.xr_n * BN))
+    kh_touch_rows(p.w, N, K, (bid & 7) % p.xg_n * p.xr_n * BN, p.xr_n * BN, 0, K / 64, smem + wave * (C::UX / C::NW) * 1024,
+                  (bid >> 3) * C::NT + tid, p.xr_m * p.xr_n * C::NT);
   // folded LayerNorm: mean and 1/std of this tile's x rows, read in the epilogue (the barriers of the K loop lie between)
   // and the two per-column terms of this (single) column tile
   float* sMu = reinterpret_cast<float*>(smem + p.ln_lds);
@@ -1373,7 +1379,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     case 40: return lora_gemm_ksplit_launch(p, 2, stream);
     case 41: return lora_gemm_ksplit_launch(p, 4, stream);
     case 42: return lora_gemm_wide_launch(p, stream);
-    case 50: case 51: case 52: case 53: case 54: case 55: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
+    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
     default: break;
   }
   // Default choice.  The limiter is the vector L1 path (every operand byte enters LDS through it), so

@@ -156,3 +156,20 @@ def test_fine_tiles_with_folded_norms_do_not_depend_on_the_rows(rows, N, K, stat
     assert torch.equal(y, yl[:rows])
     if stats:
         assert torch.equal(st, stl[:, :rows])
+
+
+@pytest.mark.parametrize("M,N,K,R", [(65, 2560, 640, 0), (988, 10240, 1280, 64), (577, 10240, 640, 0), (2048, 5120, 640, 128), (129, 10240, 64, 0)])
+def test_fine_geglu_tiles(M, N, K, R):
+    """64 x 320 and 128 x 320 tiles with the GEGLU epilogue (codes 57, 58) against the 128 x 128 kernel, bit for bit."""
+    from katz_amd import ops
+
+    say("fine geglu", M, N, K, R)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b = rnd(M, K), rnd(N, K) * 0.2, rnd(N)
+    t, bc = (rnd(M, R), rnd(N, R) * 0.05) if R else (None, None)
+    run = (lambda c: ops.lora_linear_pre(x, w, b, t, bc, geglu=True, tile=c)) if R else (lambda c: ops.lora_linear(x, w, b, geglu=True, tile=c))
+    want = run(16)
+    for c in (57, 58, 0):
+        assert torch.equal(run(c), want), c
