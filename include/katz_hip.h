@@ -400,6 +400,48 @@ int kh_conv_out_cfg_euler_bf16(const void* x, const void* w, const void* bias, c
                                void* model_input_next, void* noise_pred_out, int64_t Bl, int64_t H, int64_t W,
                                int64_t Cin, float guidance_scale, const float* coef, int latents_f32, void* stream);
 
+/* ---- One transformer block per call -----------------------------------------------------------------------
+ * BasicTransformerBlock.forward (diffusers-hf/src/diffusers/models/attention.py:283-403, layer_norm variant): self-attention,
+ * cross-attention, feed-forward, each behind a LayerNorm and with its residual, as the launches of the entry points above in
+ * that order.  The descriptor holds what stays the same from call to call (HOST memory, device pointers inside); the caller
+ * rebuilds it when an operand moves.
+ *
+ * KhLinearDesc: the operands of one LoRA linear as kh_lora_linear_split_bf16 / kh_lora_linear_norm_bf16 take them (R 0: no
+ * adapters; c1 / c2 / ca1 / ca2 / eps: the folded LayerNorm in front, NULL without).  hint_weight: 1 if the launch before this
+ * one should touch the weights (kh_set_weight_prefetch), beside the adapter matrices.
+ * KhBlockDesc: qkv stacks to_q / to_k / to_v of the self-attention; q2.w NULL: no cross-attention.  folded: the norms are part
+ * of qkv, q2 and geglu (whose operands carry them) and `stats` passes the row statistics from linear to linear; otherwise
+ * n1 .. n3 are launches of their own.  fuse_xattn: run the cross-attention inside the query projection where
+ * kh_lora_linear_xattn_ok allows.  heads * 64 = width of the attentions.
+ * KhBlockCall: x, y bf16 [B,T,C]; ctx bf16 [B,S,K of k2] projected here, or NULL and k / v with their row strides ldk / ldv and
+ * sample strides bsk / bsv (elements).  stats: as kh_lora_linear_norm_bf16 (folded only), valid for x on entry; `last`: not
+ * written for y.  flags: bits 8 (shrink as a launch of its own) and 24 of the linears' flags.  hints: issue
+ * kh_set_weight_prefetch inside the chain; tail_hint: up to three (address, bytes) for the launch after the block.
+ * workspace / counters: at least what kh_transformer_block_needs reports; counters zero when the call is enqueued. */
+typedef struct {
+  const void *w, *bias, *a_cat, *b_cat;
+  const float *col_scale, *c1, *c2, *ca1, *ca2;
+  int64_t N, K, R, n_split, r_used, geglu, hint_weight;
+  double eps;
+} KhLinearDesc;
+typedef struct {
+  KhLinearDesc qkv, out1, k2, v2, q2, out2, geglu, ff;
+  const void *n1_w, *n1_b, *n2_w, *n2_b, *n3_w, *n3_b;
+  double n1_eps, n2_eps, n3_eps, scale1, scale2;
+  int64_t heads, folded, fuse_xattn;
+} KhBlockDesc;
+typedef struct {
+  const void *x, *ctx, *k, *v;
+  void *y, *workspace;
+  int32_t* counters;
+  float* stats;
+  int64_t B, T, S, ldk, ldv, bsk, bsv, workspace_bytes, counter_ints, flags, hints, last;
+  uint64_t tail_hint[6];
+} KhBlockCall;
+int kh_transformer_block_needs(const KhBlockDesc* desc, int64_t B, int64_t T, int64_t S, int own_kv, int64_t* workspace_bytes,
+                               int64_t* counter_ints);
+int kh_transformer_block_bf16(const KhBlockDesc* desc, const KhBlockCall* call, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

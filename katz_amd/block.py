@@ -1,0 +1,313 @@
+"""BasicTransformerBlock.forward as one call into the library (kh_transformer_block_bf16).
+
+A block is ten launches of 3 us of host time each; through the single wrappers (checks, allocations, module calls) the same
+block costs 230 us, more than its GPU time for images up to 768 x 768.  What stays the same between calls (operand addresses,
+shapes, flags) is laid out once per block in a KhBlockDesc and used as long as every tensor, pack, module, hook and option it
+was made from is still the one in place; `run` gives None whenever the block has to take the path through its modules
+(other processors, hooks, formats the descriptor does not cover, call accounting).
+"""
+from __future__ import annotations
+
+import ctypes
+import operator
+import weakref
+from ctypes import c_double, c_int64, c_uint64, c_void_p
+
+import torch
+from torch import nn
+
+from . import _lib, layers, ops
+
+
+class _Linear(ctypes.Structure):   # KhLinearDesc
+    _fields_ = ([(n, c_uint64) for n in ("w", "bias", "a_cat", "b_cat", "col_scale", "c1", "c2", "ca1", "ca2")]
+                + [(n, c_int64) for n in ("N", "K", "R", "n_split", "r_used", "geglu", "hint_weight")] + [("eps", c_double)])
+
+
+class _Block(ctypes.Structure):    # KhBlockDesc
+    _fields_ = ([(n, _Linear) for n in ("qkv", "out1", "k2", "v2", "q2", "out2", "geglu", "ff")]
+                + [(n, c_uint64) for n in ("n1_w", "n1_b", "n2_w", "n2_b", "n3_w", "n3_b")]
+                + [(n, c_double) for n in ("n1_eps", "n2_eps", "n3_eps", "scale1", "scale2")]
+                + [(n, c_int64) for n in ("heads", "folded", "fuse_xattn")])
+
+
+class _Call(ctypes.Structure):     # KhBlockCall
+    _fields_ = ([(n, c_void_p) for n in ("x", "ctx", "k", "v", "y", "workspace", "counters", "stats")]
+                + [(n, c_int64) for n in ("B", "T", "S", "ldk", "ldv", "bsk", "bsv", "workspace_bytes", "counter_ints", "flags", "hints", "last")]
+                + [("tail_hint", c_uint64 * 6)])
+
+
+_addr = lambda t: 0 if t is None else t.data_ptr()
+
+
+def _options():
+    return layers.LN_FOLD, layers.XATTN_FUSE, layers.LORA_MODE, ops.WEIGHT_PREFETCH, ops.PREFETCH_MIN_K, ops.PREFETCH_SMALL_BYTES
+
+
+class _Watch:
+    """dicts[i].get(keys[i]) has to be objects[i]."""
+
+    def __init__(self):
+        self.dicts, self.keys, self.objects = [], [], []
+
+    def expect(self, owner: dict, key: str):
+        v = owner.get(key)
+        self.dicts.append(owner)
+        self.keys.append(key)
+        self.objects.append(v)
+        return v
+
+    def holds(self) -> bool:
+        return all(map(operator.is_, map(dict.get, self.dicts, self.keys), self.objects))
+
+
+class _Plan:
+    """The descriptor of a block without adapters, and the modules, parameters and options that it was made from.  The packed
+    adapters change without these whenever a server turns to another request: they are added by _Ready."""
+
+    def __init__(self, blk, folded: bool):
+        self.options = _options()
+        self.watch = _Watch()
+        self.tensors = []                                  # parameters: same version, same address
+        self.hooks = []                                    # hook tables that have to be empty
+        self.keep = []                                     # what the addresses in the descriptor belong to
+        self.linears = []                                  # (entry, layer, LayerNorm folded into it)
+        self.ready = None
+        self.desc = _Block()
+        self.seen(blk, "norm1", "attn1", "norm2", "attn2", "norm3", "ff")
+        self.usable = self.describe(blk, folded)
+        self.versions = [t._version for t in self.tensors]
+        self.addresses = [t.data_ptr() for t in self.tensors]
+
+    def holds(self) -> bool:
+        return (self.options == _options() and self.watch.holds() and [t._version for t in self.tensors] == self.versions
+                and [t.data_ptr() for t in self.tensors] == self.addresses)
+
+    def seen(self, module, *children, params=(), plain=()):
+        """Watch a module's children, parameters, plain attributes and hooks."""
+        d, expect = module.__dict__, self.watch.expect
+        expect(d, "forward")
+        self.hooks += [module._forward_hooks, module._forward_pre_hooks]
+        for n in children:
+            expect(d["_modules"], n)
+        for n in params:
+            t = expect(d["_parameters"], n)
+            if t is not None:
+                self.tensors.append(t)
+        for n in plain:
+            expect(d, n)
+
+    def linear(self, name: str, l, norm=None, stats=False) -> bool:
+        """norm: the LayerNorm folded into this layer; stats: it leaves row statistics."""
+        if type(l) is not layers.LoRALinear:
+            return False
+        l.prepare()
+        self.seen(l, params=("weight", "bias"), plain=("_rt", "geglu"))
+        _, w, b = l._rt
+        if (w.dtype != torch.bfloat16 or not w.is_cuda or not w.is_contiguous() or (b is not None and not b.is_contiguous())
+                or l.in_features % 64 or l.out_features % 8 or (b is not None and b.dtype != torch.bfloat16)
+                or (stats and l.out_features > 128 * ops.LN_SLOTS)):
+            return False
+        d = getattr(self.desc, name)
+        d.N, d.K, d.geglu = l.out_features, l.in_features, int(l.geglu)
+        c1 = c2 = None
+        if norm is not None:
+            w, c1, c2 = l._ln_terms(norm)[:3]
+            b, d.eps = None, norm.eps
+        self.keep.append(self.weights(d, w, b, c1, c2))
+        self.linears.append((name, l, norm))
+        return True
+
+    def weights(self, d: _Linear, w, b, c1, c2):
+        d.w, d.bias, d.c1, d.c2 = w.data_ptr(), _addr(b), _addr(c1), _addr(c2)
+        d.hint_weight = int(d.K >= ops.PREFETCH_MIN_K or w.numel() * 2 <= ops.PREFETCH_SMALL_BYTES)
+        return w, b, c1, c2
+
+    def describe(self, blk, folded: bool) -> bool:
+        d = self.desc
+        a1, a2, ff = blk.attn1, blk.attn2, blk.ff
+        norms = (blk.norm1, blk.norm2, blk.norm3)
+        if type(a1) is not layers.Attention or type(a2) not in (layers.Attention, type(None)) or type(ff) is not layers.FeedForward:
+            return False
+        for a in (a1,) if a2 is None else (a1, a2):
+            self.seen(a, "to_q", "to_k", "to_v", "to_out", plain=("processor", "heads", "scale", "is_cross"))
+            drop = a.to_out[1] if len(a.to_out) == 2 else None
+            self.seen(a.to_out, "0", "1")
+            if type(a.processor) is not layers.KatzAttnProcessor or type(drop) is not nn.Dropout or drop.p != 0.0:
+                return False
+            self.seen(drop, plain=("p",))
+        geglu = ff.net[0]
+        self.seen(ff, "net")
+        self.seen(ff.net, "0", "2")
+        if type(geglu) is not layers.GEGLU or geglu.enable_fused_geglu:
+            return False
+        self.seen(geglu, "proj", plain=("enable_fused_geglu",))
+        if a1.is_cross or (a2 is not None and (not a2.is_cross or a2.heads != a1.heads)) or (folded and not layers.LN_FOLD):
+            return False
+        for i, n in enumerate(norms):
+            if n is None:
+                continue
+            if type(n) is not layers.LayerNorm or n.weight.dtype != torch.bfloat16 or n.bias.dtype != torch.bfloat16:
+                return False
+            self.seen(n, params=("weight", "bias"), plain=("eps",))
+            for name, v in ((f"n{i + 1}_w", n.weight.data_ptr()), (f"n{i + 1}_b", n.bias.data_ptr()), (f"n{i + 1}_eps", n.eps)):
+                setattr(d, name, v)
+        fold = norms if folded else (None,) * 3
+        # q | k | v of the self-attention: the operands fused_qkv stacks
+        q = d.qkv
+        self.attn1, self.norm1 = a1, fold[0]
+        for l in (a1.to_q, a1.to_k, a1.to_v):
+            if type(l) is not layers.LoRALinear or l.weight.dtype != torch.bfloat16 or not l.weight.is_cuda:
+                return False
+            l.prepare()
+            self.seen(l, params=("weight", "bias"), plain=("_rt",))
+        if folded:
+            q.eps = norms[0].eps
+        q.N, q.K = 3 * a1.to_q.out_features, a1.to_q.in_features
+        self.inner = N = a1.to_q.out_features
+        if N != a1.heads * 64 or any(l.out_features != N or l.in_features != q.K for l in (a1.to_k, a1.to_v)):
+            return False
+        if not (self.linear("out1", a1.to_out[0], stats=folded) and self.linear("geglu", geglu.proj, fold[2])
+                and self.linear("ff", ff.net[2], stats=folded)):
+            return False
+        if a2 is not None and not (self.linear("q2", a2.to_q, fold[1]) and self.linear("k2", a2.to_k) and self.linear("v2", a2.to_v)
+                                   and self.linear("out2", a2.to_out[0], stats=folded)):
+            return False
+        if d.geglu.geglu != 1 or d.ff.K * 2 != d.geglu.N or d.ff.N != q.K or d.out1.N != q.K or d.out1.K != N:
+            return False
+        if a2 is not None and (d.q2.N != N or d.q2.K != q.K or d.k2.N != N or d.v2.N != N or d.k2.K != d.v2.K or d.out2.K != N or d.out2.N != q.K):
+            return False
+        d.heads, d.scale1, d.scale2 = a1.heads, a1.scale, a1.scale if a2 is None else a2.scale
+        d.folded, d.fuse_xattn = int(folded), int(layers.XATTN_FUSE)
+        self.width, self.cross, self.kv_width = q.K, a2 is not None, d.k2.K
+        self.last_key = int(d.ff.w)
+        return True
+
+
+class _Ready:
+    """A plan's descriptor with the packs that are in place now.  Made anew when they change and never written to after that:
+    another thread may be inside the library with the previous one."""
+
+    def __init__(self, plan: _Plan):
+        self.epoch, self.packs = layers._pack_epoch, _Watch()
+        self.sizes = {}                                    # (B, T, S, own_kv) -> (workspace bytes, counters)
+        self.keep = []
+        self.desc = _Block.from_buffer_copy(plan.desc)
+        self.at = ctypes.addressof(self.desc)
+        self.usable = self.fill(plan)
+
+    def holds(self) -> bool:
+        return self.epoch == layers._pack_epoch and self.packs.holds()
+
+    def fill(self, plan) -> bool:
+        expect, keep = self.packs.expect, self.keep
+        attn = plan.attn1
+        st = attn._qkv_state()
+        for l in (attn.to_q, attn.to_k, attn.to_v):
+            p = expect(l.__dict__, "_packed")
+            if p is not None:
+                expect(p.__dict__, "a_cat")
+        split = layers.LORA_MODE == "split"
+        for name, l, norm in plan.linears:
+            p = expect(l.__dict__, "_packed")
+            if p is None:
+                continue
+            if p.overflow or not split:
+                return False
+            v = p.__dict__
+            a, b, s = expect(v, "a_cat"), expect(v, "b_cat"), expect(v, "col_scale")
+            ca1 = ca2 = None
+            if norm is not None:
+                a, ca1, ca2 = l._ln_terms(norm)[3:]
+            self.operands(getattr(self.desc, name), a, b, s, ca1, ca2, p.r_used)
+        if st is None:
+            return False
+        q, norm = self.desc.qkv, plan.norm1
+        w, c1, c2, a, ca1, ca2 = attn._qkv_folded(st, norm) if norm is not None else (st["w"], None, None, st.get("a"), None, None)
+        keep.append(plan.weights(q, w, None, c1, c2))
+        refs = (w, None, None)
+        if st["R"]:
+            self.operands(q, a, st["b"], st["s"], ca1, ca2, st["r_used"])
+            q.n_split = plan.inner
+            refs = (w, a, st["b"])
+        self.first = tuple(None if t is None else weakref.ref(t) for t in refs)
+        self.first_key = int(q.w)
+        return True
+
+    def operands(self, d: _Linear, a, b, s, ca1, ca2, r_used: int):
+        d.a_cat, d.b_cat, d.col_scale, d.ca1, d.ca2 = a.data_ptr(), b.data_ptr(), s.data_ptr(), _addr(ca1), _addr(ca2)
+        d.R, d.r_used = b.shape[1], r_used
+        self.keep.append((a, b, s, ca1, ca2))
+
+    def needs(self, B, T, S, own_kv):
+        key = (B, T, S, own_kv)
+        got = self.sizes.get(key)
+        if got is None:
+            ws, n = c_int64(), c_int64()
+            _lib.check(_lib.load().kh_transformer_block_needs(self.at, B, T, S, int(own_kv), ctypes.byref(ws), ctypes.byref(n)), "kh_transformer_block_needs")
+            if len(self.sizes) >= 64:
+                self.sizes.clear()
+            got = self.sizes[key] = (ws.value, n.value)
+        return got
+
+
+_plans: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()   # block -> [plan with separate norms, plan with folded norms]
+_global_hooks = (nn.modules.module._global_forward_hooks, nn.modules.module._global_forward_pre_hooks)
+
+
+def run(blk, h, ctx, stats, last: bool):
+    """The block on h, or None: take the path through the modules.  Arguments as BasicTransformerBlock.forward's."""
+    if (ops.CALL_LOG is not None or not h.is_cuda or h.dtype != torch.bfloat16 or h.dim() != 3 or not h.is_contiguous()
+            or (stats is not None and not stats.valid) or _global_hooks[0] or _global_hooks[1]):
+        return None
+    folded = stats is not None
+    both = _plans.get(blk)
+    if both is None:
+        both = _plans[blk] = [None, None]
+    plan = both[folded]
+    if plan is None or not plan.holds():
+        plan = both[folded] = _Plan(blk, folded)
+    if not plan.usable or any(plan.hooks):
+        return None
+    ready = plan.ready
+    if ready is None or not ready.holds():
+        ready = plan.ready = _Ready(plan)
+    if not ready.usable:
+        return None
+    B, T, C = h.shape
+    if C != plan.width or (ctx is not None) != plan.cross or (folded and stats.buf.numel() != B * T * ops.LN_SLOTS * 2):
+        return None
+    call = _Call()
+    S, own_kv = 0, False
+    if plan.cross:
+        kv = blk.attn2.ctx_kv
+        if kv is not None and kv[0] is ctx:
+            _, k, v = kv
+            S = k.shape[1]
+            if k.shape != (B, S, plan.inner) or v.shape != k.shape or k.stride(2) != 1 or v.stride(2) != 1 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
+                return None
+            call.k, call.v = k.data_ptr(), v.data_ptr()
+            call.bsk, call.ldk, _ = k.stride()
+            call.bsv, call.ldv, _ = v.stride()
+        else:
+            if not ctx.is_cuda or ctx.dtype != torch.bfloat16 or ctx.dim() != 3 or not ctx.is_contiguous() or ctx.shape[0] != B or ctx.shape[2] != plan.kv_width:
+                return None
+            S, own_kv = ctx.shape[1], True
+            call.ctx = ctx.data_ptr()
+    nbytes, ints = ready.needs(B, T, S, own_kv)
+    y = torch.empty_like(h)
+    ws = h.new_empty((nbytes,), dtype=torch.uint8)
+    call.x, call.y, call.workspace, call.workspace_bytes = h.data_ptr(), y.data_ptr(), ws.data_ptr(), nbytes
+    if ints:
+        call.counters, call.counter_ints = ops._arena_ints(h.device, ints).data_ptr(), ints
+    if folded:
+        call.stats = stats.buf.data_ptr()
+    call.B, call.T, call.S, call.last = B, T, S, int(last)
+    call.flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_coop_bit()
+    ranges = ops.chain_hints(ready.first_key, ready.first, plan.last_key)
+    if ranges is not None:
+        call.hints = 1
+        for i, r in enumerate(ranges):
+            call.tail_hint[2 * i], call.tail_hint[2 * i + 1] = r
+    _lib.check(_lib.load().kh_transformer_block_bf16(ready.at, ctypes.addressof(call), ops._stream()), "kh_transformer_block_bf16")
+    return y

@@ -14,6 +14,7 @@ from __future__ import annotations
 import os
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
@@ -51,6 +52,11 @@ XATTN_FUSE = os.getenv("KATZ_XATTN_FUSE", "1") != "0"
 # epilogue (kh_conv3x3_gn_stats_nhwc_bf16), so that norm is one launch instead of two.  "0": convolution, then the norm's
 # two launches (for measurements).
 CONV_GN_FUSE = os.getenv("KATZ_CONV_GN_FUSE", "1") != "0"
+
+
+# A transformer block runs from one call into the library (kh_transformer_block_bf16) where its modules are the plain ones.
+# "0": every module calls its own entry points (for measurements).
+BLOCK_CALL = os.getenv("KATZ_BLOCK_CALL", "1") != "0"
 
 
 class RowStats:
@@ -121,7 +127,7 @@ class LoRALinear(nn.Module):
     def assign_active(self, names: Sequence[str], weights: Optional[Sequence[float]] = None) -> None:
         """set_active without the rebuild: refresh_many does that for many layers at once."""
         ads = self.adapters
-        self.active = [n for n in names if n in ads]
+        self.__dict__["active"] = [n for n in names if n in ads]
         if weights is not None:
             for n, w in zip(names, weights):
                 if n in ads:
@@ -373,7 +379,8 @@ def refresh_many(modules) -> None:
     for todo in build.values():
         todo.sort(key=lambda e: e[0]._context if e[0]._context else 1 << 30)   # context projections first, one width behind the other
         for (m, _, key), p in zip(todo, pack_many([e[0] for e in todo], [e[1] for e in todo])):
-            m._packed, m._packed_key = p, key
+            d = m.__dict__   # plain attributes: Module.__setattr__ looks through parameters, buffers and submodules first
+            d["_packed"], d["_packed_key"] = p, key
         _pack_epoch += 1
 
 
@@ -858,14 +865,11 @@ class Attention(nn.Module):
         self._qkv_w = None  # (key, stacked weights): they outlive a change of adapters
         self._qkv_ln = None # (key, W', c1, c2): the stacked weights with the norm in front folded in
 
-    def fused_qkv(self, x: torch.Tensor, ln=None):
-        """to_q / to_k / to_v of a self-attention as ONE GEMM over the stacked weights ([3N,K]: three
-        times the workgroups of a single projection, which alone covers 160 of 256 CUs) and, with
-        adapters, ONE shrink over the stacked A matrices.  Returns (q, k, v) as column views of the
-        [.., 3N] result, or None when the layers cannot be fused (then they run one by one)."""
+    def _qkv_state(self):
+        """The stacked operands of to_q / to_k / to_v (a dict), or None when the layers cannot be fused; rebuilt when a weight
+        or a pack changes."""
         layers = (self.to_q, self.to_k, self.to_v)
-        N, K = self.to_q.out_features, self.to_q.in_features
-        if self.is_cross or x.dtype != torch.bfloat16 or N % 128 != 0 or K % 64 != 0:
+        if self.is_cross or self.to_q.out_features % 128 != 0 or self.to_q.in_features % 64 != 0:
             return None
         for l in layers:
             l.prepare()
@@ -891,29 +895,43 @@ class Attention(nn.Module):
                         st["b"] = cat(bc)
                     if st["a"] is None or st["s"] is None:
                         st["a"], st["s"] = cat(a), cat(sc)
-                    for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
-                        p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
+                        for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
+                            p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
             self._qkv = st
-        if not st["ok"]:
+        return st if st["ok"] else None
+
+    def _qkv_folded(self, st: dict, norm: "LayerNorm"):
+        """(W', c1, c2, A', ca1, ca2) of the stacked projections behind `norm` (lora.fold_layer_norm)."""
+        key = norm_key(norm)
+        sig = st["sig"]
+        if self._qkv_ln is None or self._qkv_ln[0] != (key, sig[1]):
+            self._qkv_ln = ((key, sig[1]),) + fold_norm_into_weight(st["w"], None, norm.weight, norm.bias)
+        _, wp, c1, c2 = self._qkv_ln
+        if not st["R"]:
+            return wp, c1, c2, None, None, None
+        if st.get("ln_key") != key:
+            parts = [l._packed.ln for l in (self.to_q, self.to_k, self.to_v)]
+            ln = None
+            if all(t is not None and t[0] == key for t in parts):   # built with the packs, side by side
+                ln = tuple(stacked([t[j] for t in parts]) for j in (1, 2, 3))
+            if ln is None or any(t is None for t in ln):
+                ln = fold_norm_into_adapters(st["a"], norm.weight, norm.bias)
+            st["ln"], st["ln_key"] = ln, key
+        return (wp, c1, c2) + tuple(st["ln"])
+
+    def fused_qkv(self, x: torch.Tensor, ln=None):
+        """to_q / to_k / to_v of a self-attention as ONE GEMM over the stacked weights ([3N,K]: three
+        times the workgroups of a single projection, which alone covers 160 of 256 CUs) and, with
+        adapters, ONE shrink over the stacked A matrices.  Returns (q, k, v) as column views of the
+        [.., 3N] result, or None when the layers cannot be fused (then they run one by one)."""
+        st = self._qkv_state() if x.dtype == torch.bfloat16 else None
+        if st is None:
             return None
+        N = self.to_q.out_features
         if ln is not None and ln[1] is not None and ln[1].valid and LN_FOLD:
             # the norm in front is folded into the stacked GEMM (ln = (LayerNorm, RowStats of x))
             norm, stats = ln
-            key = norm_key(norm)
-            if self._qkv_ln is None or self._qkv_ln[0] != (key, sig[1]):
-                self._qkv_ln = ((key, sig[1]),) + fold_norm_into_weight(st["w"], None, norm.weight, norm.bias)
-            _, wp, c1, c2 = self._qkv_ln
-            ap = ca1 = ca2 = None
-            if st["R"]:
-                if st.get("ln_key") != key:
-                    parts = [l._packed.ln for l in layers]
-                    ln = None
-                    if all(t is not None and t[0] == key for t in parts):   # built with the packs, side by side
-                        ln = tuple(stacked([t[j] for t in parts]) for j in (1, 2, 3))
-                    if ln is None or any(t is None for t in ln):
-                        ln = fold_norm_into_adapters(st["a"], norm.weight, norm.bias)
-                    st["ln"], st["ln_key"] = ln, key
-                ap, ca1, ca2 = st["ln"]
+            wp, c1, c2, ap, ca1, ca2 = self._qkv_folded(st, norm)
             y = ops.lora_linear_norm(x, wp, None, ap, st["s"] if st["R"] else None, st["b"] if st["R"] else None,
                                      two_launches=LORA_SHRINK == "separate", n_split=N if st["R"] else 0,
                                      r_used=st["r_used"] if st["R"] else 0, ln=(stats.buf, c1, c2, ca1, ca2, norm.eps))
@@ -1000,6 +1018,10 @@ class BasicTransformerBlock(nn.Module):
     def forward(self, h, encoder_hidden_states=None, stats: Optional[RowStats] = None, last: bool = False):
         """stats: the row statistics of h as its producer left them (or invalid); on return they describe the result,
         unless `last` (nobody reads them).  Without it every norm runs as a kernel of its own."""
+        if BLOCK_CALL:
+            y = block.run(self, h, encoder_hidden_states, stats, last)
+            if y is not None:
+                return y    # with valid statistics on entry they are valid for the result
         if stats is None:
             h = self.attn1(self.norm1(h), residual=h)
             if self.attn2 is not None:
@@ -1085,9 +1107,9 @@ class ContextKVProjector:
                 if a_all is None or s_all is None:
                     a_all = torch.cat([p.a_cat for p in packs], dim=0).contiguous()
                     s_all = torch.cat([p.col_scale for p in packs], dim=0).contiguous()
-                for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
-                    p.a_cat = a_all[g * R:(g + 1) * R]
-                    p.col_scale = s_all[g * R:(g + 1) * R]
+                    for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
+                        p.a_cat = a_all[g * R:(g + 1) * R]
+                        p.col_scale = s_all[g * R:(g + 1) * R]
                 t = torch.empty((M, G * R), dtype=torch.bfloat16, device=dev)
             rows = []
             for g, l in enumerate(layers):
@@ -1095,7 +1117,7 @@ class ContextKVProjector:
                 rows.append([w.data_ptr(), 0 if b is None else b.data_ptr(), 0 if R == 0 else packs[g].b_cat.data_ptr(),
                              0 if R == 0 else t.data_ptr() + g * R * 2, y[g].data_ptr()])
             st.update(G=G, R=R, K=K, y=y, t=t, a_all=a_all, s_all=s_all,
-                      table=torch.tensor(rows, dtype=torch.int64, device=dev))
+                      table=ops.upload_table(np.array(rows, dtype=np.int64), dev))
         self._built[width] = st
         return st
 
@@ -1119,3 +1141,6 @@ class ContextKVProjector:
             ops.lora_linear_grouped(x2, st["table"], M, width, K, st["R"], st["G"] * st["R"] if st["R"] else 8)
             for i, a in enumerate(attns):
                 a.ctx_kv = (ctx, st["y"][2 * i].view(B, S, width), st["y"][2 * i + 1].view(B, S, width))
+
+
+from . import block   # noqa: E402  (needs the classes above)

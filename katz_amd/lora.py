@@ -160,16 +160,16 @@ _PIECE_DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 def pack_many_takes(layer, names: Sequence[str]) -> bool:
     """Can pack_many build this layer's pack (else: pack_adapters)?"""
-    w = layer.weight
+    w = layer._parameters["weight"]
     if not w.is_cuda or w.dtype != torch.bfloat16 or layer.in_features % 8 != 0 or layer.out_features % 8 != 0:
         return False
-    total = 0
+    total, dev = 0, w.device
     for n in names:
         ad = layer.adapters[n]
         r = ad.down.shape[0]
         total += r
         for t, shape in ((ad.down, (r, layer.in_features)), (ad.up, (layer.out_features, r))):
-            if t.dtype not in _PIECE_DTYPES or t.shape != shape or (t.is_cuda and (t.device != w.device or not t.is_contiguous() or t.data_ptr() % 16)):
+            if t.dtype not in _PIECE_DTYPES or t.shape != shape or (t.is_cuda and (t.device != dev or not t.is_contiguous() or t.data_ptr() % 16)):
                 return False
     return 0 < total <= MAX_PACKED_RANK and (not layer.geglu or layer.out_features % 64 == 0)
 

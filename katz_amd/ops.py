@@ -26,7 +26,8 @@ CALL_LOG = None
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch.cuda.current_stream() without building a Stream object (8 us of a launch's host time before)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -93,18 +94,28 @@ def _weight_prefetch_hint(weight: torch.Tensor, a_cat: Optional[torch.Tensor] = 
     key = weight.data_ptr()
     last = _pf_last[0]
     if last is not None and last != key:
-        table[last] = tuple(None if t is None else weakref.ref(t) for t in (weight, a_cat, b_cat))
-        if len(table) > 65536:     # weights come and go: forget everything rather than grow without bound
-            table.clear()
+        _learn_hint(table, last, tuple(None if t is None else weakref.ref(t) for t in (weight, a_cat, b_cat)))
     _pf_last[0] = key
+    for ptr, nbytes in _hint_ranges(table, key):
+        lib.kh_set_weight_prefetch(ptr, nbytes)
+
+
+def _learn_hint(table, last: int, refs) -> None:
+    table[last] = refs
+    if len(table) > 65536:     # weights come and go: forget everything rather than grow without bound
+        table.clear()
+
+
+def _hint_ranges(table, key: int):
+    """(address, bytes) of what the launch after the one with the weights at `key` should find on the chip."""
     nxt = table.get(key)
     if nxt is None:
-        return
+        return []
     live = [None if r is None else r() for r in nxt]
     w_next = live[0]
     if w_next is None:                # the tensor that followed last time is gone
         del table[key]
-        return
+        return []
     # The prefetch is not free for the launch that carries it (its own first operands queue behind it: up to 3.5 us
     # for 26 MB), so weights are only hinted where meeting them in HBM costs more than that: long rows (K >= 2560,
     # the feed-forward output projections and the 3x3 convolutions), whose launches are latency-bound on their
@@ -113,9 +124,23 @@ def _weight_prefetch_hint(weight: torch.Tensor, a_cat: Optional[torch.Tensor] = 
     # and always hinted.
     k_next = w_next.shape[-1] * (9 if w_next.dim() == 4 else 1)
     small = w_next.numel() * w_next.element_size() <= PREFETCH_SMALL_BYTES
-    for t in ((w_next if (k_next >= PREFETCH_MIN_K or small) else None),) + tuple(live[1:]):
-        if t is not None:
-            lib.kh_set_weight_prefetch(t.data_ptr(), t.numel() * t.element_size())
+    return [(t.data_ptr(), t.numel() * t.element_size())
+            for t in ((w_next if (k_next >= PREFETCH_MIN_K or small) else None),) + tuple(live[1:]) if t is not None]
+
+
+def chain_hints(first_key: int, first_refs, last_key: int):
+    """The prefetch bookkeeping of a chain of launches that one library call issues: its first launch's operands (weak refs to
+    weights, A_cat, B_cat) follow whatever ran before it; returns what to touch for the launch behind its last one, or None
+    where no hints are given (outside every scope)."""
+    table = _pf_next[0]
+    _pf_shrink_a[0] = None
+    if not WEIGHT_PREFETCH or table is None:
+        return None
+    last = _pf_last[0]
+    if last is not None and last != first_key:
+        _learn_hint(table, last, first_refs)
+    _pf_last[0] = last_key
+    return _hint_ranges(table, last_key)
 
 
 def lora_linear(
@@ -568,9 +593,17 @@ def upload_many(tensors: Sequence[torch.Tensor], device):
     return dst, [base + o for o in offset.tolist()]
 
 
+def upload_table(a: np.ndarray, device) -> torch.Tensor:
+    """A small host table on the device, stream-ordered: from pinned memory, because a copy from pageable memory waits for the
+    work in front of it on the stream."""
+    host = torch.from_numpy(a)
+    pinned = torch.empty(host.shape, dtype=host.dtype, pin_memory=True)
+    return pinned.copy_(host).to(device, non_blocking=True)
+
+
 def lora_pack(layers, pieces, a_start, b_start, device) -> None:
     """kh_lora_pack_bf16 on host tables (numpy int64 [n,14] and [m,6], int32 [n+1] twice)."""
-    dev = lambda a: torch.from_numpy(a).to(device, non_blocking=True)
+    dev = lambda a: upload_table(a, device)
     lt, pt, at, bt = dev(layers), dev(pieces), dev(a_start), dev(b_start)
     with torch.cuda.device(device):
         rc = _lib.load().kh_lora_pack_bf16(_ptr(lt), _ptr(pt), _ptr(at), _ptr(bt), layers.shape[0], int(a_start[-1]), int(b_start[-1]), _stream())
@@ -579,7 +612,7 @@ def lora_pack(layers, pieces, a_start, b_start, device) -> None:
 
 def lora_rescale(rows, device) -> None:
     """kh_lora_rescale on host rows (numpy int64 [n,4])."""
-    table = torch.from_numpy(rows).to(device, non_blocking=True)
+    table = upload_table(rows, device)
     with torch.cuda.device(device):
         rc = _lib.load().kh_lora_rescale(_ptr(table), rows.shape[0], _stream())
     _lib.check(rc, "kh_lora_rescale")

@@ -1,0 +1,103 @@
+"""A transformer block as one library call against the same block through its modules, bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def dev():
+    return torch.device("cuda:0")
+
+
+def say(*a):
+    print("[block]", *a, flush=True)
+
+
+def make(width, ranks, depth=2):
+    from katz_amd.layers import LoRALinear, Transformer2DModel
+
+    torch.manual_seed(width + len(ranks))
+    m = Transformer2DModel(width // 64, 64, width, depth, 2048).to(dev(), torch.bfloat16).eval()
+    for l in m.modules():
+        if isinstance(l, LoRALinear):
+            for i, r in enumerate(ranks):
+                l.add_adapter(f"a{i}", torch.randn(r, l.in_features, device=dev(), dtype=torch.bfloat16) * 0.02,
+                              torch.randn(l.out_features, r, device=dev(), dtype=torch.bfloat16) * 0.02)
+            l.set_active([f"a{i}" for i in range(len(ranks))], [0.8, 0.6][:len(ranks)])
+    return m
+
+
+def both(monkeypatch, f):
+    """f's result with the library call (which must have been taken) and without."""
+    from katz_amd import block, layers
+
+    taken, real = [], block.run
+
+    def watch(*a):
+        y = real(*a)
+        taken.append(y is not None)
+        return y
+
+    with monkeypatch.context() as mp:
+        mp.setattr(block, "run", watch)
+        got = f()
+        mp.setattr(layers, "BLOCK_CALL", False)
+        want = f()
+    assert torch.equal(got, want)
+    return taken
+
+
+@pytest.mark.parametrize("width,B,H,W,ranks", [(1280, 2, 16, 16, ()), (1280, 1, 26, 38, (16,)), (640, 2, 19, 13, (64, 32)), (640, 1, 1, 1, (128,)),
+                                               (1280, 2, 32, 32, (8,))])
+@torch.no_grad()
+def test_block_call_gives_the_modules_bits(monkeypatch, width, B, H, W, ranks):
+    say("block call", width, B, H, W, ranks)
+    m = make(width, ranks)
+    blk = m.transformer_blocks[0]
+    ctx = torch.randn(B, 77, 2048, device=dev(), dtype=torch.bfloat16)
+    h = torch.randn(B, H * W, width, device=dev(), dtype=torch.bfloat16)
+    x = torch.randn(B, width, H, W, device=dev(), dtype=torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    assert both(monkeypatch, lambda: blk(h, ctx)) == [True]                  # its norms as launches of their own
+    assert both(monkeypatch, lambda: m(x, ctx)) == [True, True]              # norms folded, statistics from block to block
+    wide = torch.randn(B, 77, 3 * width, device=dev(), dtype=torch.bfloat16)
+    for a in (b.attn2 for b in m.transformer_blocks):
+        a.ctx_kv = (ctx, wide[..., :width], wide[..., 2 * width:])           # projected elsewhere, strided
+    assert both(monkeypatch, lambda: m(x, ctx)) == [True, True]
+
+
+@torch.no_grad()
+def test_block_call_follows_every_change(monkeypatch):
+    from katz_amd.layers import LoRALinear
+
+    m = make(640, (32,), depth=1)
+    blk = m.transformer_blocks[0]
+    ctx = torch.randn(1, 77, 2048, device=dev(), dtype=torch.bfloat16)
+    x = torch.randn(1, 640, 8, 8, device=dev(), dtype=torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    run = lambda: m(x, ctx)
+    linears = [l for l in m.modules() if isinstance(l, LoRALinear)]
+    seen = [run()]
+
+    def changed(taken=True):
+        assert both(monkeypatch, run) == [taken]
+        seen.append(run())
+        assert not torch.equal(seen[-1], seen[-2])
+
+    blk.ff.net[2].weight.mul_(1.5)                                           # in place
+    changed()
+    blk.attn1.to_k.weight = torch.nn.Parameter(blk.attn1.to_k.weight * 0.5, requires_grad=False)
+    changed()
+    blk.norm2.bias.add_(0.5)
+    changed()
+    for l in linears:                                                        # a scale: the packs stay
+        l.set_active(["a0"], [3.0])
+    changed()
+    for l in linears:
+        l.set_active([])
+    changed()
+    blk.attn1.to_out[0] = LoRALinear(640, 640).to(dev(), torch.bfloat16)     # another module
+    changed()
+    hook = blk.attn2.to_q.register_forward_hook(lambda mod, args, out: out * 2)
+    x_h = torch.randn(1, 64, 640, device=dev(), dtype=torch.bfloat16)
+    assert both(monkeypatch, lambda: blk(x_h, ctx)) == [False]               # hooks are called: through the modules
+    hook.remove()
+    assert both(monkeypatch, run) == [True]
