@@ -92,6 +92,18 @@ __device__ __forceinline__ void lora_shrink_tile(const ShrinkParams& p, int m0, 
   // arrived when the first chunk has) and reduced after the loop
   KhLnTileStats<TR * 32, NTB> ln_stats;
   if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, p.M, tid);
+  // and so are the scales and norm terms of the thread's two columns, where its columns are the same on every pass of the last
+  // loop: fetched there they are a trip to memory at the end of a kernel of 5 us
+  constexpr int COLS = TC * 32, ROWS = TR * 32;
+  constexpr bool EARLY = !WT && (2 * NTB) % COLS == 0;
+  float ec[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (EARLY) {
+    const int c = r0 + (2 * tid) % COLS;
+    if (c < p.R) {
+      ec[0] = p.col_scale[c]; ec[1] = p.col_scale[c + 1];
+      if (p.ln_part != nullptr) { ec[2] = p.ln_ca1[c]; ec[3] = p.ln_ca1[c + 1]; ec[4] = p.ln_ca2[c]; ec[5] = p.ln_ca2[c + 1]; }
+    }
+  }
   if (n > 0) issue(0);
   if (n > 1) issue(1);
   if (NS > 2 && n > 2) issue(2);
@@ -135,7 +147,6 @@ __device__ __forceinline__ void lora_shrink_tile(const ShrinkParams& p, int m0, 
           part[(wave * TR * 32 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3)) * LD + j * 32 + l32] = acc[i][j][v];
   }
   __syncthreads();
-  constexpr int COLS = TC * 32, ROWS = TR * 32;
   for (int i = tid; i < ROWS * COLS / 2; i += NTB) {   // two neighbouring columns per thread
     const int rr = (2 * i) / COLS, c = (2 * i) % COLS;
     float s0 = part[rr * LD + c], s1 = part[rr * LD + c + 1];
@@ -147,10 +158,10 @@ __device__ __forceinline__ void lora_shrink_tile(const ShrinkParams& p, int m0, 
     if (m0 + rr < p.M && r0 + c < p.R) {
       if (p.ln_part != nullptr) {
         const float mu = sMu[rr], sg = sSg[rr];
-        s0 = s0 - mu * p.ln_ca1[r0 + c] + sg * p.ln_ca2[r0 + c];
-        s1 = s1 - mu * p.ln_ca1[r0 + c + 1] + sg * p.ln_ca2[r0 + c + 1];
+        s0 = s0 - mu * (EARLY ? ec[2] : p.ln_ca1[r0 + c]) + sg * (EARLY ? ec[4] : p.ln_ca2[r0 + c]);
+        s1 = s1 - mu * (EARLY ? ec[3] : p.ln_ca1[r0 + c + 1]) + sg * (EARLY ? ec[5] : p.ln_ca2[r0 + c + 1]);
       }
-      const uint32_t v = pack_bf16x2(s0 * p.col_scale[r0 + c], s1 * p.col_scale[r0 + c + 1]);
+      const uint32_t v = pack_bf16x2(s0 * (EARLY ? ec[0] : p.col_scale[r0 + c]), s1 * (EARLY ? ec[1] : p.col_scale[r0 + c + 1]));
       uint32_t* dst = reinterpret_cast<uint32_t*>(p.t + (size_t)(m0 + rr) * p.R + r0 + c);
       if (WT) __hip_atomic_store(dst, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       else *dst = v;

@@ -173,3 +173,25 @@ def test_fine_geglu_tiles(M, N, K, R):
     want = run(16)
     for c in (57, 58, 0):
         assert torch.equal(run(c), want), c
+
+
+@pytest.mark.parametrize("K", [64, 640, 1280, 2048, 5120])
+@pytest.mark.parametrize("M", [1, 16, 17, 511, 1024])
+def test_shrink_of_few_rows_gives_the_bits_of_many(M, K):
+    """16 x 16 shrink tiles (up to 256 of them) against the 32 x 32 tiles that run at 2048 rows; with padding columns left out
+    against all columns."""
+    from katz_amd import ops
+
+    say("few-row shrink", M, K)
+    d = dev()
+    g = torch.Generator().manual_seed(M + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, BF)
+    x, a, cs = rnd(2048, K), rnd(64, K) * 0.02, torch.rand(64, generator=g).to(d)
+    want = ops.lora_shrink(x, a, cs)
+    assert torch.equal(ops.lora_shrink(x[:M], a, cs), want[:M])
+    assert_close_rel(want[:M], ((x[:M].double() @ a.double().t()) * cs.double()).float(), 1e-2)
+    a[16:] = 0
+    w, b = rnd(3 * 128, K), rnd(3 * 128, 64)
+    a3, cs3 = torch.cat([a, a * 2, a * 3]), torch.cat([cs] * 3)
+    run = lambda r: ops.lora_linear_split(x[:M], w, None, a3, cs3, b, n_split=128, two_launches=True, r_used=r)
+    assert torch.equal(run(16), run(0))
