@@ -438,6 +438,10 @@ typedef struct {
   int64_t B, T, S, ldk, ldv, bsk, bsv, workspace_bytes, counter_ints, flags, hints, last;
   uint64_t tail_hint[6];
 } KhBlockCall;
+/* One linear from its descriptor: kh_lora_linear_split_bf16 (R > 0: t_scratch and counters as there) or kh_lora_linear_bf16, for a
+ * layer that is called by itself.  flags: bits 8 and 24 as above. */
+int kh_lora_linear_desc_bf16(const KhLinearDesc* desc, const void* x, const void* residual, void* y, void* t_scratch, int32_t* counters,
+                             int64_t M, int flags, void* stream);
 int kh_transformer_block_needs(const KhBlockDesc* desc, int64_t B, int64_t T, int64_t S, int own_kv, int64_t* workspace_bytes,
                                int64_t* counter_ints);
 int kh_transformer_block_bf16(const KhBlockDesc* desc, const KhBlockCall* call, void* stream);

@@ -102,9 +102,9 @@ class _Plan:
         if type(l) is not layers.LoRALinear:
             return False
         l.prepare()
-        self.seen(l, params=("weight", "bias"), plain=("_rt", "geglu"))
+        self.seen(l, params=("weight", "bias"), plain=("_rt", "geglu", "bias"))
         _, w, b = l._rt
-        if (w.dtype != torch.bfloat16 or not w.is_cuda or not w.is_contiguous() or (b is not None and not b.is_contiguous())
+        if (l.__dict__.get("bias") is not None or w.dtype != torch.bfloat16 or not w.is_cuda or not w.is_contiguous() or (b is not None and not b.is_contiguous())
                 or l.in_features % 64 or l.out_features % 8 or (b is not None and b.dtype != torch.bfloat16)
                 or (stats and l.out_features > 128 * ops.LN_SLOTS)):
             return False
@@ -160,7 +160,7 @@ class _Plan:
             if type(l) is not layers.LoRALinear or l.weight.dtype != torch.bfloat16 or not l.weight.is_cuda:
                 return False
             l.prepare()
-            self.seen(l, params=("weight", "bias"), plain=("_rt",))
+            self.seen(l, params=("weight", "bias"), plain=("_rt", "bias"))
         if folded:
             q.eps = norms[0].eps
         q.N, q.K = 3 * a1.to_q.out_features, a1.to_q.in_features
@@ -299,7 +299,7 @@ def run(blk, h, ctx, stats, last: bool):
     ws = h.new_empty((nbytes,), dtype=torch.uint8)
     call.x, call.y, call.workspace, call.workspace_bytes = h.data_ptr(), y.data_ptr(), ws.data_ptr(), nbytes
     if ints:
-        call.counters, call.counter_ints = ops._arena_ints(h.device, ints).data_ptr(), ints
+        call.counters, call.counter_ints = ops._arena_address(h.device, ints), ints
     if folded:
         call.stats = stats.buf.data_ptr()
     call.B, call.T, call.S, call.last = B, T, S, int(last)
@@ -310,4 +310,83 @@ def run(blk, h, ctx, stats, last: bool):
         for i, r in enumerate(ranges):
             call.tail_hint[2 * i], call.tail_hint[2 * i + 1] = r
     _lib.check(_lib.load().kh_transformer_block_bf16(ready.at, ctypes.addressof(call), ops._stream()), "kh_transformer_block_bf16")
+    return y
+
+
+# ---- one linear ------------------------------------------------------------------------------------------------------
+class _LinearReady:
+    """A LoRALinear's operands, checked once, and the parameters and pack they come from (never written to after it is made)."""
+
+    def __init__(self, l):
+        l.prepare()
+        params = l._parameters
+        self.weight, self.bias, self.pack = params["weight"], params.get("bias"), l._packed
+        self.seen = self.state()
+        _, w, b = l._rt
+        p = self.pack
+        self.a_cat = None if p is None else p.a_cat
+        self.usable = (type(l) is layers.LoRALinear and l.__dict__.get("bias") is None and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous()
+                       and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous()))
+                       and (p is None or (not p.overflow and layers.LORA_MODE == "split" and l.in_features % 64 == 0)))
+        if not self.usable:
+            return
+        d = self.desc = _Linear()
+        d.N, d.K, d.geglu, d.w, d.bias = l.out_features, l.in_features, int(l.geglu), w.data_ptr(), _addr(b)
+        b_cat = None
+        if p is not None:
+            b_cat = p.b_cat
+            d.a_cat, d.b_cat, d.col_scale = p.a_cat.data_ptr(), b_cat.data_ptr(), p.col_scale.data_ptr()
+            d.R, d.r_used = p.R, p.r_used
+        self.keep = (w, b, b_cat, None if p is None else p.col_scale)
+        self.refs = tuple(None if t is None else weakref.ref(t) for t in (w, self.a_cat, b_cat))
+        self.at, self.key = ctypes.addressof(d), int(d.w)
+        self.N, self.K, self.R, self.width = d.N, d.K, d.R, d.N // 2 if l.geglu else d.N
+
+    def state(self):
+        w, b = self.weight, self.bias
+        return (w._version, w.data_ptr(), 0) if b is None else (w._version, w.data_ptr(), b._version)
+
+    def holds(self, l) -> bool:
+        d, params, p = l.__dict__, l._parameters, self.pack
+        return (d["_packed"] is p and params["weight"] is self.weight and params.get("bias") is self.bias and d.get("bias") is None and self.seen == self.state()
+                and (p is None or p.a_cat is self.a_cat))
+
+
+_linears: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()   # LoRALinear -> _LinearReady
+
+
+def run_linear(l, x, residual):
+    """l on x (+ residual), or None: take the general path."""
+    if ops.CALL_LOG is not None or not x.is_cuda or x.dtype is not torch.bfloat16 or not x.is_contiguous():
+        return None
+    r = _linears.get(l)
+    if r is None or not r.holds(l):
+        r = _linears[l] = _LinearReady(l)
+    if not r.usable or (r.R and layers.LORA_MODE != "split"):
+        return None
+    shape = x.shape
+    M = x.numel() // r.K
+    if shape[-1] != r.K or M == 0:
+        return None
+    res = 0
+    if residual is not None:
+        if not residual.is_cuda or residual.dtype is not torch.bfloat16 or not residual.is_contiguous() or residual.numel() != M * r.N:
+            return None
+        res = residual.data_ptr()
+    y = x.new_empty((*shape[:-1], r.width))
+    t = counters = None
+    flags = 0
+    if r.R:
+        t = x.new_empty((M, r.R))
+        counters = ops._arena_address(x.device, (M + 127) // 128 + 1)
+        flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_coop_bit()
+    lib = _lib.load()
+    ranges = ops.chain_hints(r.key, r.refs, r.key)
+    if ranges is not None:
+        lib.kh_set_weight_prefetch(None, 0)
+        for ptr, nbytes in ranges:
+            lib.kh_set_weight_prefetch(ptr, nbytes)
+    rc = lib.kh_lora_linear_desc_bf16(r.at, x.data_ptr(), res, y.data_ptr(), None if t is None else t.data_ptr(), counters, M, flags, ops._stream())
+    if rc:
+        _lib.check(rc, "kh_lora_linear_desc_bf16")
     return y

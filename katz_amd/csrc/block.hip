@@ -4,7 +4,8 @@
 // result, a 20-argument foreign call), 230 us of Python per block where the launches themselves take 3 us each -- more than
 // the block's GPU time for images up to 768 x 768.  Everything that does not change from call to call (operands, shapes,
 // flags) is laid out once in a KhBlockDesc; a call brings the activations, one workspace and the counters.  The kernels, their
-// arguments and their order are those of the single entry points, which are what runs here.
+// arguments and their order are those of the single entry points, which are what runs here.  A linear that is called by itself
+// (kh_lora_linear_desc_bf16) saves the same checks.
 #include "kh_common.h"
 #include "../../include/katz_hip.h"
 
@@ -97,6 +98,14 @@ struct Run {
   if (const int rc__ = (call); rc__ != KH_OK) return rc__
 
 }  // namespace
+
+KH_EXPORT int kh_lora_linear_desc_bf16(const KhLinearDesc* l, const void* x, const void* residual, void* y, void* t_scratch, int32_t* counters,
+                                       int64_t M, int flags, void* stream) {
+  if (!l) return KH_ERR_INVALID_ARG;
+  if (l->R == 0) return kh_lora_linear_bf16(x, l->w, l->bias, nullptr, nullptr, nullptr, residual, y, M, l->N, l->K, 0, l->geglu ? 1 : 0, stream);
+  return kh_lora_linear_split_bf16(x, l->w, l->bias, l->a_cat, l->col_scale, l->b_cat, t_scratch, counters, residual, y, M, l->N, l->K, l->R, l->n_split,
+                                   (l->geglu ? 1 : 0) | (int)(l->r_used / 16) << 16 | flags, stream);
+}
 
 KH_EXPORT int kh_transformer_block_needs(const KhBlockDesc* d, int64_t B, int64_t T, int64_t S, int own_kv, int64_t* workspace_bytes, int64_t* counters) {
   if (!d || B <= 0 || T <= 0 || S < 0 || !workspace_bytes || !counters) return KH_ERR_INVALID_ARG;

@@ -260,6 +260,10 @@ class LoRALinear(nn.Module):
         """ln = (LayerNorm module, RowStats of x): the layer computes on norm(x); with valid statistics the norm is folded
         into the GEMM, otherwise it runs as a kernel of its own.  stats_out: left describing the result (valid) when the
         layer can write them, marked invalid otherwise."""
+        if ln is None and stats_out is None and BLOCK_CALL:
+            y = block.run_linear(self, x, residual)
+            if y is not None:
+                return y
         self.prepare()
         _, w, b = self._rt
         p = self._packed

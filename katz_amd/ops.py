@@ -289,7 +289,7 @@ def lora_linear_pre(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
 # device: a reset must not overtake launches that still use their slices (two models side by side on two streams:
 # clear once before the fork and run both under `split_counters_held`).
 SPLIT_ARENA_INTS = 1 << 16
-_split_arena: dict = {}     # (device type, index) -> [buffer, ints handed out, last slice, ever used]
+_split_arena: dict = {}     # (device type, index) -> [buffer, ints handed out, (start, length) of the last slice, ever used, address]
 
 
 def _arena(device):
@@ -300,8 +300,8 @@ def _arena(device):
             # memory allocated during a capture belongs to the graph's pool and dies with the graph
             raise RuntimeError("katz_amd: run the step once eagerly before capturing it (the LoRA counter arena is "
                                "allocated on first use and must outlive the graph)")
-        st = [torch.zeros(SPLIT_ARENA_INTS, dtype=torch.int32, device=device), 0, None, False]
-        _split_arena[key] = st
+        buf = torch.zeros(SPLIT_ARENA_INTS, dtype=torch.int32, device=device)
+        st = _split_arena[key] = [buf, 0, None, False, buf.data_ptr()]
     return st
 
 
@@ -364,21 +364,37 @@ def _split_counters(device, M: int) -> torch.Tensor:
 
 def _arena_ints(device, n: int) -> torch.Tensor:
     """n zeroed int32 of the device's counter arena (zero since the last split_counters_reset)."""
+    st = _arena_take(device, n)
+    at, _ = st[2]
+    return st[0][at:at + n]
+
+
+def _arena_address(device, n: int) -> int:
+    """The address of _arena_ints(device, n)."""
+    st = _arena_take(device, n)
+    return st[4] + 4 * st[2][0]
+
+
+def _arena_take(device, n: int) -> list:
     st = _arena(device)
     if st[1] + n > SPLIT_ARENA_INTS:
         if _arena_held[0]:
             raise RuntimeError("katz_amd: the LoRA counter arena is full inside split_counters_held()")
         split_counters_reset(device)
-    st[2] = st[0][st[1]:st[1] + n]
+    st[2] = (st[1], n)
     st[1] += n
     st[3] = True
-    return st[2]
+    return st
 
 
 def split_counters_last(device) -> Optional[torch.Tensor]:
     """The counters of the most recent lora_linear_split call on this device (for tests: arrivals per row block, then
     the time-out flag)."""
-    return _arena(device)[2]
+    st = _arena(device)
+    if st[2] is None:
+        return None
+    at, n = st[2]
+    return st[0][at:at + n]
 
 
 def lora_linear_split(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], a_cat: torch.Tensor,

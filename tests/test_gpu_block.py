@@ -101,3 +101,32 @@ def test_block_call_follows_every_change(monkeypatch):
     assert both(monkeypatch, lambda: blk(x_h, ctx)) == [False]               # hooks are called: through the modules
     hook.remove()
     assert both(monkeypatch, run) == [True]
+
+
+@pytest.mark.parametrize("rows,K,N,geglu,ranks,residual", [(1, 640, 640, False, (8,), True), (154, 2048, 1280, False, (64, 32), False), (300, 1280, 10240, True, (16,), False),
+                                                           (77, 40, 72, False, (), True), (154, 2048, 640, False, (32,), "no bias"), (65, 1280, 1280, False, (128, 64), True)])
+@torch.no_grad()
+def test_single_linear_call(monkeypatch, rows, K, N, geglu, ranks, residual):
+    from katz_amd import layers
+
+    say("single linear", rows, K, N, geglu, ranks, residual)
+    bf = dict(device=dev(), dtype=torch.bfloat16)
+    l = layers.LoRALinear(K, N, geglu=geglu, bias=residual != "no bias").to(dev(), torch.bfloat16)
+    for i, r in enumerate(ranks):
+        l.add_adapter(f"a{i}", torch.randn(r, K, **bf) * 0.02, torch.randn(N, r, **bf) * 0.02)
+    x, res = torch.randn(2, rows, K, **bf), torch.randn(2, rows, N, **bf) if residual is True else None
+
+    def check():
+        y = l(x, residual=res)
+        with monkeypatch.context() as mp:
+            mp.setattr(layers, "BLOCK_CALL", False)
+            assert torch.equal(y, l(x, residual=res))
+        return y
+
+    seen = [check()]
+    for change in (lambda: l.set_active([f"a{i}" for i in range(len(ranks))]), lambda: l.weight.mul_(2.0), lambda: l.bias is not None and l.bias.add_(1.0), lambda: l.set_active([])):
+        change()
+        seen.append(check())
+    assert not torch.equal(seen[1], seen[2]) and (l.bias is None or not torch.equal(seen[2], seen[3]))
+    with pytest.raises(Exception):
+        l(x[..., :-8].contiguous())
