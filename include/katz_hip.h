@@ -61,7 +61,8 @@ int kh_profile_end(int32_t* tags, float* ms, int capacity);
  * flags bit 0: GEGLU epilogue -- W/bias/B_cat rows are permuted so that every 64 consecutive rows are
  *   32 value rows followed by their 32 gate rows; y is [M, N/2] = value * gelu_erf(gate)
  *   (GEGLU.forward, diffusers-hf/src/diffusers/models/activations.py:139-149); N % 64 == 0, no residual.
- * flags bits 8..15: tile override for tuning (0 = automatic).  Every other bit must be zero (KH_ERR_INVALID_ARG);
+ * flags bits 8..15: tile override for tuning (0 = automatic; a tile that does not take the call's sizes or its unshrunk
+ *   adapter is refused, KH_ERR_UNSUPPORTED).  Every other bit must be zero (KH_ERR_INVALID_ARG);
  * in particular the r_used promise of the sibling entry points below (bits 16..23) has no meaning here. */
 int kh_lora_linear_bf16(const void* x, const void* w, const void* bias, const void* a_cat, const void* b_cat,
                         const float* col_scale, const void* residual, void* y, int64_t M, int64_t N, int64_t K,

@@ -530,6 +530,17 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
 
 }  // namespace
 
+// What the kernel takes, whatever the tile: whole 64-column stages, T given where there are rank columns, operands that one buffer
+// descriptor spans.
+static bool fine_ok(const LoraGemmParams& p) {
+  const size_t lim = (size_t)1 << 31;
+  if (p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return false;
+  if (p.ldt % 8 != 0 || (size_t)p.N * p.K * 2 >= lim || (size_t)p.N * p.R * 2 >= lim || (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 >= lim) return false;
+  if (p.conv_cin == 0) return (size_t)p.M * p.K * 2 < lim;
+  const size_t xb = ((size_t)(p.M / (p.conv_ho * p.conv_wo)) * p.conv_h + 1) * p.conv_w * p.conv_cin * 2 + 2 * (size_t)p.conv_cin;
+  return p.conv_cin % 64 == 0 && xb < lim && p.R == 0;
+}
+
 // Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
 // GEGLU on 64 x 320 (7), 128 x 320 (8).
 //
@@ -541,16 +552,8 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
 // 1280 on 64 x 80 16.0 against 11.7 on 128 x 80.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 31.
 // GEGLU: 512 / 10240 / 1280 30.6 -> 23.6, 988 / 10240 / 1280 48.5 -> 34.3, 2048 / 5120 / 640 28.0 -> 22.3.
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
-  const size_t lim = (size_t)1 << 31;
   const bool conv = p.conv_cin > 0;
-  if (p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return -1;
-  if (p.ldt % 8 != 0 || (size_t)p.N * p.K * 2 >= lim || (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 >= lim) return -1;
-  if (conv) {
-    const size_t xb = ((size_t)(p.M / (p.conv_ho * p.conv_wo)) * p.conv_h + 1) * p.conv_w * p.conv_cin * 2 + 2 * (size_t)p.conv_cin;
-    if (p.conv_cin % 64 != 0 || xb >= lim || p.R > 0) return -1;
-  } else if ((size_t)p.M * p.K * 2 >= lim) {
-    return -1;
-  }
+  if (!fine_ok(p)) return -1;
   const long hw = conv ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
   auto fits = [&](int bm, int bn) {
     return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && nb * ((hw + bm - 1) / bm) * (p.N / bn) <= 256;
@@ -567,7 +570,8 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
 
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
   const bool conv = p.conv_cin > 0;
-  if (p.geglu && form < 7) return KH_ERR_UNSUPPORTED;
+  // (a forced form comes here without the rule above)
+  if (!fine_ok(p) || (p.geglu ? form < 7 || p.st_part != nullptr || p.res != nullptr : form >= 7)) return KH_ERR_UNSUPPORTED;
   switch (form) {
     case 0: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 80, 0>, false>(p, stream);
     case 1: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<128, 80, 0>, false>(p, stream);
@@ -576,8 +580,8 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 4: return conv ? launch_fine<FCfg<32, 160, 4>, true>(p, stream) : launch_fine<FCfg<32, 160, 4>, false>(p, stream);
     case 5: return conv ? launch_fine<FCfg<64, 160, 4>, true>(p, stream) : launch_fine<FCfg<64, 160, 4>, false>(p, stream);
     case 6: return conv ? launch_fine<FCfg<64, 80, 4>, true>(p, stream) : KH_ERR_UNSUPPORTED;
-    case 7: return p.geglu ? launch_fine<FCfg<64, 320, 0, true>, false>(p, stream) : KH_ERR_UNSUPPORTED;
-    case 8: return p.geglu ? launch_fine<FCfg<128, 320, 0, true>, false>(p, stream) : KH_ERR_UNSUPPORTED;
+    case 7: return launch_fine<FCfg<64, 320, 0, true>, false>(p, stream);
+    case 8: return launch_fine<FCfg<128, 320, 0, true>, false>(p, stream);
     default: return KH_ERR_UNSUPPORTED;
   }
 }

@@ -79,6 +79,41 @@ def test_argument_validation_needs_no_gpu():
     assert lib.kh_group_norm_static_bf16(None, 16, None, None, None, 2, 320, 64, 32, 1e-5, 0, 1, None) == -1
 
 
+@pytest.mark.parametrize("code", [50, 51, 52, 53, 54, 55, 57, 58])
+def test_forced_fine_tiles_refuse_what_they_cannot_compute(code):
+    """A tile override (flags bits 8..15) that names a fine tile is refused before any device call where that kernel would
+    leave something out: an adapter whose T nobody has made, K columns that fill no stage, operands beyond one buffer
+    descriptor, an epilogue the form does not have.  Without a device only: a call that is not refused fails there for want
+    of one, on a GPU it would run on these addresses."""
+    import torch
+    from katz_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libkatz_hip.so not built")
+    if torch.cuda.device_count():
+        pytest.skip("needs a machine without a GPU")
+    lib = _lib.load()
+    glu, n = (1, 10240) if code >= 57 else (0, 1280)
+    flags = glu | code << 8
+
+    def linear(M, N, K, R=0, flags=flags, res=None):
+        a = 16 if R else None
+        return lib.kh_lora_linear_bf16(16, 16, None, a, a, a, res, 16, M, N, K, R, flags, None)
+
+    def pre(M, N, K, R, ldt):
+        return lib.kh_lora_linear_pre_bf16(16, 16, None, 16, ldt, 0, 16, None, 16, M, N, K, R, flags, None)
+
+    assert linear(64, n, 640, R=64) == -2                 # unshrunk adapter
+    assert linear(64, n, 96) == -2                        # K % 64
+    assert pre(64, n, 96, 64, 64) == -2
+    assert linear(1 << 20, n, 1024) == -2                 # x of 2 GiB
+    assert linear(64, 5120 * 64, 1 << 12) == -2           # W of 2.5 GiB
+    assert pre(1 << 20, n, 64, 64, 1024) == -2            # T of 2 GiB
+    assert pre(64, 5120 * 2048, 64, 128, 128) == -2       # B_cat of 2.5 GiB
+    assert linear(64, 1288 if not glu else 10304, 640) == -2     # N that the tile does not divide
+    assert linear(64, n, 640, flags=flags ^ 1) == -2      # the other epilogue
+
+
 def test_a_refused_call_drops_the_pending_weight_prefetch_hint():
     """kh_set_weight_prefetch queues up to three ranges for the next launch of the linear / convolution family (a fourth
     is refused).  A call of that family that refuses its arguments must not leave them pending for an unrelated later
