@@ -354,16 +354,21 @@ class LoRALinear(nn.Module):
 
 def refresh_many(modules) -> None:
     """refresh_adapters of many modules.  Linear layers on the GPU whose packs have to be built get them from two launches over
-    all of them, those whose scales alone have changed from one; everything else refreshes by itself."""
+    all of them, those whose scales alone have changed from one; everything else refreshes by itself.  So does every module
+    while a graph is being captured: the launches over many layers read a table that comes from the host, which no graph can
+    carry; refreshing one layer takes fills and copies on the device, which it can."""
     global _pack_epoch
     build: Dict[object, list] = {}
     scale: Dict[object, list] = {}
+    capturing = None
     for m in modules:
         if not isinstance(m, LoRALinear):
             m.refresh_adapters()
             continue
+        if capturing is None and m.weight.is_cuda:
+            capturing = torch.cuda.is_current_stream_capturing()
         names, key = m.wanted_pack()
-        if not names or m._rt is None:
+        if not names or m._rt is None or capturing:
             m.refresh_adapters()
         elif key == m._packed_key and m._packed is not None:
             p = m._packed
@@ -1101,6 +1106,8 @@ class ContextKVProjector:
         ok = uniform and LORA_MODE == "split" and all(l.weight.dtype == torch.bfloat16 and not l.geglu for l in layers)
         st = dict(epoch=_pack_epoch, M=M, ok=ok, wptr=[l.weight.data_ptr() for l in layers])
         if ok:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("katz_amd: run the step once eagerly before capturing it (the context projections' table)")
             dev = ctx.device
             G = len(layers)
             R = 0 if packs[0] is None else packs[0].R

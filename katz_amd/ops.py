@@ -589,9 +589,18 @@ def lora_linear_xattn(x: torch.Tensor, weight: torch.Tensor, k: torch.Tensor, v:
     return out
 
 
+def _no_upload_in_capture() -> None:
+    """Raise while the current stream is being captured.  A copy from host memory would become a node of the graph that reads
+    the memory again at every replay, when it has long been given back; the addresses in a table would then be anything."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("katz_amd: host memory cannot be uploaded into a graph that is being captured; run the step (or activate / "
+                           "merge the adapters) once eagerly before capturing it")
+
+
 def upload_many(tensors: Sequence[torch.Tensor], device):
     """CPU tensors to `device` in one call (kh_upload_many): returns (the device buffer, a device address per tensor).  The
     caller keeps the buffer until the work that reads it has been enqueued on the current stream."""
+    _no_upload_in_capture()
     src = [t if t.is_contiguous() else t.contiguous() for t in tensors]
     n = len(src)
     nbytes = np.fromiter((t.numel() * t.element_size() for t in src), np.int64, n)
@@ -611,7 +620,8 @@ def upload_many(tensors: Sequence[torch.Tensor], device):
 
 def upload_table(a: np.ndarray, device) -> torch.Tensor:
     """A small host table on the device, stream-ordered: from pinned memory, because a copy from pageable memory waits for the
-    work in front of it on the stream."""
+    work in front of it on the stream.  Not under a graph capture."""
+    _no_upload_in_capture()
     host = torch.from_numpy(a)
     pinned = torch.empty(host.shape, dtype=host.dtype, pin_memory=True)
     return pinned.copy_(host).to(device, non_blocking=True)
@@ -674,6 +684,7 @@ def lora_merge_grouped(weights: Sequence[torch.Tensor], ups: Sequence[torch.Tens
 
 def lora_merge_rows(rows, starts, max_rank: int, op_dtype, dev, scale: float = 1.0, layer_scales=None) -> None:
     """kh_lora_merge_grouped_bf16 on rows {W, up, down, N, K, r} that the caller has checked (lora_merge_grouped)."""
+    _no_upload_in_capture()
     lib = _lib.load()
     table = torch.from_numpy(np.array(rows, dtype=np.int64)).to(dev, non_blocking=True)
     tile_start = torch.from_numpy(np.array(starts, dtype=np.int32)).to(dev, non_blocking=True)

@@ -233,6 +233,44 @@ def test_tiny_unet_graph_replay_matches_eager(tiny_pair):
     prod.unload_lora()
 
 
+def test_capture_of_a_forward_that_scales_its_adapters(tiny_pair):
+    """cross_attention_kwargs={"scale": s} changes every layer's scales at the start of the forward and changes them back at its
+    end; a caller may capture that.  Every replay against the eager forward, with eager work of another scale and other host
+    and device allocations in between."""
+    cfg, oracle, prod = tiny_pair
+    say("capture of a scaled forward")
+    dev = torch.device("cuda:0")
+    x, ctx, added = _inputs(cfg, 2, 32, 77, seed=8)
+    x, ctx, added = x.to(dev), ctx.to(dev), _to_dev(added)
+    t = torch.tensor([300.0], device=dev)
+    prod.load_lora_into_unet(katz_lora_state_dict(random_lora(oracle.lora_linears(), 16, seed=13, std=0.05)), adapter_name="s")
+    prod.set_adapters(["s"], [0.7])
+    run = lambda s: prod(x, t, ctx, added_cond_kwargs=added, cross_attention_kwargs={"scale": s}).sample
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(2):
+                run(0.5)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = run(0.5)
+        want, other = run(0.5).clone(), run(2.0).clone()
+        assert not torch.equal(want, other)
+        for i in range(3):
+            junk = [torch.full((n,), 0x5a, dtype=torch.uint8).pin_memory() for n in (512, 4096, 1 << 16)]   # where a table might have been
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert cosine(out, want) >= 0.9995 and cosine(out, want) > cosine(out, other), i
+            assert_close_rel(out, want, 6e-2, f"replay {i}")
+            assert torch.equal(run(2.0), other)      # the replay has put the scales back
+            del junk
+    prod.unload_lora()
+
+
 def test_sdxl_unet_step_config3():
     """BASELINE config 3 at full size: latent [2,4,128,128], t=500, context [2,77,2048], pooled [2,1280],
     time_ids [2,6]; LoRA rank 64 scale 0.8 + rank 32 scale 0.6 on all 722 linears; 9+1 ControlNet

@@ -427,6 +427,50 @@ def test_pack_adapters_cuts_wide_rank_sums_into_packs_of_128():
     assert len(pack_adapters({"a": Adapter(torch.zeros(96, K), torch.zeros(N, 96))}, ["a"], K, N, torch.float32, "cpu").overflow) == 0
 
 
+def test_no_host_upload_while_a_graph_is_captured(monkeypatch):
+    """A copy from host memory inside a graph capture would be repeated by every replay from memory that has been given back:
+    the uploads refuse it, and a change of scales or adapters takes the per-layer path of fills and copies on the device."""
+    import numpy as np
+    import pytest
+    import torch
+    from katz_amd import layers, ops
+    from katz_amd.layers import ContextKVProjector, LoRALinear
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    uploads = (lambda: ops.upload_table(np.zeros((1, 4), np.int64), "cuda:0"), lambda: ops.upload_many([torch.zeros(4)], "cuda:0"),
+               lambda: ops.lora_rescale(np.zeros((1, 4), np.int64), "cuda:0"),
+               lambda: ops.lora_merge_rows([(0,) * 6], [0, 1], 8, torch.float16, "cuda:0"))
+    for upload in uploads:
+        with pytest.raises(RuntimeError, match="captured"):
+            upload()
+
+    class OnGpu(torch.nn.Parameter):      # a layer that refresh_many would hand to the launches over many layers
+        is_cuda = True
+
+    many = []
+    monkeypatch.setattr(layers, "rescale_many", lambda *a: many.append(a))
+    monkeypatch.setattr(layers, "pack_many", lambda *a: many.append(a))
+    monkeypatch.setattr(layers, "pack_many_takes", lambda *a: True)
+    l = LoRALinear(64, 64)
+    l.add_adapter("a", torch.randn(8, 64), torch.randn(64, 8))
+    l.set_active(["a"])
+    l.prepare()
+    l._parameters["weight"] = OnGpu(l.weight.detach(), requires_grad=False)
+    l._packed.col_scale = l._packed.col_scale.as_subclass(OnGpu)
+    l.global_scale = 0.25
+    layers.refresh_many([l])                                  # scales only
+    assert not many and torch.allclose(l._packed.col_scale[:8], torch.full((8,), 0.25))
+    l.add_adapter("b", torch.randn(4, 64), torch.randn(64, 4))
+    l.assign_active(["a", "b"])
+    layers.refresh_many([l])                                  # another set
+    assert not many and [n for n, _, _ in l._packed.spans] == ["a", "b"]
+
+    a = layers.Attention(64, 64, 1, 64).to(torch.bfloat16)    # the context projections' table
+    kv = ContextKVProjector([a])
+    with pytest.raises(RuntimeError, match="before capturing"):
+        kv.run(torch.zeros(1, 2, 64, dtype=torch.bfloat16))
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py --gpus N with N > 1 exits with a message: this build runs on one GPU (no collectives, no sharding)."""
     import subprocess
