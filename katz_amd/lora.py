@@ -168,6 +168,8 @@ def pack_many_takes(layer, names: Sequence[str]) -> bool:
         ad = layer.adapters[n]
         r = ad.down.shape[0]
         total += r
+        if ad.up.dtype != ad.down.dtype:      # a piece has one dtype
+            return False
         for t, shape in ((ad.down, (r, layer.in_features)), (ad.up, (layer.out_features, r))):
             if t.dtype not in _PIECE_DTYPES or t.shape != shape or (t.is_cuda and (t.device != dev or not t.is_contiguous() or t.data_ptr() % 16)):
                 return False
@@ -175,7 +177,7 @@ def pack_many_takes(layer, names: Sequence[str]) -> bool:
 
 
 def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAdapters]:
-    """pack_adapters for many layers of one device in two launches (kh_lora_pack_bf16); adapters in host memory are uploaded
+    """pack_adapters for many layers of one device (such as pack_many_takes accepts) in two launches (kh_lora_pack_bf16); adapters in host memory are uploaded
     with one call.  All packs of a kind share one buffer, in the order of `layers`, so layers that run as one launch (q / k / v of
     a self-attention, the context projections) find their stacked operands in place (`stacked`).  layer.fold_norm: a function
     that gives the LayerNorm in front of the layer or None."""
@@ -219,8 +221,6 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
         for n in ns:
             ad = l.adapters[n]
             r = ad.down.shape[0]
-            if ad.up.dtype != ad.down.dtype:
-                raise TypeError(f"adapter {n!r}: down and up have different dtypes")
             pieces.append((address(ad.down), address(ad.up), r, c, _PIECE_DTYPES[ad.down.dtype], bits(ad.multiplier(l.global_scale))))
             spans.append((n, c, r))
             c += r

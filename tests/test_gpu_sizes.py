@@ -84,6 +84,28 @@ def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
     check()
 
 
+def test_one_adapter_with_unlike_dtypes():
+    """An adapter whose matrices have two dtypes on some layers: those are packed one by one, the others together; active lists
+    and packs agree on every layer."""
+    from katz_amd.lora import pack_adapters
+    from katz_amd.unet_2d_condition import UNet2DConditionModel, UNetConfig
+
+    say("unlike dtypes")
+    d = dev()
+    torch.manual_seed(4)
+    with torch.device(d):
+        unet = UNet2DConditionModel(UNetConfig.tiny())
+    unet.to_runtime(d, BF)
+    linears = list(unet.lora_linears().values())
+    for i, l in enumerate(linears):
+        l.add_adapter("a", torch.randn(8, l.in_features, device=d, dtype=BF), torch.randn(l.out_features, 8, device=d, dtype=torch.float32 if i % 3 == 0 else BF))
+    unet.set_adapters(["a"], [0.5])
+    for l in linears:
+        ref = pack_adapters(l.adapters, ["a"], l.in_features, l.out_features, BF, d, l.global_scale, geglu_interleave=l.geglu)
+        assert l.active == ["a"] and torch.equal(l._packed.a_cat, ref.a_cat) and torch.equal(l._packed.b_cat, ref.b_cat)
+        assert torch.equal(l._packed.col_scale, ref.col_scale)
+
+
 def test_upload_many_sizes():
     """kh_upload_many: arrays smaller and larger than a staging half, empty gaps, one array, bit for bit."""
     from katz_amd import ops

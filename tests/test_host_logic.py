@@ -471,6 +471,20 @@ def test_no_host_upload_while_a_graph_is_captured(monkeypatch):
         kv.run(torch.zeros(1, 2, 64, dtype=torch.bfloat16))
 
 
+def test_adapters_with_unlike_dtypes_are_packed_one_by_one():
+    """pack_many_takes says no before anything has been changed; the launches over many layers read one dtype per adapter."""
+    from types import SimpleNamespace as NS
+
+    from katz_amd.lora import Adapter, pack_many_takes
+
+    gpu = lambda *shape, dtype=torch.bfloat16: NS(is_cuda=True, dtype=dtype, device="cuda:0", shape=shape, is_contiguous=lambda: True, data_ptr=lambda: 256)
+    layer = NS(_parameters={"weight": gpu(64, 128)}, in_features=128, out_features=64, geglu=False)
+    for down, up, takes in ((torch.bfloat16, torch.bfloat16, True), (torch.float32, torch.float32, True), (torch.bfloat16, torch.float32, False),
+                            (torch.float16, torch.bfloat16, False), (torch.float64, torch.float64, False)):
+        layer.adapters = {"a": Adapter(gpu(8, 128, dtype=down), gpu(64, 8, dtype=up))}
+        assert pack_many_takes(layer, ["a"]) == takes, (down, up)
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py --gpus N with N > 1 exits with a message: this build runs on one GPU (no collectives, no sharding)."""
     import subprocess
