@@ -78,6 +78,12 @@ class _Plan:
         self.usable = self.describe(blk, folded)
         self.versions = [t._version for t in self.tensors]
         self.addresses = [t.data_ptr() for t in self.tensors]
+        if self.usable:
+            for l in (self.attn1.to_q, self.attn1.to_k, self.attn1.to_v, *(l for _, l, _ in self.linears)):
+                layers.hold_pack(l, self)
+
+    def drop_packs(self) -> None:
+        self.ready = None
 
     def holds(self) -> bool:
         return (self.options == _options() and self.watch.holds() and [t._version for t in self.tensors] == self.versions
@@ -272,6 +278,8 @@ def run(blk, h, ctx, stats, last: bool):
     ready = plan.ready
     if ready is None or not ready.holds():
         ready = plan.ready = _Ready(plan)
+        if not ready.holds():      # another thread replaced a pack meanwhile: nobody else would drop the old one
+            plan.ready = None
     if not ready.usable:
         return None
     B, T, C = h.shape
@@ -355,6 +363,11 @@ class _LinearReady:
 _linears: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()   # LoRALinear -> _LinearReady
 
 
+def drop_linear(l) -> None:
+    """l's pack has been replaced."""
+    _linears.pop(l, None)
+
+
 def run_linear(l, x, residual):
     """l on x (+ residual), or None: take the general path."""
     if ops.CALL_LOG is not None or not x.is_cuda or x.dtype is not torch.bfloat16 or not x.is_contiguous():
@@ -362,6 +375,8 @@ def run_linear(l, x, residual):
     r = _linears.get(l)
     if r is None or not r.holds(l):
         r = _linears[l] = _LinearReady(l)
+        if not r.holds(l):         # as in run
+            drop_linear(l)
     if not r.usable or (r.R and layers.LORA_MODE != "split"):
         return None
     shape = x.shape

@@ -26,7 +26,7 @@ class GraphedUNetStep:
     rewritten; adapters on 3x3 convolutions repack on any change).
     After anything that repacks or re-derives buffers -- a different set of active adapters, `load_lora_into_unet` /
     `unload_lora`, `fuse_lora` / `unfuse_lora`, `patch_on_lora`, `load_state_dict`, another batch size or resolution --
-    build a new GraphedUNetStep; replaying the old one would compute with the old buffers.
+    build a new GraphedUNetStep; replaying the old one would compute with the old buffers, which have been given back.
     Weight-prefetch hints recorded in the graph point at tensors of this UNet only (they are learned and issued inside
     one forward of one model, ops.weight_prefetch_scope), so freeing ANOTHER model never invalidates this graph."""
 

@@ -12,6 +12,7 @@ token view [N, H*W, C] the transformer blocks need is the same memory -- the NCH
 from __future__ import annotations
 
 import os
+import weakref
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
@@ -71,6 +72,29 @@ class RowStats:
 # bumped whenever any layer rebuilds its packed adapter buffers (not on pure scale changes): consumers
 # that cache pointers into those buffers (grouped launches) rebuild when it moves
 _pack_epoch = 0
+
+# layer -> weak references to whatever has been laid out from its pack (stacked q / k / v operands, the context projections'
+# operands, descriptors of library calls).  They let go of it when it is replaced, not when they next run: the packs of one
+# activation share a buffer, and one holder that stays idle would keep all of it.
+_pack_holders: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
+
+
+def hold_pack(layer: "LoRALinear", holder) -> None:
+    """holder.drop_packs() is called when the layer's pack is replaced.  It forgets objects and changes none: another thread may
+    be reading them."""
+    refs = _pack_holders.get(layer, ())
+    if not any(r() is holder for r in refs):
+        _pack_holders[layer] = tuple(r for r in refs if r() is not None) + (weakref.ref(holder),)
+
+
+def _set_pack(layer: "LoRALinear", pack: Optional[PackedAdapters], key) -> None:
+    d = layer.__dict__   # plain attributes: Module.__setattr__ looks through parameters, buffers and submodules first
+    d["_packed"], d["_packed_key"] = pack, key
+    for r in _pack_holders.get(layer, ()):
+        h = r()
+        if h is not None:
+            h.drop_packs()
+    block.drop_linear(layer)
 
 
 class LoRALinear(nn.Module):
@@ -158,8 +182,9 @@ class LoRALinear(nn.Module):
         names, key = self.wanted_pack()
         if not names:
             if self._packed is not None:
+                _set_pack(self, None, key)
                 _pack_epoch += 1
-            self._packed, self._packed_key = None, key
+            self._packed_key = key
             return
         if key == self._packed_key and self._packed is not None:
             rescale_(self._packed, self.adapters, self.global_scale)
@@ -167,9 +192,9 @@ class LoRALinear(nn.Module):
         # more than 128 rank columns: the extra packs are applied one by one after the fused launch (forward), which for
         # a GEGLU projection means before the activation, so everything is packed in the plain row order then
         wide = sum(self.adapters[n].rank for n in names) > MAX_PACKED_RANK
-        self._packed = pack_adapters(self.adapters, names, self.in_features, self.out_features, self.weight.dtype,
-                                     self.weight.device, self.global_scale, geglu_interleave=self.geglu and not wide)
-        self._packed_key = key
+        pack = pack_adapters(self.adapters, names, self.in_features, self.out_features, self.weight.dtype, self.weight.device,
+                             self.global_scale, geglu_interleave=self.geglu and not wide)
+        _set_pack(self, pack, key)
         _pack_epoch += 1
 
     def fuse(self, lora_scale: float = 1.0, names: Optional[Sequence[str]] = None) -> None:
@@ -388,8 +413,7 @@ def refresh_many(modules) -> None:
     for todo in build.values():
         todo.sort(key=lambda e: e[0]._context if e[0]._context else 1 << 30)   # context projections first, one width behind the other
         for (m, _, key), p in zip(todo, pack_many([e[0] for e in todo], [e[1] for e in todo])):
-            d = m.__dict__   # plain attributes: Module.__setattr__ looks through parameters, buffers and submodules first
-            d["_packed"], d["_packed_key"] = p, key
+            _set_pack(m, p, key)
         _pack_epoch += 1
 
 
@@ -906,8 +930,15 @@ class Attention(nn.Module):
                         st["a"], st["s"] = cat(a), cat(sc)
                         for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
                             p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
+            for l in layers:
+                hold_pack(l, self)
             self._qkv = st
+            if any(l._packed is not p for l, p in zip(layers, packs)):
+                self.drop_packs()   # another thread replaced one meanwhile: nobody else would drop the old one
         return st if st["ok"] else None
+
+    def drop_packs(self) -> None:
+        self.__dict__["_qkv"] = None
 
     def _qkv_folded(self, st: dict, norm: "LayerNorm"):
         """(W', c1, c2, A', ca1, ca2) of the stacked projections behind `norm` (lora.fold_layer_norm)."""
@@ -1129,8 +1160,18 @@ class ContextKVProjector:
                              0 if R == 0 else t.data_ptr() + g * R * 2, y[g].data_ptr()])
             st.update(G=G, R=R, K=K, y=y, t=t, a_all=a_all, s_all=s_all,
                       table=ops.upload_table(np.array(rows, dtype=np.int64), dev))
+            for l in layers:
+                hold_pack(l, self)
         self._built[width] = st
+        if any(l._packed is not p for l, p in zip(layers, packs)):
+            self.drop_packs()   # as in Attention._qkv_state
         return st
+
+    def drop_packs(self) -> None:
+        """The results' buffers stay: the attentions' ctx_kv are views of them."""
+        for width, st in list(self._built.items()):
+            if st.get("a_all") is not None:
+                self._built[width] = dict(st, epoch=None, a_all=None, s_all=None)
 
     def run(self, ctx: torch.Tensor) -> None:
         """Project `ctx` [B,S,K] for every cross-attention; results are handed to the Attention modules."""

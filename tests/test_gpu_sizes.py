@@ -84,6 +84,55 @@ def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
     check()
 
 
+def test_packs_of_the_adapters_before_are_given_back():
+    """All packs of an activation share a buffer per kind.  After the next activation, and after unload_lora, nothing that ran
+    with them (blocks, single layers, the context projections) keeps it, without a forward in between."""
+    import gc
+    import weakref
+
+    from katz_amd.unet_2d_condition import UNet2DConditionModel, UNetConfig
+
+    say("packs given back")
+    d = dev()
+    torch.manual_seed(6)
+    cfg = UNetConfig.tiny()
+    with torch.device(d):
+        unet = UNet2DConditionModel(cfg)
+    unet.to_runtime(d, BF)
+    linears = list(unet.lora_linears().values())
+    for n in "ab":
+        for l in linears:
+            l.add_adapter(n, torch.randn(16, l.in_features, device=d, dtype=BF) * 0.02, torch.randn(l.out_features, 16, device=d, dtype=BF) * 0.02)
+    x = torch.randn(1, 4, 16, 16, device=d, dtype=BF)
+    ctx = torch.randn(1, 77, cfg.cross_attention_dim, device=d, dtype=BF)
+    pooled = cfg.projection_class_embeddings_input_dim - 6 * cfg.addition_time_embed_dim
+    added = dict(text_embeds=torch.randn(1, pooled, device=d, dtype=BF), time_ids=torch.ones(1, 6, device=d))
+
+    def run():
+        with torch.no_grad():
+            unet(x, 500.0, ctx, added_cond_kwargs=added)
+            for l in linears:
+                l(torch.zeros(1, l.in_features, device=d, dtype=BF))
+
+    unet.set_adapters(["a"])
+    for change in (lambda: unet.set_adapters(["b"]), unet.unload_lora):
+        run()
+        run()
+        packs = [l._packed for l in linears]
+        size = sum(p.a_cat.numel() + p.b_cat.numel() for p in packs) * 2
+        old = [weakref.ref(t) for p in packs for t in (p, p.a_cat, p.b_cat, p.col_scale)]
+        del packs
+        gc.collect()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        change()
+        gc.collect()
+        assert sum(r() is not None for r in old) == 0
+        grown = torch.cuda.memory_allocated() - before
+        assert grown < size // 2, (grown, size)
+    run()
+
+
 def test_one_adapter_with_unlike_dtypes():
     """An adapter whose matrices have two dtypes on some layers: those are packed one by one, the others together; active lists
     and packs agree on every layer."""

@@ -485,6 +485,30 @@ def test_adapters_with_unlike_dtypes_are_packed_one_by_one():
         assert pack_many_takes(layer, ["a"]) == takes, (down, up)
 
 
+def test_a_replaced_pack_is_let_go_of():
+    """The stacked q / k / v operands of an attention that does not run again keep nothing of the packs they came from."""
+    import gc
+    import weakref
+
+    from katz_amd.layers import Attention
+
+    a = Attention(128, None, 2, 64)
+    for l in (a.to_q, a.to_k, a.to_v):
+        l.add_adapter("a", torch.randn(8, 128), torch.randn(128, 8))
+        l.add_adapter("b", torch.randn(8, 128), torch.randn(128, 8))
+        l.set_active(["a"])
+    layers = (a.to_q, a.to_k, a.to_v)
+    for change in (lambda l: l.set_active(["b"]), lambda l: l.set_active([])):
+        st = a._qkv_state()
+        old = [weakref.ref(t) for t in [l._packed for l in layers] + [st["a"], st["b"], st["s"]]]
+        del st
+        for l in layers:
+            change(l)
+        gc.collect()
+        assert not any(r() is not None for r in old)
+    assert a._qkv_state()["R"] == 0
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py --gpus N with N > 1 exits with a message: this build runs on one GPU (no collectives, no sharding)."""
     import subprocess
