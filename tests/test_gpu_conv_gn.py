@@ -112,6 +112,44 @@ def test_statistics_against_plain_sums():
         assert torch.allclose(got[..., 1], q_ref, rtol=1e-4), "sums of squares"
 
 
+@pytest.mark.parametrize("Nb,Cin,Cout,H,W,with_res", [
+    (1, 320, 640, 8, 16, False),      # two row tiles, 20-channel groups
+    (2, 1280, 1280, 16, 16, True),    # the 16x16 level's residual blocks
+    (1, 640, 1280, 24, 40, False),    # 15 row tiles of one image
+    (1, 1280, 1280, 32, 32, True),    # exactly one round of 256 tiles
+    (3, 1280, 640, 8, 24, True),      # three images
+])
+def test_statistics_of_the_few_row_tiles(Nb, Cin, Cout, H, W, with_res):
+    """64 x 80 tiles (a convolution with statistics whose 64-row tiles fill at most one round): its result bit for bit that of
+    the convolution without statistics, the sums against sums of that result in 64 bits, the norm behind it against the oracle.
+
+    A sum's error is bounded by n * 2^-24 of the sum of magnitudes for n = Cout / G * H * W summands in any order; the tile's
+    partial sums and the per-channel term keep it well below 1e-5 of it."""
+    from katz_amd import ops
+    say("conv3x3 statistics, few rows", Nb, Cin, Cout, H, W, with_res)
+    d, G, eps = dev(), 32, 1e-5
+    g = torch.Generator().manual_seed(Nb + Cin + H + W)
+    x, w, b = randn(g, Nb, Cin, H, W), randn(g, Cout, Cin, 3, 3, std=(9 * Cin) ** -0.5), randn(g, Cout, std=0.3)
+    gamma, beta, add = bf16_round(1.0 + 0.3 * torch.randn(Cout, generator=g)), randn(g, Cout, std=0.3), randn(g, Nb, Cout, std=0.5)
+    on = lambda t: t.to(d, BF)
+    nhwc = lambda t: on(t).contiguous(memory_format=torch.channels_last)
+    xd, wp, res = nhwc(x), ops.pack_conv3x3_weight(on(w)), nhwc(randn(g, Nb, Cout, H, W)) if with_res else None
+    assert ops.conv3x3_gn_splits(xd, Cout, G) == H * W // 64
+    assert Nb * (H * W // 64) * (Cout // 80) <= 256           # one round: these tiles and no others
+    y, part, splits = ops.conv3x3_stats(xd, wp, on(b), G, add_nc=on(add), residual=res)
+    assert torch.equal(y, ops.conv3x3(xd, wp, on(b), residual=res))
+    v = (y.float() + on(add).float()[:, :, None, None]).double().reshape(Nb, G, Cout // G * H * W)
+    got = part.double().sum(dim=2)
+    assert part.shape == (Nb, G, splits, 2)
+    assert ((got[..., 0] - v.sum(-1)).abs() <= 1e-5 * v.abs().sum(-1)).all()
+    assert ((got[..., 1] - (v * v).sum(-1)).abs() <= 1e-5 * (v * v).sum(-1)).all()
+    n = ops.group_norm_from_stats(y, G, on(gamma), on(beta), eps, "silu", part, splits, add_nc=on(add))
+    conv = bf16_round(torch.nn.functional.conv2d(x, w, b, padding=1))
+    if with_res:
+        conv = bf16_round(conv + res.float().cpu())
+    assert_close_rel(n, O.group_norm(conv + add[:, :, None, None], G, gamma, beta, eps, "silu"), 2e-2, "norm on the statistics")
+
+
 @pytest.mark.parametrize("act", ["none", "silu"])
 def test_norm_behind_a_convolution_with_residual(act):
     """conv2 + skip, then the next module's GroupNorm (no per-channel term) on the statistics conv2 left."""
