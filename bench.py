@@ -106,6 +106,12 @@ def instrumented_step(unet, inputs):
         kh, kw = m.kernel_size
         conv_flops[0] += 2.0 * out.numel() * m.in_channels * kh * kw
 
+    # While calls are logged a transformer block runs launch by launch.  Which operands a launch requests ahead for the one
+    # behind it is learned from the pass before, so one such pass comes first: the timed launches then carry the requests
+    # that those of the captured step carry.
+    ops.CALL_LOG = []
+    with torch.no_grad():
+        unet(sample, t, ctx, added_cond_kwargs=added, down_block_additional_residuals=down, mid_block_additional_residual=mid)
     hooks = [m.register_forward_hook(hook) for m in unet.modules() if isinstance(m, torch.nn.Conv2d)]
     ops.CALL_LOG = []
     torch.cuda.synchronize()
@@ -469,6 +475,37 @@ def kernel_probe():
     coef = torch.tensor([4.2, 3.1, (3.1 ** 2 + 1) ** 0.5], device=dev)
     add("conv_out + guidance + Euler 2x320x128x128", lambda: ops.conv_out_cfg_euler(xo, wo, bo, lat, coef, 7.5, model_input_next=nxt),
         2.0 * 32768 * 2880 * 4, 2.0 * (xo.numel() + wo.numel() + 2 * lat.numel() + nxt.numel()))
+    # few rows: the 32x32 level of one 832 x 1216 image (26 * 38 = 988 tokens), weights as the previous round left them
+    M, R = 988, 64
+    for K, N, geglu in ((1280, 1280, False), (5120, 1280, False), (1280, 10240, True)):
+        xf, wf, bf_, af, bcf = rn(M, K), rn(N, K, std=0.02), rn(N), rn(R, K, std=0.02), rn(N, R, std=0.02)
+        sf, tf, nout = torch.full((R,), 0.8, device=dev), torch.empty(M, R, device=dev, dtype=bf), N // 2 if geglu else N
+        if not geglu:
+            add(f"lora_shrink M{M} K{K} R{R}", lambda x=xf, a=af, s=sf, t=tf: ops.lora_shrink(x, a, s, out=t), 2.0 * M * K * R,
+                2.0 * (M * K + R * K + M * R))
+        add(f"lora_gemm M{M} K{K} N{N} R{R}{' geglu' if geglu else ''}", lambda x=xf, w=wf, b=bf_, t=tf, bc=bcf, ge=geglu: ops.lora_linear_pre(x, w, b, t, bc, geglu=ge),
+            2.0 * M * N * (K + R), 2.0 * (M * K + K * N + M * nout + R * N + M * R))
+        if K == N:
+            st = ops.row_stats_buffer(M, dev)
+            add(f"lora_gemm M{M} K{K} N{N} + row statistics", lambda x=xf, w=wf, b=bf_, st=st: ops.lora_linear_norm(x, w, b, stats_out=st), 2.0 * M * N * K,
+                2.0 * (M * K + K * N + M * N))
+    xs, ws_, bs = cl(rn(1, 1280, 26, 38)), ops.pack_conv3x3_weight(rn(1280, 1280, 3, 3, std=0.01)), rn(1280)
+    add("conv3x3 1280->1280 @26x38, one image", lambda: ops.conv3x3(xs, ws_, bs), 2.0 * 988 * 1280 * 11520, 2.0 * (2 * xs.numel() + ws_.numel()))
+    xq2 = cl(rn(2, 1280, 16, 16))
+    add("conv3x3 + statistics 1280->1280 @16x16", lambda: ops.conv3x3_stats(xq2, ws_, bs, 32), 2.0 * 512 * 1280 * 11520, 2.0 * (2 * xq2.numel() + ws_.numel()))
+    # the fp32 layer (shrink, then GEMM + expand)
+    M, K, N, R = 8192, 640, 640, 32
+    x32, w32, a32, b32 = (torch.randn(*sh, device=dev, generator=g) * sd for sh, sd in (((M, K), 1.0), ((N, K), 0.02), ((R, K), 0.02), ((N, R), 0.02)))
+    s32 = torch.full((R,), 0.8, device=dev)
+    add(f"lora_linear_f32 M{M} K{K} N{N} R{R}", lambda: ops.lora_linear(x32, w32, None, a32, b32, s32), 2.0 * M * (N * K + R * K + N * R),
+        4.0 * (M * K + N * K + M * N + R * K + N * R))
+    # packing one rank-64 adapter for eight 1280-wide layers in two launches
+    from katz_amd.layers import LoRALinear
+    from katz_amd.lora import pack_many
+    packed = [LoRALinear(1280, 1280, device=dev, dtype=bf) for _ in range(8)]
+    for l in packed:
+        l.add_adapter("a", rn(64, 1280), rn(1280, 64))
+    add("lora_pack 8 layers 1280x1280 rank 64", lambda: pack_many(packed, [["a"]] * 8), 0.0, 8 * 2 * 2.0 * 2 * 64 * 1280)
     torch.cuda.synchronize()
     for _ in range(3):
         dst.copy_(src)
