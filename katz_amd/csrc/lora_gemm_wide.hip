@@ -83,9 +83,6 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_wide_kernel(const LoraGemmPa
   if (local / p.xr_n >= p.xr_m || m_blk >= p.m_tiles || n_blk >= p.n_tiles) return;  // padding of the grid
   const int m0 = m_blk * WBM, n0 = n_blk * WBN;
   const int N = p.N, K = p.K;
-  // the XCD's block of W into its L2 (2048 / 10240 / 1280: 54.2 -> 51.5 us); this wave's own first loads overwrite the LDS it lands in
-  if (kh_touch_pays(N, K, p.xr_n * WBN))
-    kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * WBN, p.xr_n * WBN, 0, K / 64, smem + wave * (WBM / 8) * 128, local * 512 + tid, p.xr_m * p.xr_n * 512);
   const int KT1 = K / 64;
   // only the first r_used rank columns of T / B_cat can be non-zero: stages beyond them are not visited, and of a
   // last stage that they fill at most half only the first two MFMA steps run
