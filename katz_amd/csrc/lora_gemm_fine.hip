@@ -2,8 +2,8 @@
 // convolutions on BM x BN output tiles small enough that a few hundred rows still give every CU a workgroup.
 //
 // Same arithmetic as the two-launch form of lora_gemm_pipe.hip (the reference's LoRA linear,
-// diffusers-hf/src/diffusers/models/lora.py:224-225, T made by a launch in front), bit for bit as the kernel that runs at
-// more rows: the order of every sum is that kernel's (below).
+// diffusers-hf/src/diffusers/models/lora.py:224-225, T made by a launch in front), bit for bit as one of the kernels for more
+// rows: the order of every sum is that kernel's (below), which is what the tests compare with.
 //
 // What bounds these calls: not the matrix pipe and not HBM's rate but a CU's operand stream.  A CU takes about 55 GB/s of
 // lines that come from memory and 110 GB/s of lines its L2 has, all CUs together 17 TB/s out of the L2s; a 128 x 128 tiling of M = 1000 /
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
     }
   } else {
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
-    // 9.4 us; 64 x 160 tiles at K 5120 42.7 -> 33.2; x, which the launch in front has just written, is not worth it)
+    // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
     auto touch = [&](int t, int n) {
       if (t < KT1)
         kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
@@ -546,11 +546,13 @@ static bool fine_ok(const LoraGemmParams& p) {
 //
 // Which of them, for a layer whose sums follow `order`: one that fits one round of the 256 CUs (a workgroup fills a CU, so a second round
 // costs as much as the first), the smaller first; -1 where none does and the larger tiles of the other families win.  A
-// convolution that leaves GroupNorm statistics does so per 64 rows.  Measured, weights cold, us (M, N, K: before -> these):
-// 512 / 1280 / 1280 18.4 -> 9.4 (with row statistics 10.9); 988 / 1280 / 1280 18.5 -> 9.5 (11.4); 2048 / 1280 / 1280 16.5 -> 13.1;
-// 988 / 1280 / 5120 44.3 -> 29.6; 2048 / 1280 / 5120 46.6 -> 40.2; 154 / 1280 / 2048 23.5 -> 12.7; a round too many: 1152 / 1280 /
-// 1280 on 64 x 80 16.0 against 11.7 on 128 x 80.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 31.
-// GEGLU: 512 / 10240 / 1280 30.6 -> 23.6, 988 / 10240 / 1280 48.5 -> 34.3, 2048 / 5120 / 640 28.0 -> 22.3.
+// convolution that leaves GroupNorm statistics does so per 64 rows.  Measured as launches without adapters in a captured chain whose
+// weights together exceed the memory-side cache, us per launch (M, N, K: the larger tiles -> these):
+// 512 / 1280 / 1280 18.3 -> 9.8 (with row statistics 19.7 -> 11.1); 988 / 1280 / 1280 18.6 -> 9.8 (19.8 -> 11.9); 2048 / 1280 / 1280
+// 16.4 -> 13.1; 988 / 1280 / 5120 43.7 -> 30.6; 2048 / 1280 / 5120 45.7 -> 39.5; 154 / 1280 / 2048 23.5 -> 12.6; a round too many:
+// 1152 / 1280 / 1280 on 64 x 80 16.3 against 12.0 on 128 x 80.  GEGLU: 512 / 10240 / 1280 29.5 -> 23.6, 988 / 10240 / 1280
+// 44.9 -> 34.7, 2048 / 5120 / 640 26.1 -> 21.3.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 30.
+// (With adapters, 1024 and more rows at N 1280 do not come here: lora_gemm_pipe_il_ok takes them first.)
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   const bool conv = p.conv_cin > 0;
   if (!fine_ok(p)) return -1;

@@ -723,7 +723,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lora_gemm_pipe_kernel(const Lor
   const int K = p.K, M = p.M, N = p.N;
   constexpr int BKP = C::BKP, ROWB = C::ROWB;
   // the XCD's block of W into its L2 (into LDS that this wave's own first loads overwrite afterwards), by at least half its CUs: 988 /
-  // 3840 / 1280 18.3 -> 16.6 us (the other instantiations have no registers for it or gain nothing)
+  // 3840 / 1280 17.4 -> 16.5 us (the other instantiations have no registers for it or gain nothing)
   if (!IL && !CONV && LNF != 3 && !XA && BM == 128 && BN == 128 && C::NT == 512 && p.grp == nullptr && p.sg_mode == 0 &&
       p.xr_m * p.xr_n >= 16 && kh_touch_pays(N, K, p.xr_n * BN))
     kh_touch_rows(p.w, N, K, (bid & 7) % p.xg_n * p.xr_n * BN, p.xr_n * BN, 0, K / 64, smem + wave * (C::UX / C::NW) * 1024,

@@ -4,7 +4,8 @@
 // laying the active adapters of a layer out as A_cat [R,K], B_cat [N,R], col_scale [R] (katz_amd/lora.py), and for a layer behind
 // a folded LayerNorm also A_cat * gamma with its two row terms.  For the 722 linears of SDXL that was some 9000 small torch
 // operations (about 90 ms of host time); the bytes are 0.4 GB read and written, so a launch over all rows of all layers is bound by
-// HBM and takes a fraction of a millisecond.  Two activations with the step behind each (768x768, ranks 64 + 32, then 16): 196 -> 93 ms.
+// HBM and takes a fraction of a millisecond.  Two activations with the step behind each (768x768, ranks 64 + 32, then 16), with the
+// one-call blocks: 181 -> 88 ms the first time a set is used, 59 where the same two sets take turns.
 #include "kh_common.h"
 
 namespace {

@@ -177,8 +177,8 @@ def pack_many_takes(layer, names: Sequence[str]) -> bool:
 
 
 def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAdapters]:
-    """pack_adapters for many layers of one device (such as pack_many_takes accepts) in two launches (kh_lora_pack_bf16); adapters in host memory are uploaded
-    with one call.  All packs of a kind share one buffer, in the order of `layers`, so layers that run as one launch (q / k / v of
+    """pack_adapters for many layers of one device (such as pack_many_takes accepts) in two launches (kh_lora_pack_bf16);
+    adapters in host memory are uploaded with one call.  All packs of a kind share one buffer, in the order of `layers`, so layers that run as one launch (q / k / v of
     a self-attention, the context projections) find their stacked operands in place (`stacked`).  layer.fold_norm: a function
     that gives the LayerNorm in front of the layer or None."""
     dev = layers[0].weight.device
