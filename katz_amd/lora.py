@@ -178,9 +178,9 @@ def pack_many_takes(layer, names: Sequence[str]) -> bool:
 
 def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAdapters]:
     """pack_adapters for many layers of one device (such as pack_many_takes accepts) in two launches (kh_lora_pack_bf16);
-    adapters in host memory are uploaded with one call.  All packs of a kind share one buffer, in the order of `layers`, so layers that run as one launch (q / k / v of
-    a self-attention, the context projections) find their stacked operands in place (`stacked`).  layer.fold_norm: a function
-    that gives the LayerNorm in front of the layer or None."""
+    adapters in host memory are uploaded with one call.  All packs of a kind share one buffer, in the order of `layers`, so
+    layers that run as one launch (q / k / v of a self-attention, the context projections) find their stacked operands in place
+    (`stacked`).  layer.fold_norm: a function that gives the LayerNorm in front of the layer or None."""
     dev = layers[0].weight.device
     host = [t for l, ns in zip(layers, names) for n in ns for t in (l.adapters[n].down, l.adapters[n].up) if not t.is_cuda]
     keep, where = None, {}
@@ -200,38 +200,39 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
     A, B, S = buf(sum(sizes_a), torch.bfloat16), buf(sum(sizes_b), torch.bfloat16), buf(sum(padded), torch.float32)
     AN = buf(sum(sizes_a[i] for i in folded), torch.bfloat16)
     C1, C2 = (buf(sum(padded[i] for i in folded), torch.float32) for _ in range(2))
-    a_views, b_views, s_views = A.split(sizes_a), B.split(sizes_b), S.split(padded)
-    an_views, c1_views, c2_views = AN.split([sizes_a[i] for i in folded]), C1.split([padded[i] for i in folded]), C2.split([padded[i] for i in folded])
     pa, pb, ps, pan, pc1, pc2 = (t.data_ptr() for t in (A, B, S, AN, C1, C2))
-    rows, pieces, packs, f = [], [], [], 0
+    # flat tables, and views made directly: thousands of short-lived tuples and tensors per activation bring on the interpreter's
+    # full collections (85 ms for the objects of this model) the sooner
+    rows, pieces, packs, n_pieces = [], [], [], 0
+    at_a = at_b = at_s = at_an = at_c = 0
     b_blocks = []
-    for i, (l, ns, R) in enumerate(zip(layers, names, padded)):
-        K, N, g = l.in_features, l.out_features, norms[i]
+    for l, ns, R, g in zip(layers, names, padded, norms):
+        K, N = l.in_features, l.out_features
         ln = None
         if g is not None:
-            rows.append((pa, pan, g.weight.data_ptr(), g.bias.data_ptr(), pc1, pc2, pb, ps, K, N, R, int(l.geglu), len(pieces), len(ns)))
-            ln = (norm_key(g), an_views[f].view(R, K), c1_views[f], c2_views[f])
-            f += 1
-            pan += 2 * R * K
-            pc1 += 4 * R
-            pc2 += 4 * R
+            rows += (pa + 2 * at_a, pan + 2 * at_an, g.weight.data_ptr(), g.bias.data_ptr(), pc1 + 4 * at_c, pc2 + 4 * at_c)
+            ln = (norm_key(g), AN.as_strided((R, K), (K, 1), at_an), C1.as_strided((R,), (1,), at_c), C2.as_strided((R,), (1,), at_c))
+            at_an += R * K
+            at_c += R
         else:
-            rows.append((pa, 0, 0, 0, 0, 0, pb, ps, K, N, R, int(l.geglu), len(pieces), len(ns)))
+            rows += (pa + 2 * at_a, 0, 0, 0, 0, 0)
+        rows += (pb + 2 * at_b, ps + 4 * at_s, K, N, R, int(l.geglu), n_pieces, len(ns))
+        n_pieces += len(ns)
         spans, c = [], 0
         for n in ns:
             ad = l.adapters[n]
             r = ad.down.shape[0]
-            pieces.append((address(ad.down), address(ad.up), r, c, _PIECE_DTYPES[ad.down.dtype], bits(ad.multiplier(l.global_scale))))
+            pieces += (address(ad.down), address(ad.up), r, c, _PIECE_DTYPES[ad.down.dtype], bits(ad.multiplier(l.global_scale)))
             spans.append((n, c, r))
             c += r
-        packs.append(PackedAdapters(a_views[i].view(R, K), b_views[i].view(N, R), s_views[i], spans, ln=ln))
+        packs.append(PackedAdapters(A.as_strided((R, K), (K, 1), at_a), B.as_strided((N, R), (R, 1), at_b), S.as_strided((R,), (1,), at_s), spans, ln=ln))
         per_block = 256 // (R // 8)
         b_blocks.append(-(-N // per_block))
-        pa += 2 * R * K
-        pb += 2 * R * N
-        ps += 4 * R
+        at_a += R * K
+        at_b += R * N
+        at_s += R
     start = lambda counts: np.concatenate([np.zeros(1, np.int32), np.cumsum(counts, dtype=np.int32)])
-    ops.lora_pack(np.array(rows, dtype=np.int64), np.array(pieces, dtype=np.int64), start(padded), start(b_blocks), dev)
+    ops.lora_pack(np.array(rows, dtype=np.int64).reshape(-1, 14), np.array(pieces, dtype=np.int64).reshape(-1, 6), start(padded), start(b_blocks), dev)
     del keep    # stream-ordered: the launches above are enqueued
     return packs
 
