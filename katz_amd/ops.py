@@ -200,8 +200,14 @@ def lora_linear(
         if geglu:
             raise ValueError("the GEGLU epilogue exists for bf16 only")
         t = torch.empty((M, R), dtype=dt, device=x.device) if R else None
-        rc = lib.kh_lora_linear_split_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale), _ptr(t),
-                                          _ptr(residual), _ptr(out), M, N, K, R, _stream())
+        n_planes = lib.kh_lora_linear_planes_f32_bytes(N, K, R)
+        if n_planes:
+            planes = torch.empty(n_planes, dtype=torch.uint8, device=x.device)
+            rc = lib.kh_lora_linear_planes_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale), _ptr(t),
+                                               _ptr(planes), _ptr(residual), _ptr(out), M, N, K, R, _stream())
+        else:
+            rc = lib.kh_lora_linear_split_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale), _ptr(t),
+                                              _ptr(residual), _ptr(out), M, N, K, R, _stream())
         if rc in (-2, -3):   # KH_ERR_UNSUPPORTED / KH_ERR_ALIGNMENT: rows that 16-byte pieces do not fill take the scalar kernel
             rc = lib.kh_lora_linear_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale),
                                         _ptr(residual), _ptr(out), M, N, K, R, _stream())

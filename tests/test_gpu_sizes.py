@@ -35,6 +35,46 @@ def test_lora_linear_f32_matrix_kernel(M, N, K, R):
     assert_close_rel(y, ref, 1e-5, "fp32 linear")
 
 
+@pytest.mark.parametrize("M,N,K,R", [(1, 5, 4, 4), (64, 80, 32, 0), (65, 81, 36, 32), (300, 1280, 100, 36), (1300, 1284, 68, 4), (8200, 640, 640, 32)], ids=str)
+def test_lora_linear_f32_on_bf16_planes(M, N, K, R):
+    """kh_lora_linear_planes_f32 on each of its tiles, ragged in every dimension, against 64 bits.
+
+    Bound, elementwise and relative to the sum of the magnitudes of the summands: the three products left out, each below 2^-23 of its
+    factors' product; seven truncations of 2^-23 in a stage's sum of its own; one rounding of 2^-24 per stage of 32 columns and per term
+    behind them; the same once more for T."""
+    from katz_amd import _lib, ops
+
+    say("lora_linear_planes_f32", M, N, K, R)
+    d, g = dev(), torch.Generator(device="cuda").manual_seed(M + N + K)
+    rn = lambda *s, std=1.0: torch.randn(*s, generator=g, device=d) * std
+    x, w, b, res = rn(M, K), rn(N, K, std=K ** -0.5), rn(N), rn(M, N)
+    A, B, sc = (rn(R, K, std=0.1), rn(N, R, std=0.1), torch.full((R,), 1.5, device=d)) if R else (None, None, None)
+    assert _lib.load().kh_lora_linear_planes_f32_bytes(N, K, R) > 0
+    y = ops.lora_linear(x, w, b, A, B, sc, residual=res)
+    f = lambda t: t.double()
+    ref, mag = f(x) @ f(w).T + f(b) + f(res), f(x).abs() @ f(w).abs().T + f(b).abs() + f(res).abs()
+    if R:
+        ref += 1.5 * (f(x) @ f(A).T) @ f(B).T
+        mag += 1.5 * (f(x).abs() @ f(A).abs().T) @ f(B).abs().T
+    assert ((f(y) - ref).abs() <= (2 * (3 + 7) + K / 32 + 4) * 2.0 ** -23 * mag).all()
+
+
+def test_lora_linear_f32_not_finite():
+    """Infinities, NaN and sums that overflow come out as full fp32 products give them (a split infinity would be NaN)."""
+    from katz_amd import ops
+
+    say("lora_linear_planes_f32, not finite")
+    d, g = dev(), torch.Generator(device="cuda").manual_seed(5)
+    x, w = torch.randn(200, 640, generator=g, device=d), torch.randn(320, 640, generator=g, device=d) * 0.02
+    w[:, 5] = torch.where(torch.arange(320, device=d) % 2 == 0, 0.5, -0.25)          # exact in bf16: its lower planes are zero
+    x[3, 5], x[100, 5], x[50, 7], w[7, 9], x[150, 5] = float("inf"), -float("inf"), float("nan"), float("inf"), 3.4e38
+    y = ops.lora_linear(x, w)
+    ref = (x.double() @ w.double().T).float()
+    assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf()) and torch.equal(y[y.isinf()], ref[ref.isinf()])
+    ok = ref.isfinite()
+    assert (y[ok] - ref[ok]).abs().le(1e-5 * ref[ok].abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("host,dtype,ranks", [(False, torch.bfloat16, (64, 32)), (True, torch.float16, (16,)), (False, torch.float32, (4, 8, 100)), (True, torch.bfloat16, (5, 7))],
                          ids=str)
 def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
