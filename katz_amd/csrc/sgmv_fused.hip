@@ -7,20 +7,26 @@
 // rounded to bf16 before it is added to y), but t never leaves the workgroup: one launch instead of two and no round
 // trip of t through memory.  Bound: HBM (x read once, y read and written once; the adapter matrices come from L2).
 //
-// A workgroup (8 waves) owns 128 rows of one segment.
-//   phase 1: T[128, 128] = x_tile . A_a^T over K in 64-column stages (ring of three, buffer-addressed LDS DMA, the
-//            operand path of lora_gemm_pipe.hip); T is rounded to bf16 and written to LDS in the stage layout, so that
+// A workgroup (8 waves) owns BM = 64 or 128 rows of one segment.
+//   phase 1: T[BM, RA] = x_tile . A_a^T over K in 64-column stages (a ring of buffer-addressed LDS DMA); RA = 64 where the adapter's rank
+//            allows, else 128.  T is rounded to bf16 and written to LDS in the stage layout, so that
 //   phase 2: for every 128-column tile of y:  acc = T . B_a[tile]^T  (K = the adapter's padded rank, one or two stages of
-//            B from L2), times the adapter's scale, rounded, transposed through LDS and added to the y pieces, which were
-//            requested together with the B tile while the previous tile was being finished.
+//            B from L2, requested while the previous tile is being finished), times the adapter's scale, rounded, transposed through
+//            LDS and added to the y pieces, which were requested five tiles ahead.
+// What bounds it at a request's sizes is not HBM's rate but the chain of latencies -- segment table, 20 stages, 5 .. 10 tiles -- in workgroups
+// that are one to a CU.  Hence as many stages under way as 128 KB hold (seven of 16 KB instead of two of 32: with 128 rows and all 128 rank rows
+// a stage took 0.45 us), the y pieces of the first five tiles requested while phase 1 runs, and 64-row blocks while they fit one
+// round of the 256 CUs, so that fewer of them repeat phase 1 for other columns.
+// 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 24.9 -> 19.8 us.
 // Rows / columns of A_a / B_a beyond the adapter's rank are zero by contract, so the padded rank only saves work.
-// Batches with few row blocks deal the column tiles of y to several workgroups (blockIdx.z), each of which repeats
+// Batches with few row blocks deal the column tiles of y to several workgroups, each of which repeats
 // phase 1 for its rows: x is then read from L2 more than once, which such small batches do not notice.
 // Grouped form (kh_sgmv_fused_grouped_bf16): several layers that read the same x with the same segments (the to_k / to_v
 // projections of every cross-attention read the one text context) in one launch, blockIdx.z = (layer, column range),
 // per-layer A / B / y from a device table: 77-row requests give a single layer's launch a few microseconds of traffic,
 // 120 layers fill the chip.
 #include "kh_common.h"
+#include <type_traits>
 
 namespace {
 
@@ -41,19 +47,19 @@ struct FusedParams {
   const uint64_t* table;   // grouped form: rows {a_all, b_all, y} of device pointers, one per layer; null: the fields above
 };
 
-constexpr int BM = 128, BR = 128;                 // rows of a workgroup, rank columns (RP <= 128)
-constexpr int STAGE = (BM + BR) * 128;            // 64 K-columns of x rows and of A rows: 32 KB
-constexpr int NST = 3;
-constexpr int T_OFF = 0, T_BYTES = 2 * BM * 128;  // phase 2: T as two 64-column stages of 128-byte rows (32 KB)
-constexpr int B_OFF = T_BYTES, B_TILE = 2 * 128 * 128;   // two buffers of a B tile (128 y columns x 128 rank columns)
-constexpr int C_OFF = B_OFF + 2 * B_TILE;         // staging of 64 output rows x (128 + 8) columns
+constexpr int RING = 128 * 1024;                  // phase 1's stages; phase 2: T, then two buffers of a B tile
+constexpr int B_TILE = 2 * 128 * 128;             // 128 y columns x 128 rank columns, as two 64-column stages
+constexpr int C_OFF = RING;                       // staging of 64 output rows x (128 + 8) columns
 constexpr int LDC = 128 + 8;
 constexpr int LDS_BYTES = C_OFF + 64 * LDC * 2;
-static_assert(NST * STAGE <= C_OFF, "phase 2's T and B buffers reuse the ring; the staging tile lies behind it");
 static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
+template <int BM>
 __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
+  constexpr int TI = BM / 64, T_BYTES = 2 * BM * 128;   // a wave's 32-row tiles; T as two 64-column stages of 128-byte rows
+  constexpr int YD = BM == 64 ? 5 : 2;                  // tiles whose y pieces are under way or here
+  static_assert(T_BYTES + 2 * B_TILE <= RING, "T and the B buffers lie in the ring");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int seg = blockIdx.y;
   const int r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1], ad = p.seg_adapter[seg];
@@ -76,96 +82,19 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3;        // 2 x 4 waves: a wave owns 64 rows x 32 columns of a 128 x 128 tile
+  const int wm = wave >> 2, wn = wave & 3;        // 2 x 4 waves: a wave owns BM / 2 rows x 32 columns of a BM x 128 tile
   const int l32 = lane & 31, lh = lane >> 5;
   const int sw = (l32 >> 1) & 7;
 
   auto clamp32 = [](size_t bytes) { return (int)(uint32_t)(bytes < 0xFFFFFFFFull ? bytes : 0xFFFFFFFFull); };
   auto mk = [&](const bf16_t* base, size_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, clamp32(bytes), 0x00020000); };
 
-  // ---- phase 1: T = x_tile . A^T ----
-  // DMA units of 8 rows x 128 bytes: 16 x units and 16 A units per stage, two of each per wave; a lane's byte offset
-  // (row, swizzled piece) never changes, the K tile is a scalar offset
-  const rsrc_t rs_x = mk(x + (size_t)m0 * K, (size_t)(M - m0) * K * 2);
-  const rsrc_t rs_a = mk(A, (size_t)RP * K * 2);
-  uint32_t vx[2], va[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int r = (wave * 2 + q) * 8 + (lane >> 3);
-    const uint32_t pcb = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
-    int row = m0 + r; row = row < M ? row : M - 1;
-    vx[q] = (uint32_t)(row - m0) * (uint32_t)K * 2u + pcb;
-    va[q] = (uint32_t)(r < RP ? r : RP - 1) * (uint32_t)K * 2u + pcb;   // (rows beyond RP: any valid row; their T columns are never used)
-  }
-  auto issue1 = [&](int t) {
-    char* stage = smem + (t % NST) * STAGE;
-    const int so = t * 128;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lptr_t)(stage + (wave * 2 + q) * 1024), 16, vx[q], so, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lptr_t)(stage + BM * 128 + (wave * 2 + q) * 1024), 16, va[q], so, 0, 0);
-    }
-  };
-  // fragments of a 64-column stage: rows (wm * 64 + i * 32 + l32) of the first operand, (wn * 32 + l32) of the second
-  struct Fr { bf16x8 a[4][2]; bf16x8 b[4]; };
-  auto read_frags = [&](const char* st_a, const char* st_b, Fr& f) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const int po = ((2 * ks + lh) ^ sw) * 16;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) f.a[ks][i] = *reinterpret_cast<const bf16x8*>(st_a + (wm * 64 + i * 32 + l32) * 128 + po);
-      f.b[ks] = *reinterpret_cast<const bf16x8*>(st_b + (wn * 32 + l32) * 128 + po);
-    }
-  };
-  f32x16 acc[2];
-  auto zero_acc = [&]() {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
-  };
-  auto mma = [&](const Fr& f, int ks_n) {   // the first ks_n 16-column steps of the stage
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      if (ks < ks_n) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[ks][i], f.b[ks], acc[i], 0, 0, 0);
-      }
-  };
-  const int KT = K / 64;
-  zero_acc();
-  issue1(0);
-  if (KT > 1) issue1(1);
-  Fr f;
-  for (int t = 0; t < KT; ++t) {
-    if (t + 1 < KT) wait_cnt<4, 0>(); else wait_cnt<0, 0>();   // this wave's loads of tile t are complete (4 per tile)
-    __builtin_amdgcn_s_barrier();                              // everyone's are, and everyone has read tile t-1
-    if (t + 2 < KT) issue1(t + 2);                             // into the stage of tile t-1
-    const char* st = smem + (t % NST) * STAGE;
-    read_frags(st, st + BM * 128, f);
-    mma(f, 4);
-  }
-  __syncthreads();   // the ring is dead
-
-  // T, rounded to bf16, into the stage layout (row r, logical 16-byte piece c of stage s at physical piece c ^ ((r/2) % 8));
-  // a lane holds column wn * 32 + l32 of rows 8 * (v / 4) + 4 * lh + (v % 4) of each of its two 32-row tiles
-  {
-    const int col = wn * 32 + l32, s = col >> 6, cc = col & 63, piece = cc >> 3, within = (cc & 7) * 2;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int r = wm * 64 + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-        *reinterpret_cast<bf16_t*>(smem + T_OFF + s * (BM * 128) + r * 128 + ((piece ^ ((r >> 1) & 7)) * 16) + within) = (bf16_t)acc[i][v];
-      }
-  }
-
-  // ---- phase 2: y tile += scale * T . B_tile^T for every 128-column tile ----
+  // ---- phase 2's requests: B tile j; the y pieces of tile j (those of the first tiles go out while phase 1 runs) ----
   const int j0 = zz * p.tiles_per_z;
   const int n_tiles = (N / 128 - j0) < p.tiles_per_z ? (N / 128 - j0) : p.tiles_per_z;   // tiles j0 .. j0 + n_tiles - 1
   const int ks_total = rank / 16;                 // MFMA steps over the padded rank (2, 4, 6 or 8)
   const int nstage = (rank + 63) / 64;            // B stages per tile (1 or 2)
-  // B tile j: rows n0 .. n0+127 of B (row stride RP), 64 rank columns per stage; 16 units per stage, two per wave
+  // B tile j: rows n0 .. n0+127 of B (row stride RP), 64 rank columns per stage; 16 units of 8 rows x 128 bytes per stage, two per wave
   const rsrc_t rs_b = mk(B, (size_t)N * RP * 2);
   uint32_t vb[2];
 #pragma unroll
@@ -174,53 +103,148 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
     vb[q] = (uint32_t)r * (uint32_t)RP * 2u + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
   }
   constexpr int CPR = 16, ECH = 64 * CPR / 512;   // 16-byte pieces per staged row; per thread and 64-row pass: 2
-  u32x4 yr[2][ECH];                               // this thread's y pieces of the tile in flight (two passes)
-  auto issue2 = [&](int j) {                      // B tile j and the y pieces of tile j
-    char* bt = smem + B_OFF + (j & 1) * B_TILE;
-    const int so = (j0 + j) * 128 * RP * 2;
+  u32x4 yr[YD][TI][ECH];                          // this thread's y pieces
+  // (the first stage of the first B tile goes out ahead of phase 1, into the staging tile)
+  auto b_stage = [&](int j, int s) { return j == 0 && s == 0 ? smem + C_OFF : smem + T_BYTES + (j & 1) * B_TILE + s * (128 * 128); };
+  auto tile_row = [&](int ps, int srow) { return m0 + (TI == 2 ? (srow >> 5) * 64 + ps * 32 + (srow & 31) : srow); };   // of a pass's staged row
+  auto issue_b = [&](int j, int s) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int q = 0; q < 2; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lptr_t)(b_stage(j, s) + (wave * 2 + q) * 1024), 16, vb[q] + s * 128, (j0 + j) * 128 * RP * 2, 0, 0);
+  };
+  auto issue_y = [&](int j, u32x4 (&d)[TI][ECH]) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        // (a second stage beyond the padded rank is still fetched when RP allows: it multiplies nothing)
-        const uint32_t off = (s * 128 < RP * 2) ? vb[q] + s * 128 : 0xFFFFFFFFu;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (lptr_t)(bt + s * (128 * 128) + (wave * 2 + q) * 1024), 16, off, so, 0, 0);
-      }
-#pragma unroll
-    for (int ps = 0; ps < 2; ++ps)
+    for (int ps = 0; ps < TI; ++ps)
 #pragma unroll
       for (int q = 0; q < ECH; ++q) {
         const int c = tid + q * 512, srow = c / CPR, ch = c % CPR;
-        int grow = m0 + (srow >> 5) * 64 + ps * 32 + (srow & 31);
+        int grow = tile_row(ps, srow);
         grow = grow < M ? grow : M - 1;
-        yr[ps][q] = *reinterpret_cast<const u32x4*>(y + (size_t)grow * N + (j0 + j) * 128 + ch * 8);
+        d[ps][q] = *reinterpret_cast<const u32x4*>(y + (size_t)grow * N + (j0 + j) * 128 + ch * 8);
       }
   };
+
+  // ---- phase 1: T = x_tile . A^T ----
+  // DMA units of 8 rows x 128 bytes: TI of x and one or two of A per wave and stage; a lane's byte offset (row, swizzled piece)
+  // never changes, the K tile is a scalar offset
+  const rsrc_t rs_x = mk(x + (size_t)m0 * K, (size_t)(M - m0) * K * 2);
+  const rsrc_t rs_a = mk(A, (size_t)RP * K * 2);
+  uint32_t vx[TI], va[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int r = (wave + 8 * q) * 8 + (lane >> 3);
+    const uint32_t pcb = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
+    if (q < TI) {
+      int row = m0 + r; row = row < M ? row : M - 1;
+      vx[q < TI ? q : 0] = (uint32_t)(row - m0) * (uint32_t)K * 2u + pcb;
+    }
+    va[q] = r < rank ? (uint32_t)r * (uint32_t)K * 2u + pcb : 0xFFFFFFFFu;   // (rows beyond the rank: zeros, not read from memory)
+  }
+  // fragments of a 64-column stage: rows (wm * BM / 2 + i * 32 + l32) of the first operand, (wn * 32 + l32) of the second
+  struct Fr { bf16x8 a[4][TI]; bf16x8 b[4]; };
+  auto read_frags = [&](const char* st_a, const char* st_b, Fr& f) {
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int po = ((2 * ks + lh) ^ sw) * 16;
+#pragma unroll
+      for (int i = 0; i < TI; ++i) f.a[ks][i] = *reinterpret_cast<const bf16x8*>(st_a + (wm * (BM / 2) + i * 32 + l32) * 128 + po);
+      f.b[ks] = *reinterpret_cast<const bf16x8*>(st_b + (wn * 32 + l32) * 128 + po);
+    }
+  };
+  f32x16 acc[TI];
+  auto zero_acc = [&]() {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+  };
+  auto mma = [&](const Fr& f, int ks_n) {   // the first ks_n 16-column steps of the stage
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      if (ks < ks_n) {
+#pragma unroll
+        for (int i = 0; i < TI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[ks][i], f.b[ks], acc[i], 0, 0, 0);
+      }
+  };
+  const int KT = K / 64;
+  zero_acc();
+  Fr f;
+  auto shrink = [&](auto au) {                    // au: A units per wave
+    constexpr int AU = decltype(au)::value, STAGE = (BM + AU * 64) * 128, NST = RING / STAGE, PD = NST - 1, CNT = TI + AU;
+    const bool mine = wn * 32 < AU * 64;          // (waves whose rank columns lie beyond RA only move operands)
+    auto issue1 = [&](int t, int st) {
+      const int so = t * 128;
+#pragma unroll
+      for (int q = 0; q < TI; ++q) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lptr_t)(smem + st + (wave + 8 * q) * 1024), 16, vx[q], so, 0, 0);
+#pragma unroll
+      for (int q = 0; q < AU; ++q)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (lptr_t)(smem + st + BM * 128 + (wave + 8 * q) * 1024), 16, va[q], so, 0, 0);
+    };
+#pragma unroll
+    for (int t = 0; t < PD; ++t)
+      if (t < KT) issue1(t, t * STAGE);
+    int st = 0, fill = PD * STAGE;                // stages of tile t and of tile t + PD
+    auto step = [&](int t) {
+      // this wave's loads of tile t are complete (y pieces among the younger ones only make it wait for more)
+      if (t + PD <= KT) wait_cnt<CNT*(PD - 1), 0>(); else wait_cnt<0, 0>();
+      __builtin_amdgcn_s_barrier();               // everyone's are, and everyone has read tile t-1
+      if (t + PD < KT) issue1(t + PD, fill);      // into the stage of tile t-1
+      if (mine) {
+        read_frags(smem + st, smem + st + BM * 128, f);
+        mma(f, 4);
+      }
+      st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+      fill = fill + STAGE == NST * STAGE ? 0 : fill + STAGE;
+    };
+    // the y pieces of tile i after step i of every YD-th part of the stages
+    int t = 0;
+#pragma unroll
+    for (int i = 0; i < YD; ++i) {
+      if (i < n_tiles) issue_y(i, yr[i]);
+      for (; t < (i + 1) * KT / YD; ++t) step(t);
+    }
+  };
+  issue_b(0, 0);
+  if (rank <= 64) shrink(std::integral_constant<int, 1>{}); else shrink(std::integral_constant<int, 2>{});
+  __syncthreads();   // the ring is dead
+  if (nstage > 1) issue_b(0, 1);
+
+  // T, rounded to bf16, into the stage layout (row r, logical 16-byte piece c of stage s at physical piece c ^ ((r/2) % 8));
+  // a lane holds column wn * 32 + l32 of rows 8 * (v / 4) + 4 * lh + (v % 4) of each of its two 32-row tiles
+  {
+    const int col = wn * 32 + l32, s = col >> 6, cc = col & 63, piece = cc >> 3, within = (cc & 7) * 2;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = wm * (BM / 2) + i * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+        *reinterpret_cast<bf16_t*>(smem + s * (BM * 128) + r * 128 + ((piece ^ ((r >> 1) & 7)) * 16) + within) = (bf16_t)acc[i][v];
+      }
+  }
+
+  // ---- phase 2: y tile += scale * T . B_tile^T for every 128-column tile ----
   const bool full = m0 + BM <= M;
   __syncthreads();   // T is written
-  issue2(0);
   bf16_t* sC = reinterpret_cast<bf16_t*>(smem + C_OFF);
-  for (int j = 0; j < n_tiles; ++j) {
-    // B tile j (this wave's share) and this thread's y pieces are here; the four stores of the tile before (younger: a
-    // wave's memory operations complete in order) may still be on their way when every thread of the tile stores
-    if (j > 0 && full) wait_cnt<2 * ECH, 0>(); else wait_cnt<0, 0>();
+  auto tile = [&](int j, u32x4 (&yc)[TI][ECH]) {
+    // B tile j (this wave's share) is here; what is younger -- a wave's memory operations complete in order --, the stores of the tile
+    // before and the y pieces requested with them, may still be on its way
+    if (j > 0 && full && j - 1 + YD < n_tiles) wait_cnt<2 * TI * ECH, 0>(); else if (j > 0 && full) wait_cnt<TI * ECH, 0>(); else wait_cnt<0, 0>();
     __builtin_amdgcn_s_barrier();
-    u32x4 yc[2][ECH];
-#pragma unroll
-    for (int ps = 0; ps < 2; ++ps)
-#pragma unroll
-      for (int q = 0; q < ECH; ++q) yc[ps][q] = yr[ps][q];
-    if (j + 1 < n_tiles) issue2(j + 1);           // flies under this tile's MFMAs and epilogue
-    const char* bt = smem + B_OFF + (j & 1) * B_TILE;
+    if (j + 1 < n_tiles) {                        // flies under this tile's MFMAs and epilogue
+      issue_b(j + 1, 0);
+      if (nstage > 1) issue_b(j + 1, 1);
+    }
     zero_acc();
     for (int s = 0; s < nstage; ++s) {
-      read_frags(smem + T_OFF + s * (BM * 128), bt + s * (128 * 128), f);
+      read_frags(smem + s * (BM * 128), b_stage(j, s), f);
       const int left = ks_total - 4 * s;
       mma(f, left < 4 ? left : 4);
     }
-    // epilogue: two passes of 64 rows (the waves' upper / lower 32-row tiles): scale, round, transpose through LDS, add y
+    if (j == 0) __syncthreads();                  // its B lies in the staging tile
+    // epilogue: passes of 64 rows (of 128: the waves' upper / lower 32-row tiles): scale, round, transpose through LDS, add y
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TI; ++i) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int row = wm * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
@@ -230,7 +254,7 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
 #pragma unroll
       for (int q = 0; q < ECH; ++q) {
         const int c = tid + q * 512, srow = c / CPR, ch = c % CPR;
-        const int grow = m0 + (srow >> 5) * 64 + i * 32 + (srow & 31);
+        const int grow = tile_row(i, srow);
         if (grow < M) {
           u32x4 o = *reinterpret_cast<const u32x4*>(sC + srow * LDC + ch * 8);
 #pragma unroll
@@ -240,6 +264,14 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
         }
       }
       __syncthreads();
+    }
+    if (j + YD < n_tiles) issue_y(j + YD, yc);
+  };
+  for (int j = 0; j < n_tiles; j += YD) {
+#pragma unroll
+    for (int i = 0; i < YD; ++i) {
+      if (j + i >= n_tiles) break;
+      tile(j + i, yr[i]);
     }
   }
 #endif
@@ -265,18 +297,27 @@ int sgmv_fused_impl(const void* x, const void* a_all, const void* b_all, void* y
   p.x = (const bf16_t*)x; p.a_all = (const bf16_t*)a_all; p.b_all = (const bf16_t*)b_all; p.y = (bf16_t*)y;
   p.seg_start = seg_start; p.seg_adapter = seg_adapter; p.adapter_rank = adapter_rank; p.adapter_scale = adapter_scale;
   p.K = (int)K; p.N = (int)N; p.RP = (int)RP; p.table = table;
-  if (hipError_t e = kh_allow_lds<sgmv_fused_kernel>(LDS_BYTES); e != hipSuccess) return (int)e;
-  // few row blocks: the column tiles of y are dealt to several workgroups (each recomputes its rows' T) until the chip is covered
-  const int64_t row_wgs = ((max_seg_rows + BM - 1) / BM) * n_segments * n_layers, n_tiles = N / 128;
-  int64_t z = row_wgs >= 256 ? 1 : (256 + row_wgs - 1) / row_wgs;
-  z = z < n_tiles ? z : n_tiles;
+  // Row blocks of 64 while they about fit one round of the CUs (not all segments have max_seg_rows rows), of 128 otherwise: two rounds of 64
+  // rows cost more than one of 128 (8 x 4096 rows: 40 against 32 us; 4 x 3136: 19 against 24).  Few row blocks: the column tiles of y are dealt to
+  // several workgroups, each of which recomputes its rows' T, while that brings their number nearer to the CUs' (7 x 744 rows: 27 us with
+  // one range, 20 with three, 28 with four, more than the CUs).
+  const int bm = (max_seg_rows + 63) / 64 * n_segments * n_layers > 320 ? 128 : 64;
+  const int64_t row_blocks = (max_seg_rows + bm - 1) / bm;
+  const int64_t row_wgs = row_blocks * n_segments * n_layers, n_tiles = N / 128;
+  int64_t z = 300 / row_wgs;
+  z = z < 1 ? 1 : z < n_tiles ? z : n_tiles;
   p.tiles_per_z = (int)((n_tiles + z - 1) / z);
   z = (n_tiles + p.tiles_per_z - 1) / p.tiles_per_z;
   p.z_per_layer = (int)z;
   if (z * n_layers > 65535) return KH_ERR_TOO_LARGE;
-  dim3 grid((unsigned)((max_seg_rows + BM - 1) / BM), (unsigned)n_segments, (unsigned)(z * n_layers));
-  kh_launch(KH_TAG_SGMV_FUSED, sgmv_fused_kernel, grid, dim3(512), LDS_BYTES, (hipStream_t)stream, p);
-  KH_RETURN_LAST_ERROR();
+  auto go = [&](auto bmc) {
+    constexpr int BM = decltype(bmc)::value;
+    if (hipError_t e = kh_allow_lds<sgmv_fused_kernel<BM>>(LDS_BYTES); e != hipSuccess) return (int)e;
+    kh_launch(KH_TAG_SGMV_FUSED, sgmv_fused_kernel<BM>, dim3((unsigned)row_blocks, (unsigned)n_segments, (unsigned)(z * n_layers)), dim3(512), LDS_BYTES,
+              (hipStream_t)stream, p);
+    KH_RETURN_LAST_ERROR();
+  };
+  return bm == 128 ? go(std::integral_constant<int, 128>{}) : go(std::integral_constant<int, 64>{});
 }
 
 }  // namespace

@@ -75,6 +75,37 @@ def test_lora_linear_f32_not_finite():
     assert (y[ok] - ref[ok]).abs().le(1e-5 * ref[ok].abs() + 1e-4).all()
 
 
+@pytest.mark.parametrize("lens,longest,K,N,RP", [
+    ([1, 63, 64, 65, 0, 129], 129, 64, 128, 128),         # 64-row blocks, one stage, one column tile
+    ([1, 63, 64, 65, 128, 200], 200, 640, 1280, 128),     # ... ten column tiles in ranges of one
+    ([127, 128, 129, 1, 300, 700], 4000, 704, 640, 128),  # 128-row blocks (the caller's bound on the rows decides), eleven stages
+    ([127, 128, 129, 1, 300, 700], 4000, 1280, 1664, 64),  # ... thirteen column tiles in one range
+], ids=str)
+def test_sgmv_fused_row_blocks(lens, longest, K, N, RP):
+    """Both row blocks of kh_sgmv_fused_bf16 at the edges of segments, ranks on either side of 64, every rank row beyond the padded rank
+    poisoned (it must not be read)."""
+    from katz_amd import ops
+
+    say("sgmv fused row blocks", lens, longest, K, N, RP)
+    d, g = dev(), torch.Generator().manual_seed(K + N)
+    ranks = [8, 64, 32, 60, 16, 100 if RP == 128 else 64]
+    start = [0]
+    for n in lens:
+        start.append(start[-1] + n)
+    x, base = bf16_round(torch.randn(start[-1], K, generator=g)), bf16_round(torch.randn(start[-1], N, generator=g))
+    adapters = [(bf16_round(torch.randn(r, K, generator=g) * 0.05), bf16_round(torch.randn(N, r, generator=g) * 0.05), 0.5 + 0.1 * i) for i, r in enumerate(ranks)]
+    a, b = torch.zeros(6, RP, K), torch.zeros(6, N, RP)
+    pad = [-(-r // 32) * 32 for r in ranks]
+    for i, (A, B, _) in enumerate(adapters):
+        a[i, :ranks[i]], b[i, :, :ranks[i]] = A, B
+        a[i, pad[i]:] = float("nan")
+    i32 = dict(dtype=torch.int32, device=d)
+    y = base.to(d, BF)
+    ops.sgmv_fused_(y, x.to(d, BF), a.to(d, BF), b.to(d, BF), torch.tensor(start, **i32), torch.arange(6, **i32), torch.tensor(pad, **i32),
+                    torch.tensor([s for _, _, s in adapters], device=d), longest)
+    assert_close_rel(y, O.sgmv(x, start, list(range(6)), adapters, base), 2e-2, "row blocks")
+
+
 @pytest.mark.parametrize("host,dtype,ranks", [(False, torch.bfloat16, (64, 32)), (True, torch.float16, (16,)), (False, torch.float32, (4, 8, 100)), (True, torch.bfloat16, (5, 7))],
                          ids=str)
 def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
