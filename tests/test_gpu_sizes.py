@@ -106,6 +106,23 @@ def test_sgmv_fused_row_blocks(lens, longest, K, N, RP):
     assert_close_rel(y, O.sgmv(x, start, list(range(6)), adapters, base), 2e-2, "row blocks")
 
 
+@pytest.mark.parametrize("N,C,H,W,G", [(1, 32, 1, 1, 4), (2, 320, 7, 9, 32), (1, 1280, 3, 11, 32), (1, 1280, 26, 38, 32), (3, 2560, 5, 13, 32), (1, 4096, 2, 17, 512),
+                                       (1, 320, 104, 152, 32)], ids=str)
+def test_group_norm_statistics_pass(N, C, H, W, G):
+    """kh_group_norm_bf16's statistics: pixel counts below, at and past whole batches of loads, one and two chunks of channels per thread, with
+    and without the per-channel term."""
+    from katz_amd import ops
+
+    say("group norm statistics", N, C, H, W, G)
+    d, g = dev(), torch.Generator().manual_seed(C + H)
+    x, gamma, beta = bf16_round(torch.randn(N, C, H, W, generator=g) + 0.5), bf16_round(1 + 0.3 * torch.randn(C, generator=g)), bf16_round(torch.randn(C, generator=g))
+    add = bf16_round(torch.randn(N, C, generator=g))
+    xd = x.to(d, BF).contiguous(memory_format=torch.channels_last)
+    for a in (None, add):
+        y = ops.group_norm(xd, G, gamma.to(d, BF), beta.to(d, BF), 1e-5, "silu", add_nc=None if a is None else a.to(d, BF))
+        assert_close_rel(y, O.group_norm(x if a is None else x + a[:, :, None, None], G, gamma, beta, 1e-5, "silu"), 2e-2, "group norm")
+
+
 @pytest.mark.parametrize("host,dtype,ranks", [(False, torch.bfloat16, (64, 32)), (True, torch.float16, (16,)), (False, torch.float32, (4, 8, 100)), (True, torch.bfloat16, (5, 7))],
                          ids=str)
 def test_packs_of_a_whole_model_in_two_launches(host, dtype, ranks):
