@@ -855,7 +855,7 @@ def main():
         "config": {"workload": "SDXL UNet2DConditionModel step, latent [2,4,128,128] (1024x1024, CFG batch 2), "
                                "2 LoRAs (r64 s0.8 + r32 s0.6) on 722 linears, 1 ControlNet residual set, HIP graph",
                    "global_batch": 2, "parallelism": "single GPU"},
-        "roofline": {"kernel": "LoRA linear GEMMs (lora_gemm_pipe / _wide / _ksplit: base GEMM + LoRA delta), all launches of "
+        "roofline": {"kernel": "LoRA linear GEMMs (lora_gemm_pipe / _wide / _fine: base GEMM + LoRA delta), all launches of "
                                "one step incl. the shrink launches",
                      "bound": "mfma", "achieved": round(achieved_tf, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved_tf / PEAK_BF16_TFLOPS, 4), "traffic": traffic,

@@ -242,24 +242,23 @@ int lora_gemm_pipe_launch_il(const LoraGemmParams& p, hipStream_t stream);
 // query projection + cross-attention in its epilogue (xa_k set)
 bool lora_gemm_pipe_xattn_ok(const LoraGemmParams& p);
 int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, hipStream_t stream);
-// Narrow-output variant (lora_gemm_ksplit.hip): (32 * row_groups) x 160 tiles, 8 waves as row_groups x k-slices;
+// (32 * row_groups) x 160 tiles whose 8 waves are row_groups x k-slices (lora_gemm_ksplit.hip), tile codes 40 and 41;
 // plain or K-extended GEMM with bias / residual, K % 64 == 0.  row_groups 2 or 4.
-bool lora_gemm_ksplit_ok(const LoraGemmParams& p);
 int lora_gemm_ksplit_launch(const LoraGemmParams& p, int row_groups, hipStream_t stream);
-// Shrink and GEMM in one launch on the 128 x 160 tiles, every workgroup computing a piece of T first (p.a_cat / col_scale /
-// b_cat set, p.t_ext = scratch for the shrink result, p.il_cnt = counters, p.r_used <= 96 of R = 128).
-bool lora_gemm_ksplit_coop_ok(const LoraGemmParams& p);
-int lora_gemm_ksplit_launch_coop(const LoraGemmParams& p, hipStream_t stream);
-int lora_gemm_ksplit_coop_timeouts(int* count, int clear);
-bool lora_gemm_ksplit_conv_ok(const LoraGemmParams& p);
-int lora_gemm_ksplit_launch_conv(const LoraGemmParams& p, int row_groups, hipStream_t stream);
 // the convolution that also leaves GroupNorm statistics (gn_cg / gn_hw set): row groups of the 160-column tiles it would run
 // on, 0 when the rules give it other tiles or the groups do not fit them
 int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
-// Fine tiles (lora_gemm_fine.hip), for sizes that give each CU at most one of them, with the sums in the order of the 128 x 128 (order 0) or
-// the 64 x 160 kernel (order 4); plain or K-extended GEMM and (order 4) 3x3 convolutions.  Form -1: not suited.
+// Fine tiles (lora_gemm_fine.hip), with the sums in the order of the 128 x 128 (order 0), the 128 x 160 (order 2) or the 64 x 160 kernel
+// (order 4); plain or K-extended GEMM and (orders 2 and 4) 3x3 convolutions.  ok: what the kernel takes at all; form: -1 where order 0
+// is not suited (orders 2 and 4: the caller has seen to N % 160 and the number of tiles).
+bool lora_gemm_fine_ok(const LoraGemmParams& p);
 int lora_gemm_fine_form(const LoraGemmParams& p, int order);
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream);
+// Shrink and GEMM in one launch on the 128 x 160 tiles, every workgroup computing a piece of T first (p.a_cat / col_scale /
+// b_cat set, p.t_ext = scratch for the shrink result, p.il_cnt = counters, p.r_used <= 96 of R = 128).
+bool lora_gemm_fine_coop_ok(const LoraGemmParams& p);
+int lora_gemm_fine_launch_coop(const LoraGemmParams& p, hipStream_t stream);
+int lora_gemm_fine_coop_timeouts(int* count, int clear);
 // Wide-tile variant (lora_gemm_wide.hip): 256 x 320 tiles, 8 waves; plain or K-extended GEMM with bias / residual /
 // GEGLU; M % 256 == 0, N % 320 == 0, K % 64 == 0.
 bool lora_gemm_wide_ok(const LoraGemmParams& p);

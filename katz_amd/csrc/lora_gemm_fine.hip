@@ -14,14 +14,19 @@
 //   * a ring of as many stages as LDS holds (up to 8), and
 //   * the XCD's block of W fetched into its L2 by all its workgroups before the K loop meets it.
 //
-// Orders (ORD): the 128 x 128 / 256 x 320 kernels add along K one 16-column step after the other (0), the 64 x 160 kernel in four
-// slices of 16 of every 64 columns that are added at the end (4).  v_mfma 16x16x32 gives the bits of two chained 16-column steps of
+// Orders (ORD): the 128 x 128 / 256 x 320 kernels add along K one 16-column step after the other (0), the 160-column kernels in four
+// slices of 16 (4) or two of 32 (2) of every 64 columns that are added at the end.  v_mfma 16x16x32 gives the bits of two chained 16-column steps of
 // 32x32x16, and 16x16x16 those of one, so 16-row tiles can follow either.  Row statistics are sums over 128 columns (order 0) or
-// 160 (order 4): layers that leave them run on tiles of that width.
+// 160 (orders 2 and 4): layers that leave them run on tiles of that width.
 //
 // Operands reach LDS by buffer loads (8 rows x 128 bytes per instruction, XOR-swizzled pieces, rows past M read zeros).
 #include "kh_common.h"
 #include "lora_gemm.h"
+#include "lora_shrink_tile.h"
+
+// Bounded waits of the cooperative shrink that have run out on this GPU; read (and cleared) by kh_lora_split_timeouts
+// together with the count of the in-launch shrink of lora_gemm_pipe.hip.
+static __device__ int kh_coop_timeout_count;
 
 namespace {
 
@@ -52,10 +57,10 @@ struct FCfg {
   static constexpr bool GLU = GLU_;                      // GEGLU epilogue
   static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : 4, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
+  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
   // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
   static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
-  static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 0 ? 2 : 1;   // a wave's MFMA tiles, its k-steps per stage
+  static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 4 ? 1 : 2;   // a wave's MFMA tiles, its k-steps per stage
   static constexpr bool DB = TM * TN * G * 4 <= 96 && !GLU;      // two fragment buffers where the registers allow it
   static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
   static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
@@ -76,9 +81,19 @@ struct FCfg {
 
 // CONV: x is an NHWC image and row m of the GEMM is output pixel m of a 3x3 convolution with padding 1 (K = 9 * Cin ordered
 // (kh, kw, ci)): a stage is 64 channels of one tap, taps outside the image read zeros (an offset beyond the buffer).
-// Rows come in segments of seg_rows (an image of the convolution, everything otherwise) that start a tile of their own.
-template <class C, bool CONV>
-__global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
+// Rows come in segments of seg_rows (an image of a convolution that leaves statistics, everything otherwise) that start a tile of their own.
+//
+// COOP: the launch computes its own shrink, cooperatively.  These tiles fill every CU, so there is no idle CU for shrink
+// workgroups beside the GEMM ones; instead EVERY workgroup first computes one piece of T -- 32 rows x 96 rank columns: the
+// n_tiles = 4 x (ldt / 128) workgroups of a row block of 128 rows share that block's 4 row quarters x ldt / 128 column
+// groups of T, workgroup n_blk takes quarter n_blk % 4 of group n_blk / 4 --, stores it write-through, zeroes the 32
+// padding columns of its group, counts itself into the row block's counter and then runs its GEMM tile; before its first
+// request for T (the last K tiles) it waits, bounded, for the row block's count and reads T past the L2.  A workgroup
+// never waits before its own piece is out, so the launch makes progress in whatever order its workgroups become
+// resident, as long as no OTHER launch whose workgroups wait for each other shares the device with it (the binding does
+// not use this form on a second stream).
+template <class C, bool CONV, bool COOP>
+__global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, NST = C::NST, PD = C::PD;
@@ -102,6 +117,30 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
   const int KT1 = K / BK, r_ext = p.r_used > 0 ? p.r_used : p.R;
   const int KT = KT1 + (EXT && p.t_ext != nullptr ? (r_ext + BK - 1) / BK : 0);
   const bool has_hi = pw < C::N_HI;
+
+  if constexpr (COOP) {
+    static_assert(SCfg<4, 1, 3>::LDS <= C::TOUCH_OFF && BM == 128, "the shrink piece's rings fit the GEMM ring; four quarters per row block");
+    // this workgroup's piece of T = bf16((x . A_cat^T) * col_scale) (with a folded LayerNorm in front: the form documented at
+    // ShrinkParams), then the padding columns, then the arrival
+    const int q4 = n_blk & 3, grp = n_blk >> 2;
+    ShrinkParams sp;
+    sp.x = p.x; sp.a_cat = p.a_cat; sp.col_scale = p.col_scale; sp.t = const_cast<bf16_t*>(p.t_ext);
+    sp.M = M; sp.K = K; sp.R = p.ldt;
+    sp.ln_part = p.ln_part; sp.ln_ca1 = p.ln_ca1; sp.ln_ca2 = p.ln_ca2; sp.ln_eps = p.ln_eps;
+    // (a quarter that starts past the last row has nothing to compute: the tile's addressing assumes m0 < M)
+    if (m0 + 32 * q4 < M) lora_shrink_tile<SCfg<4, 1, 3>, true, 512>(sp, m0 + 32 * q4, grp * 128, smem);
+    if (tid < 128) {   // columns 96 .. 127 of the group: 32 rows x 4 pieces of 16 bytes
+      const int row = m0 + 32 * q4 + (tid >> 2);
+      if (row < M) {
+        uint32_t* dst = reinterpret_cast<uint32_t*>(const_cast<bf16_t*>(p.t_ext) + (size_t)row * p.ldt + grp * 128 + 96 + (tid & 3) * 8);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) __hip_atomic_store(dst + e, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(0);                          // this thread's write-through stores have completed
+    __syncthreads();
+    if (tid == 0) __hip_atomic_fetch_add(p.il_cnt + m_blk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 
   // per-row and per-column terms: requested now, used after the K loop (older than every DMA load, so no wait falls in between)
   KhLnTileStats<BM, 512> ln_stats;
@@ -167,13 +206,27 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
     char* stage = smem + st;
     const int so = t * ROWB;
     if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
+      if (COOP && t == KT1) {
+        // first request for T: wait (bounded) until every workgroup of this row block has delivered its piece
+        if (lane == 0) {
+          int it = 0;
+          while (__hip_atomic_load(p.il_cnt + m_blk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p.n_tiles && ++it < (1 << 20))
+            __builtin_amdgcn_s_sleep(8);
+          if (it >= (1 << 20)) {
+            __hip_atomic_store(p.il_cnt + (p.M + 127) / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(&kh_coop_timeout_count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+      }
       const int c = (t - KT1) * BK;
 #pragma unroll
       for (int q = 0; q < LPS_HI; ++q) {
         if (q < LPS_LO || has_hi) {
           const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16,
-                                                   col < r_ext ? voff2[EXT ? q : 0] : OOB, c * 2, 0, 0);
+          const uint32_t vo = col < r_ext ? voff2[EXT ? q : 0] : OOB;
+          // (COOP) T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
+          if (COOP && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
+          else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 0);
         }
       }
       return;
@@ -218,7 +271,7 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
   int fa[KS], fb[KS];
 #pragma unroll
   for (int k = 0; k < KS; ++k) {
-    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * wk + lg) ^ swz(lr)) * 16;
+    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
     fa[k] = (wm * (BM / C::WM) + lr) * ROWB + po;
     fb[k] = (BM + wn * (BN / C::WN) + lr) * ROWB + po;
   }
@@ -291,14 +344,66 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
     ring_barrier();
     int st = 0;
     if constexpr (!C::DB) {
-      for (int t = 0; t < KT; ++t) {
-        if ((t & 7) == 0) touch(t + 24, 8);
-        Fr f;
-        read_frags(st, f);
-        mma(f);
+      // One set of W fragments, replaced one by one behind the matrix instructions that used them last, and two of x, a k-step each: the
+      // reads of the next k-step run under the matrix instructions of this one.  (A whole stage read and then multiplied takes the sum of both
+      // where the operands arrive in time: GEGLU on 64 x 320 tiles, 2048 / 5120 / 640, 25.2 -> 24.0 us.)  The barrier that shows the next stage lies before the last k-step, whose fragments have
+      // been read by then, so that the stage can be filled again.
+      Frag a[2][TM], b[TN];
+      auto read_a = [&](int st, int k, int set) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[set][i] = *reinterpret_cast<const Frag*>(smem + st + fa[k] + i * C::MF * ROWB);
+      };
+      auto read_b = [&](int st, int k, int j) { b[j] = *reinterpret_cast<const Frag*>(smem + st + fb[k] + j * C::MF * ROWB); };
+      auto mma1 = [&](int set, int j) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          if constexpr (C::MF == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[set][i], b[j], acc[i][j], 0, 0, 0);
+          else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][i], b[j], acc[i][j], 0, 0, 0);
+        }
+      };
+      auto kstep = [&](int set, int st_next, int k_next) {   // x in a[set]; the next k-step's fragments: step k_next of stage st_next
+        read_a(st_next, k_next, 1 - set);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          mma1(set, j);
+          read_b(st_next, k_next, j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      auto next_stage = [&]() {
         st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
-        if (t + 1 < KT) ring_barrier();
+        wait_cnt<63, 0>();
+        ring_barrier();
+      };
+      read_a(0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) read_b(0, 0, j);
+      if constexpr (KS == 2) {
+        for (int t = 0; t + 1 < KT; ++t) {
+          if ((t & 7) == 0) touch(t + 24, 8);
+          kstep(0, st, 1);
+          next_stage();
+          kstep(1, st, 0);
+        }
+        kstep(0, st, 1);
+      } else {
+        int t = 0;
+        for (; t + 2 < KT; t += 2) {
+          if ((t & 7) == 0) touch(t + 24, 8);
+          next_stage();
+          kstep(0, st, 0);
+          next_stage();
+          kstep(1, st, 0);
+        }
+        if (t + 1 < KT) {
+          next_stage();
+          kstep(0, st, 0);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) a[0][i] = a[1][i];
+        }
       }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) mma1(KS == 2 ? 1 : 0, j);
     } else {
     Fr f0, f1;
     read_frags(0, f0);
@@ -375,10 +480,10 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
 #pragma unroll
         for (int u = 0; u < UH / C::WK; ++u) {
           const int at = u * C::WK + wk, ij = at / C::G;
-          f32x4 s = part[at * 64 + lane];
+          f32x4 s = part[((pw - wk) * UH + at) * 64 + lane];
 #pragma unroll
           for (int k = 1; k < C::WK; ++k) {              // slice after slice
-            const f32x4 o = part[(k * UH + at) * 64 + lane];
+            const f32x4 o = part[((pw - wk + k) * UH + at) * 64 + lane];
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[e] += o[e];
           }
@@ -504,15 +609,15 @@ __global__ __launch_bounds__(512, 2) void lora_gemm_fine_kernel(const LoraGemmPa
 #endif
 }
 
-template <class C, bool CONV>
+template <class C, bool CONV, bool COOP = false>
 int launch_fine(LoraGemmParams p, hipStream_t stream) {
-  const int seg_rows = CONV ? p.conv_ho * p.conv_wo : p.M;
+  const int seg_rows = CONV && p.gn_part != nullptr ? p.conv_ho * p.conv_wo : p.M;
   const int seg_tiles = (seg_rows + C::BM - 1) / C::BM;
   p.m_tiles = p.M / seg_rows * seg_tiles;
   p.n_tiles = p.N / C::BN;
   if (p.N % C::BN != 0 || (p.t_nsplit > 0 && p.t_nsplit % C::BN != 0)) return KH_ERR_UNSUPPORTED;
   if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
-  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
+  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, COOP>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
   // the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
   double best = 0;
   p.xg_n = 0;
@@ -523,7 +628,7 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
     if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
   }
   const unsigned grid = 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
+  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, COOP>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
             seg_rows, seg_tiles);
   KH_RETURN_LAST_ERROR();
 }
@@ -532,7 +637,7 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
 
 // What the kernel takes, whatever the tile: whole 64-column stages, T given where there are rank columns, operands that one buffer
 // descriptor spans.
-static bool fine_ok(const LoraGemmParams& p) {
+bool lora_gemm_fine_ok(const LoraGemmParams& p) {
   const size_t lim = (size_t)1 << 31;
   if (p.grp != nullptr || p.sg_mode != 0 || p.xa_k != nullptr || p.K % 64 != 0 || (p.R > 0 && p.t_ext == nullptr)) return false;
   if (p.ldt % 8 != 0 || (size_t)p.N * p.K * 2 >= lim || (size_t)p.N * p.R * 2 >= lim || (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 >= lim) return false;
@@ -542,7 +647,13 @@ static bool fine_ok(const LoraGemmParams& p) {
 }
 
 // Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
-// GEGLU on 64 x 320 (7), 128 x 320 (8).
+// GEGLU on 64 x 320 (7), 128 x 320 (8); order 2 on 128 x 160 (9).
+//
+// Order 2: wave tiles of 64 x 160 over two k-slices and waves of their own for the operands, in place of eight 32 x 160 strips that did
+// both: 7 x 32 W and x rows read from LDS per 20 matrix instructions against 6 per 5.  us per launch, weights from HBM: convolutions 640 -> 640
+// at 2 x 64 x 64 70.9 -> 63.0, 1920 -> 640 190 -> 167, 320 -> 320 at 2 x 128 x 128 81 -> 70, 960 -> 320 198 -> 173, 640 -> 640 263 -> 235 (two
+// rounds), 1280 -> 1280 at 2 x 64 x 64 252 -> 250; linear layers 3952 / 640 / 640 14.1 -> 12.5, 8192 / 640 / 640 14.7 -> 14.0,
+// 4096 / 1280 / 5120 62.6 -> 56.5.
 //
 // Which of them, for a layer whose sums follow `order`: one that fits one round of the 256 CUs (a workgroup fills a CU, so a second round
 // costs as much as the first), the smaller first; -1 where none does and the larger tiles of the other families win.  A
@@ -554,9 +665,8 @@ static bool fine_ok(const LoraGemmParams& p) {
 // 44.9 -> 34.7, 2048 / 5120 / 640 26.1 -> 21.3.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 30.
 // (With adapters, 1024 and more rows at N 1280 do not come here: lora_gemm_pipe_il_ok takes them first.)
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
-  const bool conv = p.conv_cin > 0;
-  if (!fine_ok(p)) return -1;
-  const long hw = conv ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
+  if (!lora_gemm_fine_ok(p)) return -1;
+  const long hw = p.gn_part != nullptr ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
   auto fits = [&](int bm, int bn) {
     return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && nb * ((hw + bm - 1) / bm) * (p.N / bn) <= 256;
   };
@@ -564,16 +674,16 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
     if (order != 0 || p.st_part != nullptr || p.res != nullptr) return -1;
     return fits(64, 320) ? (hw + 63) / 64 * (p.N / 320) > 128 ? 7 : -1 : fits(128, 320) ? 8 : -1;
   }
+  if (order == 2) return 9;
   if (order == 0) return p.st_part != nullptr ? (fits(32, 128) ? 2 : fits(64, 128) ? 3 : -1) : (fits(64, 80) ? 0 : fits(128, 80) ? 1 : -1);
-  if (p.gn_part != nullptr && (p.gn_cg <= 0 || 80 % p.gn_cg != 0 || hw % 64 != 0)) return -1;
-  if (p.gn_part != nullptr ? fits(64, 80) : fits(32, 160)) return p.gn_part != nullptr ? 6 : 4;
-  return fits(64, 160) ? 5 : -1;
+  if (p.gn_part != nullptr) return 80 % p.gn_cg == 0 && fits(64, 80) ? 6 : 5;
+  return fits(32, 160) ? 4 : 5;
 }
 
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
   const bool conv = p.conv_cin > 0;
   // (a forced form comes here without the rule above)
-  if (!fine_ok(p) || (p.geglu ? form < 7 || p.st_part != nullptr || p.res != nullptr : form >= 7)) return KH_ERR_UNSUPPORTED;
+  if (!lora_gemm_fine_ok(p) || (p.geglu ? (form != 7 && form != 8) || p.st_part != nullptr || p.res != nullptr : form == 7 || form == 8)) return KH_ERR_UNSUPPORTED;
   switch (form) {
     case 0: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 80, 0>, false>(p, stream);
     case 1: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<128, 80, 0>, false>(p, stream);
@@ -584,6 +694,38 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 6: return conv ? launch_fine<FCfg<64, 80, 4>, true>(p, stream) : KH_ERR_UNSUPPORTED;
     case 7: return launch_fine<FCfg<64, 320, 0, true>, false>(p, stream);
     case 8: return launch_fine<FCfg<128, 320, 0, true>, false>(p, stream);
+    case 9: return conv ? launch_fine<FCfg<128, 160, 2>, true>(p, stream) : launch_fine<FCfg<128, 160, 2>, false>(p, stream);
     default: return KH_ERR_UNSUPPORTED;
   }
+}
+
+// The cooperative form (see the kernel): the layers whose 128 x 160 tiles fill the chip -- exactly the shapes the rule in
+// lora_gemm_pipe_launch gives these tiles --, T of one or several stacked layers with 128 packed rank columns each of which
+// at most 96 are in use, four column tiles per 128 rank columns of T.
+bool lora_gemm_fine_coop_ok(const LoraGemmParams& p) {
+  if (!(p.t_ext != nullptr && p.a_cat != nullptr && p.col_scale != nullptr && p.il_cnt != nullptr)) return false;
+  if (!lora_gemm_fine_ok(p) || p.conv_cin > 0 || p.geglu || p.t_nsplit % 160 != 0 || p.N % 160 != 0 || p.R != 128 || p.r_used <= 0 || p.r_used > 96 || p.ldt % 128 != 0) return false;
+  const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128), m128 = (p.M + 127) / 128, n160 = p.N / 160;
+  if (!(tiles > 256 && tiles <= 384 && m128 * n160 <= 256)) return false;
+  const bool t_ok = p.t_nsplit == 0 ? p.ldt == p.R : (p.N % p.t_nsplit == 0 && p.ldt == (p.N / p.t_nsplit) * p.R);
+  return t_ok && n160 == 4 * (p.ldt / 128) && n160 <= KH_LN_SLOTS;
+}
+
+// this file's share of kh_lora_split_timeouts (synchronous)
+int lora_gemm_fine_coop_timeouts(int* count, int clear) {
+  int v = 0;
+  hipError_t e = hipMemcpyFromSymbol(&v, HIP_SYMBOL(kh_coop_timeout_count), sizeof(int), 0, hipMemcpyDeviceToHost);
+  if (e != hipSuccess) return (int)e;
+  *count = v;
+  if (clear && v != 0) {
+    const int zero = 0;
+    e = hipMemcpyToSymbol(HIP_SYMBOL(kh_coop_timeout_count), &zero, sizeof(int), 0, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return (int)e;
+  }
+  return KH_OK;
+}
+
+int lora_gemm_fine_launch_coop(const LoraGemmParams& p, hipStream_t stream) {
+  if (!lora_gemm_fine_coop_ok(p)) return KH_ERR_UNSUPPORTED;
+  return launch_fine<FCfg<128, 160, 2>, false, true>(p, stream);
 }

@@ -19,11 +19,6 @@
 // waves below N_HI issue one more than the others, and every wait picks its count by a wave-uniform branch.
 #include "kh_common.h"
 #include "lora_gemm.h"
-#include "lora_shrink_tile.h"
-
-// Bounded waits of the cooperative shrink that have run out on this GPU; read (and cleared) by kh_lora_split_timeouts
-// together with the count of the in-launch shrink of lora_gemm_pipe.hip.
-static __device__ int kh_coop_timeout_count;
 
 namespace {
 
@@ -56,25 +51,8 @@ struct KCfg {
   static_assert(LDS <= 160 * 1024, "LDS budget");
 };
 
-// 16 bytes of zeros (and more): what a 3x3 convolution's DMA reads for taps that fall into the padding
-__device__ __attribute__((aligned(256))) const uint32_t ks_zero_page[64] = {0};
-
-// CONV: x is an NHWC image and row m of the GEMM is output pixel m of a 3x3 convolution with padding 1 (K = 9 * Cin
-// ordered (kh, kw, ci), see lora_gemm_pipe.hip): a stage of 64 K columns is 64 channels of one tap, the x rows of tap
-// (kh, kw) sit (kh * W + kw) * Cin elements after the row's base (the pixel above-left of its window), and rows
-// whose tap falls outside the image read zeros.
-// GNF: the epilogue also leaves the GroupNorm statistics of the result (LoraGemmParams::gn_part).
-// COOP: the launch computes its own shrink, cooperatively.  These tiles fill every CU, so there is no idle CU for shrink
-// workgroups beside the GEMM ones; instead EVERY workgroup first computes one piece of T -- 32 rows x 96 rank columns: the
-// n_tiles = 4 x (ldt / 128) workgroups of a row block of 128 rows share that block's 4 row quarters x ldt / 128 column
-// groups of T, workgroup n_blk takes quarter n_blk % 4 of group n_blk / 4 --, stores it write-through, zeroes the 32
-// padding columns of its group, counts itself into the row block's counter and then runs its GEMM tile; before its first
-// request for T (the last K tiles) it waits, bounded, for the row block's count and reads T past the L2.  A workgroup
-// never waits before its own piece is out, so the launch makes progress in whatever order its workgroups become
-// resident, as long as no OTHER launch whose workgroups wait for each other shares the device with it (the binding does
-// not use this form on a second stream).
-template <class C, bool CONV, bool GNF = false, bool COOP = false>
-__global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(const LoraGemmParams p) {
+template <class C>
+__global__ __launch_bounds__(512, 2) void lora_gemm_ksplit_kernel(const LoraGemmParams p) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int BM = C::BM, BN = C::BN, TN = C::TN, KSW = C::KSW, NST = C::NST, STAGE = C::STAGE;
@@ -84,8 +62,8 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
   const int wm = wave / C::WK, wk = wave % C::WK;
   const int l32 = lane & 31, lh = lane >> 5;
 
-  // the next launch's weights (a cooperative launch issues this after its shrink piece, whose rings use the same LDS)
-  if (!COOP) kh_prefetch_lines(p.pf, p.pf_lines, smem + wave * 1024, blockIdx.x, gridDim.x, tid, 512);
+  // the next launch's weights
+  kh_prefetch_lines(p.pf, p.pf_lines, smem + wave * 1024, blockIdx.x, gridDim.x, tid, 512);
   // tile of this workgroup: XCD b % 8 owns a block of xr_m x xr_n tiles (its W rows stay in its L2)
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   const int m_blk = (xcd / p.xg_n) * p.xr_m + local / p.xr_n;
@@ -96,29 +74,6 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
   const int KT1 = K / 64;
   const int KT = KT1 + (p.t_ext != nullptr ? p.R / 64 : 0);
   const bool has_hi = wave < N_HI;
-  if constexpr (COOP) {
-    // this workgroup's piece of T = bf16((x . A_cat^T) * col_scale) (with a folded LayerNorm in front: the form documented at
-    // ShrinkParams), then the padding columns, then the arrival
-    const int q4 = n_blk & 3, grp = n_blk >> 2;
-    ShrinkParams sp;
-    sp.x = p.x; sp.a_cat = p.a_cat; sp.col_scale = p.col_scale; sp.t = const_cast<bf16_t*>(p.t_ext);
-    sp.M = M; sp.K = K; sp.R = p.ldt;
-    sp.ln_part = p.ln_part; sp.ln_ca1 = p.ln_ca1; sp.ln_ca2 = p.ln_ca2; sp.ln_eps = p.ln_eps;
-    // (a quarter that starts past the last row has nothing to compute: the tile's addressing assumes m0 < M)
-    if (m0 + 32 * q4 < M) lora_shrink_tile<SCfg<4, 1, 3>, true, 512>(sp, m0 + 32 * q4, grp * 128, smem);
-    if (tid < 128) {   // columns 96 .. 127 of the group: 32 rows x 4 pieces of 16 bytes
-      const int row = m0 + 32 * q4 + (tid >> 2);
-      if (row < M) {
-        uint32_t* dst = reinterpret_cast<uint32_t*>(const_cast<bf16_t*>(p.t_ext) + (size_t)row * p.ldt + grp * 128 + 96 + (tid & 3) * 8);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) __hip_atomic_store(dst + e, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0);                          // this thread's write-through stores have completed
-    __syncthreads();
-    if (tid == 0) __hip_atomic_fetch_add(p.il_cnt + m_blk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    kh_prefetch_lines(p.pf, p.pf_lines, smem + wave * 1024, blockIdx.x, gridDim.x, tid, 512);
-  }
   // folded LayerNorm: mean and 1/std of this tile's x rows, read in the epilogue (the barriers of the K loop lie between)
   // and the two per-column terms of this column tile; requested here, finished once the bias loads are under way
   float* sMu = reinterpret_cast<float*>(smem + p.ln_lds);
@@ -140,11 +95,8 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
   // row lane/8, physical piece lane%8, which holds logical piece (lane%8) ^ ((row/2)%8).  The loads are buffer loads:
   // a byte offset per lane that never changes (voff: row and piece) plus a scalar byte offset per K tile, so that the
   // loop carries no vector address arithmetic (with per-lane 64-bit pointers the adds and selects of every stage sat in
-  // the same issue stream as the MFMAs and the loop ran at the sum of both).  An offset at or beyond the buffer's size
-  // reads zeros without touching memory: that is what a 3x3 convolution's taps in the padding do.
-  constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
+  // the same issue stream as the MFMAs and the loop ran at the sum of both).  Every buffer here is shorter than 2 GiB.
   uint32_t voff[LPS_HI], voff2[LPS_HI];
-  int tapmask[LPS_HI];                                 // CONV, x units: bit t = tap t of this lane's row is inside the image
   constexpr int XQ = BM / 64;                          // units q < XQ are x rows for every wave, the others W rows
 #pragma unroll
   for (int q = 0; q < LPS_HI; ++q) {
@@ -152,20 +104,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
     u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
     const int r = u * 8 + (lane >> 3);
     const uint32_t pcb = (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
-    tapmask[q] = 0;
-    if (CONV && r < BM) {
-      int row = m0 + r; row = row < M ? row : M - 1;
-      const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
-      const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
-#pragma unroll
-      for (int tap = 0; tap < 9; ++tap) {
-        const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
-        tapmask[q] |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
-      }
-      // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
-      voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
-      voff2[q] = voff[q];
-    } else if (r < BM) {
+    if (r < BM) {
       int row = m0 + r; row = row < M ? row : M - 1;
       voff[q] = (uint32_t)row * (uint32_t)K * 2u + pcb;
       voff2[q] = ((uint32_t)row * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb;
@@ -175,64 +114,28 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
       voff2[q] = (uint32_t)row * (uint32_t)p.R * 2u + pcb;
     }
   }
-  const size_t x_bytes = CONV ? (size_t)(M / (p.conv_ho * p.conv_wo)) * p.conv_h * p.conv_w * p.conv_cin * 2 : (size_t)M * K * 2;
-  const size_t x_lead = CONV ? (size_t)(p.conv_w + 1) * p.conv_cin * 2 : 0;
-  const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.x) - x_lead), 0,
-                                                         (int)(x_bytes + x_lead), 0x00020000);
+  const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.x), 0, (int)((size_t)M * K * 2), 0x00020000);
   const rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w), 0, (int)((size_t)N * K * 2), 0x00020000);
   const rsrc_t rs_t = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.t_ext != nullptr ? p.t_ext : p.x), 0,
                                                          p.t_ext != nullptr ? (int)((size_t)M * p.ldt * 2) : 0, 0x00020000);
   const rsrc_t rs_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.t_ext != nullptr ? p.b_cat : p.w), 0,
                                                          p.t_ext != nullptr ? (int)((size_t)N * p.R * 2) : 0, 0x00020000);
-  // CONV: K tiles are requested in order, so the tap and the channel offset of the next request are running scalars, and
-  // the x offsets with the current tap's padding applied change only when the tap does
-  int cv_tap = 0, cv_kw = 0, cv_c0 = 0, cv_shift = 0, cv_row = 0;
-  uint32_t xvo[XQ];
-#pragma unroll
-  for (int q = 0; q < XQ; ++q) xvo[q] = (tapmask[q] & 1) ? voff[q] : OOB;
   auto issue = [&](int t, auto stc) {                  // K tile t into ring stage stc
     char* stage = smem + decltype(stc)::value * STAGE;
-    if (CONV || t < KT1) {
+    if (t < KT1) {
       const int so = t * 128;
 #pragma unroll
       for (int q = 0; q < LPS_HI; ++q) {
         if (q < LPS_LO || has_hi) {
-          if (CONV && q < XQ)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, xvo[q], (cv_shift + cv_c0) * 2, 0, 0);
-          else
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_x : rs_w, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, voff[q], so, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_x : rs_w, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, voff[q], so, 0, 0);
         }
       }
     } else {
-      if (COOP && t == KT1) {
-        // first request for T: wait (bounded) until every workgroup of this row block has delivered its piece
-        if (lane == 0) {
-          int it = 0;
-          while (__hip_atomic_load(p.il_cnt + m_blk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p.n_tiles && ++it < (1 << 20))
-            __builtin_amdgcn_s_sleep(8);
-          if (it >= (1 << 20)) {
-            __hip_atomic_store(p.il_cnt + (p.M + 127) / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&kh_coop_timeout_count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-      }
       const int so = (t - KT1) * 128;
 #pragma unroll
       for (int q = 0; q < LPS_HI; ++q)
-        if (q < LPS_LO || has_hi) {
-          // (COOP) T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
-          if (COOP && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, voff2[q], so, 0, 17 /* sc0 sc1 */);
-          else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_b, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, voff2[q], so, 0, 0);
-        }
-    }
-    if (CONV) {
-      cv_c0 += 64;
-      if (cv_c0 == p.conv_cin) {
-        cv_c0 = 0; ++cv_tap; ++cv_kw; cv_shift += p.conv_cin;
-        if (cv_kw == 3) { cv_kw = 0; cv_row += p.conv_w * p.conv_cin; cv_shift = cv_row; }
-#pragma unroll
-        for (int q = 0; q < XQ; ++q) xvo[q] = ((tapmask[q] >> cv_tap) & 1) ? voff[q] : OOB;
-      }
+        if (q < LPS_LO || has_hi)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_b, (lptr_t)(stage + (wave + 8 * q) * 1024), 16, voff2[q], so, 0, 0);
     }
   };
   // wait until at most n of this wave's younger K tiles are outstanding (and its LDS reads are done)
@@ -408,71 +311,6 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
     }
   }
   __syncthreads();
-  if constexpr (GNF) {
-    // GroupNorm statistics as a by-product: the staged tile is BM pixels of one image times BN / gn_cg whole groups; their
-    // (sum, sum of squares) over the bf16-rounded values (residual included) plus the per-(image, channel) term -- what a GroupNorm
-    // kernel reading the stored result would take -- go to gn_part[image][group][row tile of the image].  Three short passes,
-    // sums in fixed orders (deterministic); the tile itself is stored below as usual.
-    constexpr int PCS = BN / 8, RP = 512 / PCS;               // 16-byte pieces per row, row parts (25 of 20 threads)
-    float* colp = reinterpret_cast<float*>(smem);             // [RP][BN][2]: the partial strips are dead
-    float* cols = colp + RP * BN * 2;                         // [BN][2] column sums
-    static_assert((RP * BN * 2 + BN * 2) * 4 <= C::PART, "column sums fit the dead partial strips");
-    const int cg = p.gn_cg, ng = BN / cg, G = N / cg;
-    const int n_img = m0 / p.gn_hw, split = (m0 % p.gn_hw) / BM, splits = p.gn_hw / BM;
-    if (p.res != nullptr) {
-      // the statistics are those of the stored result: the residual goes into the staged tile first (the same rounded adds
-      // the store loop would make), and the store loop below then writes the tile as it is
-#pragma unroll
-      for (int q = 0; q < C::OPT; ++q) {
-        const int c = tid + q * 512, srow = c / (BN / 8), ch = c % (BN / 8);
-        if (c < C::OPC) {
-          u32x4 o = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + ch * 8);
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            o[e] = pack_bf16x2(bf16_lo(o[e]) + bf16_lo(rr[q][e]), bf16_hi(o[e]) + bf16_hi(rr[q][e]));
-          *reinterpret_cast<u32x4*>(sC + srow * C::LDC + ch * 8) = o;
-        }
-      }
-      __syncthreads();
-    }
-    // the per-(image, channel) term enters through sum(a + t) = sum(a) + n t and sum((a + t)^2) = sum(a^2) + 2 t sum(a) + n t^2:
-    // requested now, used after the first pass
-    const float ad = (tid < BN && p.gn_add != nullptr) ? (float)p.gn_add[(size_t)n_img * N + n0 + tid] : 0.f;
-    if (tid < RP * PCS) {
-      const int ch = tid % PCS, part = tid / PCS;
-      float cs[8], cq[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) cs[e] = cq[e] = 0.f;
-#pragma unroll
-      for (int i = 0; i < (BM + RP - 1) / RP; ++i) {
-        const int r = part + i * RP;
-        if (r < BM) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(sC + r * C::LDC + ch * 8);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float a = bf16_lo(v[e]), b2 = bf16_hi(v[e]);
-            cs[2 * e] += a; cq[2 * e] = fmaf(a, a, cq[2 * e]);
-            cs[2 * e + 1] += b2; cq[2 * e + 1] = fmaf(b2, b2, cq[2 * e + 1]);
-          }
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) *reinterpret_cast<f32x2*>(colp + ((part * BN) + ch * 8 + e) * 2) = f32x2{cs[e], cq[e]};
-    }
-    __syncthreads();
-    if (tid < BN) {
-      float s = 0.f, q = 0.f;
-#pragma unroll
-      for (int part = 0; part < RP; ++part) { const f32x2 v = *reinterpret_cast<const f32x2*>(colp + (part * BN + tid) * 2); s += v[0]; q += v[1]; }
-      *reinterpret_cast<f32x2*>(cols + tid * 2) = f32x2{s + (float)BM * ad, q + 2.f * ad * s + (float)BM * ad * ad};
-    }
-    __syncthreads();
-    if (tid < ng) {
-      float s = 0.f, q = 0.f;
-      for (int c = tid * cg; c < (tid + 1) * cg; ++c) { s += cols[2 * c]; q += cols[2 * c + 1]; }
-      *reinterpret_cast<f32x2*>(p.gn_part + (((size_t)n_img * G + n0 / cg + tid) * splits + split) * 2) = f32x2{s, q};
-    }
-  }
   const KhOut yout(p.y, (size_t)M * N * 2);
   if (p.st_part != nullptr) {
     // as below, and every row's (sum, sum of squares) over this tile's columns for a following folded LayerNorm: the 20
@@ -510,7 +348,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
     const int grow = m0 + srow, gcol = n0 + ch * 8;
     if (c < C::OPC && grow < M && gcol < N) {
       u32x4 o = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + ch * 8);
-      if (!GNF && p.res != nullptr) {   // (GNF: already added into the staged tile)
+      if (p.res != nullptr) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           o[e] = pack_bf16x2(bf16_lo(o[e]) + bf16_lo(rr[q][e]), bf16_hi(o[e]) + bf16_hi(rr[q][e]));
@@ -521,14 +359,12 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_ksplit_kernel(con
 #endif
 }
 
-template <class C, bool CONV = false, bool GNF = false, bool COOP = false>
+template <class C>
 int launch_ksplit(LoraGemmParams p, hipStream_t stream) {
   p.m_tiles = (p.M + C::BM - 1) / C::BM;
   p.n_tiles = (p.N + C::BN - 1) / C::BN;
   static_assert(C::LDS + KH_LN_LDS <= 160 * 1024, "LDS budget with the row statistics");
-  static_assert(!COOP || (SCfg<4, 1, 3>::LDS <= C::LDS && C::BM == 128), "the shrink piece's rings fit the GEMM ring; four quarters per row block");
-  if (hipError_t e = kh_allow_lds<lora_gemm_ksplit_kernel<C, CONV, GNF, COOP>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
-  if ((p.ln_part != nullptr || p.st_part != nullptr) && CONV) return KH_ERR_UNSUPPORTED;
+  if (hipError_t e = kh_allow_lds<lora_gemm_ksplit_kernel<C>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
   if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
   p.ln_lds = C::LDS;
   const size_t lds = (size_t)C::LDS + (p.ln_part != nullptr ? KH_LN_LDS : 0);
@@ -542,13 +378,7 @@ int launch_ksplit(LoraGemmParams p, hipStream_t stream) {
     if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
   }
   const unsigned grid = 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  if constexpr (GNF) {
-    // whole groups per tile, whole tiles per image
-    if (p.st_part != nullptr || p.gn_cg <= 0 || C::BN % p.gn_cg != 0 || p.N % C::BN != 0 || p.gn_hw % C::BM != 0 ||
-        p.M % p.gn_hw != 0)
-      return KH_ERR_UNSUPPORTED;
-  }
-  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_ksplit_kernel<C, CONV, GNF, COOP>, dim3(grid), dim3(512), lds, stream, p);
+  kh_launch(KH_TAG_LORA_GEMM, lora_gemm_ksplit_kernel<C>, dim3(grid), dim3(512), lds, stream, p);
   KH_RETURN_LAST_ERROR();
 }
 
@@ -557,62 +387,17 @@ int launch_ksplit(LoraGemmParams p, hipStream_t stream) {
 // every operand is addressed as a buffer with 32-bit byte offsets: shorter than 2 GiB each
 static bool ks_fits_buffers(const LoraGemmParams& p) {
   const size_t lim = (size_t)1 << 31;
-  const size_t xb = p.conv_cin > 0 ? ((size_t)(p.M / (p.conv_ho * p.conv_wo)) * p.conv_h + 1) * p.conv_w * p.conv_cin * 2 + 2 * (size_t)p.conv_cin
-                                   : (size_t)p.M * p.K * 2;
-  return xb < lim && (size_t)p.N * p.K * 2 < lim && (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 < lim && (size_t)p.N * (p.R > 0 ? p.R : 1) * 2 < lim;
+  return (size_t)p.M * p.K * 2 < lim && (size_t)p.N * p.K * 2 < lim && (size_t)p.M * (p.ldt > 0 ? p.ldt : 1) * 2 < lim && (size_t)p.N * (p.R > 0 ? p.R : 1) * 2 < lim;
 }
 
-bool lora_gemm_ksplit_ok(const LoraGemmParams& p) {
+static bool lora_gemm_ksplit_ok(const LoraGemmParams& p) {
   const bool plain = p.R == 0 || p.t_ext != nullptr;
   return plain && ks_fits_buffers(p) && p.grp == nullptr && p.sg_mode == 0 && p.conv_cin == 0 && !p.geglu && p.K % 64 == 0 && p.K >= 64 &&
          (p.t_ext == nullptr || (p.R % 64 == 0 && p.ldt % 8 == 0)) && (p.t_nsplit == 0 || p.t_nsplit % 160 == 0) &&
          p.N % 8 == 0;
 }
 
-// The cooperative form (see the kernel): the layers whose 128 x 160 tiles fill the chip -- exactly the shapes the rule in
-// lora_gemm_pipe_launch gives these tiles --, T of one or several stacked layers with 128 packed rank columns each of which
-// at most 96 are in use, four column tiles per 128 rank columns of T.
-bool lora_gemm_ksplit_coop_ok(const LoraGemmParams& p) {
-  if (!(p.t_ext != nullptr && p.a_cat != nullptr && p.col_scale != nullptr && p.il_cnt != nullptr)) return false;
-  if (!lora_gemm_ksplit_ok(p) || p.N % 160 != 0 || p.R != 128 || p.r_used <= 0 || p.r_used > 96 || p.ldt % 128 != 0) return false;
-  const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128), m128 = (p.M + 127) / 128, n160 = p.N / 160;
-  if (!(tiles > 256 && tiles <= 384 && m128 * n160 <= 256)) return false;
-  const bool t_ok = p.t_nsplit == 0 ? p.ldt == p.R : (p.N % p.t_nsplit == 0 && p.ldt == (p.N / p.t_nsplit) * p.R);
-  return t_ok && n160 == 4 * (p.ldt / 128) && n160 <= KH_LN_SLOTS;
-}
-
-// this file's share of kh_lora_split_timeouts (synchronous)
-int lora_gemm_ksplit_coop_timeouts(int* count, int clear) {
-  int v = 0;
-  hipError_t e = hipMemcpyFromSymbol(&v, HIP_SYMBOL(kh_coop_timeout_count), sizeof(int), 0, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return (int)e;
-  *count = v;
-  if (clear && v != 0) {
-    const int zero = 0;
-    e = hipMemcpyToSymbol(HIP_SYMBOL(kh_coop_timeout_count), &zero, sizeof(int), 0, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return (int)e;
-  }
-  return KH_OK;
-}
-
-int lora_gemm_ksplit_launch_coop(const LoraGemmParams& p, hipStream_t stream) {
-  if (!lora_gemm_ksplit_coop_ok(p)) return KH_ERR_UNSUPPORTED;
-  return launch_ksplit<KCfg<4>, false, false, true>(p, stream);
-}
-
 int lora_gemm_ksplit_launch(const LoraGemmParams& p, int row_groups, hipStream_t stream) {
   if (!lora_gemm_ksplit_ok(p)) return KH_ERR_UNSUPPORTED;
   return row_groups == 4 ? launch_ksplit<KCfg<4>>(p, stream) : launch_ksplit<KCfg<2>>(p, stream);
-}
-
-// 3x3 convolution on the same tiles (conv_* fields set, R == 0, K == 9 * conv_cin, conv_cin % 64 == 0).
-bool lora_gemm_ksplit_conv_ok(const LoraGemmParams& p) {
-  return p.conv_cin > 0 && p.conv_cin % 64 == 0 && p.K == 9 * p.conv_cin && ks_fits_buffers(p) && p.R == 0 && p.t_ext == nullptr && p.grp == nullptr &&
-         p.sg_mode == 0 && !p.geglu && p.N % 8 == 0;
-}
-
-int lora_gemm_ksplit_launch_conv(const LoraGemmParams& p, int row_groups, hipStream_t stream) {
-  if (!lora_gemm_ksplit_conv_ok(p)) return KH_ERR_UNSUPPORTED;
-  if (p.gn_part != nullptr) return row_groups == 4 ? launch_ksplit<KCfg<4>, true, true>(p, stream) : launch_ksplit<KCfg<2>, true, true>(p, stream);
-  return row_groups == 4 ? launch_ksplit<KCfg<4>, true>(p, stream) : launch_ksplit<KCfg<2>, true>(p, stream);
 }

@@ -1236,8 +1236,8 @@ KH_EXPORT int kh_lora_split_timeouts(int32_t* count, int clear) {
     e = hipMemcpyToSymbol(HIP_SYMBOL(kh_split_timeout_count), &zero, sizeof(int), 0, hipMemcpyHostToDevice);
     if (e != hipSuccess) return (int)e;
   }
-  int v2 = 0;   // the cooperative form's waits (lora_gemm_ksplit.hip)
-  if (const int rc = lora_gemm_ksplit_coop_timeouts(&v2, clear); rc != KH_OK) return rc;
+  int v2 = 0;   // the cooperative form's waits (lora_gemm_fine.hip)
+  if (const int rc = lora_gemm_fine_coop_timeouts(&v2, clear); rc != KH_OK) return rc;
   *count = v + v2;
   return KH_OK;
 }
@@ -1323,7 +1323,7 @@ int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, hipStream_t stream) {
 // The 160-column tiles the rules below give this convolution, when the GroupNorm statistics of its result can be a
 // by-product of its epilogue: whole tiles per image, whole groups per tile.
 int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p) {
-  if (p.N % 160 != 0 || !lora_gemm_ksplit_conv_ok(p) || p.gn_cg <= 0 || 160 % p.gn_cg != 0 || p.gn_hw <= 0 || p.M % p.gn_hw != 0)
+  if (p.N % 160 != 0 || !lora_gemm_fine_ok(p) || p.gn_cg <= 0 || 160 % p.gn_cg != 0 || p.gn_hw <= 0 || p.M % p.gn_hw != 0)
     return 0;
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
   const long n160 = p.N / 160, m128 = (p.M + 127) / 128, m64 = (p.M + 63) / 64;
@@ -1336,20 +1336,16 @@ int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p) {
 int lora_gemm_pipe_launch_conv(const LoraGemmParams& p, hipStream_t stream) {
   if (p.gn_part != nullptr) {   // the caller has asked lora_gemm_conv_gn_row_groups
     const int rg = lora_gemm_conv_gn_row_groups(p);
-    if (const int form = rg == 2 ? lora_gemm_fine_form(p, 4) : -1; form >= 0) return lora_gemm_fine_launch(p, form, stream);
-    return rg == 0 ? KH_ERR_UNSUPPORTED : lora_gemm_ksplit_launch_conv(p, rg, stream);
+    return rg == 0 ? KH_ERR_UNSUPPORTED : lora_gemm_fine_launch(p, lora_gemm_fine_form(p, rg == 4 ? 2 : 4), stream);
   }
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-  // 160-column tiles (lora_gemm_ksplit.hip) by the rules of the linear layers
-  if (p.N % 160 == 0 && lora_gemm_ksplit_conv_ok(p)) {
+  // 160-column tiles (lora_gemm_fine.hip) by the rules of the linear layers
+  if (p.N % 160 == 0 && lora_gemm_fine_ok(p)) {
     const long n160 = p.N / 160, m128 = (p.M + 127) / 128, m64 = (p.M + 63) / 64;
     // (whole rounds of 128x160 tiles also where 128-column tiles would divide N: the upsamplers' 1280 -> 1280 at 64x64 took
     // 342 us on the 128x128 tiles and takes 249 us on these, 640 -> 640 at 128x128 290 -> 264 us)
-    if ((tiles > 256 && tiles <= 384 && m128 * n160 <= 256) || (m128 * n160) % 256 == 0) return lora_gemm_ksplit_launch_conv(p, 4, stream);
-    if (tiles <= 192 && m64 * n160 <= 256 && m64 * n160 > tiles && p.K >= 2560) {
-      const int form = lora_gemm_fine_form(p, 4);   // (-1: images whose partial tiles make it more than one round)
-      return form >= 0 ? lora_gemm_fine_launch(p, form, stream) : lora_gemm_ksplit_launch_conv(p, 2, stream);
-    }
+    if ((tiles > 256 && tiles <= 384 && m128 * n160 <= 256) || (m128 * n160) % 256 == 0) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 2), stream);
+    if (tiles <= 192 && m64 * n160 <= 256 && m64 * n160 > tiles && p.K >= 2560) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 4), stream);
   }
   if (tiles <= 256 && p.conv_cin % 64 == 0) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>, true>(p, stream);
   return launch_pcfg<PCfg<128, 128, 2, 2, 0, 4>, true>(p, stream);
@@ -1379,7 +1375,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     case 40: return lora_gemm_ksplit_launch(p, 2, stream);
     case 41: return lora_gemm_ksplit_launch(p, 4, stream);
     case 42: return lora_gemm_wide_launch(p, stream);
-    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
+    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: case 59: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
     default: break;
   }
   // Default choice.  The limiter is the vector L1 path (every operand byte enters LDS through it), so
@@ -1396,15 +1392,13 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
   if (plain_ok(p)) {
     const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
     // N a multiple of 160 and a tile count that leaves 128x128 tiles with a ragged last round: 160-column tiles
-    // (8 waves splitting K) give every CU exactly one.  64-row tiles pay for their extra operand traffic only
+    // give every CU exactly one.  64-row tiles pay for their extra operand traffic only
     // on long K.
-    if (p.N % 160 == 0 && lora_gemm_ksplit_ok(p)) {
+    if (!p.geglu && p.N % 160 == 0 && p.t_nsplit % 160 == 0 && lora_gemm_fine_ok(p)) {
       const long n160 = p.N / 160;
-      if (tiles > 256 && tiles <= 384 && (long)((p.M + 127) / 128) * n160 <= 256) return lora_gemm_ksplit_launch(p, 4, stream);
-      if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560) {
-        const int form = lora_gemm_fine_form(p, 4);
-        return form >= 0 ? lora_gemm_fine_launch(p, form, stream) : lora_gemm_ksplit_launch(p, 2, stream);
-      }
+      if (tiles > 256 && tiles <= 384 && (long)((p.M + 127) / 128) * n160 <= 256) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 2), stream);
+      if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560)
+        return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 4), stream);
     }
     // few enough rows for one round of small tiles
     if (const int form = lora_gemm_fine_form(p, 0); form >= 0) return lora_gemm_fine_launch(p, form, stream);

@@ -287,6 +287,26 @@ def test_fine_tiles_give_the_bits_of_the_large_ones(M, N, K, R, r_used):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used", [(1, 160, 64, 0, 0), (129, 320, 128, 64, 48), (127, 640, 640, 128, 96), (4000, 640, 576, 0, 0), (8192, 640, 2560, 128, 80)])
+def test_fine_128x160_tiles(M, N, K, R, r_used):
+    """Code 59 (128 x 160, two k-slices) against the kernel whose order of sums it keeps (41), bit for bit: partial row blocks, K shorter
+    than the ring, rank columns that fill no stage."""
+    from katz_amd import ops
+
+    say("fine 128 x 160", M, N, K, R, r_used)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N)
+    t, bc = (rnd(M, R), rnd(N, R) * 0.05) if R else (None, None)
+    if r_used:
+        t[:, r_used:] = 0
+        bc[:, r_used:] = 0
+    for rs in (None, res):
+        run = (lambda c: ops.lora_linear_pre(x, w, b, t, bc, residual=rs, tile=c, r_used=r_used)) if R else (lambda c: ops.lora_linear(x, w, b, residual=rs, tile=c))
+        assert torch.equal(run(59), run(41)), rs is not None
+
+
 @pytest.mark.parametrize("rows,N,K,stats,fold", [(33, 1280, 640, True, True), (512, 1280, 1280, True, False), (700, 640, 640, True, True), (988, 1280, 1280, False, True),
                                                  (1100, 1280, 1280, True, True), (200, 1280, 5120, True, False), (1200, 1280, 5120, True, True)])
 def test_fine_tiles_with_folded_norms_do_not_depend_on_the_rows(rows, N, K, stats, fold):
