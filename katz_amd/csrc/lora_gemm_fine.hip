@@ -61,6 +61,10 @@ struct FCfg {
   // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
   static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
   static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 4 ? 1 : 2;   // a wave's MFMA tiles, its k-steps per stage
+  // operand order of the matrix instructions: (W, x) leaves four columns of a row in a lane, so that the epilogue writes 8 bytes at a time
+  // (128 x 320: 5.6 K clocks against 8.4 K), (x, W) four rows of a column.  One x fragment per W fragment is the exception: the K loop of 64 x 80
+  // takes 8.8 K clocks with (x, W) and 9.9 K with (W, x), more than the epilogue saves.
+  static constexpr bool XW = BM == 64 && BN == 80 && ORD == 0;
   static constexpr bool DB = TM * TN * G * 4 <= 96 && !GLU;      // two fragment buffers where the registers allow it
   static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
   static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
@@ -140,17 +144,6 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
     __builtin_amdgcn_s_waitcnt(0);                          // this thread's write-through stores have completed
     __syncthreads();
     if (tid == 0) __hip_atomic_fetch_add(p.il_cnt + m_blk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-
-  // per-row and per-column terms: requested now, used after the K loop (older than every DMA load, so no wait falls in between)
-  KhLnTileStats<BM, 512> ln_stats;
-  float c1v = 0.f, c2v = 0.f;
-  uint16_t biasv = 0;
-  if (p.ln_part != nullptr) {
-    ln_stats.load(p.ln_part, m0, M, tid);
-    if (tid < BN) { c1v = p.ln_c1[n0 + tid]; c2v = p.ln_c2[n0 + tid]; }
-  } else if (p.bias != nullptr && tid < BN) {
-    biasv = reinterpret_cast<const uint16_t*>(p.bias)[n0 + tid];
   }
 
   // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
@@ -291,23 +284,45 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 4 * C::G; ++e) acc[i][j][e] = 0.f;
+  auto mfma = [&](const Frag& x, const Frag& w, Acc& c) {
+    const Frag& u = C::XW ? x : w;
+    const Frag& v = C::XW ? w : x;
+    if constexpr (HALF) c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(u, v, c, 0, 0, 0);
+    else if constexpr (C::MF == 32) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u, v, c, 0, 0, 0);
+    else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u, v, c, 0, 0, 0);
+  };
   auto mma = [&](const Fr& f) {
 #pragma unroll
     for (int k = 0; k < KS; ++k)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          if constexpr (HALF) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
-          else if constexpr (C::MF == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
-          else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[k][i], f.b[k][j], acc[i][j], 0, 0, 0);
-        }
+        for (int i = 0; i < TM; ++i) mfma(f.a[k][i], f.b[k][j], acc[i][j]);
   };
 
   // K loop.  Step t: tile t is in the computing waves' registers (cur); tile t+1 becomes visible at the barrier, after which
   // every wave has read tile t out of its stage, so that stage takes tile t + NST.  Both kinds of waves pass KT barriers.
+  // (the epilogue's per-row and per-column terms are the producers' to fetch: ten registers less in the computing waves)
+  float* sMu = reinterpret_cast<float*>(smem + C::LDS);      // [128] mean, [128] 1/std, [BN] x 2
+  float* sRs = sMu + 128;
+  float* sc1 = sRs + 128;
+  float* sc2 = sc1 + BN;
+  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && BM <= 128, "per-row and per-column terms");
   if (producer) {
-    kh_prefetch_lines(p.pf, p.pf_lines, smem + pw * 1024, blockIdx.x, gridDim.x, tid - 256, 256);
+    // requested now, used after the K loop (older than every DMA load, so no wait falls in between)
+    constexpr int CP = (BN + 255) / 256;
+    const int ptid = tid - 256;
+    KhLnTileStats<BM, 256> ln_stats;
+    float c1v[CP], c2v[CP];
+    uint16_t biasv[CP];
+    if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, M, ptid);
+#pragma unroll
+    for (int c = 0; c < CP; ++c) {
+      const int col = n0 + (ptid + 256 * c < BN ? ptid + 256 * c : 0);
+      c1v[c] = p.ln_part != nullptr ? p.ln_c1[col] : 0.f;
+      c2v[c] = p.ln_part != nullptr ? p.ln_c2[col] : 0.f;
+      biasv[c] = p.ln_part == nullptr && p.bias != nullptr ? reinterpret_cast<const uint16_t*>(p.bias)[col] : (uint16_t)0;
+    }
 #pragma unroll
     for (int t = 0; t < PD; ++t)
       if (t < KT) issue(t, t * STAGE);
@@ -325,6 +340,10 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       wait_younger(KT - 2 - t);
       ring_barrier();
     }
+    if (p.ln_part != nullptr) ln_stats.finish(K, p.ln_eps, ptid, sMu, sRs, false);
+#pragma unroll
+    for (int c = 0; c < CP; ++c)
+      if (const int col = ptid + 256 * c; col < BN) { sc1[col] = c1v[c]; sc2[col] = p.ln_part != nullptr ? c2v[c] : bf16_bits_to_f32(biasv[c]); }
   } else {
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
@@ -332,7 +351,11 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       if (t < KT1)
         kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
     };
-    touch(0, 24);
+    // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
+    // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
+    constexpr int TOUCH = C::GLU ? 8 : 24;
+    touch(0, TOUCH);
+    kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, blockIdx.x, gridDim.x, tid, 256);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
     if constexpr (C::GLU) {
 #pragma unroll 4
@@ -356,10 +379,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       auto read_b = [&](int st, int k, int j) { b[j] = *reinterpret_cast<const Frag*>(smem + st + fb[k] + j * C::MF * ROWB); };
       auto mma1 = [&](int set, int j) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          if constexpr (C::MF == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[set][i], b[j], acc[i][j], 0, 0, 0);
-          else acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[set][i], b[j], acc[i][j], 0, 0, 0);
-        }
+        for (int i = 0; i < TM; ++i) mfma(a[set][i], b[j], acc[i][j]);
       };
       auto kstep = [&](int set, int st_next, int k_next) {   // x in a[set]; the next k-step's fragments: step k_next of stage st_next
         read_a(st_next, k_next, 1 - set);
@@ -380,7 +400,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       for (int j = 0; j < TN; ++j) read_b(0, 0, j);
       if constexpr (KS == 2) {
         for (int t = 0; t + 1 < KT; ++t) {
-          if ((t & 7) == 0) touch(t + 24, 8);
+          if ((t & 7) == 0) touch(t + TOUCH, 8);
           kstep(0, st, 1);
           next_stage();
           kstep(1, st, 0);
@@ -389,7 +409,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       } else {
         int t = 0;
         for (; t + 2 < KT; t += 2) {
-          if ((t & 7) == 0) touch(t + 24, 8);
+          if ((t & 7) == 0) touch(t + TOUCH, 8);
           next_stage();
           kstep(0, st, 0);
           next_stage();
@@ -416,7 +436,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
     };
     int t = 0;
     for (; t + 2 < KT; t += 2) {
-      if ((t & 7) == 0) touch(t + 24, 8);
+      if ((t & 7) == 0) touch(t + TOUCH, 8);
       step(f0, f1);
       step(f1, f0);
     }
@@ -434,33 +454,37 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
       rr[q] = (c < C::OPC && srow < rows) ? *reinterpret_cast<const u32x4*>(p.res + (size_t)(m0 + srow) * N + n0 + ch * 8) : u32x4{0, 0, 0, 0};
     }
   }
-  float* sMu = reinterpret_cast<float*>(smem + C::LDS);      // [128] mean, [128] 1/std, [BN] x 2
-  float* sRs = sMu + 128;
-  float* sc1 = sRs + 128;
-  float* sc2 = sc1 + BN;
-  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && BM <= 128, "per-row and per-column terms");
-  if (p.ln_part != nullptr) ln_stats.finish(K, p.ln_eps, tid, sMu, sRs, false);
-  if (tid < BN) { sc1[tid] = c1v; sc2[tid] = p.ln_part != nullptr ? c2v : bf16_bits_to_f32(biasv); }
   __syncthreads();   // the ring is dead: partial sums and the staging tiles reuse it
 
   // the k-slices meet in LDS: every wave leaves all its tiles and finishes every WK-th of them
   f32x4* part = reinterpret_cast<f32x4*>(smem);
   bf16_t* sC = reinterpret_cast<bf16_t*>(smem + C::PART);
-  auto finish = [&](const f32x4 s, int i, int j, int g) {   // four rows of one column of tile (i, j)
-    const int trow = wm * (BM / C::WM) + i * C::MF + (C::MF == 32 ? 8 * g : 0) + 4 * lg, col = wn * (BN / C::WN) + j * C::MF + lr;
-    f32x4 mu = {0.f, 0.f, 0.f, 0.f}, rs = {1.f, 1.f, 1.f, 1.f};
-    if (p.ln_part != nullptr) { mu = *reinterpret_cast<const f32x4*>(sMu + trow); rs = *reinterpret_cast<const f32x4*>(sRs + trow); }
-    const float c1 = sc1[col], c2 = sc2[col];
+  auto finish = [&](const f32x4 s, int i, int j, int g) {   // the four outputs of group g of tile (i, j) in this lane
+    const int at = (C::MF == 32 ? 8 * g : 0) + 4 * lg;       // first of the four: columns of row lr (XW: rows of column lr) of the tile
+    const int row = wm * (BM / C::WM) + i * C::MF + (C::XW ? at : lr), col = wn * (BN / C::WN) + j * C::MF + (C::XW ? lr : at);
+    if constexpr (C::XW) {
+      f32x4 mu = {0.f, 0.f, 0.f, 0.f}, rs = {1.f, 1.f, 1.f, 1.f};
+      if (p.ln_part != nullptr) { mu = *reinterpret_cast<const f32x4*>(sMu + row); rs = *reinterpret_cast<const f32x4*>(sRs + row); }
+      const float c1 = sc1[col], c2 = sc2[col];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sC[(trow + e) * C::LDC + col] = (bf16_t)(rs[e] * (s[e] - mu[e] * c1) + c2);
+      for (int e = 0; e < 4; ++e) sC[(row + e) * C::LDC + col] = (bf16_t)(rs[e] * (s[e] - mu[e] * c1) + c2);
+    } else {
+      float mu = 0.f, rs = 1.f;
+      if (p.ln_part != nullptr) { mu = sMu[row]; rs = sRs[row]; }
+      const f32x4 c1 = *reinterpret_cast<const f32x4*>(sc1 + col), c2 = *reinterpret_cast<const f32x4*>(sc2 + col);
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (bf16_t)(rs * (s[e] - mu * c1[e]) + c2[e]);
+      *reinterpret_cast<bf16x4*>(sC + row * C::LDC + col) = o;
+    }
   };
   auto group = [&](const Acc& v, int g) { return f32x4{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]}; };
   if constexpr (C::WK == 1) {
     if (!producer) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) finish(group(acc[i][j], 0), i, j, 0);
+        for (int i = 0; i < TM; ++i) finish(group(acc[i][j], 0), i, j, 0);
     }
   } else {
     constexpr int UH = TM / C::NH * TN * C::G;           // groups of a pass
@@ -661,8 +685,8 @@ bool lora_gemm_fine_ok(const LoraGemmParams& p) {
 // weights together exceed the memory-side cache, us per launch (M, N, K: the larger tiles -> these):
 // 512 / 1280 / 1280 18.3 -> 9.8 (with row statistics 19.7 -> 11.1); 988 / 1280 / 1280 18.6 -> 9.8 (19.8 -> 11.9); 2048 / 1280 / 1280
 // 16.4 -> 13.1; 988 / 1280 / 5120 43.7 -> 30.6; 2048 / 1280 / 5120 45.7 -> 39.5; 154 / 1280 / 2048 23.5 -> 12.6; a round too many:
-// 1152 / 1280 / 1280 on 64 x 80 16.3 against 12.0 on 128 x 80.  GEGLU: 512 / 10240 / 1280 29.5 -> 23.6, 988 / 10240 / 1280
-// 44.9 -> 34.7, 2048 / 5120 / 640 26.1 -> 21.3.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 30.
+// 1152 / 1280 / 1280 on 64 x 80 16.3 against 12.0 on 128 x 80.  GEGLU: 512 / 10240 / 1280 29.5 -> 22.1, 988 / 10240 / 1280
+// 44.9 -> 34.9, 2048 / 5120 / 640 26.1 -> 20.9.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 30.
 // (With adapters, 1024 and more rows at N 1280 do not come here: lora_gemm_pipe_il_ok takes them first.)
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   if (!lora_gemm_fine_ok(p)) return -1;
