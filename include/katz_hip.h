@@ -106,7 +106,9 @@ int kh_lora_linear_pre_bf16(const void* x, const void* w, const void* bias, cons
  * of its row block before the last K tiles.  No workgroup waits before its own piece is out, so one such launch always
  * completes; TWO of them running at the same time on different streams can each hold the CUs the other's not yet
  * started workgroups need, and then both only end through the bounded wait.  A caller that enqueues these calls on
- * streams that may overlap sets bit 24 on all but one of the streams. */
+ * streams that may overlap sets bit 24 on all but one of the streams.
+ * Few rows (tiles smaller than 128 x 128): likewise inside the launch where those tiles leave CUs idle, in 16 x 16 or 32 x 32
+ * pieces of t_scratch and with the results of the two launches bit for bit; columns of t_scratch beyond r_used stay unwritten. */
 #define KH_SPLIT_COUNTER_INTS(M) (((M) + 127) / 128 + 1)
 int kh_lora_linear_split_bf16(const void* x, const void* w, const void* bias, const void* a_cat, const float* col_scale,
                               const void* b_cat, void* t_scratch, int32_t* counters, const void* residual, void* y,

@@ -38,6 +38,7 @@ struct LoraGemmParams {
   // row block's count before they read t_ext.  il_cnt: ceil(M / 128) + 1 ints, zero when the launch starts (arrivals
   // per row block, then a time-out flag); the launch leaves the arrivals in them.
   int il_blocks = 0;
+  int il_tile = 0, il_waves = 0;        // lora_gemm_fine.hip: rows and columns of a shrink tile, waves that share its sum
   int* il_cnt = nullptr;
   // two-launch / in-launch forms: rank columns >= r_used of t_ext and b_cat are all zero (0: unknown, use R); the
   // 128x128 / 256x128 and 256x320 kernels then skip the MFMA steps that would only add zeros
@@ -254,6 +255,14 @@ int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
 bool lora_gemm_fine_ok(const LoraGemmParams& p);
 int lora_gemm_fine_form(const LoraGemmParams& p, int order);
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream);
+// the fine tile that a call with T given runs on, -1 where another kernel is chosen
+int lora_gemm_pipe_fine_form(const LoraGemmParams& p);
+// Shrink and GEMM in one launch on fine tiles that leave CUs idle (p.a_cat / col_scale / b_cat set, p.t_ext = scratch for the shrink result,
+// p.il_cnt = counters)
+bool lora_gemm_fine_il_ok(LoraGemmParams p);
+int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream);
+// how many waves share a sum of the stand-alone shrink of this call (lora_shrink.hip)
+int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used);
 // Shrink and GEMM in one launch on the 128 x 160 tiles, every workgroup computing a piece of T first (p.a_cat / col_scale /
 // b_cat set, p.t_ext = scratch for the shrink result, p.il_cnt = counters, p.r_used <= 96 of R = 128).
 bool lora_gemm_fine_coop_ok(const LoraGemmParams& p);

@@ -594,7 +594,7 @@ KH_EXPORT int kh_lora_linear_split_launches(int64_t M, int64_t N, int64_t K, int
                                   n_split, (flags & 1) != 0);
   p.r_used = ((flags >> 16) & 0xff) * 16;
   if ((flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p)) return 1;
-  return lora_gemm_pipe_il_ok(p) ? 1 : 2;
+  return lora_gemm_pipe_il_ok(p) || lora_gemm_fine_il_ok(p) ? 1 : 2;
 }
 
 KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void* bias, const void* a_cat,
@@ -620,7 +620,7 @@ KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void
     p.r_used = ((flags >> 16) & 0xff) * 16;
     kh_take_weight_prefetch(p);
     if ((flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
-    return lora_gemm_pipe_launch_il(p, (hipStream_t)stream);
+    return lora_gemm_pipe_il_ok(p) ? lora_gemm_pipe_launch_il(p, (hipStream_t)stream) : lora_gemm_fine_launch_il(p, (hipStream_t)stream);
   }
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, nullptr, nullptr, nullptr, 0.f, (hipStream_t)stream,
                                        (int)R, ((flags >> 16) & 0xff) * 16);
@@ -697,6 +697,7 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
   if (counters != nullptr && tile_sel == 0 && (flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p))
     return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
   if (counters != nullptr && tile_sel == 0 && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_il(p, (hipStream_t)stream);
+  if (counters != nullptr && tile_sel == 0 && lora_gemm_fine_il_ok(p)) return lora_gemm_fine_launch_il(p, (hipStream_t)stream);
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
   if (rc != KH_OK) return rc;
   p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;

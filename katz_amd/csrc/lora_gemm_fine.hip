@@ -96,8 +96,15 @@ struct FCfg {
 // never waits before its own piece is out, so the launch makes progress in whatever order its workgroups become
 // resident, as long as no OTHER launch whose workgroups wait for each other shares the device with it (the binding does
 // not use this form on a second stream).
-template <class C, bool CONV, bool COOP>
-__global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
+//
+// IL: a launch whose tiles leave enough CUs idle brings the shrink along: its first il_blocks workgroups compute one 16 x 16 (or 32 x 32) tile
+// of T each, store it write-through and count themselves into the counter of their 128 rows; the GEMM workgroups wait, bounded, for
+// that count before their first request for T.  The shrink workgroups have the lowest ids and wait for nothing, so they are resident
+// before anything waits for them.
+enum { T_GIVEN = 0, T_COOP = 1, T_IL = 2 };
+constexpr int il_lds(int waves) { return waves == 8 ? cmax(SHRINK16_LDS<8>, SCfg<8, 1, 1, 2>::LDS) : cmax(SHRINK16_LDS<5>, SCfg<5, 1, 1, 3>::LDS); }
+template <class C, bool CONV, int TMODE>
+__global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, NST = C::NST, PD = C::PD;
@@ -108,8 +115,34 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
   const int pw = wave & 3, wm = pw / (C::WK * C::WN), wn = pw / C::WK % C::WN, wk = pw % C::WK;
   const int lr = lane % C::MF, lg = lane / C::MF;      // row inside an MFMA tile, 16-byte (8-byte) piece of a k-step
 
-    // tile of this workgroup: XCD b % 8 owns a block of xr_m x xr_n tiles (its W rows stay in its L2)
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  constexpr bool COOP = TMODE == T_COOP;
+  if constexpr (TMODE == T_IL) {
+    if ((int)blockIdx.x < p.il_blocks) {
+      const int r = p.r_used > 0 ? p.r_used : p.R, size = p.il_tile, gx = (p.M + size - 1) / size, ct = (r + size - 1) / size;
+      const int bx = (int)blockIdx.x % gx, by = (int)blockIdx.x / gx;
+      if (by >= ct * (p.ldt / p.R) || wave >= p.il_waves) return;      // padding to a multiple of 8 (the XCD map of the rest); idle waves
+      ShrinkParams sp;
+      sp.x = p.x; sp.a_cat = p.a_cat; sp.col_scale = p.col_scale; sp.t = const_cast<bf16_t*>(p.t_ext);
+      sp.M = p.M; sp.K = p.K; sp.R = p.ldt;
+      sp.ln_part = p.ln_part; sp.ln_ca1 = p.ln_ca1; sp.ln_ca2 = p.ln_ca2; sp.ln_eps = p.ln_eps;
+      const int r0 = by / ct * p.R + by % ct * size;
+      static_assert(il_lds(5) <= C::LDS, "the shrink tiles' rings");
+      if (il_lds(8) <= C::LDS && p.il_waves == 8) {
+        if (size == 16) lora_shrink16_tile<8, true>(sp, bx * 16, r0, smem);
+        else lora_shrink_tile<SCfg<8, 1, 1, 2>, true, 512>(sp, bx * 32, r0, smem);
+      } else {
+        if (size == 16) lora_shrink16_tile<5, true>(sp, bx * 16, r0, smem);
+        else lora_shrink_tile<SCfg<5, 1, 1, 3>, true, 320>(sp, bx * 32, r0, smem);
+      }
+      __builtin_amdgcn_s_waitcnt(0);                          // this thread's write-through stores have completed
+      __syncthreads();
+      if (tid == 0) __hip_atomic_fetch_add(p.il_cnt + bx * size / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
+  const int bid = (int)blockIdx.x - (TMODE == T_IL ? p.il_blocks : 0), n_wg = (int)gridDim.x - (TMODE == T_IL ? p.il_blocks : 0);
+  // tile of this workgroup: XCD b % 8 owns a block of xr_m x xr_n tiles (its W rows stay in its L2)
+  const int xcd = bid & 7, local = bid >> 3;
   const int m_blk = (xcd / p.xg_n) * p.xr_m + local / p.xr_n;
   const int n_blk = (xcd % p.xg_n) * p.xr_n + local % p.xr_n;
   if (local / p.xr_n >= p.xr_m || m_blk >= p.m_tiles || n_blk >= p.n_tiles) return;  // padding of the grid
@@ -199,11 +232,15 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
     char* stage = smem + st;
     const int so = t * ROWB;
     if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
-      if (COOP && t == KT1) {
-        // first request for T: wait (bounded) until every workgroup of this row block has delivered its piece
+      if (TMODE != T_GIVEN && t == KT1) {
+        // first request for T: wait (bounded) until every workgroup of these 128 rows has delivered its piece
         if (lane == 0) {
-          int it = 0;
-          while (__hip_atomic_load(p.il_cnt + m_blk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p.n_tiles && ++it < (1 << 20))
+          int it = 0, want = p.n_tiles;
+          if (TMODE == T_IL) {
+            const int left = M - m0 / 128 * 128;
+            want = ((left < 128 ? left : 128) + p.il_tile - 1) / p.il_tile * ((r_ext + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
+          }
+          while (__hip_atomic_load(p.il_cnt + m0 / 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want && ++it < (1 << 20))
             __builtin_amdgcn_s_sleep(8);
           if (it >= (1 << 20)) {
             __hip_atomic_store(p.il_cnt + (p.M + 127) / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -217,8 +254,8 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
         if (q < LPS_LO || has_hi) {
           const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
           const uint32_t vo = col < r_ext ? voff2[EXT ? q : 0] : OOB;
-          // (COOP) T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
-          if (COOP && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
+          // T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
+          if (TMODE != T_GIVEN && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
           else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 0);
         }
       }
@@ -355,7 +392,7 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
     constexpr int TOUCH = C::GLU ? 8 : 24;
     touch(0, TOUCH);
-    kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, blockIdx.x, gridDim.x, tid, 256);
+    kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
     if constexpr (C::GLU) {
 #pragma unroll 4
@@ -633,16 +670,12 @@ __global__ __launch_bounds__(512, COOP ? 1 : 2) void lora_gemm_fine_kernel(const
 #endif
 }
 
-template <class C, bool CONV, bool COOP = false>
-int launch_fine(LoraGemmParams p, hipStream_t stream) {
-  const int seg_rows = CONV && p.gn_part != nullptr ? p.conv_ho * p.conv_wo : p.M;
-  const int seg_tiles = (seg_rows + C::BM - 1) / C::BM;
-  p.m_tiles = p.M / seg_rows * seg_tiles;
+// the tiles of a call and the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
+template <class C>
+bool plan_tiles(LoraGemmParams& p, int seg_rows) {
+  if (p.N % C::BN != 0 || (p.t_nsplit > 0 && p.t_nsplit % C::BN != 0)) return false;
+  p.m_tiles = p.M / seg_rows * ((seg_rows + C::BM - 1) / C::BM);
   p.n_tiles = p.N / C::BN;
-  if (p.N % C::BN != 0 || (p.t_nsplit > 0 && p.t_nsplit % C::BN != 0)) return KH_ERR_UNSUPPORTED;
-  if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
-  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, COOP>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
-  // the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
   double best = 0;
   p.xg_n = 0;
   for (int gm = 1; gm <= 8; gm *= 2) {
@@ -651,9 +684,33 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
     const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
     if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
   }
-  const unsigned grid = 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, COOP>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
-            seg_rows, seg_tiles);
+  return p.st_part == nullptr || p.n_tiles <= KH_LN_SLOTS;
+}
+
+// ... and its shrink's: a CU each beside the GEMM's on every XCD; 16 x 16 where they fit (T is there sooner)
+template <class C>
+bool plan_il(LoraGemmParams& p) {
+  if (!plan_tiles<C>(p, p.M) || il_lds(p.il_waves) > C::LDS) return false;
+  const int r = p.r_used > 0 ? p.r_used : p.R;
+  for (p.il_tile = 16; p.il_tile <= 32; p.il_tile *= 2) {
+    const long pieces = (long)((p.M + p.il_tile - 1) / p.il_tile) * ((r + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
+    if ((pieces + 7) / 8 + (long)p.xr_m * p.xr_n > 32) continue;
+    p.il_blocks = (int)((pieces + 7) / 8 * 8);
+    return true;
+  }
+  return false;
+}
+
+template <class C, bool CONV, int TMODE = T_GIVEN>
+int launch_fine(LoraGemmParams p, hipStream_t stream) {
+  const int seg_rows = CONV && p.gn_part != nullptr ? p.conv_ho * p.conv_wo : p.M;
+  if (!plan_tiles<C>(p, seg_rows)) return KH_ERR_UNSUPPORTED;
+  if constexpr (TMODE == T_IL)
+    if (!plan_il<C>(p)) return KH_ERR_UNSUPPORTED;
+  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, TMODE>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
+  const unsigned grid = (unsigned)(TMODE == T_IL ? p.il_blocks : 0) + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
+  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, TMODE>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
+            seg_rows, (seg_rows + C::BM - 1) / C::BM);
   KH_RETURN_LAST_ERROR();
 }
 
@@ -751,5 +808,40 @@ int lora_gemm_fine_coop_timeouts(int* count, int clear) {
 
 int lora_gemm_fine_launch_coop(const LoraGemmParams& p, hipStream_t stream) {
   if (!lora_gemm_fine_coop_ok(p)) return KH_ERR_UNSUPPORTED;
-  return launch_fine<FCfg<128, 160, 2>, false, true>(p, stream);
+  return launch_fine<FCfg<128, 160, 2>, false, T_COOP>(p, stream);
+}
+
+// Shrink inside the launch (IL) for a call that two launches would run on a fine tile (order 0, and order 4 on 160 columns), where the tiles leave
+// the CUs for it; where 64 x 80 tiles leave none but 64 x 128 do, on those (no row statistics hang on the width).  The shrink's sums are those of
+// its own launch and the tiles' those of the order, so one launch and two give the same bits.
+// us per call, weights from HBM, two launches -> one: M 154 / N 1280 / K 2048, rank 96 16.6 -> 13.2; 512 / 1280 / 1280, rank 32 13.0 -> 10.1;
+// 512 / 1280 / 5120 35.5 -> 30.4; 988 / 1280 / 1280, rank 16 12.9 -> 11.7; GEGLU 640 / 10240 / 1280, rank 16 36.3 -> 33.4.
+template <class F>
+static int with_il_tile(int form, F f) {
+  switch (form) {
+    case 0: return f(FCfg<64, 80, 0>{});
+    case 1: return f(FCfg<128, 80, 0>{});
+    case 2: return f(FCfg<32, 128, 0>{});
+    case 3: return f(FCfg<64, 128, 0>{});
+    case 4: return f(FCfg<32, 160, 4>{});
+    case 7: return f(FCfg<64, 320, 0, true>{});
+    case 8: return f(FCfg<128, 320, 0, true>{});
+    default: return KH_ERR_UNSUPPORTED;
+  }
+}
+
+static int il_form(LoraGemmParams& p) {
+  if (p.a_cat == nullptr || p.col_scale == nullptr || p.t_ext == nullptr || p.il_cnt == nullptr || p.R <= 0 || p.conv_cin > 0) return -1;
+  if (p.ldt != (p.t_nsplit > 0 ? p.N / p.t_nsplit : 1) * p.R) return -1;
+  p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
+  if (p.il_waves != 5 && p.il_waves != 8) return -1;
+  const auto planned = [&](int form) { return with_il_tile(form, [&](auto c) { return plan_il<decltype(c)>(p) ? KH_OK : KH_ERR_UNSUPPORTED; }) == KH_OK; };
+  const int form = lora_gemm_pipe_fine_form(p);
+  return planned(form) ? form : form == 0 && planned(3) ? 3 : -1;
+}
+
+bool lora_gemm_fine_il_ok(LoraGemmParams p) { return il_form(p) >= 0; }
+
+int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream) {
+  return with_il_tile(il_form(p), [&](auto c) { return launch_fine<decltype(c), false, T_IL>(p, stream); });
 }

@@ -1363,6 +1363,27 @@ int lora_gemm_pipe_launch_grouped(const LoraGemmParams& p, int n_groups, hipStre
   return launch_pcfg<PCfg<128, 128, 2, 2, 0, 4>>(p, stream, n_groups);
 }
 
+// 256x320 tiles when they fill at least three quarters of whole rounds of the 256 CUs: fewer operand bytes per
+// FLOP than any smaller tile and no ragged last round
+static bool wide_fills(const LoraGemmParams& p) {
+  if (!lora_gemm_wide_ok(p)) return false;
+  const long wt = (long)(p.M / 256) * (p.N / 320), rounds = (wt + 255) / 256;
+  return wt * 4 >= rounds * 256 * 3;
+}
+
+int lora_gemm_pipe_fine_form(const LoraGemmParams& p) {
+  if (wide_fills(p) || !plain_ok(p)) return -1;
+  const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  // N a multiple of 160 and a tile count that leaves 128x128 tiles with a ragged last round: 160-column tiles
+  // give every CU exactly one.  64-row tiles pay for their extra operand traffic only on long K.
+  if (!p.geglu && p.N % 160 == 0 && p.t_nsplit % 160 == 0 && lora_gemm_fine_ok(p)) {
+    const long n160 = p.N / 160;
+    if (tiles > 256 && tiles <= 384 && (long)((p.M + 127) / 128) * n160 <= 256) return lora_gemm_fine_form(p, 2);
+    if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560) return lora_gemm_fine_form(p, 4);
+  }
+  return lora_gemm_fine_form(p, 0);   // few enough rows for one round of small tiles
+}
+
 int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t stream) {
   switch (tile_sel) {
     case 16: return launch_prank<128, 128, 2, 2, 4>(p, stream);
@@ -1383,25 +1404,10 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
   // busy with them; when the 128x128 tiles do not even fill one round of 256 CUs, one 8-wave workgroup
   // per CU with 64-column stages (full 128-byte lines) beats two 4-wave ones; 128x128 / 4 waves /
   // two workgroups per CU otherwise.
-  if (lora_gemm_wide_ok(p)) {
-    // 256x320 tiles when they fill at least three quarters of whole rounds of the 256 CUs: fewer operand bytes per
-    // FLOP than any smaller tile and no ragged last round
-    const long wt = (long)(p.M / 256) * (p.N / 320), rounds = (wt + 255) / 256;
-    if (wt * 4 >= rounds * 256 * 3) return lora_gemm_wide_launch(p, stream);
-  }
+  if (wide_fills(p)) return lora_gemm_wide_launch(p, stream);
+  if (const int form = lora_gemm_pipe_fine_form(p); form >= 0) return lora_gemm_fine_launch(p, form, stream);
   if (plain_ok(p)) {
     const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-    // N a multiple of 160 and a tile count that leaves 128x128 tiles with a ragged last round: 160-column tiles
-    // give every CU exactly one.  64-row tiles pay for their extra operand traffic only
-    // on long K.
-    if (!p.geglu && p.N % 160 == 0 && p.t_nsplit % 160 == 0 && lora_gemm_fine_ok(p)) {
-      const long n160 = p.N / 160;
-      if (tiles > 256 && tiles <= 384 && (long)((p.M + 127) / 128) * n160 <= 256) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 2), stream);
-      if (tiles <= 192 && (long)((p.M + 63) / 64) * n160 <= 256 && (long)((p.M + 63) / 64) * n160 > tiles && p.K >= 2560)
-        return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 4), stream);
-    }
-    // few enough rows for one round of small tiles
-    if (const int form = lora_gemm_fine_form(p, 0); form >= 0) return lora_gemm_fine_launch(p, form, stream);
     if (tiles >= 480 && p.K >= 1024 && !p.geglu) return deep_stage_ok(p) ? launch_pcfg<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream) : launch_pcfg<PCfg<256, 128, 4, 2, 0, 4>>(p, stream);
     if (tiles <= 256 && deep_stage_ok(p)) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
   }

@@ -50,85 +50,13 @@ int launch_shrink(const ShrinkParams& p, hipStream_t stream) {
   KH_RETURN_LAST_ERROR();
 }
 
-// Few rows: 16 x 16 tiles.  A CU takes 55 .. 110 GB/s of operand lines whatever it does with them, so a call that 32 x 32 tiles
-// spread over 62 CUs (988 rows, two column tiles) is bound by those CUs' streams: 655 KB each at K 5120, 10.2 us.  16-row tiles of
-// 16 rank columns halve the bytes of a tile, leave out the columns that are padding (rank 16 in 64: 62 tiles instead of 124 halves),
-// and four 4 KB stages per wave keep 128 KB in flight.  mfma 16x16x32 gives the bits of two chained 16-column steps of 32x32x16, the
-// chunks go to the waves as above and their sums are added in the same order: the results are those of the 32 x 32 tiles.
-// 988 rows, rank 16 in 64: K 1280 6.1 -> 4.75 us, K 5120 10.9 -> 6.8; 512 rows, rank 64, K 1280: 4.6 -> 3.5.
+// Few rows: 16 x 16 tiles (lora_shrink16_tile)
 template <int NW>
 __global__ __launch_bounds__(NW * 64) void lora_shrink16_kernel(const ShrinkParams p, int group, int tiles) {   // tiles: in use per group
 #if __HIP_DEVICE_COMPILE__
-  constexpr int NS = 4, UNITS = 4, STAGE = UNITS * 1024, LD = 20;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lr = lane & 15, lg = lane >> 4;
-  const int m0 = (int)blockIdx.x * 16, g = (int)blockIdx.y / tiles, tile = (int)blockIdx.y % tiles, r0 = g * group + tile * 16;
-  const int K = p.K, n = (K / 64 - wave + NW - 1) / NW;
-  char* ring = smem + wave * (NS * STAGE);
-  auto clamp32 = [](size_t bytes) { return (int)(uint32_t)(bytes < 0xFFFFFFFFull ? bytes : 0xFFFFFFFFull); };
-  const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.x + (size_t)m0 * K), 0, clamp32((size_t)(p.M - m0) * K * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.a_cat + (size_t)r0 * K), 0, clamp32((size_t)(p.R - r0) * K * 2), 0x00020000);
-  uint32_t voff[UNITS];
-#pragma unroll
-  for (int u = 0; u < UNITS; ++u) {                    // 8 rows of 128 bytes each: x, x, A_cat, A_cat
-    const int ru = u * 8 + (lane >> 3), row = ru & 15;
-    voff[u] = (uint32_t)(u < 2 && m0 + row >= p.M ? p.M - 1 - m0 : row) * (uint32_t)K * 2u + (uint32_t)wave * 128u + (uint32_t)(((lane & 7) ^ ((ru >> 1) & 7)) * 16);
-  }
-  auto issue = [&](int i) {
-    char* st = ring + (i % NS) * STAGE;
-#pragma unroll
-    for (int u = 0; u < UNITS; ++u)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(u < 2 ? rsx : rsa, (lptr_t)(st + u * 1024), 16, voff[u], i * (NW * 128), 0, 0);
-  };
-  KhLnTileStats<16, NW * 64> ln_stats;
-  if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, p.M, tid);
-  const int c = 2 * (tid & 7);                          // this thread's two columns of the result, row tid / 8
-  const bool last = tid < 128;
-  float cs0 = 0.f, cs1 = 0.f, a10 = 0.f, a11 = 0.f, a20 = 0.f, a21 = 0.f;
-  if (last) {
-    cs0 = p.col_scale[r0 + c]; cs1 = p.col_scale[r0 + c + 1];
-    if (p.ln_part != nullptr) { a10 = p.ln_ca1[r0 + c]; a11 = p.ln_ca1[r0 + c + 1]; a20 = p.ln_ca2[r0 + c]; a21 = p.ln_ca2[r0 + c + 1]; }
-  }
-#pragma unroll
-  for (int i = 0; i < NS; ++i)
-    if (i < n) issue(i);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int sw = (lr >> 1) & 7;
-  for (int i = 0; i < n; ++i) {
-    if (i + 3 < n) wait_vm<3 * UNITS>(); else if (i + 2 < n) wait_vm<2 * UNITS>(); else if (i + 1 < n) wait_vm<UNITS>(); else wait_vm<0>();
-    const char* st = ring + (i % NS) * STAGE + lr * 128;
-    bf16x8 a[2], b[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      a[ks] = *reinterpret_cast<const bf16x8*>(st + ((4 * ks + lg) ^ sw) * 16);
-      b[ks] = *reinterpret_cast<const bf16x8*>(st + 16 * 128 + ((4 * ks + lg) ^ sw) * 16);
-    }
-    wait_lgkm0();
-    if (i + NS < n) issue(i + NS);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks], b[ks], acc, 0, 0, 0);
-  }
-  __syncthreads();
-  float* part = reinterpret_cast<float*>(smem);         // [NW][16][LD]
-  float* sMu = part + NW * 16 * LD;
-  float* sSg = sMu + 16;
-  if (p.ln_part != nullptr) ln_stats.finish(K, p.ln_eps, tid, sMu, sSg, true);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) part[(wave * 16 + 4 * lg + e) * LD + lr] = acc[e];
-  __syncthreads();
-  const int rr = tid >> 3;
-  if (last && m0 + rr < p.M) {
-    float s0 = part[rr * LD + c], s1 = part[rr * LD + c + 1];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) { s0 += part[(w * 16 + rr) * LD + c]; s1 += part[(w * 16 + rr) * LD + c + 1]; }
-    if (p.ln_part != nullptr) {
-      const float mu = sMu[rr], sg = sSg[rr];
-      s0 = s0 - mu * a10 + sg * a20;
-      s1 = s1 - mu * a11 + sg * a21;
-    }
-    *reinterpret_cast<uint32_t*>(p.t + (size_t)(m0 + rr) * p.R + r0 + c) = pack_bf16x2(s0 * cs0, s1 * cs1);
-  }
+  const int tid = threadIdx.x, m0 = (int)blockIdx.x * 16, g = (int)blockIdx.y / tiles, tile = (int)blockIdx.y % tiles;
+  lora_shrink16_tile<NW, false>(p, m0, g * group + tile * 16, smem);
   if (tile == tiles - 1) {                              // the group's padding columns of these rows
     const int pieces = group / 8 - tiles * 2;
     for (int i = tid; i < 16 * pieces; i += NW * 64) {
@@ -141,7 +69,7 @@ __global__ __launch_bounds__(NW * 64) void lora_shrink16_kernel(const ShrinkPara
 
 template <int NW>
 int launch_shrink16(const ShrinkParams& p, int group, int tiles, hipStream_t stream) {
-  constexpr int LDS = NW * 4 * 4096;
+  constexpr int LDS = SHRINK16_LDS<NW>;
   if (hipError_t e = kh_allow_lds<lora_shrink16_kernel<NW>>(LDS); e != hipSuccess) return (int)e;
   dim3 grid((unsigned)((p.M + 15) / 16), (unsigned)(p.R / group * tiles));
   kh_launch(KH_TAG_LORA_SHRINK, lora_shrink16_kernel<NW>, grid, dim3(NW * 64), LDS, stream, p, group, tiles);
@@ -161,6 +89,14 @@ int launch_shrink_k(const ShrinkParams& p, hipStream_t stream) {
 KH_EXPORT int kh_lora_shrink_bf16(const void* x, const void* a_cat, const float* col_scale, void* t, int64_t M,
                                   int64_t K, int64_t R, void* stream) {
   return lora_shrink_ln_launch(x, a_cat, col_scale, t, M, K, R, nullptr, nullptr, nullptr, 0.f, (hipStream_t)stream, 0, 0);
+}
+
+// How many waves the rules below give a sum: chunk t of 64 columns is added up by wave t % waves, then wave after wave.
+int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used) {
+  const int64_t kc = K / 64;
+  if (group == 128 && r_used > 64 && r_used <= 96 && R % 128 == 0 && R >= 256 && M >= 4096) return 1;
+  if (R % 64 == 0 && (((M + 63) / 64) * (R / 64) >= 160 || ((M + 31) / 32) * (R / 64) >= 256)) return kc % 4 == 0 || kc % 5 != 0 ? 4 : 5;
+  return kc % 8 == 0 || kc % 5 != 0 ? 8 : 5;
 }
 
 // The shrink, optionally of a layer with a folded LayerNorm (ln_part != nullptr; see ShrinkParams).

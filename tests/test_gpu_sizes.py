@@ -337,6 +337,70 @@ def test_fine_tiles_with_folded_norms_do_not_depend_on_the_rows(rows, N, K, stat
         assert torch.equal(st, stl[:, :rows])
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used,kind", [
+    (1, 1280, 64, 32, 16, ""), (33, 640, 640, 32, 32, "res"), (154, 1280, 2048, 128, 96, ""), (129, 1280, 1280, 128, 128, "res fold"),
+    (512, 1280, 1280, 64, 32, "res stats"), (31, 1280, 1280, 64, 64, "fold stats"), (988, 1280, 1280, 64, 16, "res stats fold"),
+    (988, 1280, 1280, 128, 96, "res stats"), (700, 640, 640, 32, 32, "stats"), (200, 1280, 5120, 64, 16, "res stats"),
+    (512, 1280, 5120, 64, 64, "res stats"), (300, 1920, 640, 32, 16, "stack fold"), (65, 3840, 1280, 64, 64, "stack"),
+    (988, 1280, 1280, 64, 16, "res"), (512, 3840, 1280, 64, 32, "stack fold"), (300, 10240, 1280, 64, 16, "geglu fold"), (640, 10240, 1280, 64, 64, "geglu")])
+def test_few_rows_bring_their_shrink_along(M, N, K, R, r_used, kind):
+    """Fine tiles that leave CUs idle: the shrink runs on those, in 16 x 16 or 32 x 32 tiles.  One launch and two give the same bits (results
+    and row statistics), columns of T that nobody writes are never read; and the result is right."""
+    from katz_amd import ops
+    from katz_amd.lora import fold_norm_into_adapters, fold_norm_into_weight, interleave_geglu_rows
+
+    say("in-launch shrink of few rows", M, N, K, R, r_used, kind)
+    d = dev()
+    kind = kind.split()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    parts = 3 if "stack" in kind else 1
+    split = N // 3 if parts == 3 else 0
+    x, w, b = rnd(M, K), rnd(N, K) * 0.03, rnd(N)
+    A, B = rnd(parts, R, K) * 0.05, rnd(N, R) * 0.05
+    A[:, r_used:], B[:, r_used:] = 0, 0
+    A, B0 = A.reshape(parts * R, K), B
+    w0, b0, A0 = w, b, A
+    geglu = "geglu" in kind
+    if geglu:
+        w, b, B = interleave_geglu_rows(w), interleave_geglu_rows(b), interleave_geglu_rows(B)
+    s = torch.rand(parts * R + 1, generator=g).to(d)[1:]      # (an array that is not 16-byte aligned)
+    res = rnd(M, N) if "res" in kind else None
+    ln, xn = None, x
+    if "fold" in kind:
+        gamma, beta = 1 + 0.1 * rnd(K), 0.1 * rnd(K)
+        w, c1, c2 = fold_norm_into_weight(w, b, gamma, beta)
+        A, ca1, ca2 = fold_norm_into_adapters(A, gamma, beta)
+        st = ops.row_stats_buffer(M, d).zero_()
+        st[0, :, 0], st[0, :, 1] = x.float().sum(1), (x.float() ** 2).sum(1)
+        ln, b = (st, c1, c2, ca1, ca2, 1e-5), None
+        xn = torch.nn.functional.layer_norm(x.double(), (K,), gamma.double(), beta.double(), 1e-5)
+    if "stats" not in kind:   # (asked for the call without statistics, which has tiles of its own)
+        assert ops._lib.load().kh_lora_linear_split_launches(M, N, K, R, split, int(geglu) | r_used // 16 << 16) == 1
+    ops.split_counters_reset(d)
+    out = []
+    for two in (False, True):
+        junk = torch.full((M, parts * R), float("nan"), device=d, dtype=torch.bfloat16)     # the next scratch of this size
+        del junk
+        so = ops.row_stats_buffer(M, d).zero_() if "stats" in kind else None
+        y = ops.lora_linear_norm(x, w, b, residual=res, a_cat=A, col_scale=s, b_cat=B, geglu=geglu, n_split=split, r_used=r_used, two_launches=two,
+                                 ln=ln, stats_out=so)
+        out.append((y, so))
+    ops.check_split_timeouts(d)
+    assert torch.equal(out[0][0], out[1][0])
+    if "stats" in kind:
+        assert torch.equal(out[0][1], out[1][1])
+    xd, step = xn.double(), N // parts
+    ref = torch.cat([xd @ w0[j * step:(j + 1) * step].double().T + b0[j * step:(j + 1) * step].double()
+                     + ((xd @ A0[j * R:(j + 1) * R].double().T) * s[j * R:(j + 1) * R].double()) @ B0[j * step:(j + 1) * step].double().T for j in range(parts)], 1)
+    if geglu:
+        ref = ref[:, :N // 2] * torch.nn.functional.gelu(ref[:, N // 2:])
+    if res is not None:
+        ref = ref + res.double()
+    # bf16 roundings of T, of the folded weights, of the result: 2^-9 each, two of them before a sum
+    assert ((out[0][0].double() - ref).norm() / ref.norm()).item() < 8e-3
+
+
 @pytest.mark.parametrize("M,N,K,R", [(65, 2560, 640, 0), (988, 10240, 1280, 64), (577, 10240, 640, 0), (2048, 5120, 640, 128), (129, 10240, 64, 0)])
 def test_fine_geglu_tiles(M, N, K, R):
     """64 x 320 and 128 x 320 tiles with the GEGLU epilogue (codes 57, 58) against the 128 x 128 kernel, bit for bit."""
