@@ -39,6 +39,14 @@ __device__ __forceinline__ void wait_cnt() {  // gfx9 encoding: vmcnt = [15:14|3
   __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((LGKM & 15) << 8) | ((VM >> 4) << 14));
 }
 
+// until at most n K tiles of LPS loads each are outstanding (n >= N: N tiles)
+template <int LPS, int N>
+__device__ __forceinline__ void wait_tiles(int n) {
+  if constexpr (N <= 0) wait_cnt<0, 0>();
+  else if (n >= N) wait_cnt<LPS * N, 0>();
+  else wait_tiles<LPS, N - 1>(n);
+}
+
 // a bare barrier (a fence would drain the prefetches), kept in place among the memory accesses around it
 __device__ __forceinline__ void ring_barrier() {
   asm volatile("" ::: "memory");
@@ -57,7 +65,8 @@ struct FCfg {
   static constexpr bool GLU = GLU_;                      // GEGLU epilogue
   static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 || BN % 128 != 0 ? 1 : (BM == 32 ? 4 : 2), WM = 4 / (WK * WN);
+  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
+                       WM = 4 / (WK * WN);
   // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
   static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
   static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 4 ? 1 : 2;   // a wave's MFMA tiles, its k-steps per stage
@@ -75,7 +84,7 @@ struct FCfg {
   static constexpr int NH = WK > 1 && 4 * TM * TN * G > 80 ? 2 : 1;
   static constexpr int PART = GLU ? 0 : WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
   static constexpr int TAIL = PART + BM * LDC * 2;
-  static constexpr int NST = cmin(8, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;   // as many stages as fit, but at most 8
+  static constexpr int NST = cmin(16, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;  // as many stages as fit, but at most 16
   static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + 1024;   // (where prefetched dwords nobody reads land)
   static constexpr int OPC = BM * (BN / 8), OPT = (OPC + 511) / 512;             // 16-byte output pieces: per tile, per thread
   static_assert(WM * WN * WK == 4 && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
@@ -281,16 +290,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   };
   // until at most n of this wave's younger K tiles are outstanding (and its LDS reads are done)
   auto wait_younger = [&](int n) {
-    if (n >= PD - 1) { if (has_hi) wait_cnt<LPS_HI * (PD - 1), 0>(); else wait_cnt<LPS_LO * (PD - 1), 0>(); return; }
-    switch (n) {
-      case 6: if (has_hi) wait_cnt<LPS_HI * (PD > 6 ? 6 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 6 ? 6 : 0), 0>(); break;
-      case 5: if (has_hi) wait_cnt<LPS_HI * (PD > 5 ? 5 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 5 ? 5 : 0), 0>(); break;
-      case 4: if (has_hi) wait_cnt<LPS_HI * (PD > 4 ? 4 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 4 ? 4 : 0), 0>(); break;
-      case 3: if (has_hi) wait_cnt<LPS_HI * (PD > 3 ? 3 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 3 ? 3 : 0), 0>(); break;
-      case 2: if (has_hi) wait_cnt<LPS_HI * (PD > 2 ? 2 : 0), 0>(); else wait_cnt<LPS_LO * (PD > 2 ? 2 : 0), 0>(); break;
-      case 1: if (has_hi) wait_cnt<LPS_HI, 0>(); else wait_cnt<LPS_LO, 0>(); break;
-      default: wait_cnt<0, 0>(); break;
-    }
+    if (has_hi) wait_tiles<LPS_HI, PD - 1>(n); else wait_tiles<LPS_LO, PD - 1>(n);
   };
 
   // fragments: row lr of each block of MF rows; of a k-step the lane's 16-byte piece lg (16x16x16: its 8 bytes lg)
@@ -360,21 +360,27 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
       c2v[c] = p.ln_part != nullptr ? p.ln_c2[col] : 0.f;
       biasv[c] = p.ln_part == nullptr && p.bias != nullptr ? reinterpret_cast<const uint16_t*>(p.bias)[col] : (uint16_t)0;
     }
+    // K tiles go out in order as their stages come free; those of a T that is being made beside this tile once the loop is under
+    // way (the wait for it holds up every step behind it; 300 / 640 / 640, rank 64, on 32 x 64 tiles: 10.4 us with it in front of the loop, 6.6 here)
+    const int KTI = TMODE == T_IL ? KT1 : KT;
 #pragma unroll
     for (int t = 0; t < PD; ++t)
-      if (t < KT) issue(t, t * STAGE);
-    wait_younger(KT - 1);
+      if (t < KTI) issue(t, t * STAGE);
+    wait_younger(KTI - 1);
     ring_barrier();
-    if (KT > PD) issue(PD, PD * STAGE);
+    if (KTI > PD) issue(PD, PD * STAGE);
     int st = 0, t = 0;                                 // stage of tile t
-    for (; t + NST < KT; ++t) {
+    for (; t + NST < KTI; ++t) {
       wait_younger(PD - 1);
       ring_barrier();
       issue(t + NST, st);
       st = st + STAGE == NST * STAGE ? 0 : st + STAGE;
     }
+    int next = KTI;                                    // first tile that is not out yet
     for (; t + 1 < KT; ++t) {
-      wait_younger(KT - 2 - t);
+      if constexpr (TMODE == T_IL)
+        for (; next < KT && next < t + NST && (t >= 4 || 2 * t >= KT1 - 1); ++next) issue(next, next % NST * STAGE);
+      wait_younger(next - t - 2);
       ring_barrier();
     }
     if (p.ln_part != nullptr) ln_stats.finish(K, p.ln_eps, ptid, sMu, sRs, false);
@@ -728,7 +734,8 @@ bool lora_gemm_fine_ok(const LoraGemmParams& p) {
 }
 
 // Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
-// GEGLU on 64 x 320 (7), 128 x 320 (8); order 2 on 128 x 160 (9).
+// GEGLU on 64 x 320 (7), 128 x 320 (8); order 2 on 128 x 160 (9); order 0 on 32 x 32 (10), 32 x 64 (11), 64 x 64 (12);
+// order 4 on 32 x 32 (13), 32 x 64 (14), 64 x 64 (15).
 //
 // Order 2: wave tiles of 64 x 160 over two k-slices and waves of their own for the operands, in place of eight 32 x 160 strips that did
 // both: 7 x 32 W and x rows read from LDS per 20 matrix instructions against 6 per 5.  us per launch, weights from HBM: convolutions 640 -> 640
@@ -736,15 +743,46 @@ bool lora_gemm_fine_ok(const LoraGemmParams& p) {
 // rounds), 1280 -> 1280 at 2 x 64 x 64 252 -> 250; linear layers 3952 / 640 / 640 14.1 -> 12.5, 8192 / 640 / 640 14.7 -> 14.0,
 // 4096 / 1280 / 5120 62.6 -> 56.5.
 //
-// Which of them, for a layer whose sums follow `order`: one that fits one round of the 256 CUs (a workgroup fills a CU, so a second round
-// costs as much as the first), the smaller first; -1 where none does and the larger tiles of the other families win.  A
-// convolution that leaves GroupNorm statistics does so per 64 rows.  Measured as launches without adapters in a captured chain whose
-// weights together exceed the memory-side cache, us per launch (M, N, K: the larger tiles -> these):
-// 512 / 1280 / 1280 18.3 -> 9.8 (with row statistics 19.7 -> 11.1); 988 / 1280 / 1280 18.6 -> 9.8 (19.8 -> 11.9); 2048 / 1280 / 1280
-// 16.4 -> 13.1; 988 / 1280 / 5120 43.7 -> 30.6; 2048 / 1280 / 5120 45.7 -> 39.5; 154 / 1280 / 2048 23.5 -> 12.6; a round too many:
-// 1152 / 1280 / 1280 on 64 x 80 16.3 against 12.0 on 128 x 80.  GEGLU: 512 / 10240 / 1280 29.5 -> 22.1, 988 / 10240 / 1280
-// 44.9 -> 34.9, 2048 / 5120 / 640 26.1 -> 20.9.  Convolutions: 988 pixels 1280 -> 1280 84 -> 61, 2048 pixels 640 -> 640 46 -> 30.
-// (With adapters, 1024 and more rows at N 1280 do not come here: lora_gemm_pipe_il_ok takes them first.)
+// Few rows: the shrink of a call with adapters runs inside the launch, on CUs that its tiles leave idle (T_IL).  The shrink's sums are those of
+// its own launch and the tiles' those of the order, so one launch and two give the same bits.
+template <class F>
+static int with_il_tile(int form, F f) {
+  switch (form) {
+    case 0: return f(FCfg<64, 80, 0>{});
+    case 1: return f(FCfg<128, 80, 0>{});
+    case 2: return f(FCfg<32, 128, 0>{});
+    case 3: return f(FCfg<64, 128, 0>{});
+    case 4: return f(FCfg<32, 160, 4>{});
+    case 5: return f(FCfg<64, 160, 4>{});
+    case 7: return f(FCfg<64, 320, 0, true>{});
+    case 8: return f(FCfg<128, 320, 0, true>{});
+    case 10: return f(FCfg<32, 32, 0>{});
+    case 11: return f(FCfg<32, 64, 0>{});
+    case 12: return f(FCfg<64, 64, 0>{});
+    case 13: return f(FCfg<32, 32, 4>{});
+    case 14: return f(FCfg<32, 64, 4>{});
+    case 15: return f(FCfg<64, 64, 4>{});
+    default: return KH_ERR_UNSUPPORTED;
+  }
+}
+
+// the pieces of T (16 or 32 wide) that a launch of this form brings along; 0: it leaves no CUs for them
+static int shrink_beside(LoraGemmParams& p, int form) {
+  if (p.t_ext == nullptr || p.R <= 0 || p.ldt != (p.t_nsplit > 0 ? p.N / p.t_nsplit : 1) * p.R) return 0;
+  p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
+  if (p.il_waves != 5 && p.il_waves != 8) return 0;
+  return with_il_tile(form, [&](auto c) { return plan_il<decltype(c)>(p) ? KH_OK : KH_ERR_UNSUPPORTED; }) == KH_OK ? p.il_tile : 0;
+}
+
+// Which of them, for a layer whose sums follow `order`; -1 where none fits and the larger tiles of the other families win.  A
+// convolution that leaves GroupNorm statistics does so per 64 rows.
+//
+// Linear layers: a CU's time is the rows it streams, BM + BN of K columns each, so the tile with the fewest of them whose workgroups fit
+// one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  With adapters, the first that leaves the
+// CUs for 16 x 16 pieces of the shrink; then, where the loop is long enough to hide the larger pieces, for 32 x 32 ones; else two launches.
+// us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
+// 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
+// 512 / 1280 / 1280, 32 10.1 -> 9.3; 300 / 640 / 640, 64 7.3 -> 6.4; no adapters: 154 / 640 / 2048 12.1 -> 8.3, 655 / 1280 / 2048 12.2 -> 11.1.
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   if (!lora_gemm_fine_ok(p)) return -1;
   const long hw = p.gn_part != nullptr ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
@@ -756,9 +794,27 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
     return fits(64, 320) ? (hw + 63) / 64 * (p.N / 320) > 128 ? 7 : -1 : fits(128, 320) ? 8 : -1;
   }
   if (order == 2) return 9;
-  if (order == 0) return p.st_part != nullptr ? (fits(32, 128) ? 2 : fits(64, 128) ? 3 : -1) : (fits(64, 80) ? 0 : fits(128, 80) ? 1 : -1);
-  if (p.gn_part != nullptr) return 80 % p.gn_cg == 0 && fits(64, 80) ? 6 : 5;
-  return fits(32, 160) ? 4 : 5;
+  if (p.conv_cin > 0) return p.gn_part != nullptr ? (80 % p.gn_cg == 0 && fits(64, 80) ? 6 : 5) : fits(32, 160) ? 4 : 5;
+  struct Tile { int form, bm, bn; };
+  constexpr Tile tiles0[] = {{10, 32, 32}, {11, 32, 64}, {12, 64, 64}, {0, 64, 80}, {2, 32, 128}, {3, 64, 128}, {1, 128, 80}};
+  constexpr Tile tiles4[] = {{13, 32, 32}, {14, 32, 64}, {15, 64, 64}, {4, 32, 160}, {5, 64, 160}};
+  const bool stats = p.st_part != nullptr, adapters = p.t_ext != nullptr;
+  auto first = [&](int piece) {          // piece: the shrink's pieces beside the tiles, 0: none needed
+    auto of = [&](const Tile* t, int n, int width) {
+      for (; n > 0; ++t, --n) {
+        if (!fits(t->bm, t->bn) || (stats && t->bn != width)) continue;
+        if (LoraGemmParams q = p; piece == 0 || shrink_beside(q, t->form) == piece) return t->form;
+      }
+      return -1;
+    };
+    return order == 0 ? of(tiles0, 7, 128) : of(tiles4, 5, 160);
+  };
+  if (adapters) {
+    if (const int f = first(16); f >= 0) return f;
+    if (p.K >= 1280)
+      if (const int f = first(32); f >= 0) return f;
+  }
+  return first(0);
 }
 
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
@@ -776,6 +832,12 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 7: return launch_fine<FCfg<64, 320, 0, true>, false>(p, stream);
     case 8: return launch_fine<FCfg<128, 320, 0, true>, false>(p, stream);
     case 9: return conv ? launch_fine<FCfg<128, 160, 2>, true>(p, stream) : launch_fine<FCfg<128, 160, 2>, false>(p, stream);
+    case 10: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 32, 0>, false>(p, stream);
+    case 11: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 64, 0>, false>(p, stream);
+    case 12: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 64, 0>, false>(p, stream);
+    case 13: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 32, 4>, false>(p, stream);
+    case 14: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 64, 4>, false>(p, stream);
+    case 15: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 64, 4>, false>(p, stream);
     default: return KH_ERR_UNSUPPORTED;
   }
 }
@@ -811,33 +873,14 @@ int lora_gemm_fine_launch_coop(const LoraGemmParams& p, hipStream_t stream) {
   return launch_fine<FCfg<128, 160, 2>, false, T_COOP>(p, stream);
 }
 
-// Shrink inside the launch (IL) for a call that two launches would run on a fine tile (order 0, and order 4 on 160 columns), where the tiles leave
-// the CUs for it; where 64 x 80 tiles leave none but 64 x 128 do, on those (no row statistics hang on the width).  The shrink's sums are those of
-// its own launch and the tiles' those of the order, so one launch and two give the same bits.
-// us per call, weights from HBM, two launches -> one: M 154 / N 1280 / K 2048, rank 96 16.6 -> 13.2; 512 / 1280 / 1280, rank 32 13.0 -> 10.1;
-// 512 / 1280 / 5120 35.5 -> 30.4; 988 / 1280 / 1280, rank 16 12.9 -> 11.7; GEGLU 640 / 10240 / 1280, rank 16 36.3 -> 33.4.
-template <class F>
-static int with_il_tile(int form, F f) {
-  switch (form) {
-    case 0: return f(FCfg<64, 80, 0>{});
-    case 1: return f(FCfg<128, 80, 0>{});
-    case 2: return f(FCfg<32, 128, 0>{});
-    case 3: return f(FCfg<64, 128, 0>{});
-    case 4: return f(FCfg<32, 160, 4>{});
-    case 7: return f(FCfg<64, 320, 0, true>{});
-    case 8: return f(FCfg<128, 320, 0, true>{});
-    default: return KH_ERR_UNSUPPORTED;
-  }
-}
-
+// Shrink inside the launch (IL): the form of lora_gemm_fine_form, where its tiles leave the CUs.
+// us per call, weights from HBM, two launches -> one: M 154 / N 1280 / K 2048, rank 96 14.9 -> 10.7; 512 / 1280 / 1280, rank 32 12.9 -> 9.3;
+// 512 / 1280 / 5120 30.9 -> 24.0; 988 / 1280 / 1280, rank 16 15.8 -> 12.2 (64 x 80 tiles and two launches 13.7); GEGLU 640 / 10240 / 1280, rank 16 36.3 -> 33.4.
 static int il_form(LoraGemmParams& p) {
-  if (p.a_cat == nullptr || p.col_scale == nullptr || p.t_ext == nullptr || p.il_cnt == nullptr || p.R <= 0 || p.conv_cin > 0) return -1;
-  if (p.ldt != (p.t_nsplit > 0 ? p.N / p.t_nsplit : 1) * p.R) return -1;
-  p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
-  if (p.il_waves != 5 && p.il_waves != 8) return -1;
-  const auto planned = [&](int form) { return with_il_tile(form, [&](auto c) { return plan_il<decltype(c)>(p) ? KH_OK : KH_ERR_UNSUPPORTED; }) == KH_OK; };
+  if (p.a_cat == nullptr || p.col_scale == nullptr || p.il_cnt == nullptr || p.conv_cin > 0) return -1;
   const int form = lora_gemm_pipe_fine_form(p);
-  return planned(form) ? form : form == 0 && planned(3) ? 3 : -1;
+  const int piece = shrink_beside(p, form);
+  return piece == 16 || (piece == 32 && p.K >= 1280) ? form : -1;   // (the rule of the forms)
 }
 
 bool lora_gemm_fine_il_ok(LoraGemmParams p) { return il_form(p) >= 0; }

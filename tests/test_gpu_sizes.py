@@ -287,6 +287,63 @@ def test_fine_tiles_give_the_bits_of_the_large_ones(M, N, K, R, r_used):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used", [(1, 640, 64, 0, 0), (33, 640, 128, 64, 16), (64, 1280, 960, 128, 96), (65, 640, 1024, 64, 0), (154, 1280, 2048, 0, 0),
+                                            (31, 1280, 5120, 64, 32), (63, 320, 192, 32, 0)])
+def test_narrow_tiles_give_the_bits_of_the_large_ones(M, N, K, R, r_used):
+    """Codes 60 .. 62 (32 x 32, 32 x 64, 64 x 64) add up like the 128 x 128 kernel (16), 63 .. 65 like the 64 x 160 one (40): edges of their rows,
+    K shorter and longer than their rings of up to 16 stages, rank columns that fill no stage."""
+    from katz_amd import ops
+
+    say("narrow tiles", M, N, K, R, r_used)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N)
+    t, bc = (rnd(M, R), rnd(N, R) * 0.05) if R else (None, None)
+    if r_used:
+        t[:, r_used:] = 0
+        bc[:, r_used:] = 0
+    for rs in (None, res):
+        run = (lambda c: ops.lora_linear_pre(x, w, b, t, bc, residual=rs, tile=c, r_used=r_used)) if R else (lambda c: ops.lora_linear(x, w, b, residual=rs, tile=c))
+        for codes, ref in (((60, 61, 62), 16), ((63, 64, 65), 40)):
+            if ref == 40 and R % 64:
+                continue
+            want = run(ref)
+            for c in codes:
+                assert torch.equal(run(c), want), (c, rs is not None)
+
+
+@pytest.mark.parametrize("M,N,K,R,r_used,stats", [(1, 640, 64, 64, 16, False), (65, 640, 640, 64, 64, True), (300, 640, 640, 64, 64, False), (77, 1280, 2048, 64, 32, False),
+                                                  (33, 1280, 128, 128, 96, False), (512, 1280, 5120, 64, 32, False), (1000, 640, 2560, 64, 16, True),
+                                                  (200, 640, 2560, 128, 96, False), (700, 1280, 1280, 64, 16, True), (900, 1280, 5120, 64, 16, True)])
+def test_few_rows_forms_of_the_dispatch(M, N, K, R, r_used, stats):
+    """The form the sizes choose, as one launch and as two: the same bits (results and row statistics), a right result, no wait that ran out."""
+    from katz_amd import ops
+
+    say("forms of the dispatch", M, N, K, R, r_used, stats)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res, A, B = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N), rnd(R, K) * 0.05, rnd(N, R) * 0.05
+    A[r_used:], B[:, r_used:] = 0, 0
+    s = torch.rand(R, generator=g).to(d)
+    ops.split_counters_reset(d)
+    out = []
+    for two in (False, True):
+        so = ops.row_stats_buffer(M, d).zero_() if stats else None
+        out.append((ops.lora_linear_norm(x, w, b, residual=res, a_cat=A, col_scale=s, b_cat=B, r_used=r_used, two_launches=two, stats_out=so), so))
+    ops.check_split_timeouts(d)
+    assert torch.equal(out[0][0], out[1][0])
+    y = out[0][0].double()
+    if stats:
+        assert torch.equal(out[0][1], out[1][1])
+        got = out[0][1].double().sum(0)
+        # fp32 sums of N values of size about 1: N * 2^-24 of their absolute sum at most
+        assert torch.allclose(got[:, 0], y.sum(1), atol=N * N * 2.0 ** -24, rtol=0) and torch.allclose(got[:, 1], (y * y).sum(1), rtol=N * 2.0 ** -24)
+    ref = x.double() @ w.double().T + b.double() + ((x.double() @ A.double().T) * s.double()) @ B.double().T + res.double()
+    assert ((y - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
+
+
 @pytest.mark.parametrize("M,N,K,R,r_used", [(1, 160, 64, 0, 0), (129, 320, 128, 64, 48), (127, 640, 640, 128, 96), (4000, 640, 576, 0, 0), (8192, 640, 2560, 128, 80)])
 def test_fine_128x160_tiles(M, N, K, R, r_used):
     """Code 59 (128 x 160, two k-slices) against the kernel whose order of sums it keeps (41), bit for bit: partial row blocks, K shorter
