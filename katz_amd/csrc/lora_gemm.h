@@ -39,6 +39,7 @@ struct LoraGemmParams {
   // per row block, then a time-out flag); the launch leaves the arrivals in them.
   int il_blocks = 0;
   int il_tile = 0, il_waves = 0;        // lora_gemm_fine.hip: rows and columns of a shrink tile, waves that share its sum
+  int il_cols = 0;                      // column tiles of T per 64 rows beside 128 x 128 and 256 x 128 tiles (il_col_tiles)
   int* il_cnt = nullptr;
   // two-launch / in-launch forms: rank columns >= r_used of t_ext and b_cat are all zero (0: unknown, use R); the
   // 128x128 / 256x128 and 256x320 kernels then skip the MFMA steps that would only add zeros
@@ -82,6 +83,21 @@ struct LoraGemmParams {
 
 // bit 24 of the `flags` of kh_lora_linear_split_bf16 / _norm_bf16: do not use the cooperative in-launch shrink (see include/katz_hip.h)
 constexpr int KH_FLAG_NO_COOP = 1 << 24;
+
+// Weight prefetch of a launch with its own shrink: by the idle waves of the shrink workgroups when the first range is short
+__host__ __device__ inline bool il_prefetch_by_idle_waves(const LoraGemmParams& p) { return p.pf_lines[0] <= ((8u << 20) >> 7); }
+
+// In-launch shrink on 64 x 32 tiles: a single layer with R = 64 columns of T, or with 128 of which at most the first 96 are
+// in use (two adapters of ranks 64 + 32, say), short enough in K that its GEMM tiles would otherwise wait for T, and
+// small enough in M that the two or three tiles per 64 rows fit beside the GEMM tiles (M 2048 / N 1280 / K 1280, rank 64: 19.2 us on one 64 x 64
+// tile per 64 rows).  The GEMM tiles never multiply the columns the shrink leaves unwritten (r_used bounds their K loop).
+// Decided on the host: the kernels get the number of column tiles (p.il_cols), more than one per 64 columns of T where they are narrow.
+inline int il_col_tiles(const LoraGemmParams& p) {
+  const int narrow = p.ldt != p.R ? 0 : p.R == 64 ? 2 : p.R == 128 && p.r_used > 0 && p.r_used <= 96 ? 3 : 0;
+  const bool fits = (long)((p.M + 127) / 128) * ((p.N + 127) / 128) + (long)((p.M + 63) / 64) * narrow <= 256;
+  return narrow > 0 && p.K <= 2560 && fits ? narrow : p.ldt / 64;
+}
+__device__ __forceinline__ bool il_narrow(const LoraGemmParams& p) { return p.il_cols * 64 > p.ldt; }
 
 // The pending weight prefetch of this host thread (kh_set_weight_prefetch), handed to the next launch.
 void kh_take_weight_prefetch(LoraGemmParams& p);
@@ -261,6 +277,7 @@ int lora_gemm_pipe_fine_form(const LoraGemmParams& p);
 // p.il_cnt = counters)
 bool lora_gemm_fine_il_ok(LoraGemmParams p);
 int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream);
+int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream);   // ... on 128 x 128 tiles, for lora_gemm_pipe_il_ok
 // how many waves share a sum of the stand-alone shrink of this call (lora_shrink.hip)
 int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used);
 // Shrink and GEMM in one launch on the 128 x 160 tiles, every workgroup computing a piece of T first (p.a_cat / col_scale /

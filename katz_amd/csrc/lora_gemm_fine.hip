@@ -111,6 +111,8 @@ struct FCfg {
 // that count before their first request for T.  The shrink workgroups have the lowest ids and wait for nothing, so they are resident
 // before anything waits for them.
 enum { T_GIVEN = 0, T_COOP = 1, T_IL = 2 };
+using ILTileWide = SCfg<4, 2, 2>;               // the pieces beside 128 x 128 tiles: 64 x 64 ...
+using ILTileNarrow = SCfg<4, 2, 1>;             // ... and 64 x 32 (il_narrow)
 constexpr int il_lds(int waves) { return waves == 8 ? cmax(SHRINK16_LDS<8>, SCfg<8, 1, 1, 2>::LDS) : cmax(SHRINK16_LDS<5>, SCfg<5, 1, 1, 3>::LDS); }
 template <class C, bool CONV, int TMODE>
 __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
@@ -127,16 +129,42 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   constexpr bool COOP = TMODE == T_COOP;
   if constexpr (TMODE == T_IL) {
     if ((int)blockIdx.x < p.il_blocks) {
-      const int r = p.r_used > 0 ? p.r_used : p.R, size = p.il_tile, gx = (p.M + size - 1) / size, ct = (r + size - 1) / size;
+      constexpr bool BIG = BM == 128 && BN == 128;
+      const int r = p.r_used > 0 ? p.r_used : p.R, size = BIG ? 64 : p.il_tile, gx = (p.M + size - 1) / size, ct = BIG ? p.il_cols : (r + size - 1) / size;
       const int bx = (int)blockIdx.x % gx, by = (int)blockIdx.x / gx;
-      if (by >= ct * (p.ldt / p.R) || wave >= p.il_waves) return;      // padding to a multiple of 8 (the XCD map of the rest); idle waves
+      // padding to a multiple of 8 (the XCD map of the rest); idle waves
+      if (by >= (BIG ? ct : ct * (p.ldt / p.R)) || (!BIG && wave >= p.il_waves)) return;
+      if (BIG && wave >= 4) {
+        // The piece is the work of waves 0 .. 3.  When most of its own loads are out, the others hint the next launch's weights (by the GEMM workgroups
+        // in front of their own operands the 1024 x 1024 step took 2 % longer) and fetch what is left of the XCD's block of W into its L2: M 2048 /
+        // N 1280 / K 1280, rank 96, weights from HBM / from the memory-side cache 17.7 / 16.8 us, 17.9 / 18.1 by the computing waves as in the other
+        // forms, 20.1 / 16.4 by nobody.  (The piece's barriers wait until these waves have ended.)
+        const int xcd = (int)blockIdx.x & 7, wgs = (gx * ct - xcd + 7) / 8, KT1 = p.K / BK;
+        char* lds = smem + C::TOUCH_OFF + (wave - 4) * 256;
+        auto touch = [&](int t) {
+          kh_touch_rows(p.w, p.N, p.K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, 8, lds, ((int)blockIdx.x >> 3) * 256 + tid - 256, wgs * 256);
+        };
+        __builtin_amdgcn_s_sleep(127);                       // 8128 clocks, about 10 stages of the K loop
+        const bool hints = il_prefetch_by_idle_waves(p);
+        if (hints) kh_prefetch_lines_idle(p.pf, p.pf_lines, lds, (int)blockIdx.x, gx * ct, tid - 256, 256);
+        for (int t = p.pf[0] != nullptr ? 24 : 8; t < KT1; t += 8) {   // (a caller that hints has had these weights hinted, too)
+          touch(t);
+          if (t >= 24) __builtin_amdgcn_s_sleep(48);
+        }
+        __builtin_amdgcn_s_waitcnt(0);                        // (nothing lands in LDS that is no longer this workgroup's)
+        return;
+      }
       ShrinkParams sp;
       sp.x = p.x; sp.a_cat = p.a_cat; sp.col_scale = p.col_scale; sp.t = const_cast<bf16_t*>(p.t_ext);
       sp.M = p.M; sp.K = p.K; sp.R = p.ldt;
       sp.ln_part = p.ln_part; sp.ln_ca1 = p.ln_ca1; sp.ln_ca2 = p.ln_ca2; sp.ln_eps = p.ln_eps;
       const int r0 = by / ct * p.R + by % ct * size;
+      static_assert(cmax(ILTileWide::LDS, ILTileNarrow::LDS) <= C::TOUCH_OFF || !BIG, "the shrink tiles' rings");
       static_assert(il_lds(5) <= C::LDS, "the shrink tiles' rings");
-      if (il_lds(8) <= C::LDS && p.il_waves == 8) {
+      if constexpr (BIG) {
+        if (il_narrow(p)) lora_shrink_tile<ILTileNarrow, true, 256>(sp, bx * 64, by * 32, smem);
+        else lora_shrink_tile<ILTileWide, true, 256>(sp, bx * 64, by * 64, smem);
+      } else if (il_lds(8) <= C::LDS && p.il_waves == 8) {
         if (size == 16) lora_shrink16_tile<8, true>(sp, bx * 16, r0, smem);
         else lora_shrink_tile<SCfg<8, 1, 1, 2>, true, 512>(sp, bx * 32, r0, smem);
       } else {
@@ -247,7 +275,8 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
           int it = 0, want = p.n_tiles;
           if (TMODE == T_IL) {
             const int left = M - m0 / 128 * 128;
-            want = ((left < 128 ? left : 128) + p.il_tile - 1) / p.il_tile * ((r_ext + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
+            if (BM == 128 && BN == 128) want = ((left < 128 ? left : 128) + 63) / 64 * p.il_cols;
+            else want = ((left < 128 ? left : 128) + p.il_tile - 1) / p.il_tile * ((r_ext + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
           }
           while (__hip_atomic_load(p.il_cnt + m0 / 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want && ++it < (1 << 20))
             __builtin_amdgcn_s_sleep(8);
@@ -391,14 +420,15 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
     auto touch = [&](int t, int n) {
-      if (t < KT1)
+      if (!(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
         kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
     constexpr int TOUCH = C::GLU ? 8 : 24;
     touch(0, TOUCH);
-    kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
+    if (!(TMODE == T_IL && BM == 128 && BN == 128 && il_prefetch_by_idle_waves(p)))
+      kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
     if constexpr (C::GLU) {
 #pragma unroll 4
@@ -711,7 +741,7 @@ template <class C, bool CONV, int TMODE = T_GIVEN>
 int launch_fine(LoraGemmParams p, hipStream_t stream) {
   const int seg_rows = CONV && p.gn_part != nullptr ? p.conv_ho * p.conv_wo : p.M;
   if (!plan_tiles<C>(p, seg_rows)) return KH_ERR_UNSUPPORTED;
-  if constexpr (TMODE == T_IL)
+  if constexpr (TMODE == T_IL && !(C::BM == 128 && C::BN == 128))
     if (!plan_il<C>(p)) return KH_ERR_UNSUPPORTED;
   if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, TMODE>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
   const unsigned grid = (unsigned)(TMODE == T_IL ? p.il_blocks : 0) + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
@@ -881,6 +911,16 @@ static int il_form(LoraGemmParams& p) {
   const int form = lora_gemm_pipe_fine_form(p);
   const int piece = shrink_beside(p, form);
   return piece == 16 || (piece == 32 && p.K >= 1280) ? form : -1;   // (the rule of the forms)
+}
+
+// Shrink inside the launch, 128 x 128 tiles: the calls of lora_gemm_pipe_il_ok's first kind.  Against the kernel of lora_gemm_pipe.hip, whose eight
+// waves both moved operands and computed 64 x 32 each, us per call with statistics, rank 96, weights from the memory-side cache / from HBM:
+// 2048 / 1280 / 1280 17.2 -> 16.8 / 20.0 -> 17.7; 2048 / 1280 / 5120 41.5 -> 38.5 / 54.5 -> 43.3; rank 64 without statistics 18.0 -> 16.3 / -.
+int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream) {
+  using C = FCfg<128, 128, 0>;
+  p.il_cols = il_col_tiles(p);
+  p.il_blocks = ((p.M + 63) / 64 * p.il_cols + 7) / 8 * 8;
+  return launch_fine<C, false, T_IL>(p, stream);
 }
 
 bool lora_gemm_fine_il_ok(LoraGemmParams p) { return il_form(p) >= 0; }

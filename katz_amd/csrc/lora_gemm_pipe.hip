@@ -596,19 +596,6 @@ using ILTileNarrow = SCfg<4, 2, 1>;             // ... and 64 x 32 (see il_narro
 constexpr int IL_SHRINK_LDS = ILTileWide::LDS > ILTileNarrow::LDS ? ILTileWide::LDS : ILTileNarrow::LDS;
 constexpr int IL_PF_OFF = IL_SHRINK_LDS;        // in-launch shrink workgroups: LDS offset of their prefetch landing zone (1 KB)
 
-// Weight prefetch of a launch with its own shrink: by the idle waves of the shrink workgroups when the first range is short
-__host__ __device__ inline bool il_prefetch_by_idle_waves(const LoraGemmParams& p) { return p.pf_lines[0] <= ((8u << 20) >> 7); }
-
-// In-launch shrink on 64 x 32 tiles: a single layer (T has R = 128 columns) of which at most the first 96 rank columns are
-// in use (two adapters of ranks 64 + 32, say), short enough in K that its GEMM tiles would otherwise wait for T, and
-// small enough in M that the three tiles per 64 rows fit beside the GEMM tiles.  The GEMM tiles never multiply the
-// columns the shrink leaves unwritten (r_used bounds their K loop).
-__host__ __device__ inline bool il_narrow(const LoraGemmParams& p) {
-  return p.R == 128 && p.ldt == 128 && p.r_used > 0 && p.r_used <= 96 && p.K <= 2560 &&
-         (long)((p.M + 127) / 128) * ((p.N + 127) / 128) + (long)((p.M + 63) / 64) * 3 <= 256;
-}
-__host__ __device__ inline int il_col_tiles(const LoraGemmParams& p) { return il_narrow(p) ? 3 : p.ldt / 64; }
-
 // LNF bit 0: the instantiation can fold a LayerNorm in front of the layer into its epilogue (ln_part); bit 1: it can write
 // the row statistics for one behind it (st_part).  The plain one (0) carries none of that code.
 // XA: the output tile is an attention's queries and the epilogue runs the cross-attention on it (XAttnTile).
@@ -627,7 +614,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lora_gemm_pipe_kernel(const Lor
       // loop, and a short layer's shrink tile is not done by then: what a tile streams through its 160 KB of LDS sets
       // when T arrives, and 96 tiles still find a CU each beside 160 GEMM tiles
       const bool narrow = il_narrow(pin);
-      const int gx = (pin.M + 63) / 64, gy = il_col_tiles(pin);
+      const int gx = (pin.M + 63) / 64, gy = pin.il_cols;
       if ((int)blockIdx.x >= gx * gy) return;               // padding to a multiple of 8 (the XCD map of the rest)
       const int bx = blockIdx.x % gx, by = blockIdx.x / gx;
       ShrinkParams sp;
@@ -938,7 +925,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lora_gemm_pipe_kernel(const Lor
         constexpr int TPB = BM / 64;                                                   // 64-row shrink tiles per row block
         const int gx = (M + 63) / 64, rt = gx - TPB * m_blk < TPB ? gx - TPB * m_blk : TPB;
         k_loop2<C, CONV, true>(smem, d, rs, KT, KT1, lane, wave, wm, wn, l32, lh, sw, acc, ConvGeom{0, 0},
-                               p.il_cnt + m_blk, rt * il_col_tiles(p), p.il_cnt + (p.M + 127) / 128, half_last);
+                               p.il_cnt + m_blk, rt * p.il_cols, p.il_cnt + (p.M + 127) / 128, half_last);
       } else {
         k_loop2<C, CONV, false>(smem, d, rs, KT, KT1, lane, wave, wm, wn, l32, lh, sw, acc, ConvGeom{p.conv_w, p.conv_cin},
                                 nullptr, 0, nullptr, half_last);
@@ -1218,7 +1205,7 @@ static int il_form(const LoraGemmParams& p) {
                   p.col_scale != nullptr && p.il_cnt != nullptr && t_ok && p.grp == nullptr && p.sg_mode == 0 && p.conv_cin == 0 &&
                   !p.geglu && p.M >= 1024;
   if (!ok) return 0;
-  if (tiles <= 192 && tiles + shr <= 256) return 1;
+  if (tiles <= 192 && tiles + shr <= 256) return p.xa_k != nullptr || (p.N % 128 == 0 && lora_gemm_fine_ok(p)) ? 1 : 0;
   if (tiles >= 480 && p.K >= 1024 && (long)((p.M + 255) / 256) * ((p.N + 127) / 128) <= 256 && shr <= 256) return 2;
   return 0;
 }
@@ -1264,43 +1251,42 @@ static int launch_il(const LoraGemmParams& pin, hipStream_t stream) {
     const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
     if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
   }
-  const int shr = ((p.M + 63) / 64) * il_col_tiles(p);
+  p.il_cols = il_col_tiles(p);
+  const int shr = ((p.M + 63) / 64) * p.il_cols;
   p.il_blocks = (shr + 7) / 8 * 8;
   const unsigned grid = (unsigned)p.il_blocks + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  if (p.xa_k != nullptr) {
-    if constexpr (std::is_same<C, PCfg<128, 128, 2, 4, 0, 4, 64>>::value) {
-      if (p.res != nullptr || p.st_part != nullptr || p.M % 128 != 0 || p.N % 128 != 0) return KH_ERR_UNSUPPORTED;
-      auto go = [&](auto lnf) {
-        constexpr int L = decltype(lnf)::value;
-        if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L, true>>(LDS_LN); e != hipSuccess) return (int)e;
-        kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L, true>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
-        KH_RETURN_LAST_ERROR();
-      };
-      return p.ln_part != nullptr ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 0>{});
-    } else {
-      return KH_ERR_UNSUPPORTED;
-    }
-  }
-  if (p.ln_part != nullptr || p.st_part != nullptr) {
-    if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
+  if constexpr (std::is_same<C, PCfg<128, 128, 2, 4, 0, 4, 64>>::value) {   // only behind a query projection
+    if (p.xa_k == nullptr || p.res != nullptr || p.st_part != nullptr || p.M % 128 != 0 || p.N % 128 != 0) return KH_ERR_UNSUPPORTED;
     auto go = [&](auto lnf) {
       constexpr int L = decltype(lnf)::value;
-      if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L>>(LDS_LN); e != hipSuccess) return (int)e;
-      kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
+      if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L, true>>(LDS_LN); e != hipSuccess) return (int)e;
+      kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L, true>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
       KH_RETURN_LAST_ERROR();
     };
-    if (p.ln_part != nullptr && p.st_part != nullptr) return go(std::integral_constant<int, 3>{});
-    if (p.ln_part != nullptr) return go(std::integral_constant<int, 1>{});
-    return go(std::integral_constant<int, 2>{});
+    return p.ln_part != nullptr ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 0>{});
+  } else {
+    if (p.xa_k != nullptr) return KH_ERR_UNSUPPORTED;
+    if (p.ln_part != nullptr || p.st_part != nullptr) {
+      if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
+      auto go = [&](auto lnf) {
+        constexpr int L = decltype(lnf)::value;
+        if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L>>(LDS_LN); e != hipSuccess) return (int)e;
+        kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
+        KH_RETURN_LAST_ERROR();
+      };
+      if (p.ln_part != nullptr && p.st_part != nullptr) return go(std::integral_constant<int, 3>{});
+      if (p.ln_part != nullptr) return go(std::integral_constant<int, 1>{});
+      return go(std::integral_constant<int, 2>{});
+    }
+    if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true>>(LDS); e != hipSuccess) return (int)e;
+    kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true>, dim3(grid), dim3(C::NT), (size_t)LDS, stream, p);
+    KH_RETURN_LAST_ERROR();
   }
-  if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true>>(LDS); e != hipSuccess) return (int)e;
-  kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true>, dim3(grid), dim3(C::NT), (size_t)LDS, stream, p);
-  KH_RETURN_LAST_ERROR();
 }
 
 int lora_gemm_pipe_launch_il(const LoraGemmParams& p, hipStream_t stream) {
   switch (il_form(p)) {
-    case 1: return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
+    case 1: return lora_gemm_fine_launch_il128(p, stream);
     case 2: return launch_il<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream);
     default: return KH_ERR_UNSUPPORTED;
   }

@@ -344,6 +344,40 @@ def test_few_rows_forms_of_the_dispatch(M, N, K, R, r_used, stats):
     assert ((y - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used,stats", [(1024, 1280, 1280, 64, 64, False), (1100, 640, 128, 64, 16, True), (3952, 640, 640, 64, 16, True), (4096, 640, 640, 64, 64, False),
+                                                  (3968, 640, 64, 64, 16, False), (2048, 1280, 5120, 128, 96, True), (1985, 1280, 1280, 128, 96, False), (1537, 1280, 1280, 128, 128, False)])
+def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
+    """One round of 128 x 128 tiles with 64 x 64 or 64 x 32 pieces of the shrink beside them, ragged last row blocks, a K loop much shorter than
+    the shrink (the tiles wait for T): against the same call with T made in front, and against float64; repeated, on a T that starts as NaNs."""
+    from katz_amd import ops
+
+    say("shrink beside 128 x 128 tiles", M, N, K, R, r_used, stats)
+    d = dev()
+    assert ops._lib.load().kh_lora_linear_split_launches(M, N, K, R, 0, r_used // 16 << 16) == 1
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res, A, B = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(M, N), rnd(R, K) * 0.05, rnd(N, R) * 0.05
+    A[r_used:], B[:, r_used:] = 0, 0
+    s = torch.rand(R, generator=g).to(d)
+
+    def run(two):
+        ops.split_counters_reset(d)
+        junk = torch.full((M, R), float("nan"), device=d, dtype=torch.bfloat16)     # the next scratch of this size
+        del junk
+        so = ops.row_stats_buffer(M, d).zero_() if stats else None
+        return ops.lora_linear_norm(x, w, b, residual=res, a_cat=A, col_scale=s, b_cat=B, r_used=r_used, two_launches=two, stats_out=so), so
+
+    y, so = run(False)
+    for _ in range(3):
+        again, so2 = run(False)
+        assert torch.equal(again, y) and (so is None or torch.equal(so, so2))
+    ops.check_split_timeouts(d)
+    y2, _ = run(True)
+    assert (y != y2).float().mean().item() < 5e-3      # the shrinks add up in different orders: a few last bits of T
+    ref = x.double() @ w.double().T + b.double() + ((x.double() @ A.double().T) * s.double()) @ B.double().T + res.double()
+    assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
+
+
 @pytest.mark.parametrize("M,N,K,R,r_used", [(1, 160, 64, 0, 0), (129, 320, 128, 64, 48), (127, 640, 640, 128, 96), (4000, 640, 576, 0, 0), (8192, 640, 2560, 128, 80)])
 def test_fine_128x160_tiles(M, N, K, R, r_used):
     """Code 59 (128 x 160, two k-slices) against the kernel whose order of sums it keeps (41), bit for bit: partial row blocks, K shorter
