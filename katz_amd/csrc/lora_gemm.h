@@ -277,6 +277,8 @@ int lora_gemm_pipe_fine_form(const LoraGemmParams& p);
 // p.il_cnt = counters)
 bool lora_gemm_fine_il_ok(LoraGemmParams p);
 int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream);
+bool lora_gemm_fine_grouped_ok(const LoraGemmParams& p);     // many layers on the same few rows (p.grp)
+int lora_gemm_fine_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream);
 int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream);   // ... on 128 x 128 tiles, for lora_gemm_pipe_il_ok
 // how many waves share a sum of the stand-alone shrink of this call (lora_shrink.hip)
 int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used);

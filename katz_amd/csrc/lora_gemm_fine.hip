@@ -74,7 +74,7 @@ struct FCfg {
   // (128 x 320: 5.6 K clocks against 8.4 K), (x, W) four rows of a column.  One x fragment per W fragment is the exception: the K loop of 64 x 80
   // takes 8.8 K clocks with (x, W) and 9.9 K with (W, x), more than the epilogue saves.
   static constexpr bool XW = BM == 64 && BN == 80 && ORD == 0;
-  static constexpr bool DB = TM * TN * G * 4 <= 96 && !GLU;      // two fragment buffers where the registers allow it
+  static constexpr bool DB = TM * TN * G * 4 <= 96 && BM <= 128 && !GLU;      // two fragment buffers where the registers allow it
   static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
   static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
   static constexpr int UNITS = ROWS / UR, LPS_LO = UNITS / 4, N_HI = UNITS % 4, LPS_HI = LPS_LO + (N_HI ? 1 : 0);
@@ -110,12 +110,14 @@ struct FCfg {
 // of T each, store it write-through and count themselves into the counter of their 128 rows; the GEMM workgroups wait, bounded, for
 // that count before their first request for T.  The shrink workgroups have the lowest ids and wait for nothing, so they are resident
 // before anything waits for them.
-enum { T_GIVEN = 0, T_COOP = 1, T_IL = 2 };
+//
+// GRP: n_groups layers that read the same few rows in one launch (LoraGemmParams::grp, T given); a workgroup takes one tile of one layer.
+enum { T_GIVEN = 0, T_COOP = 1, T_IL = 2, T_GRP = 3 };
 using ILTileWide = SCfg<4, 2, 2>;               // the pieces beside 128 x 128 tiles: 64 x 64 ...
 using ILTileNarrow = SCfg<4, 2, 1>;             // ... and 64 x 32 (il_narrow)
 constexpr int il_lds(int waves) { return waves == 8 ? cmax(SHRINK16_LDS<8>, SCfg<8, 1, 1, 2>::LDS) : cmax(SHRINK16_LDS<5>, SCfg<5, 1, 1, 3>::LDS); }
 template <class C, bool CONV, int TMODE>
-__global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p, const int seg_rows, const int seg_tiles) {
+__global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p0, const int seg_rows, const int seg_tiles) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, NST = C::NST, PD = C::PD;
@@ -126,7 +128,24 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   const int pw = wave & 3, wm = pw / (C::WK * C::WN), wn = pw / C::WK % C::WN, wk = pw % C::WK;
   const int lr = lane % C::MF, lg = lane / C::MF;      // row inside an MFMA tile, 16-byte (8-byte) piece of a k-step
 
-  constexpr bool COOP = TMODE == T_COOP;
+  constexpr bool COOP = TMODE == T_COOP, GRP = TMODE == T_GRP;
+  // GRP: the row tiles of a layer's columns follow each other on one XCD, so that W comes from memory once
+  LoraGemmParams pg;
+  int gm_blk = 0, gn_blk = 0;
+  if constexpr (GRP) {
+    const int local = (int)blockIdx.x >> 3, tile = local / p0.m_tiles * 8 + ((int)blockIdx.x & 7), layer = tile / p0.n_tiles;
+    if (layer >= p0.il_blocks) return;                 // (il_blocks: the number of layers)
+    gm_blk = local % p0.m_tiles;
+    gn_blk = tile - layer * p0.n_tiles;
+    const uint64_t* const g = p0.grp + (size_t)layer * 5;
+    pg = p0;
+    pg.w = reinterpret_cast<const bf16_t*>(g[0]);
+    pg.bias = reinterpret_cast<const bf16_t*>(g[1]);
+    pg.b_cat = reinterpret_cast<const bf16_t*>(g[2]);
+    pg.t_ext = reinterpret_cast<const bf16_t*>(g[3]);
+    pg.y = reinterpret_cast<bf16_t*>(g[4]);
+  }
+  const LoraGemmParams& p = GRP ? pg : p0;
   if constexpr (TMODE == T_IL) {
     if ((int)blockIdx.x < p.il_blocks) {
       constexpr bool BIG = BM == 128 && BN == 128;
@@ -180,9 +199,9 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   const int bid = (int)blockIdx.x - (TMODE == T_IL ? p.il_blocks : 0), n_wg = (int)gridDim.x - (TMODE == T_IL ? p.il_blocks : 0);
   // tile of this workgroup: XCD b % 8 owns a block of xr_m x xr_n tiles (its W rows stay in its L2)
   const int xcd = bid & 7, local = bid >> 3;
-  const int m_blk = (xcd / p.xg_n) * p.xr_m + local / p.xr_n;
-  const int n_blk = (xcd % p.xg_n) * p.xr_n + local % p.xr_n;
-  if (local / p.xr_n >= p.xr_m || m_blk >= p.m_tiles || n_blk >= p.n_tiles) return;  // padding of the grid
+  const int m_blk = GRP ? gm_blk : (xcd / p.xg_n) * p.xr_m + local / p.xr_n;
+  const int n_blk = GRP ? gn_blk : (xcd % p.xg_n) * p.xr_n + local % p.xr_n;
+  if (!GRP && (local / p.xr_n >= p.xr_m || m_blk >= p.m_tiles || n_blk >= p.n_tiles)) return;  // padding of the grid
   const int M = p.M, N = p.N, K = p.K;
   const int seg = m_blk / seg_tiles, m0 = seg * seg_rows + (m_blk % seg_tiles) * BM, n0 = n_blk * BN;
   const int seg_end = (seg + 1) * seg_rows, rows = (seg_end < M ? seg_end : M) - m0;   // rows of this tile that exist (may exceed BM)
@@ -269,7 +288,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     char* stage = smem + st;
     const int so = t * ROWB;
     if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
-      if (TMODE != T_GIVEN && t == KT1) {
+      if ((COOP || TMODE == T_IL) && t == KT1) {
         // first request for T: wait (bounded) until every workgroup of these 128 rows has delivered its piece
         if (lane == 0) {
           int it = 0, want = p.n_tiles;
@@ -293,7 +312,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
           const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
           const uint32_t vo = col < r_ext ? voff2[EXT ? q : 0] : OOB;
           // T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
-          if (TMODE != T_GIVEN && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
+          if ((COOP || TMODE == T_IL) && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
           else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 0);
         }
       }
@@ -373,12 +392,12 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   float* sRs = sMu + 128;
   float* sc1 = sRs + 128;
   float* sc2 = sc1 + BN;
-  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && BM <= 128, "per-row and per-column terms");
+  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && (BM <= 128 || GRP), "per-row and per-column terms");
   if (producer) {
     // requested now, used after the K loop (older than every DMA load, so no wait falls in between)
     constexpr int CP = (BN + 255) / 256;
     const int ptid = tid - 256;
-    KhLnTileStats<BM, 256> ln_stats;
+    KhLnTileStats<cmin(BM, 128), 256> ln_stats;
     float c1v[CP], c2v[CP];
     uint16_t biasv[CP];
     if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, M, ptid);
@@ -420,14 +439,14 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
     auto touch = [&](int t, int n) {
-      if (!(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
+      if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
         kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
     constexpr int TOUCH = C::GLU ? 8 : 24;
     touch(0, TOUCH);
-    if (!(TMODE == T_IL && BM == 128 && BN == 128 && il_prefetch_by_idle_waves(p)))
+    if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128 && il_prefetch_by_idle_waves(p)))
       kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
     if constexpr (C::GLU) {
@@ -911,6 +930,35 @@ static int il_form(LoraGemmParams& p) {
   const int form = lora_gemm_pipe_fine_form(p);
   const int piece = shrink_beside(p, form);
   return piece == 16 || (piece == 32 && p.K >= 1280) ? form : -1;   // (the rule of the forms)
+}
+
+// Many layers on the same few rows (the context projections of every cross-attention).  Bound by their weights, which come from memory once each: a
+// tile is 128 columns of a layer, and so many of its rows, up to 160, that no second workgroup asks for those weights.  us per launch, two-per-CU tiles of
+// 128 x 128 -> these: 120 layers of 2048 -> 1280, 154 rows, rank columns 128 284 -> 188 (3.4 TB/s of weights), 77 rows, 64 199 -> 151, 308 rows, 64 440 -> 269,
+// 20 rows, 64 175 -> 136; 20 layers of 2048 -> 640, 154 rows, 128 34.8 -> 19.3; 60 layers, 600 rows, 64 316 -> 239.
+template <int BM>
+static int launch_grouped(LoraGemmParams p, int n_groups, hipStream_t stream) {
+  using C = FCfg<BM, 128, 0>;
+  p.m_tiles = (p.M + BM - 1) / BM;
+  p.n_tiles = p.N / 128;
+  p.il_blocks = n_groups;
+  const long tiles = (long)n_groups * p.n_tiles, grid = (tiles + 7) / 8 * 8 * p.m_tiles;
+  if (grid > 0x7fffffffL) return KH_ERR_TOO_LARGE;
+  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, false, T_GRP>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
+  kh_launch(KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, false, T_GRP>, dim3((unsigned)grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p, p.M, p.m_tiles);
+  KH_RETURN_LAST_ERROR();
+}
+
+bool lora_gemm_fine_grouped_ok(const LoraGemmParams& p) {
+  const size_t lim = (size_t)1 << 31;
+  return p.K % 64 == 0 && p.N % 128 == 0 && p.M <= 640 && (size_t)p.M * p.K * 2 < lim && (size_t)p.N * p.K * 2 < lim && (size_t)p.N * (p.R > 0 ? p.R : 1) * 2 < lim &&
+         (size_t)p.M * p.ldt * 2 < lim;
+}
+
+int lora_gemm_fine_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream) {
+  const int tiles = (p.M + 159) / 160, rows = (p.M + tiles - 1) / tiles;
+  return rows <= 32 ? launch_grouped<32>(p, n_groups, stream) : rows <= 64 ? launch_grouped<64>(p, n_groups, stream) : rows <= 96 ? launch_grouped<96>(p, n_groups, stream)
+         : rows <= 128 ? launch_grouped<128>(p, n_groups, stream) : launch_grouped<160>(p, n_groups, stream);
 }
 
 // Shrink inside the launch, 128 x 128 tiles: the calls of lora_gemm_pipe_il_ok's first kind.  Against the kernel of lora_gemm_pipe.hip, whose eight

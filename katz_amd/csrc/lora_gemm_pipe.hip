@@ -1346,6 +1346,7 @@ int lora_gemm_pipe_launch_sgmv(const LoraGemmParams& p, int n_segments, hipStrea
 }
 
 int lora_gemm_pipe_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream) {
+  if (lora_gemm_fine_grouped_ok(p)) return lora_gemm_fine_launch_grouped(p, n_groups, stream);
   return launch_pcfg<PCfg<128, 128, 2, 2, 0, 4>>(p, stream, n_groups);
 }
 

@@ -378,6 +378,30 @@ def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("M,N,K,R,layers", [(1, 128, 64, 0, 1), (32, 640, 128, 32, 3), (77, 1280, 2048, 64, 5), (96, 640, 640, 128, 2), (128, 128, 1280, 0, 11), (154, 1280, 2048, 128, 4),
+                                            (161, 640, 192, 64, 3), (308, 1280, 256, 96, 3), (640, 640, 128, 0, 2), (641, 640, 128, 64, 2)])
+def test_grouped_layers_of_few_rows(M, N, K, R, layers):
+    """Layers on the same rows in one launch, T a column slice of one wide shrink result with garbage beside it: the bits of the 128 x 128 kernel
+    (code 16) layer by layer, whatever the row tiles; rows behind the last stay untouched."""
+    import numpy as np
+    from katz_amd import ops
+
+    say("grouped layers", M, N, K, R, layers)
+    d = dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b = rnd(M, K), rnd(layers, N, K) * 0.03, rnd(layers, N)
+    t, bc = (rnd(M, layers * R), rnd(layers, N, R) * 0.05) if R else (None, None)
+    y = torch.full((layers, M + 1, N), 7.0, device=d, dtype=torch.bfloat16)
+    rows = [[w[i].data_ptr(), b[i].data_ptr() if i % 2 == 0 else 0, bc[i].data_ptr() if R else 0, t.data_ptr() + i * R * 2 if R else 0, y[i].data_ptr()] for i in range(layers)]
+    ops.lora_linear_grouped(x, ops.upload_table(np.array(rows, dtype=np.int64), d), M, N, K, R, layers * R if R else 8)
+    for i in range(layers):
+        bias = b[i] if i % 2 == 0 else None
+        want = ops.lora_linear_pre(x, w[i], bias, t[:, i * R:(i + 1) * R], bc[i], tile=16) if R else ops.lora_linear(x, w[i], bias, tile=16)
+        assert torch.equal(y[i, :M], want), i
+        assert bool((y[i, M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M,N,K,R,r_used", [(1, 160, 64, 0, 0), (129, 320, 128, 64, 48), (127, 640, 640, 128, 96), (4000, 640, 576, 0, 0), (8192, 640, 2560, 128, 80)])
 def test_fine_128x160_tiles(M, N, K, R, r_used):
     """Code 59 (128 x 160, two k-slices) against the kernel whose order of sums it keeps (41), bit for bit: partial row blocks, K shorter
