@@ -7,12 +7,19 @@
 // materialised.
 //
 // One workgroup = 4 (or 2) waves = 128 (64) queries of one (batch, head); each wave owns 32 queries.
-// Per 64-key tile (K and V^T staged in LDS, double buffered):
+// Per 64-key tile (K and V in LDS, three stages):
 //   S^T = K . Q^T      (A = K fragment from LDS, B = Q fragment held in registers)
 //   so every lane holds 32 scores of ONE query (query = lane%32): the row max / row sum are
 //   in-lane reductions plus one exchange between the two 32-lane halves.
-//   O^T += V^T . P^T   (A = V^T fragment from LDS, B = P straight from the score registers:
+//   O^T += V^T . P^T   (A = V^T fragment from LDS, transposed by the read (ds_read_tr16_b64), B = P straight from the score registers:
 //   the MFMA K index is a free permutation as long as both operands agree on it.)
+//
+// What bounds it: the vector ALU (exp, scale, maximum, conversion: about 1000 of the 1300 clocks a wave spends on a tile with three waves per SIMD) and,
+// on most grids, the last round of workgroups (640 on 256 CUs: three on some, 2.5 on average).  K and V went through registers before, V transposed by
+// eight 4-byte LDS writes and 16 vector instructions per thread and tile; by DMA into unpadded swizzled tiles, us per call (batch, tokens, heads):
+// 2 x 4096 x 10 129 -> 120, 2 x 3952 x 10 125 -> 114, 2 x 1024 x 20 27.2 -> 24.8, 1 x 3952 x 10 86.7 -> 78.7, 1 x 988 x 20 18.7 -> 17.4, 2 x 256 x 20 6.9 -> 5.9,
+// 988 queries on 77 keys 6.7 -> 5.8.  Same bits.  Transposing reads as inline assembly, without the compiler's wait for every DMA in front of them and
+// with the DMA a whole step ahead, measured the same; 64 queries per workgroup everywhere 160 us at 2 x 4096 x 10, 25.5 at 2 x 1024 x 20.
 #include "kh_common.h"
 #include <type_traits>
 
@@ -20,8 +27,6 @@ namespace {
 
 constexpr int HD = 64;        // head dim
 constexpr int KV = 64;        // keys per tile
-constexpr int LDH = HD + 8;   // padded LDS rows (144 B)
-constexpr int LDV = KV + 8;
 constexpr float NEG_BIG = -1.0e30f;
 constexpr float RESCALE_LOG2 = 8.0f;   // the running maximum moves only for jumps above 2^8
 
@@ -34,15 +39,29 @@ struct AttnParams {
   int q_blocks;
 };
 
+typedef __attribute__((address_space(3))) void* lptr_t;
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef __attribute__((address_space(3))) bf16x4* ltr_t;
+
+constexpr int ROWB = HD * 2;                 // bytes of a K or V row in LDS, unpadded
+constexpr int TILE = KV * ROWB;              // of a tile of either
+constexpr int NST = 3;                       // stages of K and V
+
+template <int VM>
+__device__ __forceinline__ void wait_vm() {  // vmcnt = VM, the other counters unconstrained (gfx9 encoding)
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (15 << 8) | ((VM >> 4) << 14));
+}
+
 template <int NW>   // waves per workgroup: NW*32 queries
 // Two waves per SIMD at least: that caps a wave at 256 registers, which makes the compiler keep MFMA results in
 // VGPRs (the softmax reads them every tile; from AGPRs every score and every rescaled output costs extra moves).
 __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams p) {
-  constexpr int NT = NW * 64, KCH = 512 / NT, VCH = 256 / NT;
-  __shared__ __attribute__((aligned(16))) bf16_t sK[2][KV * LDH];
-  __shared__ __attribute__((aligned(16))) bf16_t sVt[2][HD * LDV];
+#if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
+  constexpr int UPW = 8 / NW;                // 1 KB DMA instructions per wave and tile of K, and of V
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // [NST][K tile, V tile] (named arrays: the compiler waits for every DMA in front of a read)
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, lh = lane >> 5;
   const uint32_t total = (uint32_t)p.q_blocks * p.H * p.B;
   const uint32_t logical = xcd_remap(blockIdx.x, total);
@@ -72,83 +91,47 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
 
   const int n_tiles = (p.S + KV - 1) / KV;
 
-  // staging registers: K tile = 64 keys x 8 chunks (2 per thread); V tile = 32 key pairs x 8 chunks (1 pair per thread)
-  u32x4 rk[KCH], rv[VCH][2];
-  // A full tile is read at (uniform tile base) + (per-thread byte offset fixed for the whole kernel): no per-tile
-  // address arithmetic in the vector ALU, which is the unit this kernel is bound by.  Only a last, partial
-  // tile clamps its rows.
-  uint32_t koff[KCH], voff[VCH][2];
+  // K and V tiles go straight to LDS, two tiles ahead: a DMA instruction is 8 keys of 128 bytes, lane l key l / 8, and the 16-byte piece it fetches
+  // is swizzled by the key so that the reads below spread over the banks.  Keys past S lie beyond the buffer: zeros.
+  auto swz_k = [](int key) { return (key >> 1) & 7; };
+  auto swz_v = [](int key) { return (key & 2) << 1; };
+  uint32_t koff[UPW], voff[UPW];
 #pragma unroll
-  for (int i = 0; i < KCH; ++i) {
-    const int c = tid + i * NT, row = c >> 3, ch = c & 7;
-    koff[i] = (uint32_t)((row * p.ldk + ch * 8) * 2);
+  for (int i = 0; i < UPW; ++i) {
+    const int key = (wave * UPW + i) * 8 + (lane >> 3);
+    koff[i] = (uint32_t)key * (uint32_t)p.ldk * 2u + (uint32_t)(((lane & 7) ^ swz_k(key)) * 16);
+    voff[i] = (uint32_t)key * (uint32_t)p.ldv * 2u + (uint32_t)(((lane & 7) ^ swz_v(key)) * 16);
   }
+  auto load_tile = [&](int t, int st) {      // tile t into the stage at byte st
+    const int s0 = t * KV, last = (p.S - s0 < KV ? p.S - s0 : KV) - 1;
+    const rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(kp + (size_t)s0 * p.ldk), 0, (int)(uint32_t)((last * p.ldk + HD) * 2), 0x00020000);
+    const rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(vp + (size_t)s0 * p.ldv), 0, (int)(uint32_t)((last * p.ldv + HD) * 2), 0x00020000);
 #pragma unroll
-  for (int j = 0; j < VCH; ++j) {
-    const int c = tid + j * NT, v_kp = c & 31, v_dch = c >> 5;
+    for (int i = 0; i < UPW; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lptr_t)(smem + st + (wave * UPW + i) * 1024), 16, koff[i], 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) voff[j][i] = (uint32_t)(((2 * v_kp + i) * p.ldv + v_dch * 8) * 2);
+    for (int i = 0; i < UPW; ++i) __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lptr_t)(smem + st + TILE + (wave * UPW + i) * 1024), 16, voff[i], 0, 0, 0);
+  };
+  // K fragment: key l32 of 32, pieces 2 ks + lh.  V^T fragment: ds_read_tr16_b64 gives lane i of 16 the i-th element of four rows of which the lanes
+  // 4r .. 4r + 3 address the r-th (32 bytes): four keys of dimension i.
+  int ka[4], va[2];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) ka[ks] = l32 * ROWB + ((2 * ks + lh) ^ swz_k(l32)) * 16;
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt) {
+    const int r = (lane & 15) >> 2, piece = dt * 4 + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+    va[dt] = TILE + (4 * lh + r) * ROWB + (piece ^ swz_v(r)) * 16 + (lane & 1) * 8;
   }
-  auto load_tile = [&](int t) {
-    const int s0 = t * KV;
-    if (s0 + KV <= p.S) {
-      const char* kb = reinterpret_cast<const char*>(kp + (size_t)s0 * p.ldk);
-      const char* vb = reinterpret_cast<const char*>(vp + (size_t)s0 * p.ldv);
-#pragma unroll
-      for (int i = 0; i < KCH; ++i) rk[i] = *reinterpret_cast<const u32x4*>(kb + koff[i]);
-#pragma unroll
-      for (int j = 0; j < VCH; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) rv[j][i] = *reinterpret_cast<const u32x4*>(vb + voff[j][i]);
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < KCH; ++i) {
-      const int c = tid + i * NT, row = c >> 3, ch = c & 7;
-      int gr = s0 + row; gr = gr < p.S ? gr : p.S - 1;
-      rk[i] = *reinterpret_cast<const u32x4*>(kp + (size_t)gr * p.ldk + ch * 8);
-    }
-#pragma unroll
-    for (int j = 0; j < VCH; ++j) {
-      const int c = tid + j * NT, v_kp = c & 31, v_dch = c >> 5;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        int gr = s0 + 2 * v_kp + i; gr = gr < p.S ? gr : p.S - 1;
-        rv[j][i] = *reinterpret_cast<const u32x4*>(vp + (size_t)gr * p.ldv + v_dch * 8);
-      }
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < KCH; ++i) {
-      const int c = tid + i * NT, row = c >> 3, ch = c & 7;
-      *reinterpret_cast<u32x4*>(&sK[buf][row * LDH + ch * 8]) = rk[i];
-    }
-    // transpose: element e of the pair (key 2kp, key 2kp+1) -> sVt[d = dch*8+e][2kp .. 2kp+1] as one dword
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&sVt[buf][0]);
-#pragma unroll
-    for (int j = 0; j < VCH; ++j) {
-      const int c = tid + j * NT, v_kp = c & 31, v_dch = c >> 5;
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const uint32_t a = rv[j][0][w], c2 = rv[j][1][w];
-        const uint32_t lo = (a & 0xffffu) | (c2 << 16);          // d = dch*8 + 2w
-        const uint32_t hi = (a >> 16) | (c2 & 0xffff0000u);      // d = dch*8 + 2w + 1
-        dst[((v_dch * 8 + 2 * w) * LDV) / 2 + v_kp] = lo;
-        dst[((v_dch * 8 + 2 * w + 1) * LDV) / 2 + v_kp] = hi;
-      }
-    }
-  };
-
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
+  load_tile(0, 0);
+  if (n_tiles > 1) load_tile(1, 2 * TILE);
+  int stg = 0;                               // stage of the current tile
 
   // One 64-key tile.  MASK: the tile may reach beyond S (only the last one can).
   auto tile_step = [&](int t, auto mask_tag) {
     constexpr bool MASK = decltype(mask_tag)::value;
-    const int buf = t & 1;
-    if (t + 1 < n_tiles) load_tile(t + 1);
+    if (t + 1 < n_tiles) wait_vm<2 * UPW>(); else wait_vm<0>();      // this wave's share of tile t is there
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();            // everybody's; and nobody reads tile t - 1 any more, whose stage tile t + 2 takes
+    asm volatile("" ::: "memory");
 
     // S^T tiles: st[kt][v] : key = t*64 + kt*32 + 8*(v/4) + 4*lh + v%4, query = l32
     f32x16 st[2];
@@ -157,7 +140,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
     for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(&sK[buf][(kt * 32 + l32) * LDH + ks * 16 + lh * 8]);
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(smem + stg + ka[ks] + kt * 32 * ROWB);
         st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], ks == 0 ? zero : st[kt], 0, 0, 0);
       }
     }
@@ -217,9 +200,10 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
       for (int s = 0; s < 2; ++s) {
 #pragma unroll
         for (int dt = 0; dt < 2; ++dt) {
-          const bf16_t* base = &sVt[buf][(dt * 32 + l32) * LDV + kt * 32 + 16 * s + 4 * lh];
-          const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(base);
-          const bf16x4 v1 = *reinterpret_cast<const bf16x4*>(base + 8);
+          // (the swizzle repeats every four keys)
+          const char* base = smem + stg + va[dt] + (kt * 32 + 16 * s) * ROWB;
+          const bf16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((ltr_t)(base));
+          const bf16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((ltr_t)(base + 8 * ROWB));
           bf16x8 vf;
 #pragma unroll
           for (int e = 0; e < 4; ++e) { vf[e] = v0[e]; vf[4 + e] = v1[e]; }
@@ -229,8 +213,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
       }
     l_run += rsum[0];
 
-    if (t + 1 < n_tiles) store_tile(buf ^ 1);
-    __syncthreads();
+    // (behind the reads of V: the compiler waits for every DMA that is out in front of a transposing read)
+    if (t + 2 < n_tiles) load_tile(t + 2, stg >= 2 * TILE ? stg - 2 * TILE : stg + 4 * TILE);
+    stg = stg == 2 * (NST - 1) * TILE ? 0 : stg + 2 * TILE;
   };
   const int full_tiles = p.S / KV;
   for (int t = 0; t < full_tiles; ++t) tile_step(t, std::false_type{});
@@ -240,7 +225,6 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
   // A lane holds runs of 4 dims (8 bytes); lanes l and l + 32 hold the two halves of every 16-byte piece of their query's
   // row.  Two pieces at a time, the pair trades halves (v_permlane32_swap: the upper half of the first register against the
   // lower half of the second), after which lane l owns the even piece and lane l + 32 the odd one: 16-byte stores.
-#if __HIP_DEVICE_COMPILE__
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
@@ -284,8 +268,8 @@ KH_EXPORT int kh_attention_bf16(const void* q, const void* k, const void* v, voi
   const long grid = (long)p.q_blocks * H * B;
   if (grid > 0x7fffffffL) return KH_ERR_TOO_LARGE;
   if (small)
-    kh_launch(KH_TAG_ATTENTION, attention_kernel<2>, dim3((unsigned)grid), dim3(128), 0, (hipStream_t)stream, p);
+    kh_launch(KH_TAG_ATTENTION, attention_kernel<2>, dim3((unsigned)grid), dim3(128), 2 * NST * TILE, (hipStream_t)stream, p);
   else
-    kh_launch(KH_TAG_ATTENTION, attention_kernel<4>, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, p);
+    kh_launch(KH_TAG_ATTENTION, attention_kernel<4>, dim3((unsigned)grid), dim3(256), 2 * NST * TILE, (hipStream_t)stream, p);
   KH_RETURN_LAST_ERROR();
 }

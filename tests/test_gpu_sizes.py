@@ -378,6 +378,30 @@ def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("B,T,S,heads", [(1, 1, 1, 1), (2, 33, 63, 3), (1, 130, 64, 2), (3, 5, 65, 2), (1, 300, 127, 1), (2, 64, 128, 2), (1, 127, 129, 3), (1, 256, 192, 2),
+                                         (1, 40, 193, 2), (1, 129, 400, 1), (2, 700, 321, 20)])
+def test_attention_tiles_of_keys(B, T, S, heads):
+    """One, two, three and more tiles of 64 keys, partial last ones, both sizes of workgroups; k and v are column slices of one tensor whose rows behind the
+    last key, and columns beside them, are NaN: nothing of those may be used."""
+    from katz_amd import ops
+
+    say("attention tiles", B, T, S, heads)
+    d = dev()
+    g = torch.Generator().manual_seed(B + T + S + heads)
+    c = heads * 64
+    q = torch.randn(B, T, c, generator=g).to(d, BF)
+    kv = torch.full((B, S + 70, 2 * c + 64), float("nan"), device=d, dtype=BF)
+    kv[:, :S, :2 * c] = torch.randn(B, S, 2 * c, generator=g).to(d, BF) * 2
+    k, v = kv[:, :S, :c], kv[:, :S, c:2 * c]
+    o = ops.attention(q, k, v, heads)
+    split = lambda t: t.double().reshape(B, -1, heads, 64).transpose(1, 2)
+    p = torch.softmax(split(q) @ split(k).transpose(-1, -2).contiguous() / 8, -1)
+    ref = (p @ split(v)).transpose(1, 2).reshape(B, T, c)
+    # the probabilities and the result are rounded to bf16: 2^-9 each
+    assert ((o.double() - ref).norm() / ref.norm()).item() < 6e-3
+    assert torch.equal(ops.attention(q, k, v, heads), o)
+
+
 @pytest.mark.parametrize("M,N,K,R,layers", [(1, 128, 64, 0, 1), (32, 640, 128, 32, 3), (77, 1280, 2048, 64, 5), (96, 640, 640, 128, 2), (128, 128, 1280, 0, 11), (154, 1280, 2048, 128, 4),
                                             (161, 640, 192, 64, 3), (308, 1280, 256, 96, 3), (640, 640, 128, 0, 2), (641, 640, 128, 64, 2)])
 def test_grouped_layers_of_few_rows(M, N, K, R, layers):
