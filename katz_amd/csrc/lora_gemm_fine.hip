@@ -835,9 +835,9 @@ static int shrink_beside(LoraGemmParams& p, int form) {
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   if (!lora_gemm_fine_ok(p)) return -1;
   const long hw = p.gn_part != nullptr ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
-  auto fits = [&](int bm, int bn) {
-    return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && nb * ((hw + bm - 1) / bm) * (p.N / bn) <= 256;
-  };
+  auto tiles_of = [&](int bm, int bn) { return nb * ((hw + bm - 1) / bm) * (p.N / bn); };
+  auto fits = [&](int bm, int bn) { return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && tiles_of(bm, bn) <= 256; };
+  auto pieces_of = [&](int size) { return (long)((p.M + size - 1) / size) * (((p.r_used > 0 ? p.r_used : p.R) + size - 1) / size) * (p.ldt / p.R); };
   if (p.geglu) {   // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
     if (order != 0 || p.st_part != nullptr || p.res != nullptr) return -1;
     return fits(64, 320) ? (hw + 63) / 64 * (p.N / 320) > 128 ? 7 : -1 : fits(128, 320) ? 8 : -1;
@@ -852,13 +852,15 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
     auto of = [&](const Tile* t, int n, int width) {
       for (; n > 0; ++t, --n) {
         if (!fits(t->bm, t->bn) || (stats && t->bn != width)) continue;
-        if (LoraGemmParams q = p; piece == 0 || shrink_beside(q, t->form) == piece) return t->form;
+        if (piece == 0) return t->form;
+        if (tiles_of(t->bm, t->bn) + pieces_of(piece) > 256) continue;      // (a part of what shrink_beside asks, and much cheaper)
+        if (LoraGemmParams q = p; shrink_beside(q, t->form) == piece) return t->form;
       }
       return -1;
     };
     return order == 0 ? of(tiles0, 7, 128) : of(tiles4, 5, 160);
   };
-  if (adapters) {
+  if (adapters && p.R > 0) {
     if (const int f = first(16); f >= 0) return f;
     if (p.K >= 1280)
       if (const int f = first(32); f >= 0) return f;
