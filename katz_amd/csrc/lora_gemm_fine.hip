@@ -840,7 +840,11 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   auto pieces_of = [&](int size) { return (long)((p.M + size - 1) / size) * (((p.r_used > 0 ? p.r_used : p.R) + size - 1) / size) * (p.ldt / p.R); };
   if (p.geglu) {   // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
     if (order != 0 || p.st_part != nullptr || p.res != nullptr) return -1;
-    return fits(64, 320) ? (hw + 63) / 64 * (p.N / 320) > 128 ? 7 : -1 : fits(128, 320) ? 8 : -1;
+    if (fits(64, 320)) return tiles_of(64, 320) > 128 ? 7 : -1;
+    // 128 x 320 also in several rounds that are nearly full, where the rows are ragged for 256 x 320 (1976 / 10240 / 1280, R 128 79 -> 70 us, 1800 75 -> 69;
+    // K 640 gains nothing, 3952 / 5120 / 640 44.6 against 45.6; 11 of 16 of a round full: 1300 / 10240 / 1280 59 against 66)
+    const long t = p.N % 320 == 0 ? tiles_of(128, 320) : 0, rounds = (t + 255) / 256;
+    return fits(128, 320) || (t > 256 && p.t_nsplit % 320 == 0 && p.K >= 1024 && t * 8 >= rounds * 256 * 7) ? 8 : -1;
   }
   if (order == 2) return 9;
   if (p.conv_cin > 0) return p.gn_part != nullptr ? (80 % p.gn_cg == 0 && fits(64, 80) ? 6 : 5) : fits(32, 160) ? 4 : 5;

@@ -1395,7 +1395,10 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
   if (const int form = lora_gemm_pipe_fine_form(p); form >= 0) return lora_gemm_fine_launch(p, form, stream);
   if (plain_ok(p)) {
     const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-    if (tiles >= 480 && p.K >= 1024 && !p.geglu) return deep_stage_ok(p) ? launch_pcfg<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream) : launch_pcfg<PCfg<256, 128, 4, 2, 0, 4>>(p, stream);
+    // (between one and two rounds of 128x128 tiles one of 256x128, us with T given, R 128: M 1536 / N 3840 / K 1280 30.4 -> 25.1, 1800 33.3 -> 24.7,
+    // 5120 / 1280 / 1280 28.9 -> 23.5, 5120 / 1280 / 5120 88 -> 70, 3952 / 1920 / 640 21.2 -> 16.7, 3000 / 1920 / 640 17.3 -> 13.9)
+    const bool one_round = tiles > 256 && (long)((p.M + 255) / 256) * ((p.N + 127) / 128) <= 256;
+    if (((tiles >= 480 && p.K >= 1024) || (one_round && p.K >= 640)) && !p.geglu) return deep_stage_ok(p) ? launch_pcfg<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream) : launch_pcfg<PCfg<256, 128, 4, 2, 0, 4>>(p, stream);
     if (tiles <= 256 && deep_stage_ok(p)) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
   }
   return launch_prank<128, 128, 2, 2, 4>(p, stream);

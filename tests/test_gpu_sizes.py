@@ -378,6 +378,24 @@ def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("M,N,K,split,geglu", [(1976, 10240, 1280, False, True), (1793, 10240, 1024, False, True), (3952, 1920, 640, True, False), (1500, 3840, 1280, True, False),
+                                               (2900, 1920, 640, False, False), (4993, 1280, 1280, False, False), (4100, 1920, 704, True, False)])
+def test_one_round_and_nearly_full_rounds(M, N, K, split, geglu):
+    """256 x 128 tiles between one and two rounds of 128 x 128, GEGLU on rounds of 128 x 320 tiles: the bits of the 128 x 128 kernel (code 16)."""
+    from katz_amd import ops
+
+    say("one round, nearly full rounds", M, N, K, split, geglu)
+    d = dev()
+    R = 128
+    g = torch.Generator().manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, t, bc = rnd(M, K), rnd(N, K) * 0.1, rnd(N), rnd(M, (3 if split else 1) * R), rnd(N, R) * 0.05
+    t.view(M, -1, R)[:, :, 96:] = 0
+    bc[:, 96:] = 0
+    run = lambda c: ops.lora_linear_pre(x, w, b, t, bc, geglu=geglu, tile=c, n_split=N // 3 if split else 0, r_used=96)
+    assert torch.equal(run(0), run(16))
+
+
 @pytest.mark.parametrize("B,T,S,heads", [(1, 1, 1, 1), (2, 33, 63, 3), (1, 130, 64, 2), (3, 5, 65, 2), (1, 300, 127, 1), (2, 64, 128, 2), (1, 127, 129, 3), (1, 256, 192, 2),
                                          (1, 40, 193, 2), (1, 129, 400, 1), (2, 700, 321, 20)])
 def test_attention_tiles_of_keys(B, T, S, heads):
