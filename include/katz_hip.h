@@ -238,8 +238,9 @@ int kh_lora_linear_f32(const float* x, const float* w, const float* bias, const 
 int kh_lora_linear_split_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,
                              const float* col_scale, float* t_scratch, const float* residual, float* y, int64_t M,
                              int64_t N, int64_t K, int64_t R, void* stream);
-/* The same on the bf16 matrix instruction at fp32 precision: every operand is the sum of three bf16 numbers (exactly, 24 bits), and the
- * six of the nine products that weigh more than 2^-24 are summed in fp32; results that are not finite are formed with the fp32 instruction.
+/* The same on the bf16 matrix instruction at fp32 precision: every operand is the sum of three bf16 numbers (exactly, 24 bits), and six of
+ * the nine products are summed in fp32, each of the three left out at most 2^-24 of its factors' product.  Tiles that meet an operand below
+ * 2^-103 (whose lower parts bf16 does not hold) or whose sums are not finite are formed with the fp32 instruction.
  * planes: scratch of kh_lora_linear_planes_f32_bytes(N, K, R) bytes, 16-byte aligned (the split W and B_cat; 0: not taken, K of 2^22 or
  * more than a GiB of scratch).  Everything else as above. */
 int64_t kh_lora_linear_planes_f32_bytes(int64_t N, int64_t K, int64_t R);

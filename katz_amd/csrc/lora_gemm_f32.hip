@@ -3,16 +3,18 @@
 // The reference's LoRA linear (diffusers-hf/src/diffusers/models/lora.py:222-232, :451-457) in full precision.
 //
 // The fp32 matrix instruction gives 256 FLOP per clock and CU, bf16's sixteen times that.  So every operand is split into three bf16 numbers
-// that add up to it exactly (24 bits = 8 + 8 + 8), and the six of their nine products that can weigh more than 2^-24 of the whole are
-// summed in fp32 by the bf16 instruction: 2.7 times the fp32 rate.  The sums of 32 columns are formed apart and added to the running sum
-// with rounding (the matrix instruction truncates), so the error is below that of the fp32 instruction: against 64 bits 1.1e-7 instead
-// of 4.7e-7 at K 640, 2.6e-7 instead of 13e-7 at K 5120 (2-norm, normal inputs).
+// that add up to it exactly (24 bits = 8 + 8 + 8), and six of their nine products are summed in fp32 by the bf16 instruction, all but the three that
+// are at most 2^-24 of their factors' product each (x: lower parts of 2^-7 and 2^-16, W: 2^-8 and 2^-17): 2.7 times the fp32 rate.  The sums of 32
+// columns are formed apart and added to the running sum with rounding (the matrix instruction truncates), so the error is below that of the fp32
+// instruction: against 64 bits 1.0e-7 instead of 4.5e-7 at K 640, 2.5e-7 instead of 13e-7 at K 5120 (2-norm, normal inputs).
+// Three bf16 numbers hold operands from 2^-103 on; tiles that meet smaller ones, or whose sums are not finite, are formed by the fp32 instruction
+// (M 8192, N = K 640: 110 us where every tile is).
 //
 // Two launches.  The first forms T = (x A_cat^T) * col_scale (fp32 instruction, kept in fp32) and splits W and B_cat once into planes that the
 // GEMM moves as they are; x is split by the GEMM itself (its planes would be one and a half times x's bytes, out and in again), whose rank
 // columns are extra K steps.  What bounds the GEMM then: the matrix pipe, 1920 clocks of a 128 x 160 tile's 32-column stage at the 1.7 - 2
 // GHz it leaves, beside about 1750 clocks of LDS traffic; measured 1.5 us a stage and 11 us around them.
-// M 8192, N = K 640, rank 32: 84.6 -> 50.8 us for both launches (fp32 instruction on 64 x 64 tiles before); M 64, K 5120, N 1280: 164 -> 138.
+// M 8192, N = K 640, rank 32: 84.6 -> 50.3 us for both launches (fp32 instruction on 64 x 64 tiles before).
 #include "kh_common.h"
 
 namespace {
@@ -50,7 +52,7 @@ __device__ __forceinline__ void vm_wait() {    // vmcnt = [15:14|3:0]
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-// a = hi + mid + lo exactly: hi the upper 16 bits of a, mid = bf16(a - hi), lo = a - hi - mid (8 bits are left of the 24).  Four at a time.
+// a = hi + mid + lo exactly, 8 bits of a's 24 each.  x: hi is the upper half of a (|mid| <= 2^-7 |a|, |lo| <= 2^-16 |a|).  Four at a time.
 __device__ __forceinline__ void split4(const f32x4 v, u32x2& hi, u32x2& mid, u32x2& lo) {
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
@@ -64,6 +66,29 @@ __device__ __forceinline__ void split4(const f32x4 v, u32x2& hi, u32x2& mid, u32
     lo[e] = pack_bf16x2(ar - bf16_lo(m), br - bf16_hi(m));
   }
 }
+// W and B_cat, which are split once: hi is the number nearest to a (2^-8, 2^-17), so that no product left out exceeds 2^-24 of its factors'
+__device__ __forceinline__ void split4_nearest(const f32x4 v, u32x2& hi, u32x2& mid, u32x2& lo) {
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float a = v[2 * e], b = v[2 * e + 1];
+    hi[e] = pack_bf16x2(a, b);
+    const float ar = a - bf16_lo(hi[e]), br = b - bf16_hi(hi[e]);
+    mid[e] = pack_bf16x2(ar, br);
+    lo[e] = pack_bf16x2(ar - bf16_lo(mid[e]), br - bf16_hi(mid[e]));
+  }
+}
+
+// the smallest operand so far that is not zero: its bits shifted left by one, less one
+__device__ __forceinline__ void track_least(const f32x4 v, uint32_t& least) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t t = (__float_as_uint(v[e]) << 1) - 1u;
+    least = least < t ? least : t;
+  }
+}
+// The three planes hold a number exactly where bf16 reaches down to its last bit, and as normal numbers from 2^-103 on.  Smaller ones would lose
+// their lower planes (rows of 2^-118 came out 9e-6 off, of 2^-122 1.5e-4), so the tiles that meet them are formed by the fp32 instruction.
+__device__ __forceinline__ bool too_small(uint32_t least) { return least < (24u << 24) - 1u; }
 
 // W and B_cat as the GEMM's W operand: per stage of 32 K columns (those of W, then those of B_cat, zeros behind the last) and group of 16 rows
 // three blocks of 1 KB, the planes hi, mid and lo, in the order in which the 64 lanes of a wave hold a matrix operand (lane 16 g + r: columns
@@ -77,8 +102,12 @@ __device__ __forceinline__ void split_w_block(const F32Params& p, int block, int
   const f32x4 v0 = in && k < len ? *reinterpret_cast<const f32x4*>(src) : f32x4{0, 0, 0, 0};
   const f32x4 v1 = in && k + 4 < len ? *reinterpret_cast<const f32x4*>(src + 4) : f32x4{0, 0, 0, 0};
   u32x2 h[2], m[2], l[2];
-  split4(v0, h[0], m[0], l[0]);
-  split4(v1, h[1], m[1], l[1]);
+  uint32_t least = 0xffffffffu;
+  track_least(v0, least);
+  track_least(v1, least);
+  split4_nearest(v0, h[0], m[0], l[0]);
+  split4_nearest(v1, h[1], m[1], l[1]);
+  if (too_small(least)) h[0][0] = 0x7fc07fc0u;             // (NaN: no sum of this row of W will be finite)
   char* dst = const_cast<char*>(reinterpret_cast<const char*>(p.planes)) + (size_t)block * 3072 + lane * 16;
   *reinterpret_cast<u32x4*>(dst) = u32x4{h[0][0], h[0][1], h[1][0], h[1][1]};
   *reinterpret_cast<u32x4*>(dst + 1024) = u32x4{m[0][0], m[0][1], m[1][0], m[1][1]};
@@ -89,7 +118,7 @@ __device__ __forceinline__ void split_w_block(const F32Params& p, int block, int
 template <int WM_, int WN_, int TM_>
 struct GCfg {
   static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = 5, NT = WM * WN * 64, BM = WM * TM * 16, BN = WN * 80;
-  static constexpr int PLANE = BM * FK * 2, XST = 3 * PLANE, WST = BN / 16 * 3072, NSW = 3, WOFF = 2 * XST, LDS = WOFF + NSW * WST;
+  static constexpr int PLANE = BM * FK * 2, XST = 3 * PLANE, WST = BN / 16 * 3072, NSW = 3, WOFF = 2 * XST, FLAG = WOFF + NSW * WST, LDS = FLAG + 16;   // FLAG: x has an operand too small for its planes
   static constexpr int PI = BM * 8 / NT;                                  // pieces of four columns of x a thread has of a stage
   static constexpr int WB = BN / 16 * 3, DU = (WB + WM * WN - 1) / (WM * WN);   // blocks of W: of a stage, of a wave
   static constexpr int AHEAD = 3;                                         // stages of x on their way from memory
@@ -118,6 +147,7 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
   const int c4 = (tid & 7) * 4;
   const rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.x + (size_t)m0 * p.K), 0, 0x7fffffff, 0x00020000);
   const rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.R > 0 ? p.t + (size_t)m0 * p.R : p.x), 0, 0x7fffffff, 0x00020000);
+  uint32_t least = 0xffffffffu;
   uint32_t offk[C::PI], offr[C::PI];
   int to[C::PI];
 #pragma unroll
@@ -157,7 +187,7 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
     }
   };
 
-  // The six products whose weight is above 2^-24 of the whole, summed for the stage alone and then added: the matrix instruction cuts off
+  // The six products that can weigh more than 2^-24, summed for the stage alone and then added: the matrix instruction cuts off
   // what it adds to, which on a running sum of one sign would build up.
   f32x4 acc[TM][TN];
 #pragma unroll
@@ -210,7 +240,12 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
       if (q == 5) { read_x(0); read_w(0); }
       if (q < C::PI) store(t + 2, q, g);
     }
+    f32x4 was[C::PI];
+#pragma unroll
+    for (int q = 0; q < C::PI; ++q) was[q] = g[q];
     load(t + 2 + AHEAD, g);
+#pragma unroll
+    for (int q = 0; q < C::PI; ++q) track_least(was[q], least);       // (not in front of the loads: 64 rows, K 5120, N 1280 120 us, 125 .. 128 there)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -221,6 +256,8 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
     stage_barrier();                                         // stage t + 1 has been read, stage t + 2 is there
   };
   f32x4 g[AHEAD][C::PI], g0[C::PI];                          // (loads past the last stage: zeros)
+  int* const flag = reinterpret_cast<int*>(smem + C::FLAG);
+  if (tid == 0) *flag = 0;
   load(0, g0);
   load(1, g[1]);
   load(2, g[2]);
@@ -228,7 +265,12 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
   __builtin_amdgcn_sched_barrier(0);
   next_fetch(0); next_fetch(1);
 #pragma unroll
-  for (int q = 0; q < C::PI; ++q) { store(0, q, g0); store(1, q, g[1]); }
+  for (int q = 0; q < C::PI; ++q) {
+    store(0, q, g0);
+    store(1, q, g[1]);
+    track_least(g0[q], least);
+    track_least(g[1][q], least);
+  }
   __builtin_amdgcn_sched_barrier(0);
   load(4, g[1]);
   __builtin_amdgcn_sched_barrier(0);
@@ -248,10 +290,12 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
     }
   }
   vm_wait<0>();                                              // (no load into LDS outlives the wave)
+  if (too_small(least)) *flag = 1;
+  stage_barrier();
 
-  // A result that is not finite (an input that is not, or an overflow) says nothing about what full products give: such waves form their
-  // tile again, with the fp32 instruction, straight from memory.
-  bool bad = false;
+  // A result that is not finite (an input that is not, an overflow, an operand too small for three bf16 numbers) says nothing about what full
+  // products give: such waves form their tile again, with the fp32 instruction, straight from memory.
+  bool bad = *flag != 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -266,22 +310,28 @@ __global__ __launch_bounds__(C::NT, 2) void lora_gemm_f32_split_kernel(const F32
     for (int part = 0; part < (p.R > 0 ? 2 : 1); ++part) {
       const float *xp = part ? p.t : p.x, *wp = part ? p.b_cat : p.w;
       const int len = part ? p.R : p.K;
-      for (int k = lg; k < len; k += 4) {                    // (a multiple of 4: all lanes alike)
-        float xv[TM], wv[TN];
+      for (int k0 = 0; k0 < len; k0 += 16) {                 // lane lg holds columns k0 + 4 lg .. + 3 of both operands: element e of all lanes is a step
+        const int k = k0 + 4 * lg;
+        f32x4 xv[TM], wv[TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
           const int row = m0 + wm * (TM * 16) + i * 16 + lr;
-          xv[i] = xp[(size_t)(row < p.M ? row : p.M - 1) * len + k];
+          xv[i] = k < len ? *reinterpret_cast<const f32x4*>(xp + (size_t)(row < p.M ? row : p.M - 1) * len + k) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int row = n0 + wn * 80 + j * 16 + lr;
-          wv[j] = wp[(size_t)(row < p.N ? row : p.N - 1) * len + k];
+          wv[j] = k < len ? *reinterpret_cast<const f32x4*>(wp + (size_t)(row < p.N ? row : p.N - 1) * len + k) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j], xv[i], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < TN; ++j) {
+            f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[j][e], xv[i][e], c, 0, 0, 0);
+            acc[i][j] += c;
+          }
       }
     }
   }

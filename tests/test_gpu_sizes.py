@@ -39,8 +39,8 @@ def test_lora_linear_f32_matrix_kernel(M, N, K, R):
 def test_lora_linear_f32_on_bf16_planes(M, N, K, R):
     """kh_lora_linear_planes_f32 on each of its tiles, ragged in every dimension, against 64 bits.
 
-    Bound, elementwise and relative to the sum of the magnitudes of the summands: the three products left out, each below 2^-23 of its
-    factors' product; seven truncations of 2^-23 in a stage's sum of its own; one rounding of 2^-24 per stage of 32 columns and per term
+    Bound, elementwise and relative to the sum of the magnitudes of the summands: the three products left out, each at most 2^-24 of its
+    factors' product (2^-23 is allowed for); seven truncations of 2^-23 in a stage's sum of its own; one rounding of 2^-24 per stage of 32 columns and per term
     behind them; the same once more for T."""
     from katz_amd import _lib, ops
 
@@ -57,6 +57,51 @@ def test_lora_linear_f32_on_bf16_planes(M, N, K, R):
         ref += 1.5 * (f(x) @ f(A).T) @ f(B).T
         mag += 1.5 * (f(x).abs() @ f(A).abs().T) @ f(B).abs().T
     assert ((f(y) - ref).abs() <= (2 * (3 + 7) + K / 32 + 4) * 2.0 ** -23 * mag).all()
+
+
+@pytest.mark.parametrize("where,e", [("x", -108), ("x", -118), ("w", -122), ("x", -126), ("b", -119), ("one", -122)])
+def test_lora_linear_f32_of_small_operands(where, e):
+    """Operands whose lower bf16 planes would be subnormal or vanish keep their 24 bits: all of x, W or B_cat at 2^e, or one column of x at 2^e that
+    meets weights of 2^100, among others of ordinary size.  The bound of test_lora_linear_f32_on_bf16_planes with the sixteen truncations of the
+    fp32 instruction in place of its seven, and the place of the last subnormal bit (2^-149) per summand."""
+    from katz_amd import ops
+
+    say("lora_linear_f32, small operands", where, e)
+    d, g = dev(), torch.Generator(device="cuda").manual_seed(-e)
+    M, N, K, R = 200, 240, 128, 32
+    rn = lambda *s, std=1.0: torch.randn(*s, generator=g, device=d) * std
+    x, w, A, B, sc = rn(M, K), rn(N, K), rn(R, K, std=0.1), rn(N, R), torch.ones(R, device=d)
+    small = lambda t: (t.double() * 2.0 ** e).float()
+    if where == "x":
+        x = small(x)
+    elif where == "w":
+        w, B = small(w), small(B)
+    elif where == "b":
+        w.zero_()
+        B = small(B)
+    else:
+        small_one = small(x[77:79, 5])
+        x *= 2.0 ** -24
+        x[:, 5] = 0
+        x[77:79, 5], w[:, 5] = small_one, w[:, 5] * 2.0 ** 100
+    y = ops.lora_linear(x, w, None, A, B, sc)
+    f = lambda t: t.double()
+    ref, mag = f(x) @ f(w).T + (f(x) @ f(A).T) @ f(B).T, f(x).abs() @ f(w).abs().T + (f(x).abs() @ f(A).abs().T) @ f(B).abs().T
+    assert ((f(y) - ref).abs() <= (2 * (3 + 16) + K / 32 + 4) * 2.0 ** -23 * mag + (K + R) * 2.0 ** -149).all()
+    assert (f(y) - ref).norm() <= 1e-6 * ref.norm()      # (4e-7 where the fp32 instruction forms the tile)
+
+
+def test_lora_linear_f32_products_left_out():
+    """Single products of numbers whose planes weigh most: what is left out is at most 2^-23 of the product, the last addition cuts off as much again."""
+    from katz_amd import ops
+
+    say("lora_linear_f32, products left out")
+    d, g = dev(), torch.Generator(device="cuda").manual_seed(8)
+    col = torch.cat([1 + 2.0 ** -7 * (1 - 2.0 ** -7 * torch.rand(320, generator=g, device=d)), 1 + torch.rand(320, generator=g, device=d)])
+    x, w = torch.zeros(640, 4, device=d), torch.zeros(640, 4, device=d)
+    x[:, 1], w[:, 1] = col, col.flip(0)
+    y, ref = ops.lora_linear(x, w).double(), x.double() @ w.double().T
+    assert ((y - ref).abs() <= 2.0 ** -22 * ref).all(), ((y - ref).abs() / ref).max()
 
 
 def test_lora_linear_f32_not_finite():
