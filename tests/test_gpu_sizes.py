@@ -20,10 +20,10 @@ def say(*a):
 
 @pytest.mark.parametrize("M,N,K,R", [(1, 1, 4, 0), (64, 64, 32, 32), (65, 63, 36, 4), (31, 130, 100, 36), (200, 70, 644, 128), (129, 640, 640, 32)])
 def test_lora_linear_f32_matrix_kernel(M, N, K, R):
-    """kh_lora_linear_split_f32: ragged tiles in every dimension, column counts that are no multiple of 4, all K remainders."""
+    """lora_linear in fp32: ragged tiles in every dimension, column counts that are no multiple of 4, all K remainders."""
     from katz_amd import ops
 
-    say("lora_linear_split_f32", M, N, K, R)
+    say("lora_linear, fp32", M, N, K, R)
     g = torch.Generator().manual_seed(M + N)
     x, w, b, res = (torch.randn(*s, generator=g) for s in ((M, K), (N, K), (N,), (M, N)))
     A, Bm = (torch.randn(R, K, generator=g) * 0.1, torch.randn(N, R, generator=g) * 0.1) if R else (None, None)
@@ -33,6 +33,36 @@ def test_lora_linear_f32_matrix_kernel(M, N, K, R):
     torch.cuda.synchronize()
     ref = O.lora_linear(x.double(), w.double(), b.double(), [(A.double(), Bm.double(), 1.5)] if R else [], res.double()).float()
     assert_close_rel(y, ref, 1e-5, "fp32 linear")
+
+
+@pytest.mark.parametrize("M,N,K,R", [(1, 1, 4, 0), (64, 64, 32, 32), (65, 63, 36, 4), (31, 130, 100, 36), (200, 70, 644, 128), (300, 1280, 640, 32), (129, 65, 64, 0)])
+def test_lora_linear_split_f32(M, N, K, R):
+    """kh_lora_linear_split_f32 (the fp32 instruction, no planes: the shrink without workgroups that split) at ragged tiles in every dimension, column
+    counts that are no multiple of 4 and all K remainders, behind a T and in front of a guard that it must not touch, against 64 bits.
+
+    Bound, elementwise and relative to the sum of the magnitudes of the summands: a truncation of 2^-23 for every two columns of K and R
+    (the matrix instruction adds two), one rounding per term behind them; the same once more for T."""
+    from katz_amd import _lib, ops
+
+    say("kh_lora_linear_split_f32", M, N, K, R)
+    lib, d, g = _lib.load(), dev(), torch.Generator(device="cuda").manual_seed(M + N + K)
+    rn = lambda *s, std=1.0: torch.randn(*s, generator=g, device=d) * std
+    x, w, b, res = rn(M, K), rn(N, K, std=K ** -0.5), rn(N), rn(M, N)
+    A, B, sc = (rn(R, K, std=0.1), rn(N, R, std=0.1), torch.full((R,), 1.5, device=d)) if R else (None, None, None)
+    t, y = torch.full((M * R + 32,), 7.0, device=d), torch.full((M * N + 32,), 7.0, device=d)
+    p = lambda z: None if z is None else z.data_ptr()
+    rc = lib.kh_lora_linear_split_f32(p(x), p(w), p(b), p(A), p(B), p(sc), p(t) if R else None, p(res), p(y), M, N, K, R, ops._stream())
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert (t[M * R:] == 7).all() and (y[M * N:] == 7).all()
+    f = lambda z: z.double()
+    ref, mag = f(x) @ f(w).T + f(b) + f(res), f(x).abs() @ f(w).abs().T + f(b).abs() + f(res).abs()
+    if R:
+        want = 1.5 * f(x) @ f(A).T
+        assert ((f(t[:M * R].view(M, R)) - want).abs() <= (K / 2 + 10) * 2.0 ** -23 * 1.5 * (f(x).abs() @ f(A).abs().T)).all()
+        ref += want @ f(B).T
+        mag += 1.5 * (f(x).abs() @ f(A).abs().T) @ f(B).abs().T
+    assert ((f(y[:M * N].view(M, N)) - ref).abs() <= (K + R + 14) * 2.0 ** -23 * mag).all()
 
 
 @pytest.mark.parametrize("M,N,K,R", [(1, 5, 4, 4), (64, 80, 32, 0), (65, 81, 36, 32), (300, 1280, 100, 36), (1300, 1284, 68, 4), (8200, 640, 640, 32)], ids=str)
