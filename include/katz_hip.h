@@ -244,6 +244,8 @@ int kh_lora_linear_split_f32(const float* x, const float* w, const float* bias, 
  * planes: scratch of kh_lora_linear_planes_f32_bytes(N, K, R) bytes, 16-byte aligned (the split W and B_cat; 0: not taken, K of 2^22 or
  * more than a GiB of scratch).  Everything else as above. */
 int64_t kh_lora_linear_planes_f32_bytes(int64_t N, int64_t K, int64_t R);
+/* 1 where these planes pay for their scratch and passes over W, 0 where kh_lora_linear_split_f32 is the faster (few rows on many columns). */
+int kh_lora_linear_planes_f32_pays(int64_t M, int64_t N, int64_t K, int64_t R);
 int kh_lora_linear_planes_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,
                               const float* col_scale, float* t_scratch, void* planes, const float* residual, float* y, int64_t M,
                               int64_t N, int64_t K, int64_t R, void* stream);

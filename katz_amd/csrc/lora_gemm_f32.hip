@@ -448,7 +448,10 @@ __global__ __launch_bounds__(512) void lora_prepare_f32_kernel(const F32Params p
 #endif
 }
 
-// The same without scratch for the planes: both operands on the fp32 matrix instruction (64 x 64 tiles, four waves of one 32 x 32 tile).
+// The same without planes: both operands on the fp32 matrix instruction (64 x 64 tiles, four waves of one 32 x 32 tile), for few rows on many columns
+// (kh_lora_linear_planes_f32_pays) and for calls whose planes take more than a GiB.  A stage's 32 columns are summed in two chains apart from the
+// running sum, which the matrix instruction would cut off at every addition: K 640 / 1280 / 5120 4.5e-7 / 6.4e-7 / 13e-7 -> 1.2e-7 / 1.4e-7 / 2.4e-7
+// against 64 bits (planes 1.0e-7 / 1.3e-7 / 2.4e-7), for 12 % of the launch (64 x 10240 x 1280 32.2 -> 36.3 us).
 __global__ __launch_bounds__(256, 4) void lora_gemm_f32_mfma_kernel(const F32Params p) {
   __shared__ __attribute__((aligned(16))) float sm[2][2 * FB * FLD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, lh = lane >> 5;
@@ -495,10 +498,14 @@ __global__ __launch_bounds__(256, 4) void lora_gemm_f32_mfma_kernel(const F32Par
     const float* s = sm[t & 1];
     const float* sx = s + (wm * 32 + l32) * FLD + 4 * lh;
     const float* sw = s + (FB + wn * 32 + l32) * FLD + 4 * lh;
+    f32x16 c[2];                                 // the stage's own sums
+#pragma unroll
+    for (int e = 0; e < 16; ++e) c[0][e] = c[1][e] = 0.f;
 #pragma unroll
     for (int g = 0; g < FK / 8; ++g)             // W first: a lane then holds one output row and runs of four columns
-      acc = mma8(*reinterpret_cast<const f32x4*>(sw + 8 * g), *reinterpret_cast<const f32x4*>(sx + 8 * g), acc);
+      c[g % 2] = mma8(*reinterpret_cast<const f32x4*>(sw + 8 * g), *reinterpret_cast<const f32x4*>(sx + 8 * g), c[g % 2]);
     if (t + 1 < KT) store(sm[(t + 1) & 1]);      // that buffer was last read before the barrier above
+    acc += c[0] + c[1];
   }
   const int row = m0 + wm * 32 + l32;
   if (row >= p.M) return;
@@ -560,6 +567,20 @@ KH_EXPORT int64_t kh_lora_linear_planes_f32_bytes(int64_t N, int64_t K, int64_t 
   if (N <= 0 || K <= 0 || R < 0 || N > (1 << 24) || K >= (1 << 22) || R > 128) return 0;
   const int64_t bytes = ((K + FK - 1) / FK + (R + FK - 1) / FK) * ((N + 15) / 16) * 3072;
   return bytes <= ((int64_t)1 << 30) ? bytes : 0;
+}
+
+// Planes cost W three times more (read, written, read again as 6 of 4 bytes), the fp32 instruction the matrix pipe.  Estimates of both launches in us,
+// within 10 % of what was measured for 1 .. 1024 rows at 640 x 640 .. 12288 x 12288: some 6 us before and behind the loop, a pass over W at
+// 5 TB/s, 4 us where x comes in several rows of tiles, and per stage of 32 columns the time of the tile that is taken (rounds of 256 CUs).  Planes
+// give the smaller error and stay up to a tenth slower.  M / N / K, planes / fp32 instruction: 64 / 10240 / 1280 62.8 / 49.6; 192 / 5120 / 640 33.0 / 27.6;
+// 128 / 8192 / 8192 344 / 266; 256 / 12288 / 12288 1010 / 755; 256 / 10240 / 1280 78 / 87; 64 / 1280 / 5120 136 / 167; 1024 / 640 / 640 26.6 / 26.3.
+KH_EXPORT int kh_lora_linear_planes_f32_pays(int64_t M, int64_t N, int64_t K, int64_t R) {
+  if (M <= 0 || N <= 0 || K <= 0 || R < 0 || M > (1 << 24) || N > (1 << 24) || K > (1 << 24) || R > 128) return 0;
+  auto rounds = [&](int64_t bm, int64_t bn) { return (double)(((M + bm - 1) / bm * ((N + bn - 1) / bn) + 255) / 256); };
+  const double stages = (double)((K + FK - 1) / FK + (R + FK - 1) / FK), small = rounds(64, 80), mid = 1.1 * rounds(128, 80), big = 1.65 * rounds(128, 160);
+  const double tile = small == 1 ? 0.77 : small == 2 ? 1.16 : 0.25 + 0.5 * small, least = tile < mid ? tile : mid, instr = 0.2 + 0.59 * rounds(FB, FB);
+  const double planes = 6 + 2e-6 * (double)N * (double)K + (M > 64 ? 4 : 0) + stages * (least < big ? least : big);
+  return planes <= 1.1 * (5.5 + stages * (instr > 0.98 ? instr : 0.98)) ? 1 : 0;
 }
 
 KH_EXPORT int kh_lora_linear_planes_f32(const float* x, const float* w, const float* bias, const float* a_cat, const float* b_cat,

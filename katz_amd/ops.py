@@ -200,7 +200,7 @@ def lora_linear(
         if geglu:
             raise ValueError("the GEGLU epilogue exists for bf16 only")
         t = torch.empty((M, R), dtype=dt, device=x.device) if R else None
-        n_planes = lib.kh_lora_linear_planes_f32_bytes(N, K, R)
+        n_planes = lib.kh_lora_linear_planes_f32_bytes(N, K, R) if lib.kh_lora_linear_planes_f32_pays(M, N, K, R) else 0
         if n_planes:
             planes = torch.empty(n_planes, dtype=torch.uint8, device=x.device)
             rc = lib.kh_lora_linear_planes_f32(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(b_cat), _ptr(col_scale), _ptr(t),

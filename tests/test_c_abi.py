@@ -140,3 +140,20 @@ def test_a_refused_call_drops_the_pending_weight_prefetch_hint():
         for _ in range(3):                                               # ... and gone after the refused call
             assert lib.kh_set_weight_prefetch(4096, 1 << 20) == 0
         assert lib.kh_set_weight_prefetch(None, 0) == 0
+
+
+def test_planes_of_the_fp32_linear_only_where_they_pay():
+    """Few rows on many columns take the fp32 instruction: planes there cost up to two thirds more (64 x 12288 x 12288: 640 against 390 us)."""
+    from katz_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libkatz_hip.so not built")
+    pays = _lib.load().kh_lora_linear_planes_f32_pays
+    for m, n, k in ((64, 10240, 1280), (1, 8192, 8192), (192, 5120, 640), (256, 12288, 12288)):
+        assert pays(m, n, k, 32) == 0, (m, n, k)
+    for n, k in ((640, 640), (1280, 1280), (640, 2048), (1280, 2048), (640, 2560), (1280, 5120)):
+        for m in (1, 64, 65, 200, 1000, 1024, 1025, 4096, 16384):
+            assert pays(m, n, k, 32) == 1 and pays(m, n, k, 128) == 1, (m, n, k)
+    for m, n, k in ((512, 5120, 640), (256, 10240, 1280), (1024, 12288, 12288)):
+        assert pays(m, n, k, 32) == 1, (m, n, k)
+    assert pays(0, 640, 640, 0) == 0 and pays(64, 640, 640, 129) == 0 and pays(64, 1 << 25, 640, 0) == 0

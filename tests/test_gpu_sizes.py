@@ -65,6 +65,21 @@ def test_lora_linear_split_f32(M, N, K, R):
     assert ((f(y[:M * N].view(M, N)) - ref).abs() <= (K + R + 14) * 2.0 ** -23 * mag).all()
 
 
+def test_lora_linear_f32_of_few_rows_on_many_columns():
+    """lora_linear takes the form without planes where they do not pay: its bits."""
+    from katz_amd import _lib, ops
+
+    M, N, K, R = 100, 5120, 64, 32
+    say("lora_linear, fp32, few rows", M, N, K, R)
+    lib, d, g = _lib.load(), dev(), torch.Generator(device="cuda").manual_seed(3)
+    assert lib.kh_lora_linear_planes_f32_bytes(N, K, R) > 0 and lib.kh_lora_linear_planes_f32_pays(M, N, K, R) == 0
+    x, w, A, B = (torch.randn(*s, generator=g, device=d) for s in ((M, K), (N, K), (R, K), (N, R)))
+    sc, t, y = torch.full((R,), 0.5, device=d), torch.empty(M, R, device=d), torch.empty(M, N, device=d)
+    assert lib.kh_lora_linear_split_f32(x.data_ptr(), w.data_ptr(), None, A.data_ptr(), B.data_ptr(), sc.data_ptr(), t.data_ptr(), None, y.data_ptr(),
+                                        M, N, K, R, ops._stream()) == 0
+    assert torch.equal(ops.lora_linear(x, w, None, A, B, sc), y)
+
+
 @pytest.mark.parametrize("M,N,K,R", [(1, 5, 4, 4), (64, 80, 32, 0), (65, 81, 36, 32), (300, 1280, 100, 36), (1300, 1284, 68, 4), (8200, 640, 640, 32)], ids=str)
 def test_lora_linear_f32_on_bf16_planes(M, N, K, R):
     """kh_lora_linear_planes_f32 on each of its tiles, ragged in every dimension, against 64 bits.
