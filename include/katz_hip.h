@@ -99,14 +99,16 @@ int kh_lora_linear_pre_bf16(const void* x, const void* w, const void* bias, cons
  * call is then undefined).  n_split > 0: w / bias / b_cat stack N / n_split layers of n_split rows each (q, k, v of a
  * self-attention), a_cat / col_scale stack their A matrices ([N / n_split * R, K]) and t_scratch is [M, N / n_split * R],
  * as for kh_lora_linear_pre_bf16.  K % 64 == 0, R % 32 == 0, R <= 128.  flags: bit 0 GEGLU, bits 8..15: 1 = always two
- * launches, bits 16..23: r_used / 16 as above, bit 24: never the cooperative form (below).
+ * launches, bits 16..23: r_used / 16 as above, bit 24: two launches wherever one would have workgroups that wait for others of it (below).
  * Cooperative form: where the GEMM's 128x160 tiles give every CU exactly one workgroup (N = 640 at M = 8192), R = 128 and
  * 0 < r_used <= 96, no CU is idle, and EVERY workgroup first computes a 32-row x 96-column piece of its row block's
  * t_scratch, counts itself into `counters` and only then runs its tile, waiting (bounded, as above) for the four pieces
- * of its row block before the last K tiles.  No workgroup waits before its own piece is out, so one such launch always
- * completes; TWO of them running at the same time on different streams can each hold the CUs the other's not yet
- * started workgroups need, and then both only end through the bounded wait.  A caller that enqueues these calls on
- * streams that may overlap sets bit 24 on all but one of the streams.
+ * of its row block before the last K tiles.  No workgroup waits before its own piece is out.
+ * Streams: every one-launch form makes workgroups wait for others of the same launch, and one such launch always completes, beside any
+ * launches that do not wait.  TWO of them at the same time on different streams need not, whichever forms they are (cooperative, q / k / v, few
+ * rows, cross-attention): the XCDs take up workgroups independently, so one launch's waiting workgroups can fill the CUs of an XCD that the other
+ * launch's pieces have yet to start on, and the other way round on another XCD, and then both only end through the bounded wait.
+ * A caller that enqueues these calls on streams that may overlap sets bit 24 on all but one of the streams.
  * Few rows (tiles smaller than 128 x 128): likewise inside the launch where those tiles leave CUs idle, in 16 x 16 or 32 x 32
  * pieces of t_scratch and with the results of the two launches bit for bit; columns of t_scratch beyond r_used stay unwritten. */
 #define KH_SPLIT_COUNTER_INTS(M) (((M) + 127) / 128 + 1)
@@ -145,7 +147,7 @@ int kh_lora_linear_norm_bf16(const void* x, const void* w, const void* bias, con
  * the GEMM's epilogue keeps the tile in LDS, loads the S keys / values of its two heads and runs the attention there.
  * x [M,K] with M = B * T (rows of sample b: b*T .. b*T + T - 1), w [N,K], N = heads * 64; k, v: [B,S,N] views (row
  * strides ldk / ldv, sample strides bsk / bsv, in elements); o [M,N] with row stride ldo, head h at columns 64 h.
- * The projection's arguments (bias, adapters, t_scratch, counters, folded LayerNorm, flags bits 8..23) are
+ * The projection's arguments (bias, adapters, t_scratch, counters, folded LayerNorm, flags bits 8..24) are
  * kh_lora_linear_norm_bf16's, without residual, statistics, GEGLU and n_split.  M % 128 == 0, T % 128 == 0, N % 128 == 0,
  * K % 64 == 0, R % 64 == 0, R <= 128, S <= 96, at most 256 tiles of 128 x 128: kh_lora_linear_xattn_ok says whether a
  * shape is taken (1) or not (0: run the projection and kh_attention_bf16).  Against those two calls the result differs
@@ -184,6 +186,8 @@ int kh_set_weight_prefetch(const void* weights, int64_t bytes);
 /* How many kernel launches kh_lora_linear_split_bf16 makes for this shape when counters are given (1 or 2; negative:
  * KH_ERR_*).  No counterpart in the reference; for callers that account per launch (benchmarks). */
 int kh_lora_linear_split_launches(int64_t M, int64_t N, int64_t K, int64_t R, int64_t n_split, int flags);
+/* The same for kh_lora_linear_xattn_bf16 (KH_ERR_UNSUPPORTED where that refuses the shape). */
+int kh_lora_linear_xattn_launches(int64_t M, int64_t N, int64_t K, int64_t R, int64_t T, int64_t S, int flags);
 /* n_groups layers that read the SAME x in one launch (the context K/V projections of every cross-attention
  * of the UNet: 140 GEMMs of 154 rows each, which individually cannot fill the chip):
  *   y_g = x W_g^T + bias_g + t_g B_cat_g^T        g = 0 .. n_groups-1, all with the same M, N, K, R

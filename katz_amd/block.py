@@ -311,7 +311,7 @@ def run(blk, h, ctx, stats, last: bool):
     if folded:
         call.stats = stats.buf.data_ptr()
     call.B, call.T, call.S, call.last = B, T, S, int(last)
-    call.flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_coop_bit()
+    call.flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_wait_bit()
     ranges = ops.chain_hints(ready.first_key, ready.first, plan.last_key)
     if ranges is not None:
         call.hints = 1
@@ -394,7 +394,7 @@ def run_linear(l, x, residual):
     if r.R:
         t = x.new_empty((M, r.R))
         counters = ops._arena_address(x.device, (M + 127) // 128 + 1)
-        flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_coop_bit()
+        flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_wait_bit()
     lib = _lib.load()
     ranges = ops.chain_hints(r.key, r.refs, r.key)
     if ranges is not None:

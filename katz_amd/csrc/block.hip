@@ -169,7 +169,7 @@ KH_EXPORT int kh_transformer_block_bf16(const KhBlockDesc* desc, const KhBlockCa
       if (c.hints) hint(d.out2);
       KH_STEP(kh_lora_linear_xattn_bf16(n, q.w, ln ? nullptr : q.bias, q.a_cat, q.col_scale, q.b_cat, q.R ? ws + w.t : nullptr, r.take(q, M), ln,
                                         ln ? q.c1 : nullptr, ln ? q.c2 : nullptr, ln ? q.ca1 : nullptr, ln ? q.ca2 : nullptr, ln ? (float)q.eps : 0.f, k, v,
-                                        ws + w.att, M, q.N, q.K, q.R, c.T, c.S, ldk, ldv, inner, bsk, bsv, (float)d.scale2, r.flags(q) | (1 << 24), stream));
+                                        ws + w.att, M, q.N, q.K, q.R, c.T, c.S, ldk, ldv, inner, bsk, bsv, (float)d.scale2, r.flags(q), stream));
     } else {
       KH_STEP(r.linear(q, n, nullptr, ws + w.wide, M, ln, nullptr, &d.out2));
       KH_STEP(kh_attention_bf16(ws + w.wide, k, v, ws + w.att, c.B, d.heads, c.T, c.S, 64, inner, ldk, ldv, inner, inner * c.T, bsk, bsv, inner * c.T,

@@ -81,8 +81,8 @@ struct LoraGemmParams {
   uint32_t pf_lines[3] = {0, 0, 0};
 };
 
-// bit 24 of the `flags` of kh_lora_linear_split_bf16 / _norm_bf16: do not use the cooperative in-launch shrink (see include/katz_hip.h)
-constexpr int KH_FLAG_NO_COOP = 1 << 24;
+// bit 24 of the `flags` of kh_lora_linear_split_bf16 / _norm_bf16 / _xattn_bf16: no launch whose workgroups wait for others of it (see include/katz_hip.h)
+constexpr int KH_FLAG_NO_WAIT = 1 << 24;
 
 // Weight prefetch of a launch with its own shrink: by the idle waves of the shrink workgroups when the first range is short
 __host__ __device__ inline bool il_prefetch_by_idle_waves(const LoraGemmParams& p) { return p.pf_lines[0] <= ((8u << 20) >> 7); }

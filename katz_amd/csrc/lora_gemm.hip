@@ -586,15 +586,14 @@ static LoraGemmParams split_params(const void* x, const void* w, const void* bia
 KH_EXPORT int kh_lora_linear_split_launches(int64_t M, int64_t N, int64_t K, int64_t R, int64_t n_split, int flags) {
   if (M <= 0 || N <= 0 || K <= 0 || R <= 0 || M > (1 << 24) || N > (1 << 24) || K > (1 << 24)) return KH_ERR_INVALID_ARG;
   if (n_split < 0 || (n_split > 0 && N % n_split != 0)) return KH_ERR_INVALID_ARG;
-  if (((flags >> 8) & 0xff) != 0) return 2;
+  if (((flags >> 8) & 0xff) != 0 || (flags & KH_FLAG_NO_WAIT) != 0) return 2;
   static int32_t dummy_counter;                  // the rule only asks whether counters were given
   static const char dummy = 0;
   LoraGemmParams p = split_params(&dummy, &dummy, nullptr, &dummy, reinterpret_cast<const float*>(&dummy), &dummy,
                                   const_cast<char*>(&dummy), &dummy_counter, nullptr, const_cast<char*>(&dummy), M, N, K, R,
                                   n_split, (flags & 1) != 0);
   p.r_used = ((flags >> 16) & 0xff) * 16;
-  if ((flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p)) return 1;
-  return lora_gemm_pipe_il_ok(p) || lora_gemm_fine_il_ok(p) ? 1 : 2;
+  return lora_gemm_fine_coop_ok(p) || lora_gemm_pipe_il_ok(p) || lora_gemm_fine_il_ok(p) ? 1 : 2;
 }
 
 KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void* bias, const void* a_cat,
@@ -619,7 +618,7 @@ KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void
     LoraGemmParams p = split_params(x, w, bias, a_cat, col_scale, b_cat, t_scratch, counters, residual, y, M, N, K, R, n_split, geglu);
     p.r_used = ((flags >> 16) & 0xff) * 16;
     kh_take_weight_prefetch(p);
-    if ((flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
+    if (lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
     return lora_gemm_pipe_il_ok(p) ? lora_gemm_pipe_launch_il(p, (hipStream_t)stream) : lora_gemm_fine_launch_il(p, (hipStream_t)stream);
   }
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, nullptr, nullptr, nullptr, 0.f, (hipStream_t)stream,
@@ -667,6 +666,7 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
   p.ln_part = ln_part; p.ln_c1 = ln_c1; p.ln_c2 = ln_c2; p.ln_ca1 = ln_ca1; p.ln_ca2 = ln_ca2; p.ln_eps = ln_eps;
   p.st_part = stats_out;
   const int tile_sel = (flags >> 8) & 0xff;
+  const bool may_wait = counters != nullptr && tile_sel == 0 && (flags & KH_FLAG_NO_WAIT) == 0;
   if (xa != nullptr) {
     // the projection's result never reaches memory: its 128 x 128 tiles are 128 queries of two heads each
     if (!xa->k || !xa->v || !xa->o || xa->T <= 0 || xa->S <= 0 || M % xa->T != 0) return KH_ERR_INVALID_ARG;
@@ -683,7 +683,7 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
     if (!lora_gemm_pipe_xattn_ok(p)) return KH_ERR_UNSUPPORTED;
     kh_take_weight_prefetch(p);
     if (R == 0) return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
-    if (counters != nullptr && tile_sel == 0 && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
+    if (may_wait && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
     const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
     if (rc != KH_OK) return rc;
     p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;
@@ -694,10 +694,9 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
     p.ldt = 0; p.t_nsplit = 0; p.il_cnt = nullptr;
     return lora_gemm_pipe_launch(p, tile_sel, (hipStream_t)stream);
   }
-  if (counters != nullptr && tile_sel == 0 && (flags & KH_FLAG_NO_COOP) == 0 && lora_gemm_fine_coop_ok(p))
-    return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
-  if (counters != nullptr && tile_sel == 0 && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_il(p, (hipStream_t)stream);
-  if (counters != nullptr && tile_sel == 0 && lora_gemm_fine_il_ok(p)) return lora_gemm_fine_launch_il(p, (hipStream_t)stream);
+  if (may_wait && lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
+  if (may_wait && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_il(p, (hipStream_t)stream);
+  if (may_wait && lora_gemm_fine_il_ok(p)) return lora_gemm_fine_launch_il(p, (hipStream_t)stream);
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
   if (rc != KH_OK) return rc;
   p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;
@@ -732,6 +731,20 @@ KH_EXPORT int kh_lora_linear_xattn_ok(int64_t M, int64_t N, int64_t K, int64_t R
   if (M <= 0 || N <= 0 || K <= 0 || R < 0 || T <= 0 || S <= 0 || M > (1 << 24) || N > (1 << 24) || K > (1 << 24)) return 0;
   if (M % 128 != 0 || N % 128 != 0 || K % 64 != 0 || R % 64 != 0 || R > 128 || T % 128 != 0 || M % T != 0 || S > 96) return 0;
   return (M / 128) * (N / 128) <= 256 ? 1 : 0;
+}
+
+// See include/katz_hip.h: launches of kh_lora_linear_xattn_bf16 when counters are given.
+KH_EXPORT int kh_lora_linear_xattn_launches(int64_t M, int64_t N, int64_t K, int64_t R, int64_t T, int64_t S, int flags) {
+  if (!kh_lora_linear_xattn_ok(M, N, K, R, T, S)) return KH_ERR_UNSUPPORTED;
+  if (R == 0) return 1;
+  if (((flags >> 8) & 0xff) != 0 || (flags & KH_FLAG_NO_WAIT) != 0) return 2;
+  static int32_t dummy_counter;                  // the rule only asks whether counters were given
+  static const char dummy = 0;
+  LoraGemmParams p = split_params(&dummy, &dummy, nullptr, &dummy, reinterpret_cast<const float*>(&dummy), &dummy, const_cast<char*>(&dummy),
+                                  &dummy_counter, nullptr, nullptr, M, N, K, R, 0, false);
+  p.r_used = ((flags >> 16) & 0xff) * 16;
+  p.xa_k = reinterpret_cast<const bf16_t*>(&dummy);
+  return lora_gemm_pipe_il_ok(p) ? 1 : 2;
 }
 
 // 3x3 convolution, padding 1, NHWC, as an implicit GEMM on the pipelined kernel; see include/katz_hip.h.

@@ -236,10 +236,10 @@ def lora_shrink(x: torch.Tensor, a_cat: torch.Tensor, col_scale: torch.Tensor, o
     return out
 
 
-def _no_coop_bit() -> int:
-    """Flag bit 24 of the split / norm entry points: inside side_branch() the cooperative in-launch shrink is off.  Its
-    workgroups wait for each other, and two such launches running side by side on two streams could each hold the CUs
-    the other one's last workgroups need."""
+def _no_wait_bit() -> int:
+    """Flag bit 24 of the split / norm / xattn entry points: inside side_branch() no launch's workgroups wait for others of
+    it (the shrink is a launch of its own).  Two launches that wait, side by side on two streams, could each hold the CUs
+    that workgroups the other one waits for need."""
     return (1 << 24) if _ws_slot[0] > 0 else 0
 
 
@@ -433,7 +433,7 @@ def lora_linear_split(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
     out = torch.empty(tuple(x.shape[:-1]) + (n_out,), dtype=BF16, device=x.device)
     t = torch.empty((M, RT), dtype=BF16, device=x.device)
     cnt = _split_counters(x.device, M)
-    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16) | _no_coop_bit()
+    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16) | _no_wait_bit()
     if CALL_LOG is not None:   # one entry per kernel launch
         if lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2:
             CALL_LOG.append(("lora_shrink", M, K, RT))
@@ -511,7 +511,7 @@ def lora_linear_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     if R:
         t = torch.empty((M, RT), dtype=BF16, device=x.device)
         cnt = _split_counters(x.device, M)
-    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | _no_coop_bit()
+    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | _no_wait_bit()
     if CALL_LOG is not None:   # one entry per kernel launch
         if R and lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2:
             CALL_LOG.append(("lora_shrink", M, K, RT))
@@ -580,10 +580,9 @@ def lora_linear_xattn(x: torch.Tensor, weight: torch.Tensor, k: torch.Tensor, v:
     if R:
         t = torch.empty((M, R), dtype=BF16, device=x.device)
         cnt = _split_counters(x.device, M)
-    # bit 24: the cooperative shrink belongs to another kernel family (the launch count below must not count on it)
-    flags = ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | (1 << 24)
+    flags = ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | _no_wait_bit()
     if CALL_LOG is not None:   # one entry per kernel launch
-        if R and lib.kh_lora_linear_split_launches(M, N, K, R, 0, flags) == 2:
+        if R and lib.kh_lora_linear_xattn_launches(M, N, K, R, T, S, flags) == 2:
             CALL_LOG.append(("lora_shrink", M, K, R))
         CALL_LOG.append(("lora_linear_xattn", M, N, K, R, heads, T, S))
     _weight_prefetch_hint(weight, a_cat, b_cat)
@@ -848,8 +847,8 @@ _ws_slot: list = [0]
 
 @contextlib.contextmanager
 def side_branch():
-    """Ops called inside this context take their shared scratch (the GroupNorm partial sums) from a second buffer, so
-    that they may run on another stream beside ops called outside it."""
+    """Ops called inside this context take their shared scratch (the GroupNorm partial sums) from a second buffer and make
+    no launch whose workgroups wait for others of it, so that they may run on another stream beside ops called outside it."""
     _ws_slot[0] += 1
     try:
         yield

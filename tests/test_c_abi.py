@@ -157,3 +157,32 @@ def test_planes_of_the_fp32_linear_only_where_they_pay():
     for m, n, k in ((512, 5120, 640), (256, 10240, 1280), (1024, 12288, 12288)):
         assert pays(m, n, k, 32) == 1, (m, n, k)
     assert pays(0, 640, 640, 0) == 0 and pays(64, 640, 640, 129) == 0 and pays(64, 1 << 25, 640, 0) == 0
+
+
+@pytest.mark.parametrize("M,N,K,R,r_used,n_split", [(154, 1280, 2048, 128, 96, 0), (512, 1280, 1280, 32, 32, 0), (300, 1920, 640, 32, 16, 640), (2048, 1280, 1280, 64, 64, 0),
+                                                    (2048, 3840, 1280, 128, 96, 1280), (8192, 640, 640, 128, 96, 0)])
+def test_bit_24_selects_two_launches_in_every_form(M, N, K, R, r_used, n_split):
+    """A second stream's launches must not wait inside themselves: few rows, 128 x 128 tiles, q / k / v, cooperative."""
+    from katz_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libkatz_hip.so not built")
+    launches = _lib.load().kh_lora_linear_split_launches
+    flags = r_used // 16 << 16
+    assert launches(M, N, K, R, n_split, flags) == 1
+    assert launches(M, N, K, R, n_split, flags | 1 << 24) == 2
+    assert launches(M, N, K, R, n_split, flags | 1 << 8) == 2
+
+
+def test_launches_of_the_query_projection_with_its_attention():
+    from katz_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libkatz_hip.so not built")
+    launches = _lib.load().kh_lora_linear_xattn_launches
+    assert launches(2048, 1280, 1280, 64, 1024, 77, 0) == 1
+    assert launches(2048, 1280, 1280, 64, 1024, 77, 1 << 24) == 2
+    assert launches(2048, 1280, 1280, 64, 1024, 77, 1 << 8) == 2
+    assert launches(512, 1280, 1280, 64, 256, 77, 0) == 2          # its 128 x 128 tiles bring no shrink along below 1024 rows
+    assert launches(512, 1280, 1280, 0, 256, 77, 0) == 1
+    assert launches(2048, 1280, 1280, 64, 1000, 77, 0) == -2       # T % 128

@@ -685,3 +685,38 @@ def test_shrink_of_few_rows_gives_the_bits_of_many(M, K):
     a3, cs3 = torch.cat([a, a * 2, a * 3]), torch.cat([cs] * 3)
     run = lambda r: ops.lora_linear_split(x[:M], w, None, a3, cs3, b, n_split=128, two_launches=True, r_used=r)
     assert torch.equal(run(16), run(0))
+
+
+@pytest.mark.parametrize("M,N,K,R,r_used,n_split,entry", [(154, 1280, 2048, 128, 96, 0, "split"), (154, 1280, 2048, 128, 96, 0, "norm"), (2048, 1280, 1280, 64, 64, 0, "norm"),
+                                                          (2048, 3840, 1280, 128, 96, 1280, "split"), (8192, 640, 640, 128, 96, 0, "norm"), (2048, 1280, 1280, 64, 64, 0, "xattn")])
+def test_bit_24_leaves_the_counters_alone(M, N, K, R, r_used, n_split, entry):
+    """With bit 24 of the flags no workgroup counts itself in or waits: counters stay as they are, and the bits are those of two launches."""
+    from katz_amd import _lib, ops
+
+    say("bit 24", M, N, K, R, r_used, n_split, entry)
+    lib, d, g = _lib.load(), dev(), torch.Generator().manual_seed(M + N)
+    parts = N // n_split if n_split else 1
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(d, BF)
+    x, w, A, B = rnd(M, K), rnd(N, K, std=0.03), rnd(parts, R, K, std=0.05), rnd(N, R, std=0.05)
+    A[:, r_used:], B[:, r_used:] = 0, 0
+    s, kv = torch.rand(parts * R, generator=g).to(d), rnd(2, 2, 77, N)
+    p = lambda t: t.data_ptr()
+
+    def run(flags):
+        t, y = torch.zeros(M, parts * R, dtype=BF, device=d), torch.zeros(M, N, dtype=BF, device=d)
+        cnt = torch.full(((M + 127) // 128 + 1,), 5, dtype=torch.int32, device=d)
+        flags |= r_used // 16 << 16
+        if entry == "split":
+            rc = lib.kh_lora_linear_split_bf16(p(x), p(w), None, p(A), p(s), p(B), p(t), p(cnt), None, p(y), M, N, K, R, n_split, flags, ops._stream())
+        elif entry == "norm":
+            rc = lib.kh_lora_linear_norm_bf16(p(x), p(w), None, p(A), p(s), p(B), p(t), p(cnt), None, p(y), None, None, None, None, None, 0.0, None, M, N, K, R,
+                                              n_split, flags, ops._stream())
+        else:
+            rc = lib.kh_lora_linear_xattn_bf16(p(x), p(w), None, p(A), p(s), p(B), p(t), p(cnt), None, None, None, None, None, 0.0, p(kv[0]), p(kv[1]), p(y), M, N, K, R,
+                                               M // 2, 77, N, N, N, 77 * N, 77 * N, 0.125, flags, ops._stream())
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert (cnt == 5).all()
+        return y
+
+    assert torch.equal(run(1 << 24), run(1 << 8))
