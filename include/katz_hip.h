@@ -33,6 +33,8 @@ extern "C" {
 
 /* ABI version, bumped on any signature change. */
 int kh_version(void);
+/* The stream capture that `stream` is part of (*id is a HOST pointer; 0: none). */
+int kh_stream_capture_id(void* stream, uint64_t* id);
 /* Static string for a KH_ERR_* code or a hipError_t (host pointer, never NULL). */
 const char* kh_error_string(int code);
 
@@ -435,7 +437,7 @@ int kh_conv_out_cfg_euler_bf16(const void* x, const void* w, const void* bias, c
  * sample strides bsk / bsv (elements).  stats: as kh_lora_linear_norm_bf16 (folded only), valid for x on entry; `last`: not
  * written for y.  flags: bits 8 (shrink as a launch of its own) and 24 of the linears' flags.  hints: issue
  * kh_set_weight_prefetch inside the chain; tail_hint: up to three (address, bytes) for the launch after the block.
- * workspace / counters: at least what kh_transformer_block_needs reports; counters zero when the call is enqueued. */
+ * workspace / counters: at least what kh_transformer_block_needs reports; counters zero when the call is enqueued, NULL where bit 8 or 24 is set. */
 typedef struct {
   const void *w, *bias, *a_cat, *b_cat;
   const float *col_scale, *c1, *c2, *ca1, *ca2;

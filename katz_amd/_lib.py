@@ -17,6 +17,7 @@ _I = c_int64
 # name -> (restype, argtypes); mirrors include/katz_hip.h one to one
 SIGNATURES = {
     "kh_version": (c_int, []),
+    "kh_stream_capture_id": (c_int, [_P, _P]),
     "kh_error_string": (c_char_p, [c_int]),
     "kh_profile_begin": (c_int, []),
     "kh_profile_end": (c_int, [_P, _P, c_int]),

@@ -306,18 +306,24 @@ def run(blk, h, ctx, stats, last: bool):
     y = torch.empty_like(h)
     ws = h.new_empty((nbytes,), dtype=torch.uint8)
     call.x, call.y, call.workspace, call.workspace_bytes = h.data_ptr(), y.data_ptr(), ws.data_ptr(), nbytes
-    if ints:
-        call.counters, call.counter_ints = ops._arena_address(h.device, ints), ints
     if folded:
         call.stats = stats.buf.data_ptr()
     call.B, call.T, call.S, call.last = B, T, S, int(last)
-    call.flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_wait_bit()
     ranges = ops.chain_hints(ready.first_key, ready.first, plan.last_key)
     if ranges is not None:
         call.hints = 1
         for i, r in enumerate(ranges):
             call.tail_hint[2 * i], call.tail_hint[2 * i + 1] = r
-    _lib.check(_lib.load().kh_transformer_block_bf16(ready.at, ctypes.addressof(call), ops._stream()), "kh_transformer_block_bf16")
+    lib, counters, call.flags = _lib.load(), 0, (1 << 8) if layers.LORA_SHRINK == "separate" else 0
+    if ints and not call.flags:
+        counters = ops.counters_begin(h.device, ints)
+        call.counters, call.counter_ints, call.flags = counters, ints, 0 if counters else 1 << 24
+    try:
+        rc = lib.kh_transformer_block_bf16(ready.at, ctypes.addressof(call), ops._stream())
+    finally:
+        if counters:
+            ops.counters_end(h.device)
+    _lib.check(rc, "kh_transformer_block_bf16")
     return y
 
 
@@ -347,7 +353,7 @@ class _LinearReady:
             d.R, d.r_used = p.R, p.r_used
         self.keep = (w, b, b_cat, None if p is None else p.col_scale)
         self.refs = tuple(None if t is None else weakref.ref(t) for t in (w, self.a_cat, b_cat))
-        self.at, self.key = ctypes.addressof(d), int(d.w)
+        self.at, self.key, self.device = ctypes.addressof(d), int(d.w), w.device
         self.N, self.K, self.R, self.width = d.N, d.K, d.R, d.N // 2 if l.geglu else d.N
 
     def state(self):
@@ -389,19 +395,21 @@ def run_linear(l, x, residual):
             return None
         res = residual.data_ptr()
     y = x.new_empty((*shape[:-1], r.width))
-    t = counters = None
-    flags = 0
-    if r.R:
-        t = x.new_empty((M, r.R))
-        counters = ops._arena_address(x.device, (M + 127) // 128 + 1)
-        flags = ((1 << 8) if layers.LORA_SHRINK == "separate" else 0) | ops._no_wait_bit()
-    lib = _lib.load()
+    t = x.new_empty((M, r.R)) if r.R else None
+    lib, counters, flags = _lib.load(), 0, (1 << 8) if layers.LORA_SHRINK == "separate" else 0
     ranges = ops.chain_hints(r.key, r.refs, r.key)
     if ranges is not None:
         lib.kh_set_weight_prefetch(None, 0)
         for ptr, nbytes in ranges:
             lib.kh_set_weight_prefetch(ptr, nbytes)
-    rc = lib.kh_lora_linear_desc_bf16(r.at, x.data_ptr(), res, y.data_ptr(), None if t is None else t.data_ptr(), counters, M, flags, ops._stream())
+    stream = ops._stream()
+    if r.R and not flags:
+        counters = ops.counters_begin(r.device, (M + 127) // 128 + 1, stream)
+    try:
+        rc = lib.kh_lora_linear_desc_bf16(r.at, x.data_ptr(), res, y.data_ptr(), None if t is None else t.data_ptr(), counters or None, M, flags, stream)
+    finally:
+        if counters:
+            ops.counters_end(r.device)
     if rc:
         _lib.check(rc, "kh_lora_linear_desc_bf16")
     return y

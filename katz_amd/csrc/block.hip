@@ -67,7 +67,8 @@ struct Run {
   const Layout w;
   int32_t* counters;
 
-  int32_t* take(const KhLinearDesc& l, int64_t rows) {
+  int32_t* take(const KhLinearDesc& l, int64_t rows) {   // (none where every linear is two launches)
+    if (counters == nullptr) return nullptr;
     int32_t* p = l.R == 0 ? nullptr : counters;
     counters += counters_of(l, rows);
     return p;
@@ -130,9 +131,10 @@ KH_EXPORT int kh_transformer_block_bf16(const KhBlockDesc* desc, const KhBlockCa
     return KH_ERR_INVALID_ARG;
   const Layout w = layout(d, M, Mc, cross, own_kv);
   if (w.bytes > c.workspace_bytes || !kh_aligned16(c.workspace)) return KH_ERR_INVALID_ARG;
-  const int64_t ints = counter_ints(d, M, Mc, cross, own_kv);
+  const bool waits = (c.flags & ((1 << 8) | (1 << 24))) == 0;
+  const int64_t ints = waits ? counter_ints(d, M, Mc, cross, own_kv) : 0;
   if (ints > c.counter_ints || (ints > 0 && !c.counters)) return KH_ERR_INVALID_ARG;
-  Run r{c, stream, (char*)c.workspace, w, c.counters};
+  Run r{c, stream, (char*)c.workspace, w, waits ? c.counters : nullptr};
   char* const ws = r.ws;
   const float* const ln = d.folded ? c.stats : nullptr;
   float* const stats = d.folded ? c.stats : nullptr;

@@ -58,6 +58,16 @@ KH_EXPORT int kh_profile_end(int32_t* tags, float* ms, int capacity) {
 
 KH_EXPORT int kh_version(void) { return 2; }
 
+// See include/katz_hip.h.
+KH_EXPORT int kh_stream_capture_id(void* stream, uint64_t* id) {
+  if (!id) return KH_ERR_INVALID_ARG;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long n = 0;
+  const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream, &status, &n);
+  *id = e == hipSuccess && status == hipStreamCaptureStatusActive ? (uint64_t)n : 0;
+  return (int)e;
+}
+
 KH_EXPORT const char* kh_error_string(int code) {
   switch (code) {
     case KH_OK: return "ok";

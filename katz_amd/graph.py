@@ -42,9 +42,12 @@ class GraphedUNetStep:
         self.down = None if down_block_additional_residuals is None else [cl(r) for r in down_block_additional_residuals]
         self.mid = None if mid_block_additional_residual is None else cl(mid_block_additional_residual)
         unet.prepare()
+        from . import ops
+
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side), torch.no_grad():
+            ops.claim_waits(sample.device)   # (so that the warm-up runs the launches that will be recorded)
             for _ in range(warmup):   # workspace and counter allocation, lazy packing: all before capture
                 self._run()
         torch.cuda.current_stream().wait_stream(side)
@@ -61,6 +64,8 @@ class GraphedUNetStep:
     def __call__(self, sample=None, timestep=None, encoder_hidden_states=None, added_cond_kwargs=None,
                  down_block_additional_residuals=None, mid_block_additional_residual=None) -> torch.Tensor:
         """Refresh whichever static inputs are given, replay, return the (static) output tensor."""
+        from . import ops
+
         if sample is not None:
             self.sample.copy_(sample)
         if timestep is not None:
@@ -75,6 +80,7 @@ class GraphedUNetStep:
                 dst.copy_(src)
         if mid_block_additional_residual is not None:
             self.mid.copy_(mid_block_additional_residual)
+        ops.claim_waits(self.sample.device)
         self.graph.replay()
         return self.out
 
@@ -154,6 +160,7 @@ class GraphedDenoiseStep:
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side), torch.no_grad():
+            ops.claim_waits(dev)             # (so that the warm-up runs the launches that will be recorded)
             if self.hoist:
                 self.cond_emb = controlnet.embed_condition(self.cond)
             self._project_context()
@@ -250,6 +257,7 @@ class GraphedDenoiseStep:
             self.model_input.copy_((torch.cat([latents] * 2).float() / table[0, 3]).to(torch.bfloat16))
             for i in range(table.shape[0]):
                 self.row.copy_(table[i])
+                self._ops.claim_waits(dev)
                 self.graph.replay()
         if check:
             self._ops.check_split_timeouts(dev)

@@ -11,6 +11,7 @@ import contextlib
 import ctypes
 import math
 import os
+import threading
 import weakref
 from typing import Optional, Sequence
 
@@ -236,13 +237,6 @@ def lora_shrink(x: torch.Tensor, a_cat: torch.Tensor, col_scale: torch.Tensor, o
     return out
 
 
-def _no_wait_bit() -> int:
-    """Flag bit 24 of the split / norm / xattn entry points: inside side_branch() no launch's workgroups wait for others of
-    it (the shrink is a launch of its own).  Two launches that wait, side by side on two streams, could each hold the CUs
-    that workgroups the other one waits for need."""
-    return (1 << 24) if _ws_slot[0] > 0 else 0
-
-
 def _r_used_bits(r_used: int, R: int) -> int:
     if r_used < 0 or r_used > R or r_used % 16:
         raise ValueError(f"r_used must be a multiple of 16 in [0, {R}], got {r_used}")
@@ -285,30 +279,123 @@ def lora_linear_pre(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.
     return out
 
 
-# Counters of kh_lora_linear_split_bf16's in-launch shrink.  Every call needs ceil(M / 128) + 1 zeroed int32 and leaves
-# them dirty, so they come from one arena per device: calls take consecutive slices, and `split_counters_reset`
-# clears the WHOLE arena with one fill kernel (256 KB: as cheap as any fill) and starts over.  The whole arena, not
-# just what the host handed out since the last reset: a reset recorded into a HIP graph runs at replay time, when the
-# host's count says nothing about what eager forwards or other graphs have dirtied in between.  The UNet / ControlNet
-# forward resets at its start (inside a captured graph that is one fill node per step and the same slices on every
-# replay); a caller that never resets is served until the arena is full, then it is reset for him.  One stream per
-# device: a reset must not overtake launches that still use their slices (two models side by side on two streams:
-# clear once before the fork and run both under `split_counters_held`).
+# Counters of the launches that carry their shrink (kh_lora_linear_split_bf16 and its kin).  Every call needs ceil(M / 128) + 1
+# zeroed int32 and leaves them dirty, so they come from an arena: calls take consecutive slices, and `split_counters_reset`
+# clears the WHOLE arena with one fill kernel (256 KB: as cheap as any fill) and starts over.  The UNet / ControlNet forward
+# resets at its start; a caller that never resets is served until the arena is full, then it is reset for him.
+#
+# Slices, fills and launches have to follow each other in one order, and two launches whose workgroups wait must not run side
+# by side (see kh_lora_linear_split_bf16).  So a device's arena belongs to one stream at a time.  A call on another stream takes
+# it over when that stream has nothing left to do, and otherwise does without counters, as two launches; a lock is held from
+# the hand-out until the launch is enqueued, whatever threads there are.  `claim_waits` takes the arena over by waiting.
+#
+# Launches recorded into a graph have an arena of their own, since they run at replay, when the host's account of the other
+# says nothing.  They get slices of it only behind a reset recorded into the SAME graph on the same stream (a captured model
+# forward begins with one): without it a second replay would find the first one's arrivals and read T before it is there.
+# A bare captured layer runs as two launches.  Graphs share that arena; replays belong on one stream or behind `claim_waits`.
 SPLIT_ARENA_INTS = 1 << 16
-_split_arena: dict = {}     # (device type, index) -> [buffer, ints handed out, (start, length) of the last slice, ever used, address]
 
 
-def _arena(device):
-    key = (device.type, device.index)
-    st = _split_arena.get(key)
+class _Arena:
+    def __init__(self, device):
+        self.buf = torch.zeros(SPLIT_ARENA_INTS, dtype=torch.int32, device=device)
+        self.at, self.pos = self.buf.data_ptr(), 0      # its address, ints handed out
+
+    def clear(self):
+        self.buf.zero_()
+        self.pos = 0
+
+
+class _Counters:
+    """What a device's launches that wait share; everything but `lock` is read and written under it."""
+
+    def __init__(self, device):
+        self.lock = threading.Lock()
+        self.acquire, self.release = self.lock.acquire, self.lock.release
+        self.eager, self.graphs = _Arena(device), _Arena(device)
+        self.owner = self.stream = None      # the stream the eager arena belongs to: its handle, its Stream
+        self.recorded = None                 # (capture, stream) of the reset that clears `graphs`
+        self.last, self.last_ints = None, 0  # arena and ints of the last slice
+
+
+_split_counters: dict = {}     # device index -> _Counters
+_split_new = threading.Lock()
+_capturing = torch._C._cuda_isCurrentStreamCapturing if hasattr(torch._C, "_cuda_isCurrentStreamCapturing") else lambda: False
+
+
+def _capture_id() -> int:
+    """The capture the current stream is part of."""
+    n = ctypes.c_uint64(0)
+    _lib.check(_lib.load().kh_stream_capture_id(_stream(), ctypes.byref(n)), "kh_stream_capture_id")
+    return n.value
+
+
+def _counters_of(device) -> _Counters:
+    st = _split_counters.get(device.index)
     if st is None:
-        if torch.cuda.is_current_stream_capturing():
+        if _capturing():
             # memory allocated during a capture belongs to the graph's pool and dies with the graph
             raise RuntimeError("katz_amd: run the step once eagerly before capturing it (the LoRA counter arena is "
                                "allocated on first use and must outlive the graph)")
-        buf = torch.zeros(SPLIT_ARENA_INTS, dtype=torch.int32, device=device)
-        st = _split_arena[key] = [buf, 0, None, False, buf.data_ptr()]
+        with _split_new:
+            st = _split_counters.get(device.index)
+            if st is None:
+                st = _split_counters[device.index] = _Counters(device)
     return st
+
+
+def _owns(st: _Counters, stream: int) -> bool:
+    """Does the eager arena belong to the current stream, or can it (nothing is left of what its owner enqueued)?"""
+    if st.owner == stream:
+        return True
+    if st.stream is not None and not st.stream.query():
+        return False
+    st.owner, st.stream = stream, torch.cuda.current_stream()
+    return True
+
+
+def counters_begin(device, n: int, stream: Optional[int] = None) -> int:
+    """The address of n zeroed int32 for one launch that carries its shrink, the device's lock held until counters_end(device);
+    or 0: no such launch now, the call makes two."""
+    st = _split_counters.get(device.index) or _counters_of(device)
+    if _ws_slot[0]:
+        return 0
+    if stream is None:
+        stream = _stream()
+    st.acquire()
+    if st.owner == stream and not _capturing():
+        arena = st.eager
+        at = arena.pos
+        if at + n <= SPLIT_ARENA_INTS:
+            arena.pos = at + n
+            st.last, st.last_ints = arena, n
+            return arena.at + 4 * at
+    return _counters_begin_slow(st, n, stream)
+
+
+def _counters_begin_slow(st: _Counters, n: int, stream: int) -> int:
+    at = 0
+    try:
+        if _capturing():
+            arena = st.graphs if st.recorded is not None and st.recorded == (_capture_id(), stream) else None
+        else:
+            arena = st.eager if _owns(st, stream) else None
+        if arena is not None:
+            if arena.pos + n > SPLIT_ARENA_INTS:
+                if _arena_held[0]:
+                    raise RuntimeError("katz_amd: the LoRA counter arena is full inside split_counters_held()")
+                arena.clear()
+            at = arena.at + 4 * arena.pos
+            arena.pos += n
+            st.last, st.last_ints = arena, n
+    finally:
+        if not at:
+            st.release()
+    return at
+
+
+def counters_end(device) -> None:
+    _split_counters[device.index].release()
 
 
 _arena_held: list = [0]
@@ -327,15 +414,32 @@ def split_counters_held():
 
 
 def split_counters_reset(device) -> None:
-    """Clear every counter of the device's arena with one fill kernel.  Outside graph capture the fill is skipped
-    while no counter has ever been handed out; under capture it is always recorded, because by the time the graph is
-    replayed other forwards may have dirtied the arena."""
-    if _arena_held[0]:
+    """Clear every counter of the current stream's arena with one fill kernel: under capture the graphs', always, because by the
+    time the graph is replayed other graphs may have dirtied it; otherwise the eager one, if it belongs to this stream and
+    counters have been handed out.  Inside side_branch(), where no launch waits, there is nothing to clear."""
+    if _arena_held[0] or _ws_slot[0]:
         return
-    st = _arena(device)
-    if st[3] or torch.cuda.is_current_stream_capturing():
-        st[0].zero_()
-    st[1] = 0
+    st = _counters_of(device)
+    with st.lock:
+        if _capturing():
+            st.graphs.clear()
+            st.recorded = (_capture_id(), _stream())
+        elif _owns(st, _stream()):
+            if st.eager.pos:
+                st.eager.clear()
+
+
+def claim_waits(device) -> None:
+    """Launches that wait belong to the current stream from here on; it first waits for what the stream they belonged to has
+    enqueued.  For a captured graph with such launches, before it is replayed."""
+    st = _counters_of(device)
+    with st.lock:
+        stream = _stream()
+        if st.owner != stream:
+            current = torch.cuda.current_stream()
+            if st.stream is not None:
+                current.wait_stream(st.stream)
+            st.owner, st.stream = stream, current
 
 
 class SplitTimeoutError(_lib.KatzHipError):
@@ -364,43 +468,25 @@ def check_split_timeouts(device=None) -> None:
                                 "the LoRA linears of the affected steps read an incomplete shrink result")
 
 
-def _split_counters(device, M: int) -> torch.Tensor:
-    return _arena_ints(device, (M + 127) // 128 + 1)   # KH_SPLIT_COUNTER_INTS(M)
+def _counter_ints(M: int) -> int:
+    return (M + 127) // 128 + 1   # KH_SPLIT_COUNTER_INTS(M)
 
 
-def _arena_ints(device, n: int) -> torch.Tensor:
-    """n zeroed int32 of the device's counter arena (zero since the last split_counters_reset)."""
-    st = _arena_take(device, n)
-    at, _ = st[2]
-    return st[0][at:at + n]
-
-
-def _arena_address(device, n: int) -> int:
-    """The address of _arena_ints(device, n)."""
-    st = _arena_take(device, n)
-    return st[4] + 4 * st[2][0]
-
-
-def _arena_take(device, n: int) -> list:
-    st = _arena(device)
-    if st[1] + n > SPLIT_ARENA_INTS:
-        if _arena_held[0]:
-            raise RuntimeError("katz_amd: the LoRA counter arena is full inside split_counters_held()")
-        split_counters_reset(device)
-    st[2] = (st[1], n)
-    st[1] += n
-    st[3] = True
-    return st
+def _arena_ints(device, n: int) -> Optional[torch.Tensor]:
+    """n zeroed int32 as counters_begin hands them out (for tests)."""
+    if not counters_begin(device, n):
+        return None
+    try:
+        return split_counters_last(device)
+    finally:
+        counters_end(device)
 
 
 def split_counters_last(device) -> Optional[torch.Tensor]:
-    """The counters of the most recent lora_linear_split call on this device (for tests: arrivals per row block, then
+    """The counters of the most recent launch on this device that carried its shrink (for tests: arrivals per row block, then
     the time-out flag)."""
-    st = _arena(device)
-    if st[2] is None:
-        return None
-    at, n = st[2]
-    return st[0][at:at + n]
+    st = _counters_of(device)
+    return None if st.last is None else st.last.buf[st.last.pos - st.last_ints:st.last.pos]
 
 
 def lora_linear_split(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], a_cat: torch.Tensor,
@@ -432,15 +518,19 @@ def lora_linear_split(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
     n_out = N // 2 if geglu else N
     out = torch.empty(tuple(x.shape[:-1]) + (n_out,), dtype=BF16, device=x.device)
     t = torch.empty((M, RT), dtype=BF16, device=x.device)
-    cnt = _split_counters(x.device, M)
-    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16) | _no_wait_bit()
-    if CALL_LOG is not None:   # one entry per kernel launch
-        if lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2:
-            CALL_LOG.append(("lora_shrink", M, K, RT))
-        CALL_LOG.append(("lora_linear", M, N, K, R, bool(geglu), residual is not None))
-    _weight_prefetch_hint(weight, a_cat, b_cat)
-    rc = lib.kh_lora_linear_split_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
-                                       _ptr(cnt), _ptr(residual), _ptr(out), M, N, K, R, n_split, flags, _stream())
+    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16)
+    cnt = 0 if two_launches else counters_begin(x.device, _counter_ints(M))
+    try:
+        if CALL_LOG is not None:   # one entry per kernel launch
+            if not cnt or lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2:
+                CALL_LOG.append(("lora_shrink", M, K, RT))
+            CALL_LOG.append(("lora_linear", M, N, K, R, bool(geglu), residual is not None))
+        _weight_prefetch_hint(weight, a_cat, b_cat)
+        rc = lib.kh_lora_linear_split_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
+                                           cnt or None, _ptr(residual), _ptr(out), M, N, K, R, n_split, flags, _stream())
+    finally:
+        if cnt:
+            counters_end(x.device)
     _lib.check(rc, "kh_lora_linear_split_bf16")
     return out
 
@@ -507,19 +597,21 @@ def lora_linear_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
             raise ValueError("stats_out must be a row_stats_buffer for the rows of the output")
     n_out = N // 2 if geglu else N
     out = torch.empty(tuple(x.shape[:-1]) + (n_out,), dtype=BF16, device=x.device)
-    t = cnt = None
-    if R:
-        t = torch.empty((M, RT), dtype=BF16, device=x.device)
-        cnt = _split_counters(x.device, M)
-    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | _no_wait_bit()
-    if CALL_LOG is not None:   # one entry per kernel launch
-        if R and lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2:
-            CALL_LOG.append(("lora_shrink", M, K, RT))
-        CALL_LOG.append(("lora_linear", M, N, K, R, bool(geglu), residual is not None, ln is not None, stats_out is not None))
-    _weight_prefetch_hint(weight, a_cat, b_cat)
-    rc = lib.kh_lora_linear_norm_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
-                                      _ptr(cnt), _ptr(residual), _ptr(out), _ptr(part), _ptr(c1), _ptr(c2), _ptr(ca1), _ptr(ca2),
-                                      float(eps), _ptr(stats_out), M, N, K, R, n_split, flags, _stream())
+    t = torch.empty((M, RT), dtype=BF16, device=x.device) if R else None
+    flags = (1 if geglu else 0) | ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0)
+    cnt = counters_begin(x.device, _counter_ints(M)) if R and not two_launches else 0
+    try:
+        if CALL_LOG is not None:   # one entry per kernel launch
+            if R and (not cnt or lib.kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 2):
+                CALL_LOG.append(("lora_shrink", M, K, RT))
+            CALL_LOG.append(("lora_linear", M, N, K, R, bool(geglu), residual is not None, ln is not None, stats_out is not None))
+        _weight_prefetch_hint(weight, a_cat, b_cat)
+        rc = lib.kh_lora_linear_norm_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
+                                          cnt or None, _ptr(residual), _ptr(out), _ptr(part), _ptr(c1), _ptr(c2), _ptr(ca1), _ptr(ca2),
+                                          float(eps), _ptr(stats_out), M, N, K, R, n_split, flags, _stream())
+    finally:
+        if cnt:
+            counters_end(x.device)
     _lib.check(rc, "kh_lora_linear_norm_bf16")
     return out
 
@@ -576,20 +668,22 @@ def lora_linear_xattn(x: torch.Tensor, weight: torch.Tensor, k: torch.Tensor, v:
     if scale is None:
         scale = 1.0 / 8.0
     out = torch.empty((B, T, N), dtype=BF16, device=x.device)
-    t = cnt = None
-    if R:
-        t = torch.empty((M, R), dtype=BF16, device=x.device)
-        cnt = _split_counters(x.device, M)
-    flags = ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0) | _no_wait_bit()
-    if CALL_LOG is not None:   # one entry per kernel launch
-        if R and lib.kh_lora_linear_xattn_launches(M, N, K, R, T, S, flags) == 2:
-            CALL_LOG.append(("lora_shrink", M, K, R))
-        CALL_LOG.append(("lora_linear_xattn", M, N, K, R, heads, T, S))
-    _weight_prefetch_hint(weight, a_cat, b_cat)
-    rc = lib.kh_lora_linear_xattn_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
-                                       _ptr(cnt), _ptr(part), _ptr(c1), _ptr(c2), _ptr(ca1), _ptr(ca2), float(eps),
-                                       _ptr(k), _ptr(v), _ptr(out), M, N, K, R, T, S, k.stride(1), v.stride(1), out.stride(1),
-                                       k.stride(0), v.stride(0), float(scale), flags, _stream())
+    t = torch.empty((M, R), dtype=BF16, device=x.device) if R else None
+    flags = ((1 if two_launches else 0) << 8) | (_r_used_bits(r_used, R) << 16 if R else 0)
+    cnt = counters_begin(x.device, _counter_ints(M)) if R and not two_launches else 0
+    try:
+        if CALL_LOG is not None:   # one entry per kernel launch
+            if R and (not cnt or lib.kh_lora_linear_xattn_launches(M, N, K, R, T, S, flags) == 2):
+                CALL_LOG.append(("lora_shrink", M, K, R))
+            CALL_LOG.append(("lora_linear_xattn", M, N, K, R, heads, T, S))
+        _weight_prefetch_hint(weight, a_cat, b_cat)
+        rc = lib.kh_lora_linear_xattn_bf16(_ptr(x), _ptr(weight), _ptr(bias), _ptr(a_cat), _ptr(col_scale), _ptr(b_cat), _ptr(t),
+                                           cnt or None, _ptr(part), _ptr(c1), _ptr(c2), _ptr(ca1), _ptr(ca2), float(eps),
+                                           _ptr(k), _ptr(v), _ptr(out), M, N, K, R, T, S, k.stride(1), v.stride(1), out.stride(1),
+                                           k.stride(0), v.stride(0), float(scale), flags, _stream())
+    finally:
+        if cnt:
+            counters_end(x.device)
     _lib.check(rc, "kh_lora_linear_xattn_bf16")
     return out
 

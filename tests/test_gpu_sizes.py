@@ -720,3 +720,65 @@ def test_bit_24_leaves_the_counters_alone(M, N, K, R, r_used, n_split, entry):
         return y
 
     assert torch.equal(run(1 << 24), run(1 << 8))
+
+
+@pytest.mark.parametrize("M,N,K,R", [(154, 1280, 2048, 32), (2048, 1280, 1280, 64)])
+@pytest.mark.parametrize("reset", [False, True])
+def test_captured_layers_see_their_own_inputs(M, N, K, R, reset):
+    """A layer in a graph of its own runs as two launches, one behind a reset in the same graph (a model's forward) with its shrink inside; either way
+    every replay gives the eager result of the inputs it finds, with eager calls in between."""
+    from katz_amd import ops
+
+    say("captured layers", M, N, K, R, reset)
+    d, g = dev(), torch.Generator().manual_seed(M)
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(d, BF)
+    xs, w, A, B = rnd(4, M, K), rnd(N, K, std=0.03), rnd(R, K, std=0.05), rnd(N, R, std=0.5)
+    sc, x = torch.ones(R, device=d), torch.zeros(M, K, dtype=BF, device=d)
+    call = lambda two=False: ops.lora_linear_split(x, w, None, A, sc, B, two_launches=two)
+    assert ops._lib.load().kh_lora_linear_split_launches(M, N, K, R, 0, 0) == 1
+    call()
+    st = ops._split_counters[0]
+    torch.cuda.synchronize()
+    graph, before = torch.cuda.CUDAGraph(), (st.graphs.pos, st.eager.pos)
+    with torch.cuda.graph(graph):
+        if reset:
+            ops.split_counters_reset(d)
+        outs = [call() for _ in range(3)]
+    if reset:
+        assert st.graphs.pos == 3 * ((M + 127) // 128 + 1) and st.eager.pos == before[1]
+    else:
+        assert (st.graphs.pos, st.eager.pos) == before
+    for v in xs:
+        x.copy_(v)
+        want = call(not reset)
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        for o in outs:
+            assert torch.equal(o, want)
+    ops.check_split_timeouts(d)
+
+
+def test_two_streams_of_few_row_calls():
+    """Calls of few rows on two streams at once, one of them resetting: the bits of a quiet device on both."""
+    from katz_amd import ops
+
+    say("few rows on two streams")
+    d, g = dev(), torch.Generator().manual_seed(4)
+    M, N, K, R = 154, 1280, 2048, 64
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(d, BF)
+    x, w, A, B, sc = rnd(2, M, K), rnd(N, K, std=0.03), rnd(R, K, std=0.05), rnd(N, R, std=0.05), torch.ones(R, device=d)
+    call = lambda i: ops.lora_linear_split(x[i], w, None, A, sc, B)
+    want = [call(0), call(1)]
+    torch.cuda.synchronize()
+    streams, got = [torch.cuda.Stream(), torch.cuda.Stream()], ([], [])
+    for n in range(60):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                if i and n % 5 == 0:
+                    ops.split_counters_reset(d)
+                got[i].append(call(i))
+    torch.cuda.synchronize()
+    for i in (0, 1):
+        assert all(torch.equal(y, want[i]) for y in got[i])
+    ops.check_split_timeouts(d)

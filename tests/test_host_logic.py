@@ -634,3 +634,130 @@ def test_weight_prefetch_hints_never_cross_models_or_forwards(monkeypatch):
     del cnet, tc
     gc.collect()
     assert len(ops._pf_tables) == n - 1
+
+
+class _FakeStreams:
+    """Streams and captures as the counters see them, without a GPU."""
+
+    class Stream:
+        def __init__(self, owner, handle):
+            self.owner, self.handle, self.waited = owner, handle, []
+
+        def query(self):
+            return self.handle not in self.owner.busy
+
+        def wait_stream(self, other):
+            self.waited.append(other.handle)
+
+    def __init__(self, monkeypatch):
+        import torch
+        from katz_amd import ops
+
+        self.current, self.capture, self.busy = 1, 0, set()
+        self.streams = {h: self.Stream(self, h) for h in range(1, 9)}
+        monkeypatch.setattr(ops, "_split_counters", {})
+        monkeypatch.setattr(ops, "_stream", lambda: self.current)
+        monkeypatch.setattr(ops, "_capturing", lambda: self.capture != 0)
+        monkeypatch.setattr(ops, "_capture_id", lambda: self.capture)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda: self.streams[self.current])
+
+    def take(self, n=4):
+        """A launch's counters; those of the eager arena as (0, first int), a graph's as (1, first int), None: two launches."""
+        import torch
+        from katz_amd import ops
+
+        dev = torch.device("cpu")
+        at = ops.counters_begin(dev, n)
+        if not at:
+            return None
+        ops.counters_end(dev)
+        st = ops._split_counters[None]
+        return next((i, (at - a.at) // 4) for i, a in enumerate((st.eager, st.graphs)) if 0 <= at - a.at < 4 * ops.SPLIT_ARENA_INTS)
+
+
+def test_counters_belong_to_one_stream_at_a_time(monkeypatch):
+    """A launch that waits is made on one stream only while another still has some under way, and that other one's reset does not
+    clear counters in use."""
+    import torch
+    from katz_amd import ops
+
+    f, dev = _FakeStreams(monkeypatch), torch.device("cpu")
+    assert f.take() == (0, 0) and f.take() == (0, 4)
+    st = ops._split_counters[None]
+    st.eager.buf[:8] = 7                                 # arrivals of launches on stream 1
+    f.busy, f.current = {1}, 2
+    assert f.take() is None
+    ops.split_counters_reset(dev)                        # a model on stream 2 starts its forward
+    assert st.eager.buf[:8].tolist() == [7] * 8 and st.eager.pos == 8
+    f.current = 1
+    assert f.take() == (0, 8)
+    f.busy, f.current = set(), 2                         # stream 1 has finished
+    assert f.take() == (0, 12)                           # (slices nobody has used since the last reset)
+    f.busy, f.current = {2}, 1
+    assert f.take() is None
+    ops.claim_waits(dev)                                 # a graph's replay: behind stream 2, the owner from here on
+    assert f.streams[1].waited == [2] and f.take() == (0, 16)
+    ops.split_counters_reset(dev)
+    assert st.eager.buf[:8].tolist() == [0] * 8 and f.take() == (0, 0)
+    with ops.side_branch():
+        assert f.take() is None
+        ops.split_counters_reset(dev)
+    assert st.eager.pos == 4
+
+
+def test_graphs_take_counters_only_behind_their_own_reset(monkeypatch):
+    """A captured launch may wait only where the same graph clears its counters first: on a second replay it would find the first
+    one's arrivals."""
+    import torch
+    from katz_amd import ops
+
+    f, dev = _FakeStreams(monkeypatch), torch.device("cpu")
+    assert f.take() == (0, 0)
+    f.current, f.capture = 3, 11
+    assert f.take() is None                              # a layer captured by itself
+    ops.split_counters_reset(dev)                        # a model's forward
+    assert f.take() == (1, 0) and f.take() == (1, 4)
+    f.current = 4
+    assert f.take() is None                              # a fork of that capture
+    f.current, f.capture = 3, 12
+    assert f.take() is None                              # the next graph
+    ops.split_counters_reset(dev)
+    assert f.take() == (1, 0)
+    f.current, f.capture = 1, 0
+    assert f.take() == (0, 4)                            # eager launches are not in the way
+
+
+def test_threads_hand_out_and_launch_in_one_order(monkeypatch):
+    """From the hand-out of a slice until its launch is enqueued no other thread gets one or resets, and every slice is another."""
+    import threading
+
+    import torch
+    from katz_amd import ops
+
+    f, dev = _FakeStreams(monkeypatch), torch.device("cpu")
+    first = ops.counters_begin(dev, 4)
+    order = []
+
+    def other():
+        order.append(("other", ops.counters_begin(dev, 4)))
+        ops.counters_end(dev)
+
+    th = threading.Thread(target=other)
+    th.start()
+    th.join(0.2)
+    assert th.is_alive()
+    order.append(("first", first))
+    ops.counters_end(dev)
+    th.join(10)
+    assert [n for n, _ in order] == ["first", "other"] and order[1][1] == first + 16
+    got = []
+
+    def many():
+        for _ in range(500):
+            got.append(ops.counters_begin(dev, 3))
+            ops.counters_end(dev)
+
+    threads = [threading.Thread(target=many) for _ in range(8)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert len(set(got)) == 4000
