@@ -12,10 +12,10 @@
 //            allows, else 128.  T is rounded to bf16 and written to LDS in the stage layout, so that
 //   phase 2: for every 128-column tile of y:  acc = T . B_a[tile]^T  (K = the adapter's padded rank, one or two stages of
 //            B from L2, requested while the previous tile is being finished), times the adapter's scale, rounded, transposed through
-//            LDS and added to the y pieces, which were requested five tiles ahead.
+//            LDS and added to the y pieces, which were requested five tiles ahead (128 rows: one).
 // What bounds it at a request's sizes is not HBM's rate but the chain of latencies -- segment table, 20 stages, 5 .. 10 tiles -- in workgroups
 // that are one to a CU.  Hence as many stages under way as 128 KB hold (seven of 16 KB instead of two of 32: with 128 rows and all 128 rank rows
-// a stage took 0.45 us), the y pieces of the first five tiles requested while phase 1 runs, and 64-row blocks while they fit one
+// a stage took 0.45 us), the y pieces of the first five tiles (128 rows: of the first) requested while phase 1 runs, and 64-row blocks while they fit one
 // round of the 256 CUs, so that fewer of them repeat phase 1 for other columns.
 // 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 24.9 -> 19.8 us.
 // Rows / columns of A_a / B_a beyond the adapter's rank are zero by contract, so the padded rank only saves work.
@@ -58,7 +58,9 @@ template <int BM>
 __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   constexpr int TI = BM / 64, T_BYTES = 2 * BM * 128;   // a wave's 32-row tiles; T as two 64-column stages of 128-byte rows
-  constexpr int YD = BM == 64 ? 5 : 2;                  // tiles whose y pieces are under way or here
+  // tiles whose y pieces are under way or here.  128 rows: those of the second tile would only be in the way of phase 1's short ring (8 x 4096 rows
+  // at 640 33.1 -> 32.3 us without them, rank 64 29.9 -> 29.3, at 1280 55.9 -> 53.9)
+  constexpr int YD = BM == 64 ? 5 : 1;
   static_assert(T_BYTES + 2 * B_TILE <= RING, "T and the B buffers lie in the ring");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int seg = blockIdx.y;
