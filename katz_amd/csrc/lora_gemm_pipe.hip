@@ -1195,8 +1195,11 @@ bool plain_ok(const LoraGemmParams& p) { return p.R == 0 || p.t_ext != nullptr; 
 // against 17.8 + 4.6 for the two launches (the GEMM workgroups run 2 us slower beside the shrink, whether or not they
 // have to wait for it); inside the UNet step, K = 5120: 53 us against 49 + 12 (there the two-launch GEMM would use the
 // 64x160 tiles, which fill every CU and leave the shrink no room).
-// 0: not suited; 1: 128x128 tiles that leave CUs idle; 2: 256x128 tiles for the stacked q/k/v projection (the shrink
-// tiles take a round of CUs first, the GEMM tiles follow as they free up: still shorter than two launches)
+// 0: not suited; 1: 128x128 tiles that leave CUs idle (lora_gemm_fine.hip); 2: 256x128 tiles for the stacked q/k/v projection (the shrink
+// tiles take a round of CUs first, the GEMM tiles follow as they free up: still shorter than two launches); 3: 128x128 tiles of this file, for a
+// query projection with its attention and for columns that are no multiple of 128.  The latter from K 1024 on, where no fine tile smaller than
+// 128 x 80 takes the call (M / N / K, rank, weights from HBM, us in two launches / in one: 2048 / 1216 / 1280, 96 21.0 / 17.9, 2560 38.2 / 31.2, 1024
+// 17.8 / 14.1, 640 14.4 / 16.8; 1024 / 1000 / 1280, 64 20.5 / 17.0; 1536 / 1600 / 1280, 64 18.4 / 17.6; 2048 / 480 / 1280, 64 on 64 x 80 tiles 13.1 / 17.0).
 static int il_form(const LoraGemmParams& p) {
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
   const long shr = (long)((p.M + 63) / 64) * il_col_tiles(p);
@@ -1205,7 +1208,12 @@ static int il_form(const LoraGemmParams& p) {
                   p.col_scale != nullptr && p.il_cnt != nullptr && t_ok && p.grp == nullptr && p.sg_mode == 0 && p.conv_cin == 0 &&
                   !p.geglu && p.M >= 1024;
   if (!ok) return 0;
-  if (tiles <= 192 && tiles + shr <= 256) return p.xa_k != nullptr || (p.N % 128 == 0 && lora_gemm_fine_ok(p)) ? 1 : 0;
+  if (tiles <= 192 && tiles + shr <= 256) {
+    if (p.xa_k != nullptr) return 3;
+    if (p.N % 128 == 0 && lora_gemm_fine_ok(p)) return 1;
+    const int fine = p.K >= 1024 ? lora_gemm_pipe_fine_form(p) : 0;
+    return fine == -1 || (fine == 1 && !lora_gemm_fine_il_ok(p)) ? 3 : 0;
+  }
   if (tiles >= 480 && p.K >= 1024 && (long)((p.M + 255) / 256) * ((p.N + 127) / 128) <= 256 && shr <= 256) return 2;
   return 0;
 }
@@ -1255,39 +1263,42 @@ static int launch_il(const LoraGemmParams& pin, hipStream_t stream) {
   const int shr = ((p.M + 63) / 64) * p.il_cols;
   p.il_blocks = (shr + 7) / 8 * 8;
   const unsigned grid = (unsigned)p.il_blocks + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  if constexpr (std::is_same<C, PCfg<128, 128, 2, 4, 0, 4, 64>>::value) {   // only behind a query projection
-    if (p.xa_k == nullptr || p.res != nullptr || p.st_part != nullptr || p.M % 128 != 0 || p.N % 128 != 0) return KH_ERR_UNSUPPORTED;
-    auto go = [&](auto lnf) {
-      constexpr int L = decltype(lnf)::value;
-      if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L, true>>(LDS_LN); e != hipSuccess) return (int)e;
-      kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L, true>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
-      KH_RETURN_LAST_ERROR();
-    };
-    return p.ln_part != nullptr ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 0>{});
-  } else {
-    if (p.xa_k != nullptr) return KH_ERR_UNSUPPORTED;
-    if (p.ln_part != nullptr || p.st_part != nullptr) {
-      if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
+  if (p.xa_k != nullptr) {   // behind a query projection
+    if constexpr (std::is_same<C, PCfg<128, 128, 2, 4, 0, 4, 64>>::value) {
+      if (p.res != nullptr || p.st_part != nullptr || p.M % 128 != 0 || p.N % 128 != 0) return KH_ERR_UNSUPPORTED;
       auto go = [&](auto lnf) {
         constexpr int L = decltype(lnf)::value;
-        if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L>>(LDS_LN); e != hipSuccess) return (int)e;
-        kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
+        if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L, true>>(LDS_LN); e != hipSuccess) return (int)e;
+        kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L, true>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
         KH_RETURN_LAST_ERROR();
       };
-      if (p.ln_part != nullptr && p.st_part != nullptr) return go(std::integral_constant<int, 3>{});
-      if (p.ln_part != nullptr) return go(std::integral_constant<int, 1>{});
-      return go(std::integral_constant<int, 2>{});
+      return p.ln_part != nullptr ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 0>{});
+    } else {
+      return KH_ERR_UNSUPPORTED;
     }
-    if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true>>(LDS); e != hipSuccess) return (int)e;
-    kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true>, dim3(grid), dim3(C::NT), (size_t)LDS, stream, p);
-    KH_RETURN_LAST_ERROR();
   }
+  if (p.ln_part != nullptr || p.st_part != nullptr) {
+    if (p.st_part != nullptr && p.n_tiles > KH_LN_SLOTS) return KH_ERR_UNSUPPORTED;
+    auto go = [&](auto lnf) {
+      constexpr int L = decltype(lnf)::value;
+      if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true, L>>(LDS_LN); e != hipSuccess) return (int)e;
+      kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true, L>, dim3(grid), dim3(C::NT), (size_t)LDS_LN, stream, p);
+      KH_RETURN_LAST_ERROR();
+    };
+    if (p.ln_part != nullptr && p.st_part != nullptr) return go(std::integral_constant<int, 3>{});
+    if (p.ln_part != nullptr) return go(std::integral_constant<int, 1>{});
+    return go(std::integral_constant<int, 2>{});
+  }
+  if (hipError_t e = kh_allow_lds<lora_gemm_pipe_kernel<C, false, true>>(LDS); e != hipSuccess) return (int)e;
+  kh_launch(KH_TAG_LORA_GEMM, lora_gemm_pipe_kernel<C, false, true>, dim3(grid), dim3(C::NT), (size_t)LDS, stream, p);
+  KH_RETURN_LAST_ERROR();
 }
 
 int lora_gemm_pipe_launch_il(const LoraGemmParams& p, hipStream_t stream) {
   switch (il_form(p)) {
     case 1: return lora_gemm_fine_launch_il128(p, stream);
     case 2: return launch_il<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream);
+    case 3: return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
     default: return KH_ERR_UNSUPPORTED;
   }
 }
@@ -1302,7 +1313,7 @@ bool lora_gemm_pipe_xattn_ok(const LoraGemmParams& p) {
 
 int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, hipStream_t stream) {
   if (p.xa_k == nullptr || !lora_gemm_pipe_xattn_ok(p)) return KH_ERR_UNSUPPORTED;
-  if (p.a_cat != nullptr && p.il_cnt != nullptr && il_form(p) == 1) return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
+  if (p.a_cat != nullptr && p.il_cnt != nullptr && il_form(p) == 3) return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
   return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
 }
 

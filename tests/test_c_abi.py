@@ -186,3 +186,15 @@ def test_launches_of_the_query_projection_with_its_attention():
     assert launches(512, 1280, 1280, 64, 256, 77, 0) == 2          # its 128 x 128 tiles bring no shrink along below 1024 rows
     assert launches(512, 1280, 1280, 0, 256, 77, 0) == 1
     assert launches(2048, 1280, 1280, 64, 1000, 77, 0) == -2       # T % 128
+
+
+def test_ragged_columns_bring_their_shrink_along():
+    """N no multiple of 128: one launch from K 1024 on where no small tile takes the call, as for whole column tiles."""
+    from katz_amd import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libkatz_hip.so not built")
+    launches = _lib.load().kh_lora_linear_split_launches
+    for m, n, k, r, ru in ((2048, 1216, 1280, 64, 64), (1024, 1000, 1280, 128, 96), (1100, 1352, 1024, 64, 64), (1536, 1600, 1280, 64, 64)):
+        assert launches(m, n, k, r, 0, ru // 16 << 16) == 1, (m, n, k, r)
+    assert launches(2048, 1216, 640, 64, 0, 4 << 16) == 2

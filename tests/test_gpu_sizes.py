@@ -468,6 +468,55 @@ def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used,kind", [(1024, 1000, 1024, 64, 64, "res"), (2048, 1216, 1280, 128, 96, "res stats"), (1100, 1352, 1280, 128, 96, "fold"), (3000, 968, 1024, 64, 16, ""),
+                                                 (1536, 1600, 1280, 64, 64, "stats fold"), (1025, 1288, 2560, 64, 64, "")])
+def test_shrink_beside_ragged_columns(M, N, K, R, r_used, kind):
+    """Column counts that are no multiple of 128, the shrink inside the launch: the last column tile and the last row block ragged, row statistics and a
+    folded LayerNorm, behind a T that starts as NaNs; against two launches and float64."""
+    from katz_amd import ops
+    from katz_amd.lora import fold_norm_into_adapters, fold_norm_into_weight
+
+    say("shrink beside ragged columns", M, N, K, R, r_used, kind)
+    d, kind = dev(), kind.split()
+    if "stats" not in kind:
+        assert ops._lib.load().kh_lora_linear_split_launches(M, N, K, R, 0, r_used // 16 << 16) == 1
+    g = torch.Generator().manual_seed(M + N + K + R)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, BF)
+    x, w, b, A, B = rnd(M, K), rnd(N, K) * 0.03, rnd(N), rnd(R, K) * 0.05, rnd(N, R) * 0.05
+    A[r_used:], B[:, r_used:] = 0, 0
+    s, res, ln, xn, w0, b0, A0 = torch.rand(R, generator=g).to(d), rnd(M, N) if "res" in kind else None, None, x, w, b, A
+    if "fold" in kind:
+        gamma, beta = 1 + 0.1 * rnd(K), 0.1 * rnd(K)
+        w, c1, c2 = fold_norm_into_weight(w, b, gamma, beta)
+        A, ca1, ca2 = fold_norm_into_adapters(A, gamma, beta)
+        st = ops.row_stats_buffer(M, d).zero_()
+        st[0, :, 0], st[0, :, 1] = x.float().sum(1), (x.float() ** 2).sum(1)
+        ln, b = (st, c1, c2, ca1, ca2, 1e-5), None
+        xn = torch.nn.functional.layer_norm(x.double(), (K,), gamma.double(), beta.double(), 1e-5)
+
+    def run(two):
+        ops.split_counters_reset(d)
+        junk = torch.full((M, R), float("nan"), device=d, dtype=BF)     # the next scratch of this size
+        del junk
+        so = ops.row_stats_buffer(M, d).zero_() if "stats" in kind else None
+        return ops.lora_linear_norm(x, w, b, residual=res, a_cat=A, col_scale=s, b_cat=B, r_used=r_used, two_launches=two, ln=ln, stats_out=so), so
+
+    y, so = run(False)
+    assert ops.split_counters_last(d)[:-1].gt(0).all()      # (its workgroups have counted themselves in)
+    again, so2 = run(False)
+    assert torch.equal(again, y) and (so is None or torch.equal(so, so2))
+    ops.check_split_timeouts(d)
+    y2, _ = run(True)
+    assert (y != y2).float().mean().item() < 5e-3           # the shrinks add up in different orders: a few last bits of T
+    if so is not None:
+        got, yd = so.double().sum(0), y.double()
+        # fp32 sums of N values of size about 1: N * 2^-24 of their absolute sum at most
+        assert torch.allclose(got[:, 0], yd.sum(1), atol=N * N * 2.0 ** -24, rtol=0) and torch.allclose(got[:, 1], (yd * yd).sum(1), rtol=N * 2.0 ** -24)
+    f = lambda t: t.double()
+    ref = f(xn) @ f(w0).T + f(b0) + ((f(xn) @ f(A0).T) * f(s)) @ f(B).T + (0 if res is None else f(res))
+    assert ((f(y) - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T, of folded weights and of the result: 2^-9 each
+
+
 @pytest.mark.parametrize("M,N,K,split,geglu", [(1976, 10240, 1280, False, True), (1793, 10240, 1024, False, True), (3952, 1920, 640, True, False), (1500, 3840, 1280, True, False),
                                                (2900, 1920, 640, False, False), (4993, 1280, 1280, False, False), (4100, 1920, 704, True, False)])
 def test_one_round_and_nearly_full_rounds(M, N, K, split, geglu):
