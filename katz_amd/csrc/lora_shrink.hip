@@ -76,12 +76,39 @@ int launch_shrink16(const ShrinkParams& p, int group, int tiles, hipStream_t str
   KH_RETURN_LAST_ERROR();
 }
 
-template <int TR, int TC, int NWA, int NWB>
-int launch_shrink_k(const ShrinkParams& p, hipStream_t stream) {
-  // prefer a wave count that deals the 64-column chunks out evenly
-  const int KC = p.K / 64;
-  if (KC % NWA == 0 || KC % NWB != 0) return launch_shrink<SCfg<NWA, TR, TC>>(p, stream);
-  return launch_shrink<SCfg<NWB, TR, TC>>(p, stream);
+// What a call's sizes choose: the tiles, and how many waves share a sum (chunk t of 64 columns is added up by wave t % waves, then wave after wave).
+enum ShrinkTiles { GROUP_32x96, TILE_64x64, TILE_32x64, TILE_16x16, TILE_32x32 };
+struct ShrinkPlan {
+  ShrinkTiles tiles;
+  int waves;
+  int group, used;      // rank columns of a layer; 16-column tiles of them that are in use (TILE_16x16)
+};
+
+ShrinkPlan shrink_plan(int64_t M, int64_t K, int64_t R, int group, int r_used) {
+  const int64_t kc = K / 64;
+  const auto even = [&](int a, int b) { return kc % a == 0 || kc % b != 0 ? a : b; };   // prefer a count that deals the chunks out evenly
+  const int grp = group > 0 ? group : (int)R, used = (group > 0 && r_used > 0 && r_used < group ? r_used : grp) / 16;
+  // several stacked layers of rank 96 in 128 on many rows (q / k / v of the 64 x 64 level): one-wave workgroups, each a
+  // 32-row x 96-column tile of one layer over the whole K, five to a CU.  With K this short a tile is a handful of chunks
+  // and its time is load latency, not bytes: more independent workgroups per CU win (16.3 us against 20.8 with the 64 x 64
+  // tiles below at M 8192, K 640, three layers; 64 x 96 tiles of four waves 21.4, 128 x 96 tiles of two waves 25.3, although
+  // both read fewer bytes).  A single layer (R 128) stays with the 64 x 64 tiles: 8.4 us against 13.2.
+  if (group == 128 && r_used > 64 && r_used <= 96 && R % 128 == 0 && R >= 256 && M >= 4096) return {GROUP_32x96, 1, grp, used};
+  // the largest output tile that still gives most CUs a workgroup (a 64x64 tile reads half the bytes per output of a 32x64 one)
+  if (R % 64 == 0 && ((M + 63) / 64) * (R / 64) >= 160) return {TILE_64x64, even(4, 5), grp, used};
+  if (R % 64 == 0 && ((M + 31) / 32) * (R / 64) >= 256) return {TILE_32x64, even(4, 5), grp, used};
+  // 16 x 16 tiles while they get a CU each (the wave counts are those of the 32 x 32 tiles: the order of the sum)
+  return {R % grp == 0 && (M + 15) / 16 * (R / grp) * used <= 256 ? TILE_16x16 : TILE_32x32, even(8, 5), grp, used};
+}
+
+template <int TR, int TC>
+int launch_shrink_waves(const ShrinkParams& p, int waves, hipStream_t stream) {
+  switch (waves) {
+    case 4: if constexpr (TC == 2) return launch_shrink<SCfg<4, TR, TC>>(p, stream); break;
+    case 5: return launch_shrink<SCfg<5, TR, TC>>(p, stream);
+    case 8: if constexpr (TC == 1) return launch_shrink<SCfg<8, TR, TC>>(p, stream); break;
+  }
+  return KH_ERR_UNSUPPORTED;
 }
 
 }  // namespace
@@ -91,13 +118,8 @@ KH_EXPORT int kh_lora_shrink_bf16(const void* x, const void* a_cat, const float*
   return lora_shrink_ln_launch(x, a_cat, col_scale, t, M, K, R, nullptr, nullptr, nullptr, 0.f, (hipStream_t)stream, 0, 0);
 }
 
-// How many waves the rules below give a sum: chunk t of 64 columns is added up by wave t % waves, then wave after wave.
-int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used) {
-  const int64_t kc = K / 64;
-  if (group == 128 && r_used > 64 && r_used <= 96 && R % 128 == 0 && R >= 256 && M >= 4096) return 1;
-  if (R % 64 == 0 && (((M + 63) / 64) * (R / 64) >= 160 || ((M + 31) / 32) * (R / 64) >= 256)) return kc % 4 == 0 || kc % 5 != 0 ? 4 : 5;
-  return kc % 8 == 0 || kc % 5 != 0 ? 8 : 5;
-}
+// For launches that bring their shrink along with the sums of its own launch.
+int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used) { return shrink_plan(M, K, R, group, r_used).waves; }
 
 // The shrink, optionally of a layer with a folded LayerNorm (ln_part != nullptr; see ShrinkParams).
 // group / r_used (both 0: nothing known): the R columns are stacked layers of `group` packed rank columns each, of which
@@ -114,19 +136,12 @@ int lora_shrink_ln_launch(const void* x, const void* a_cat, const float* col_sca
   p.x = (const bf16_t*)x; p.a_cat = (const bf16_t*)a_cat; p.col_scale = col_scale; p.t = (bf16_t*)t;
   p.M = (int)M; p.K = (int)K; p.R = (int)R;
   p.ln_part = ln_part; p.ln_ca1 = ln_ca1; p.ln_ca2 = ln_ca2; p.ln_eps = ln_eps;
-  // several stacked layers of rank 96 in 128 on many rows (q / k / v of the 64 x 64 level): one-wave workgroups, each a
-  // 32-row x 96-column tile of one layer over the whole K, five to a CU.  With K this short a tile is a handful of chunks
-  // and its time is load latency, not bytes: more independent workgroups per CU win (16.3 us against 20.8 with the 64 x 64
-  // tiles below at M 8192, K 640, three layers; 64 x 96 tiles of four waves 21.4, 128 x 96 tiles of two waves 25.3, although
-  // both read fewer bytes).  A single layer (R 128) stays with the 64 x 64 tiles: 8.4 us against 13.2.
-  if (group == 128 && r_used > 64 && r_used <= 96 && R % 128 == 0 && R >= 256 && M >= 4096)
-    return launch_shrink<SCfg<1, 1, 3>, 128>(p, s);
-  // the largest output tile that still gives most CUs a workgroup (a 64x64 tile reads half the bytes per output of a 32x64 one)
-  if (R % 64 == 0 && ((M + 63) / 64) * (R / 64) >= 160) return launch_shrink_k<2, 2, 4, 5>(p, s);
-  if (R % 64 == 0 && ((M + 31) / 32) * (R / 64) >= 256) return launch_shrink_k<1, 2, 4, 5>(p, s);
-  // 16 x 16 tiles while they get a CU each (the wave counts are those of the 32 x 32 tiles: the order of the sum)
-  const int grp = group > 0 ? group : (int)R, tiles = (group > 0 && r_used > 0 && r_used < group ? r_used : grp) / 16;
-  if (R % grp == 0 && (M + 15) / 16 * (R / grp) * tiles <= 256)
-    return (K / 64) % 8 == 0 || (K / 64) % 5 != 0 ? launch_shrink16<8>(p, grp, tiles, s) : launch_shrink16<5>(p, grp, tiles, s);
-  return launch_shrink_k<1, 1, 8, 5>(p, s);
+  const ShrinkPlan plan = shrink_plan(M, K, R, group, r_used);
+  switch (plan.tiles) {
+    case GROUP_32x96: return launch_shrink<SCfg<1, 1, 3>, 128>(p, s);
+    case TILE_64x64: return launch_shrink_waves<2, 2>(p, plan.waves, s);
+    case TILE_32x64: return launch_shrink_waves<1, 2>(p, plan.waves, s);
+    case TILE_16x16: return plan.waves == 8 ? launch_shrink16<8>(p, plan.group, plan.used, s) : launch_shrink16<5>(p, plan.group, plan.used, s);
+    default: return launch_shrink_waves<1, 1>(p, plan.waves, s);
+  }
 }
