@@ -827,8 +827,10 @@ static int shrink_beside(LoraGemmParams& p, int form) {
 // convolution that leaves GroupNorm statistics does so per 64 rows.
 //
 // Linear layers: a CU's time is the rows it streams, BM + BN of K columns each, so the tile with the fewest of them whose workgroups fit
-// one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  With adapters, the first that leaves the
-// CUs for 16 x 16 pieces of the shrink; then, where the loop is long enough to hide the larger pieces, for 32 x 32 ones; else two launches.
+// one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  Where the launch is to bring its shrink along,
+// the first that leaves the CUs for 16 x 16 pieces of it; then, where the loop is long enough to hide the larger pieces, for 32 x 32 ones; else two
+// launches.  A T that is given leaves all CUs to the tiles (988 / 1280 / 1280, 64 11.3 us on tiles that leave some -> 10.0, K 5120 35.6 -> 30.7; 700 / 640 /
+// 2560 22.4 -> 11.2): the order of the sums is the same.
 // us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
 // 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
 // 512 / 1280 / 1280, 32 10.1 -> 9.3; 300 / 640 / 640, 64 7.3 -> 6.4; no adapters: 154 / 640 / 2048 12.1 -> 8.3, 655 / 1280 / 2048 12.2 -> 11.1.
@@ -851,7 +853,7 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   struct Tile { int form, bm, bn; };
   constexpr Tile tiles0[] = {{10, 32, 32}, {11, 32, 64}, {12, 64, 64}, {0, 64, 80}, {2, 32, 128}, {3, 64, 128}, {1, 128, 80}};
   constexpr Tile tiles4[] = {{13, 32, 32}, {14, 32, 64}, {15, 64, 64}, {4, 32, 160}, {5, 64, 160}};
-  const bool stats = p.st_part != nullptr, adapters = p.t_ext != nullptr;
+  const bool stats = p.st_part != nullptr, brings = p.t_ext != nullptr && p.a_cat != nullptr && p.R > 0;   // (a T that is given needs no CUs)
   auto first = [&](int piece) {          // piece: the shrink's pieces beside the tiles, 0: none needed
     auto of = [&](const Tile* t, int n, int width) {
       for (; n > 0; ++t, --n) {
@@ -864,7 +866,7 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
     };
     return order == 0 ? of(tiles0, 7, 128) : of(tiles4, 5, 160);
   };
-  if (adapters && p.R > 0) {
+  if (brings) {
     if (const int f = first(16); f >= 0) return f;
     if (p.K >= 1280)
       if (const int f = first(32); f >= 0) return f;
