@@ -828,8 +828,10 @@ static int shrink_beside(LoraGemmParams& p, int form) {
 //
 // Linear layers: a CU's time is the rows it streams, BM + BN of K columns each, so the tile with the fewest of them whose workgroups fit
 // one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  Where the launch is to bring its shrink along,
-// the first that leaves the CUs for 16 x 16 pieces of it; then, where the loop is long enough to hide the larger pieces, for 32 x 32 ones; else two
-// launches.  A T that is given leaves all CUs to the tiles (988 / 1280 / 1280, 64 11.3 us on tiles that leave some -> 10.0, K 5120 35.6 -> 30.7; 700 / 640 /
+// the first that leaves the CUs for 16 x 16 pieces of it; where the loop is long enough to hide the larger pieces, the first that leaves them for
+// 32 x 32 ones if there is no other, or if its loop (us: 3 + 2.9e-5 a row and column of K) and those pieces (8 + 2.3e-3 K) are through before the larger
+// tile's loop (16 / 32: 512 / 1280 / 5120, 96 40.3 / 24.6, 154 21.6 / 20.5, 700 / 640 / 2560, 64 22.4 / 14.1, 400 / 1280 / 2048, 96 16.2 / 12.5; against that 308 / 1280 /
+// 2048, 64 12.0 / 13.3, 512 / 640 / 2560, 64 13.7 / 14.7, 308 / 1280 / 1280, 64 8.4 / 11.3); else two launches.  A T that is given leaves all CUs to the tiles (988 / 1280 / 1280, 64 11.3 us on tiles that leave some -> 10.0, K 5120 35.6 -> 30.7; 700 / 640 /
 // 2560 22.4 -> 11.2): the order of the sums is the same.
 // us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
 // 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
@@ -854,24 +856,28 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   constexpr Tile tiles0[] = {{10, 32, 32}, {11, 32, 64}, {12, 64, 64}, {0, 64, 80}, {2, 32, 128}, {3, 64, 128}, {1, 128, 80}};
   constexpr Tile tiles4[] = {{13, 32, 32}, {14, 32, 64}, {15, 64, 64}, {4, 32, 160}, {5, 64, 160}};
   const bool stats = p.st_part != nullptr, brings = p.t_ext != nullptr && p.a_cat != nullptr && p.R > 0;   // (a T that is given needs no CUs)
-  auto first = [&](int piece) {          // piece: the shrink's pieces beside the tiles, 0: none needed
-    auto of = [&](const Tile* t, int n, int width) {
-      for (; n > 0; ++t, --n) {
-        if (!fits(t->bm, t->bn) || (stats && t->bn != width)) continue;
-        if (piece == 0) return t->form;
-        if (tiles_of(t->bm, t->bn) + pieces_of(piece) > 256) continue;      // (a part of what shrink_beside asks, and much cheaper)
-        if (LoraGemmParams q = p; shrink_beside(q, t->form) == piece) return t->form;
-      }
-      return -1;
-    };
-    return order == 0 ? of(tiles0, 7, 128) : of(tiles4, 5, 160);
+  const Tile* const all = order == 0 ? tiles0 : tiles4;
+  const Tile* const end = all + (order == 0 ? 7 : 5);
+  const int width = order == 0 ? 128 : 160;
+  auto first = [&](int piece, const Tile* stop) {       // piece: the shrink's pieces beside the tiles, 0: none needed
+    for (const Tile* t = all; t != stop; ++t) {
+      if (!fits(t->bm, t->bn) || (stats && t->bn != width)) continue;
+      if (piece == 0) return t;
+      if (tiles_of(t->bm, t->bn) + pieces_of(piece) > 256) continue;      // (a part of what shrink_beside asks, and much cheaper)
+      if (LoraGemmParams q = p; shrink_beside(q, t->form) == piece) return t;
+    }
+    return stop;
   };
   if (brings) {
-    if (const int f = first(16); f >= 0) return f;
-    if (p.K >= 1280)
-      if (const int f = first(32); f >= 0) return f;
+    const Tile* const a = first(16, end);
+    const Tile* const b = p.K >= 1280 ? first(32, a) : a;      // (a smaller tile, if any)
+    auto loop = [&](const Tile* t) { return 3 + 2.9e-5 * p.K * (t->bm + t->bn); };
+    const double pieces = 8 + 2.3e-3 * p.K;
+    if (b != a && (a == end || (loop(b) < loop(a) && pieces < loop(a)))) return b->form;
+    if (a != end) return a->form;
   }
-  return first(0);
+  const Tile* const t = first(0, end);
+  return t != end ? t->form : -1;
 }
 
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {

@@ -434,6 +434,16 @@ def test_few_rows_forms_of_the_dispatch(M, N, K, R, r_used, stats):
     assert ((y - ref).norm() / ref.norm()).item() < 8e-3      # bf16 roundings of T and of the result: 2^-9 each
 
 
+@pytest.mark.parametrize("M,N,K,R,r_used,stats", [(512, 1280, 5120, 128, 96, True), (512, 1280, 5120, 128, 96, False), (154, 1280, 5120, 128, 96, False),
+                                                  (700, 640, 2560, 64, 64, True), (450, 1280, 2048, 128, 96, False), (1536, 640, 2560, 32, 16, False), (308, 1280, 2048, 64, 64, False)])
+def test_few_rows_with_larger_pieces(M, N, K, R, r_used, stats):
+    """Calls on either side of the line between a large tile beside 16 x 16 pieces of the shrink and a smaller one beside 32 x 32 pieces."""
+    from katz_amd import ops
+
+    assert ops._lib.load().kh_lora_linear_split_launches(M, N, K, R, 0, r_used // 16 << 16) == 1
+    test_few_rows_forms_of_the_dispatch(M, N, K, R, r_used, stats)
+
+
 @pytest.mark.parametrize("M,N,K,R,r_used,stats", [(1024, 1280, 1280, 64, 64, False), (1100, 640, 128, 64, 16, True), (3952, 640, 640, 64, 16, True), (4096, 640, 640, 64, 64, False),
                                                   (3968, 640, 64, 64, 16, False), (2048, 1280, 5120, 128, 96, True), (1985, 1280, 1280, 128, 96, False), (1537, 1280, 1280, 128, 128, False)])
 def test_shrink_beside_128x128_tiles(M, N, K, R, r_used, stats):
