@@ -87,6 +87,26 @@ constexpr int KH_FLAG_NO_WAIT = 1 << 24;
 // Weight prefetch of a launch with its own shrink: by the idle waves of the shrink workgroups when the first range is short
 __host__ __device__ inline bool il_prefetch_by_idle_waves(const LoraGemmParams& p) { return p.pf_lines[0] <= ((8u << 20) >> 7); }
 
+// The XCD grid of mt x nt tiles of bm x bn: the one whose per-XCD block of rm x rn tiles touches the fewest operand rows, padding counted as cost.
+struct KhXcdGrid { int gn, rm, rn; };      // XCDs side by side in a row of tiles; the block
+inline KhXcdGrid kh_xcd_grid(int mt, int nt, int bm, int bn) {
+  KhXcdGrid g = {0, 0, 0};
+  double best = 0;
+  for (int gm = 1; gm <= 8; gm *= 2) {
+    const int gn = 8 / gm, rm = (mt + gm - 1) / gm, rn = (nt + gn - 1) / gn;
+    const double cost = ((double)rm * bm + (double)rn * bn) * (8.0 * rm * rn) / ((double)mt * nt);
+    if (g.gn == 0 || cost < best) { best = cost; g = {gn, rm, rn}; }
+  }
+  return g;
+}
+
+// Do `cols` column tiles of T per 64 rows find a CU each beside the 128 x 128 GEMM tiles, on every XCD?  (2304 / 1280 / 1280: 72 pieces and 180 tiles
+// are 252 in all but 9 + 25 on an XCD: a second round, 21.3 us in place of 19.4 with 36 pieces; K 2048 27.4 and 23.4)
+inline bool il_fits_beside(const LoraGemmParams& p, int cols) {
+  const KhXcdGrid g = kh_xcd_grid((p.M + 127) / 128, (p.N + 127) / 128, 128, 128);
+  return ((p.M + 63) / 64 * cols + 7) / 8 + g.rm * g.rn <= 32;
+}
+
 // In-launch shrink on 64 x 32 tiles: a single layer with R = 64 columns of T, or with 128 of which at most the first 96 are
 // in use (two adapters of ranks 64 + 32, say), short enough in K that its GEMM tiles would otherwise wait for T, and
 // small enough in M that the two or three tiles per 64 rows fit beside the GEMM tiles (M 2048 / N 1280 / K 1280, rank 64: 19.2 us on one 64 x 64
@@ -94,8 +114,7 @@ __host__ __device__ inline bool il_prefetch_by_idle_waves(const LoraGemmParams& 
 // Decided on the host: the kernels get the number of column tiles (p.il_cols), more than one per 64 columns of T where they are narrow.
 inline int il_col_tiles(const LoraGemmParams& p) {
   const int narrow = p.ldt != p.R ? 0 : p.R == 64 ? 2 : p.R == 128 && p.r_used > 0 && p.r_used <= 96 ? 3 : 0;
-  const bool fits = (long)((p.M + 127) / 128) * ((p.N + 127) / 128) + (long)((p.M + 63) / 64) * narrow <= 256;
-  return narrow > 0 && p.K <= 2560 && fits ? narrow : p.ldt / 64;
+  return narrow > 0 && p.K <= 2560 && il_fits_beside(p, narrow) ? narrow : p.ldt / 64;
 }
 __device__ __forceinline__ bool il_narrow(const LoraGemmParams& p) { return p.il_cols * 64 > p.ldt; }
 

@@ -725,20 +725,14 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
 #endif
 }
 
-// the tiles of a call and the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
+// the tiles of a call and their XCD grid
 template <class C>
 bool plan_tiles(LoraGemmParams& p, int seg_rows) {
   if (p.N % C::BN != 0 || (p.t_nsplit > 0 && p.t_nsplit % C::BN != 0)) return false;
   p.m_tiles = p.M / seg_rows * ((seg_rows + C::BM - 1) / C::BM);
   p.n_tiles = p.N / C::BN;
-  double best = 0;
-  p.xg_n = 0;
-  for (int gm = 1; gm <= 8; gm *= 2) {
-    const int gn = 8 / gm;
-    const int rm = (p.m_tiles + gm - 1) / gm, rn = (p.n_tiles + gn - 1) / gn;
-    const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
-    if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
-  }
+  const KhXcdGrid g = kh_xcd_grid(p.m_tiles, p.n_tiles, C::BM, C::BN);
+  p.xg_n = g.gn; p.xr_m = g.rm; p.xr_n = g.rn;
   return p.st_part == nullptr || p.n_tiles <= KH_LN_SLOTS;
 }
 

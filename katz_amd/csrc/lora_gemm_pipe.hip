@@ -1124,14 +1124,8 @@ int launch_pcfg(LoraGemmParams p, hipStream_t stream, int n_groups = 1) {
   unsigned grid = (unsigned)(p.m_tiles * p.n_chunks);
   p.xg_n = p.xr_m = p.xr_n = 0;
   if (C::NRT == 0 && !KH_DBG(p, 8)) {
-    // choose the XCD grid whose per-XCD block touches the fewest operand rows, padding counted as cost
-    double best = 0;
-    for (int gm = 1; gm <= 8; gm *= 2) {
-      const int gn = 8 / gm;
-      const int rm = (p.m_tiles + gm - 1) / gm, rn = (p.n_tiles + gn - 1) / gn;
-      const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
-      if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
-    }
+    const KhXcdGrid g = kh_xcd_grid(p.m_tiles, p.n_tiles, C::BM, C::BN);
+    p.xg_n = g.gn; p.xr_m = g.rm; p.xr_n = g.rn;
     grid = 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
   }
   if (p.xa_k != nullptr) {   // cross-attention in the epilogue: the 128x128 / 8-wave tiles only
@@ -1200,6 +1194,10 @@ bool plain_ok(const LoraGemmParams& p) { return p.R == 0 || p.t_ext != nullptr; 
 // query projection with its attention and for columns that are no multiple of 128.  The latter from K 1024 on, where no fine tile smaller than
 // 128 x 80 takes the call (M / N / K, rank, weights from HBM, us in two launches / in one: 2048 / 1216 / 1280, 96 21.0 / 17.9, 2560 38.2 / 31.2, 1024
 // 17.8 / 14.1, 640 14.4 / 16.8; 1024 / 1000 / 1280, 64 20.5 / 17.0; 1536 / 1600 / 1280, 64 18.4 / 17.6; 2048 / 480 / 1280, 64 on 64 x 80 tiles 13.1 / 17.0).
+// Form 3 also takes from form 1 (same bits; form 1 / form 3, weights from HBM) pieces that do not fit beside the tiles on every XCD (2304 / 1280 / 2048, 128
+// 34.8 / 30.1, K 5120 66.3 / 59.4; a transformer block of 2304 rows, rank 128 376 / 359) and loops below 1024 columns on up to half a round of tiles
+// (1024 / 640 / 640, 64 13.8 / 11.7, 1280 / 1280 / 640, 64 14.6 / 13.2).  Not pieces of 64 x 64 in general: alone 2048 / 1280 / 1280, 128 takes 20.6 / 18.4, but form 1
+// hints the next weights better and the step at 768 x 768 with rank 128 19.51 / 19.74 ms.
 static int il_form(const LoraGemmParams& p) {
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
   const long shr = (long)((p.M + 63) / 64) * il_col_tiles(p);
@@ -1210,7 +1208,10 @@ static int il_form(const LoraGemmParams& p) {
   if (!ok) return 0;
   if (tiles <= 192 && tiles + shr <= 256) {
     if (p.xa_k != nullptr) return 3;
-    if (p.N % 128 == 0 && lora_gemm_fine_ok(p)) return 1;
+    if (p.N % 128 == 0 && lora_gemm_fine_ok(p)) {
+      const int cols = il_col_tiles(p);
+      return il_fits_beside(p, cols) && (p.K >= 1024 || tiles > 128) ? 1 : 3;
+    }
     const int fine = p.K >= 1024 ? lora_gemm_pipe_fine_form(p) : 0;
     return fine == -1 || (fine == 1 && !lora_gemm_fine_il_ok(p)) ? 3 : 0;
   }
@@ -1251,14 +1252,8 @@ static int launch_il(const LoraGemmParams& pin, hipStream_t stream) {
   constexpr int LDS_LN = (int)C::LDS_BYTES + KH_LN_LDS > SL ? (int)C::LDS_BYTES + KH_LN_LDS : SL;
   static_assert(LDS_LN <= 160 * 1024, "LDS of one workgroup");
   p.ln_lds = (int)C::LDS_BYTES;
-  double best = 0;
-  p.xg_n = 0;
-  for (int gm = 1; gm <= 8; gm *= 2) {
-    const int gn = 8 / gm;
-    const int rm = (p.m_tiles + gm - 1) / gm, rn = (p.n_tiles + gn - 1) / gn;
-    const double cost = ((double)rm * C::BM + (double)rn * C::BN) * (8.0 * rm * rn) / ((double)p.m_tiles * p.n_tiles);
-    if (p.xg_n == 0 || cost < best) { best = cost; p.xg_n = gn; p.xr_m = rm; p.xr_n = rn; }
-  }
+  const KhXcdGrid g = kh_xcd_grid(p.m_tiles, p.n_tiles, C::BM, C::BN);
+  p.xg_n = g.gn; p.xr_m = g.rm; p.xr_n = g.rn;
   p.il_cols = il_col_tiles(p);
   const int shr = ((p.M + 63) / 64) * p.il_cols;
   p.il_blocks = (shr + 7) / 8 * 8;
