@@ -108,7 +108,8 @@ class GraphedDenoiseStep:
 
     overlap (default on, KATZ_CN_OVERLAP=0 switches it off): inside the graph the ControlNet runs on a second stream
     beside the UNet's down and mid blocks, which do not read its residuals; the UNet waits for it right after its mid
-    block.  Same kernels, same results bit for bit; the 50-step loop at 1024x1024 measured 1769 -> 1610 ms.
+    block.  Same results bit for bit (a ControlNet that has adapters itself: up to the order of its shrinks' sums, which are launches
+    of their own on a second stream); the 50-step loop at 1024x1024 measured 1769 -> 1610 ms.
 
     Build it (and call `run`) from a stream that is neither capturing nor itself a fork inside someone else's capture:
     with overlap on, the capture forks a second stream from the capturing one, and a fork from an already forked stream
@@ -216,8 +217,8 @@ class GraphedDenoiseStep:
     def _models_side_by_side(self, t):
         """The ControlNet on a second stream beside the UNet's down and mid blocks, which do not need its residuals:
         many of either model's launches leave CUs idle (160 tiles on 256 CUs) and every launch has a ramp and a tail.
-        The counter arena is cleared once before the fork and neither forward resets it; the ControlNet's ops take a
-        scratch buffer of their own; the UNet waits for the second stream right after its mid block."""
+        The counter arena is cleared once before the fork and neither forward resets it; the ControlNet's launches take no
+        counters and its ops a scratch buffer of their own; the UNet waits for the second stream right after its mid block."""
         from . import ops
 
         main = torch.cuda.current_stream()
