@@ -273,11 +273,11 @@ int lora_gemm_pipe_launch_sgmv(const LoraGemmParams& p, int n_segments, hipStrea
 int lora_gemm_pipe_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream);
 // Shrink and GEMM in one launch for shapes whose 128x128 tiles leave CUs idle (p.a_cat / col_scale / b_cat set, p.t_ext =
 // scratch for the shrink result, p.il_cnt = counters); KH_ERR_UNSUPPORTED when the shape does not qualify.
-bool lora_gemm_pipe_il_ok(const LoraGemmParams& p);
-int lora_gemm_pipe_launch_il(const LoraGemmParams& p, hipStream_t stream);
+int lora_gemm_pipe_il_form(const LoraGemmParams& p);          // 0: not taken
+int lora_gemm_pipe_launch_il(const LoraGemmParams& p, int form, hipStream_t stream);
 // query projection + cross-attention in its epilogue (xa_k set)
 bool lora_gemm_pipe_xattn_ok(const LoraGemmParams& p);
-int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, hipStream_t stream);
+int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, bool il, hipStream_t stream);     // il: with its shrink (the call has an il form)
 // (32 * row_groups) x 160 tiles whose 8 waves are row_groups x k-slices (lora_gemm_ksplit.hip), tile codes 40 and 41;
 // plain or K-extended GEMM with bias / residual, K % 64 == 0.  row_groups 2 or 4.
 int lora_gemm_ksplit_launch(const LoraGemmParams& p, int row_groups, hipStream_t stream);
@@ -294,11 +294,11 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
 int lora_gemm_pipe_fine_form(const LoraGemmParams& p);
 // Shrink and GEMM in one launch on fine tiles that leave CUs idle (p.a_cat / col_scale / b_cat set, p.t_ext = scratch for the shrink result,
 // p.il_cnt = counters)
-bool lora_gemm_fine_il_ok(LoraGemmParams p);
-int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream);
+int lora_gemm_fine_il_form(LoraGemmParams p);                 // -1: not taken
+int lora_gemm_fine_launch_il(LoraGemmParams p, int form, hipStream_t stream);
 bool lora_gemm_fine_grouped_ok(const LoraGemmParams& p);     // many layers on the same few rows (p.grp)
 int lora_gemm_fine_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream);
-int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream);   // ... on 128 x 128 tiles, for lora_gemm_pipe_il_ok
+int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream);   // ... on 128 x 128 tiles, for lora_gemm_pipe_launch_il
 // how many waves share a sum of the stand-alone shrink of this call (lora_shrink.hip)
 int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used);
 // Shrink and GEMM in one launch on the 128 x 160 tiles, every workgroup computing a piece of T first (p.a_cat / col_scale /

@@ -583,6 +583,29 @@ static LoraGemmParams split_params(const void* x, const void* w, const void* bia
   return p;
 }
 
+// The launch that carries its shrink, where the sizes give the call one (p with counters).
+namespace {
+struct InLaunch {
+  enum Kind { NONE, COOP, PIPE, FINE } kind;
+  int form;
+
+  static InLaunch of(const LoraGemmParams& p) {
+    if (lora_gemm_fine_coop_ok(p)) return {COOP, 0};
+    if (const int form = lora_gemm_pipe_il_form(p); form != 0) return {PIPE, form};
+    if (const int form = lora_gemm_fine_il_form(p); form >= 0) return {FINE, form};
+    return {NONE, 0};
+  }
+  int launch(const LoraGemmParams& p, hipStream_t stream) const {
+    switch (kind) {
+      case COOP: return lora_gemm_fine_launch_coop(p, stream);
+      case PIPE: return lora_gemm_pipe_launch_il(p, form, stream);
+      case FINE: return lora_gemm_fine_launch_il(p, form, stream);
+      default: return KH_ERR_UNSUPPORTED;
+    }
+  }
+};
+}  // namespace
+
 KH_EXPORT int kh_lora_linear_split_launches(int64_t M, int64_t N, int64_t K, int64_t R, int64_t n_split, int flags) {
   if (M <= 0 || N <= 0 || K <= 0 || R <= 0 || M > (1 << 24) || N > (1 << 24) || K > (1 << 24)) return KH_ERR_INVALID_ARG;
   if (n_split < 0 || (n_split > 0 && N % n_split != 0)) return KH_ERR_INVALID_ARG;
@@ -593,7 +616,7 @@ KH_EXPORT int kh_lora_linear_split_launches(int64_t M, int64_t N, int64_t K, int
                                   const_cast<char*>(&dummy), &dummy_counter, nullptr, const_cast<char*>(&dummy), M, N, K, R,
                                   n_split, (flags & 1) != 0);
   p.r_used = ((flags >> 16) & 0xff) * 16;
-  return lora_gemm_fine_coop_ok(p) || lora_gemm_pipe_il_ok(p) || lora_gemm_fine_il_ok(p) ? 1 : 2;
+  return InLaunch::of(p).kind != InLaunch::NONE ? 1 : 2;
 }
 
 KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void* bias, const void* a_cat,
@@ -614,12 +637,13 @@ KH_EXPORT int kh_lora_linear_split_bf16(const void* x, const void* w, const void
   if (!kh_aligned16(x) || !kh_aligned16(w) || !kh_aligned16(y) || !kh_aligned16(a_cat) || !kh_aligned16(b_cat) ||
       !kh_aligned16(t_scratch) || (residual && !kh_aligned16(residual)))
     return KH_ERR_ALIGNMENT;
-  if (counters != nullptr && kh_lora_linear_split_launches(M, N, K, R, n_split, flags) == 1) {
+  if (counters != nullptr && ((flags >> 8) & 0xff) == 0 && (flags & KH_FLAG_NO_WAIT) == 0) {
     LoraGemmParams p = split_params(x, w, bias, a_cat, col_scale, b_cat, t_scratch, counters, residual, y, M, N, K, R, n_split, geglu);
     p.r_used = ((flags >> 16) & 0xff) * 16;
-    kh_take_weight_prefetch(p);
-    if (lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
-    return lora_gemm_pipe_il_ok(p) ? lora_gemm_pipe_launch_il(p, (hipStream_t)stream) : lora_gemm_fine_launch_il(p, (hipStream_t)stream);
+    if (const InLaunch il = InLaunch::of(p); il.kind != InLaunch::NONE) {
+      kh_take_weight_prefetch(p);
+      return il.launch(p, (hipStream_t)stream);
+    }
   }
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, nullptr, nullptr, nullptr, 0.f, (hipStream_t)stream,
                                        (int)R, ((flags >> 16) & 0xff) * 16);
@@ -682,21 +706,20 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
     if (R == 0) { p.ldt = 0; p.t_nsplit = 0; p.il_cnt = nullptr; }
     if (!lora_gemm_pipe_xattn_ok(p)) return KH_ERR_UNSUPPORTED;
     kh_take_weight_prefetch(p);
-    if (R == 0) return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
-    if (may_wait && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
+    if (R == 0) return lora_gemm_pipe_launch_xattn(p, false, (hipStream_t)stream);
+    if (may_wait && lora_gemm_pipe_il_form(p) != 0) return lora_gemm_pipe_launch_xattn(p, true, (hipStream_t)stream);
     const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
     if (rc != KH_OK) return rc;
     p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;
-    return lora_gemm_pipe_launch_xattn(p, (hipStream_t)stream);
+    return lora_gemm_pipe_launch_xattn(p, false, (hipStream_t)stream);
   }
   kh_take_weight_prefetch(p);
   if (R == 0) {
     p.ldt = 0; p.t_nsplit = 0; p.il_cnt = nullptr;
     return lora_gemm_pipe_launch(p, tile_sel, (hipStream_t)stream);
   }
-  if (may_wait && lora_gemm_fine_coop_ok(p)) return lora_gemm_fine_launch_coop(p, (hipStream_t)stream);
-  if (may_wait && lora_gemm_pipe_il_ok(p)) return lora_gemm_pipe_launch_il(p, (hipStream_t)stream);
-  if (may_wait && lora_gemm_fine_il_ok(p)) return lora_gemm_fine_launch_il(p, (hipStream_t)stream);
+  if (may_wait)
+    if (const InLaunch il = InLaunch::of(p); il.kind != InLaunch::NONE) return il.launch(p, (hipStream_t)stream);
   const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
   if (rc != KH_OK) return rc;
   p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;
@@ -744,7 +767,7 @@ KH_EXPORT int kh_lora_linear_xattn_launches(int64_t M, int64_t N, int64_t K, int
                                   &dummy_counter, nullptr, nullptr, M, N, K, R, 0, false);
   p.r_used = ((flags >> 16) & 0xff) * 16;
   p.xa_k = reinterpret_cast<const bf16_t*>(&dummy);
-  return lora_gemm_pipe_il_ok(p) ? 1 : 2;
+  return lora_gemm_pipe_il_form(p) != 0 ? 1 : 2;
 }
 
 // 3x3 convolution, padding 1, NHWC, as an implicit GEMM on the pipelined kernel; see include/katz_hip.h.

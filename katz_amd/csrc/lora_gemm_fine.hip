@@ -933,7 +933,7 @@ int lora_gemm_fine_launch_coop(const LoraGemmParams& p, hipStream_t stream) {
 // Shrink inside the launch (IL): the form of lora_gemm_fine_form, where its tiles leave the CUs.
 // us per call, weights from HBM, two launches -> one: M 154 / N 1280 / K 2048, rank 96 14.9 -> 10.7; 512 / 1280 / 1280, rank 32 12.9 -> 9.3;
 // 512 / 1280 / 5120 30.9 -> 24.0; 988 / 1280 / 1280, rank 16 15.8 -> 12.2 (64 x 80 tiles and two launches 13.7); GEGLU 640 / 10240 / 1280, rank 16 36.3 -> 33.4.
-static int il_form(LoraGemmParams& p) {
+int lora_gemm_fine_il_form(LoraGemmParams p) {
   if (p.a_cat == nullptr || p.col_scale == nullptr || p.il_cnt == nullptr || p.conv_cin > 0) return -1;
   const int form = lora_gemm_pipe_fine_form(p);
   const int piece = shrink_beside(p, form);
@@ -969,7 +969,7 @@ int lora_gemm_fine_launch_grouped(const LoraGemmParams& p, int n_groups, hipStre
          : rows <= 128 ? launch_grouped<128>(p, n_groups, stream) : launch_grouped<160>(p, n_groups, stream);
 }
 
-// Shrink inside the launch, 128 x 128 tiles: the calls of lora_gemm_pipe_il_ok's first kind.  Against the kernel of lora_gemm_pipe.hip, whose eight
+// Shrink inside the launch, 128 x 128 tiles: form 1 of lora_gemm_pipe_il_form.  Against the kernel of lora_gemm_pipe.hip, whose eight
 // waves both moved operands and computed 64 x 32 each, us per call with statistics, rank 96, weights from the memory-side cache / from HBM:
 // 2048 / 1280 / 1280 17.2 -> 16.8 / 20.0 -> 17.7; 2048 / 1280 / 5120 41.5 -> 38.5 / 54.5 -> 43.3; rank 64 without statistics 18.0 -> 16.3 / -.
 int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream) {
@@ -979,8 +979,7 @@ int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream) {
   return launch_fine<C, false, T_IL>(p, stream);
 }
 
-bool lora_gemm_fine_il_ok(LoraGemmParams p) { return il_form(p) >= 0; }
-
-int lora_gemm_fine_launch_il(LoraGemmParams p, hipStream_t stream) {
-  return with_il_tile(il_form(p), [&](auto c) { return launch_fine<decltype(c), false, T_IL>(p, stream); });
+int lora_gemm_fine_launch_il(LoraGemmParams p, int form, hipStream_t stream) {
+  p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
+  return with_il_tile(form, [&](auto c) { return launch_fine<decltype(c), false, T_IL>(p, stream); });
 }

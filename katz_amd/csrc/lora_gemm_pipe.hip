@@ -1198,7 +1198,7 @@ bool plain_ok(const LoraGemmParams& p) { return p.R == 0 || p.t_ext != nullptr; 
 // 34.8 / 30.1, K 5120 66.3 / 59.4; a transformer block of 2304 rows, rank 128 376 / 359) and loops below 1024 columns on up to half a round of tiles
 // (1024 / 640 / 640, 64 13.8 / 11.7, 1280 / 1280 / 640, 64 14.6 / 13.2).  Not pieces of 64 x 64 in general: alone 2048 / 1280 / 1280, 128 takes 20.6 / 18.4, but form 1
 // hints the next weights better and the step at 768 x 768 with rank 128 19.51 / 19.74 ms.
-static int il_form(const LoraGemmParams& p) {
+int lora_gemm_pipe_il_form(const LoraGemmParams& p) {
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
   const long shr = (long)((p.M + 63) / 64) * il_col_tiles(p);
   const bool t_ok = p.t_nsplit == 0 ? p.ldt == p.R : (p.N % p.t_nsplit == 0 && p.ldt == (p.N / p.t_nsplit) * p.R && p.t_nsplit % 128 == 0);
@@ -1213,13 +1213,11 @@ static int il_form(const LoraGemmParams& p) {
       return il_fits_beside(p, cols) && (p.K >= 1024 || tiles > 128) ? 1 : 3;
     }
     const int fine = p.K >= 1024 ? lora_gemm_pipe_fine_form(p) : 0;
-    return fine == -1 || (fine == 1 && !lora_gemm_fine_il_ok(p)) ? 3 : 0;
+    return fine == -1 || (fine == 1 && lora_gemm_fine_il_form(p) < 0) ? 3 : 0;
   }
   if (tiles >= 480 && p.K >= 1024 && (long)((p.M + 255) / 256) * ((p.N + 127) / 128) <= 256 && shr <= 256) return 2;
   return 0;
 }
-
-bool lora_gemm_pipe_il_ok(const LoraGemmParams& p) { return il_form(p) != 0; }
 
 // See include/katz_hip.h.  Synchronous (a blocking 4-byte copy on the null stream of the current device).
 KH_EXPORT int kh_lora_split_timeouts(int32_t* count, int clear) {
@@ -1289,8 +1287,8 @@ static int launch_il(const LoraGemmParams& pin, hipStream_t stream) {
   KH_RETURN_LAST_ERROR();
 }
 
-int lora_gemm_pipe_launch_il(const LoraGemmParams& p, hipStream_t stream) {
-  switch (il_form(p)) {
+int lora_gemm_pipe_launch_il(const LoraGemmParams& p, int form, hipStream_t stream) {
+  switch (form) {
     case 1: return lora_gemm_fine_launch_il128(p, stream);
     case 2: return launch_il<PCfg<256, 128, 4, 2, 0, 3, 64>>(p, stream);
     case 3: return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
@@ -1306,9 +1304,9 @@ bool lora_gemm_pipe_xattn_ok(const LoraGemmParams& p) {
          p.M % p.xa_T == 0 && p.xa_S >= 1 && p.xa_S <= 96 && !p.geglu && p.res == nullptr && p.st_part == nullptr;
 }
 
-int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, hipStream_t stream) {
+int lora_gemm_pipe_launch_xattn(const LoraGemmParams& p, bool il, hipStream_t stream) {
   if (p.xa_k == nullptr || !lora_gemm_pipe_xattn_ok(p)) return KH_ERR_UNSUPPORTED;
-  if (p.a_cat != nullptr && p.il_cnt != nullptr && il_form(p) == 3) return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
+  if (il) return launch_il<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
   return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>>(p, stream);
 }
 
