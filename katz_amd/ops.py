@@ -323,10 +323,10 @@ _split_new = threading.Lock()
 _capturing = torch._C._cuda_isCurrentStreamCapturing if hasattr(torch._C, "_cuda_isCurrentStreamCapturing") else lambda: False
 
 
-def _capture_id() -> int:
-    """The capture the current stream is part of."""
+def _capture_id(stream: Optional[int] = None) -> int:
+    """The capture this stream (the current one) is part of, 0: none."""
     n = ctypes.c_uint64(0)
-    _lib.check(_lib.load().kh_stream_capture_id(_stream(), ctypes.byref(n)), "kh_stream_capture_id")
+    _lib.check(_lib.load().kh_stream_capture_id(_stream() if stream is None else stream, ctypes.byref(n)), "kh_stream_capture_id")
     return n.value
 
 
@@ -348,7 +348,8 @@ def _owns(st: _Counters, stream: int) -> bool:
     """Does the eager arena belong to the current stream, or can it (nothing is left of what its owner enqueued)?"""
     if st.owner == stream:
         return True
-    if st.stream is not None and not st.stream.query():
+    # (a stream that another thread is capturing must not be queried: that would end the capture)
+    if st.stream is not None and (_capture_id(st.owner) or not st.stream.query()):
         return False
     st.owner, st.stream = stream, torch.cuda.current_stream()
     return True
@@ -437,7 +438,7 @@ def claim_waits(device) -> None:
         stream = _stream()
         if st.owner != stream:
             current = torch.cuda.current_stream()
-            if st.stream is not None:
+            if st.stream is not None and not _capture_id(st.owner):      # (a capture runs nothing, and begins on a device at rest)
                 current.wait_stream(st.stream)
             st.owner, st.stream = stream, current
 

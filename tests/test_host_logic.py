@@ -644,6 +644,7 @@ class _FakeStreams:
             self.owner, self.handle, self.waited = owner, handle, []
 
         def query(self):
+            assert self.handle not in self.owner.captured
             return self.handle not in self.owner.busy
 
         def wait_stream(self, other):
@@ -653,12 +654,12 @@ class _FakeStreams:
         import torch
         from katz_amd import ops
 
-        self.current, self.capture, self.busy = 1, 0, set()
+        self.current, self.capture, self.busy, self.captured = 1, 0, set(), set()
         self.streams = {h: self.Stream(self, h) for h in range(1, 9)}
         monkeypatch.setattr(ops, "_split_counters", {})
         monkeypatch.setattr(ops, "_stream", lambda: self.current)
         monkeypatch.setattr(ops, "_capturing", lambda: self.capture != 0)
-        monkeypatch.setattr(ops, "_capture_id", lambda: self.capture)
+        monkeypatch.setattr(ops, "_capture_id", lambda h=None: self.capture if h is None else int(h in self.captured))
         monkeypatch.setattr(torch.cuda, "current_stream", lambda: self.streams[self.current])
 
     def take(self, n=4):
@@ -703,6 +704,10 @@ def test_counters_belong_to_one_stream_at_a_time(monkeypatch):
         assert f.take() is None
         ops.split_counters_reset(dev)
     assert st.eager.pos == 4
+    f.captured, f.current = {1}, 2                       # another thread captures on the owner: it is left alone
+    assert f.take() is None
+    f.captured = set()
+    assert f.take() == (0, 4)
 
 
 def test_graphs_take_counters_only_behind_their_own_reset(monkeypatch):
