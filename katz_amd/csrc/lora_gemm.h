@@ -298,6 +298,9 @@ int lora_gemm_fine_il_form(LoraGemmParams p);                 // -1: not taken
 int lora_gemm_fine_launch_il(LoraGemmParams p, int form, hipStream_t stream);
 bool lora_gemm_fine_grouped_ok(const LoraGemmParams& p);     // many layers on the same few rows (p.grp)
 int lora_gemm_fine_launch_grouped(const LoraGemmParams& p, int n_groups, hipStream_t stream);
+// a query projection with its cross-attention: 1 or 2 launches, 0 where lora_gemm_pipe_launch_xattn takes it; two launches: the second, T given
+int lora_gemm_fine_xattn_launches(const LoraGemmParams& p, bool may_wait);
+int lora_gemm_fine_launch_xattn(const LoraGemmParams& p, bool may_wait, hipStream_t stream);
 int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream);   // ... on 128 x 128 tiles, for lora_gemm_pipe_launch_il
 // how many waves share a sum of the stand-alone shrink of this call (lora_shrink.hip)
 int lora_shrink_waves(int64_t M, int64_t K, int64_t R, int group, int r_used);

@@ -661,6 +661,12 @@ struct XAttnArgs {   // the attention behind a query projection (kh_lora_linear_
 };
 }  // namespace
 
+// Does the launch of a query projection with its attention bring its shrink along?  (p with counters)
+static bool xattn_one_launch(const LoraGemmParams& p) {
+  const int n = lora_gemm_fine_xattn_launches(p, true);
+  return n == 0 ? lora_gemm_pipe_il_form(p) != 0 : n == 1;
+}
+
 static int lora_linear_norm_impl(const void* x, const void* w, const void* bias, const void* a_cat,
                                  const float* col_scale, const void* b_cat, void* t_scratch, int32_t* counters,
                                  const void* residual, void* y, const float* ln_part, const float* ln_c1,
@@ -706,12 +712,16 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
     if (R == 0) { p.ldt = 0; p.t_nsplit = 0; p.il_cnt = nullptr; }
     if (!lora_gemm_pipe_xattn_ok(p)) return KH_ERR_UNSUPPORTED;
     kh_take_weight_prefetch(p);
-    if (R == 0) return lora_gemm_pipe_launch_xattn(p, false, (hipStream_t)stream);
-    if (may_wait && lora_gemm_pipe_il_form(p) != 0) return lora_gemm_pipe_launch_xattn(p, true, (hipStream_t)stream);
+    const auto go = [&](bool waits) {   // (pieces of T that do not fit beside the tiles, operands of 2 GiB: the kernel of lora_gemm_pipe.hip)
+      return lora_gemm_fine_xattn_launches(p, waits) != 0 ? lora_gemm_fine_launch_xattn(p, waits, (hipStream_t)stream)
+                                                          : lora_gemm_pipe_launch_xattn(p, waits, (hipStream_t)stream);
+    };
+    if (R == 0) return go(false);
+    if (may_wait && xattn_one_launch(p)) return go(true);
     const int rc = lora_shrink_ln_launch(x, a_cat, col_scale, t_scratch, M, K, RT, ln_part, ln_ca1, ln_ca2, ln_eps, (hipStream_t)stream, (int)R, p.r_used);
     if (rc != KH_OK) return rc;
     p.a_cat = nullptr; p.col_scale = nullptr; p.il_cnt = nullptr;
-    return lora_gemm_pipe_launch_xattn(p, false, (hipStream_t)stream);
+    return go(false);
   }
   kh_take_weight_prefetch(p);
   if (R == 0) {
@@ -767,7 +777,7 @@ KH_EXPORT int kh_lora_linear_xattn_launches(int64_t M, int64_t N, int64_t K, int
                                   &dummy_counter, nullptr, nullptr, M, N, K, R, 0, false);
   p.r_used = ((flags >> 16) & 0xff) * 16;
   p.xa_k = reinterpret_cast<const bf16_t*>(&dummy);
-  return lora_gemm_pipe_il_form(p) != 0 ? 1 : 2;
+  return xattn_one_launch(p) ? 1 : 2;
 }
 
 // 3x3 convolution, padding 1, NHWC, as an implicit GEMM on the pipelined kernel; see include/katz_hip.h.

@@ -23,6 +23,7 @@
 #include "kh_common.h"
 #include "lora_gemm.h"
 #include "lora_shrink_tile.h"
+#include "xattn_tile.h"
 
 // Bounded waits of the cooperative shrink that have run out on this GPU; read (and cleared) by kh_lora_split_timeouts
 // together with the count of the in-launch shrink of lora_gemm_pipe.hip.
@@ -116,7 +117,10 @@ enum { T_GIVEN = 0, T_COOP = 1, T_IL = 2, T_GRP = 3 };
 using ILTileWide = SCfg<4, 2, 2>;               // the pieces beside 128 x 128 tiles: 64 x 64 ...
 using ILTileNarrow = SCfg<4, 2, 1>;             // ... and 64 x 32 (il_narrow)
 constexpr int il_lds(int waves) { return waves == 8 ? cmax(SHRINK16_LDS<8>, SCfg<8, 1, 1, 2>::LDS) : cmax(SHRINK16_LDS<5>, SCfg<5, 1, 1, 3>::LDS); }
-template <class C, bool CONV, int TMODE>
+//
+// XA: the layer is an attention's to_q; a tile's rows are queries of one sample, its columns whole heads, and the epilogue runs the cross-attention on
+// them (xattn_tile.h).
+template <class C, bool CONV, int TMODE, bool XA = false>
 __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p0, const int seg_rows, const int seg_tiles) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -393,6 +397,8 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   float* sc1 = sRs + 128;
   float* sc2 = sc1 + BN;
   static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && (BM <= 128 || GRP), "per-row and per-column terms");
+  typedef XAttnFine<cmax(BN / 64, 1), 256, C::LDC> XAttn;
+  XAttn kv;                                            // XA: the keys and values, in the producers
   if (producer) {
     // requested now, used after the K loop (older than every DMA load, so no wait falls in between)
     constexpr int CP = (BN + 255) / 256;
@@ -401,6 +407,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     float c1v[CP], c2v[CP];
     uint16_t biasv[CP];
     if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, M, ptid);
+    if constexpr (XA) kv.load(p, m0, n0, ptid);
 #pragma unroll
     for (int c = 0; c < CP; ++c) {
       const int col = n0 + (ptid + 256 * c < BN ? ptid + 256 * c : 0);
@@ -547,6 +554,8 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     }
   }
   __syncthreads();   // the ring is dead: partial sums and the staging tiles reuse it
+  if constexpr (XA)
+    if (producer) kv.store(smem + (C::TAIL + 15) / 16 * 16, tid - 256);
 
   // the k-slices meet in LDS: every wave leaves all its tiles and finishes every WK-th of them
   f32x4* part = reinterpret_cast<f32x4*>(smem);
@@ -609,6 +618,12 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     }
   }
   __syncthreads();
+  if constexpr (XA) {
+    static_assert(C::WK == 1 && !C::GLU && !CONV && BN % 64 == 0 && C::LDC % 8 == 0 && (C::TAIL + 15) / 16 * 16 + XAttn::LDS_BYTES <= C::LDS, "cross-attention");
+    static_assert(BN / 64 * (BM / 32) <= 8, "a wave per 32 queries of a head");
+    if (wave < BN / 64 * (BM / 32)) XAttn::unit(p, sC, smem + (C::TAIL + 15) / 16 * 16, wave / (BM / 32), wave % (BM / 32), m0, n0, lane);
+    return;
+  }
   if constexpr (C::GLU) {
     // staged columns come in groups of 64 = 32 value columns then their 32 gate columns
     constexpr int OPR = BN / 16, GCH = (BM * OPR + 511) / 512;
@@ -750,15 +765,15 @@ bool plan_il(LoraGemmParams& p) {
   return false;
 }
 
-template <class C, bool CONV, int TMODE = T_GIVEN>
+template <class C, bool CONV, int TMODE = T_GIVEN, bool XA = false>
 int launch_fine(LoraGemmParams p, hipStream_t stream) {
   const int seg_rows = CONV && p.gn_part != nullptr ? p.conv_ho * p.conv_wo : p.M;
   if (!plan_tiles<C>(p, seg_rows)) return KH_ERR_UNSUPPORTED;
   if constexpr (TMODE == T_IL && !(C::BM == 128 && C::BN == 128))
     if (!plan_il<C>(p)) return KH_ERR_UNSUPPORTED;
-  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, TMODE>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
+  if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, TMODE, XA>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
   const unsigned grid = (unsigned)(TMODE == T_IL ? p.il_blocks : 0) + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, TMODE>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
+  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, TMODE, XA>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
             seg_rows, (seg_rows + C::BM - 1) / C::BM);
   KH_RETURN_LAST_ERROR();
 }
@@ -982,4 +997,70 @@ int lora_gemm_fine_launch_il128(LoraGemmParams p, hipStream_t stream) {
 int lora_gemm_fine_launch_il(LoraGemmParams p, int form, hipStream_t stream) {
   p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
   return with_il_tile(form, [&](auto c) { return launch_fine<decltype(c), false, T_IL>(p, stream); });
+}
+
+// A query projection with its cross-attention in the epilogue (the shapes of lora_gemm_pipe_xattn_ok: whole 128-row and 128-column tiles, samples of
+// whole 128-row tiles).  Fewer than 1024 rows: the tile of the projection alone, by the rule of the forms, with the shrink beside it where 16 x 16
+// pieces find CUs; else 128 x 128.  Bound by the operand stream like the projection alone; the attention adds 1 to 2 us at the end.  Against 128 x 128
+// tiles whose eight waves both move operands and compute (lora_gemm_pipe.hip) and, below 1024 rows, a shrink in a launch of its own, us per call, weights
+// from HBM, 77 keys: 512 / 1280 / 1280, rank 32 of 64 24.7 -> 11.3, rank 64 25.6 -> 16.1, without adapters 20.6 -> 11.2; 256 / 640 / 640, 16 18.0 -> 9.2;
+// 768 / 1280 / 1280, 48 25.4 -> 15.0; 896, 64 26.0 -> 19.2; 1024, 16 23.0 -> 21.3; 1536, 32 23.1 -> 19.8; 2048, rank 96 24.0 -> 19.2, without 21.4 -> 19.0.
+// Same bits.  Pieces of T that do not fit beside the tiles on every XCD stay there (2304 / 1280 / 1280, 128 26.8).
+namespace {
+template <class F>
+int with_xattn_tile(int form, F f) {
+  switch (form) {
+    case 2: return f(FCfg<32, 128, 0>{});
+    case 3: return f(FCfg<64, 128, 0>{});
+    case 11: return f(FCfg<32, 64, 0>{});
+    case 12: return f(FCfg<64, 64, 0>{});
+    default: return f(FCfg<128, 128, 0>{});
+  }
+}
+
+// the projection alone, as the rule of the forms sees it
+LoraGemmParams xattn_projection(const LoraGemmParams& p) {
+  LoraGemmParams q = p;
+  q.xa_k = nullptr;
+  return q;
+}
+
+// form and whether it brings the shrink; form -1: lora_gemm_pipe.hip's tiles
+struct XAttnForm { int form; bool il; };
+XAttnForm xattn_form(const LoraGemmParams& p, bool may_wait) {
+  LoraGemmParams q = xattn_projection(p);
+  if (!lora_gemm_fine_ok(q)) return {-1, false};
+  const bool brings = may_wait && q.R > 0 && q.a_cat != nullptr && q.il_cnt != nullptr;
+  if (brings && lora_gemm_pipe_il_form(p) != 0) return il_fits_beside(q, il_col_tiles(q)) ? XAttnForm{16, true} : XAttnForm{-1, false};
+  if (q.M >= 1024) return {16, false};
+  // whole heads: the forms of 64 and 128 columns in the order of their operand rows
+  for (const int piece : {16, 0}) {
+    if (piece != 0 && !brings) continue;
+    for (const int form : {11, 12, 2, 3}) {
+      const int bm = form == 2 || form == 11 ? 32 : 64, bn = form == 2 || form == 3 ? 128 : 64;
+      if ((long)(q.M / bm) * (q.N / bn) > 256) continue;
+      if (piece == 0 || shrink_beside(q, form) == piece) return {form, piece != 0};
+    }
+  }
+  return {16, false};
+}
+}  // namespace
+
+int lora_gemm_fine_xattn_launches(const LoraGemmParams& p, bool may_wait) {
+  const XAttnForm f = xattn_form(p, may_wait);
+  return f.form < 0 ? 0 : p.R == 0 || f.il ? 1 : 2;
+}
+
+int lora_gemm_fine_launch_xattn(const LoraGemmParams& pin, bool may_wait, hipStream_t stream) {
+  const XAttnForm f = xattn_form(pin, may_wait);
+  if (f.form < 0) return KH_ERR_UNSUPPORTED;
+  LoraGemmParams p = pin;
+  if (!f.il) return with_xattn_tile(f.form, [&](auto c) { return launch_fine<decltype(c), false, T_GIVEN, true>(p, stream); });
+  if (f.form == 16) {
+    p.il_cols = il_col_tiles(p);
+    p.il_blocks = ((p.M + 63) / 64 * p.il_cols + 7) / 8 * 8;
+  } else {
+    p.il_waves = lora_shrink_waves(p.M, p.K, p.ldt, p.R, p.r_used);
+  }
+  return with_xattn_tile(f.form, [&](auto c) { return launch_fine<decltype(c), false, T_IL, true>(p, stream); });
 }

@@ -223,3 +223,35 @@ def test_transformer_with_and_without_the_fused_attention(monkeypatch, adapters)
     say(f"  cosine against the oracle: fused {c1:.6f}, separate {c0:.6f}; fused against separate {c10:.6f}")
     assert c1 >= 0.9995 and c0 >= 0.9995 and c10 >= 0.9995
     assert_close_rel(y1, ref, 6e-2, "transformer with the attention inside the query projection")
+
+
+@pytest.mark.parametrize("B,T,heads,K,R,used", [
+    (2, 256, 20, 1280, 64, 32),     # 64 x 64 tiles, 16 x 16 pieces of T beside them
+    (2, 256, 20, 1280, 128, 128),   # no CUs for the pieces: two launches
+    (1, 128, 2, 64, 64, 16),        # 32 x 64 tiles, a loop of one stage
+    (1, 768, 20, 1280, 64, 64),     # 64 x 128 tiles
+    (1, 256, 20, 1280, 0, 0),       # 32 x 64 tiles, no adapters
+    (7, 128, 20, 320, 128, 96),     # 896 rows
+    (1, 1024, 20, 1280, 64, 16),    # 128 x 128 tiles
+])
+def test_few_queries_on_small_tiles(B, T, heads, K, R, used):
+    """Tiles below 128 x 128: against the oracle; the shrink beside them gives the bits of two launches, and rows that a larger batch computes on other tiles
+    are the same."""
+    from katz_amd import ops
+    say("xattn, small tiles", B, T, heads, K, R, used)
+    d, S = dev(), 77
+    x, w, k, v, A, Bm = _case(B, T, heads, K, S, R, seed=B + T + K + R)
+    kw = {}
+    if R:
+        A[used:], Bm[:, used:] = 0, 0
+        kw = dict(a_cat=A.to(d, BF), col_scale=torch.full((R,), 0.6, device=d), b_cat=Bm.to(d, BF), r_used=used)
+    xd, wd, kd, vd = (t.to(d, BF) for t in (x, w, k, v))
+    o = ops.lora_linear_xattn(xd, wd, kd, vd, heads, **kw)
+    assert_close_rel(o, _ref(x, w, k, v, heads, A, Bm, 0.6), CHAIN_TOL, "projection + attention on small tiles")
+    if R and B * T < 1024:      # (from there on the shrink beside the tiles deals its chunks to other waves than its own launch does)
+        assert torch.equal(o, ops.lora_linear_xattn(xd, wd, kd, vd, heads, two_launches=True, **kw))
+    n = 2048 // (B * T)
+    if not R and n > 1:
+        more = ops.lora_linear_xattn(*(t.repeat(n, 1, 1) if t.dim() == 3 else t for t in (xd, wd, kd, vd)), heads)
+        assert torch.equal(o, more[:B]) and torch.equal(o, more[-B:])
+    ops.check_split_timeouts()
