@@ -1000,10 +1000,10 @@ int lora_gemm_fine_launch_il(LoraGemmParams p, int form, hipStream_t stream) {
 }
 
 // A query projection with its cross-attention in the epilogue (the shapes of lora_gemm_pipe_xattn_ok: whole 128-row and 128-column tiles, samples of
-// whole 128-row tiles).  Fewer than 1024 rows: the tile of the projection alone, by the rule of the forms, with the shrink beside it where 16 x 16
+// whole 128-row tiles).  Fewer than 1024 rows: the tile of the projection alone, with the shrink beside it where 16 x 16
 // pieces find CUs; else 128 x 128.  Bound by the operand stream like the projection alone; the attention adds 1 to 2 us at the end.  Against 128 x 128
 // tiles whose eight waves both move operands and compute (lora_gemm_pipe.hip) and, below 1024 rows, a shrink in a launch of its own, us per call, weights
-// from HBM, 77 keys: 512 / 1280 / 1280, rank 32 of 64 24.7 -> 11.3, rank 64 25.6 -> 16.1, without adapters 20.6 -> 11.2; 256 / 640 / 640, 16 18.0 -> 9.2;
+// from HBM, 77 keys: 512 / 1280 / 1280, rank 32 of 64 24.7 -> 11.3, rank 64 25.6 -> 15.1, without adapters 20.6 -> 11.2; 256 / 640 / 640, 16 18.0 -> 9.2;
 // 768 / 1280 / 1280, 48 25.4 -> 15.0; 896, 64 26.0 -> 19.2; 1024, 16 23.0 -> 21.3; 1536, 32 23.1 -> 19.8; 2048, rank 96 24.0 -> 19.2, without 21.4 -> 19.0.
 // Same bits.  Pieces of T that do not fit beside the tiles on every XCD stay there (2304 / 1280 / 1280, 128 26.8).
 namespace {
@@ -1033,14 +1033,10 @@ XAttnForm xattn_form(const LoraGemmParams& p, bool may_wait) {
   const bool brings = may_wait && q.R > 0 && q.a_cat != nullptr && q.il_cnt != nullptr;
   if (brings && lora_gemm_pipe_il_form(p) != 0) return il_fits_beside(q, il_col_tiles(q)) ? XAttnForm{16, true} : XAttnForm{-1, false};
   if (q.M >= 1024) return {16, false};
-  // whole heads: the forms of 64 and 128 columns in the order of their operand rows
-  for (const int piece : {16, 0}) {
-    if (piece != 0 && !brings) continue;
-    for (const int form : {11, 12, 2, 3}) {
-      const int bm = form == 2 || form == 11 ? 32 : 64, bn = form == 2 || form == 3 ? 128 : 64;
-      if ((long)(q.M / bm) * (q.N / bn) > 256) continue;
-      if (piece == 0 || shrink_beside(q, form) == piece) return {form, piece != 0};
-    }
+  // whole heads: the first of 64 and 128 columns in the order of their operand rows
+  for (const int form : {11, 12, 2, 3}) {
+    const int bm = form == 2 || form == 11 ? 32 : 64, bn = form == 2 || form == 3 ? 128 : 64;
+    if ((long)(q.M / bm) * (q.N / bn) <= 256) return {form, brings && shrink_beside(q, form) == 16};
   }
   return {16, false};
 }
