@@ -152,15 +152,18 @@ __device__ __forceinline__ void kh_prefetch_lines(const void* const (&pf)[3], co
 // taking lines i, i + n, ... (loaded like the hint above: into LDS nobody reads).  The workgroups of an XCD that share the block take
 // a share each.  Without it all of them meet the same cold lines at the same time, and a CU takes about 55 GB/s of lines that come from
 // memory, 110 GB/s of lines its L2 has.
+// NC: nc's largest value where that is known, so that a line's row and column come without a division.
+template <int NC = 0>
 __device__ __forceinline__ void kh_touch_rows(const bf16_t* w, int N, int K, int row0, int rows, int c0, int nc, char* wave_lds, int i, int n) {
 #if __HIP_DEVICE_COMPILE__
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(w), 0, (int)((size_t)N * K * 2), 0x00020000);
   if (row0 + rows > N) rows = N - row0;
   if (64 * (c0 + nc) > K) nc = K / 64 - c0;
-  for (int l = i; l < rows * nc; l += n) {
-    const int r = l / nc;
+  const int per = NC > 0 ? NC : nc;
+  for (int l = i; l < rows * per; l += n) {
+    const int r = l / per, c = l - r * per;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)wave_lds, 4,
-                                             (uint32_t)(row0 + r) * (uint32_t)K * 2u + (uint32_t)(c0 + l - r * nc) * 128u, 0, 0, 0);
+                                             c < nc ? (uint32_t)(row0 + r) * (uint32_t)K * 2u + (uint32_t)(c0 + c) * 128u : 0xFFFFFFFFu, 0, 0, 0);
   }
 #endif
 }

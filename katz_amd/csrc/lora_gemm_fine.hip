@@ -68,9 +68,11 @@ struct FCfg {
   // computing waves: WM row groups x WN column groups x WK k-slices
   static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
                        WM = 4 / (WK * WN);
-  // 32-row MFMA tiles for the slices where the tile divides into them (16x16x16 has half the rate), 16-row tiles otherwise
-  static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
-  static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN), KS = ORD == 4 ? 1 : 2;   // a wave's MFMA tiles, its k-steps per stage
+  // 32-row MFMA tiles for the slices where the tile divides into them, and for GEGLU on 128 rows, whose 160 accumulators leave no room for a 32-column
+  // step of 16-row fragments (72 registers against 36: 56 spilled); 16-row tiles otherwise (16x16x16 has half the rate)
+  static constexpr int MF = (ORD != 0 && BN % 32 == 0) || (GLU && BM == 128) ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
+  static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN);                           // a wave's MFMA tiles
+  static constexpr int KS = ORD == 4 ? 1 : ORD == 0 && MF == 32 ? 4 : 2;                   // its k-steps per stage
   // operand order of the matrix instructions: (W, x) leaves four columns of a row in a lane, so that the epilogue writes 8 bytes at a time
   // (128 x 320: 5.6 K clocks against 8.4 K), (x, W) four rows of a column.  One x fragment per W fragment is the exception: the K loop of 64 x 80
   // takes 8.8 K clocks with (x, W) and 9.9 K with (W, x), more than the epilogue saves.
@@ -88,6 +90,7 @@ struct FCfg {
   static constexpr int NST = cmin(16, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;  // as many stages as fit, but at most 16
   static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + 1024;   // (where prefetched dwords nobody reads land)
   static constexpr int OPC = BM * (BN / 8), OPT = (OPC + 511) / 512;             // 16-byte output pieces: per tile, per thread
+  static_assert(ORD != 4 || MF == 32 || KS == 1, "k-steps");
   static_assert(WM * WN * WK == 4 && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
   static_assert(BM % 32 == 0 && XQ * UR * 4 == BM && ROWS % UR == 0, "whole DMA instructions");
   static_assert(NST >= 2 && LPS_HI * (PD - 1) < 63 && LDS + KH_LN_LDS <= 160 * 1024, "ring");
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
         const int xcd = (int)blockIdx.x & 7, wgs = (gx * ct - xcd + 7) / 8, KT1 = p.K / BK;
         char* lds = smem + C::TOUCH_OFF + (wave - 4) * 256;
         auto touch = [&](int t) {
-          kh_touch_rows(p.w, p.N, p.K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, 8, lds, ((int)blockIdx.x >> 3) * 256 + tid - 256, wgs * 256);
+          kh_touch_rows<8>(p.w, p.N, p.K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, 8, lds, ((int)blockIdx.x >> 3) * 256 + tid - 256, wgs * 256);
         };
         __builtin_amdgcn_s_sleep(127);                       // 8128 clocks, about 10 stages of the K loop
         const bool hints = il_prefetch_by_idle_waves(p);
@@ -239,112 +242,8 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     if (tid == 0) __hip_atomic_fetch_add(p.il_cnt + m_blk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
-  // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row): 16 rows at one piece fill the 64 banks.
+  // of a stage row, the piece that a 16-byte piece is stored as: 16 rows at one piece fill the 64 banks
   auto swz = [](int row) { return (PPR == 8 ? row >> 1 : row) & (PPR - 1); };
-  constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
-  uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
-  int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
-#pragma unroll
-  for (int q = 0; q < LPS_HI; ++q) {
-    int u = pw + 4 * q;
-    u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
-    const int r = u * UR + lane / PPR;
-    const uint32_t pcb = (uint32_t)(((lane % PPR) ^ swz(r)) * 16);
-    if (CONV && q < XQ) {
-      int row = m0 + r; row = row < M ? row : M - 1;
-      const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
-      const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
-      int mask = 0;
-#pragma unroll
-      for (int tap = 0; tap < 9; ++tap) {
-        const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
-        mask |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
-      }
-      tapmask[q < XQ ? q : 0] = mask;
-      // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
-      voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
-    } else if (q < XQ) {
-      voff[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + pcb;        // rows past M lie beyond the buffer: zeros
-    } else {
-      voff[q] = (uint32_t)(n0 + r - BM) * (uint32_t)K * 2u + pcb;
-    }
-    if (EXT && p.t_ext != nullptr)
-      voff2[q] = q < XQ ? ((uint32_t)(m0 + r) * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb
-                        : (uint32_t)(n0 + r - BM) * (uint32_t)p.R * 2u + pcb;
-  }
-  const size_t x_bytes = CONV ? (size_t)(M / (p.conv_ho * p.conv_wo)) * p.conv_h * p.conv_w * p.conv_cin * 2 : (size_t)M * K * 2;
-  const size_t x_lead = CONV ? (size_t)(p.conv_w + 1) * p.conv_cin * 2 : 0;
-  const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.x) - x_lead), 0,
-                                                         (int)(x_bytes + x_lead), 0x00020000);
-  const rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w), 0, (int)((size_t)N * K * 2), 0x00020000);
-  const bool has_t = EXT && p.t_ext != nullptr;
-  const rsrc_t rs_t = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.t_ext : p.x), 0,
-                                                         has_t ? (int)((size_t)M * p.ldt * 2) : 0, 0x00020000);
-  const rsrc_t rs_bx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.b_cat : p.w), 0,
-                                                          has_t ? (int)((size_t)N * p.R * 2) : 0, 0x00020000);
-  // CONV: K tiles are requested in order, so the tap and the channel offset of the next request are running scalars
-  int cv_tap = 0, cv_kw = 0, cv_c0 = 0, cv_shift = 0, cv_row = 0;
-  uint32_t xvo[XQ];
-#pragma unroll
-  for (int q = 0; q < XQ; ++q) xvo[q] = (!CONV || (tapmask[CONV ? q : 0] & 1)) ? voff[q] : OOB;
-  auto issue = [&](int t, int st) {                    // K tile t into the ring stage at byte offset st
-    char* stage = smem + st;
-    const int so = t * ROWB;
-    if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
-      if ((COOP || TMODE == T_IL) && t == KT1) {
-        // first request for T: wait (bounded) until every workgroup of these 128 rows has delivered its piece
-        if (lane == 0) {
-          int it = 0, want = p.n_tiles;
-          if (TMODE == T_IL) {
-            const int left = M - m0 / 128 * 128;
-            if (BM == 128 && BN == 128) want = ((left < 128 ? left : 128) + 63) / 64 * p.il_cols;
-            else want = ((left < 128 ? left : 128) + p.il_tile - 1) / p.il_tile * ((r_ext + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
-          }
-          while (__hip_atomic_load(p.il_cnt + m0 / 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want && ++it < (1 << 20))
-            __builtin_amdgcn_s_sleep(8);
-          if (it >= (1 << 20)) {
-            __hip_atomic_store(p.il_cnt + (p.M + 127) / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&kh_coop_timeout_count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-      }
-      const int c = (t - KT1) * BK;
-#pragma unroll
-      for (int q = 0; q < LPS_HI; ++q) {
-        if (q < LPS_LO || has_hi) {
-          const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
-          const uint32_t vo = col < r_ext ? voff2[EXT ? q : 0] : OOB;
-          // T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
-          if ((COOP || TMODE == T_IL) && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
-          else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 0);
-        }
-      }
-      return;
-    }
-#pragma unroll
-    for (int q = 0; q < LPS_HI; ++q) {
-      if (q < LPS_LO || has_hi) {
-        lptr_t dst = (lptr_t)(stage + (pw + 4 * q) * 1024);
-        if (q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, dst, 16, xvo[q], CONV ? (cv_shift + cv_c0) * 2 : so, 0, 0);
-        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, voff[q], so, 0, 0);
-      }
-    }
-    if (CONV) {
-      cv_c0 += BK;
-      if (cv_c0 == p.conv_cin) {
-        cv_c0 = 0; ++cv_tap; ++cv_kw; cv_shift += p.conv_cin;
-        if (cv_kw == 3) { cv_kw = 0; cv_row += p.conv_w * p.conv_cin; cv_shift = cv_row; }
-#pragma unroll
-        for (int q = 0; q < XQ; ++q) xvo[q] = ((tapmask[CONV ? q : 0] >> cv_tap) & 1) ? voff[q] : OOB;
-      }
-    }
-  };
-  // until at most n of this wave's younger K tiles are outstanding (and its LDS reads are done)
-  auto wait_younger = [&](int n) {
-    if (has_hi) wait_tiles<LPS_HI, PD - 1>(n); else wait_tiles<LPS_LO, PD - 1>(n);
-  };
-
   // fragments: row lr of each block of MF rows; of a k-step the lane's 16-byte piece lg (16x16x16: its 8 bytes lg)
   constexpr bool HALF = C::ORD == 4 && C::MF == 16;
   using Frag = typename std::conditional<HALF, s16x4, bf16x8>::type;
@@ -353,7 +252,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   int fa[KS], fb[KS];
 #pragma unroll
   for (int k = 0; k < KS; ++k) {
-    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
+    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::MF == 16 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
     fa[k] = (wm * (BM / C::WM) + lr) * ROWB + po;
     fb[k] = (BM + wn * (BN / C::WN) + lr) * ROWB + po;
   }
@@ -400,6 +299,112 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   typedef XAttnFine<cmax(BN / 64, 1), 256, C::LDC> XAttn;
   XAttn kv;                                            // XA: the keys and values, in the producers
   if (producer) {
+    // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
+    // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row).  (Here and
+    // not in front of the branch: the 128 x 320 tiles then kept these offsets over the computing waves' loop, in scratch memory.)
+    constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
+    uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
+    int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
+#pragma unroll
+    for (int q = 0; q < LPS_HI; ++q) {
+      int u = pw + 4 * q;
+      u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
+      const int r = u * UR + lane / PPR;
+      const uint32_t pcb = (uint32_t)(((lane % PPR) ^ swz(r)) * 16);
+      if (CONV && q < XQ) {
+        int row = m0 + r; row = row < M ? row : M - 1;
+        const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
+        const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
+        int mask = 0;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+          const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
+          mask |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
+        }
+        tapmask[q < XQ ? q : 0] = mask;
+        // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
+        voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
+      } else if (q < XQ) {
+        voff[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + pcb;        // rows past M lie beyond the buffer: zeros
+      } else {
+        voff[q] = (uint32_t)(n0 + r - BM) * (uint32_t)K * 2u + pcb;
+      }
+      if (EXT && p.t_ext != nullptr)
+        voff2[q] = q < XQ ? ((uint32_t)(m0 + r) * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb
+                          : (uint32_t)(n0 + r - BM) * (uint32_t)p.R * 2u + pcb;
+    }
+    const size_t x_bytes = CONV ? (size_t)(M / (p.conv_ho * p.conv_wo)) * p.conv_h * p.conv_w * p.conv_cin * 2 : (size_t)M * K * 2;
+    const size_t x_lead = CONV ? (size_t)(p.conv_w + 1) * p.conv_cin * 2 : 0;
+    const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.x) - x_lead), 0,
+                                                           (int)(x_bytes + x_lead), 0x00020000);
+    const rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w), 0, (int)((size_t)N * K * 2), 0x00020000);
+    const bool has_t = EXT && p.t_ext != nullptr;
+    const rsrc_t rs_t = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.t_ext : p.x), 0,
+                                                           has_t ? (int)((size_t)M * p.ldt * 2) : 0, 0x00020000);
+    const rsrc_t rs_bx = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(has_t ? p.b_cat : p.w), 0,
+                                                            has_t ? (int)((size_t)N * p.R * 2) : 0, 0x00020000);
+    // CONV: K tiles are requested in order, so the tap and the channel offset of the next request are running scalars
+    int cv_tap = 0, cv_kw = 0, cv_c0 = 0, cv_shift = 0, cv_row = 0;
+    uint32_t xvo[XQ];
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) xvo[q] = (!CONV || (tapmask[CONV ? q : 0] & 1)) ? voff[q] : OOB;
+    auto issue = [&](int t, int st) {                    // K tile t into the ring stage at byte offset st
+      char* stage = smem + st;
+      const int so = t * ROWB;
+      if (EXT && t >= KT1) {                             // columns of T and B_cat; past the last rank column: zeros
+        if ((COOP || TMODE == T_IL) && t == KT1) {
+          // first request for T: wait (bounded) until every workgroup of these 128 rows has delivered its piece
+          if (lane == 0) {
+            int it = 0, want = p.n_tiles;
+            if (TMODE == T_IL) {
+              const int left = M - m0 / 128 * 128;
+              if (BM == 128 && BN == 128) want = ((left < 128 ? left : 128) + 63) / 64 * p.il_cols;
+              else want = ((left < 128 ? left : 128) + p.il_tile - 1) / p.il_tile * ((r_ext + p.il_tile - 1) / p.il_tile) * (p.ldt / p.R);
+            }
+            while (__hip_atomic_load(p.il_cnt + m0 / 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want && ++it < (1 << 20))
+              __builtin_amdgcn_s_sleep(8);
+            if (it >= (1 << 20)) {
+              __hip_atomic_store(p.il_cnt + (p.M + 127) / 128, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              __hip_atomic_fetch_add(&kh_coop_timeout_count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+          }
+        }
+        const int c = (t - KT1) * BK;
+#pragma unroll
+        for (int q = 0; q < LPS_HI; ++q) {
+          if (q < LPS_LO || has_hi) {
+            const int r = (pw + 4 * q) * UR + lane / PPR, col = c + ((lane % PPR) ^ swz(r)) * 8;
+            const uint32_t vo = col < r_ext ? voff2[EXT ? q : 0] : OOB;
+            // T was written inside this launch, maybe on another XCD: read past the (non-coherent) L2
+            if ((COOP || TMODE == T_IL) && q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_t, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 17 /* sc0 sc1 */);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(q < XQ ? rs_t : rs_bx, (lptr_t)(stage + (pw + 4 * q) * 1024), 16, vo, c * 2, 0, 0);
+          }
+        }
+        return;
+      }
+#pragma unroll
+      for (int q = 0; q < LPS_HI; ++q) {
+        if (q < LPS_LO || has_hi) {
+          lptr_t dst = (lptr_t)(stage + (pw + 4 * q) * 1024);
+          if (q < XQ) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_x, dst, 16, xvo[q], CONV ? (cv_shift + cv_c0) * 2 : so, 0, 0);
+          else __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_w, dst, 16, voff[q], so, 0, 0);
+        }
+      }
+      if (CONV) {
+        cv_c0 += BK;
+        if (cv_c0 == p.conv_cin) {
+          cv_c0 = 0; ++cv_tap; ++cv_kw; cv_shift += p.conv_cin;
+          if (cv_kw == 3) { cv_kw = 0; cv_row += p.conv_w * p.conv_cin; cv_shift = cv_row; }
+#pragma unroll
+          for (int q = 0; q < XQ; ++q) xvo[q] = ((tapmask[CONV ? q : 0] >> cv_tap) & 1) ? voff[q] : OOB;
+        }
+      }
+    };
+    // until at most n of this wave's younger K tiles are outstanding (and its LDS reads are done)
+    auto wait_younger = [&](int n) {
+      if (has_hi) wait_tiles<LPS_HI, PD - 1>(n); else wait_tiles<LPS_LO, PD - 1>(n);
+    };
+
     // requested now, used after the K loop (older than every DMA load, so no wait falls in between)
     constexpr int CP = (BN + 255) / 256;
     const int ptid = tid - 256;
@@ -445,14 +450,15 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   } else {
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
-    auto touch = [&](int t, int n) {
+    auto touch = [&](int t, auto n) {
       if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
-        kh_touch_rows(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
+        kh_touch_rows<decltype(n)::value>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
     constexpr int TOUCH = C::GLU ? 8 : 24;
-    touch(0, TOUCH);
+    constexpr std::integral_constant<int, 8> EIGHT{};
+    touch(0, std::integral_constant<int, TOUCH>{});
     if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128 && il_prefetch_by_idle_waves(p)))
       kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
@@ -497,18 +503,22 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
       read_a(0, 0, 0);
 #pragma unroll
       for (int j = 0; j < TN; ++j) read_b(0, 0, j);
-      if constexpr (KS == 2) {
+      if constexpr (KS % 2 == 0) {
+        auto stage_steps = [&]() {                     // all k-steps but the last
+#pragma unroll
+          for (int k = 0; k + 1 < KS; ++k) kstep(k & 1, st, k + 1);
+        };
         for (int t = 0; t + 1 < KT; ++t) {
-          if ((t & 7) == 0) touch(t + TOUCH, 8);
-          kstep(0, st, 1);
+          if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
+          stage_steps();
           next_stage();
           kstep(1, st, 0);
         }
-        kstep(0, st, 1);
+        stage_steps();
       } else {
         int t = 0;
         for (; t + 2 < KT; t += 2) {
-          if ((t & 7) == 0) touch(t + TOUCH, 8);
+          if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
           next_stage();
           kstep(0, st, 0);
           next_stage();
@@ -522,7 +532,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
         }
       }
 #pragma unroll
-      for (int j = 0; j < TN; ++j) mma1(KS == 2 ? 1 : 0, j);
+      for (int j = 0; j < TN; ++j) mma1(KS % 2 == 0 ? 1 : 0, j);
     } else {
     Fr f0, f1;
     read_frags(0, f0);
@@ -535,7 +545,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     };
     int t = 0;
     for (; t + 2 < KT; t += 2) {
-      if ((t & 7) == 0) touch(t + TOUCH, 8);
+      if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
       step(f0, f1);
       step(f1, f0);
     }
@@ -585,7 +595,9 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) finish(group(acc[i][j], 0), i, j, 0);
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int g = 0; g < C::G; ++g) finish(group(acc[i][j], g), i, j, g);
     }
   } else {
     constexpr int UH = TM / C::NH * TN * C::G;           // groups of a pass

@@ -713,7 +713,7 @@ __global__ __launch_bounds__(C::NT, C::OCC) void lora_gemm_pipe_kernel(const Lor
   // 3840 / 1280 17.4 -> 16.5 us (the other instantiations have no registers for it or gain nothing)
   if (!IL && !CONV && LNF != 3 && !XA && BM == 128 && BN == 128 && C::NT == 512 && p.grp == nullptr && p.sg_mode == 0 &&
       p.xr_m * p.xr_n >= 16 && kh_touch_pays(N, K, p.xr_n * BN))
-    kh_touch_rows(p.w, N, K, (bid & 7) % p.xg_n * p.xr_n * BN, p.xr_n * BN, 0, K / 64, smem + wave * (C::UX / C::NW) * 1024,
+    kh_touch_rows<>(p.w, N, K, (bid & 7) % p.xg_n * p.xr_n * BN, p.xr_n * BN, 0, K / 64, smem + wave * (C::UX / C::NW) * 1024,
                   (bid >> 3) * C::NT + tid, p.xr_m * p.xr_n * C::NT);
   // folded LayerNorm: mean and 1/std of this tile's x rows, read in the epilogue (the barriers of the K loop lie between)
   // and the two per-column terms of this (single) column tile
