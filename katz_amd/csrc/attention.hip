@@ -52,6 +52,12 @@ __device__ __forceinline__ void wait_vm() {  // vmcnt = VM, the other counters u
   __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | (15 << 8) | ((VM >> 4) << 14));
 }
 
+// the larger of lanes l and l + 32, in both, without a trip through LDS
+__device__ __forceinline__ float half_max(float v) {
+  const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+
 template <int NW>   // waves per workgroup: NW*32 queries
 // Two waves per SIMD at least: that caps a wave at 256 registers, which makes the compiler keep MFMA results in
 // VGPRs (the softmax reads them every tile; from AGPRs every score and every rescaled output costs extra moves).
@@ -159,7 +165,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(const AttnParams 
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int v = 0; v < 16; ++v) mx = fmaxf(mx, st[kt][v]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = half_max(mx);
     // Lazy running maximum: the reference point of the exponentials only moves when the row maximum has grown by
     // more than 2^RESCALE_LOG2 in the exponent domain; until then p = exp2(s - m) may exceed 1 (by at most that
     // factor, harmless in fp32 / bf16) and numerator and denominator stay consistent.  Moving it rescales
