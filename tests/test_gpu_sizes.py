@@ -841,3 +841,22 @@ def test_two_streams_of_few_row_calls():
     for i in (0, 1):
         assert all(torch.equal(y, want[i]) for y in got[i])
     ops.check_split_timeouts(d)
+
+
+@pytest.mark.parametrize("T,S", [(200, 333), (128, 64), (65, 1), (64, 77), (1, 130), (97, 96)])
+def test_attention_waves_of_16_queries(T, S):
+    """A few heads run on waves of 16 queries, hundreds on waves of 32, the numbers between on both: the same rows, the same bits, and the oracle's values."""
+    from katz_amd import ops
+    from oracle import ops as O
+
+    say("attention, waves of 16 and 32 queries", T, S)
+    d, g, H = dev(), torch.Generator().manual_seed(T + S), 2
+    q, k, v = (torch.randn(3, n, H * 64, generator=g).to(d, BF) for n in (T, S, S))
+    k[:, S // 2:] *= 8                                    # the running maximum moves
+    o = ops.attention(q, k, v, H)
+    assert_close_rel(o, O.attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), H), 2e-2)
+    blocks = (T + 127) // 128
+    for units in (256 + 12, 256 + 160):                   # 128 queries each: 256 of them whole and the rest halved; all whole
+        n = units // (3 * H * blocks) + 1
+        more = ops.attention(*(t.repeat(n, 1, 1) for t in (q, k, v)), H)
+        assert torch.equal(more.view(n, *o.shape), o.expand(n, *o.shape))
