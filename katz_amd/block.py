@@ -17,6 +17,7 @@ import torch
 from torch import nn
 
 from . import _lib, layers, ops
+from .lora import PooledPack, norm_key, stacked_packs
 
 
 class _Linear(ctypes.Structure):   # KhLinearDesc
@@ -79,7 +80,7 @@ class _Plan:
         self.versions = [t._version for t in self.tensors]
         self.addresses = [t.data_ptr() for t in self.tensors]
         if self.usable:
-            for l in (self.attn1.to_q, self.attn1.to_k, self.attn1.to_v, *(l for _, l, _ in self.linears)):
+            for l in (self.attn1.to_q, self.attn1.to_k, self.attn1.to_v, *(l for _, l, _, _ in self.linears)):
                 layers.hold_pack(l, self)
 
     def drop_packs(self) -> None:
@@ -121,8 +122,22 @@ class _Plan:
             w, c1, c2 = l._ln_terms(norm)[:3]
             b, d.eps = None, norm.eps
         self.keep.append(self.weights(d, w, b, c1, c2))
-        self.linears.append((name, l, norm))
+        self.linears.append((name, l, norm, None if norm is None else norm_key(norm)))
         return True
+
+    def stacked_weights(self):
+        """The operands of q | k | v that do not depend on the packs, and the folded norm's key; None where the layers are not stacked."""
+        got = self.qkv_weights
+        if got is None:
+            a, norm = self.attn1, self.norm1
+            q = (a.to_q, a.to_k, a.to_v)
+            if a.to_q.out_features % 128 != 0 or a.to_q.in_features % 64 != 0 or any(l.bias is not None for l in q):
+                return None
+            key = tuple((l.weight.data_ptr(), l.weight._version) for l in q)
+            w = a._qkv_weights(key)
+            nk = None if norm is None else norm_key(norm)
+            got = self.qkv_weights = ((w, None, None) if norm is None else tuple(a._qkv_norm_weights(w, norm, nk, key)), nk)
+        return got
 
     def weights(self, d: _Linear, w, b, c1, c2):
         d.w, d.bias, d.c1, d.c2 = w.data_ptr(), _addr(b), _addr(c1), _addr(c2)
@@ -167,6 +182,7 @@ class _Plan:
                 return False
             l.prepare()
             self.seen(l, params=("weight", "bias"), plain=("_rt", "bias"))
+        self.qkv_weights = None
         if folded:
             q.eps = norms[0].eps
         q.N, q.K = 3 * a1.to_q.out_features, a1.to_q.in_features
@@ -208,34 +224,60 @@ class _Ready:
     def fill(self, plan) -> bool:
         expect, keep = self.packs.expect, self.keep
         attn = plan.attn1
-        st = attn._qkv_state()
+        qkv = []
         for l in (attn.to_q, attn.to_k, attn.to_v):
             p = expect(l.__dict__, "_packed")
+            qkv.append(p)
             if p is not None:
                 expect(p.__dict__, "a_cat")
         split = layers.LORA_MODE == "split"
-        for name, l, norm in plan.linears:
+        for name, l, norm, nk in plan.linears:
             p = expect(l.__dict__, "_packed")
             if p is None:
                 continue
             if p.overflow or not split:
                 return False
-            v = p.__dict__
+            v, d = p.__dict__, getattr(self.desc, name)
             a, b, s = expect(v, "a_cat"), expect(v, "b_cat"), expect(v, "col_scale")
+            at = p.addresses(nk) if type(p) is PooledPack else None
+            if at is not None:                             # by address: no views are made
+                d.a_cat, d.b_cat, d.col_scale, d.ca1, d.ca2 = at
+                d.R, d.r_used = p.shape[0], p.used
+                keep.append(p)
+                continue
+            a, b, s = p.a_cat, p.b_cat, p.col_scale
             ca1 = ca2 = None
             if norm is not None:
                 a, ca1, ca2 = l._ln_terms(norm)[3:]
-            self.operands(getattr(self.desc, name), a, b, s, ca1, ca2, p.r_used)
-        if st is None:
-            return False
+            self.operands(d, a, b, s, ca1, ca2, p.r_used)
         q, norm = self.desc.qkv, plan.norm1
-        w, c1, c2, a, ca1, ca2 = attn._qkv_folded(st, norm) if norm is not None else (st["w"], None, None, st.get("a"), None, None)
-        keep.append(plan.weights(q, w, None, c1, c2))
-        refs = (w, None, None)
-        if st["R"]:
-            self.operands(q, a, st["b"], st["s"], ca1, ca2, st["r_used"])
-            q.n_split = plan.inner
-            refs = (w, a, st["b"])
+        st, first = None, qkv[0]
+        weights = plan.stacked_weights() if split and type(first) is PooledPack else None
+        side_by_side = stacked_packs(qkv) if weights is not None else None
+        if side_by_side is not None:
+            (w, c1, c2), nk = weights
+            at = [p.addresses(nk) for p in qkv]
+            if None not in at:
+                st = weights
+                plan.weights(q, w, None, c1, c2)
+                q.a_cat, q.b_cat, q.col_scale, q.ca1, q.ca2 = at[0]
+                q.R, q.r_used, q.n_split = first.shape[0], max(p.used for p in qkv), plan.inner
+                a, b, _ = side_by_side                     # (hints hold them weakly)
+                if nk is not None:
+                    a = first.pool[3].as_strided(a.shape, a.stride(), first.at[3])
+                keep += (qkv, w, c1, c2, a, b)
+                refs = (w, a, b)
+        if st is None:
+            st = attn._qkv_state()
+            if st is None:
+                return False
+            w, c1, c2, a, ca1, ca2 = attn._qkv_folded(st, norm) if norm is not None else (st["w"], None, None, st.get("a"), None, None)
+            keep.append(plan.weights(q, w, None, c1, c2))
+            refs = (w, None, None)
+            if st["R"]:
+                self.operands(q, a, st["b"], st["s"], ca1, ca2, st["r_used"])
+                q.n_split = plan.inner
+                refs = (w, a, st["b"])
         self.first = tuple(None if t is None else weakref.ref(t) for t in refs)
         self.first_key = int(q.w)
         return True

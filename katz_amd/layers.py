@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from . import ops
 from .lora import (MAX_PACKED_RANK, Adapter, PackedAdapters, fold_norm_into_adapters, fold_norm_into_weight, interleave_geglu_rows,
-                   norm_key, pack_adapters, pack_many, pack_many_takes, rescale_, rescale_many, stacked)
+                   norm_key, pack_adapters, pack_many, pack_many_takes, rescale_, rescale_many, stacked, stacked_norm_terms, stacked_packs)
 
 CL = torch.channels_last
 
@@ -914,22 +914,24 @@ class Attention(nn.Module):
             ok = same and (packs[0] is None or LORA_MODE == "split") and all(l.bias is None for l in layers)
             st = dict(sig=sig, ok=ok)
             if ok:
-                if self._qkv_w is None or self._qkv_w[0] != sig[1]:
-                    self._qkv_w = (sig[1], torch.cat([l.weight.detach() for l in layers], dim=0).contiguous())
-                st["w"] = self._qkv_w[1]
+                st["w"] = self._qkv_weights(sig[1])
                 st["R"] = 0 if packs[0] is None else packs[0].R
                 if st["R"]:
                     R = st["R"]
                     st["r_used"] = max(p.r_used for p in packs)
                     cat = lambda ts: torch.cat(ts, dim=0).contiguous()
-                    a, sc, bc = ([getattr(p, n) for p in packs] for n in ("a_cat", "col_scale", "b_cat"))
-                    st["a"], st["s"], st["b"] = stacked(a), stacked(sc), stacked(bc)
-                    if st["b"] is None:
-                        st["b"] = cat(bc)
-                    if st["a"] is None or st["s"] is None:
-                        st["a"], st["s"] = cat(a), cat(sc)
-                        for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
-                            p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
+                    side_by_side = stacked_packs(packs)
+                    if side_by_side is not None:
+                        st["a"], st["b"], st["s"] = side_by_side
+                    else:
+                        a, sc, bc = ([getattr(p, n) for p in packs] for n in ("a_cat", "col_scale", "b_cat"))
+                        st["a"], st["s"], st["b"] = stacked(a), stacked(sc), stacked(bc)
+                        if st["b"] is None:
+                            st["b"] = cat(bc)
+                        if st["a"] is None or st["s"] is None:
+                            st["a"], st["s"] = cat(a), cat(sc)
+                            for g, p in enumerate(packs):  # the layers now read (and rescale) the stacked storage
+                                p.a_cat, p.col_scale = st["a"][g * R:(g + 1) * R], st["s"][g * R:(g + 1) * R]
             for l in layers:
                 hold_pack(l, self)
             self._qkv = st
@@ -937,24 +939,30 @@ class Attention(nn.Module):
                 self.drop_packs()   # another thread replaced one meanwhile: nobody else would drop the old one
         return st if st["ok"] else None
 
+    def _qkv_weights(self, key) -> torch.Tensor:
+        """The stacked weights; key: (address, version) of each."""
+        if self._qkv_w is None or self._qkv_w[0] != key:
+            self._qkv_w = (key, torch.cat([l.weight.detach() for l in (self.to_q, self.to_k, self.to_v)], dim=0).contiguous())
+        return self._qkv_w[1]
+
+    def _qkv_norm_weights(self, w: torch.Tensor, norm: "LayerNorm", key, weights_key):
+        """(W', c1, c2) of the stacked weights behind `norm`; key: its norm_key."""
+        if self._qkv_ln is None or self._qkv_ln[0] != (key, weights_key):
+            self._qkv_ln = ((key, weights_key),) + fold_norm_into_weight(w, None, norm.weight, norm.bias)
+        return self._qkv_ln[1:]
+
     def drop_packs(self) -> None:
         self.__dict__["_qkv"] = None
 
     def _qkv_folded(self, st: dict, norm: "LayerNorm"):
         """(W', c1, c2, A', ca1, ca2) of the stacked projections behind `norm` (lora.fold_layer_norm)."""
         key = norm_key(norm)
-        sig = st["sig"]
-        if self._qkv_ln is None or self._qkv_ln[0] != (key, sig[1]):
-            self._qkv_ln = ((key, sig[1]),) + fold_norm_into_weight(st["w"], None, norm.weight, norm.bias)
-        _, wp, c1, c2 = self._qkv_ln
+        wp, c1, c2 = self._qkv_norm_weights(st["w"], norm, key, st["sig"][1])
         if not st["R"]:
             return wp, c1, c2, None, None, None
         if st.get("ln_key") != key:
-            parts = [l._packed.ln for l in (self.to_q, self.to_k, self.to_v)]
-            ln = None
-            if all(t is not None and t[0] == key for t in parts):   # built with the packs, side by side
-                ln = tuple(stacked([t[j] for t in parts]) for j in (1, 2, 3))
-            if ln is None or any(t is None for t in ln):
+            ln = stacked_norm_terms([l._packed for l in (self.to_q, self.to_k, self.to_v)], key)     # built with the packs, side by side
+            if ln is None:
                 ln = fold_norm_into_adapters(st["a"], norm.weight, norm.bias)
             st["ln"], st["ln_key"] = ln, key
         return (wp, c1, c2) + tuple(st["ln"])
@@ -1143,9 +1151,13 @@ class ContextKVProjector:
             G = len(layers)
             R = 0 if packs[0] is None else packs[0].R
             y = torch.empty((G, M, width), dtype=torch.bfloat16, device=dev)
-            t = a_all = s_all = None
+            t = a_all = s_all = side_by_side = None
             if R > 0:
-                a_all, s_all = stacked([p.a_cat for p in packs]), stacked([p.col_scale for p in packs])
+                side_by_side = stacked_packs(packs)
+                if side_by_side is not None:
+                    a_all, _, s_all = side_by_side
+                else:
+                    a_all, s_all = stacked([p.a_cat for p in packs]), stacked([p.col_scale for p in packs])
                 if a_all is None or s_all is None:
                     a_all = torch.cat([p.a_cat for p in packs], dim=0).contiguous()
                     s_all = torch.cat([p.col_scale for p in packs], dim=0).contiguous()
@@ -1153,11 +1165,12 @@ class ContextKVProjector:
                         p.a_cat = a_all[g * R:(g + 1) * R]
                         p.col_scale = s_all[g * R:(g + 1) * R]
                 t = torch.empty((M, G * R), dtype=torch.bfloat16, device=dev)
+            b_at = (lambda p: p.addresses()[1]) if side_by_side is not None else (lambda p: p.b_cat.data_ptr())
             rows = []
             for g, l in enumerate(layers):
                 _, w, b = l._rt
-                rows.append([w.data_ptr(), 0 if b is None else b.data_ptr(), 0 if R == 0 else packs[g].b_cat.data_ptr(),
-                             0 if R == 0 else t.data_ptr() + g * R * 2, y[g].data_ptr()])
+                rows.append([w.data_ptr(), 0 if b is None else b.data_ptr(), 0 if R == 0 else b_at(packs[g]),
+                             0 if R == 0 else t.data_ptr() + g * R * 2, y.data_ptr() + g * M * width * 2])
             st.update(G=G, R=R, K=K, y=y, t=t, a_all=a_all, s_all=s_all,
                       table=ops.upload_table(np.array(rows, dtype=np.int64), dev))
             for l in layers:

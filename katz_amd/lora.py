@@ -72,6 +72,101 @@ class PackedAdapters:
         return min(self.R, (used + 15) // 16 * 16)
 
 
+class PooledPack(PackedAdapters):
+    """A layer's share of the buffers that pack_many fills for many layers.  An activation makes hundreds of these and most are only ever read by address, so
+    the tensors are views that are made when somebody asks for them; one that is assigned (`moved`) takes the view's place."""
+
+    def __init__(self, pool: Sequence[torch.Tensor], at: Sequence[int], shape: Sequence[int], names: Sequence[str], ranks: Sequence[int], used: int,
+                 norm: Optional[tuple]):
+        d = self.__dict__
+        d["pool"], d["at"], d["shape"] = pool, at, shape           # buffers (A, B, scales, A * norm, its two terms), offsets in elements, (R, K, N)
+        d["names"], d["ranks"], d["used"], d["norm"] = names, ranks, used, norm
+
+    def _view(self, name: str, which: int, size: tuple, stride: tuple):
+        d = self.__dict__
+        v = d.get(name) if name in d else d.get("_" + name)
+        return d.setdefault("_" + name, self.pool[which].as_strided(size, stride, self.at[which])) if v is None else v
+
+    def _move(self, name: str, v) -> None:
+        self.__dict__[name] = v
+
+    @property
+    def moved(self) -> bool:
+        d = self.__dict__
+        return "a_cat" in d or "b_cat" in d or "col_scale" in d
+
+    R = property(lambda self: self.shape[0])
+    r_used = property(lambda self: self.used)
+    overflow = property(lambda self: ())
+    a_cat = property(lambda self: self._view("a_cat", 0, (self.shape[0], self.shape[1]), (self.shape[1], 1)), lambda self, v: self._move("a_cat", v))
+    b_cat = property(lambda self: self._view("b_cat", 1, (self.shape[2], self.shape[0]), (self.shape[0], 1)), lambda self, v: self._move("b_cat", v))
+    col_scale = property(lambda self: self._view("col_scale", 2, (self.shape[0],), (1,)), lambda self, v: self._move("col_scale", v))
+
+    @property
+    def spans(self):
+        out, c = [], 0
+        for n, r in zip(self.names, self.ranks):
+            out.append((n, c, r))
+            c += r
+        return out
+
+    @property
+    def ln(self):
+        d = self.__dict__
+        if d.get("ln") is None and self.norm is not None:
+            R, K, _ = self.shape
+            _, _, _, an, c1, c2 = self.pool
+            at, c = self.at[3:]
+            d.setdefault("ln", (self.norm, an.as_strided((R, K), (K, 1), at), c1.as_strided((R,), (1,), c), c2.as_strided((R,), (1,), c)))
+        return d.get("ln")
+
+    @ln.setter
+    def ln(self, v):
+        self.__dict__["ln"] = v
+
+    def addresses(self, norm: Optional[tuple] = None):
+        """(A, B, scales, terms 1 and 2), with a norm_key A and the terms behind that norm; None where a tensor has been moved or the norm is another one."""
+        d = self.__dict__
+        if self.moved or (norm is not None and norm != d["norm"]):
+            return None
+        pool, at = d["pool"], d["at"]
+        b, s = pool[1].data_ptr() + 2 * at[1], pool[2].data_ptr() + 4 * at[2]
+        if norm is None:
+            return pool[0].data_ptr() + 2 * at[0], b, s, 0, 0
+        if d.get("ln") is not None and d["ln"][0] != norm:
+            return None
+        return pool[3].data_ptr() + 2 * at[3], b, s, pool[4].data_ptr() + 4 * at[4], pool[5].data_ptr() + 4 * at[4]
+
+    def followed_by(self, other) -> bool:
+        """Do `other`'s rows lie behind this pack's in every buffer?"""
+        R, K, N = self.shape
+        return (type(other) is PooledPack and other.pool is self.pool and not self.moved and not other.moved and other.shape[0] == R and other.shape[1] == K
+                and other.at[0] == self.at[0] + R * K and other.at[1] == self.at[1] + R * N and other.at[2] == self.at[2] + R
+                and (self.norm != other.norm or self.norm is None or (other.at[3] == self.at[3] + R * K and other.at[4] == self.at[4] + R)))
+
+
+def stacked_packs(packs: Sequence[PackedAdapters]):
+    """A_cat, B_cat and the scales of packs that lie one behind the other in a pool, as one tensor each; None otherwise."""
+    first = packs[0]
+    if type(first) is not PooledPack or first.moved or not all(p.followed_by(q) for p, q in zip(packs[:-1], packs[1:])):
+        return None
+    R, K, _ = first.shape
+    (A, B, S), n = first.pool[:3], len(packs)
+    return (A.as_strided((n * R, K), (K, 1), first.at[0]), B.as_strided((sum(p.shape[2] for p in packs), R), (R, 1), first.at[1]),
+            S.as_strided((n * R,), (1,), first.at[2]))
+
+
+def stacked_norm_terms(packs: Sequence[PackedAdapters], norm: tuple):
+    """A_cat behind a folded LayerNorm (its norm_key) and the two terms of stacked_packs' packs, as one tensor each; None where they are not in place."""
+    if stacked_packs(packs) is None or any(p.addresses(norm) is None for p in packs):
+        return None
+    R, K, _ = packs[0].shape
+    at, c = packs[0].at[3:]
+    _, _, _, an, c1, c2 = packs[0].pool
+    n = R * len(packs)
+    return an.as_strided((n, K), (K, 1), at), c1.as_strided((n,), (1,), c), c2.as_strided((n,), (1,), c)
+
+
 def interleave_geglu_rows(t: torch.Tensor) -> torch.Tensor:
     """Reorder the output-feature axis (dim 0) of a GEGLU projection tensor from
     [value(0..D) | gate(0..D)] (hidden, gate = proj(x).chunk(2, -1),
@@ -155,84 +250,98 @@ def stacked(views: Sequence[torch.Tensor]) -> Optional[torch.Tensor]:
     return first.as_strided((rows,) + tuple(first.shape[1:]), first.stride())
 
 
+_PACK_F, _UNPACK_I = struct.Struct("<f").pack, struct.Struct("<I").unpack
 _PIECE_DTYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
 def pack_many_takes(layer, names: Sequence[str]) -> bool:
     """Can pack_many build this layer's pack (else: pack_adapters)?"""
     w = layer._parameters["weight"]
-    if not w.is_cuda or w.dtype != torch.bfloat16 or layer.in_features % 8 != 0 or layer.out_features % 8 != 0:
+    K, N, adapters = layer.in_features, layer.out_features, layer.adapters
+    if not w.is_cuda or w.dtype != torch.bfloat16 or K % 8 != 0 or N % 8 != 0:
         return False
     total, dev = 0, w.device
     for n in names:
-        ad = layer.adapters[n]
-        r = ad.down.shape[0]
+        ad = adapters[n]
+        down, up = ad.down, ad.up
+        r, dtype = down.shape[0], down.dtype
         total += r
-        if ad.up.dtype != ad.down.dtype:      # a piece has one dtype
+        if up.dtype != dtype or dtype not in _PIECE_DTYPES or down.shape != (r, K) or up.shape != (N, r):      # (a piece has one dtype)
             return False
-        for t, shape in ((ad.down, (r, layer.in_features)), (ad.up, (layer.out_features, r))):
-            if t.dtype not in _PIECE_DTYPES or t.shape != shape or (t.is_cuda and (t.device != dev or not t.is_contiguous() or t.data_ptr() % 16)):
-                return False
-    return 0 < total <= MAX_PACKED_RANK and (not layer.geglu or layer.out_features % 64 == 0)
+        if down.is_cuda and (down.device != dev or not down.is_contiguous() or down.data_ptr() % 16):
+            return False
+        if up.is_cuda and (up.device != dev or not up.is_contiguous() or up.data_ptr() % 16):
+            return False
+    return 0 < total <= MAX_PACKED_RANK and (not layer.geglu or N % 64 == 0)
 
 
 def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAdapters]:
     """pack_adapters for many layers of one device (such as pack_many_takes accepts) in two launches (kh_lora_pack_bf16);
     adapters in host memory are uploaded with one call.  All packs of a kind share one buffer, in the order of `layers`, so
     layers that run as one launch (q / k / v of a self-attention, the context projections) find their stacked operands in place
-    (`stacked`).  layer.fold_norm: a function that gives the LayerNorm in front of the layer or None."""
+    (`stacked`, PooledPack.followed_by).  layer.fold_norm: a function that gives the LayerNorm in front of the layer or None."""
     dev = layers[0].weight.device
     host = [t for l, ns in zip(layers, names) for n in ns for t in (l.adapters[n].down, l.adapters[n].up) if not t.is_cuda]
     keep, where = None, {}
     if host:
         keep, addresses = ops.upload_many(host, dev)
         where = {id(t): a for t, a in zip(host, addresses)}
-    address = lambda t: t.data_ptr() if t.is_cuda else where[id(t)]
-    bits = lambda x: struct.unpack("<I", struct.pack("<f", x))[0]
-    ranks = [sum(l.adapters[n].rank for n in ns) for l, ns in zip(layers, names)]
-    padded = [-(-r // RANK_PAD) * RANK_PAD for r in ranks]
-    norms = [l.fold_norm() for l in layers]
-    norms = [g if g is not None and g.weight.dtype == torch.bfloat16 and g.weight.device == dev else None for g in norms]
-    sizes_a = [R * l.in_features for l, R in zip(layers, padded)]
-    sizes_b = [R * l.out_features for l, R in zip(layers, padded)]
-    folded = [i for i, g in enumerate(norms) if g is not None]
-    buf = lambda n, dt: torch.empty((n,), dtype=dt, device=dev)
-    A, B, S = buf(sum(sizes_a), torch.bfloat16), buf(sum(sizes_b), torch.bfloat16), buf(sum(padded), torch.float32)
-    AN = buf(sum(sizes_a[i] for i in folded), torch.bfloat16)
-    C1, C2 = (buf(sum(padded[i] for i in folded), torch.float32) for _ in range(2))
-    pa, pb, ps, pan, pc1, pc2 = (t.data_ptr() for t in (A, B, S, AN, C1, C2))
-    # flat tables, and views made directly: thousands of short-lived tuples and tensors per activation bring on the interpreter's
-    # full collections (85 ms for the objects of this model) the sooner
+    # One walk that leaves offsets and flat tables, then the buffers.  What an activation makes is counted: thousands of short-lived tuples and tensors
+    # bring on the interpreter's full collections (125 ms for the objects of three of these models) the sooner, and views of every layer's operands
+    # alone took 3 ms.
     rows, pieces, packs, n_pieces = [], [], [], 0
     at_a = at_b = at_s = at_an = at_c = 0
-    b_blocks = []
-    for l, ns, R, g in zip(layers, names, padded, norms):
-        K, N = l.in_features, l.out_features
-        ln = None
-        if g is not None:
-            rows += (pa + 2 * at_a, pan + 2 * at_an, g.weight.data_ptr(), g.bias.data_ptr(), pc1 + 4 * at_c, pc2 + 4 * at_c)
-            ln = (norm_key(g), AN.as_strided((R, K), (K, 1), at_an), C1.as_strided((R,), (1,), at_c), C2.as_strided((R,), (1,), at_c))
-            at_an += R * K
-            at_c += R
-        else:
-            rows += (pa + 2 * at_a, 0, 0, 0, 0, 0)
-        rows += (pb + 2 * at_b, ps + 4 * at_s, K, N, R, int(l.geglu), n_pieces, len(ns))
-        n_pieces += len(ns)
-        spans, c = [], 0
+    b_blocks, padded, keys = [], [], {}
+    pool = []
+    for l, ns in zip(layers, names):
+        d = l.__dict__
+        K, N, ads = d["in_features"], d["out_features"], d["adapters"]
+        scale, c, ranks = d["global_scale"], 0, []
         for n in ns:
-            ad = l.adapters[n]
-            r = ad.down.shape[0]
-            pieces += (address(ad.down), address(ad.up), r, c, _PIECE_DTYPES[ad.down.dtype], bits(ad.multiplier(l.global_scale)))
-            spans.append((n, c, r))
+            ad = ads[n]
+            down, up = ad.down, ad.up
+            r = down.shape[0]
+            if where and not down.is_cuda:
+                pa = where[id(down)]
+            else:
+                pa = down.data_ptr()
+            if where and not up.is_cuda:
+                pb = where[id(up)]
+            else:
+                pb = up.data_ptr()
+            mult = float(ad.weight) * float(r if ad.alpha is None else ad.alpha) / float(r) * float(scale)      # Adapter.multiplier
+            pieces += (pa, pb, r, c, _PIECE_DTYPES[down.dtype], _UNPACK_I(_PACK_F(mult))[0])
+            ranks.append(r)
             c += r
-        packs.append(PackedAdapters(A.as_strided((R, K), (K, 1), at_a), B.as_strided((N, R), (R, 1), at_b), S.as_strided((R,), (1,), at_s), spans, ln=ln))
-        per_block = 256 // (R // 8)
-        b_blocks.append(-(-N // per_block))
+        R = -(-c // RANK_PAD) * RANK_PAD
+        g, nk = l.fold_norm(), None
+        if g is not None:
+            nk = keys.get(id(g))
+            if nk is None:
+                w = g.weight
+                nk = keys[id(g)] = (norm_key(g), w.data_ptr(), g.bias.data_ptr()) if w.dtype == torch.bfloat16 and w.device == dev else ()
+        rows += (at_a, at_an if nk else -1) + (nk[1:] if nk else (0, 0)) + (at_c, at_c, at_b, at_s, K, N, R, int(d["geglu"]), n_pieces, len(ns))
+        packs.append(PooledPack(pool, (at_a, at_b, at_s, at_an, at_c), (R, K, N), ns, ranks, min(R, (c + 15) // 16 * 16), nk[0] if nk else None))
+        n_pieces += len(ns)
+        padded.append(R)
+        b_blocks.append(-(-N // (256 // (R // 8))))
         at_a += R * K
         at_b += R * N
         at_s += R
+        if nk:
+            at_an += R * K
+            at_c += R
+    buf = lambda n, dt: torch.empty((n,), dtype=dt, device=dev)
+    pool += (buf(at_a, torch.bfloat16), buf(at_b, torch.bfloat16), buf(at_s, torch.float32), buf(at_an, torch.bfloat16), buf(at_c, torch.float32), buf(at_c, torch.float32))
+    base = [t.data_ptr() for t in pool]
+    table = np.array(rows, dtype=np.int64).reshape(-1, 14)
+    folded = table[:, 1] >= 0
+    for col, which, size in ((0, 0, 2), (1, 3, 2), (4, 4, 4), (5, 5, 4), (6, 1, 2), (7, 2, 4)):    # offsets -> addresses
+        table[:, col] = base[which] + size * table[:, col]
+    for col in (1, 4, 5):
+        table[~folded, col] = 0
     start = lambda counts: np.concatenate([np.zeros(1, np.int32), np.cumsum(counts, dtype=np.int32)])
-    ops.lora_pack(np.array(rows, dtype=np.int64).reshape(-1, 14), np.array(pieces, dtype=np.int64).reshape(-1, 6), start(padded), start(b_blocks), dev)
+    ops.lora_pack(table, np.array(pieces, dtype=np.int64).reshape(-1, 6), start(padded), start(b_blocks), dev)
     del keep    # stream-ordered: the launches above are enqueued
     return packs
 

@@ -766,3 +766,37 @@ def test_threads_hand_out_and_launch_in_one_order(monkeypatch):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert len(set(got)) == 4000
+
+
+def test_packs_of_a_pool_are_views_made_on_demand():
+    """PooledPack: the views, the addresses that stand for them, and what puts a pack out of its place in the pool."""
+    from katz_amd.lora import PackedAdapters, PooledPack, stacked_norm_terms, stacked_packs
+
+    R, K, N, n = 64, 16, 24, 3
+    pool = [torch.randn(n * R * K).bfloat16(), torch.randn(n * R * N).bfloat16(), torch.randn(n * R), torch.randn(n * R * K).bfloat16(), torch.randn(n * R), torch.randn(n * R)]
+    key = (1, 2, 3, 4)
+    make = lambda: [PooledPack(pool, (i * R * K, i * R * N, i * R, i * R * K, i * R), (R, K, N), ["a", "b"], [8, 20], 32, key) for i in range(n)]
+    packs = make()
+    for i, p in enumerate(packs):
+        assert isinstance(p, PackedAdapters) and p.R == R and p.r_used == 32 and p.spans == [("a", 0, 8), ("b", 8, 20)] and not p.overflow
+        at, at_norm = p.addresses(), p.addresses(key)
+        assert torch.equal(p.a_cat, pool[0].view(n, R, K)[i]) and torch.equal(p.b_cat, pool[1].view(n, N, R)[i]) and torch.equal(p.col_scale, pool[2].view(n, R)[i])
+        assert at == (p.a_cat.data_ptr(), p.b_cat.data_ptr(), p.col_scale.data_ptr(), 0, 0) and p.a_cat is p.a_cat
+        assert p.ln[0] == key and at_norm == (p.ln[1].data_ptr(), *at[1:3], p.ln[2].data_ptr(), p.ln[3].data_ptr())
+        assert p.addresses((5, 6)) is None                        # another norm
+    a, b, s = stacked_packs(packs)
+    assert torch.equal(a, pool[0].view(-1, K)) and torch.equal(b, pool[1].view(-1, R)) and torch.equal(s, pool[2])
+    ap, c1, c2 = stacked_norm_terms(packs, key)
+    assert torch.equal(ap, pool[3].view(-1, K)) and torch.equal(c1, pool[4]) and torch.equal(c2, pool[5])
+    assert stacked_norm_terms(packs, (5, 6)) is None and stacked_packs(packs[::-1]) is None and stacked_packs([packs[0], packs[2]]) is None
+    other = PooledPack(list(pool), packs[1].at, (R, K, N), ["a"], [8], 16, key)
+    plain = PackedAdapters(packs[1].a_cat, packs[1].b_cat, packs[1].col_scale)
+    assert stacked_packs([packs[0], other]) is None and stacked_packs([packs[0], plain]) is None and stacked_packs([plain, packs[2]]) is None
+    for name in ("a_cat", "b_cat", "col_scale"):                  # a tensor of its own takes the view's place
+        packs = make()
+        mine = torch.zeros(1)
+        setattr(packs[1], name, mine)
+        assert getattr(packs[1], name) is mine and packs[1].addresses() is None and stacked_packs(packs) is None and stacked_packs(packs[1:2]) is None
+    packs = make()
+    packs[1].ln = ((7,), None, None, None)                        # the terms of a norm that changed meanwhile
+    assert packs[1].ln[0] == (7,) and packs[1].addresses(key) is None and packs[1].addresses() is not None and stacked_norm_terms(packs, key) is None
