@@ -177,17 +177,19 @@ __device__ __forceinline__ void kh_prefetch_lines_idle(const void* const (&pf)[3
 #if __HIP_DEVICE_COMPILE__
   if (pf[0] == nullptr) return;
   const uint32_t first = ((uint32_t)wg * (uint32_t)nt + (uint32_t)tid) << 7, step = ((uint32_t)n_wg * (uint32_t)nt) << 7;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    if (pf[k] == nullptr) continue;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(pf[k]), 0, (int)(lines[k] << 7), 0x00020000);
-    const uint32_t bytes = lines[k] << 7;                       // at most 2 GiB
+  // (three calls: indexed in a loop the arrays went to scratch memory in some kernels)
+  auto range = [&](const void* at, uint32_t n, uint32_t cap) {
+    if (at == nullptr) return;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, (int)(n << 7), 0x00020000);
+    const uint32_t bytes = n << 7;                       // at most 2 GiB
     uint32_t rounds = (bytes + step - 1) / step;
-    const uint32_t cap = k == 0 ? 16u : 4u;
     rounds = rounds < cap ? rounds : cap;
     for (uint32_t r = 0; r < rounds; ++r)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)wave_lds, 4, first + r * step, 0, 0, 0);
-  }
+  };
+  range(pf[0], lines[0], 16u);
+  range(pf[1], lines[1], 4u);
+  range(pf[2], lines[2], 4u);
 #endif
 }
 
@@ -292,6 +294,7 @@ int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
 // is not suited (orders 2 and 4: the caller has seen to N % 160 and the number of tiles).
 bool lora_gemm_fine_ok(const LoraGemmParams& p);
 int lora_gemm_fine_form(const LoraGemmParams& p, int order);
+int lora_gemm_geglu_form(const LoraGemmParams& p);           // of a GEGLU projection; -2: the 256 x 320 tiles of lora_gemm_wide.hip, -1: neither
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream);
 // the fine tile that a call with T given runs on, -1 where another kernel is chosen
 int lora_gemm_pipe_fine_form(const LoraGemmParams& p);

@@ -64,20 +64,21 @@ template <int BM_, int BN_, int ORD_, bool GLU_ = false>
 struct FCfg {
   static constexpr int BM = BM_, BN = BN_, ORD = ORD_;
   static constexpr bool GLU = GLU_;                      // GEGLU epilogue
+  static constexpr int CW = GLU ? 8 : 4, CT = CW * 64, NT = CT + 256;   // computing waves (and four that move operands), their threads, all threads
   static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? (BM == 64 ? 4 : 2) : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
-                       WM = 4 / (WK * WN);
-  // 32-row MFMA tiles for the slices where the tile divides into them, and for GEGLU on 128 rows, whose 160 accumulators leave no room for a 32-column
-  // step of 16-row fragments (72 registers against 36: 56 spilled); 16-row tiles otherwise (16x16x16 has half the rate)
-  static constexpr int MF = (ORD != 0 && BN % 32 == 0) || (GLU && BM == 128) ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
+  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? 4 : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
+                       WM = CW / (WK * WN);
+  // 32-row MFMA tiles for the slices where the tile divides into them, 16-row tiles otherwise (16x16x16 has half the rate)
+  static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
   static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN);                           // a wave's MFMA tiles
-  static constexpr int KS = ORD == 4 ? 1 : ORD == 0 && MF == 32 ? 4 : 2;                   // its k-steps per stage
+  static constexpr int KS = ORD == 4 ? 1 : 2;                                            // its k-steps per stage
   // operand order of the matrix instructions: (W, x) leaves four columns of a row in a lane, so that the epilogue writes 8 bytes at a time
   // (128 x 320: 5.6 K clocks against 8.4 K), (x, W) four rows of a column.  One x fragment per W fragment is the exception: the K loop of 64 x 80
   // takes 8.8 K clocks with (x, W) and 9.9 K with (W, x), more than the epilogue saves.
   static constexpr bool XW = BM == 64 && BN == 80 && ORD == 0;
   static constexpr bool DB = TM * TN * G * 4 <= 96 && BM <= 128 && !GLU;      // two fragment buffers where the registers allow it
+  static constexpr bool SA = CW == 8;                    // one buffer of x fragments: 168 registers a wave
   static constexpr int BK = 64, ROWB = BK * 2, PPR = BK / 8, UR = 64 / PPR;      // a stage row's bytes, 16-byte pieces; rows per DMA instruction
   static constexpr int ROWS = BM + BN, STAGE = ROWS * ROWB;
   static constexpr int UNITS = ROWS / UR, LPS_LO = UNITS / 4, N_HI = UNITS % 4, LPS_HI = LPS_LO + (N_HI ? 1 : 0);
@@ -88,10 +89,9 @@ struct FCfg {
   static constexpr int PART = GLU ? 0 : WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
   static constexpr int TAIL = PART + BM * LDC * 2;
   static constexpr int NST = cmin(16, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;  // as many stages as fit, but at most 16
-  static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + 1024;   // (where prefetched dwords nobody reads land)
-  static constexpr int OPC = BM * (BN / 8), OPT = (OPC + 511) / 512;             // 16-byte output pieces: per tile, per thread
-  static_assert(ORD != 4 || MF == 32 || KS == 1, "k-steps");
-  static_assert(WM * WN * WK == 4 && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
+  static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + CW * 256;   // (where prefetched dwords nobody reads land)
+  static constexpr int OPC = BM * (BN / 8), OPT = (OPC + NT - 1) / NT;             // 16-byte output pieces: per tile, per thread
+  static_assert(WM * WN * WK == CW && TM * MF * WM == BM && TN * MF * WN == BN && TM % NH == 0 && TM / NH * TN * G % WK == 0, "tile");
   static_assert(BM % 32 == 0 && XQ * UR * 4 == BM && ROWS % UR == 0, "whole DMA instructions");
   static_assert(NST >= 2 && LPS_HI * (PD - 1) < 63 && LDS + KH_LN_LDS <= 160 * 1024, "ring");
 };
@@ -124,15 +124,15 @@ constexpr int il_lds(int waves) { return waves == 8 ? cmax(SHRINK16_LDS<8>, SCfg
 // XA: the layer is an attention's to_q; a tile's rows are queries of one sample, its columns whole heads, and the epilogue runs the cross-attention on
 // them (xattn_tile.h).
 template <class C, bool CONV, int TMODE, bool XA = false>
-__global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p0, const int seg_rows, const int seg_tiles) {
+__global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) void lora_gemm_fine_kernel(const LoraGemmParams p0, const int seg_rows, const int seg_tiles) {
 #if __HIP_DEVICE_COMPILE__   // the host pass only needs the kernel's symbol (it cannot lower the buffer-resource type)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, NST = C::NST, PD = C::PD;
   constexpr int BK = C::BK, ROWB = C::ROWB, UR = C::UR, PPR = C::PPR, STAGE = C::STAGE, LPS_LO = C::LPS_LO, LPS_HI = C::LPS_HI, XQ = C::XQ;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool producer = wave >= 4;                     // waves 4 .. 7 move operands, waves 0 .. 3 compute
-  const int pw = wave & 3, wm = pw / (C::WK * C::WN), wn = pw / C::WK % C::WN, wk = pw % C::WK;
+  const bool producer = wave >= C::CW;                 // the last four waves move operands, the others compute
+  const int pw = C::CW == 4 || producer ? wave & 3 : wave & (C::CW - 1), wm = pw / (C::WK * C::WN), wn = pw / C::WK % C::WN, wk = pw % C::WK;
   const int lr = lane % C::MF, lg = lane / C::MF;      // row inside an MFMA tile, 16-byte (8-byte) piece of a k-step
 
   constexpr bool COOP = TMODE == T_COOP, GRP = TMODE == T_GRP;
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   int fa[KS], fb[KS];
 #pragma unroll
   for (int k = 0; k < KS; ++k) {
-    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::MF == 16 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
+    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
     fa[k] = (wm * (BM / C::WM) + lr) * ROWB + po;
     fb[k] = (BM + wn * (BN / C::WN) + lr) * ROWB + po;
   }
@@ -291,11 +291,12 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   // K loop.  Step t: tile t is in the computing waves' registers (cur); tile t+1 becomes visible at the barrier, after which
   // every wave has read tile t out of its stage, so that stage takes tile t + NST.  Both kinds of waves pass KT barriers.
   // (the epilogue's per-row and per-column terms are the producers' to fetch: ten registers less in the computing waves)
-  float* sMu = reinterpret_cast<float*>(smem + C::LDS);      // [128] mean, [128] 1/std, [BN] x 2
-  float* sRs = sMu + 128;
-  float* sc1 = sRs + 128;
+  float* sMu = reinterpret_cast<float*>(smem + C::LDS);      // [LNR] mean, [LNR] 1/std, [BN] x 2
+  constexpr int LNR = cmax(BM, 128);
+  float* sRs = sMu + LNR;
+  float* sc1 = sRs + LNR;
   float* sc2 = sc1 + BN;
-  static_assert((256 + 2 * BN) * 4 <= KH_LN_LDS && (BM <= 128 || GRP), "per-row and per-column terms");
+  static_assert((2 * LNR + 2 * BN) * 4 <= KH_LN_LDS, "per-row and per-column terms");
   typedef XAttnFine<cmax(BN / 64, 1), 256, C::LDC> XAttn;
   XAttn kv;                                            // XA: the keys and values, in the producers
   if (producer) {
@@ -407,8 +408,8 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
 
     // requested now, used after the K loop (older than every DMA load, so no wait falls in between)
     constexpr int CP = (BN + 255) / 256;
-    const int ptid = tid - 256;
-    KhLnTileStats<cmin(BM, 128), 256> ln_stats;
+    const int ptid = tid - C::CT;
+    KhLnTileStats<GRP ? cmin(BM, 128) : BM, 256> ln_stats;
     float c1v[CP], c2v[CP];
     uint16_t biasv[CP];
     if (p.ln_part != nullptr) ln_stats.load(p.ln_part, m0, M, ptid);
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
     auto touch = [&](int t, auto n) {
       if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
-        kh_touch_rows<decltype(n)::value>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * 256 + tid, p.xr_m * p.xr_n * 256);
+        kh_touch_rows<decltype(n)::value>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * C::CT + tid, p.xr_m * p.xr_n * C::CT);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
@@ -460,18 +461,60 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
     constexpr std::integral_constant<int, 8> EIGHT{};
     touch(0, std::integral_constant<int, TOUCH>{});
     if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128 && il_prefetch_by_idle_waves(p)))
-      kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, 256);
+      kh_prefetch_lines(p.pf, p.pf_lines, smem + C::TOUCH_OFF + pw * 256, bid, n_wg, tid, C::CT);
     uint16_t* gtab = reinterpret_cast<uint16_t*>(smem + C::TAB_OFF);
     if constexpr (C::GLU) {
 #pragma unroll 4
-      for (int i = tid; i < 2 * GTAB_N; i += 256) {
+      for (int i = tid; i < 2 * GTAB_N; i += C::CT) {
         const uint32_t bits = (uint32_t)(i >= GTAB_N ? 0x8000 + (i - GTAB_N) : i) + GTAB_LO;
         gtab[i] = (uint16_t)pack_bf16x2(kh_gelu_erf(bf16_lo(bits)), 0.f);
       }
     }
     ring_barrier();
     int st = 0;
-    if constexpr (!C::DB) {
+    if constexpr (C::SA) {
+      // Two waves per SIMD compute, so that one's reads run under the other's matrix instructions, and a wave has 168 registers: one set of x fragments,
+      // each replaced behind the instruction of a k-step that used it last, and two fragments of W.  The barrier that shows the next stage lies behind the
+      // reads of this stage's last fragments, three columns before its end.
+      static_assert(KS == 2 && TN >= 3 && C::MF == 16, "columns of a stage");
+      Frag a[TM], b[2];
+      auto read_a = [&](int st, int k, int i) { a[i] = *reinterpret_cast<const Frag*>(smem + st + fa[k] + i * C::MF * ROWB); };
+      auto read_b = [&](int st, int g, int to) { b[to] = *reinterpret_cast<const Frag*>(smem + st + fb[g / TN] + g % TN * C::MF * ROWB); };
+      auto stage = [&](auto last_tag) {
+        constexpr bool LAST = decltype(last_tag)::value;
+        int nxt = st;
+#pragma unroll
+        for (int g = 0; g < 2 * TN; ++g) {
+          const int k = g / TN, j = g % TN;
+          if (!LAST && g == 2 * TN - 2) {
+            nxt = st + STAGE == NST * STAGE ? 0 : st + STAGE;
+            wait_cnt<63, 0>();
+            ring_barrier();
+          }
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            mfma(a[i], b[g & 1], acc[i][j]);
+            if (j == TN - 1 && (k == 0 || !LAST)) {
+              read_a(k == 0 ? st : nxt, 1 - k, i);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+          if (g + 2 < 2 * TN) read_b(st, g + 2, g & 1);
+          else if (!LAST) read_b(nxt, g + 2 - 2 * TN, g & 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        st = nxt;
+      };
+#pragma unroll
+      for (int i = 0; i < TM; ++i) read_a(0, 0, i);
+      read_b(0, 0, 0);
+      read_b(0, 1, 1);
+      for (int t = 0; t + 1 < KT; ++t) {
+        if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
+        stage(std::false_type{});
+      }
+      stage(std::true_type{});
+    } else if constexpr (!C::DB) {
       // One set of W fragments, replaced one by one behind the matrix instructions that used them last, and two of x, a k-step each: the
       // reads of the next k-step run under the matrix instructions of this one.  (A whole stage read and then multiplied takes the sum of both
       // where the operands arrive in time: GEGLU on 64 x 320 tiles, 2048 / 5120 / 640, 25.2 -> 24.0 us.)  The barrier that shows the next stage lies before the last k-step, whose fragments have
@@ -503,18 +546,14 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
       read_a(0, 0, 0);
 #pragma unroll
       for (int j = 0; j < TN; ++j) read_b(0, 0, j);
-      if constexpr (KS % 2 == 0) {
-        auto stage_steps = [&]() {                     // all k-steps but the last
-#pragma unroll
-          for (int k = 0; k + 1 < KS; ++k) kstep(k & 1, st, k + 1);
-        };
+      if constexpr (KS == 2) {
         for (int t = 0; t + 1 < KT; ++t) {
           if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
-          stage_steps();
+          kstep(0, st, 1);
           next_stage();
           kstep(1, st, 0);
         }
-        stage_steps();
+        kstep(0, st, 1);
       } else {
         int t = 0;
         for (; t + 2 < KT; t += 2) {
@@ -532,7 +571,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
         }
       }
 #pragma unroll
-      for (int j = 0; j < TN; ++j) mma1(KS % 2 == 0 ? 1 : 0, j);
+      for (int j = 0; j < TN; ++j) mma1(KS == 2 ? 1 : 0, j);
     } else {
     Fr f0, f1;
     read_frags(0, f0);
@@ -559,13 +598,13 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   if (p.res != nullptr) {
 #pragma unroll
     for (int q = 0; q < C::OPT; ++q) {
-      const int c = tid + q * 512, srow = c / (BN / 8), ch = c % (BN / 8);
+      const int c = tid + q * C::NT, srow = c / (BN / 8), ch = c % (BN / 8);
       rr[q] = (c < C::OPC && srow < rows) ? *reinterpret_cast<const u32x4*>(p.res + (size_t)(m0 + srow) * N + n0 + ch * 8) : u32x4{0, 0, 0, 0};
     }
   }
   __syncthreads();   // the ring is dead: partial sums and the staging tiles reuse it
   if constexpr (XA)
-    if (producer) kv.store(smem + (C::TAIL + 15) / 16 * 16, tid - 256);
+    if (producer) kv.store(smem + (C::TAIL + 15) / 16 * 16, tid - C::CT);
 
   // the k-slices meet in LDS: every wave leaves all its tiles and finishes every WK-th of them
   f32x4* part = reinterpret_cast<f32x4*>(smem);
@@ -595,9 +634,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int g = 0; g < C::G; ++g) finish(group(acc[i][j], g), i, j, g);
+        for (int i = 0; i < TM; ++i) finish(group(acc[i][j], 0), i, j, 0);
     }
   } else {
     constexpr int UH = TM / C::NH * TN * C::G;           // groups of a pass
@@ -638,13 +675,13 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   }
   if constexpr (C::GLU) {
     // staged columns come in groups of 64 = 32 value columns then their 32 gate columns
-    constexpr int OPR = BN / 16, GCH = (BM * OPR + 511) / 512;
+    constexpr int OPR = BN / 16, GCH = (BM * OPR + C::NT - 1) / C::NT;
     const int out_ld = N / 2;
     const KhOut gout(p.y, (size_t)M * out_ld * 2);
     const uint16_t* gtab = reinterpret_cast<const uint16_t*>(smem + C::TAB_OFF);
 #pragma unroll
     for (int q = 0; q < GCH; ++q) {
-      const int c = tid + q * 512, srow = c / OPR, oc = c % OPR, grp = oc >> 2, sub = oc & 3;
+      const int c = tid + q * C::NT, srow = c / OPR, oc = c % OPR, grp = oc >> 2, sub = oc & 3;
       if (c >= BM * OPR || srow >= rows) continue;
       const u32x4 hv = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + grp * 64 + sub * 8);
       const u32x4 gv = *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + grp * 64 + 32 + sub * 8);
@@ -674,7 +711,7 @@ __global__ __launch_bounds__(512, TMODE == T_COOP ? 1 : 2) void lora_gemm_fine_k
   float* sp = reinterpret_cast<float*>(smem);          // row statistics: [BM][BN / 8][2], the partial sums are dead
 #pragma unroll
   for (int q = 0; q < C::OPT; ++q) {
-    const int c = tid + q * 512, srow = c / (BN / 8), ch = c % (BN / 8);
+    const int c = tid + q * C::NT, srow = c / (BN / 8), ch = c % (BN / 8);
     const bool ok = c < C::OPC && srow < rows;
     u32x4 o = ok ? *reinterpret_cast<const u32x4*>(sC + srow * C::LDC + ch * 8) : u32x4{0, 0, 0, 0};
     if (p.res != nullptr) {
@@ -785,7 +822,7 @@ int launch_fine(LoraGemmParams p, hipStream_t stream) {
     if (!plan_il<C>(p)) return KH_ERR_UNSUPPORTED;
   if (hipError_t e = kh_allow_lds<lora_gemm_fine_kernel<C, CONV, TMODE, XA>>(C::LDS + KH_LN_LDS); e != hipSuccess) return (int)e;
   const unsigned grid = (unsigned)(TMODE == T_IL ? p.il_blocks : 0) + 8u * (unsigned)p.xr_m * (unsigned)p.xr_n;
-  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, TMODE, XA>, dim3(grid), dim3(512), (size_t)C::LDS + KH_LN_LDS, stream, p,
+  kh_launch(CONV ? KH_TAG_CONV : KH_TAG_LORA_GEMM, lora_gemm_fine_kernel<C, CONV, TMODE, XA>, dim3(grid), dim3(C::NT), (size_t)C::LDS + KH_LN_LDS, stream, p,
             seg_rows, (seg_rows + C::BM - 1) / C::BM);
   KH_RETURN_LAST_ERROR();
 }
@@ -804,7 +841,7 @@ bool lora_gemm_fine_ok(const LoraGemmParams& p) {
 }
 
 // Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
-// GEGLU on 64 x 320 (7), 128 x 320 (8); order 2 on 128 x 160 (9); order 0 on 32 x 32 (10), 32 x 64 (11), 64 x 64 (12);
+// GEGLU on 64 x 320 (7), 128 x 320 (8), 160 x 320 (17), 192 x 320 (18); order 2 on 128 x 160 (9); order 0 on 32 x 32 (10), 32 x 64 (11), 64 x 64 (12);
 // order 4 on 32 x 32 (13), 32 x 64 (14), 64 x 64 (15).
 //
 // Order 2: wave tiles of 64 x 160 over two k-slices and waves of their own for the operands, in place of eight 32 x 160 strips that did
@@ -857,19 +894,36 @@ static int shrink_beside(LoraGemmParams& p, int form) {
 // us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
 // 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
 // 512 / 1280 / 1280, 32 10.1 -> 9.3; 300 / 640 / 640, 64 7.3 -> 6.4; no adapters: 154 / 640 / 2048 12.1 -> 8.3, 655 / 1280 / 2048 12.2 -> 11.1.
+// GEGLU projections: of 64 / 128 / 160 / 192 x 320 tiles and the 256 x 320 ones of lora_gemm_wide.hip (-2) those whose rounds of the CUs take least; -1: 128 x 128 tiles.
+// A round costs about 100 rows more than its tiles have (its start, its epilogue; the 256-row tiles, whose waves move their own operands, 150).
+// us per launch without adapters, weights from HBM, before (in several rounds 128 x 320 on four computing waves, or 128 x 128) -> now: N 10240 / K 1280, M 512 22.7 ->
+// 22.1, 1024 34.5 -> 31.4, 1152 48 -> 34.6, 1280 55.5 -> 35.5, 1400 57.4 -> 40.3, 1536 47.8 -> 40.5, 1800 69.8 -> 56.0, 1976 71.4 -> 58.1, 2048 (256 rows) 55.8, 58.9 on 128;
+// N 5120 / K 640, M 1100 17.8 -> 16.0, 2304 28.7 -> 21.5, 3072 30.1 -> 25.7, 3952 44.2 -> 35.4, 4096 (256 rows) 33.7, 4608 50.3 -> 40.5, 6000 64.6 -> 50.6, 7200 77.7 -> 62.8,
+// 8192 (256 rows) 64.2, 69.6 on 192.
+int lora_gemm_geglu_form(const LoraGemmParams& p) {
+  if (!lora_gemm_fine_ok(p) || p.st_part != nullptr || p.res != nullptr || p.N % 320 != 0 || p.t_nsplit % 320 != 0) return -1;
+  if ((long)((p.M + 63) / 64) * (p.N / 320) <= 128) return -1;           // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
+  const auto cost = [&](int bm, int more) {
+    const KhXcdGrid g = kh_xcd_grid((p.M + bm - 1) / bm, p.N / 320, bm, 320);
+    return ((long)g.rm * g.rn + 31) / 32 * (bm + more);
+  };
+  constexpr struct { int form, bm; } tiles[] = {{7, 64}, {8, 128}, {17, 160}, {18, 192}};
+  int best = -1;
+  long least = 0;
+  for (const auto& t : tiles)
+    if (const long c = cost(t.bm, 100); best < 0 || c < least) { least = c; best = t.form; }
+  return lora_gemm_wide_ok(p) && cost(256, 150) < least ? -2 : best;
+}
+
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   if (!lora_gemm_fine_ok(p)) return -1;
   const long hw = p.gn_part != nullptr ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
   auto tiles_of = [&](int bm, int bn) { return nb * ((hw + bm - 1) / bm) * (p.N / bn); };
   auto fits = [&](int bm, int bn) { return p.N % bn == 0 && p.t_nsplit % bn == 0 && (p.st_part == nullptr || p.N / bn <= KH_LN_SLOTS) && tiles_of(bm, bn) <= 256; };
   auto pieces_of = [&](int size) { return (long)((p.M + size - 1) / size) * (((p.r_used > 0 ? p.r_used : p.R) + size - 1) / size) * (p.ldt / p.R); };
-  if (p.geglu) {   // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
-    if (order != 0 || p.st_part != nullptr || p.res != nullptr) return -1;
-    if (fits(64, 320)) return tiles_of(64, 320) > 128 ? 7 : -1;
-    // 128 x 320 also in several rounds that are nearly full, where the rows are ragged for 256 x 320 (1976 / 10240 / 1280, R 128 79 -> 70 us, 1800 75 -> 69;
-    // K 640 gains nothing, 3952 / 5120 / 640 44.6 against 45.6; 11 of 16 of a round full: 1300 / 10240 / 1280 59 against 66)
-    const long t = p.N % 320 == 0 ? tiles_of(128, 320) : 0, rounds = (t + 255) / 256;
-    return fits(128, 320) || (t > 256 && p.t_nsplit % 320 == 0 && p.K >= 1024 && t * 8 >= rounds * 256 * 7) ? 8 : -1;
+  if (p.geglu) {
+    const int form = order == 0 ? lora_gemm_geglu_form(p) : -1;
+    return form >= 0 ? form : -1;
   }
   if (order == 2) return 9;
   if (p.conv_cin > 0) return p.gn_part != nullptr ? (80 % p.gn_cg == 0 && fits(64, 80) ? 6 : 5) : fits(32, 160) ? 4 : 5;
@@ -904,7 +958,7 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
   const bool conv = p.conv_cin > 0;
   // (a forced form comes here without the rule above)
-  if (!lora_gemm_fine_ok(p) || (p.geglu ? (form != 7 && form != 8) || p.st_part != nullptr || p.res != nullptr : form == 7 || form == 8)) return KH_ERR_UNSUPPORTED;
+  if (!lora_gemm_fine_ok(p) || (p.geglu ? (form != 7 && form != 8 && form != 17 && form != 18) || p.st_part != nullptr || p.res != nullptr : form == 7 || form == 8 || form == 17 || form == 18)) return KH_ERR_UNSUPPORTED;
   switch (form) {
     case 0: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<64, 80, 0>, false>(p, stream);
     case 1: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<128, 80, 0>, false>(p, stream);
@@ -915,6 +969,8 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 6: return conv ? launch_fine<FCfg<64, 80, 4>, true>(p, stream) : KH_ERR_UNSUPPORTED;
     case 7: return launch_fine<FCfg<64, 320, 0, true>, false>(p, stream);
     case 8: return launch_fine<FCfg<128, 320, 0, true>, false>(p, stream);
+    case 17: return launch_fine<FCfg<160, 320, 0, true>, false>(p, stream);
+    case 18: return launch_fine<FCfg<192, 320, 0, true>, false>(p, stream);
     case 9: return conv ? launch_fine<FCfg<128, 160, 2>, true>(p, stream) : launch_fine<FCfg<128, 160, 2>, false>(p, stream);
     case 10: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 32, 0>, false>(p, stream);
     case 11: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 64, 0>, false>(p, stream);

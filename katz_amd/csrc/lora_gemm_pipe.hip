@@ -1358,6 +1358,7 @@ int lora_gemm_pipe_launch_grouped(const LoraGemmParams& p, int n_groups, hipStre
 // FLOP than any smaller tile and no ragged last round
 static bool wide_fills(const LoraGemmParams& p) {
   if (!lora_gemm_wide_ok(p)) return false;
+  if (p.geglu && lora_gemm_fine_ok(p)) return lora_gemm_geglu_form(p) == -2;
   const long wt = (long)(p.M / 256) * (p.N / 320), rounds = (wt + 255) / 256;
   return wt * 4 >= rounds * 256 * 3;
 }
@@ -1387,7 +1388,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     case 40: return lora_gemm_ksplit_launch(p, 2, stream);
     case 41: return lora_gemm_ksplit_launch(p, 4, stream);
     case 42: return lora_gemm_wide_launch(p, stream);
-    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: case 59: case 60: case 61: case 62: case 63: case 64: case 65: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
+    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: case 59: case 60: case 61: case 62: case 63: case 64: case 65: case 67: case 68: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
     default: break;
   }
   // Default choice.  The limiter is the vector L1 path (every operand byte enters LDS through it), so

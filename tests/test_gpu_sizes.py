@@ -860,3 +860,45 @@ def test_attention_waves_of_16_queries(T, S):
         n = units // (3 * H * blocks) + 1
         more = ops.attention(*(t.repeat(n, 1, 1) for t in (q, k, v)), H)
         assert torch.equal(more.view(n, *o.shape), o.expand(n, *o.shape))
+
+
+@pytest.mark.parametrize("M,N,K,R", [(1, 320, 64, 0), (95, 640, 128, 32), (160, 640, 192, 64), (161, 320, 64, 128), (193, 960, 320, 64), (385, 640, 1280, 128), (1153, 10240, 640, 64)])
+def test_geglu_tiles_of_160_and_192_rows(M, N, K, R):
+    """Eight computing waves of 80 or 96 rows x 80 columns: ragged rows, one to many stages, rank columns; the bits of the 128 x 128 kernel (code 16)."""
+    from katz_amd import ops
+
+    say("geglu, 160 and 192 rows", M, N, K, R)
+    d, g = dev(), torch.Generator().manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b = rnd(M, K), rnd(N, K) * K ** -0.5, rnd(N)
+    t, bc = (rnd(M, R), rnd(N, R) * 0.05) if R else (None, None)
+    run = (lambda c: ops.lora_linear_pre(x, w, b, t, bc, geglu=True, tile=c)) if R else (lambda c: ops.lora_linear(x, w, b, geglu=True, tile=c))
+    want = run(16)
+    for code in (57, 58, 67, 68):
+        assert torch.equal(run(code), want), code
+
+
+@pytest.mark.parametrize("M,N,K,ln", [(1100, 10240, 1280, True), (1300, 10240, 1280, True), (4500, 5120, 640, True), (2500, 5120, 640, False), (2048, 10240, 1280, False)])
+def test_geglu_on_the_tiles_whose_rounds_take_least(M, N, K, ln):
+    """What the rule chooses between 1024 and 2048 rows and at several rounds: the
+    bits of the 128 x 128 kernel where nothing is folded, the oracle's arithmetic otherwise."""
+    from katz_amd import ops
+    from katz_amd.lora import fold_norm_into_weight
+
+    say("geglu, chosen tiles", M, N, K, ln)
+    d, g = dev(), torch.Generator().manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b = rnd(M, K), rnd(N, K) * K ** -0.5, rnd(N)
+    if not ln:
+        assert torch.equal(ops.lora_linear(x, w, b, geglu=True), ops.lora_linear(x, w, b, geglu=True, tile=16))
+        return
+    gamma, beta = 1 + rnd(K) * 0.1, rnd(K) * 0.1
+    wp, c1, c2 = fold_norm_into_weight(w, b, gamma, beta)
+    part = torch.zeros(ops.LN_SLOTS, M, 2, device=d)
+    part[0, :, 0], part[0, :, 1] = x.float().sum(1), (x.float() ** 2).sum(1)
+    y = ops.lora_linear_norm(x, wp, None, geglu=True, ln=(part, c1, c2, None, None, 1e-5))
+    n = torch.nn.functional.layer_norm(x.double(), (K,), gamma.double(), beta.double(), 1e-5)
+    h = (n @ w.double().T + b.double()).view(M, N // 64, 2, 32)
+    ref = (h[:, :, 0] * torch.nn.functional.gelu(h[:, :, 1])).reshape(M, N // 2)
+    # bf16 roundings of the folded weights, of value and gate and of the product: 2^-9 each
+    assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3
