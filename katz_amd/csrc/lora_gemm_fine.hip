@@ -64,15 +64,15 @@ template <int BM_, int BN_, int ORD_, bool GLU_ = false>
 struct FCfg {
   static constexpr int BM = BM_, BN = BN_, ORD = ORD_;
   static constexpr bool GLU = GLU_;                      // GEGLU epilogue
-  static constexpr int CW = GLU ? 8 : 4, CT = CW * 64, NT = CT + 256;   // computing waves (and four that move operands), their threads, all threads
+  static constexpr int CW = GLU || ORD == 2 ? 8 : 4, CT = CW * 64, NT = CT + 256;   // computing waves (and four that move operands), their threads, all threads
   static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? 4 : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
+  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? 4 : ORD == 2 ? 2 : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
                        WM = CW / (WK * WN);
   // 32-row MFMA tiles for the slices where the tile divides into them, 16-row tiles otherwise (16x16x16 has half the rate)
-  static constexpr int MF = ORD != 0 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
+  static constexpr int MF = ORD == 4 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
   static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN);                           // a wave's MFMA tiles
-  static constexpr int KS = ORD == 4 ? 1 : 2;                                            // its k-steps per stage
+  static constexpr int KS = ORD == 0 ? 2 : 1;                                            // its k-steps per stage
   // operand order of the matrix instructions: (W, x) leaves four columns of a row in a lane, so that the epilogue writes 8 bytes at a time
   // (128 x 320: 5.6 K clocks against 8.4 K), (x, W) four rows of a column.  One x fragment per W fragment is the exception: the K loop of 64 x 80
   // takes 8.8 K clocks with (x, W) and 9.9 K with (W, x), more than the epilogue saves.
@@ -85,8 +85,8 @@ struct FCfg {
   static constexpr int XQ = BM / UR / 4;                                         // DMA units q < XQ are x rows for every wave
   static constexpr int LDC = BN + 8;
   // partial sums of the k-slices (NH passes over the row tiles) / row statistics
-  static constexpr int NH = WK > 1 && 4 * TM * TN * G > 80 ? 2 : 1;
-  static constexpr int PART = GLU ? 0 : WK > 1 ? 4 * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
+  static constexpr int NH = WK > 1 && CW * TM * TN * G > 80 ? 2 : 1;
+  static constexpr int PART = GLU ? 0 : WK > 1 ? CW * TM / NH * TN * G * 1024 : (BM * (BN / 8) * 8 + 1023) / 1024 * 1024;
   static constexpr int TAIL = PART + BM * LDC * 2;
   static constexpr int NST = cmin(16, (159 * 1024 - KH_LN_LDS - TAB) / STAGE), PD = NST - 1;  // as many stages as fit, but at most 16
   static constexpr int TAB_OFF = cmax(NST * STAGE, TAIL), TOUCH_OFF = TAB_OFF + TAB, LDS = TOUCH_OFF + CW * 256;   // (where prefetched dwords nobody reads land)
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
     sp.M = M; sp.K = K; sp.R = p.ldt;
     sp.ln_part = p.ln_part; sp.ln_ca1 = p.ln_ca1; sp.ln_ca2 = p.ln_ca2; sp.ln_eps = p.ln_eps;
     // (a quarter that starts past the last row has nothing to compute: the tile's addressing assumes m0 < M)
-    if (m0 + 32 * q4 < M) lora_shrink_tile<SCfg<4, 1, 3>, true, 512>(sp, m0 + 32 * q4, grp * 128, smem);
+    if (m0 + 32 * q4 < M) lora_shrink_tile<SCfg<4, 1, 3>, true, C::NT>(sp, m0 + 32 * q4, grp * 128, smem);
     if (tid < 128) {   // columns 96 .. 127 of the group: 32 rows x 4 pieces of 16 bytes
       const int row = m0 + 32 * q4 + (tid >> 2);
       if (row < M) {
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
   int fa[KS], fb[KS];
 #pragma unroll
   for (int k = 0; k < KS; ++k) {
-    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::ORD == 0 ? 4 * k + lg : 2 * (KS * wk + k) + lg) ^ swz(lr)) * 16;
+    const int po = HALF ? ((2 * wk + (lg >> 1)) ^ swz(lr)) * 16 + (lg & 1) * 8 : ((C::MF == 16 ? 4 * (C::ORD == 0 ? k : wk) + lg : 2 * wk + lg) ^ swz(lr)) * 16;
     fa[k] = (wm * (BM / C::WM) + lr) * ROWB + po;
     fb[k] = (BM + wn * (BN / C::WN) + lr) * ROWB + po;
   }
@@ -476,39 +476,40 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
       // Two waves per SIMD compute, so that one's reads run under the other's matrix instructions, and a wave has 168 registers: one set of x fragments,
       // each replaced behind the instruction of a k-step that used it last, and two fragments of W.  The barrier that shows the next stage lies behind the
       // reads of this stage's last fragments, three columns before its end.
-      static_assert(KS == 2 && TN >= 3 && C::MF == 16, "columns of a stage");
-      Frag a[TM], b[2];
+      static_assert(TN >= 3 && C::MF == 16, "columns of a stage");
+      constexpr int G = KS * TN, NB = G % 2 == 0 ? 2 : TN;   // columns of a stage; fragments of W in registers (a stage ends where it began)
+      Frag a[TM], b[NB];
       auto read_a = [&](int st, int k, int i) { a[i] = *reinterpret_cast<const Frag*>(smem + st + fa[k] + i * C::MF * ROWB); };
-      auto read_b = [&](int st, int g, int to) { b[to] = *reinterpret_cast<const Frag*>(smem + st + fb[g / TN] + g % TN * C::MF * ROWB); };
+      auto read_b = [&](int st, int g) { b[g % NB] = *reinterpret_cast<const Frag*>(smem + st + fb[g / TN] + g % TN * C::MF * ROWB); };
       auto stage = [&](auto last_tag) {
         constexpr bool LAST = decltype(last_tag)::value;
         int nxt = st;
 #pragma unroll
-        for (int g = 0; g < 2 * TN; ++g) {
+        for (int g = 0; g < G; ++g) {
           const int k = g / TN, j = g % TN;
-          if (!LAST && g == 2 * TN - 2) {
+          if (!LAST && g == G - NB) {
             nxt = st + STAGE == NST * STAGE ? 0 : st + STAGE;
             wait_cnt<63, 0>();
             ring_barrier();
           }
 #pragma unroll
           for (int i = 0; i < TM; ++i) {
-            mfma(a[i], b[g & 1], acc[i][j]);
-            if (j == TN - 1 && (k == 0 || !LAST)) {
-              read_a(k == 0 ? st : nxt, 1 - k, i);
+            mfma(a[i], b[g % NB], acc[i][j]);
+            if (j == TN - 1 && (k + 1 < KS || !LAST)) {
+              read_a(k + 1 < KS ? st : nxt, k + 1 < KS ? k + 1 : 0, i);
               __builtin_amdgcn_sched_barrier(0);
             }
           }
-          if (g + 2 < 2 * TN) read_b(st, g + 2, g & 1);
-          else if (!LAST) read_b(nxt, g + 2 - 2 * TN, g & 1);
+          if (g + NB < G) read_b(st, g + NB);
+          else if (!LAST) read_b(nxt, g + NB - G);
           __builtin_amdgcn_sched_barrier(0);
         }
         st = nxt;
       };
 #pragma unroll
       for (int i = 0; i < TM; ++i) read_a(0, 0, i);
-      read_b(0, 0, 0);
-      read_b(0, 1, 1);
+#pragma unroll
+      for (int g = 0; g < NB; ++g) read_b(0, g);
       for (int t = 0; t + 1 < KT; ++t) {
         if ((t & 7) == 0) touch(t + TOUCH, EIGHT);
         stage(std::false_type{});
