@@ -294,6 +294,7 @@ int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
 // is not suited (orders 2 and 4: the caller has seen to N % 160 and the number of tiles).
 bool lora_gemm_fine_ok(const LoraGemmParams& p);
 int lora_gemm_fine_form(const LoraGemmParams& p, int order);
+int lora_gemm_rounds_form(const LoraGemmParams& p);          // of a convolution or a linear layer with many rows in order 0; -1: none
 int lora_gemm_geglu_form(const LoraGemmParams& p);           // of a GEGLU projection; -2: the 256 x 320 tiles of lora_gemm_wide.hip, -1: neither
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream);
 // the fine tile that a call with T given runs on, -1 where another kernel is chosen

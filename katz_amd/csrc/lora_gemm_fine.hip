@@ -67,7 +67,7 @@ struct FCfg {
   static constexpr int CW = GLU || ORD == 2 ? 8 : 4, CT = CW * 64, NT = CT + 256;   // computing waves (and four that move operands), their threads, all threads
   static constexpr int TAB = GLU ? 2 * GTAB_N * 2 : 0;   // its table of bf16(gelu(gate)), see lora_gemm_wide.hip
   // computing waves: WM row groups x WN column groups x WK k-slices
-  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? 4 : ORD == 2 ? 2 : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 ? 1 : 2,
+  static constexpr int WK = ORD == 0 ? 1 : ORD, WN = GLU ? 4 : ORD == 2 ? 2 : ORD != 0 ? 1 : BM == 32 ? (BN >= 64 ? 4 : 2) : BN % 128 != 0 && BN != 160 ? 1 : 2,
                        WM = CW / (WK * WN);
   // 32-row MFMA tiles for the slices where the tile divides into them, 16-row tiles otherwise (16x16x16 has half the rate)
   static constexpr int MF = ORD == 4 && BN % 32 == 0 ? 32 : 16, G = MF == 32 ? 4 : 1;     // G: groups of four rows per lane and tile
@@ -956,6 +956,36 @@ int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   return t != end ? t->form : -1;
 }
 
+// Many rows, sums in the order of the 128 x 128 kernel: of 128 x 128 (convolutions) and 128 / 160 / 192 x 160 tiles those whose rounds of the CUs stream the fewest rows
+// (us go with rounds x (BM + BN): one round of 160 x 160 / 192 x 160 at 1536 / 3840 / 1280 21.1 / 21.3, of 256 x 128 24.3; 1800 rows: two of the first 34.0, one of the second
+// 23.6 and of the third 24.9; convolutions 320 -> 320 at 2 x 104 x 152, two rounds of 128 / 160 / 192 61.5 / 62.7 / 70.7).  A round is what the fullest XCD gets.
+static long rounds_cost(const LoraGemmParams& p, int bm, int bn) {
+  const KhXcdGrid g = kh_xcd_grid((p.M + bm - 1) / bm, (p.N + bn - 1) / bn, bm, bn);
+  return ((long)g.rm * g.rn + 31) / 32 * (bm + bn);
+}
+
+// -1: none divides the columns, or others win.
+// Convolutions, before on 128 x 128 tiles whose waves both move operands and compute, two workgroups to a CU or one (us, weights from HBM): 320 -> 320 at 2 x 72 x 72 47.7 -> 27.6,
+// 2 x 96 x 96 52.6 -> 34.2, 2 x 104 x 152 81.3 -> 60.2, 2 x 128 x 120 80.7 -> 60.6, 640 -> 320 at 2 x 96 x 96 95 -> 60.5, 2 x 88 x 120 108 -> 69.5, 640 -> 640 at 2 x 64 x 76 94 -> 65,
+// 1280 -> 640 at 2 x 56 x 56 166 -> 99, 1280 -> 1280 at 4 x 24 x 24 100 -> 83, 2 x 36 x 36 90 -> 87.  Few tiles with a short sum are faster there (128 -> 320 at 2 x 64 x 64, 192 tiles, 15.0
+// against 16.4; 1280 -> 1280 at 8 x 8 88 against 112).
+// Linear layers without row statistics (which go by 128 columns), before on 256 x 128 or 128 x 128 tiles, T given: 1300 / 3840 / 1280 21.8 -> 19.0, 1536 25.5 -> 21.1, 1800
+// 25.4 -> 23.6, 5120 / 1280 / 1280 22.7 -> 19.8, K 5120 71.7 -> 60.6, 4608 / 1920 / 640 25.8 -> 21.4, 6000 27.5 -> 24.2, 10000 / 640 / 640 14.5 -> 12.9.
+int lora_gemm_rounds_form(const LoraGemmParams& p) {
+  const bool conv = p.conv_cin > 0;
+  if (!lora_gemm_fine_ok(p) || p.gn_part != nullptr || p.st_part != nullptr || p.geglu) return -1;
+  const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  if (conv ? tiles <= 128 || (tiles <= 192 && p.K < 2560) : tiles <= 256) return -1;
+  int best = -1;
+  long least = conv ? 0 : rounds_cost(p, 256, 128);
+  constexpr struct { int form, bm, bn; } all[] = {{16, 128, 128}, {19, 128, 160}, {20, 160, 160}, {21, 192, 160}};
+  for (const auto& t : all) {
+    if (p.N % t.bn != 0 || (p.t_nsplit > 0 && p.t_nsplit % t.bn != 0) || (!conv && t.form == 16)) continue;
+    if (const long c = rounds_cost(p, t.bm, t.bn); least == 0 || c < least) { least = c; best = t.form; }
+  }
+  return best;
+}
+
 int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream) {
   const bool conv = p.conv_cin > 0;
   // (a forced form comes here without the rule above)
@@ -972,6 +1002,10 @@ int lora_gemm_fine_launch(const LoraGemmParams& p, int form, hipStream_t stream)
     case 8: return launch_fine<FCfg<128, 320, 0, true>, false>(p, stream);
     case 17: return launch_fine<FCfg<160, 320, 0, true>, false>(p, stream);
     case 18: return launch_fine<FCfg<192, 320, 0, true>, false>(p, stream);
+    case 16: return conv ? launch_fine<FCfg<128, 128, 0>, true>(p, stream) : launch_fine<FCfg<128, 128, 0>, false>(p, stream);
+    case 19: return conv ? launch_fine<FCfg<128, 160, 0>, true>(p, stream) : launch_fine<FCfg<128, 160, 0>, false>(p, stream);
+    case 20: return conv ? launch_fine<FCfg<160, 160, 0>, true>(p, stream) : launch_fine<FCfg<160, 160, 0>, false>(p, stream);
+    case 21: return conv ? launch_fine<FCfg<192, 160, 0>, true>(p, stream) : launch_fine<FCfg<192, 160, 0>, false>(p, stream);
     case 9: return conv ? launch_fine<FCfg<128, 160, 2>, true>(p, stream) : launch_fine<FCfg<128, 160, 2>, false>(p, stream);
     case 10: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 32, 0>, false>(p, stream);
     case 11: return conv ? KH_ERR_UNSUPPORTED : launch_fine<FCfg<32, 64, 0>, false>(p, stream);

@@ -1337,6 +1337,7 @@ int lora_gemm_pipe_launch_conv(const LoraGemmParams& p, hipStream_t stream) {
     if ((tiles > 256 && tiles <= 384 && m128 * n160 <= 256) || (m128 * n160) % 256 == 0) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 2), stream);
     if (tiles <= 192 && m64 * n160 <= 256 && m64 * n160 > tiles && p.K >= 2560) return lora_gemm_fine_launch(p, lora_gemm_fine_form(p, 4), stream);
   }
+  if (const int form = lora_gemm_rounds_form(p); form >= 0) return lora_gemm_fine_launch(p, form, stream);
   if (tiles <= 256 && p.conv_cin % 64 == 0) return launch_pcfg<PCfg<128, 128, 2, 4, 0, 4, 64>, true>(p, stream);
   return launch_pcfg<PCfg<128, 128, 2, 2, 0, 4>, true>(p, stream);
 }
@@ -1388,7 +1389,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
     case 40: return lora_gemm_ksplit_launch(p, 2, stream);
     case 41: return lora_gemm_ksplit_launch(p, 4, stream);
     case 42: return lora_gemm_wide_launch(p, stream);
-    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: case 59: case 60: case 61: case 62: case 63: case 64: case 65: case 67: case 68: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
+    case 50: case 51: case 52: case 53: case 54: case 55: case 57: case 58: case 59: case 60: case 61: case 62: case 63: case 64: case 65: case 66: case 67: case 68: case 69: case 70: case 71: return lora_gemm_fine_launch(p, tile_sel - 50, stream);
     default: break;
   }
   // Default choice.  The limiter is the vector L1 path (every operand byte enters LDS through it), so
@@ -1398,6 +1399,7 @@ int lora_gemm_pipe_launch(const LoraGemmParams& p, int tile_sel, hipStream_t str
   // two workgroups per CU otherwise.
   if (wide_fills(p)) return lora_gemm_wide_launch(p, stream);
   if (const int form = lora_gemm_pipe_fine_form(p); form >= 0) return lora_gemm_fine_launch(p, form, stream);
+  if (const int form = plain_ok(p) ? lora_gemm_rounds_form(p) : -1; form >= 0) return lora_gemm_fine_launch(p, form, stream);
   if (plain_ok(p)) {
     const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
     // (between one and two rounds of 128x128 tiles one of 256x128, us with T given, R 128: M 1536 / N 3840 / K 1280 30.4 -> 25.1, 1800 33.3 -> 24.7,

@@ -902,3 +902,50 @@ def test_geglu_on_the_tiles_whose_rounds_take_least(M, N, K, ln):
     ref = (h[:, :, 0] * torch.nn.functional.gelu(h[:, :, 1])).reshape(M, N // 2)
     # bf16 roundings of the folded weights, of value and gate and of the product: 2^-9 each
     assert ((y.double() - ref).norm() / ref.norm()).item() < 8e-3
+
+
+@pytest.mark.parametrize("M,N,K,R,split", [(1, 640, 64, 0, False), (159, 320, 128, 64, False), (193, 960, 320, 32, True), (321, 160, 640, 128, False), (1300, 3840, 1280, 128, True),
+                                           (4608, 1920, 640, 0, False)])
+def test_tiles_of_160_columns_and_many_rows(M, N, K, R, split):
+    """128 / 160 / 192 x 160 tiles in the order of the 128 x 128 kernel (codes 69 to 71) and 128 x 128 with operand waves (66): its bits, ragged rows, rank columns, one to
+    many stages; and those of the tile that is chosen."""
+    from katz_amd import ops
+
+    say("160 columns, many rows", M, N, K, R, split)
+    d, g, P = dev(), torch.Generator().manual_seed(M + N + K), 3 if split else 1
+    rnd = lambda *s: torch.randn(*s, generator=g).to(d, torch.bfloat16)
+    x, w, b, res = rnd(M, K), rnd(N, K) * K ** -0.5, rnd(N), rnd(M, N)
+    t, bc = (rnd(M, P * R), rnd(N, R) * 0.05) if R else (None, None)
+    run = ((lambda c: ops.lora_linear_pre(x, w, b, t, bc, residual=res, tile=c, n_split=N // 3 if split and N // 3 % 128 == 0 else 0)) if R
+           else (lambda c: ops.lora_linear(x, w, b, residual=res, tile=c)))
+    if split and N // 3 % 128:
+        t = t[:, :R].contiguous()
+    want = run(16)
+    for code in (69, 70, 71) + ((66,) if N % 128 == 0 else ()):
+        assert torch.equal(run(code), want), code
+    if M > 1024:
+        assert torch.equal(run(0), want)
+
+
+@pytest.mark.parametrize("Nb,H,W,Cin,Cout,stride,res", [(2, 72, 72, 64, 320, 1, False), (2, 96, 97, 64, 320, 1, True), (1, 104, 152, 128, 640, 1, True), (2, 77, 64, 64, 640, 1, False),
+                                                        (3, 110, 96, 64, 960, 2, False), (5, 24, 24, 320, 1280, 1, True)])
+def test_convolutions_of_many_pixels_on_tiles_by_their_rounds(Nb, H, W, Cin, Cout, stride, res):
+    """Pixel counts whose 128 x 128 tiles are neither few nor whole rounds: ragged last rows, stride 2, a residual; against float64, first image
+    and last rows, and the same bits twice."""
+    from katz_amd import ops
+
+    say("convolution, many pixels", Nb, H, W, Cin, Cout, stride, res)
+    d, g = dev(), torch.Generator().manual_seed(H + W + Cin)
+    x = torch.randn(Nb, Cin, H, W, generator=g).to(d, torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    w = (torch.randn(Cout, Cin, 3, 3, generator=g) * (9 * Cin) ** -0.5).to(d, torch.bfloat16)
+    b = torch.randn(Cout, generator=g).to(d, torch.bfloat16)
+    ref = torch.nn.functional.conv2d(x.double().cpu()[:1], w.double().cpu(), b.double().cpu(), stride=stride, padding=1)
+    r = torch.randn(Nb, *ref.shape[1:], generator=g).to(d, torch.bfloat16).contiguous(memory_format=torch.channels_last) if res else None
+    y = ops.conv3x3(x, ops.pack_conv3x3_weight(w), b, stride=stride, residual=r)
+    # one rounding of the sum to bf16, one more of the sum with the residual: 2^-9 each
+    want = ref if r is None else ref + r[:1].double().cpu()
+    assert ((y[:1].double().cpu() - want).norm() / want.norm()).item() < 5e-3
+    last = torch.nn.functional.conv2d(x[-1:, :, -8:].double().cpu(), w.double().cpu(), b.double().cpu(), stride=stride, padding=1)[:, :, -2:]
+    want = last if r is None else last + r[-1:, :, -2:].double().cpu()
+    assert ((y[-1:, :, -2:].double().cpu() - want).norm() / want.norm()).item() < 5e-3
+    assert torch.equal(ops.conv3x3(x, ops.pack_conv3x3_weight(w), b, stride=stride, residual=r), y)
