@@ -949,3 +949,48 @@ def test_convolutions_of_many_pixels_on_tiles_by_their_rounds(Nb, H, W, Cin, Cou
     want = last if r is None else last + r[-1:, :, -2:].double().cpu()
     assert ((y[-1:, :, -2:].double().cpu() - want).norm() / want.norm()).item() < 5e-3
     assert torch.equal(ops.conv3x3(x, ops.pack_conv3x3_weight(w), b, stride=stride, residual=r), y)
+
+
+@pytest.mark.parametrize("lens,longest,K,N,RP", [
+    ([1, 0, 65, 200, 64, 70], 200, 576, 1280, 128),                           # ranges of one column tile, nine stages
+    ([650] * 4 + [0, 30], 650, 512, 640, 64),                                 # a full ring of stages
+    ([1] * 64, 1, 320, 1280, 128),                                            # as many segments as lanes, one row each
+    ([3] * 65, 3, 384, 1280, 128),                                            # one more: dealt by the host
+    ([700] * 12 + [1024], 1024, 128, 1664, 128),                              # 148 blocks: thirteen column tiles each, beyond the first five
+    ([1500] * 16, 4096, 640, 256, 64),                                        # 128-row blocks: less than a round
+    ([2100] * 16, 2100, 640, 640, 128),                                       # ... a round and sixteen blocks in ranges
+], ids=str)
+def test_sgmv_fused_dealt_by_the_segments(lens, longest, K, N, RP):
+    """Every row of every segment and every column range exactly once, whatever the lengths: against the products in float64 with t and
+    the delta rounded to bf16 as the kernel rounds them.  Tolerance: a result that falls on the other side of a rounding of t (2^-9 of
+    it, over sqrt(rank) terms) or of the delta and the sum (2^-8 each): 2^-7 of the largest."""
+    from katz_amd import ops
+
+    say("sgmv fused dealt", lens, longest, K, N, RP)
+    d = dev()
+    torch.manual_seed(K + N)
+    start = [0]
+    for n in lens:
+        start.append(start[-1] + n)
+    ranks = [32, 64, 96, 128] if RP == 128 else [32, 64]
+    a, b = torch.randn(len(ranks), RP, K, device=d) * K ** -0.5, torch.randn(len(ranks), N, RP, device=d) * RP ** -0.5
+    for i, r in enumerate(ranks):
+        a[i, r:], b[i, :, r:] = 0, 0
+    a, b = a.to(BF), b.to(BF)
+    x, base = torch.randn(start[-1], K, device=d).to(BF), torch.randn(start[-1], N, device=d).to(BF)
+    who = [i % len(ranks) if i % 7 != 3 else -1 for i in range(len(lens))]     # (every seventh segment has no adapter)
+    who = [w if n > 0 else 10 ** 6 for w, n in zip(who, lens)]                 # (an empty one may name any)
+    scale = [0.5 + 0.25 * i for i in range(len(ranks))]
+    i32 = dict(dtype=torch.int32, device=d)
+    y = base.clone()
+    ops.sgmv_fused_(y, x, a, b, torch.tensor(start, **i32), torch.tensor(who, **i32), torch.tensor(ranks, **i32), torch.tensor(scale, device=d), longest)
+    for i, w in enumerate(who):
+        s, e = start[i], start[i + 1]
+        if s == e or w < 0:
+            assert torch.equal(y[s:e], base[s:e])
+            continue
+        t = (x[s:e].double() @ a[w].double().T).to(BF).double()
+        delta = (scale[w] * (t @ b[w].double().T)).to(BF).double()
+        ref = (base[s:e].double() + delta).to(BF).double()
+        err = (y[s:e].double() - ref).abs().max()
+        assert err <= 2 ** -7 * ref.abs().max(), (i, w, float(err))
