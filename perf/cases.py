@@ -497,14 +497,3 @@ def tolerance(case):
     if kind in ("step", "eager", "switch", "loop"):
         return dict(rel=2e-2)       # some 700 layers, each rounding its result to bf16
     return dict(rel=1e-2)
-
-
-def listed():
-    import random
-    out = [dict(name="requests_mixed", kind="requests", layer=1, tokens="1024,988,1024,256,1024,576,988,1024", ranks="64,8,128,32,16,64,128,32")]
-    rng = random.Random(3)
-    while len(out) < 8:
-        c = draw(rng)
-        if c["kind"] == "requests":
-            out.append(dict(name=f"req{len(out)}", **c))
-    return out
