@@ -994,3 +994,29 @@ def test_sgmv_fused_dealt_by_the_segments(lens, longest, K, N, RP):
         ref = (base[s:e].double() + delta).to(BF).double()
         err = (y[s:e].double() - ref).abs().max()
         assert err <= 2 ** -7 * ref.abs().max(), (i, w, float(err))
+
+
+@pytest.mark.parametrize("shapes,r,dt", [
+    ([(128, 128)], 128, torch.float16),                                        # two turns of 64 ranks
+    ([(130, 260), (1, 8), (257, 1284)], 96, torch.bfloat16),                   # a turn and a half, pieces of 8 bytes, ragged tiles
+    ([(64, 7), (129, 131)], 20, torch.float16),                                # element by element, rank in no whole piece
+    ([(8, 16)] * 70 + [(200, 136)] + [(16, 8)] * 70, 8, torch.bfloat16),       # more layers than lanes
+], ids=lambda v: str(v)[:40])
+def test_merge_tiles(shapes, r, dt):
+    """kh_lora_merge_grouped_bf16 at the edges of tiles, of turns over the rank and of the search for a tile's layer, against float64: one
+    rounding to bf16 (2^-9 relative) and r products in fp32 (2^-24 r of the sum of their sizes)."""
+    from katz_amd import ops
+
+    say("merge tiles", shapes[:3], r, dt)
+    d = dev()
+    torch.manual_seed(r)
+    w = [torch.randn(n, k, device=d).to(BF) for n, k in shapes]
+    up = [torch.randn(n, r, device=d).to(dt) for n, _ in shapes]
+    down = [torch.randn(r, k, device=d).to(dt) for _, k in shapes]
+    scales = [0.5 + i / len(shapes) for i in range(len(shapes))]
+    was = [x.clone() for x in w]
+    ops.lora_merge_grouped(w, up, down, scale=0.3, layer_scales=scales)
+    for x, x0, u, v, s in zip(w, was, up, down, scales):
+        ref = x0.double() + 0.3 * s * (u.double() @ v.double())
+        size = x0.double().abs() + 0.3 * s * (u.double().abs() @ v.double().abs())
+        assert ((x.double() - ref).abs() <= ref.abs() * 2 ** -8 + size * (r + 4) * 2 ** -23).all(), tuple(x.shape)
