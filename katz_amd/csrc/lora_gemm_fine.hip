@@ -168,7 +168,10 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
         const int xcd = (int)blockIdx.x & 7, wgs = (gx * ct - xcd + 7) / 8, KT1 = p.K / BK;
         char* lds = smem + C::TOUCH_OFF + (wave - 4) * 256;
         auto touch = [&](int t) {
-          kh_touch_rows<8>(p.w, p.N, p.K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, 8, lds, ((int)blockIdx.x >> 3) * 256 + tid - 256, wgs * 256);
+          const int rows = p.xr_n * BN, row0 = (xcd % p.xg_n) * rows, i = ((int)blockIdx.x >> 3) * 256 + tid - 256;
+          // (the last, shorter block by its true width: 3952 / 640 / 640 20.1 us instead of 19.7 with the constant)
+          if (t + 8 <= KT1) kh_touch_rows<8>(p.w, p.N, p.K, row0, rows, t, 8, lds, i, wgs * 256);
+          else kh_touch_rows(p.w, p.N, p.K, row0, rows, t, 8, lds, i, wgs * 256);
         };
         __builtin_amdgcn_s_sleep(127);                       // 8128 clocks, about 10 stages of the K loop
         const bool hints = il_prefetch_by_idle_waves(p);
@@ -244,6 +247,45 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
 
   // of a stage row, the piece that a 16-byte piece is stored as: 16 rows at one piece fill the 64 banks
   auto swz = [](int row) { return (PPR == 8 ? row >> 1 : row) & (PPR - 1); };
+  // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
+  // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row).  (With eight computing waves only in the waves that move
+  // operands: the 128 x 320 tiles kept these offsets over the computing waves' loop, in scratch memory.  With four ahead of the branch: behind it
+  // 988 / 1280 / 1280 took 13.0 us instead of 12.8.)
+  constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
+  uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
+  int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
+  constexpr bool AHEAD = C::CW == 4 && !(BM == 128 && BN == 128);
+  auto offsets = [&] {
+#pragma unroll
+    for (int q = 0; q < LPS_HI; ++q) {
+      int u = pw + 4 * q;
+      u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
+      const int r = u * UR + lane / PPR;
+      const uint32_t pcb = (uint32_t)(((lane % PPR) ^ swz(r)) * 16);
+      if (CONV && q < XQ) {
+        int row = m0 + r; row = row < M ? row : M - 1;
+        const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
+        const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
+        int mask = 0;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+          const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
+          mask |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
+        }
+        tapmask[q < XQ ? q : 0] = mask;
+        // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
+        voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
+      } else if (q < XQ) {
+        voff[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + pcb;        // rows past M lie beyond the buffer: zeros
+      } else {
+        voff[q] = (uint32_t)(n0 + r - BM) * (uint32_t)K * 2u + pcb;
+      }
+      if (EXT && p.t_ext != nullptr)
+        voff2[q] = q < XQ ? ((uint32_t)(m0 + r) * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb
+                          : (uint32_t)(n0 + r - BM) * (uint32_t)p.R * 2u + pcb;
+    }
+  };
+  if constexpr (AHEAD) offsets();
   // fragments: row lr of each block of MF rows; of a k-step the lane's 16-byte piece lg (16x16x16: its 8 bytes lg)
   constexpr bool HALF = C::ORD == 4 && C::MF == 16;
   using Frag = typename std::conditional<HALF, s16x4, bf16x8>::type;
@@ -300,40 +342,7 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
   typedef XAttnFine<cmax(BN / 64, 1), 256, C::LDC> XAttn;
   XAttn kv;                                            // XA: the keys and values, in the producers
   if (producer) {
-    // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
-    // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row).  (Here and
-    // not in front of the branch: the 128 x 320 tiles then kept these offsets over the computing waves' loop, in scratch memory.)
-    constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
-    uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
-    int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
-#pragma unroll
-    for (int q = 0; q < LPS_HI; ++q) {
-      int u = pw + 4 * q;
-      u = u < C::UNITS ? u : C::UNITS - 1;               // never issued (has_hi), keep the offset valid
-      const int r = u * UR + lane / PPR;
-      const uint32_t pcb = (uint32_t)(((lane % PPR) ^ swz(r)) * 16);
-      if (CONV && q < XQ) {
-        int row = m0 + r; row = row < M ? row : M - 1;
-        const int wo = row % p.conv_wo, t2 = row / p.conv_wo, ho = t2 % p.conv_ho, nb = t2 / p.conv_ho;
-        const int hi0 = ho * p.conv_stride - 1, wi0 = wo * p.conv_stride - 1;
-        int mask = 0;
-#pragma unroll
-        for (int tap = 0; tap < 9; ++tap) {
-          const int hi = hi0 + tap / 3, wi = wi0 + tap % 3;
-          mask |= (hi >= 0 && hi < p.conv_h && wi >= 0 && wi < p.conv_w) ? (1 << tap) : 0;
-        }
-        tapmask[q < XQ ? q : 0] = mask;
-        // relative to one row and one pixel in front of the image (the buffer's base), so that it is never negative
-        voff[q] = (uint32_t)(((nb * p.conv_h + hi0 + 1) * p.conv_w + wi0 + 1) * p.conv_cin) * 2u + pcb;
-      } else if (q < XQ) {
-        voff[q] = (uint32_t)(m0 + r) * (uint32_t)K * 2u + pcb;        // rows past M lie beyond the buffer: zeros
-      } else {
-        voff[q] = (uint32_t)(n0 + r - BM) * (uint32_t)K * 2u + pcb;
-      }
-      if (EXT && p.t_ext != nullptr)
-        voff2[q] = q < XQ ? ((uint32_t)(m0 + r) * (uint32_t)p.ldt + (uint32_t)(p.t_nsplit > 0 ? (n0 / p.t_nsplit) * p.R : 0)) * 2u + pcb
-                          : (uint32_t)(n0 + r - BM) * (uint32_t)p.R * 2u + pcb;
-    }
+    if constexpr (!AHEAD) offsets();
     const size_t x_bytes = CONV ? (size_t)(M / (p.conv_ho * p.conv_wo)) * p.conv_h * p.conv_w * p.conv_cin * 2 : (size_t)M * K * 2;
     const size_t x_lead = CONV ? (size_t)(p.conv_w + 1) * p.conv_cin * 2 : 0;
     const rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(p.x) - x_lead), 0,
@@ -451,9 +460,10 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
   } else {
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
+    // (lines by a constant division only where eight waves share them: with four 154 / 1280 / 2048 took 10.9 us instead of 10.7)
     auto touch = [&](int t, auto n) {
       if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
-        kh_touch_rows<decltype(n)::value>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * C::CT + tid, p.xr_m * p.xr_n * C::CT);
+        kh_touch_rows<C::CW == 8 ? decltype(n)::value : 0>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * C::CT + tid, p.xr_m * p.xr_n * C::CT);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
