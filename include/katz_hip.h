@@ -145,8 +145,8 @@ int kh_lora_linear_norm_bf16(const void* x, const void* w, const void* bias, con
  * q = kh_lora_linear_norm_bf16(x, ...) never written to memory.  The reference runs to_q, then the attention processor
  * on its result (diffusers-hf/src/diffusers/models/attention_processor.py:1231-1296: attn.to_q :1256, head split
  * :1269-1272, F.scaled_dot_product_attention :1276); on the SDXL text context (S = 77 keys) the attention alone is a
- * launch of a few microseconds whose 128 queries x 2 heads are exactly one 128 x 128 output tile of the projection, so
- * the GEMM's epilogue keeps the tile in LDS, loads the S keys / values of its two heads and runs the attention there.
+ * launch of a few microseconds whose queries by whole heads are an output tile of the projection (128 x 128; 32 or 64 rows, one or
+ * two heads below 1024 rows), so the GEMM's epilogue keeps the tile in LDS, loads the S keys / values of its heads and runs the attention there.
  * x [M,K] with M = B * T (rows of sample b: b*T .. b*T + T - 1), w [N,K], N = heads * 64; k, v: [B,S,N] views (row
  * strides ldk / ldv, sample strides bsk / bsv, in elements); o [M,N] with row stride ldo, head h at columns 64 h.
  * The projection's arguments (bias, adapters, t_scratch, counters, folded LayerNorm, flags bits 8..24) are

@@ -9,9 +9,10 @@
 // lines that come from memory and 110 GB/s of lines its L2 has, all CUs together 17 TB/s out of the L2s; a 128 x 128 tiling of M = 1000 /
 // N = 1280 streams 32 KB a stage into each of 80 CUs and takes 16 us, whether M is 150 or 2000.  Hence
 //   * small tiles: 64 x 80 gives 256 workgroups there, 18 KB a stage;
-//   * four waves that only move operands beside four that only compute: a wave that does both stands in the queue of the address
-//     unit (16 clocks per 1 KB instruction) while its MFMAs wait (64 x 160 tiles: 1330 clocks a stage together, 860 apart);
-//   * a ring of as many stages as LDS holds (up to 8), and
+//   * four waves that only move operands beside four or eight that only compute: a wave that does both stands in the queue of the address
+//     unit (16 clocks per 1 KB instruction) while its MFMAs wait (64 x 160 tiles: 1330 clocks a stage together, 860 apart).  Eight (GEGLU and
+//     order 2) are two to a SIMD, so that one's LDS reads run under the other's MFMAs;
+//   * a ring of as many stages as LDS holds (up to 16), and
 //   * the XCD's block of W fetched into its L2 by all its workgroups before the K loop meets it.
 //
 // Orders (ORD): the 128 x 128 / 256 x 320 kernels add along K one 16-column step after the other (0), the 160-column kernels in four
@@ -248,13 +249,15 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
   // of a stage row, the piece that a 16-byte piece is stored as: 16 rows at one piece fill the 64 banks
   auto swz = [](int row) { return (PPR == 8 ? row >> 1 : row) & (PPR - 1); };
   // DMA of this lane: unit u = pw + 4*q covers stage rows u*UR .. u*UR+UR-1 (x rows, W rows); LDS slot = lane: row
-  // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row).  (With eight computing waves only in the waves that move
-  // operands: the 128 x 320 tiles kept these offsets over the computing waves' loop, in scratch memory.  With four ahead of the branch: behind it
-  // 988 / 1280 / 1280 took 13.0 us instead of 12.8.)
+  // lane/PPR, physical piece lane%PPR, which holds logical piece (lane%PPR) ^ swz(row).  Formed by the waves that move operands only (large tiles kept
+  // these offsets over the computing waves' loop, in scratch memory; 1 / 1280 / 1280 8.7 -> 8.45 us, 154 / 640 / 2048 9.6 -> 9.45), or by all ahead of the
+  // branch where that is faster (988 / 1280 / 1280 12.7 us instead of 13.05).
   constexpr uint32_t OOB = 0x80000000u;                // every buffer here is shorter than 2 GiB
   uint32_t voff[LPS_HI], voff2[EXT ? LPS_HI : 1];
   int tapmask[CONV ? XQ : 1];                          // CONV: bit t = tap t of this lane's row is inside the image
-  constexpr bool AHEAD = C::CW == 4 && !(BM == 128 && BN == 128);
+  constexpr bool AHEAD = C::CW == 4 && BM * BN < 128 * 128 && !(BM == 32 && BN == 32);
+  // (behind the branch the kernel's arguments would be a load of their own: here they come with the others)
+  if constexpr (C::CW == 4 && !AHEAD && BM * BN <= 128 * 128) asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.t_ext), "s"(p.b_cat), "s"(p.ldt), "s"(p.t_nsplit));
   auto offsets = [&] {
 #pragma unroll
     for (int q = 0; q < LPS_HI; ++q) {
@@ -460,10 +463,10 @@ __global__ __launch_bounds__(C::NT, TMODE == T_COOP ? 1 : C::CW == 8 ? 3 : 2) vo
   } else {
     // W's lines into the XCD's L2 ahead of the ring (kh_touch_rows): 24 stages now, then 8 every 8 stages (M 988, N 1280, K 1280: 10.4 ->
     // 9.9 us; K 5120 38.4 -> 30.5; x, which the launch in front has just written, is not worth it)
-    // (lines by a constant division only where eight waves share them: with four 154 / 1280 / 2048 took 10.9 us instead of 10.7)
+    // (lines by a constant division only for large tiles: 154 / 1280 / 2048 took 10.9 us with it instead of 10.7, 3952 / 640 / 640 20.1 instead of 19.9)
     auto touch = [&](int t, auto n) {
       if (!GRP && !(TMODE == T_IL && BM == 128 && BN == 128) && t < KT1)
-        kh_touch_rows<C::CW == 8 ? decltype(n)::value : 0>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * C::CT + tid, p.xr_m * p.xr_n * C::CT);
+        kh_touch_rows<(BM * BN > 128 * 128) ? decltype(n)::value : 0>(p.w, N, K, (xcd % p.xg_n) * p.xr_n * BN, p.xr_n * BN, t, n, smem + C::TOUCH_OFF + pw * 256, local * C::CT + tid, p.xr_m * p.xr_n * C::CT);
     };
     // (a GEGLU projection has so many columns that its first tile queued behind 24 stages: 988 / 10240 / 1280 from HBM 36.4 -> 34.7 us).
     // The next launch's weights come behind this launch's own first lines, from waves that wait for them anyway.
@@ -853,13 +856,12 @@ bool lora_gemm_fine_ok(const LoraGemmParams& p) {
 
 // Forms: order 0 on 64 x 80 (0), 128 x 80 (1), 32 x 128 (2), 64 x 128 (3); order 4 on 32 x 160 (4), 64 x 160 (5), 64 x 80 (6);
 // GEGLU on 64 x 320 (7), 128 x 320 (8), 160 x 320 (17), 192 x 320 (18); order 2 on 128 x 160 (9); order 0 on 32 x 32 (10), 32 x 64 (11), 64 x 64 (12);
-// order 4 on 32 x 32 (13), 32 x 64 (14), 64 x 64 (15).
+// order 4 on 32 x 32 (13), 32 x 64 (14), 64 x 64 (15); order 0 on 128 x 128 (16), 128 x 160 (19), 160 x 160 (20), 192 x 160 (21).
 //
-// Order 2: wave tiles of 64 x 160 over two k-slices and waves of their own for the operands, in place of eight 32 x 160 strips that did
-// both: 7 x 32 W and x rows read from LDS per 20 matrix instructions against 6 per 5.  us per launch, weights from HBM: convolutions 640 -> 640
-// at 2 x 64 x 64 70.9 -> 63.0, 1920 -> 640 190 -> 167, 320 -> 320 at 2 x 128 x 128 81 -> 70, 960 -> 320 198 -> 173, 640 -> 640 263 -> 235 (two
-// rounds), 1280 -> 1280 at 2 x 64 x 64 252 -> 250; linear layers 3952 / 640 / 640 14.1 -> 12.5, 8192 / 640 / 640 14.7 -> 14.0,
-// 4096 / 1280 / 5120 62.6 -> 56.5.
+// Order 2: eight waves of 64 x 80, two k-slices of four, and waves of their own for the operands, in place of eight 32 x 160 strips that did
+// both.  us per launch, weights from HBM (strips, then four waves of 64 x 160): convolutions 640 -> 640 at 2 x 64 x 64 70.9 -> 63.0, 1920 -> 640 190 -> 167, 960 -> 320 at
+// 2 x 128 x 128 198 -> 173; (four, then eight) 640 -> 640 at 2 x 64 x 64 62.0 -> 59.2, 320 -> 320 at 2 x 128 x 128 69.9 -> 66.1, 1280 -> 1280 at 2 x 64 x 64 239 -> 214, 1920 -> 640 159 both;
+// linear layers with adapters 8192 / 640 / 640 20.1 -> 18.6, 8192 / 640 / 2560 44.3 -> 42.0.
 //
 // Few rows: the shrink of a call with adapters runs inside the launch, on CUs that its tiles leave idle (T_IL).  The shrink's sums are those of
 // its own launch and the tiles' those of the order, so one launch and two give the same bits.
@@ -977,15 +979,16 @@ static long rounds_cost(const LoraGemmParams& p, int bm, int bn) {
 // -1: none divides the columns, or others win.
 // Convolutions, before on 128 x 128 tiles whose waves both move operands and compute, two workgroups to a CU or one (us, weights from HBM): 320 -> 320 at 2 x 72 x 72 47.7 -> 27.6,
 // 2 x 96 x 96 52.6 -> 34.2, 2 x 104 x 152 81.3 -> 60.2, 2 x 128 x 120 80.7 -> 60.6, 640 -> 320 at 2 x 96 x 96 95 -> 60.5, 2 x 88 x 120 108 -> 69.5, 640 -> 640 at 2 x 64 x 76 94 -> 65,
-// 1280 -> 640 at 2 x 56 x 56 166 -> 99, 1280 -> 1280 at 4 x 24 x 24 100 -> 83, 2 x 36 x 36 90 -> 87.  Few tiles with a short sum are faster there (128 -> 320 at 2 x 64 x 64, 192 tiles, 15.0
-// against 16.4; 1280 -> 1280 at 8 x 8 88 against 112).
+// 1280 -> 640 at 2 x 56 x 56 166 -> 99, 1280 -> 1280 at 4 x 24 x 24 100 -> 83, 2 x 36 x 36 90 -> 87.  One round of 128 x 128 is as fast there or faster
+// unless its columns are many (320 -> 320 at 1 x 104 x 88 29.1 against 31.1, 640 -> 640 at 2 x 44 x 44 41.9 against 42.2; 640 -> 1280 at 2 x 36 x 32 53.7 against 46.8), and so are few tiles
+// with a short sum (128 -> 320 at 2 x 64 x 64, 192 tiles, 15.0 against 16.4; 1280 -> 1280 at 8 x 8 88 against 112).
 // Linear layers without row statistics (which go by 128 columns), before on 256 x 128 or 128 x 128 tiles, T given: 1300 / 3840 / 1280 21.8 -> 19.0, 1536 25.5 -> 21.1, 1800
 // 25.4 -> 23.6, 5120 / 1280 / 1280 22.7 -> 19.8, K 5120 71.7 -> 60.6, 4608 / 1920 / 640 25.8 -> 21.4, 6000 27.5 -> 24.2, 10000 / 640 / 640 14.5 -> 12.9.
 int lora_gemm_rounds_form(const LoraGemmParams& p) {
   const bool conv = p.conv_cin > 0;
   if (!lora_gemm_fine_ok(p) || p.gn_part != nullptr || p.st_part != nullptr || p.geglu) return -1;
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-  if (conv ? tiles <= 128 || (tiles <= 192 && p.K < 2560) : tiles <= 256) return -1;
+  if (conv ? tiles <= 128 || (rounds_cost(p, 128, 128) == 256 && (p.K < 2560 || p.N < 1024)) : tiles <= 256) return -1;
   int best = -1;
   long least = conv ? 0 : rounds_cost(p, 256, 128);
   constexpr struct { int form, bm, bn; } all[] = {{16, 128, 128}, {19, 128, 160}, {20, 160, 160}, {21, 192, 160}};
