@@ -18,12 +18,12 @@
 // read while the stage before is multiplied, the y pieces of the first five tiles (128 rows: of the first) requested while phase 1 runs, the
 // results written through the L2 (behind plain stores the launch ended with all of y still to be written: 1 us of 20), and 64-row blocks while
 // they fit one round of the 256 CUs, so that fewer of them repeat phase 1 for other columns.
-// 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 20.2 -> 18.7 us, all of rank 32 19.7 -> 15.2; 2 x 1024 rows 13.5 -> 12.8.
+// 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 20.2 -> 17.6 us, all of rank 32 19.7 -> 15.2; 2 x 1024 rows 13.5 -> 12.9.
 // Rows / columns of A_a / B_a beyond the adapter's rank are zero by contract, so the padded rank only saves work.
 // Batches with few row blocks deal the column tiles of y to several workgroups, each of which repeats phase 1 for its rows: x is then read from
 // L2 more than once, which such small batches do not notice.  How many is decided by the segments' true lengths, which only the device knows
 // (up to 64 segments): with the host's bound -- every segment as long as the longest -- five segments of 650 rows were 275 workgroups, a
-// second round for 19 of them (27.2 -> 11.4 us), and 16 of 1280 .. 2852 rows at 640 a second round of nine (40.1 -> 32.7).
+// second round for 19 of them (27.2 -> 11.5 us), and 16 of 1280 .. 2852 rows at 640 a second round of nine (40.1 -> 33.0).
 // Grouped form (kh_sgmv_fused_grouped_bf16): several layers that read the same x with the same segments (the to_k / to_v
 // projections of every cross-attention read the one text context) in one launch,
 // per-layer A / B / y from a device table: 77-row requests give a single layer's launch a few microseconds of traffic,
@@ -89,34 +89,49 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
     const int rows = a >= 0 && end > st ? end - st : 0;
     int rk = 0;
     float sc = 0.f;
-    if (rows > 0) { rk = p.adapter_rank[a]; sc = p.adapter_scale[a]; }   // (under way beside the sum)
+    if (rows > 0) { rk = p.adapter_rank[a]; sc = p.adapter_scale[a]; }
     int blocks = (rows + BM - 1) / BM;
     blocks = blocks < p.row_blocks ? blocks : p.row_blocks;
-    int sum = blocks;
+    // (blocks of adapters of more than 64 in the upper half of the word, where 64 segments' blocks fit half a word)
+    const bool halves = p.row_blocks < 1024;
+    int sum = blocks | (halves && rk > 64 ? blocks << 16 : 0);
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o, 64); if (lane >= o) sum += v; }
-    const int per_layer = __builtin_amdgcn_readlane(sum, 63), nb = per_layer * p.n_layers;
+    const int total = __builtin_amdgcn_readlane(sum, 63), heavy = halves ? (int)((unsigned)total >> 16) : 0, per_layer = halves ? total & 0xffff : total;
+    const int nb = per_layer * p.n_layers;
+    int upto = halves ? sum & 0xffff : sum;       // blocks up to this lane's segment
     wait_cnt<0, 0>();                             // (or the compiler waits for them, and all behind them, among phase 1's loads)
     const int u = (int)blockIdx.x, full = nb / CUS * CUS;
-    int b = u;
+    int b = u, last = nb;
     j0 = 0; n_tiles = all_tiles;
     if (u >= full) {
       const int left = nb - full, left8 = (left + 7) & ~7;
       if (left == 0) return;
       int z = CUS / left8;
       z = z < all_tiles ? z : all_tiles;
+      int v = u - full;
+      // A range more for the blocks of adapters of more than 64 where that fits beside the others: a stage of theirs is 24 KB, of the others 12 or 16
+      // (8 requests of mixed ranks 18.6 -> 17.6 us, 16 of 357 .. 961 rows 26.0 -> 22.9; waiting for the ranks before the sum costs all calls 0.1)
+      const int h8 = (heavy + 7) & ~7, l8 = (nb - heavy + 7) & ~7;
+      if (full == 0 && p.n_layers == 1 && heavy > 0 && heavy < nb && z < all_tiles && h8 * (z + 1) + l8 * z <= CUS) {
+        const bool mine = v < h8 * (z + 1);
+        upto = mine ? (int)((unsigned)sum >> 16) : upto - (int)((unsigned)sum >> 16);
+        v = mine ? v : v - h8 * (z + 1);
+        last = mine ? heavy : nb - heavy;
+        z = mine ? z + 1 : z;
+      }
       const int per = (all_tiles + z - 1) / z;
       z = (all_tiles + per - 1) / per;
-      const int v = u - full, w = v % (8 * z);
+      const int w = v % (8 * z);
       b = full + v / (8 * z) * 8 + w % 8;
-      if (b >= nb) return;                        // uniform over the workgroup
+      if (b >= last) return;                      // uniform over the workgroup
       j0 = w / 8 * per;
       n_tiles = all_tiles - j0 < per ? all_tiles - j0 : per;
     }
     layer = b / per_layer;
     const int bl = b % per_layer;
-    const int seg = __builtin_ctzll(__ballot(sum > bl));
-    m0 = (bl - (__builtin_amdgcn_readlane(sum, seg) - __builtin_amdgcn_readlane(blocks, seg))) * BM;
+    const int seg = __builtin_ctzll(__ballot(upto > bl));
+    m0 = (bl - (__builtin_amdgcn_readlane(upto, seg) - __builtin_amdgcn_readlane(blocks, seg))) * BM;
     r0 = __builtin_amdgcn_readlane(st, seg);
     M = __builtin_amdgcn_readlane(rows, seg);     // rows of this segment
     ad = __builtin_amdgcn_readlane(a, seg);

@@ -959,6 +959,8 @@ def test_convolutions_of_many_pixels_on_tiles_by_their_rounds(Nb, H, W, Cin, Cou
     ([700] * 12 + [1024], 1024, 128, 1664, 128),                              # 148 blocks: thirteen column tiles each, beyond the first five
     ([1500] * 16, 4096, 640, 256, 64),                                        # 128-row blocks: less than a round
     ([2100] * 16, 2100, 640, 640, 128),                                       # ... a round and sixteen blocks in ranges
+    ([900, 64, 1, 300, 129, 900], 900, 448, 640, 128),                        # adapters of more than 64 in a range more than the others
+    ([100, 30, 500], 200000, 128, 256, 128),                                  # a bound on the rows far above them
 ], ids=str)
 def test_sgmv_fused_dealt_by_the_segments(lens, longest, K, N, RP):
     """Every row of every segment and every column range exactly once, whatever the lengths: against the products in float64 with t and
