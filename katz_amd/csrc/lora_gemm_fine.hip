@@ -986,8 +986,12 @@ static long rounds_cost(const LoraGemmParams& p, int bm, int bn) {
 // 25.4 -> 23.6, 5120 / 1280 / 1280 22.7 -> 19.8, K 5120 71.7 -> 60.6, 4608 / 1920 / 640 25.8 -> 21.4, 6000 27.5 -> 24.2, 10000 / 640 / 640 14.5 -> 12.9.
 int lora_gemm_rounds_form(const LoraGemmParams& p) {
   const bool conv = p.conv_cin > 0;
-  if (!lora_gemm_fine_ok(p) || p.gn_part != nullptr || p.st_part != nullptr || p.geglu) return -1;
+  if (!lora_gemm_fine_ok(p) || p.gn_part != nullptr || p.geglu) return -1;
   const long tiles = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
+  // one round of 128 x 128 with a long sum (us, T given or none, before on tiles whose eight waves do both): 2304 / 1280 / 5120 53.5 -> 42.4, 2432 51.4 -> 41.8, K 2560 29.5 -> 23.2,
+  // 4608 / 640 / 2560, R 128 47.3 -> 41.9 with its shrink, 700 / 3840 / 2560 26.9 -> 25.7; half a round is as fast there (1024 / 2048 / 4096 25.7, 26.3 here), and so are shorter sums
+  if (!conv && tiles > 128 && tiles <= 256 && p.K >= 2560 && p.N % 128 == 0 && p.t_nsplit % 128 == 0 && (p.st_part == nullptr || p.N / 128 <= KH_LN_SLOTS) && rounds_cost(p, 128, 128) == 256) return 16;
+  if (p.st_part != nullptr) return -1;
   if (conv ? tiles <= 128 || (rounds_cost(p, 128, 128) == 256 && (p.K < 2560 || p.N < 1024)) : tiles <= 256) return -1;
   int best = -1;
   long least = conv ? 0 : rounds_cost(p, 256, 128);

@@ -905,7 +905,7 @@ def test_geglu_on_the_tiles_whose_rounds_take_least(M, N, K, ln):
 
 
 @pytest.mark.parametrize("M,N,K,R,split", [(1, 640, 64, 0, False), (159, 320, 128, 64, False), (193, 960, 320, 32, True), (321, 160, 640, 128, False), (1300, 3840, 1280, 128, True),
-                                           (4608, 1920, 640, 0, False)])
+                                           (4608, 1920, 640, 0, False), (2304, 1280, 2560, 64, False), (2430, 1280, 2624, 0, False)])
 def test_tiles_of_160_columns_and_many_rows(M, N, K, R, split):
     """128 / 160 / 192 x 160 tiles in the order of the 128 x 128 kernel (codes 69 to 71) and 128 x 128 with operand waves (66): its bits, ragged rows, rank columns, one to
     many stages; and those of the tile that is chosen."""
