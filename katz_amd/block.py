@@ -235,14 +235,15 @@ class _Ready:
             p = expect(l.__dict__, "_packed")
             if p is None:
                 continue
-            if p.overflow or not split:
-                return False
             v, d = p.__dict__, getattr(self.desc, name)
-            a, b, s = expect(v, "a_cat"), expect(v, "b_cat"), expect(v, "col_scale")
+            if v.get("overflow") or not split:             # (PooledPack makes its list when it is asked)
+                return False
+            for t in ("a_cat", "b_cat", "col_scale"):
+                expect(v, t)
             at = p.addresses(nk) if type(p) is PooledPack else None
             if at is not None:                             # by address: no views are made
                 d.a_cat, d.b_cat, d.col_scale, d.ca1, d.ca2 = at
-                d.R, d.r_used = p.shape[0], p.used
+                d.R, d.r_used = p.R, p.r_used
                 keep.append(p)
                 continue
             a, b, s = p.a_cat, p.b_cat, p.col_scale
@@ -261,7 +262,7 @@ class _Ready:
                 st = weights
                 plan.weights(q, w, None, c1, c2)
                 q.a_cat, q.b_cat, q.col_scale, q.ca1, q.ca2 = at[0]
-                q.R, q.r_used, q.n_split = first.shape[0], max(p.used for p in qkv), plan.inner
+                q.R, q.r_used, q.n_split = first.R, max(p.r_used for p in qkv), plan.inner
                 a, b, _ = side_by_side                     # (hints hold them weakly)
                 if nk is not None:
                     a = first.pool[3].as_strided(a.shape, a.stride(), first.at[3])

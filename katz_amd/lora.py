@@ -80,7 +80,7 @@ class PooledPack(PackedAdapters):
                  norm: Optional[tuple]):
         d = self.__dict__
         d["pool"], d["at"], d["shape"] = pool, at, shape           # buffers (A, B, scales, A * norm, its two terms), offsets in elements, (R, K, N)
-        d["names"], d["ranks"], d["used"], d["norm"] = names, ranks, used, norm
+        d["names"], d["ranks"], d["used"], d["norm"] = names, ranks, used, norm    # used: r_used of these names and ranks
 
     def _view(self, name: str, which: int, size: tuple, stride: tuple):
         d = self.__dict__
@@ -93,22 +93,37 @@ class PooledPack(PackedAdapters):
     @property
     def moved(self) -> bool:
         d = self.__dict__
-        return "a_cat" in d or "b_cat" in d or "col_scale" in d
+        return "a_cat" in d or "b_cat" in d or "col_scale" in d or bool(d.get("overflow"))
 
-    R = property(lambda self: self.shape[0])
-    r_used = property(lambda self: self.used)
-    overflow = property(lambda self: ())
+    R = property(lambda self: self.shape[0] if "a_cat" not in self.__dict__ else self.a_cat.shape[0])
+    r_used = property(lambda self: self.used if "spans" not in self.__dict__ else PackedAdapters.r_used.fget(self))
     a_cat = property(lambda self: self._view("a_cat", 0, (self.shape[0], self.shape[1]), (self.shape[1], 1)), lambda self, v: self._move("a_cat", v))
     b_cat = property(lambda self: self._view("b_cat", 1, (self.shape[2], self.shape[0]), (self.shape[0], 1)), lambda self, v: self._move("b_cat", v))
     col_scale = property(lambda self: self._view("col_scale", 2, (self.shape[0],), (1,)), lambda self, v: self._move("col_scale", v))
 
+    # (lists of this pack, as a PackedAdapters has them: made when somebody asks, kept from then on)
+    @property
+    def overflow(self):
+        return self.__dict__.setdefault("overflow", [])
+
+    @overflow.setter
+    def overflow(self, v):
+        self.__dict__["overflow"] = v
+
     @property
     def spans(self):
-        out, c = [], 0
-        for n, r in zip(self.names, self.ranks):
-            out.append((n, c, r))
-            c += r
-        return out
+        d = self.__dict__
+        if "spans" not in d:
+            out, c = [], 0
+            for n, r in zip(self.names, self.ranks):
+                out.append((n, c, r))
+                c += r
+            d.setdefault("spans", out)
+        return d["spans"]
+
+    @spans.setter
+    def spans(self, v):
+        self.__dict__["spans"] = v
 
     @property
     def ln(self):

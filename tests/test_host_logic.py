@@ -800,3 +800,27 @@ def test_packs_of_a_pool_are_views_made_on_demand():
     packs = make()
     packs[1].ln = ((7,), None, None, None)                        # the terms of a norm that changed meanwhile
     assert packs[1].ln[0] == (7,) and packs[1].addresses(key) is None and packs[1].addresses() is not None and stacked_norm_terms(packs, key) is None
+
+
+def test_fields_of_a_pooled_pack_can_be_assigned():
+    """PooledPack stands wherever a PackedAdapters does: `spans` and `overflow` are lists of its own that can be filled and replaced, and what is derived
+    from them and from the tensors follows."""
+    from katz_amd.lora import PackedAdapters, PooledPack, stacked_packs
+
+    R, K, N, n = 64, 16, 24, 3
+    pool = [torch.randn(n * R * K).bfloat16(), torch.randn(n * R * N).bfloat16(), torch.randn(n * R)]
+    packs = [PooledPack(pool, (i * R * K, i * R * N, i * R, 0, 0), (R, K, N), ["a", "b"], [8, 20], 32, None) for i in range(n)]
+    p = packs[1]
+    assert p.r_used == 32 and p.overflow == [] and p.overflow is p.overflow and p.spans is p.spans and packs[0].overflow is not p.overflow
+    p.spans.append(("c", 28, 12))
+    assert p.r_used == 48
+    p.spans = [("a", 0, 8)]
+    assert p.spans == [("a", 0, 8)] and p.r_used == 16 and p.addresses() is not None and stacked_packs(packs) is not None
+    more = PackedAdapters(p.a_cat, p.b_cat, p.col_scale)
+    for assign in (lambda: p.overflow.append(more), lambda: setattr(p, "overflow", [more])):    # not one launch's any more
+        assign()
+        assert p.overflow == [more] and p.addresses() is None and stacked_packs(packs) is None
+        p.overflow = []
+        assert p.addresses() is not None and stacked_packs(packs) is not None
+    p.a_cat = torch.zeros(128, K)
+    assert p.R == 128 and packs[0].R == R
