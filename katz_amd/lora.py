@@ -307,7 +307,7 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
     rows, pieces, packs, n_pieces = [], [], [], 0
     at_a = at_b = at_s = at_an = at_c = 0
     b_blocks, padded, keys = [], [], {}
-    pool = []
+    pool, plain = [], []                               # plain: without the folded norms' buffers, so that a pack that needs none does not keep them
     for l, ns in zip(layers, names):
         d = l.__dict__
         K, N, ads = d["in_features"], d["out_features"], d["adapters"]
@@ -336,7 +336,7 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
                 w = g.weight
                 nk = keys[id(g)] = (norm_key(g), w.data_ptr(), g.bias.data_ptr()) if w.dtype == torch.bfloat16 and w.device == dev else ()
         rows += (at_a, at_an if nk else -1) + (nk[1:] if nk else (0, 0)) + (at_c, at_c, at_b, at_s, K, N, R, int(d["geglu"]), n_pieces, len(ns))
-        packs.append(PooledPack(pool, (at_a, at_b, at_s, at_an, at_c), (R, K, N), ns, ranks, min(R, (c + 15) // 16 * 16), nk[0] if nk else None))
+        packs.append(PooledPack(pool if nk else plain, (at_a, at_b, at_s, at_an, at_c), (R, K, N), ns, ranks, min(R, (c + 15) // 16 * 16), nk[0] if nk else None))
         n_pieces += len(ns)
         padded.append(R)
         b_blocks.append(-(-N // (256 // (R // 8))))
@@ -348,6 +348,7 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
             at_c += R
     buf = lambda n, dt: torch.empty((n,), dtype=dt, device=dev)
     pool += (buf(at_a, torch.bfloat16), buf(at_b, torch.bfloat16), buf(at_s, torch.float32), buf(at_an, torch.bfloat16), buf(at_c, torch.float32), buf(at_c, torch.float32))
+    plain += pool[:3]
     base = [t.data_ptr() for t in pool]
     table = np.array(rows, dtype=np.int64).reshape(-1, 14)
     folded = table[:, 1] >= 0

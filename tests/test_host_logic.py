@@ -824,3 +824,31 @@ def test_fields_of_a_pooled_pack_can_be_assigned():
         assert p.addresses() is not None and stacked_packs(packs) is not None
     p.a_cat = torch.zeros(128, K)
     assert p.R == 128 and packs[0].R == R
+
+
+def test_packs_without_a_norm_do_not_keep_the_folded_buffers(monkeypatch):
+    """pack_many's buffers for folded norms are given back with the last pack behind a norm, whatever other packs of the call stay; packs of one kind still
+    lie one behind the other."""
+    import gc
+    import weakref
+
+    from katz_amd import ops
+    from katz_amd.lora import Adapter, pack_many, stacked_packs
+    import katz_amd.layers as L
+
+    monkeypatch.setattr(ops, "upload_many", lambda ts, dev: (None, [t.data_ptr() for t in ts]))
+    monkeypatch.setattr(ops, "lora_pack", lambda *a: None)
+    norm = L.LayerNorm(16).bfloat16()
+    layers = []
+    for i in range(4):
+        l = L.LoRALinear(16, 24, bias=False).bfloat16()
+        l.adapters["a"] = Adapter(torch.randn(8, 16).bfloat16(), torch.randn(24, 8).bfloat16())
+        l.fold_norm = (lambda: norm) if i < 2 else (lambda: None)
+        layers.append(l)
+    packs = pack_many(layers, [["a"]] * 4)
+    assert all(p.ln is not None for p in packs[:2]) and all(p.ln is None for p in packs[2:])
+    assert stacked_packs(packs[:2]) is not None and stacked_packs(packs[2:]) is not None
+    folded, shared = [weakref.ref(t) for t in packs[0].pool[3:]], [weakref.ref(t) for t in packs[0].pool[:3]]
+    del packs[:2]
+    gc.collect()
+    assert len(folded) == 3 and all(r() is None for r in folded) and all(r() is not None for r in shared)
