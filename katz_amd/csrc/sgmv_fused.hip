@@ -94,12 +94,13 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
     blocks = blocks < p.row_blocks ? blocks : p.row_blocks;
     // (blocks of adapters of more than 64 in the upper half of the word, where 64 segments' blocks fit half a word)
     const bool halves = p.row_blocks < 1024;
-    int sum = blocks | (halves && rk > 64 ? blocks << 16 : 0);
+    uint32_t sum = (uint32_t)blocks | (halves && rk > 64 ? (uint32_t)blocks << 16 : 0u);
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(sum, o, 64); if (lane >= o) sum += v; }
-    const int total = __builtin_amdgcn_readlane(sum, 63), heavy = halves ? (int)((unsigned)total >> 16) : 0, per_layer = halves ? total & 0xffff : total;
+    for (int o = 1; o < 64; o <<= 1) { const uint32_t v = __shfl_up(sum, o, 64); if (lane >= o) sum += v; }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)sum, 63);
+    const int heavy = halves ? (int)(total >> 16) : 0, per_layer = (int)(halves ? total & 0xffff : total);
     const int nb = per_layer * p.n_layers;
-    int upto = halves ? sum & 0xffff : sum;       // blocks up to this lane's segment
+    int upto = (int)(halves ? sum & 0xffff : sum);       // blocks up to this lane's segment
     wait_cnt<0, 0>();                             // (or the compiler waits for them, and all behind them, among phase 1's loads)
     const int u = (int)blockIdx.x, full = nb / CUS * CUS;
     int b = u, last = nb;
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
       const int h8 = (heavy + 7) & ~7, l8 = (nb - heavy + 7) & ~7;
       if (full == 0 && p.n_layers == 1 && heavy > 0 && heavy < nb && z < all_tiles && h8 * (z + 1) + l8 * z <= CUS) {
         const bool mine = v < h8 * (z + 1);
-        upto = mine ? (int)((unsigned)sum >> 16) : upto - (int)((unsigned)sum >> 16);
+        upto = mine ? (int)(sum >> 16) : upto - (int)(sum >> 16);
         v = mine ? v : v - h8 * (z + 1);
         last = mine ? heavy : nb - heavy;
         z = mine ? z + 1 : z;

@@ -998,6 +998,28 @@ def test_sgmv_fused_dealt_by_the_segments(lens, longest, K, N, RP):
         assert err <= 2 ** -7 * ref.abs().max(), (i, w, float(err))
 
 
+def test_sgmv_fused_of_many_heavy_blocks():
+    """More row blocks of adapters of more than 64 than half of a signed word's upper half counts (64 x 516 of 128 rows): every row once.  Tolerance as
+    above."""
+    from katz_amd import ops
+
+    n, rows, K, N = 64, 66000, 64, 128
+    say("sgmv fused, many heavy blocks", n, rows, K, N)
+    d = dev()
+    torch.manual_seed(1)
+    a, b = (torch.randn(2, 128, K, device=d) * K ** -0.5).to(BF), (torch.randn(2, N, 128, device=d) * 128 ** -0.5).to(BF)
+    a[1, 96:], b[1, :, 96:] = 0, 0
+    x, base = torch.randn(n * rows, K, device=d, dtype=BF), torch.randn(n * rows, N, device=d, dtype=BF)
+    i32 = dict(dtype=torch.int32, device=d)
+    y = base.clone()
+    ops.sgmv_fused_(y, x, a, b, torch.arange(n + 1, **i32) * rows, torch.arange(n, **i32) % 2, torch.tensor([128, 96], **i32), torch.tensor([0.5, 0.75], device=d), rows)
+    for i in range(n):
+        s = slice(i * rows, (i + 1) * rows)
+        t = (x[s].double() @ a[i % 2].double().T).to(BF).double()
+        ref = (base[s].double() + ((0.5 + 0.25 * (i % 2)) * (t @ b[i % 2].double().T)).to(BF).double()).to(BF).double()
+        assert (y[s].double() - ref).abs().max() <= 2 ** -7 * ref.abs().max(), i
+
+
 @pytest.mark.parametrize("shapes,r,dt", [
     ([(128, 128)], 128, torch.float16),                                        # two turns of 64 ranks
     ([(130, 260), (1, 8), (257, 1284)], 96, torch.bfloat16),                   # a turn and a half, pieces of 8 bytes, ragged tiles
