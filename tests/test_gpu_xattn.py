@@ -255,3 +255,72 @@ def test_few_queries_on_small_tiles(B, T, heads, K, R, used):
         more = ops.lora_linear_xattn(*(t.repeat(n, 1, 1) if t.dim() == 3 else t for t in (xd, wd, kd, vd)), heads)
         assert torch.equal(o, more[:B]) and torch.equal(o, more[-B:])
     ops.check_split_timeouts()
+
+
+@pytest.mark.parametrize("B,T,heads,K,R,used", [
+    (1, 128, 2, 64, 0, 0),          # 32 x 64 tiles, a loop of one stage
+    (1, 128, 20, 1280, 64, 16),     # ... with pieces of T beside them
+    (2, 256, 20, 1280, 64, 32),     # 64 x 64 tiles and pieces
+    (2, 256, 20, 1280, 0, 0),
+    (1, 768, 20, 1280, 64, 64),     # 64 x 128 tiles
+    (3, 128, 10, 640, 128, 96),     # rank columns of two groups
+])
+def test_folded_layer_norm_on_small_tiles(B, T, heads, K, R, used):
+    """norm2 folded into the projections of below 1024 rows, the form that a model runs: the rows' and columns' terms in 32- and 64-row tiles and the pieces of
+    T that carry the norm's share.  Against the oracle and float64; one launch and two, and strided and contiguous k / v, give the same bits."""
+    from katz_amd import ops
+    from katz_amd.lora import fold_layer_norm
+    say("xattn behind a folded LayerNorm, small tiles", B, T, heads, K, R, used)
+    d, S = dev(), 77
+    M, N = B * T, heads * 64
+    x, w, k, v, A, Bm = _case(B, T, heads, K, S, R, seed=31 + M + K + R)
+    if R:
+        A[used:], Bm[:, used:] = 0, 0
+    g = torch.Generator().manual_seed(32)
+    x = bf16_round(x * 2.0 + 0.5)
+    gamma, beta = bf16_round(1.0 + 0.2 * torch.randn(K, generator=g)), randn(g, K, std=0.2)
+    st = torch.zeros((ops.LN_SLOTS, M, 2), dtype=torch.float32)
+    xf = x.reshape(M, K).float()
+    st[0, :, 0], st[0, :, 1] = xf.sum(-1), (xf * xf).sum(-1)
+    st = st.to(d)
+    scale = 0.8
+    wp, c1, c2, ap, ca1, ca2 = fold_layer_norm(w.to(d, BF), None, gamma.to(d, BF), beta.to(d, BF), None if A is None else A.to(d, BF))
+    kw = dict(ln=(st, c1, c2, ca1, ca2, 1e-5))
+    if R:
+        kw.update(a_cat=ap, col_scale=torch.full((R,), scale, device=d), b_cat=Bm.to(d, BF), r_used=used)
+    kd, vd = torch.cat([k, v], -1).to(d, BF).split(N, dim=-1)
+    o = ops.lora_linear_xattn(x.to(d, BF), wp, kd, vd, heads, **kw)
+    ref = _ref(x, w, k, v, heads, A, Bm, scale, ln=(gamma, beta))
+    exact = _ref(x, w, k, v, heads, A, Bm, scale, ln=(gamma, beta), exact=True)
+    say(f"  rms error against float64: {_rms_err(o, exact):.2e} (reference's rounding {_rms_err(bf16_round(ref), exact):.2e})")
+    assert_close_rel(o, ref, CHAIN_TOL, "folded LayerNorm + projection + attention on small tiles")
+    assert torch.equal(o, ops.lora_linear_xattn(x.to(d, BF), wp, k.to(d, BF), v.to(d, BF), heads, **kw)), "strided k / v"
+    if R:
+        assert torch.equal(o, ops.lora_linear_xattn(x.to(d, BF), wp, kd, vd, heads, two_launches=True, **kw)), "two launches"
+    ops.check_split_timeouts()
+
+
+@pytest.mark.parametrize("R", [0, 64])
+def test_rows_of_two_gibibytes(R):
+    """x of 2 GiB, more than one descriptor of the fine tiles spans: another kernel's 128 x 128 tiles, the same bits as for the last rows by themselves
+    (T aside, whose sums a few rows deal to other waves), and the library's two calls."""
+    from katz_amd import ops
+    say("xattn, 2 GiB of x", R)
+    d = dev()
+    B, T, heads, K, S = 1, 32768, 2, 32768, 77
+    N = heads * 64
+    torch.manual_seed(R)
+    x, w = torch.randn(B, T, K, device=d, dtype=BF), (torch.randn(N, K, device=d) * K ** -0.5).to(BF)
+    k, v = torch.randn(B, S, N, device=d, dtype=BF), torch.randn(B, S, N, device=d, dtype=BF)
+    assert x.numel() * 2 == 1 << 31 and ops.lora_linear_xattn_ok(B * T, N, K, R, T, S, heads)
+    kw = {}
+    if R:
+        kw = dict(a_cat=(torch.randn(R, K, device=d) * K ** -0.5).to(BF), col_scale=torch.full((R,), 0.5, device=d), b_cat=(torch.randn(N, R, device=d) * 0.1).to(BF))
+    o = ops.lora_linear_xattn(x, w, k, v, heads, **kw)
+    q = ops.lora_linear_split(x, w, None, kw["a_cat"], kw["col_scale"], kw["b_cat"]) if R else ops.lora_linear(x, w, None)
+    assert_close_rel(o, ops.attention(q, k, v, heads).float().cpu(), CHAIN_TOL, "one launch against the library's two calls")
+    few = ops.lora_linear_xattn(x[:, -128:].contiguous(), w, k, v, heads, **kw)
+    assert_close_rel(o[:, -128:], few.float().cpu(), 1e-2, "the last rows by themselves")
+    if not R:
+        assert torch.equal(o[:, -128:], few)
+    ops.check_split_timeouts()
