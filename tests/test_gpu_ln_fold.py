@@ -321,3 +321,66 @@ def test_transformer_with_and_without_the_fold(monkeypatch):
     say(f"  cosine against the oracle: folded {c1:.6f}, separate norms {c0:.6f}; folded against separate {c10:.6f}")
     assert c1 >= 0.9995 and c0 >= 0.9995 and c10 >= 0.9995
     assert_close_rel(y1, ref, 6e-2, "transformer with folded LayerNorms")
+
+
+@pytest.mark.parametrize("M,N,K,R,n_split", [
+    (1300, 3840, 1280, 128, 1280),   # stacked q / k / v between one and two rounds
+    (1800, 3840, 1280, 0, 0),
+    (4608, 1920, 640, 64, 640),
+    (191, 960, 128, 64, 0),          # less than a tile of 192 rows
+])
+def test_folded_norm_on_tiles_of_160_columns_and_many_rows(M, N, K, R, n_split):
+    """128 / 160 / 192 x 160 tiles (codes 69 to 71) and the tile that is chosen, behind a folded norm: the bits of the 128 x 128 kernel (16), terms of rows beyond
+    128 and slices of T by n_split among them; and no less accurate than LayerNorm, rounding and linear."""
+    from katz_amd import _lib, ops
+    from katz_amd.lora import fold_layer_norm
+    say("folded LayerNorm, 160 columns", M, N, K, R, n_split)
+    lib, d = _lib.load(), dev()
+    h, gamma, beta, w, b, A, B = _fold_case(M, N, K, R, seed=M + N + K + R, n_split=n_split)
+    scale = 0.8
+    wp, c1, c2, ap, ca1, ca2 = fold_layer_norm(w.to(d, BF), b.to(d, BF), gamma.to(d, BF), beta.to(d, BF), None if A is None else A.to(d, BF))
+    st, hd = _stats_from(h, d), h.to(d, BF)
+    RT = 0 if A is None else A.shape[0]
+    s, bc = (torch.full((RT,), scale, device=d), B.to(d, BF)) if R else (None, None)
+    p = lambda t: None if t is None else t.data_ptr()
+
+    def run(tile):
+        y, t = torch.zeros(M, N, dtype=BF, device=d), torch.zeros(M, max(RT, 1), dtype=BF, device=d)
+        rc = lib.kh_lora_linear_norm_bf16(p(hd), p(wp), None, p(ap), p(s), p(bc), p(t) if R else None, None, None, p(y), p(st), p(c1), p(c2), p(ca1), p(ca2), 1e-5, None,
+                                          M, N, K, R, n_split, tile << 8, ops._stream())
+        assert rc == 0, tile
+        return y
+
+    want = run(16)
+    for tile in (69, 70, 71, 0):
+        assert torch.equal(run(tile), want), tile
+    ref = _ref_fold(h, gamma, beta, w, b, A, B, scale, n_split)
+    exact = _ref_fold(h, gamma, beta, w, b, A, B, scale, n_split, exact=True)
+    assert _rms_err(want, exact) <= 1.25 * _rms_err(bf16_round(ref), exact) + 1e-4
+    assert_close_rel(want, exact.float(), 2e-2, "folded LayerNorm + linear")
+
+
+@pytest.mark.parametrize("M,N,K,R,res", [(2304, 1280, 2560, 0, True), (2300, 1280, 2560, 64, False), (4200, 640, 2624, 128, True)])
+def test_row_statistics_of_long_sums_in_one_round(M, N, K, R, res):
+    """One round of 128 x 128 tiles with a long sum and T given or none (chosen: operand waves beside four that compute): result and row statistics have the
+    bits of the tiles whose waves do both (code 32)."""
+    from katz_amd import _lib, ops
+    say("row statistics, long sums", M, N, K, R, res)
+    lib, d = _lib.load(), dev()
+    g = torch.Generator().manual_seed(M + N + K + R)
+    x, w, b, r = (t.to(d, BF) for t in (randn(g, M, K), randn(g, N, K, std=0.03), randn(g, N, std=0.1), randn(g, M, N)))
+    A, B, s = randn(g, max(R, 1), K, std=0.05).to(d, BF), randn(g, N, max(R, 1), std=0.05).to(d, BF), torch.full((max(R, 1),), 0.7, device=d)
+    p = lambda t: t.data_ptr()
+
+    def run(tile):
+        y, t, st = torch.zeros(M, N, dtype=BF, device=d), torch.zeros(M, max(R, 1), dtype=BF, device=d), ops.row_stats_buffer(M, d).fill_(float("nan"))
+        rc = lib.kh_lora_linear_norm_bf16(p(x), p(w), p(b), p(A), p(s), p(B), p(t), None, p(r) if res else None, p(y), None, None, None, None, None, 0.0, p(st),
+                                          M, N, K, R, 0, tile << 8, ops._stream())
+        assert rc == 0, tile
+        return y, st
+
+    (y, st), (y0, st0) = run(0), run(32)
+    assert torch.equal(y, y0) and torch.equal(st, st0)
+    s1, s2 = _stats_of(y)
+    got = st.double().sum(0)
+    assert torch.allclose(got[:, 0], s1.double(), rtol=1e-3, atol=1e-2 * float(s2.max().sqrt())) and torch.allclose(got[:, 1], s2.double(), rtol=1e-3)
