@@ -951,6 +951,25 @@ def test_convolutions_of_many_pixels_on_tiles_by_their_rounds(Nb, H, W, Cin, Cou
     assert torch.equal(ops.conv3x3(x, ops.pack_conv3x3_weight(w), b, stride=stride, residual=r), y)
 
 
+@pytest.mark.parametrize("Nb,H,W,Cin,Cout,stride,res", [(2, 72, 72, 64, 320, 1, False), (2, 96, 97, 64, 320, 1, True), (1, 104, 152, 128, 640, 1, True), (3, 110, 96, 64, 960, 2, False),
+                                                        (2, 36, 32, 640, 1280, 1, True), (2, 36, 36, 1280, 1280, 1, False), (2, 56, 40, 384, 1280, 1, False)])
+def test_convolutions_by_their_rounds_have_the_bits_of_the_large_tiles(Nb, H, W, Cin, Cout, stride, res):
+    """Eight columns less leave a width that no other tile divides, so that the 128 x 128 kernel takes the convolution: the columns that both have are the same."""
+    from katz_amd import ops
+
+    say("convolution, same bits", Nb, H, W, Cin, Cout, stride, res)
+    d, g = dev(), torch.Generator().manual_seed(H + W + Cin)
+    x = torch.randn(Nb, Cin, H, W, generator=g).to(d, torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    w = (torch.randn(Cout, Cin, 3, 3, generator=g) * (9 * Cin) ** -0.5).to(d, torch.bfloat16)
+    b = torch.randn(Cout, generator=g).to(d, torch.bfloat16)
+    r = torch.randn(Nb, Cout, (H - 1) // stride + 1, (W - 1) // stride + 1, generator=g).to(d, torch.bfloat16).contiguous(memory_format=torch.channels_last) if res else None
+    n = Cout - 8
+    y = ops.conv3x3(x, ops.pack_conv3x3_weight(w), b, stride=stride, residual=r)
+    y0 = ops.conv3x3(x, ops.pack_conv3x3_weight(w[:n].contiguous()), b[:n].contiguous(), stride=stride,
+                     residual=None if r is None else r[:, :n].contiguous(memory_format=torch.channels_last))
+    assert torch.equal(y[:, :n], y0)
+
+
 @pytest.mark.parametrize("lens,longest,K,N,RP", [
     ([1, 0, 65, 200, 64, 70], 200, 576, 1280, 128),                           # ranges of one column tile, nine stages
     ([650] * 4 + [0, 30], 650, 512, 640, 64),                                 # a full ring of stages
@@ -996,6 +1015,43 @@ def test_sgmv_fused_dealt_by_the_segments(lens, longest, K, N, RP):
         ref = (base[s:e].double() + delta).to(BF).double()
         err = (y[s:e].double() - ref).abs().max()
         assert err <= 2 ** -7 * ref.abs().max(), (i, w, float(err))
+
+
+@pytest.mark.parametrize("layers,lens,longest", [
+    (53, [64, 1, 30, 0, 63, 40], 64),                      # 64-row blocks, four a layer (an empty segment, one without an adapter): 212, less than a round
+    (62, [64, 1, 30, 63, 40], 64),                         # ... 248
+    (53, [64, 1, 30, 7, 63, 40], 64),                      # five a layer, 265: a round and nine of the last two layers in ranges
+    (37, [130, 1, 77, 128, 300, 0, 129], 300),             # 128-row blocks, nine a layer, 333: a layer cut by the end of the round
+    (101, [200, 0, 129, 31], 200),                         # three a layer, 303
+], ids=str)
+def test_sgmv_fused_grouped_in_whole_rounds_and_ranges(layers, lens, longest):
+    """Many layers dealt on the device, whole rounds of the CUs and what is left: each layer has the bits of its own launch, and rows without an adapter stay."""
+    from katz_amd import ops
+
+    say("sgmv fused grouped, rounds", layers, lens, longest)
+    d, K, N, RP = dev(), 128, 384, 128
+    torch.manual_seed(layers)
+    start = [0]
+    for n in lens:
+        start.append(start[-1] + n)
+    ranks = [32, 128, 64, 96]
+    who = [i % 4 for i in range(len(lens))]
+    who[2] = -1
+    i32 = dict(dtype=torch.int32, device=d)
+    rows, ss, sa = start[-1], torch.tensor(start, **i32), torch.tensor(who, **i32)
+    rk, sc = torch.tensor(ranks, **i32), torch.tensor([0.5, 0.75, 1.0, 1.25], device=d)
+    x = torch.randn(rows, K, device=d).to(BF)
+    a, b = (torch.randn(layers, 4, RP, K, device=d) * K ** -0.5).to(BF), (torch.randn(layers, 4, N, RP, device=d) * RP ** -0.5).to(BF)
+    for i, r in enumerate(ranks):
+        a[:, i, r:], b[:, i, :, r:] = 0, 0
+    base = torch.randn(layers, rows, N, device=d).to(BF)
+    y, want = base.clone(), base.clone()
+    ops.sgmv_fused_grouped_(list(y), x, list(a), list(b), ss, sa, rk, sc, longest)
+    for l in range(layers):
+        ops.sgmv_fused_(want[l], x, a[l], b[l], ss, sa, rk, sc, longest)
+        assert torch.equal(y[l], want[l]), l
+    assert torch.equal(y[:, start[2]:start[3]], base[:, start[2]:start[3]])
+    assert not torch.equal(y[-1, start[-2]:], base[-1, start[-2]:])
 
 
 def test_sgmv_fused_of_many_heavy_blocks():
