@@ -236,14 +236,14 @@ class _Ready:
             if p is None:
                 continue
             v, d = p.__dict__, getattr(self.desc, name)
-            if v.get("overflow") or not split:             # (PooledPack makes its list when it is asked)
+            if p.wide or not split:
                 return False
             for t in ("a_cat", "b_cat", "col_scale"):
                 expect(v, t)
             at = p.addresses(nk) if type(p) is PooledPack else None
             if at is not None:                             # by address: no views are made
                 d.a_cat, d.b_cat, d.col_scale, d.ca1, d.ca2 = at
-                d.R, d.r_used = p.R, p.r_used
+                d.R, d.r_used = p.shape[0], p.r_used
                 keep.append(p)
                 continue
             a, b, s = p.a_cat, p.b_cat, p.col_scale
@@ -262,7 +262,7 @@ class _Ready:
                 st = weights
                 plan.weights(q, w, None, c1, c2)
                 q.a_cat, q.b_cat, q.col_scale, q.ca1, q.ca2 = at[0]
-                q.R, q.r_used, q.n_split = first.R, max(p.r_used for p in qkv), plan.inner
+                q.R, q.r_used, q.n_split = first.shape[0], max(p.r_used for p in qkv), plan.inner
                 a, b, _ = side_by_side                     # (hints hold them weakly)
                 if nk is not None:
                     a = first.pool[3].as_strided(a.shape, a.stride(), first.at[3])
@@ -384,7 +384,7 @@ class _LinearReady:
         self.a_cat = None if p is None else p.a_cat
         self.usable = (type(l) is layers.LoRALinear and l.__dict__.get("bias") is None and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous()
                        and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous()))
-                       and (p is None or (not p.overflow and layers.LORA_MODE == "split" and l.in_features % 64 == 0)))
+                       and (p is None or (not p.wide and layers.LORA_MODE == "split" and l.in_features % 64 == 0)))
         if not self.usable:
             return
         d = self.desc = _Linear()
@@ -393,7 +393,7 @@ class _LinearReady:
         if p is not None:
             b_cat = p.b_cat
             d.a_cat, d.b_cat, d.col_scale = p.a_cat.data_ptr(), b_cat.data_ptr(), p.col_scale.data_ptr()
-            d.R, d.r_used = p.R, p.r_used
+            d.R, d.r_used = p.shape[0], p.r_used
         self.keep = (w, b, b_cat, None if p is None else p.col_scale)
         self.refs = tuple(None if t is None else weakref.ref(t) for t in (w, self.a_cat, b_cat))
         self.at, self.key, self.device = ctypes.addressof(d), int(d.w), w.device

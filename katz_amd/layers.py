@@ -263,7 +263,7 @@ class LoRALinear(nn.Module):
         """Can this call go through kh_lora_linear_norm_bf16 (a folded LayerNorm in front, row statistics out)?"""
         p = self._packed
         return (LN_FOLD and x.dtype == torch.bfloat16 and self.weight.dtype == torch.bfloat16 and self.in_features % 64 == 0
-                and self.out_features % 8 == 0 and (p is None or (not p.overflow and LORA_MODE == "split"))
+                and self.out_features % 8 == 0 and (p is None or (not p.wide and LORA_MODE == "split"))
                 and (not stats or (self.out_features <= 128 * ops.LN_SLOTS and not self.geglu)))
 
     def _ln_terms(self, norm: "LayerNorm"):
@@ -317,7 +317,7 @@ class LoRALinear(nn.Module):
             stats_out.valid = False
         if p is None:
             return ops.lora_linear(x, w, b, residual=residual, geglu=self.geglu)
-        if p.overflow:
+        if p.wide:
             return self._forward_wide(x, residual, p)
         if LORA_MODE == "split" and x.dtype == torch.bfloat16 and self.in_features % 64 == 0:
             return ops.lora_linear_split(x, w, b, p.a_cat, p.col_scale, p.b_cat, residual=residual, geglu=self.geglu,
@@ -335,7 +335,7 @@ class LoRALinear(nn.Module):
         p = self._packed
         B, T, K = x.shape
         R = 0 if p is None else p.R
-        if w.dtype != torch.bfloat16 or (p is not None and (p.overflow or LORA_MODE != "split")):
+        if w.dtype != torch.bfloat16 or (p is not None and (p.wide or LORA_MODE != "split")):
             return None
         if k.shape != (B, k.shape[1], self.out_features) or v.shape != k.shape or k.stride(-1) != 1 or v.stride(-1) != 1:
             return None
@@ -910,7 +910,7 @@ class Attention(nn.Module):
         st = self._qkv
         if st is None or st["sig"] != sig:
             packs = [l._packed for l in layers]
-            same = all(p is None for p in packs) or (all(p is not None and not p.overflow for p in packs) and len({p.R for p in packs}) == 1)
+            same = all(p is None for p in packs) or (all(p is not None and not p.wide for p in packs) and len({p.R for p in packs}) == 1)
             ok = same and (packs[0] is None or LORA_MODE == "split") and all(l.bias is None for l in layers)
             st = dict(sig=sig, ok=ok)
             if ok:
@@ -1141,7 +1141,7 @@ class ContextKVProjector:
             l.prepare()
         K = layers[0].in_features
         packs = [l._packed for l in layers]
-        uniform = all(p is None for p in packs) or (all(p is not None and not p.overflow for p in packs) and len({p.R for p in packs}) == 1)
+        uniform = all(p is None for p in packs) or (all(p is not None and not p.wide for p in packs) and len({p.R for p in packs}) == 1)
         ok = uniform and LORA_MODE == "split" and all(l.weight.dtype == torch.bfloat16 and not l.geglu for l in layers)
         st = dict(epoch=_pack_epoch, M=M, ok=ok, wptr=[l.weight.data_ptr() for l in layers])
         if ok:

@@ -65,6 +65,11 @@ class PackedAdapters:
         return self.a_cat.shape[0]
 
     @property
+    def wide(self) -> bool:
+        """More rank columns than one launch takes?  (Does not make a PooledPack's list.)"""
+        return bool(self.__dict__.get("overflow"))
+
+    @property
     def r_used(self) -> int:
         """Rank columns that can be non-zero (the adapters' ranks side by side), rounded up to the 16 columns of one
         MFMA step; the columns from there to R are zero padding."""
