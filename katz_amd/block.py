@@ -393,7 +393,7 @@ class _LinearReady:
         if p is not None:
             b_cat = p.b_cat
             d.a_cat, d.b_cat, d.col_scale = p.a_cat.data_ptr(), b_cat.data_ptr(), p.col_scale.data_ptr()
-            d.R, d.r_used = p.shape[0], p.r_used
+            d.R, d.r_used = p.R, p.r_used
         self.keep = (w, b, b_cat, None if p is None else p.col_scale)
         self.refs = tuple(None if t is None else weakref.ref(t) for t in (w, self.a_cat, b_cat))
         self.at, self.key, self.device = ctypes.addressof(d), int(d.w), w.device
