@@ -16,9 +16,9 @@
 //
 // What bounds it: the vector ALU (exp, scale, maximum, conversion: about 1000 of the 1200 clocks a wave of 32 queries spends on a tile with three waves per
 // SIMD) and, before the last round's workgroups were halved, that round (620 of 128 queries on 256 CUs: three on some, 2.4 on average).  A wave of 16
-// reads as many bytes of K and V from LDS as one of 32, so only those workgroups are halved that would leave CUs idle.  us per call, all of 128 queries
-// (64 on two waves for short keys on small grids) -> now (batch, tokens, heads): 2 x 4096 x 10 109.2 -> 97.4, 2 x 3952 x 10 105.0 -> 93.1, 2 x 1024 x 20 22.5 -> 20.0, 1 x 3952 x 10
-// 71.3 -> 59.5, 1 x 988 x 20 16.3 -> 15.8, 2 x 256 x 20 5.6 -> 4.9, 988 queries on 77 keys 5.5 -> 4.8, 2 x 3952 x 10 on 77 9.3 -> 8.8.
+// reads as many bytes of K and V from LDS as one of 32, so only those workgroups are halved that would leave CUs idle.  us per launch in a graph, all of 128
+// queries (64 on two waves for short keys on small grids) -> now, one run (batch, tokens, heads): 2 x 4096 x 10 113.3 -> 100.5, 2 x 3952 x 10 109.7 -> 95.8, 2 x 1024 x 20 23.5 -> 20.6,
+// 1 x 3952 x 10 73.6 -> 60.3, 1 x 988 x 20 16.8 -> 15.7, 2 x 256 x 20 5.7 -> 4.9, 988 queries on 77 keys 5.5 -> 4.8, 2 x 3952 x 10 on 77 9.4 -> 8.7.
 // K and V by DMA into unpadded swizzled tiles, V transposed by the read, took 114 us where registers and eight 4-byte
 // LDS writes a thread took 125 (2 x 3952 x 10).  Transposing reads as inline assembly, without the compiler's wait for every DMA in front of
 // them and with the DMA a whole step ahead, measured the same; 64 queries per workgroup everywhere 113 us at 2 x 3952 x 10.

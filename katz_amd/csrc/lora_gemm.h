@@ -63,8 +63,9 @@ struct LoraGemmParams {
   // of the NEXT launch of this family, so that they wait in the memory-side cache when that launch asks for them (a
   // step reads 2.5 GB of weights once each: every launch would otherwise meet its weights in HBM, where the XCDs that
   // share a weight block each fetch it again).  Set from kh_set_weight_prefetch by the entry points.
-  // Cross-attention in the epilogue (xa_k != nullptr; the 128x128 / 8-wave tiles only): the layer is an attention's to_q
-  // and a 128 x 128 output tile holds 128 queries of two 64-wide heads; instead of storing them the workgroup runs
+  // Cross-attention in the epilogue (xa_k != nullptr): the layer is an attention's to_q and an output tile holds queries of
+  // one sample by whole 64-wide heads -- 32, 64 or 128 queries of one or two heads on the fine tiles (xattn_tile.h), 128 of two
+  // on the 128x128 / 8-wave tiles (lora_gemm_pipe.hip); instead of storing them the workgroup runs
   // softmax(q k^T * scale) v for them against the xa_S <= 96 keys of those heads and stores that to xa_o (rows like y's,
   // head h at columns 64 h).  Rows m belong to batch sample m / xa_T (xa_T % 128 == 0); k / v: [B, S, heads * 64] views.
   const bf16_t* xa_k = nullptr; const bf16_t* xa_v = nullptr; bf16_t* xa_o = nullptr;
@@ -121,7 +122,9 @@ __device__ __forceinline__ bool il_narrow(const LoraGemmParams& p) { return p.il
 // The pending weight prefetch of this host thread (kh_set_weight_prefetch), handed to the next launch.
 void kh_take_weight_prefetch(LoraGemmParams& p);
 
-constexpr int KH_LN_LDS = 4096;    // bytes of dynamic LDS a launch with a folded LayerNorm adds: mean, 1/std of up to 256 rows, c1, c2 of up to 256 columns
+// bytes of dynamic LDS a launch with a folded LayerNorm adds: mean, 1/std of a tile's rows, c1, c2 of its columns, 2 * max(BM, 128) + 2 * BN floats at most
+// (192 x 320 tiles use all of it)
+constexpr int KH_LN_LDS = 4096;
 constexpr int KH_LN_SLOTS = 16;     // partial pairs per row: at most 16 column tiles (N <= 2048 with 128-column tiles)
 
 // Touch lines first, first + n_wg * NT, ... of the prefetch range: one dword per line and lane, loaded into 256 bytes of
@@ -290,8 +293,8 @@ int lora_gemm_ksplit_launch(const LoraGemmParams& p, int row_groups, hipStream_t
 // on, 0 when the rules give it other tiles or the groups do not fit them
 int lora_gemm_conv_gn_row_groups(const LoraGemmParams& p);
 // Fine tiles (lora_gemm_fine.hip), with the sums in the order of the 128 x 128 (order 0), the 128 x 160 (order 2) or the 64 x 160 kernel
-// (order 4); plain or K-extended GEMM and (orders 2 and 4) 3x3 convolutions.  ok: what the kernel takes at all; form: -1 where order 0
-// is not suited (orders 2 and 4: the caller has seen to N % 160 and the number of tiles).
+// (order 4); plain or K-extended GEMM and 3x3 convolutions (in order 0 on 128 x 128 and 128 / 160 / 192 x 160, without GroupNorm statistics).
+// ok: what the kernel takes at all; form: -1 where order 0 is not suited (orders 2 and 4: the caller has seen to N % 160 and the number of tiles).
 bool lora_gemm_fine_ok(const LoraGemmParams& p);
 int lora_gemm_fine_form(const LoraGemmParams& p, int order);
 int lora_gemm_rounds_form(const LoraGemmParams& p);          // of a convolution or a linear layer with many rows in order 0; -1: none

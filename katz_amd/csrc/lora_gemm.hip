@@ -698,7 +698,7 @@ static int lora_linear_norm_impl(const void* x, const void* w, const void* bias,
   const int tile_sel = (flags >> 8) & 0xff;
   const bool may_wait = counters != nullptr && tile_sel == 0 && (flags & KH_FLAG_NO_WAIT) == 0;
   if (xa != nullptr) {
-    // the projection's result never reaches memory: its 128 x 128 tiles are 128 queries of two heads each
+    // the projection's result never reaches memory: its tiles are queries of one sample by whole heads (LoraGemmParams::xa_k)
     if (!xa->k || !xa->v || !xa->o || xa->T <= 0 || xa->S <= 0 || M % xa->T != 0) return KH_ERR_INVALID_ARG;
     if (residual != nullptr || stats_out != nullptr || geglu || n_split != 0 || (tile_sel != 0 && tile_sel != 1)) return KH_ERR_INVALID_ARG;
     if (xa->S > 96 || xa->T % 128 != 0 || N % 128 != 0 || (R % 64) != 0) return KH_ERR_UNSUPPORTED;

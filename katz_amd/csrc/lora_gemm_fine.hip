@@ -894,25 +894,14 @@ static int shrink_beside(LoraGemmParams& p, int form) {
   return with_il_tile(form, [&](auto c) { return plan_il<decltype(c)>(p) ? KH_OK : KH_ERR_UNSUPPORTED; }) == KH_OK ? p.il_tile : 0;
 }
 
-// Which of them, for a layer whose sums follow `order`; -1 where none fits and the larger tiles of the other families win.  A
-// convolution that leaves GroupNorm statistics does so per 64 rows.
-//
-// Linear layers: a CU's time is the rows it streams, BM + BN of K columns each, so the tile with the fewest of them whose workgroups fit
-// one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  Where the launch is to bring its shrink along,
-// the first that leaves the CUs for 16 x 16 pieces of it; where the loop is long enough to hide the larger pieces, the first that leaves them for
-// 32 x 32 ones if there is no other, or if its loop (us: 3 + 2.9e-5 a row and column of K) and those pieces (8 + 2.3e-3 K) are through before the larger
-// tile's loop (16 / 32: 512 / 1280 / 5120, 96 40.3 / 24.6, 154 21.6 / 20.5, 700 / 640 / 2560, 64 22.4 / 14.1, 400 / 1280 / 2048, 96 16.2 / 12.5; against that 308 / 1280 /
-// 2048, 64 12.0 / 13.3, 512 / 640 / 2560, 64 13.7 / 14.7, 308 / 1280 / 1280, 64 8.4 / 11.3); else two launches.  A T that is given leaves all CUs to the tiles (988 / 1280 / 1280, 64 11.3 us on tiles that leave some -> 10.0, K 5120 35.6 -> 30.7; 700 / 640 /
-// 2560 22.4 -> 11.2): the order of the sums is the same.
-// us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
-// 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
-// 512 / 1280 / 1280, 32 10.1 -> 9.3; 300 / 640 / 640, 64 7.3 -> 6.4; no adapters: 154 / 640 / 2048 12.1 -> 8.3, 655 / 1280 / 2048 12.2 -> 11.1.
 // GEGLU projections: of 64 / 128 / 160 / 192 x 320 tiles and the 256 x 320 ones of lora_gemm_wide.hip (-2) those whose rounds of the CUs take least; -1: 128 x 128 tiles.
 // A round costs about 100 rows more than its tiles have (its start, its epilogue; the 256-row tiles, whose waves move their own operands, 150).
 // us per launch without adapters, weights from HBM, before (in several rounds 128 x 320 on four computing waves, or 128 x 128) -> now: N 10240 / K 1280, M 512 22.7 ->
 // 22.1, 1024 34.5 -> 31.4, 1152 48 -> 34.6, 1280 55.5 -> 35.5, 1400 57.4 -> 40.3, 1536 47.8 -> 40.5, 1800 69.8 -> 56.0, 1976 71.4 -> 58.1, 2048 (256 rows) 55.8, 58.9 on 128;
 // N 5120 / K 640, M 1100 17.8 -> 16.0, 2304 28.7 -> 21.5, 3072 30.1 -> 25.7, 3952 44.2 -> 35.4, 4096 (256 rows) 33.7, 4608 50.3 -> 40.5, 6000 64.6 -> 50.6, 7200 77.7 -> 62.8,
 // 8192 (256 rows) 64.2, 69.6 on 192.
+// The 192-row tile has eight registers more than its wave: four lane constants and a fragment of the last stage go through scratch, 36 bytes a lane, all of it
+// ahead of the loop over K or behind it.
 int lora_gemm_geglu_form(const LoraGemmParams& p) {
   if (!lora_gemm_fine_ok(p) || p.st_part != nullptr || p.res != nullptr || p.N % 320 != 0 || p.t_nsplit % 320 != 0) return -1;
   if ((long)((p.M + 63) / 64) * (p.N / 320) <= 128) return -1;           // (up to half a round of 64 x 320 the 128 x 128 tiles are as fast)
@@ -928,6 +917,19 @@ int lora_gemm_geglu_form(const LoraGemmParams& p) {
   return lora_gemm_wide_ok(p) && cost(256, 150) < least ? -2 : best;
 }
 
+// Which of them, for a layer whose sums follow `order`; -1 where none fits and the larger tiles of the other families win.  A
+// convolution that leaves GroupNorm statistics does so per 64 rows.
+//
+// Linear layers: a CU's time is the rows it streams, BM + BN of K columns each, so the tile with the fewest of them whose workgroups fit
+// one round of the 256 CUs (a workgroup fills a CU, so a second round costs as much as the first).  Where the launch is to bring its shrink along,
+// the first that leaves the CUs for 16 x 16 pieces of it; where the loop is long enough to hide the larger pieces, the first that leaves them for
+// 32 x 32 ones if there is no other, or if its loop (us: 3 + 2.9e-5 a row and column of K) and those pieces (8 + 2.3e-3 K) are through before the larger
+// tile's loop (16 / 32: 512 / 1280 / 5120, 96 40.3 / 24.6, 154 21.6 / 20.5, 700 / 640 / 2560, 64 22.4 / 14.1, 400 / 1280 / 2048, 96 16.2 / 12.5; against that 308 / 1280 /
+// 2048, 64 12.0 / 13.3, 512 / 640 / 2560, 64 13.7 / 14.7, 308 / 1280 / 1280, 64 8.4 / 11.3); else two launches.  A T that is given leaves all CUs to the tiles (988 / 1280 / 1280, 64 11.3 us on tiles that leave some -> 10.0, K 5120 35.6 -> 30.7; 700 / 640 /
+// 2560 22.4 -> 11.2): the order of the sums is the same.
+// us per call, weights from HBM (M / N / K, rank: without the tiles of 32 and 64 columns -> now): 1 / 1280 / 1280, 16 12.1 -> 8.4;
+// 77 / 1280 / 2048, 32 14.1 -> 9.2; 154 / 1280 / 2048, 96 13.4 -> 10.7; 64 / 1280 / 5120, 32 36.7 -> 17.4; 256 / 1280 / 5120, 32 32.1 -> 20.6;
+// 512 / 1280 / 1280, 32 10.1 -> 9.3; 300 / 640 / 640, 64 7.3 -> 6.4; no adapters: 154 / 640 / 2048 12.1 -> 8.3, 655 / 1280 / 2048 12.2 -> 11.1.
 int lora_gemm_fine_form(const LoraGemmParams& p, int order) {
   if (!lora_gemm_fine_ok(p)) return -1;
   const long hw = p.gn_part != nullptr ? (long)p.conv_ho * p.conv_wo : p.M, nb = p.M / hw;
@@ -979,9 +981,11 @@ static long rounds_cost(const LoraGemmParams& p, int bm, int bn) {
 // -1: none divides the columns, or others win.
 // Convolutions, before on 128 x 128 tiles whose waves both move operands and compute, two workgroups to a CU or one (us, weights from HBM): 320 -> 320 at 2 x 72 x 72 47.7 -> 27.6,
 // 2 x 96 x 96 52.6 -> 34.2, 2 x 104 x 152 81.3 -> 60.2, 2 x 128 x 120 80.7 -> 60.6, 640 -> 320 at 2 x 96 x 96 95 -> 60.5, 2 x 88 x 120 108 -> 69.5, 640 -> 640 at 2 x 64 x 76 94 -> 65,
-// 1280 -> 640 at 2 x 56 x 56 166 -> 99, 1280 -> 1280 at 4 x 24 x 24 100 -> 83, 2 x 36 x 36 90 -> 87.  One round of 128 x 128 is as fast there or faster
-// unless its columns are many (320 -> 320 at 1 x 104 x 88 29.1 against 31.1, 640 -> 640 at 2 x 44 x 44 41.9 against 42.2; 640 -> 1280 at 2 x 36 x 32 53.7 against 46.8), and so are few tiles
-// with a short sum (128 -> 320 at 2 x 64 x 64, 192 tiles, 15.0 against 16.4; 1280 -> 1280 at 8 x 8 88 against 112).
+// 1280 -> 640 at 2 x 56 x 56 166 -> 99, 1280 -> 1280 at 4 x 24 x 24 100 -> 83, 2 x 36 x 36 90 -> 87.
+// Where 128 x 128 is one round (that kernel, these tiles): few columns are as fast there or faster (320 -> 320 at 1 x 104 x 88 25.6, 27.6, at 2 x 68 x 68 26.2, 27.7,
+// 960 -> 320 at 2 x 64 x 72 64.0, 65.7), many are faster here (640 -> 1280 at 2 x 36 x 32 53.7, 46.8); 640 may be either (640 -> 640 at 2 x 46 x 46 43.4, 43.5, at 2 x 48 x 48 45.1, 45.9,
+// 1920 -> 640 at 2 x 56 x 56 137 both, 320 -> 640 at 2 x 52 x 52 27.5, 26.8, 960 -> 640 at 2 x 48 x 56 70.7, 66.0, 1280 -> 640 at 2 x 48 x 52 96.2, 84.1) and stays there.  So do
+// short sums (128 -> 320 at 2 x 64 x 64 14.3, 16.4, 256 -> 320 at 2 x 70 x 70 22.5, 23.8) and few tiles (1280 -> 1280 at 8 x 8 88, 112).
 // Linear layers without row statistics (which go by 128 columns), before on 256 x 128 or 128 x 128 tiles, T given: 1300 / 3840 / 1280 21.8 -> 19.0, 1536 25.5 -> 21.1, 1800
 // 25.4 -> 23.6, 5120 / 1280 / 1280 22.7 -> 19.8, K 5120 71.7 -> 60.6, 4608 / 1920 / 640 25.8 -> 21.4, 6000 27.5 -> 24.2, 10000 / 640 / 640 14.5 -> 12.9.
 int lora_gemm_rounds_form(const LoraGemmParams& p) {

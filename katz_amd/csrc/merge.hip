@@ -12,7 +12,7 @@
 //   * the up tile [128, r] and the down tile [r, 128] go to LDS, 64 ranks at a time, down with its rank axis turned inside;
 //   * W' = bf16(float(W) + scale * acc): fp32 accumulate, one rounding (the reference rounds the product and the
 //     scaled product to half first).
-// 345 MB of weights (1280 wide, five blocks), float16 operands of rank 64: 324 -> 178 us (4.0 TB/s); rank 128 435 -> 229, rank 16 278 -> 159;
+// 345 MB of weights (1280 wide, five blocks), float16 operands of rank 64: 325 -> 179 us (4.0 TB/s); rank 128 439 -> 234, rank 16 278 -> 159;
 // 640 wide, six blocks, rank 32: 90 -> 51.  Workgroups of 512 threads with half the rows per wave: 205 us, four of 256 to a CU spill: 280.
 // Adapter operands may be bf16 or fp16 storage (Katz keeps adapters as float16 arrays in shared memory,
 // load_lora_shm_multi.py:49-61): fp16 operands use the f16 MFMA, so nothing is converted on the way.
@@ -24,7 +24,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int MG_BM = 128, MG_BN = 128, MG_THREADS = 256;
 constexpr int MG_RMAX = 128;                 // largest rank
-constexpr int MG_RC = 64;                    // ranks in LDS at a time: with 128 two workgroups fit a CU in place of three (rank 128: 301 us instead of 229)
+constexpr int MG_RC = 64;                    // ranks in LDS at a time: with 128 two workgroups fit a CU in place of three (rank 128: 301 us instead of 234)
 
 struct MergeRow {       // one layer; mirrors the six 64-bit words of the table in include/katz_hip.h
   uint64_t w, up, down; // device addresses: W [N,K] bf16, up [N,r], down [r,K]
@@ -162,7 +162,7 @@ __global__ __launch_bounds__(MG_THREADS, 3) void lora_merge_kernel(const MergeRo
         u32x4 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = sums(old[i][j][e], e);
-        *reinterpret_cast<u32x4*>(W + (size_t)row * K + col) = o;   // (through the L2: 182 us instead of 178)
+        *reinterpret_cast<u32x4*>(W + (size_t)row * K + col) = o;   // (through the L2: 182 us instead of 179)
       } else if (half) {
 #pragma unroll
         for (int e = 0; e < 4; e += 2)

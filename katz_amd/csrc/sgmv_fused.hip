@@ -18,7 +18,7 @@
 // read while the stage before is multiplied, the y pieces of the first five tiles (128 rows: of the first) requested while phase 1 runs, the
 // results written through the L2 (behind plain stores the launch ended with all of y still to be written: 1 us of 20), and 64-row blocks while
 // they fit one round of the 256 CUs, so that fewer of them repeat phase 1 for other columns.
-// 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 20.2 -> 17.6 us, all of rank 32 19.7 -> 15.2; 2 x 1024 rows 13.5 -> 12.9.
+// 8 requests of 256 .. 1024 rows at 1280 -> 1280, ranks 8 .. 128: 20.1 -> 17.6 us, all of rank 32 19.5 -> 15.1; 2 x 1024 rows 13.5 -> 12.9 (launches in a graph).
 // Rows / columns of A_a / B_a beyond the adapter's rank are zero by contract, so the padded rank only saves work.
 // Batches with few row blocks deal the column tiles of y to several workgroups, each of which repeats phase 1 for its rows: x is then read from
 // L2 more than once, which such small batches do not notice.  How many is decided by the segments' true lengths, which only the device knows
@@ -112,7 +112,8 @@ __global__ __launch_bounds__(512, 2) void sgmv_fused_kernel(const FusedParams p)
       z = z < all_tiles ? z : all_tiles;
       int v = u - full;
       // A range more for the blocks of adapters of more than 64 where that fits beside the others: a stage of theirs is 24 KB, of the others 12 or 16
-      // (8 requests of mixed ranks 18.6 -> 17.6 us, 16 of 357 .. 961 rows 26.0 -> 22.9; waiting for the ranks before the sum costs all calls 0.1)
+      // (8 requests of mixed ranks 18.6 -> 17.6 us, 16 of 357 .. 961 rows 26.0 -> 22.9; the wait for the ranks before the sum
+      // does not show: within 0.05 either way without it)
       const int h8 = (heavy + 7) & ~7, l8 = (nb - heavy + 7) & ~7;
       if (full == 0 && p.n_layers == 1 && heavy > 0 && heavy < nb && z < all_tiles && h8 * (z + 1) + l8 * z <= CUS) {
         const bool mine = v < h8 * (z + 1);

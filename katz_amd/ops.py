@@ -629,7 +629,7 @@ def lora_linear_xattn(x: torch.Tensor, weight: torch.Tensor, k: torch.Tensor, v:
                       b_cat: Optional[torch.Tensor] = None, two_launches: bool = False, r_used: int = 0,
                       ln=None) -> torch.Tensor:
     """attention(lora_linear_norm(x, weight, ...), k, v) in one launch (kh_lora_linear_xattn_bf16): the query projection of a
-    cross-attention over a short context (S <= 96) whose 128 x 128 output tiles (128 queries of two heads) go through the
+    cross-attention over a short context (S <= 96) whose output tiles (32 to 128 queries of whole heads) go through the
     attention inside the GEMM's epilogue instead of to memory.  x [B,T,K]; k / v [B,S,heads*64] (last-dim-contiguous
     views); the other arguments as for lora_linear_norm.  Returns [B,T,heads*64]."""
     lib = _lib.load()
