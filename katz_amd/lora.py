@@ -341,7 +341,7 @@ def pack_many(layers: Sequence, names: Sequence[Sequence[str]]) -> List[PackedAd
                 w = g.weight
                 nk = keys[id(g)] = (norm_key(g), w.data_ptr(), g.bias.data_ptr()) if w.dtype == torch.bfloat16 and w.device == dev else ()
         rows += (at_a, at_an if nk else -1) + (nk[1:] if nk else (0, 0)) + (at_c, at_c, at_b, at_s, K, N, R, int(d["geglu"]), n_pieces, len(ns))
-        packs.append(PooledPack(pool if nk else plain, (at_a, at_b, at_s, at_an, at_c), (R, K, N), ns, ranks, min(R, (c + 15) // 16 * 16), nk[0] if nk else None))
+        packs.append(PooledPack(pool if nk else plain, (at_a, at_b, at_s, at_an, at_c), (R, K, N), tuple(ns), ranks, min(R, (c + 15) // 16 * 16), nk[0] if nk else None))
         n_pieces += len(ns)
         padded.append(R)
         b_blocks.append(-(-N // (256 // (R // 8))))

@@ -852,3 +852,24 @@ def test_packs_without_a_norm_do_not_keep_the_folded_buffers(monkeypatch):
     del packs[:2]
     gc.collect()
     assert len(folded) == 3 and all(r() is None for r in folded) and all(r() is not None for r in shared)
+
+
+def test_a_pack_keeps_the_names_it_was_made_with(monkeypatch):
+    """pack_many's callers may go on using their lists of names: a pack's spans, made when somebody asks for them, are those of the call, as is what is
+    rescaled by them."""
+    from katz_amd import ops
+    from katz_amd.lora import Adapter, pack_many, rescale_
+    import katz_amd.layers as L
+
+    monkeypatch.setattr(ops, "upload_many", lambda ts, dev: (None, [t.data_ptr() for t in ts]))
+    monkeypatch.setattr(ops, "lora_pack", lambda *a: None)
+    l = L.LoRALinear(16, 24, bias=False).bfloat16()
+    for n, r in (("a", 8), ("b", 16)):
+        l.adapters[n] = Adapter(torch.randn(r, 16).bfloat16(), torch.randn(24, r).bfloat16(), weight=0.25 if n == "a" else 0.5)
+    names = ["a", "b"]
+    p, = pack_many([l], [names])
+    names[:] = ["b"]
+    assert p.spans == [("a", 0, 8), ("b", 8, 16)] and p.r_used == 32
+    p.col_scale.zero_()
+    rescale_(p, l.adapters)
+    assert p.col_scale[:24].tolist() == [0.25] * 8 + [0.5] * 16 and not p.col_scale[24:].any()
