@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the adapter-augmented SDXL UNet step on one MI355X.
 
-Workload (the configuration the metric is quoted on): one bf16
+Workload (the configuration that the metric is quoted on): one bf16
 UNet2DConditionModel denoising step, random-init SDXL weights, latent [2,4,128,128] (CFG batch 2,
 1024x1024), t=500, context [2,77,2048], pooled text [2,1280], time_ids [2,6]; two LoRAs (rank 64 scale
 0.8, rank 32 scale 0.6) on all 722 attention / feed-forward / projection linears, one ControlNet
@@ -47,7 +47,7 @@ def build_product(device, seed=0):
     return unet.to_runtime(device, torch.bfloat16)
 
 
-LORA_SPECS = (("r64", 64, 0.8), ("r32", 32, 0.6))   # (adapter name, rank, weight): BASELINE.json configs[2]
+LORA_SPECS = (("r64", 64, 0.8), ("r32", 32, 0.6))   # (adapter name, rank, weight)
 
 
 def add_random_loras(unet, device, specs=LORA_SPECS, seed=10):
@@ -152,7 +152,7 @@ def cpu_model():
 
 
 def sgmv_rooflines(dev):
-    """Segmented shrink / expand (BASELINE.json configs[3]: 8 requests, one adapter each, ranks from {8..128}) at the
+    """Segmented shrink / expand (8 requests, one adapter each, ranks from {8..128}) at the
     two SDXL widths, timed per launch with HIP events; algorithmic bytes: shrink 2(sum T K + sum r K + sum T r), expand
     2(sum T r + sum r N + 2 sum T N) (y is read, updated and written)."""
     import torch
@@ -290,7 +290,7 @@ def cpu_baseline_sample(cores, reps=3):
 
 
 def cpu_baseline_full_step(cores):
-    """ONE full step of BASELINE.json configs[2] on the fp32 CPU oracle (oracle/unet_sdxl.py, the restatement of the
+    """ONE full step of the workload on the fp32 CPU oracle (oracle/unet_sdxl.py, the restatement of the
     reference's diffusers path: 2.57 B parameters, both LoRAs unmerged on all 722 linears, the 9 + 1 ControlNet residuals),
     on `cores` threads.  The weights are random (their values do not change the time): the model is created without
     torch's initialisers and filled from one pool of normal numbers scaled per tensor, which takes seconds instead of
@@ -361,7 +361,7 @@ def traffic_from_profiles(kernel_prefix):
 
 
 def kernel_probe():
-    """Counter / trace run of the individual kernels at the shapes of BASELINE.json's configurations, three times
+    """Counter / trace run of the individual kernels at the shapes of the measured workloads, three times
     each, preceded by a 64 MiB device copy of known size (the calibration of FETCH_SIZE / WRITE_SIZE).
     Used as  rocprofv3 --kernel-trace --stats -- python3 bench.py --kernel-probe  (durations) and
     rocprofv3 --pmc <counter> -- python3 bench.py --kernel-probe  (one counter per run).  Prints, as JSON, the
@@ -565,7 +565,7 @@ def merge_probe():
 
 
 def loop_bench(args):
-    """the 50-step guided denoise loop at 1024x1024 -- random-init SDXL UNet with the two
+    """The 50-step guided denoise loop at 1024x1024 -- random-init SDXL UNet with the two
     LoRAs, random-init SDXL-size ControlNet (from_unet, conditioning image [2,3,1024,1024] uniform[0,1], scale 0.5),
     Euler discrete scheduler (SDXL schedule), guidance 7.5, seeded latents x init_noise_sigma; every step is one replay
     of one captured graph holding ControlNet -> UNet -> guidance + Euler.  Prints one JSON line: end-to-end ms of the
@@ -668,7 +668,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--loop", action="store_true",
-                    help="BASELINE configs[4]: the 50-step ControlNet + UNet + Euler denoise loop, end-to-end ms")
+                    help="the 50-step ControlNet + UNet + Euler denoise loop, end-to-end ms")
     ap.add_argument("--merge-probe", action="store_true",
                     help="time Katz's patch_on_lora (merge of a rank-64 adapter into all 722 SDXL linears)")
     ap.add_argument("--loop-steps", type=int, default=50)
@@ -677,10 +677,10 @@ def main():
     ap.add_argument("--context-kv-per-step", action="store_true",
                     help="--loop: project the text context's K / V inside every step (as the reference does) instead of once per loop")
     ap.add_argument("--kernel-probe", action="store_true",
-                    help="run only a 64 MiB copy and each kernel at its BASELINE shapes three times (for rocprofv3)")
+                    help="run only a 64 MiB copy and each kernel at its measured shapes three times (for rocprofv3)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build runs on ONE GPU only (no collectives, no sharding); --gpus must be 1",
+        print("bench.py: runs on ONE GPU only (no collectives, no sharding); --gpus must be 1",
               file=sys.stderr)
         sys.exit(2)
 

@@ -72,7 +72,7 @@ class _Plan:
         self.tensors = []                                  # parameters: same version, same address
         self.hooks = []                                    # hook tables that have to be empty
         self.keep = []                                     # what the addresses in the descriptor belong to
-        self.linears = []                                  # (entry, layer, LayerNorm folded into it)
+        self.linears = []                                  # (entry, layer, LayerNorm folded into it, its norm_key)
         self.ready = None
         self.desc = _Block()
         self.seen(blk, "norm1", "attn1", "norm2", "attn2", "norm3", "ff")

@@ -178,7 +178,7 @@ class UNet2DConditionModel(nn.Module):
         self._ctx_kv = None
         # The reference's switches (read at construction, unet_2d_condition.py:511, resnet.py:330, normalization.py:31).
         # ENABLE_CUDA_GRAPH=1: forward replays a captured HIP graph of the step (see _forward_graphed).
-        # ENABLE_FUSED_NORM_SILU / ENABLE_CHANNELS_LAST: accepted and recorded; this build always runs the fused
+        # ENABLE_FUSED_NORM_SILU / ENABLE_CHANNELS_LAST: accepted and recorded; what always runs is the fused
         # GroupNorm+SiLU kernel on NHWC memory, which is what the reference does with both switched on, so they change
         # nothing here.  ENABLE_FUSED_GEGLU is read by layers.GEGLU.
         from .layers import env_flag

@@ -5,7 +5,7 @@ Source data (JSON, read as text; nothing of the reference is executed):
   /root/reference/lora_info_shm/TheLastBen_Papercut_SDXL.json                   lora key -> {shape, nbytes}
   /root/reference/lora_info_shm/TheLastBen_Papercut_SDXL_alphas.json            alpha per module
 Output: {"<unet weight key>": {"down_key": ..., "up_key": ..., "down": [r, in], "up": [out, r], "alpha": a}}
-Run in the build container only (the reference tree does not exist on the GPU box).
+Needs the reference tree.
 """
 import json
 from pathlib import Path

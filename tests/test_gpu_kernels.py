@@ -200,7 +200,7 @@ def test_lora_linear_bf16_geglu_epilogue():
 
 
 def test_lora_linear_f32_config1():
-    """BASELINE config 1: x [2,4096,640], W [640,640], rank 32, scale 0.8, fp32, <= 1e-4."""
+    """x [2,4096,640], W [640,640], rank 32, scale 0.8, fp32, <= 1e-4."""
     from katz_amd import ops
 
     say("lora_linear_f32 config1")
@@ -476,7 +476,7 @@ def test_upsample_nearest2x(shape):
                                    (77, 2048, 640), (77, 2048, 1280),        # cross-attention to_k / to_v (context 2048)
                                    (1024, 1280, 10240), (1024, 5120, 1280)], ids=str)   # feed-forward in / out
 def test_sgmv_heterogeneous_batch(T, K, N):
-    """BASELINE config 4: 8 requests, each with its own adapter, ranks drawn (seed 2) from {8,16,32,64,128}, on every
+    """8 requests, each with its own adapter, ranks drawn (seed 2) from {8,16,32,64,128}, on every
     shape class of the SDXL attention linears (self-attention and to_out d x d, cross-attention to_k / to_v 2048 -> d)
     plus the feed-forward widths."""
     from katz_amd import ops

@@ -510,7 +510,7 @@ def test_a_replaced_pack_is_let_go_of():
 
 
 def test_bench_refuses_more_than_one_gpu():
-    """bench.py --gpus N with N > 1 exits with a message: this build runs on one GPU (no collectives, no sharding)."""
+    """bench.py --gpus N with N > 1 exits with a message: it runs on one GPU (no collectives, no sharding)."""
     import subprocess
     import sys
     from pathlib import Path
