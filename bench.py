@@ -131,8 +131,8 @@ def instrumented_step(unet, inputs):
 
 
 def host_cores():
-    """Threads for the CPU baseline: the share of the host this job has been given (OMP_NUM_THREADS, which the GPU
-    boxes set to their per-GPU share of cores), never more than the CPUs visible."""
+    """Threads for the CPU baseline: the share of the host this job has been given (OMP_NUM_THREADS where
+    it is set), never more than the CPUs visible."""
     n = os.cpu_count() or 1
     try:
         n = min(n, int(os.environ.get("OMP_NUM_THREADS", n)))
